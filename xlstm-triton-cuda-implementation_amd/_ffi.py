@@ -120,6 +120,23 @@ def lib():
     return _lib
 
 
+_native = None
+
+
+def native():
+    """The operators' host path in native code (csrc/mlstm_torch.cpp).  Raises if it has not been built, like ``lib``."""
+    global _native
+    if _native is None:
+        lib()
+        try:
+            from . import _native as module
+        except ImportError as e:
+            raise ImportError(f"{os.path.join(_HERE, '_native.so')} is missing or does not load ({e}): build it with "
+                              f"`make -C {os.path.join(_HERE, 'csrc')}` (or __graft_entry__.build())") from None
+        _native = module
+    return _native
+
+
 def exported_symbols():
     return ["mlstm_forward", "mlstm_backward", "mlstm_forward_ex", "mlstm_forward_noalloc_ex", "mlstm_backward_ex", "mlstm_scan_forward_ex",
             "mlstm_scan_backward_ex", "mlstm_scan_forward_save_ex", "mlstm_scan_backward_saved_ex", "slstm_saved_bytes", "slstm_workspace_bytes", "slstm_forward_ex", "slstm_backward_ex", "mlstm_forward_lx", "mlstm_backward_lx", "mlstm_forward_save_lx", "mlstm_backward_saved_lx",

@@ -209,11 +209,25 @@ def mlstm_backward_saved_hip(dh, q, k, v, f, i, h, m, b, saved, precise=False, g
 
 def mlstm_matmul(q, k, v, f, i, SB=16, num_warps=8):
     """Forward only, no autograd (reference mlstm_matmul.py:121-129)."""
-    return mlstm_forward_hip(q, k, v, f, i)[0]
+    h = _ffi.native().matmul(q, k, v, f, i)
+    return h if h is not None else mlstm_forward_hip(q, k, v, f, i)[0]
+
+
+# Triton_mLSTM and its variants go to the native host path (csrc/mlstm_torch.cpp: checks, allocations, launches and the graph's
+# node in C++), which returns None for whatever it does not serve: padded and widened head dimensions, layouts that need a copy
+# first, arguments that are an error.  Those take the autograd functions below.
+def _native_matmul(q, k, v, f, i, precise, gate_form):
+    form = _ffi.GATE_FORMS.get(gate_form)
+    return None if form is None else _ffi.native().matmul_train(q, k, v, f, i, precise, form)
 
 
 class Triton_mLSTM(torch.autograd.Function):
     """Drop-in for the reference's autograd function of the same name (mlstm_matmul.py:368-405)."""
+
+    @classmethod
+    def apply(cls, q, k, v, f, i, SB=16, num_warps=8, gate_form="raw"):
+        h = _native_matmul(q, k, v, f, i, 0, gate_form)
+        return h if h is not None else super().apply(q, k, v, f, i, SB, num_warps, gate_form)
 
     @staticmethod
     def forward(ctx, q, k, v, f, i, SB=16, num_warps=8, gate_form="raw"):
@@ -241,6 +255,11 @@ class Triton_mLSTM_precise(torch.autograd.Function):
     weights of every second product enter it as two terms, so that results and gradients agree with an fp32
     evaluation of the reference's formulas element by element at rtol 2e-2 / atol 2e-3.  Slower: no chunking, half as
     many MFMAs again.  Same call signature."""
+
+    @classmethod
+    def apply(cls, q, k, v, f, i, SB=16, num_warps=8, gate_form="raw"):
+        h = _native_matmul(q, k, v, f, i, 1, gate_form)
+        return h if h is not None else super().apply(q, k, v, f, i, SB, num_warps, gate_form)
 
     @staticmethod
     def forward(ctx, q, k, v, f, i, SB=16, num_warps=8, gate_form="raw"):
@@ -323,11 +342,17 @@ def mlstm_backward_gated_hip(dhg, q, k, v, f, i, o, h=None, m=None, b=None):
 
 def mlstm_matmul_gated(q, k, v, f, i, o, SB=16, num_warps=8):
     """Forward only, no autograd: the value mlstm_scan(q, k, v, f, i, o) returns, computed in the matmul form."""
-    return mlstm_forward_gated_hip(q, k, v, f, i, o)[0]
+    h = _ffi.native().gated(q, k, v, f, i, o)
+    return h if h is not None else mlstm_forward_gated_hip(q, k, v, f, i, o)[0]
 
 
 class Triton_mLSTM_gated(torch.autograd.Function):
     """``Triton_mLSTM_gated.apply(q, k, v, f, i, o, SB, NUM_WARPS)``: Triton_mLSTM followed by the silu(o) gate."""
+
+    @classmethod
+    def apply(cls, q, k, v, f, i, o, SB=16, num_warps=8):
+        h = _ffi.native().gated_train(q, k, v, f, i, o)
+        return h if h is not None else super().apply(q, k, v, f, i, o, SB, num_warps)
 
     @staticmethod
     def forward(ctx, q, k, v, f, i, o, SB=16, num_warps=8):

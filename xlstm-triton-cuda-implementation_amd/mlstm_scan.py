@@ -104,6 +104,9 @@ class Scan_mLSTM(torch.autograd.Function):
 
 
 def mlstm_scan(q, k, v, f, i, o, reduce_block_size=4, value_block_size=4, num_warps=8):
+    h = _ffi.native().scan(q, k, v, f, i, o)   # (None: nothing the native host path serves)
+    if h is not None:
+        return h
     if torch.is_grad_enabled() and any(t.requires_grad for t in (q, k, v, f, i, o)):
         return Scan_mLSTM.apply(q, k, v, f, i, o)
     return mlstm_scan_forward_hip(q, k, v, f, i, o)

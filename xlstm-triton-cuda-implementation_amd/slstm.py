@@ -76,6 +76,9 @@ class HIP_sLSTM(torch.autograd.Function):
 
 
 def slstm(wx, r, b, forget_sigmoid=False):
+    h = _ffi.native().slstm(wx, r, b, 1 if forget_sigmoid else 0)   # (None: nothing the native host path serves)
+    if h is not None:
+        return h
     if torch.is_grad_enabled() and any(t.requires_grad for t in (wx, r, b)):
         return HIP_sLSTM.apply(wx, r, b, forget_sigmoid)
     return slstm_forward_hip(wx, r, b, forget_sigmoid, save=False)[0]
