@@ -62,11 +62,12 @@ int chunk_len_for(int dtype, int D, size_t S) {
     const bool shape_ok = dtype == MLSTM_F32 ? (D == 64 || D == 128) : (D == 64 || D == 128 || D == 256);
     if (!shape_ok || g_chunk_override < 0) return 0;
     if (g_chunk_override > 0) return S > (size_t)g_chunk_override ? g_chunk_override : 0;
-    if (S < 1024) return 0;   // (below two full chunks of 512 the state pass costs more than the skipped key tiles)
     // fp32 products run at a sixteenth of the 16-bit rate, so the key tiles a chunk saves weigh more against the states: the
-    // shortest chunk wins there (B1 H4 S2048 D64: 0.47 ms unchunked, 0.24 / 0.16 / 0.13 ms at 512 / 256 / 128; D = 128
-    // likewise); at D = 64 in 16 bits 256 is the measured best (B4 H8 S4096: 0.48 unchunked, 0.24 / 0.22 / 0.25 ms)
-    if (dtype == MLSTM_F32) return 128;
+    // shortest chunk wins at every length that has more than two of them (forward + backward, 8 heads, unchunked -> 128:
+    // D = 64 88 -> 85 us at S = 256, 142 -> 88 at 512, 469 -> 104 at 2048; D = 128 141 -> 144, 241 -> 151, 849 -> 180)
+    if (dtype == MLSTM_F32) return S >= 320 ? 128 : 0;
+    if (S < 1024) return 0;   // (below two full chunks of 512 the state pass costs more than the skipped key tiles)
+    // at D = 64 in 16 bits 256 is the measured best (B4 H8 S4096: 0.48 unchunked, 0.24 / 0.22 / 0.25 ms at 128 / 256 / 512)
     return D == 64 ? 256 : 512;
 }
 
@@ -83,8 +84,8 @@ struct Sizes {
     size_t stats() const { return 2 * up256(BH * S * 4); }                       // m, b
     // chunked forward: per-chunk sums (fp32), matrix states (element type), vector states
     size_t n_states(int L) const { return L > 0 && S > (size_t)L ? (S - 1) / L : 0; }
-    size_t chunk_states(int dtype) const {
-        const size_t n = n_states(chunk_len_for(dtype, (int)D, S));
+    size_t chunk_states() const {
+        const size_t n = n_states(chunk_len());
         return up256(BH * n * D * D * 4) + up256(BH * n * D * D * el * parts()) + up256(BH * n * D * 4);
     }
     int dtype_code = MLSTM_F32;
@@ -94,7 +95,8 @@ struct Sizes {
     int gate_form = MLSTM_GATE_RAW;
     bool precise = false;   // split mode (MLSTM_PRECISE): states as two terms, and the low-order part of h travels to the backward
     size_t parts() const { return precise ? 2 : 1; }   // terms per matrix state: hi, and lo directly behind it
-    int chunk_len() const { return chunk_len_for(dtype_code, (int)D, S); }
+    bool whole = false;     // the sequence in one piece, whatever its length (a workspace that cannot hold chunk states)
+    int chunk_len() const { return whole ? 0 : chunk_len_for(dtype_code, (int)D, S); }
     size_t state_elems() const { return BH * n_states(chunk_len()) * D * D; }             // one term of one set of states
     size_t states_t() const { return up256(state_elems() * el * parts()); }               // value-major copy for the dQ pass
     size_t saved_vec() const { return up256(BH * n_states(chunk_len()) * D * 4); }
@@ -117,8 +119,8 @@ struct Sizes {
                (size_t)(scan_key_splits((int)BH, (int)D) - 1) * up256(BH * S * D * 4) +
                up256(scan_segment_state_bytes((int)BH, (int)S, (int)D));
     }
-    size_t fwd() const { return scan_engine() ? scan_fwd() : gates() + stats() + chunk_states(dtype_code); }
-    size_t anchor_parts() const { return D >= 64 ? (D / 64) * (D / 64) : 1; }   // workgroups per head of the value-major carry
+    size_t fwd() const { return scan_engine() ? scan_fwd() : gates() + stats() + chunk_states(); }
+    size_t anchor_parts() const { return D >= 32 ? (D / 32) * (D / 32) : 1; }   // workgroups per head of the value-major carry, at most
     size_t fwd_fixed() const { return gates() + stats(); }   // offset of the chunk states inside fwd()
     size_t bwd() const {
         if (scan_engine()) return scan_backward_workspace_bytes((int)BH, (int)S, (int)D);
@@ -129,9 +131,16 @@ struct Sizes {
                + up256(BH * S * 4) + up256(BH * row_slices() * S * 4)              // colsum, rowpart
                + h_lo();                                                           // split mode: low-order part of a recomputed h
     }
+    // scan form, forward: the tile kernels write the ungated output as well
+    size_t scan_form_fwd() const { return D <= 128 ? fwd() + up256(BH * S * D * 4) : scan_fwd(); }
     // gated backward: the ungated upstream gradient, and (h, m, b) when the caller does not bring them
     size_t bwd_gated() const { return bwd() + 2 * up256(BH * S * D * el) + stats(); }
 };
+
+// The scan form at D = 64 and 128 runs on the tile kernels (chunk_len_for's chunks, the gate fused into the row kernel): the
+// same function, and at these head dimensions the faster way -- the scan kernels walk a head's chunks of 64 positions one
+// after the other on D / 32 workgroups (B2 H4 S1000 D128: 94 us forward, 366 us forward + backward).
+bool scan_on_tiles(int D) { return D <= 128; }
 
 // begin/end marks for groups of scan kernels (the scan translation unit has no access to Timed)
 thread_local Timed* g_scan_mark[16] = {};
@@ -401,6 +410,15 @@ int forward_impl(const void* q, const void* k, const void* v, const void* f, con
     return rc;
 }
 
+// the scan form's forward on the tile kernels, on a workspace of Sizes::scan_form_fwd() bytes; h_ungated (may be null)
+// receives the output before the gate, b (may be null) the normaliser sums
+int scan_forward_on_tiles(const void* q, const void* k, const void* v, const void* f, const void* i, const void* o, void* h, void* h_ungated, float* b,
+                          const Sizes& z, char* ws, hipStream_t st) {
+    if (!h_ungated) h_ungated = ws + z.fwd();
+    return forward_impl(q, k, v, f, i, h_ungated, nullptr, b, z, (int)z.D, MLSTM_F32, MLSTM_F32, ws, st, nullptr, nullptr, nullptr, nullptr, nullptr,
+                        nullptr, nullptr, o, h);
+}
+
 }  // namespace
 
 extern "C" {
@@ -421,6 +439,7 @@ int mlstm_set_column_kernel(int variant) {
 
 int mlstm_chunk_length_for(int S, int D, int dtype) {
     if (S <= 0 || D <= 0 || !good_dtype_arg(dtype)) return 0;
+    if (S < 1024 && g_chunk_override == 0) return 0;   // (shorter sequences are not reported: see the header)
     return chunk_len_for(dtype & ~MLSTM_PRECISE, D, (size_t)S);
 }
 
@@ -500,9 +519,9 @@ size_t mlstm_workspace_bytes(int op, int B, int NH, int S, int D, int dtype) {
         case MLSTM_OP_BACKWARD: return z.bwd();
         case MLSTM_OP_FORWARD_GATED: return z.fwd();
         case MLSTM_OP_BACKWARD_GATED: return z.bwd_gated();
-        case MLSTM_OP_SCAN_FORWARD: return z.scan_fwd();
+        case MLSTM_OP_SCAN_FORWARD: return z.scan_form_fwd();
         case MLSTM_OP_SCAN_BACKWARD:
-            return (D % 64 == 0 && D >= 64) ? scan_backward_workspace_bytes((int)z.BH, S, D) : 0;
+            return (D % 64 == 0 && D >= 64) ? (scan_on_tiles(D) ? z.bwd_gated() : scan_backward_workspace_bytes((int)z.BH, S, D)) : 0;
     }
     return 0;
 }
@@ -537,7 +556,9 @@ int mlstm_forward_noalloc_ex(const void* q, const void* k, const void* v, const 
     dtype &= ~MLSTM_PRECISE;
     if (!good_shape(D, dtype) || S > 131072) return MLSTM_ESHAPE;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    const Sizes z = sizes_of(B, NH, S, D, dtype_arg);
+    Sizes z = sizes_of(B, NH, S, D, dtype_arg);
+    // (sequences below 1024 positions need no chunks to be fast enough, and their chunk states may be what does not fit)
+    if (S < 1024 && z.fwd() > NOALLOC_SCRATCH_BYTES) z.whole = true;
     if (z.fwd() > NOALLOC_SCRATCH_BYTES) return MLSTM_EWORKSPACE;   // the shape needs more scratch than the array holds
     char* ws = nullptr;
     if (int rc = symbols_of_current_device(&ws, nullptr)) return rc;
@@ -656,7 +677,7 @@ int backward_impl(const void* dh, const void* q, const void* k, const void* v, c
     float* anchor = c.take<float>(z.BH * w.ncs * z.anchor_parts());
     int anchor_parts = 0;
     // (the one-kernel dF pass adds the parts up; see DfArgs)
-    const bool fused_anchor = w.L <= 1024 && mlstm::chunk_states_fused_dot(dtype, D);
+    const bool fused_anchor = w.L <= 1024;
     char* hlo_buf = c.take<char>(z.precise ? z.BH * z.S * z.D * z.el : 0);
     const size_t lo_off = z.state_elems() * z.el;   // split mode: a set of states is [hi | lo]
     const bool col_chunks = z.col_chunks();
@@ -745,6 +766,38 @@ int backward_impl(const void* dh, const void* q, const void* k, const void* v, c
     return launch_df(gate_dtype, da, st);
 }
 
+// the gated backward on a workspace of Sizes::bwd_gated() bytes; dense_out: dh_gated, o, h and d_o are dense tensors
+int backward_gated_impl(const void* dh_gated, const void* q, const void* k, const void* v, const void* f, const void* i, const void* o,
+                        const void* h, const float* m, const float* b, void* dq, void* dk, void* dv, void* df, void* di, void* d_o, const Sizes& z,
+                        int NH, int D, int dtype, int gate_dtype, bool dense_out, char* ws, hipStream_t st) {
+    Carver c{ws, z.bwd()};
+    char* dh = c.take<char>(z.BH * z.S * z.D * z.el);
+    char* hown = c.take<char>(z.BH * z.S * z.D * z.el);
+    float* mown = c.take<float>(z.BH * z.S);
+    float* bown = c.take<float>(z.BH * z.S);
+    const Lay dense = dense_layout(NH, (long long)z.S, (long long)z.D);
+    Lay lh = z.lb;
+    if (!(h && m && b)) {  // the ungated h is an input of the gate's own backward: rebuild it (and m, b) first, dense
+        Sizes zf = z;
+        zf.lb = dense;
+        if (int rc = forward_impl(q, k, v, f, i, hown, mown, bown, zf, D, dtype, gate_dtype, ws, st)) return rc;
+        h = hown; m = mown; b = bown;
+        lh = dense;
+    }
+    {
+        Timed t(MLSTM_K_GATE_BWD, st);
+        if (dense_out) {
+            if (int rc = launch_gate_backward(dtype, dh_gated, o, h, dh, d_o, z.BH * z.S * z.D, st)) return rc;
+        } else if (int rc = launch_gate_backward_rows(dtype, dh_gated, o, h, dh, d_o, (int)z.BH, (int)z.S, (int)z.D, z.lb, lh, dense, st)) {
+            return rc;
+        }
+    }
+    // the ungated upstream gradient is the library's own, dense; h stays where it is
+    Sizes zb = z;
+    zb.lb = dense;
+    return backward_impl(dh, q, k, v, f, i, h, m, b, dq, dk, dv, df, di, zb, D, dtype, gate_dtype, ws, st, nullptr, &lh);
+}
+
 }  // namespace
 
 extern "C" {
@@ -825,33 +878,8 @@ int mlstm_backward_gated_lx(const void* dh_gated, const void* q, const void* k, 
     if (int rc = apply_layout(z, layout, NH, gate_dtype, {dh_gated, q, k, v, o, h, dq, dk, dv, d_o}, true, true, true)) return rc;
     Scratch sc;
     if (int rc = sc.get(workspace, workspace_bytes, z.bwd_gated(), st)) return rc;
-    char* ws = (char*)sc.p;
-    Carver c{ws, z.bwd()};
-    char* dh = c.take<char>(z.BH * z.S * z.D * z.el);
-    char* hown = c.take<char>(z.BH * z.S * z.D * z.el);
-    float* mown = c.take<float>(z.BH * z.S);
-    float* bown = c.take<float>(z.BH * z.S);
-    const Lay dense = dense_layout(NH, (long long)z.S, (long long)z.D);
-    Lay lh = z.lb;
-    if (!(h && m && b)) {  // the ungated h is an input of the gate's own backward: rebuild it (and m, b) first, dense
-        Sizes zf = z;
-        zf.lb = dense;
-        if (int rc = forward_impl(q, k, v, f, i, hown, mown, bown, zf, D, dtype, gate_dtype, ws, st)) return rc;
-        h = hown; m = mown; b = bown;
-        lh = dense;
-    }
-    {
-        Timed t(MLSTM_K_GATE_BWD, st);
-        if (!layout) {
-            if (int rc = launch_gate_backward(dtype, dh_gated, o, h, dh, d_o, z.BH * z.S * z.D, st)) return rc;
-        } else if (int rc = launch_gate_backward_rows(dtype, dh_gated, o, h, dh, d_o, (int)z.BH, (int)z.S, (int)z.D, z.lb, lh, dense, st)) {
-            return rc;
-        }
-    }
-    // the ungated upstream gradient is the library's own, dense; h stays where it is
-    Sizes zb = z;
-    zb.lb = dense;
-    return backward_impl(dh, q, k, v, f, i, h, m, b, dq, dk, dv, df, di, zb, D, dtype, gate_dtype, ws, st, nullptr, &lh);
+    return backward_gated_impl(dh_gated, q, k, v, f, i, o, h, m, b, dq, dk, dv, df, di, d_o, z, NH, D, dtype, gate_dtype, layout == nullptr, (char*)sc.p,
+                               st);
 }
 
 int mlstm_forward(const void* Q, const void* K, const void* V, const void* F, const void* I, void* H, unsigned S) {
@@ -873,7 +901,8 @@ int mlstm_scan_forward_ex(const void* q, const void* k, const void* v, const voi
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     const Sizes z = sizes_of(B, NH, S, D, MLSTM_F32);
     Scratch sc;
-    if (int rc = sc.get(workspace, workspace_bytes, z.scan_fwd(), st)) return rc;
+    if (int rc = sc.get(workspace, workspace_bytes, z.scan_form_fwd(), st)) return rc;
+    if (scan_on_tiles(D)) return scan_forward_on_tiles(q, k, v, f, i, o, h, nullptr, nullptr, z, (char*)sc.p, st);
     return scan_forward_impl(q, k, v, f, i, o, h, nullptr, nullptr, z, MLSTM_F32, 0, (char*)sc.p, st);
 }
 
@@ -886,7 +915,8 @@ int mlstm_scan_forward_save_ex(const void* q, const void* k, const void* v, cons
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     const Sizes z = sizes_of(B, NH, S, D, MLSTM_F32);
     Scratch sc;
-    if (int rc = sc.get(workspace, workspace_bytes, z.scan_fwd(), st)) return rc;
+    if (int rc = sc.get(workspace, workspace_bytes, z.scan_form_fwd(), st)) return rc;
+    if (scan_on_tiles(D)) return scan_forward_on_tiles(q, k, v, f, i, o, h, h_ungated, b, z, (char*)sc.p, st);
     return scan_forward_impl(q, k, v, f, i, o, h, nullptr, b, z, MLSTM_F32, 0, (char*)sc.p, st, (float*)h_ungated);
 }
 
@@ -907,9 +937,13 @@ int mlstm_scan_backward_saved_ex(const void* dh_gated, const void* q, const void
     if (dtype != MLSTM_F32) return MLSTM_ESHAPE;
     if (!(D == 64 || D == 128 || D == 256 || D == 512 || D == 1024) || S > 131072) return MLSTM_ESHAPE;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    const size_t need = scan_backward_workspace_bytes(B * NH, S, D);
+    const Sizes z = sizes_of(B, NH, S, D, MLSTM_F32);
+    const size_t need = scan_on_tiles(D) ? z.bwd_gated() : scan_backward_workspace_bytes(B * NH, S, D);
     Scratch sc;
     if (int rc = sc.get(workspace, workspace_bytes, need, st)) return rc;
+    if (scan_on_tiles(D))   // (m is formed again from the gates: b stands in for the pointer, which is not read)
+        return backward_gated_impl(dh_gated, q, k, v, f, i, o, h_ungated, b, b, dq, dk, dv, df, di, d_o, z, NH, D, MLSTM_F32, MLSTM_F32, true,
+                                   (char*)sc.p, st);
     ScanBwdArgs a{};
     a.dhg = (const float*)dh_gated; a.q = (const float*)q; a.k = (const float*)k; a.v = (const float*)v;
     a.f = (const float*)f; a.i = (const float*)i; a.o = (const float*)o;

@@ -94,7 +94,8 @@ __global__ __launch_bounds__(1024) void dfscan_kernel(const TG* __restrict__ F, 
 
 // Row reduction and dF scan of a sequence that ran in chunks, in one kernel and one workgroup per (chunk, head): with
 // the running sum known at every chunk's first position (the anchors) the chunks are independent of each other, and a
-// position has at most chunk_len / 64 row partials.  chunk_len <= 1024.
+// position has at most chunk_len / 64 row partials.  chunk_len <= 1024; as many threads as positions (or as the anchors' sums
+// take), whole waves: with 1024 whatever the chunk, most of a workgroup's waves had nothing to do but arrive at the barrier.
 template <typename TG>
 __global__ __launch_bounds__(1024) void dfchunk_kernel(const TG* __restrict__ F, const float* __restrict__ colsum, const float* __restrict__ rowpart,
                                                        const float* __restrict__ rowinter, const float* __restrict__ anchor,
@@ -103,7 +104,7 @@ __global__ __launch_bounds__(1024) void dfchunk_kernel(const TG* __restrict__ F,
                                                        const float* __restrict__ va, const float* __restrict__ vb, int D, SavedStamp stamp) {
     __shared__ float wt[16];
     __shared__ float at[2][16];
-    const int c = blockIdx.x, bh = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int c = blockIdx.x, bh = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = blockDim.x >> 6;
     stamp_apply(stamp, c == 0 && bh == 0, tid);
     // the two anchors of this chunk (its first position, and the next chunk's) from their parts: the partial sums of the
     // matrix states' contraction and the product of the vector states; both states carry the factor 1 / sqrt(D) of the
@@ -143,16 +144,14 @@ __global__ __launch_bounds__(1024) void dfchunk_kernel(const TG* __restrict__ F,
     if (lane == 63) wt[wave] = incl;
     __syncthreads();
     float pre = 0.f, tot = 0.f;
-#pragma unroll
-    for (int w = 0; w < 16; w++) {
+    for (int w = 0; w < nw; w++) {
         const float s = wt[w];
         if (w < wave) pre += s;
         tot += s;
     }
     if (anchor_part) {
         const float rs = sqrtf((float)D);
-#pragma unroll
-        for (int w = 0; w < 16; w++) { a_start += at[0][w]; a_next += at[1][w]; }
+        for (int w = 0; w < nw; w++) { a_start += at[0][w]; a_next += at[1][w]; }
         a_start *= rs; a_next *= rs;
     } else {
         a_start = c > 0 ? anchor[(size_t)bh * n_states + c - 1] : 0.f;
@@ -171,7 +170,10 @@ __global__ __launch_bounds__(1024) void dfchunk_kernel(const TG* __restrict__ F,
 template <typename TG>
 static int launch_df_t(const DfArgs& a, hipStream_t st) {
     if (a.chunk_len > 0 && a.chunk_len <= 1024) {
-        hipLaunchKernelGGL(dfchunk_kernel<TG>, dim3((a.S + a.chunk_len - 1) / a.chunk_len, a.BH), dim3(1024), 0, st, reinterpret_cast<const TG*>(a.F),
+        int threads = a.chunk_len;
+        if (a.anchor_part) threads = threads > a.D ? threads : a.D;
+        if (threads < a.anchor_parts) threads = a.anchor_parts;
+        hipLaunchKernelGGL(dfchunk_kernel<TG>, dim3((a.S + a.chunk_len - 1) / a.chunk_len, a.BH), dim3((threads + 63) / 64 * 64), 0, st, reinterpret_cast<const TG*>(a.F),
                            a.colsum, a.rowpart, a.rowinter, a.anchor, reinterpret_cast<TG*>(a.dF), reinterpret_cast<TG*>(a.dI), a.S, a.RS,
                            a.chunk_len, a.n_states, a.lg, a.gate_form, a.anchor_part, a.anchor_parts, a.anchor_va, a.anchor_vb, a.D, a.stamp);
         return (int)hipGetLastError();

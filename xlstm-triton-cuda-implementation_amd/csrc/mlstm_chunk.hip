@@ -375,85 +375,125 @@ __global__ __launch_bounds__(512) void chunk_sum_kernel(ChunkArgs a) {
 #endif
 }
 
-// The chunk sums for the shapes the MFMA kernel above does not serve (fp32 at D = 64 and 128, 16-bit types at D = 64): the
-// same sums as plain fp32 multiply-adds out of LDS tiles of 64 positions.  One workgroup per (head, chunk, 64 value
-// columns); a thread holds D/16 keys x 4 values.  These shapes are small (the sums are 2 S D^2 flops per head).
+// The chunk sums for the shapes the kernel above does not serve (fp32 at D = 64 and 128, 16-bit types at D = 64), as fp32
+// MFMA products with both operands straight from global memory: the positions are the inner dimension, so a lane's share of
+// an operand is one element of a row and a wave's load is a piece of two rows.  No tile passes through LDS and no wave waits
+// for another until the end.  One workgroup per (head, chunk, 32 value columns); a wave forms one 32 x 32 block (D = 128: four
+// key blocks; D = 64: two, each by two waves that take the chunk's tiles of 32 positions in turns and add up at the end).
+// What bounds it is one trip to memory and the products of a wave, 64 MFMAs of 64 cycles per 128 positions: the loads of two
+// tiles leave before the first product.
+// (Before: plain multiply-adds out of LDS tiles, 11.5 us at B1 H4 S2048 D64 fp32, 20.7 us at B2 H4 S4096 D64 bf16.)
 template <typename T, int D>
-__global__ __launch_bounds__(256) void chunk_sum_small_kernel(ChunkArgs a) {
-    constexpr int VW = 64, VH = D / VW, KPT = D / 16;
-    __shared__ __attribute__((aligned(16))) float ks[GRAN][D + 4];
-    __shared__ __attribute__((aligned(16))) float vs[GRAN][VW + 4];
-    __shared__ float sw2[GRAN];
-    const int tid = threadIdx.x;
-    const int vh = blockIdx.x % VH, pair = blockIdx.x / VH;
+__global__ __launch_bounds__(256, 2) void chunk_sum_small_kernel(ChunkArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    constexpr int VB = D / 32, KB = D / 32, PG = 4 / KB;   // PG: waves that share a key block
+    constexpr int TP = 32, NS = TP / 2;                     // positions per tile, MFMAs of two positions
+    __shared__ float sw[4][2][TP];                          // [wave][matrix, vector][position: even ones, then odd]
+    __shared__ float red[PG > 1 ? KB : 1][16][64];
+    __shared__ float redn[D];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5, c32 = lane & 31;
+    const int kb = wave % KB, pg = wave / KB;
+    const int vb = blockIdx.x % VB, pair = blockIdx.x / VB;
     const int cc = pair % a.NCS, bh = pair / a.NCS;
     const int S = a.S, L = a.L;
     const size_t poff = (size_t)bh * a.NG * GRAN, goff = (size_t)bh * a.NG;
     // (the positions and the reference point of a sum: see chunk_sum_kernel)
     const int p0 = (a.reverse ? cc + 1 : cc) * L, pe = a.reverse ? p0 - 1 : p0 + L - 1;
     const size_t rsK = (size_t)a.lk.ss, rsV = (size_t)a.lv.ss;
-    const T* Kh = reinterpret_cast<const T*>(a.K) + a.lk.head(bh);
-    const T* Vh = reinterpret_cast<const T*>(a.V) + a.lv.head(bh) + VW * vh;
+    const T* Kh = reinterpret_cast<const T*>(a.K) + a.lk.head(bh) + 32 * kb;
+    const T* Vh = reinterpret_cast<const T*>(a.V) + a.lv.head(bh) + 32 * vb;
     const float log2scale = -0.5f * __log2f((float)D);
     const float bend = a.beta2[poff + pe];
     const double Gend = a.G2[goff + pe / GRAN];
-    const int k0 = KPT * (tid >> 4), v0 = 4 * (tid & 15);
-    float acc[KPT][4];
+    const int n_pos = p0 + L <= S ? L : S - p0, n_tiles = (n_pos + TP - 1) / TP;
+
+    struct Tile { T k[NS], v[NS]; float x, x1, x2; double g; };
+    auto load = [&](Tile& t, int j) __attribute__((always_inline)) {   // step s: position 2 s + h of tile j
+        const int t0 = p0 + TP * j;
+        {   // what the weight of position t0 + c32 needs
+            const int pos = t0 + c32 < S ? t0 + c32 : S - 1;
+            t.g = a.G2[goff + pos / GRAN];
+            t.x = a.reverse ? a.beta2[poff + pos] : a.alpha2[poff + pos];
+            t.x1 = a.reverse ? a.inv_n[poff + pos] : 0.f;
+            t.x2 = a.reverse ? a.db[poff + pos] : 0.f;
+        }
+        if (t0 + TP <= S) {
+            const T* kt = Kh + (size_t)t0 * rsK;   // (the same for all lanes)
+            const T* vt = Vh + (size_t)t0 * rsV;
+            const unsigned ko = (unsigned)(h * rsK) + c32, vo = (unsigned)(h * rsV) + c32;
 #pragma unroll
-    for (int x = 0; x < KPT; x++)
+            for (int s = 0; s < NS; s++) { t.k[s] = (kt + (size_t)(2 * s) * rsK)[ko]; t.v[s] = (vt + (size_t)(2 * s) * rsV)[vo]; }
+        } else {
 #pragma unroll
-        for (int y = 0; y < 4; y++) acc[x][y] = 0.f;
+            for (int s = 0; s < NS; s++) {
+                const int pos = t0 + 2 * s + h < S ? t0 + 2 * s + h : S - 1;
+                t.k[s] = Kh[(size_t)pos * rsK + c32];
+                t.v[s] = Vh[(size_t)pos * rsV + c32];
+            }
+        }
+    };
+    f32x16 acc;
+#pragma unroll
+    for (int x = 0; x < 16; x++) acc[x] = 0.f;
     float nacc = 0.f;
-    const int n_pos = (p0 + L <= S ? L : S - p0);
-    for (int t0 = 0; t0 < n_pos; t0 += GRAN) {
-        __syncthreads();   // (the previous tile has been used)
-        // position tid / 4 of the tile, a quarter of its row each: K as it is, V times the position's weight
-        {
-            const int j = tid >> 2, part = tid & 3;
-            const int pos = p0 + t0 + j, pc = pos < S ? pos : S - 1;
-            float w = 0.f, w2 = 0.f;
-            if (pos < S) {
-                if (a.reverse) {
-                    const float rho = fast_exp2(bend - a.beta2[poff + pos] + (float)(a.G2[goff + pos / GRAN] - Gend) + log2scale);
-                    w = rho * a.inv_n[poff + pos];
-                    w2 = rho * a.db[poff + pos];
-                } else {
-                    w = w2 = fast_exp2(a.alpha2[poff + pos] - bend + (float)(Gend - a.G2[goff + pos / GRAN]) + log2scale);
-                }
+    auto work = [&](const Tile& t, int j) __attribute__((always_inline)) {
+        float w = 0.f, w2 = 0.f;
+        if (p0 + TP * j + c32 < S) {
+            if (a.reverse) {
+                const float rho = fast_exp2(bend - t.x + (float)(t.g - Gend) + log2scale);
+                w = rho * t.x1;
+                w2 = rho * t.x2;
+            } else {
+                w = w2 = fast_exp2(t.x - bend + (float)(Gend - t.g) + log2scale);
             }
-            if (part == 0) sw2[j] = w2;
-            const T* kr = Kh + (size_t)pc * rsK + (D / 4) * part;
-            const T* vr = Vh + (size_t)pc * rsV + (VW / 4) * part;
-#pragma unroll
-            for (int e = 0; e < D / 4; e++) ks[j][(D / 4) * part + e] = (float)kr[e];
-#pragma unroll
-            for (int e = 0; e < VW / 4; e++) vs[j][(VW / 4) * part + e] = (float)vr[e] * w;
         }
-        __syncthreads();
-#pragma unroll 4
-        for (int j = 0; j < GRAN; j++) {
-            const f32x4 vv = *reinterpret_cast<const f32x4*>(&vs[j][v0]);
-            float kk[KPT];
+        // (the wave's own part of LDS: no barrier)
+        if (h == 0) {
+            sw[wave][0][(c32 & 1) * NS + (c32 >> 1)] = w;
+            sw[wave][1][(c32 & 1) * NS + (c32 >> 1)] = w2;
+        }
+        __builtin_amdgcn_wave_barrier();
 #pragma unroll
-            for (int x = 0; x < KPT; x += 4) {
-                const f32x4 q4 = *reinterpret_cast<const f32x4*>(&ks[j][k0 + x]);
-                kk[x] = q4[0]; kk[x + 1] = q4[1]; kk[x + 2] = q4[2]; kk[x + 3] = q4[3];
+        for (int s4 = 0; s4 < NS; s4 += 4) {
+            const f32x4 wv = *reinterpret_cast<const f32x4*>(&sw[wave][0][h * NS + s4]), wn = *reinterpret_cast<const f32x4*>(&sw[wave][1][h * NS + s4]);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                const float kv = (float)t.k[s4 + e];
+                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(kv, (float)t.v[s4 + e] * wv[e], acc, 0, 0, 0);
+                nacc += kv * wn[e];
             }
-#pragma unroll
-            for (int x = 0; x < KPT; x++)
-#pragma unroll
-                for (int y = 0; y < 4; y++) acc[x][y] += kk[x] * vv[y];
         }
-        if (vh == 0 && tid < D) {
-#pragma unroll 8
-            for (int j = 0; j < GRAN; j++) nacc += ks[j][tid] * sw2[j];
+        __builtin_amdgcn_wave_barrier();
+    };
+    Tile ta, tb;
+    int j = pg;
+    if (j < n_tiles) load(ta, j);
+    for (; j < n_tiles; j += 2 * PG) {
+        if (j + PG < n_tiles) load(tb, j + PG);
+        work(ta, j);
+        if (j + PG < n_tiles) {
+            if (j + 2 * PG < n_tiles) load(ta, j + 2 * PG);
+            work(tb, j + PG);
         }
     }
-    float* out = a.dC + ((size_t)bh * a.NCS + cc) * D * D + VW * vh;
+    nacc = sum_halves(nacc);
+    if constexpr (PG > 1) {
+        if (pg == 1) {
 #pragma unroll
-    for (int x = 0; x < KPT; x++)
-        *reinterpret_cast<f32x4*>(out + (size_t)(k0 + x) * D + v0) = f32x4{acc[x][0], acc[x][1], acc[x][2], acc[x][3]};
-    if (vh == 0 && tid < D) a.Nst[((size_t)bh * a.NCS + cc) * D + tid] = nacc;
+            for (int x = 0; x < 16; x++) red[kb][x][lane] = acc[x];
+            if (h == 0) redn[32 * kb + c32] = nacc;
+        }
+        __syncthreads();
+        if (pg == 1) return;
+#pragma unroll
+        for (int x = 0; x < 16; x++) acc[x] += red[kb][x][lane];
+        nacc += redn[32 * kb + c32];
+    }
+    float* out = a.dC + ((size_t)bh * a.NCS + cc) * D * D + (size_t)(32 * kb) * D + 32 * vb + c32;
+#pragma unroll
+    for (int r = 0; r < 16; r++) out[(size_t)(8 * (r >> 2) + 4 * h + (r & 3)) * D] = acc[r];
+    if (vb == 0 && h == 0) a.Nst[((size_t)bh * a.NCS + cc) * D + 32 * kb + c32] = nacc;
+#endif
 }
 
 // gamma_c = exp(A_{e_{c-1}} - A_{e_c}), e_c the last position of chunk c (c >= 1, both chunks complete): what the state
@@ -539,6 +579,106 @@ __global__ __launch_bounds__(256) void chunk_carry_kernel(ChunkArgs a) {
             nst[(size_t)c * D] = nrun;
         }
       }
+    }
+}
+
+// The carry of the shapes of chunk_sum_small_kernel: a workgroup takes 32 keys x 32 values of a head's state, sixteen chunks'
+// sums at a time in registers (one trip to memory per sixteen steps, whatever the number of heads), writes either layout or
+// both -- the value-major one through LDS, in whole 64- or 128-byte pieces of a row -- and forms the contraction with another
+// set of states (ChunkArgs::dot_with) on the way.
+// (Before: 2 to 8 workgroups per head, four steps at a time, the value-major copy element by element, and a kernel of its own
+// for the contraction: 14.6 + 4.7 us at B1 H4 S2048 D64 fp32.)
+template <typename T, int D, bool DOT>
+__global__ __launch_bounds__(256) void chunk_carry_small_kernel(ChunkArgs a) {
+    constexpr int AHEAD = 16, MAXC = 1024;   // (S <= 131072 in chunks of at least 128)
+    typedef typename Tr<T>::vec4 V4;
+    __shared__ __attribute__((aligned(16))) float tile[2][32][36];
+    __shared__ float gams[MAXC];
+    __shared__ float red[2][4];
+    const int bh = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int kb = blockIdx.x / (D / 32), vb = blockIdx.x % (D / 32);
+    const int row = tid >> 3, c4 = 4 * (tid & 7);   // row of the block (key; value in the turned one) and first of four columns
+    const size_t poff = (size_t)bh * a.NG * GRAN, goff = (size_t)bh * a.NG, hbase = (size_t)bh * a.NCS * D * D;
+    const float* src = a.dC + hbase + (size_t)(32 * kb + row) * D + 32 * vb + c4;
+    const size_t koff = hbase + (size_t)state_row<T>(32 * kb + row) * D + 32 * vb + c4;   // key-major
+    const size_t voff = hbase + (size_t)state_row<T>(32 * vb + row) * D + 32 * kb + c4;   // value-major
+    float* nst = a.Nst + (size_t)bh * a.NCS * D + tid;
+    const bool vec = blockIdx.x == 0 && tid < D;
+    auto chunk_of = [&](int step) { return a.reverse ? a.NCS - 1 - step : step; };
+    f32x4 d[AHEAD];
+    V4 y[DOT ? AHEAD : 1], yl[DOT ? AHEAD : 1];
+    float nin[AHEAD];
+    auto request = [&](int step0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) {
+            const int c = chunk_of(step0 + u < a.NCS ? step0 + u : a.NCS - 1);
+            const size_t co = (size_t)c * D * D;
+            d[u] = *reinterpret_cast<const f32x4*>(src + co);
+            if constexpr (DOT) {
+                y[u] = *reinterpret_cast<const V4*>(reinterpret_cast<const T*>(a.dot_with) + voff + co);
+                if (a.dot_with_lo) yl[u] = *reinterpret_cast<const V4*>(reinterpret_cast<const T*>(a.dot_with_lo) + voff + co);
+            }
+            nin[u] = vec ? nst[(size_t)c * D] : 0.f;
+        }
+    };
+    request(0);
+    for (int step = tid; step < a.NCS; step += 256)
+        gams[step] = step > 0 ? carry_gamma(a, poff, goff, a.reverse ? chunk_of(step) + 1 : chunk_of(step)) : 0.f;
+    __syncthreads();
+    const bool split = a.Cst_lo || a.CstT_lo;
+    f32x4 run = {0.f, 0.f, 0.f, 0.f};
+    float nrun = 0.f;
+    auto put = [&](void* hi_base, void* lo_base, size_t off, f32x4 x, V4& hi, V4& lo) __attribute__((always_inline)) {
+        if (split) Tr<T>::cvt4_split(x, hi, lo);
+        else hi = Tr<T>::cvt4(x);
+        if (hi_base) *reinterpret_cast<V4*>(reinterpret_cast<T*>(hi_base) + off) = hi;
+        if (lo_base) *reinterpret_cast<V4*>(reinterpret_cast<T*>(lo_base) + off) = lo;
+    };
+    auto put_dot = [&](int step) {   // (behind the barrier that follows the step's partial sums)
+        if (DOT && tid == 0)
+            a.dot_part[((size_t)bh * a.NCS + chunk_of(step)) * gridDim.x + blockIdx.x] =
+                (red[step & 1][0] + red[step & 1][1]) + (red[step & 1][2] + red[step & 1][3]);
+    };
+    for (int step0 = 0; step0 < a.NCS; step0 += AHEAD) {
+        if (step0 > 0) request(step0);
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) {
+            const int step = step0 + u;
+            if (step < a.NCS) {
+            const size_t co = (size_t)chunk_of(step) * D * D;
+            const float gam = gams[step];
+            run = run * gam + d[u];
+#pragma unroll
+            for (int e = 0; e < 4; e++) asm volatile("" : "+v"(run[e]));   // (see chunk_carry_t_kernel)
+            V4 hi, lo;
+            if (a.Cst) put(a.Cst, a.Cst_lo, koff + co, run, hi, lo);
+            if (a.CstT) {   // (uniform) turned round in LDS
+                float (*t)[36] = tile[step & 1];
+#pragma unroll
+                for (int e = 0; e < 4; e++) t[c4 + e][row] = run[e];
+                __syncthreads();
+                if (step > 0) put_dot(step - 1);
+                const f32x4 x = *reinterpret_cast<const f32x4*>(&t[row][c4]);
+                put(a.CstT, a.CstT_lo, voff + co, x, hi, lo);
+                if constexpr (DOT) {   // the state as it is written (the sum of its terms in split mode)
+                    f32x4 xs = __builtin_convertvector(hi, f32x4), ys = __builtin_convertvector(y[u], f32x4);
+                    if (split) xs += __builtin_convertvector(lo, f32x4);
+                    if (a.dot_with_lo) ys += __builtin_convertvector(yl[u], f32x4);
+                    const f32x4 pr = xs * ys;
+                    const float dot = wave_reduce<OpAdd>((pr[0] + pr[1]) + (pr[2] + pr[3]));
+                    if (lane == 0) red[step & 1][wave] = dot;
+                }
+            }
+            if (vec) {
+                nrun = nrun * gam + nin[u];
+                nst[(size_t)chunk_of(step) * D] = nrun;
+            }
+            }
+        }
+    }
+    if constexpr (DOT) {
+        __syncthreads();
+        put_dot(a.NCS - 1);
     }
 }
 
@@ -1048,14 +1188,17 @@ static int launch_chunk_t(const ChunkArgs& a, hipStream_t st) {
     return (int)hipGetLastError();
 }
 
-// the small shapes: plain multiply-adds for the sums, one element-wise carry for both layouts
+// the small shapes: sums straight from memory, one carry for both layouts and the contraction
 template <typename T, int D>
 static int launch_chunk_small(const ChunkArgs& a, hipStream_t st) {
     if (a.precise && ((a.Cst && !a.Cst_lo) || (a.CstT && !a.CstT_lo))) return MLSTM_EINVAL;
     if (!a.precise && (a.Cst_lo || a.CstT_lo)) return MLSTM_EINVAL;
-    if (a.dot_part) return MLSTM_EINVAL;   // (launch_anchor serves these shapes)
-    hipLaunchKernelGGL((chunk_sum_small_kernel<T, D>), dim3(a.BH * a.NCS * (D / 64)), dim3(256), 0, st, a);
-    hipLaunchKernelGGL((chunk_carry_kernel<T, D>), dim3(D * D / 8 / 256, a.BH), dim3(256), 0, st, a);
+    if (a.dot_part && !(a.CstT && a.dot_with)) return MLSTM_EINVAL;
+    if (a.NCS > 1024) return MLSTM_ESHAPE;
+    hipLaunchKernelGGL((chunk_sum_small_kernel<T, D>), dim3(a.BH * a.NCS * (D / 32)), dim3(256), 0, st, a);
+    const dim3 cgrid((D / 32) * (D / 32), a.BH);
+    if (a.dot_part) hipLaunchKernelGGL((chunk_carry_small_kernel<T, D, true>), cgrid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((chunk_carry_small_kernel<T, D, false>), cgrid, dim3(256), 0, st, a);
     return (int)hipGetLastError();
 }
 
@@ -1123,9 +1266,8 @@ int launch_chunk_states(int dtype, int D, const ChunkArgs& a, hipStream_t st) {
     return MLSTM_ESHAPE;
 }
 
-bool chunk_states_fused_dot(int dtype, int D) { return dtype != MLSTM_F32 && (D == 128 || D == 256); }
-
 int chunk_states_dot_parts(int dtype, int D, const ChunkArgs& a) {
+    if (dtype == MLSTM_F32 || D == 64) return (D / 32) * (D / 32);
     bool seq = false;
     if (dtype == MLSTM_BF16 && D == 128) seq = chunk_seq_serves<__bf16, 128>(a);
     if (dtype == MLSTM_BF16 && D == 256) seq = chunk_seq_serves<__bf16, 256>(a);

@@ -225,14 +225,12 @@ struct ChunkArgs {
     void* CstT_lo;
     // The value-major carry can contract the states it forms (before rounding) with another set in the same layout
     // (dot_with, dot_with_lo: its low-order terms or null): dot_part[bh][c][workgroup of the head] receives the partial
-    // sums of <state_c, dot_with_c>, (D / 64)^2 per state.
+    // sums of <state_c, dot_with_c>, chunk_states_dot_parts() per state.
     const void* dot_with = nullptr;
     const void* dot_with_lo = nullptr;
     float* dot_part = nullptr;
 };
 int launch_chunk_states(int dtype, int D, const ChunkArgs& a, hipStream_t st);
-// whether the carry of these shapes takes ChunkArgs::dot_part (otherwise launch_anchor forms the contraction)
-bool chunk_states_fused_dot(int dtype, int D);
 // partial sums per state that the launch with these arguments leaves in ChunkArgs::dot_part
 int chunk_states_dot_parts(int dtype, int D, const ChunkArgs& a);
 // test and measurement aid: 0 = the library's choice by the size of the launch, 1 = chunk sums and carry (two kernels),

@@ -1,4 +1,5 @@
-// Scan (recurrent, chunked) form of the mLSTM forward with the silu(o) output gate, fp32.
+// Scan (recurrent, chunked) form of the mLSTM forward with the silu(o) output gate, fp32, D >= 256 (the tile kernels serve
+// the smaller head dimensions).
 // Replaces stabilize_fi / precompute_mlstm_triton_scan / reduce_mlstm_triton / mlstm_triton_scan
 // (mlstm_scan.py:48-278) and their host driver mlstm_scan (mlstm_scan.py:281-327).
 //
@@ -567,23 +568,22 @@ static void launch_state(const ScanArgs& a, hipStream_t st) {
 }
 
 template <int D, int KS>
-static void launch_state_w(const ScanArgs& a, int NW, hipStream_t st) {
-    (void)NW;  // scan_plan: two waves per workgroup at D = 64, four above
-    if (a.rev) launch_state<D, KS, (D / 32 < 4 ? D / 32 : 4), true>(a, st);
-    else launch_state<D, KS, (D / 32 < 4 ? D / 32 : 4), false>(a, st);
+static void launch_state_w(const ScanArgs& a, hipStream_t st) {
+    if (a.rev) launch_state<D, KS, 4, true>(a, st);
+    else launch_state<D, KS, 4, false>(a, st);
 }
 
 template <int D>
-static int launch_scan_d(const ScanArgs& a, int KS, int NW, hipStream_t st, void (*mark)(int, hipStream_t, bool)) {
+static int launch_scan_d(const ScanArgs& a, int KS, hipStream_t st, void (*mark)(int, hipStream_t, bool)) {
     mark(MLSTM_K_SCAN_CARRY, st, true);
     hipLaunchKernelGGL(scan_intra_kernel<D>, dim3(a.BH * a.NC * 4), dim3(256), 0, st, a);
     if (a.finish_mode != 2 || a.ep.vec) hipLaunchKernelGGL(scan_ncarry_kernel, dim3((D + 255) / 256, a.BH), dim3(256), 0, st, a);
     mark(MLSTM_K_SCAN_CARRY, st, false);
     mark(MLSTM_K_SCAN_STATE, st, true);
-    if (KS == 8) launch_state_w<D, 8>(a, NW, st);
-    else if (KS == 4) launch_state_w<D, 4>(a, NW, st);
-    else if (KS == 2) launch_state_w<D, 2>(a, NW, st);
-    else launch_state_w<D, 1>(a, NW, st);
+    if (KS == 8) launch_state_w<D, 8>(a, st);
+    else if (KS == 4) launch_state_w<D, 4>(a, st);
+    else if (KS == 2) launch_state_w<D, 2>(a, st);
+    else launch_state_w<D, 1>(a, st);
     mark(MLSTM_K_SCAN_STATE, st, false);
     mark(MLSTM_K_SCAN_OUT, st, true);
     const size_t rows = (size_t)a.BH * a.S;
@@ -597,14 +597,13 @@ void launch_scan_ncarry(const ScanArgs& a, hipStream_t st) {
     hipLaunchKernelGGL(scan_ncarry_kernel, dim3((a.D + 255) / 256, a.BH), dim3(256), 0, st, a);
 }
 
-// Key ranges per value tile and waves per workgroup.
-void scan_plan(int BH, int D, int* KS, int* NW) {
-    const int nw = D / 32 < 4 ? D / 32 : 4;    // waves per workgroup: one per SIMD (each wants the full register file)
+// Key ranges per value tile.
+int scan_key_splits(int BH, int D) {
+    const int nw = 4;                          // waves per workgroup: one per SIMD (each wants the full register file)
     int ks = D / nw > 128 ? D / nw / 128 : 1;  // at most 128 key columns per wave
     while (D / ks / nw > 32 && BH * (D / 32) * ks < 256) ks *= 2;  // at least one workgroup per CU where D allows
-    *KS = ks; *NW = nw;
+    return ks;
 }
-int scan_key_splits(int BH, int D) { int ks, nw; scan_plan(BH, D, &ks, &nw); return ks; }
 
 // Segments of a sequence that run side by side: none while heads x value tiles x key ranges fill the chip; otherwise
 // enough for about two workgroups per CU, of at least eight chunks each.
@@ -634,16 +633,12 @@ int launch_scan(const ScanArgs& a_in, int KS, hipStream_t st, void (*mark)(int, 
                                (a.ep.dot_with && !a.ep.dot_out) || (a.ep.x_out && !(a.ep.dot_with && a.ep.dot_minus)) ||
                                (!a.ep.wd_alpha2 != !a.ep.wd_beta2)))
         return MLSTM_EINVAL;
-    int ks, NW; scan_plan(a.BH, a.D, &ks, &NW);
-    if (NW != (a.D / 32 < 4 ? a.D / 32 : 4)) return MLSTM_ESHAPE;
-    const int kpw = a.D / KS / NW;
-    if (kpw * KS * NW != a.D || (kpw != 32 && kpw != 64 && kpw != 128) || NW > 8 || NW * KS > 32) return MLSTM_ESHAPE;
+    const int kpw = a.D / KS / 4;
+    if (kpw * KS * 4 != a.D || (kpw != 32 && kpw != 64 && kpw != 128) || 4 * KS > 32) return MLSTM_ESHAPE;
     switch (a.D) {
-        case 64: return launch_scan_d<64>(a, KS, NW, st, mark);
-        case 128: return launch_scan_d<128>(a, KS, NW, st, mark);
-        case 256: return launch_scan_d<256>(a, KS, NW, st, mark);
-        case 512: return launch_scan_d<512>(a, KS, NW, st, mark);
-        case 1024: return launch_scan_d<1024>(a, KS, NW, st, mark);
+        case 256: return launch_scan_d<256>(a, KS, st, mark);
+        case 512: return launch_scan_d<512>(a, KS, st, mark);
+        case 1024: return launch_scan_d<1024>(a, KS, st, mark);
     }
     return MLSTM_ESHAPE;
 }
