@@ -27,9 +27,7 @@ namespace mlstm {
 // tile hands it rows 16 s + 4 h + e (e < 4) and 16 s + 8 + 4 h + e - 4 (e >= 4).  Tile row u (mod 16) therefore holds
 // state row PERM16(u): the two middle groups of four swap places.
 __device__ __forceinline__ int perm16(int u) { return (u & ~12) | ((u & 4) << 1) | ((u & 8) >> 1); }
-// (fp32 tiles are read one element per lane, in the natural order)
-template <typename T>
-__device__ __forceinline__ int state_row(int u) { return sizeof(T) == 2 ? ((u & ~15) | perm16(u & 15)) : u; }
+__device__ __forceinline__ int state_row(int u) { return (u & ~15) | perm16(u & 15); }
 
 // STRICT: split mode, the weighted V rows go to LDS as two tiles, hi and lo (ChunkArgs::precise)
 template <typename T, int D, bool STRICT = false>
@@ -62,11 +60,6 @@ __device__ __forceinline__ void unpack8(const u32x4& d, float (&x)[8]) {
         for (int e = 0; e < 8; e++) x[e] = (float)v[e];
     }
 }
-
-template <int... I, typename F>
-__device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F&& f) { (f(std::integral_constant<int, I>{}), ...); }
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) { static_for_impl(std::make_integer_sequence<int, N>{}, f); }
 
 // NTT: tiles per chunk as a compile-time constant (the tile loop is then straight-line code), or 0 for any chunk length
 template <typename T, int D, int NTT, bool STRICT>
@@ -513,7 +506,7 @@ __global__ __launch_bounds__(256) void chunk_carry_kernel(ChunkArgs a) {
     const int L = a.L;
     const size_t hbase = (size_t)bh * a.NCS * D * D;
     const float* src = a.dC + hbase + (size_t)k * D + v8;
-    const size_t koff = hbase + (size_t)state_row<T>(k) * D + v8;   // key-major: eight values of key k
+    const size_t koff = hbase + (size_t)state_row(k) * D + v8;   // key-major: eight values of key k
     float* nst = a.Nst + (size_t)bh * a.NCS * D + tid;
     const bool vec = blockIdx.x == 0 && tid < D;
     f32x4 run0 = {0.f, 0.f, 0.f, 0.f}, run1 = {0.f, 0.f, 0.f, 0.f};
@@ -569,7 +562,7 @@ __global__ __launch_bounds__(256) void chunk_carry_kernel(ChunkArgs a) {
             T* tl = a.CstT_lo ? reinterpret_cast<T*>(a.CstT_lo) + hbase + (size_t)c * D * D + k : nullptr;
 #pragma unroll
             for (int e = 0; e < 8; e++) {
-                const size_t r = (size_t)state_row<T>(v8 + e) * D;
+                const size_t r = (size_t)state_row(v8 + e) * D;
                 t[r] = e < 4 ? o.lo[e & 3] : o.hi[e & 3];
                 if (tl) tl[r] = e < 4 ? rest.lo[e & 3] : rest.hi[e & 3];
             }
@@ -600,8 +593,8 @@ __global__ __launch_bounds__(256) void chunk_carry_small_kernel(ChunkArgs a) {
     const int row = tid >> 3, c4 = 4 * (tid & 7);   // row of the block (key; value in the turned one) and first of four columns
     const size_t poff = (size_t)bh * a.NG * GRAN, goff = (size_t)bh * a.NG, hbase = (size_t)bh * a.NCS * D * D;
     const float* src = a.dC + hbase + (size_t)(32 * kb + row) * D + 32 * vb + c4;
-    const size_t koff = hbase + (size_t)state_row<T>(32 * kb + row) * D + 32 * vb + c4;   // key-major
-    const size_t voff = hbase + (size_t)state_row<T>(32 * vb + row) * D + 32 * kb + c4;   // value-major
+    const size_t koff = hbase + (size_t)state_row(32 * kb + row) * D + 32 * vb + c4;   // key-major
+    const size_t voff = hbase + (size_t)state_row(32 * vb + row) * D + 32 * kb + c4;   // value-major
     float* nst = a.Nst + (size_t)bh * a.NCS * D + tid;
     const bool vec = blockIdx.x == 0 && tid < D;
     auto chunk_of = [&](int step) { return a.reverse ? a.NCS - 1 - step : step; };
@@ -1072,7 +1065,7 @@ __global__ __launch_bounds__(512) void chunk_seq_kernel(ChunkArgs a) {
 #pragma unroll
                 for (int nb = 0; nb < NB; nb++) {
                     const int vg = VW * vh + 32 * (NB * wv + nb) + c32;
-                    const size_t vrow_off = sbase + (size_t)state_row<T>(vg) * D;
+                    const size_t vrow_off = sbase + (size_t)state_row(vg) * D;
 #pragma unroll
                     for (int g4 = 0; g4 < 4; g4++) {
                         const int kg = 64 * kq + 32 * wk + 8 * g4 + 4 * h;
@@ -1080,7 +1073,7 @@ __global__ __launch_bounds__(512) void chunk_seq_kernel(ChunkArgs a) {
                         if (a.CstT) *reinterpret_cast<typename R::vec4*>(reinterpret_cast<T*>(a.CstT) + vrow_off + kg) = hi;
                         if (a.Cst) {
 #pragma unroll
-                            for (int e = 0; e < 4; e++) reinterpret_cast<T*>(a.Cst)[sbase + (size_t)state_row<T>(kg + e) * D + vg] = hi[e];
+                            for (int e = 0; e < 4; e++) reinterpret_cast<T*>(a.Cst)[sbase + (size_t)state_row(kg + e) * D + vg] = hi[e];
                         }
                         if constexpr (DOT) {
                             const f32x4 o = __builtin_convertvector(*reinterpret_cast<const typename R::vec4*>(reinterpret_cast<const T*>(a.dot_with) + vrow_off + kg), f32x4);

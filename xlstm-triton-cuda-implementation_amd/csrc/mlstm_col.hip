@@ -27,15 +27,18 @@ namespace mlstm {
 
 template <typename T, int D, bool STRICT = false>
 struct ColCfg {
-    // G / W tiles [query][key], written by lanes in phase A and read transposed in phase B.  16-bit: 128-byte rows,
-    // 16-byte chunk c of row q stored at chunk c ^ gkey(q); fp32: rows padded by 8 floats.
-    static constexpr int LDG = Tr<T>::HALF ? GRAN : GRAN + 8;
+    // G / W tiles [query][key] of 16-bit elements, written by lanes in phase A and read transposed in phase B: 128-byte rows,
+    // 16-byte chunk c of row q stored at chunk c ^ gkey(q).  fp32: three tiles each, the terms (Tr<float>) that the products
+    // of phase B take: every weight is split once, by the lane that forms it, not by each of the waves that read it.
+    typedef typename std::conditional<Tr<T>::HALF, T, __bf16>::type TG;
+    static constexpr int LDG = GRAN;
     static constexpr size_t TILE_ELEMS = (size_t)GRAN * D;
     static constexpr size_t STAGE_BYTES = 2 * TILE_ELEMS * sizeof(T) + 3 * GRAN * sizeof(float);  // Q, dH, (beta, 1/n, db)
-    static constexpr size_t G_BYTES = (size_t)GRAN * LDG * sizeof(T);
+    static constexpr size_t G_BYTES = (size_t)GRAN * LDG * sizeof(TG);
     // G, W (split mode: and their low-order terms), row-sum scratch.  With the two extra tiles the 16-bit D = 256 case
     // no longer fits two query stages and runs single-staged.
-    static constexpr size_t GW_BYTES = (STRICT ? 4 : 2) * G_BYTES;
+    static constexpr int PLANES = !Tr<T>::HALF ? 3 : (STRICT ? 2 : 1);
+    static constexpr size_t GW_BYTES = 2 * PLANES * G_BYTES;
     static constexpr size_t FIXED_BYTES = GW_BYTES + 6 * GRAN * sizeof(float);   // + row sums [2][64], far column sums [4][64]
     static constexpr int STAGES = (2 * STAGE_BYTES + FIXED_BYTES + 2048 * sizeof(float) <= 160 * 1024) ? 2 : 1;
     static constexpr size_t LDS_BYTES = STAGES * STAGE_BYTES + FIXED_BYTES;  // plus one float per key tile, appended at launch
@@ -70,11 +73,14 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
 #define ST_Q(st) (reinterpret_cast<T*>(smem + (st) * Cfg::STAGE_BYTES))
 #define ST_DH(st) (ST_Q(st) + Cfg::TILE_ELEMS)
 #define ST_ROW(st) (reinterpret_cast<float*>(ST_DH(st) + Cfg::TILE_ELEMS))
-    T* const Gs = reinterpret_cast<T*>(smem + STAGES * Cfg::STAGE_BYTES);
-    T* const Ws = Gs + GRAN * LDG;
-    T* const Gl = Ws + GRAN * LDG;                                    // split mode: low-order terms of G and W
-    T* const Wl = Gl + GRAN * LDG;
-    float* const rowtmp = reinterpret_cast<float*>(Gs + (STRICT ? 4 : 2) * GRAN * LDG);  // [2][64]
+    typedef typename Cfg::TG TG;
+    TG* const Gs = reinterpret_cast<TG*>(smem + STAGES * Cfg::STAGE_BYTES);
+    TG* const Ws = Gs + GRAN * LDG;
+    TG* const Gl = Ws + GRAN * LDG;                                   // split mode: low-order terms of G and W (fp32: the middle ones)
+    TG* const Wl = Gl + GRAN * LDG;
+    TG* const Gz = Wl + GRAN * LDG;                                   // fp32: the last terms
+    TG* const Wz = Gz + GRAN * LDG;
+    float* const rowtmp = reinterpret_cast<float*>(Gs + 2 * Cfg::PLANES * GRAN * LDG);  // [2][64]
     float* const cpart = rowtmp + 2 * GRAN;                                               // [4][64]
     // granule bases minus this key tile's (see row kernel)
     float* const sG = reinterpret_cast<float*>(smem + Cfg::LDS_BYTES + (a.chunk_len > 0 ? Cfg::EXTRA_CHUNK_BYTES : 0));
@@ -129,7 +135,7 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
     const int NGe = a.chunk_len > 0 ? ((chunk + 1) * tpc < NG ? (chunk + 1) * tpc : NG) : NG;
     const bool has_state = a.chunk_len > 0 && chunk < a.n_states;   // (uniform over the workgroup)
     constexpr int NTL = D / GRAN;   // 64-row tiles of a state
-    T* const Kt = STAGES == 2 ? ST_Q(1) : Gs;
+    T* const Kt = STAGES == 2 ? ST_Q(1) : reinterpret_cast<T*>(Gs);
     T* const Vt = STAGES == 2 ? ST_DH(1) : reinterpret_cast<T*>(smem + Cfg::LDS_BYTES);
     const size_t sbase = has_state ? ((size_t)bh * a.n_states + chunk) * D * D : 0;
     const T* const Evc = reinterpret_cast<const T*>(a.Ev) + sbase;
@@ -169,6 +175,9 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
     for (int r = 0; r < 16; r++) al[r] = a.alpha2[poff + kstartA + 8 * (r >> 2) + 4 * h + (r & 3)];
 #pragma unroll
     for (int s = 0; s < NS; s++) { pin(kf[s]); pin(vf[s]); }
+    typename R::terms kt[NS], vt[NS];
+#pragma unroll
+    for (int s = 0; s < NS; s++) { kt[s] = R::split(kf[s]); vt[s] = R::split(vf[s]); }
     // factorised weights for the steps below the diagonal: ekr[r] = exp2(alpha_key(r) - c0), c0 the block maximum
     float ekr[16], amaxA;
     {
@@ -200,8 +209,9 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
     constexpr bool FAST_TR = R::HALF && Swz<T, D>::CPR >= 16;
     SwzRowReader<T, D> qrd;
     qrd.init(lane);
-    SwzTransReader<typename std::conditional<FAST_TR, T, __bf16>::type, FAST_TR ? D : 256> trd;
-    if constexpr (FAST_TR) trd.init(lane, BOTH_KB ? wave * NXW : 0);
+    constexpr bool F32 = !R::HALF;
+    typename std::conditional<F32, SwzTransReaderF32<D>, SwzTransReader<typename std::conditional<FAST_TR, T, __bf16>::type, FAST_TR ? D : 256>>::type trd;
+    if constexpr (FAST_TR || F32) trd.init(lane, BOTH_KB ? wave * NXW : 0);
 
     // ---- state phase (sequences in chunks)
     // (k_j . dK_j of the state part, the far column sums, stay in cpart[0..63] until the end of the kernel)
@@ -215,7 +225,7 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
         for (int kb = 0; kb < NKB; kb++) wk[kb] = fast_exp2(a.alpha2[poff + GRAN * jt + 32 * (BOTH_KB ? kb : kbB) + c32] - bend + (float)dG);
         auto col_block = [&](int x) { return BOTH_KB ? wave * NXW + x : dsel + 2 * x; };
         auto rd_tr = [&](const T* tile, int tt, int x) {
-            if constexpr (FAST_TR) return trd.read(tile, KW * tt, BOTH_KB ? x : col_block(x));
+            if constexpr (FAST_TR || F32) return trd.read(tile, KW * tt, BOTH_KB ? x : col_block(x));
             else return swz_frag_transposed<T, D>(tile, KW * tt, 32 * col_block(x), lane);
         };
 #pragma unroll
@@ -250,8 +260,8 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
                 const int r0v = 32 * col_block(x);
                 if (r0v / GRAN != tau) continue;
                 const int rl = r0v % GRAN + c32;
-                // (16-bit states keep their rows in the contraction order of the transposing reads, see mlstm_chunk.hip)
-                const int own = R::HALF ? ((rl & ~15) | ((rl & 3) | ((rl & 4) << 1) | ((rl & 8) >> 1))) : rl;
+                // (the states keep their rows in the contraction order of the transposing reads, see mlstm_chunk.hip)
+                const int own = (rl & ~15) | ((rl & 3) | ((rl & 4) << 1) | ((rl & 8) >> 1));
 #pragma unroll
                 for (int t = 0; t < NS; t++) {
                     frag kB[NKB];
@@ -319,11 +329,12 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
                 gwoff[kb][x] = q * GRAN + ((c ^ gkey(q)) << 3) + 4 * (j & 1);
             }
     }
-    auto gw_read = [&](const T* tile, int t, int kb) {
+    typedef typename Tr<TG>::frag gfrag;
+    auto gw_read = [&](const TG* tile, int t, int kb) {
         s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_PTR(s16x4))(tile + gwoff[kb][0] + 16 * t * GRAN));
         s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_PTR(s16x4))(tile + gwoff[kb][1] + 16 * t * GRAN));
         s16x8 both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
-        return __builtin_bit_cast(frag, both);
+        return __builtin_bit_cast(gfrag, both);
     };
 
     // One step = one 64-query tile.  FIRST (the diagonal tile, it == jt) carries the causal masks and the skipped
@@ -365,6 +376,16 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
             // The operand reads run AHEAD fragments in front of the MFMAs that consume them (a wave issues in order:
             // without the explicit interleave the reads of a batch and its MFMAs would take turns).
             constexpr int AHEAD = NS < 4 ? NS : 4;
+            if constexpr (F32) {
+                sacc = f32x16{}; dacc = f32x16{};
+                R::template stream<2 * NS>([&](auto n) { return n & 1 ? qrd.read(dHs, qbA, n >> 1) : qrd.read(Qs, qbA, n >> 1); },
+                                           [&](auto n, const auto& f, auto&& between) {
+                                               if constexpr (SPREAD && STAGES == 2) {
+                                                   if (n % 4 == 0) tdma.issue_range(lq, gq, (n / 4) * PW / (NS / 2), (n / 4 + 1) * PW / (NS / 2), ra);
+                                               }
+                                               R::mma_between(n & 1 ? dacc : sacc, n & 1 ? vt[n >> 1] : kt[n >> 1], f, between);
+                                           });
+            } else {
             frag qf[NS], hf[NS];
 #pragma unroll
             for (int s = 0; s < AHEAD; s++) { qf[s] = qrd.read(Qs, qbA, s); hf[s] = qrd.read(dHs, qbA, s); }
@@ -378,9 +399,10 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
                     const f32x16 z = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
                     sacc = z; dacc = z;
                 }
-                R::mma(sacc, kf[s], qf[s]);
-                R::mma(dacc, vf[s], hf[s]);
+                R::mma(sacc, kt[s], qf[s]);
+                R::mma(dacc, vt[s], hf[s]);
                 __builtin_amdgcn_sched_barrier(0);
+            }
             }
             const float crow = log2scale - srow[32 * qbA + c32] + sG[it];
             const float inv = srow[GRAN + 32 * qbA + c32], dbv = srow[2 * GRAN + 32 * qbA + c32];
@@ -420,20 +442,24 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
                 f32x4 gv, wv;
 #pragma unroll
                 for (int c = 0; c < 4; c++) { gv[c] = g[4 * a4 + c]; wv[c] = w[4 * a4 + c]; }
-                int off;  // element offset of keys 32*kbA + 8*a4 + 4*h .. +3 of row 32*qbA + c32
-                if constexpr (R::HALF) off = (32 * qbA + c32) * GRAN + (((4 * kbA + a4) ^ gkey(c32)) << 3) + 4 * h;
-                else off = (32 * qbA + c32) * LDG + 32 * kbA + 8 * a4 + 4 * h;
-                if constexpr (STRICT) {
-                    typename R::vec4 ghi, glo, whi, wlo;
+                // element offset of keys 32*kbA + 8*a4 + 4*h .. +3 of row 32*qbA + c32
+                const int off = (32 * qbA + c32) * GRAN + (((4 * kbA + a4) ^ gkey(c32)) << 3) + 4 * h;
+                typedef typename Tr<TG>::vec4 G4;
+                auto put = [&](TG* tile, G4 x) { *reinterpret_cast<G4*>(tile + off) = x; };
+                if constexpr (F32) {
+                    const typename R::terms t = R::split(__builtin_shufflevector(gv, wv, 0, 1, 2, 3, 4, 5, 6, 7));
+                    put(Gs, __builtin_shufflevector(t.hi, t.hi, 0, 1, 2, 3)); put(Ws, __builtin_shufflevector(t.hi, t.hi, 4, 5, 6, 7));
+                    put(Gl, __builtin_shufflevector(t.mid, t.mid, 0, 1, 2, 3)); put(Wl, __builtin_shufflevector(t.mid, t.mid, 4, 5, 6, 7));
+                    put(Gz, __builtin_shufflevector(t.lo, t.lo, 0, 1, 2, 3)); put(Wz, __builtin_shufflevector(t.lo, t.lo, 4, 5, 6, 7));
+                } else if constexpr (STRICT) {
+                    G4 ghi, glo, whi, wlo;
                     R::cvt4_split(gv, ghi, glo);
                     R::cvt4_split(wv, whi, wlo);
-                    *reinterpret_cast<typename R::vec4*>(Gs + off) = ghi;
-                    *reinterpret_cast<typename R::vec4*>(Ws + off) = whi;
-                    *reinterpret_cast<typename R::vec4*>(Gl + off) = glo;
-                    *reinterpret_cast<typename R::vec4*>(Wl + off) = wlo;
+                    put(Gs, ghi); put(Ws, whi);
+                    put(Gl, glo); put(Wl, wlo);
                 } else {
-                    *reinterpret_cast<typename R::vec4*>(Gs + off) = R::cvt4(gv);
-                    *reinterpret_cast<typename R::vec4*>(Ws + off) = R::cvt4(wv);
+                    put(Gs, R::cvt4(gv));
+                    put(Ws, R::cvt4(wv));
                 }
             }
             const float rs = sum_halves(rsum);
@@ -447,18 +473,39 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
         float rp0 = 0.f, rp1 = 0.f;
         if (tid < GRAN) { rp0 = rowtmp[tid]; rp1 = rowtmp[GRAN + tid]; }
         // operand fragments of contraction step t: the next step's are read while this step's MFMAs run
+        if constexpr (F32) {
+            // product n = ((2 t + which) NXW + x): column block x of Q (which = 0: dK) or dH (dV), with both key blocks' terms
+            auto dblk = [&](int x) { return BOTH_KB ? x : dsel + 2 * x; };
+            typename R::terms gw[NKB];
+            R::template stream<2 * NQS * NXW>(
+                [&](auto n) { constexpr int m = n / NXW; return trd.read(m & 1 ? dHs : Qs, KW * (m >> 1), dblk(n % NXW)); },
+                [&](auto n, const auto& f, auto&& between) {
+                    constexpr int x = n % NXW, which = (n / NXW) & 1, t = n / NXW / 2;
+                    if constexpr (SPREAD && STAGES == 2) {
+                        if constexpr (x == 0 && which == 0) tdma.issue_range(ldh, gdh, t * PW / NQS, (t + 1) * PW / NQS, rb);
+                    }
+                    if constexpr (x == 0) {
+#pragma unroll
+                        for (int kb = 0; kb < NKB; kb++) {
+                            gw[kb].hi = gw_read(which ? Ws : Gs, t, kb);
+                            gw[kb].mid = gw_read(which ? Wl : Gl, t, kb);
+                            gw[kb].lo = gw_read(which ? Wz : Gz, t, kb);
+                        }
+                    }
+#pragma unroll
+                    for (int kb = 0; kb < NKB; kb++) {
+                        if (kb == 0) R::mma_between(which ? dvacc[kb][x] : dkacc[kb][x], f, gw[kb], between);
+                        else R::mma(which ? dvacc[kb][x] : dkacc[kb][x], f, gw[kb]);
+                    }
+                });
+        } else {
         frag gB[2][NKB], wB[2][NKB], qa[2][NXW], ha[2][NXW];
         // (split mode: the low-order fragments are single-buffered, read at the start of their own step behind the
         // MFMAs on the high-order ones: a second set of them does not fit the registers at D = 256)
         frag gL[STRICT ? NKB : 1], wL[STRICT ? NKB : 1];
         auto read_gw = [&](int t, int kb) {
-            if constexpr (R::HALF) {
-                gB[t & 1][kb] = gw_read(Gs, t, kb);
-                wB[t & 1][kb] = gw_read(Ws, t, kb);
-            } else {
-                gB[t & 1][kb] = frag_transposed<T>(Gs, LDG, KW * t, 32 * (BOTH_KB ? kb : kbB), lane);
-                wB[t & 1][kb] = frag_transposed<T>(Ws, LDG, KW * t, 32 * (BOTH_KB ? kb : kbB), lane);
-            }
+            gB[t & 1][kb] = gw_read(Gs, t, kb);
+            wB[t & 1][kb] = gw_read(Ws, t, kb);
         };
         auto read_qh = [&](int t, int x) {
             const int dblk = BOTH_KB ? wave * NXW + x : dsel + 2 * x;
@@ -497,6 +544,7 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
+        }
         }
         if (tid < GRAN && qi0 + tid < S) a.rowpart[((size_t)bh * a.RS + (a.RS == NG ? jt : jt % a.RS)) * S + qi0 + tid] = rp0 + rp1;
         if constexpr (STAGES == 1) {

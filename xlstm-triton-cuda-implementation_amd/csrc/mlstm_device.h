@@ -4,17 +4,20 @@
 // Lane conventions, measured on MI355X hardware and used everywhere below (l = lane id, h = l / 32):
 //   v_mfma_f32_32x32x16_{bf16,f16}: A holds row l%32, k = 8h..8h+7; B holds column l%32, k = 8h..8h+7;
 //   the 16 accumulator registers r of a lane are column l%32, row 8*(r/4) + 4h + r%4.
-//   v_mfma_f32_32x32x2_f32: A row l%32, k = h; B column l%32, k = h; same accumulator layout.
+//   v_mfma_f32_32x32x2_f32 (scan form, chunk sums): A row l%32, k = h; B column l%32, k = h; same accumulator layout.
 //   ds_read_b64_tr_b16: inside a block of 16 lanes, lanes 4r..4r+3 address "row r" (4 elements each);
 //   lane j of the block receives element j of rows 0..3.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
+#include <utility>
 
 namespace mlstm {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(4))) _Float16 f16x4;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
@@ -28,13 +31,18 @@ constexpr float LOG2E = 1.4426950408889634f;
 constexpr double LOG2E_D = 1.4426950408889634074;
 constexpr int GRAN = 64;  // positions per gate granule == keys per key tile
 
+template <int... I, typename F>
+__device__ __forceinline__ void static_for_impl(std::integer_sequence<int, I...>, F&& f) { (f(std::integral_constant<int, I>{}), ...); }
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) { static_for_impl(std::make_integer_sequence<int, N>{}, f); }
+
 #define LDS_PTR(T) T __attribute__((address_space(3)))*
 
 __device__ __forceinline__ float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
 // ---------------------------------------------------------------------------------------------
-// Per-element-type traits.  A "macro step" contracts KW elements: one 32x32x16 MFMA for the 16-bit
-// types, four 32x32x2 MFMAs for fp32.  A fragment is the 16 bytes one lane contributes to it.
+// Per-element-type traits.  A "macro step" contracts KW = 16 elements: one 32x32x16 MFMA for the 16-bit
+// types, six on the terms of fp32 operands.  A fragment is the eight elements one lane contributes to it.
 // ---------------------------------------------------------------------------------------------
 template <typename T> struct Tr;
 
@@ -43,6 +51,8 @@ template <> struct Tr<__bf16> {
     static constexpr bool HALF = true;
     typedef bf16x8 frag;
     typedef bf16x4 vec4;
+    typedef frag terms;   // what mma takes: for these types the fragment itself
+    static __device__ __forceinline__ terms split(frag x) { return x; }
     static __device__ __forceinline__ void mma(f32x16& c, frag a, frag b) {
         c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
     }
@@ -74,6 +84,8 @@ template <> struct Tr<_Float16> {
     static constexpr bool HALF = true;
     typedef f16x8 frag;
     typedef f16x4 vec4;
+    typedef frag terms;   // what mma takes: for these types the fragment itself
+    static __device__ __forceinline__ terms split(frag x) { return x; }
     static __device__ __forceinline__ void mma(f32x16& c, frag a, frag b) {
         c = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
     }
@@ -99,24 +111,115 @@ template <> struct Tr<_Float16> {
     }
 };
 
+// fp32 operands run on the bf16 matrix units as three terms, x = hi + mid + lo with hi = bf16(x), mid = bf16(x - hi),
+// lo = bf16(x - hi - mid): 24 significant bits, all of an fp32 value.  A product is the six products of terms down to 2^-18 of
+// hi hi; what is left out (mid lo, lo mid, lo lo) is below 2^-26 of a product, a quarter of the rounding of ONE fp32 addition,
+// and the sums have a sixteenth of the roundings of 32x32x2 products.  Six bf16 products take 192 cycles per 32x32x16 block
+// where v_mfma_f32_32x32x2_f32 takes 512; splitting an operand is 44 vector instructions per fragment, which run beside them.
 template <> struct Tr<float> {
-    static constexpr int EPL = 4, KW = 8;
+    static constexpr int EPL = 8, KW = 16;
     static constexpr bool HALF = false;
-    typedef f32x4 frag;
+    typedef f32x8 frag;
     typedef f32x4 vec4;
-    static __device__ __forceinline__ void mma(f32x16& c, frag a, frag b) {
+    struct terms { bf16x8 hi, mid, lo; };
+    // Two values at a time: one conversion packs their terms, and v_dot2_f32_bf16 subtracts either term of a pair from its
+    // value in one instruction (x - 1 t0 - 0 t1, exact: both differences have at most 16 significant bits).
+    static __device__ __forceinline__ terms split(frag x) {
+        terms t;
+        // (-1, 0) and (0, -1) out of registers: as a literal the pair (-1, 0) becomes the operand -1.0, which the instruction
+        // takes for the fp32 pattern, (0, -1)
+        int first_bits = 0x0000bf80, second_bits = (int)0xbf800000;
+        asm("" : "+s"(first_bits), "+s"(second_bits));
+        const bf16x2 first = __builtin_bit_cast(bf16x2, first_bits), second = __builtin_bit_cast(bf16x2, second_bits);
+        auto pack = [](float a, float b) __attribute__((always_inline)) { return __builtin_convertvector(f32x2{a, b}, bf16x2); };
 #pragma unroll
-        for (int e = 0; e < 4; e++) c = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], b[e], c, 0, 0, 0);
+        for (int e = 0; e < 8; e += 2) {
+            float a = x[e], b = x[e + 1];
+            const bf16x2 hi = pack(a, b);
+            a = __builtin_amdgcn_fdot2_f32_bf16(hi, first, a, false);
+            b = __builtin_amdgcn_fdot2_f32_bf16(hi, second, b, false);
+            const bf16x2 mid = pack(a, b);
+            a = __builtin_amdgcn_fdot2_f32_bf16(mid, first, a, false);
+            b = __builtin_amdgcn_fdot2_f32_bf16(mid, second, b, false);
+            const bf16x2 lo = pack(a, b);
+            t.hi[e] = hi[0]; t.hi[e + 1] = hi[1];
+            t.mid[e] = mid[0]; t.mid[e + 1] = mid[1];
+            t.lo[e] = lo[0]; t.lo[e + 1] = lo[1];
+        }
+        return t;
+    }
+    static __device__ __forceinline__ terms split(const terms& t) { return t; }
+    // the six products, smallest first, with something else between them (a vector instruction costs nothing while the matrix
+    // unit works: six products keep it busy for 192 cycles, 48 instructions' worth)
+    template <typename F>
+    static __device__ __forceinline__ void mma_between(f32x16& c, const terms& a, const terms& b, F&& between) {
+        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.lo, b.hi, c, 0, 0, 0);
+        between(std::integral_constant<int, 0>{});
+        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.hi, b.lo, c, 0, 0, 0);
+        between(std::integral_constant<int, 1>{});
+        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.mid, b.mid, c, 0, 0, 0);
+        between(std::integral_constant<int, 2>{});
+        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.mid, b.hi, c, 0, 0, 0);
+        between(std::integral_constant<int, 3>{});
+        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.hi, b.mid, c, 0, 0, 0);
+        between(std::integral_constant<int, 4>{});
+        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.hi, b.hi, c, 0, 0, 0);
+    }
+    template <typename A, typename B>
+    static __device__ __forceinline__ void mma(f32x16& c, const A& a, const B& b) {
+        mma_between(c, split(a), split(b), [](auto) {});
+    }
+    // N products in a row whose one operand is a fragment from LDS (read(n), its reads running AHEAD products in front) and
+    // whose other operand has been split before (product(n, terms) calls mma_between): fragment n + 1 is split between the
+    // MFMAs of product n.
+    template <int N, int AHEAD = 2, typename Read, typename Product>
+    static __device__ __forceinline__ void stream(Read&& read, Product&& product) {
+        frag raw[AHEAD + 1];
+        static_for<AHEAD + 1>([&](auto n) __attribute__((always_inline)) { if constexpr (decltype(n)::value < N) raw[n] = read(n); });
+        terms cur = split(raw[0]);
+        static_for<N>([&](auto nc) __attribute__((always_inline)) {
+            constexpr int n = decltype(nc)::value;
+            if constexpr (n + AHEAD + 1 < N) raw[(n + AHEAD + 1) % (AHEAD + 1)] = read(std::integral_constant<int, n + AHEAD + 1>{});
+            terms next = cur;
+            float x[8];
+            bf16x2 p[4];
+            int first_bits = 0x0000bf80, second_bits = (int)0xbf800000;   // (see split)
+            asm("" : "+s"(first_bits), "+s"(second_bits));
+            product(nc, cur, [&](auto ic) __attribute__((always_inline)) {
+                constexpr int i = decltype(ic)::value;
+                if constexpr (n + 1 < N) {
+                    if constexpr (i == 0) {
+#pragma unroll
+                        for (int e = 0; e < 8; e++) x[e] = raw[(n + 1) % (AHEAD + 1)][e];
+                    }
+                    if constexpr (i % 2 == 0) {   // a term of every pair
+#pragma unroll
+                        for (int e = 0; e < 4; e++) p[e] = __builtin_convertvector(f32x2{x[2 * e], x[2 * e + 1]}, bf16x2);
+                        bf16x8& t = i == 0 ? next.hi : (i == 2 ? next.mid : next.lo);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) { t[2 * e] = p[e][0]; t[2 * e + 1] = p[e][1]; }
+                    } else {                      // and what it leaves
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            x[2 * e] = __builtin_amdgcn_fdot2_f32_bf16(p[e], __builtin_bit_cast(bf16x2, first_bits), x[2 * e], false);
+                            x[2 * e + 1] = __builtin_amdgcn_fdot2_f32_bf16(p[e], __builtin_bit_cast(bf16x2, second_bits), x[2 * e + 1], false);
+                        }
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            });
+            cur = next;
+        });
     }
     static __device__ __forceinline__ frag from_acc(const f32x16& c, int t) {
         frag x;
 #pragma unroll
-        for (int e = 0; e < 4; e++) x[e] = c[4 * t + e];
+        for (int e = 0; e < 8; e++) x[e] = c[8 * t + e];
         return x;
     }
     static __device__ __forceinline__ vec4 cvt4(f32x4 x) { return x; }
-    // (fp32 operands are exact: there is no split mode; these keep the shared templates well-formed)
-    static __device__ __forceinline__ void from_acc_split(const f32x16& c, int t, frag& hi, frag& lo) { hi = from_acc(c, t); lo = frag{0.f, 0.f, 0.f, 0.f}; }
+    // (there is no split mode for fp32 tensors; these keep the shared templates well-formed)
+    static __device__ __forceinline__ void from_acc_split(const f32x16& c, int t, frag& hi, frag& lo) { hi = from_acc(c, t); lo = frag{}; }
     static __device__ __forceinline__ void cvt4_split(f32x4 x, vec4& hi, vec4& lo) { hi = x; lo = vec4{0.f, 0.f, 0.f, 0.f}; }
 };
 
@@ -136,13 +239,17 @@ __device__ __forceinline__ typename Tr<T>::vec4 gate4(typename Tr<T>::vec4 h, ty
 // KW*s + EPL*h + e.
 template <typename T>
 __device__ __forceinline__ typename Tr<T>::frag frag_rowmajor(const T* row, int s, int h) {
-    return *reinterpret_cast<const typename Tr<T>::frag*>(row + Tr<T>::KW * s + Tr<T>::EPL * h);
+    if constexpr (Tr<T>::HALF) return *reinterpret_cast<const typename Tr<T>::frag*>(row + Tr<T>::KW * s + Tr<T>::EPL * h);
+    else {
+        const f32x4 *p = reinterpret_cast<const f32x4*>(row + Tr<T>::KW * s + Tr<T>::EPL * h);
+        return __builtin_shufflevector(p[0], p[1], 0, 1, 2, 3, 4, 5, 6, 7);
+    }
 }
 
 // Transposed fragment out of an LDS tile stored row-major [contraction index][column], row stride ldt:
 // the lane receives column cb + l%32 for the contraction indices of one macro step starting at row kr.
-// 16-bit: element e = 4x + e' is row kr + 8x + 4h + e'; fp32: element e is row kr + 4h + e.  Both match
-// Tr<T>::from_acc, so an accumulator block can be the other operand without any lane exchange.
+// Element e = 4x + e' is row kr + 8x + 4h + e'.  That matches Tr<T>::from_acc, so an accumulator block can be the other
+// operand without any lane exchange.
 template <typename T>
 __device__ __forceinline__ typename Tr<T>::frag frag_transposed(const T* tile, int ldt, int kr, int cb, int lane) {
     const int h = lane >> 5;
@@ -158,7 +265,7 @@ __device__ __forceinline__ typename Tr<T>::frag frag_transposed(const T* tile, i
         const T* p = tile + (kr + 4 * h) * ldt + cb + (lane & 31);
         typename Tr<T>::frag f;
 #pragma unroll
-        for (int e = 0; e < 4; e++) f[e] = p[e * ldt];
+        for (int e = 0; e < 8; e++) f[e] = p[(8 * (e >> 2) + (e & 3)) * ldt];
         return f;
     }
 }
@@ -420,11 +527,22 @@ struct RowVec3Dma {
     }
 };
 
+// A lane's fragment of a swizzled row from the byte offset of its first element: one 16-byte chunk, or for fp32 an even chunk
+// and the odd one behind it, which the swizzle leaves next to each other (`off2` = off ^ 16).
+template <typename T>
+__device__ __forceinline__ typename Tr<T>::frag swz_frag_at(const char* base, int off, int off2) {
+    if constexpr (Tr<T>::HALF) return *reinterpret_cast<const typename Tr<T>::frag*>(base + off);
+    else {
+        const f32x4 lo = *reinterpret_cast<const f32x4*>(base + off), hi = *reinterpret_cast<const f32x4*>(base + off2);
+        return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+    }
+}
+
 // Row-major fragment of a swizzled tile: lane owns row r, macro step s (columns KW*s + EPL*h ..).
 template <typename T, int D>
 __device__ __forceinline__ typename Tr<T>::frag swz_frag_rowmajor(const T* tile, int r, int s, int h) {
-    const char* base = reinterpret_cast<const char*>(tile);
-    return *reinterpret_cast<const typename Tr<T>::frag*>(base + Swz<T, D>::off(r, Tr<T>::KW * s + Tr<T>::EPL * h));
+    const int off = Swz<T, D>::off(r, Tr<T>::KW * s + Tr<T>::EPL * h);
+    return swz_frag_at<T>(reinterpret_cast<const char*>(tile), off, off ^ 16);
 }
 
 // Transposed fragment of a swizzled tile (see frag_transposed for the element order).
@@ -443,7 +561,7 @@ __device__ __forceinline__ typename Tr<T>::frag swz_frag_transposed(const T* til
     } else {
         typename Tr<T>::frag f;
 #pragma unroll
-        for (int e = 0; e < 4; e++) f[e] = *reinterpret_cast<const float*>(base + Z::off(kr + 4 * h + e, cb + (lane & 31)));
+        for (int e = 0; e < 8; e++) f[e] = *reinterpret_cast<const float*>(base + Z::off(kr + 8 * (e >> 2) + 4 * h + (e & 3), cb + (lane & 31)));
         return f;
     }
 }
@@ -451,11 +569,12 @@ __device__ __forceinline__ typename Tr<T>::frag swz_frag_transposed(const T* til
 // Per-lane byte offsets for the two fragment kinds of a swizzled tile, precomputed once per kernel so that every
 // read in the unrolled loops is "one address register + immediate".  XOR swizzling is not affine in the chunk index,
 // but the key only touches chunk bits 0..3, and it only depends on the row modulo 16:
-//   row-major reads: chunk = 2s + h, so macro steps s and s + 8 differ by 256 bytes and rows r and r + 32 by 32 rows;
+//   row-major reads: chunk = 2s + h (fp32: 4s + 2h), so macro steps s and s + 8 (fp32: s + 4) differ by 256 bytes and rows
+//   r and r + 32 by 32 rows;
 //   transposed reads (16-bit): column block d and d + 4 differ by 256 bytes, rows kr and kr + 16 by 16 rows.
 template <typename T, int D>
 struct SwzRowReader {
-    static constexpr int NS = D / Tr<T>::KW, KO = NS < 8 ? NS : 8;
+    static constexpr int NS = D / Tr<T>::KW, PER = 256 / (Tr<T>::KW * (int)sizeof(T)), KO = NS < PER ? NS : PER;
     int off[KO];
     __device__ __forceinline__ void init(int lane) {
 #pragma unroll
@@ -464,7 +583,7 @@ struct SwzRowReader {
     // fragment of row 32*rb + (lane & 31), macro step s
     __device__ __forceinline__ typename Tr<T>::frag read(const T* tile, int rb, int s) const {
         const char* base = reinterpret_cast<const char*>(tile);
-        return *reinterpret_cast<const typename Tr<T>::frag*>(base + off[s % KO] + (s / KO) * 256 + rb * 32 * Swz<T, D>::ROW_BYTES);
+        return swz_frag_at<T>(base + (s / KO) * 256 + rb * 32 * Swz<T, D>::ROW_BYTES, off[s % KO], off[s % KO] ^ 16);
     }
 };
 
@@ -478,6 +597,26 @@ struct SwzRowReaderX {
     __device__ __forceinline__ typename Tr<T>::frag read(const T* tile, int rb, int s) const {
         const char* base = reinterpret_cast<const char*>(tile);
         return *reinterpret_cast<const typename Tr<T>::frag*>(base + (off0 ^ ((s % 8) << 5)) + (s / 8) * 256 + rb * 32 * Swz<T, D>::ROW_BYTES);
+    }
+};
+
+// fp32: a fragment is eight dwords of eight rows; the row offsets and the key's meeting with an even and an odd column block.
+template <int D>
+struct SwzTransReaderF32 {
+    static_assert(Swz<float, D>::CPR >= 16, "tiles of at least 256 bytes per row");
+    int off[2][8];
+    __device__ __forceinline__ void init(int lane, int cb0 = 0) {
+#pragma unroll
+        for (int v = 0; v < 2; v++)
+#pragma unroll
+            for (int e = 0; e < 8; e++) off[v][e] = Swz<float, D>::off(8 * (e >> 2) + 4 * (lane >> 5) + (e & 3), 32 * (cb0 + v) + (lane & 31));
+    }
+    __device__ __forceinline__ f32x8 read(const float* tile, int kr, int d) const {
+        const char* base = reinterpret_cast<const char*>(tile) + kr * Swz<float, D>::ROW_BYTES + (d >> 1) * 256;
+        f32x8 f;
+#pragma unroll
+        for (int e = 0; e < 8; e++) f[e] = *reinterpret_cast<const float*>(base + off[d & 1][e]);
+        return f;
     }
 };
 

@@ -111,6 +111,9 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
 #pragma unroll
     for (int s = 0; s < NS; s++) pin(xf[s]);
     pin(crow_base); pin(inv_n); pin(dbv);
+    typename R::terms xt[NS];   // the rows' operand of every first product
+#pragma unroll
+    for (int s = 0; s < NS; s++) xt[s] = R::split(xf[s]);
 
     f32x16 oacc[NDB];
 #pragma unroll
@@ -122,8 +125,9 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
     constexpr bool FAST_TR = R::HALF && Swz<T, D>::CPR >= 16;  // precomputed offsets for the transposing reads
     SwzRowReader<T, D> krd;
     krd.init(lane);
-    SwzTransReader<typename std::conditional<FAST_TR, T, __bf16>::type, FAST_TR ? D : 256> vrd;
-    if constexpr (FAST_TR) vrd.init(lane);
+    constexpr bool F32 = !R::HALF;
+    typename std::conditional<F32, SwzTransReaderF32<D>, SwzTransReader<typename std::conditional<FAST_TR, T, __bf16>::type, FAST_TR ? D : 256>>::type vrd;
+    if constexpr (FAST_TR || F32) vrd.init(lane);
 
     const int last_row = (q0 + ROW_BQ - 1 < S - 1) ? q0 + ROW_BQ - 1 : S - 1;
     const int nJ = last_row / GRAN + 1;
@@ -155,6 +159,14 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
     // first product of both 32-key blocks of a tile, S^T (or dC^T) in accumulator layout; the two accumulation
     // chains are interleaved so that consecutive MFMAs never depend on each other
     auto gemm1x2 = [&](const T* y1, f32x16& s0, f32x16& s1, auto&& hook) {
+        if constexpr (F32) {
+            s0 = f32x16{}; s1 = f32x16{};
+            R::template stream<2 * NS>([&](auto n) { return krd.read(y1, n & 1, n >> 1); }, [&](auto n, const auto& kf, auto&& between) {
+                if (n % 4 == 0) hook(n / 4, NS / 2);
+                R::mma_between(n & 1 ? s1 : s0, kf, xt[n >> 1], between);
+            });
+            return;
+        }
         constexpr int BATCH = NS < 4 ? NS : 4;  // fragments fetched ahead of the MFMAs that consume them
 #pragma unroll
         for (int b0 = 0; b0 < NS; b0 += BATCH) {
@@ -168,16 +180,21 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
                     const f32x16 z = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
                     s0 = z; s1 = z;
                 }
-                R::mma(s0, k0[s], xf[b0 + s]);
-                R::mma(s1, k1[s], xf[b0 + s]);
+                R::mma(s0, k0[s], xt[b0 + s]);
+                R::mma(s1, k1[s], xt[b0 + s]);
             }
         }
     };
     auto gemm1 = [&](const T* y1, int kb, f32x16& sacc) {
 #pragma unroll
         for (int r = 0; r < 16; r++) sacc[r] = 0.f;
+        if constexpr (F32) {
+            R::template stream<NS>([&](auto n) { return krd.read(y1, kb, n); },
+                                   [&](auto n, const auto& kf, auto&& between) { R::mma_between(sacc, kf, xt[n], between); });
+        } else {
 #pragma unroll
-        for (int s = 0; s < NS; s++) R::mma(sacc, krd.read(y1, kb, s), xf[s]);
+            for (int s = 0; s < NS; s++) R::mma(sacc, krd.read(y1, kb, s), xt[s]);
+        }
     };
     // gate weights; `diag` masks the keys above the diagonal of a diagonal block
     auto weigh = [&](f32x16& sacc, const float* sal, int kb, float crow, bool diag) {
@@ -223,6 +240,15 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
     };
     // second product: accumulate this key block into the output
     auto gemm2 = [&](const T* y2, const f32x16& sacc, int kb, auto&& hook) {
+        if constexpr (F32) {
+            const typename R::terms p[2] = {R::split(R::from_acc(sacc, 0)), R::split(R::from_acc(sacc, 1))};
+            R::template stream<2 * NDB>([&](auto n) { return vrd.read(y2, 32 * kb + KW * (n / NDB), n % NDB); },
+                                        [&](auto n, const auto& vf, auto&& between) {
+                                            if (n % NDB == 0) hook(2 * kb + n / NDB, 4);
+                                            R::mma_between(oacc[n % NDB], vf, p[n / NDB], between);
+                                        });
+            return;
+        }
 #pragma unroll
         for (int t = 0; t < NSTEP32; t++) {
             hook(kb * NSTEP32 + t, 2 * NSTEP32);
@@ -232,7 +258,7 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
             frag vf[NDB];
 #pragma unroll
             for (int d = 0; d < NDB; d++) {
-                if constexpr (FAST_TR) vf[d] = vrd.read(y2, 32 * kb + KW * t, d);
+                if constexpr (FAST_TR || F32) vf[d] = vrd.read(y2, 32 * kb + KW * t, d);
                 else vf[d] = swz_frag_transposed<T, D>(y2, 32 * kb + KW * t, 32 * d, lane);
             }
 #pragma unroll
@@ -283,7 +309,7 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
                 const f32x16 z = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
                 s0 = z; s1 = z;
             }
-            R::mma(s0, kq[s], xf[s]);
+            R::mma(s0, kq[s], xt[s]);
             __builtin_amdgcn_sched_barrier(0);
         }
         // ---- S1, weighing S0 (16 registers over NS MFMAs)
@@ -294,7 +320,7 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
         for (int s = 0; s < NS; s++) {
             if (s % 4 == 0) hook1(NS / 4 + s / 4, 2 * (NS / 4));
             if (s + AH < NS) kr[s + AH] = krd.read(y1, 1, s + AH);
-            R::mma(s1, kr[s], xf[s]);
+            R::mma(s1, kr[s], xt[s]);
 #pragma unroll
             for (int r = s * 16 / NS; r < (s + 1) * 16 / NS; r++) weigh_reg(s0, r, ek0, er0, blk0);
             __builtin_amdgcn_sched_barrier(0);
@@ -358,8 +384,15 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
             else ROW_DMA(0, 0);
             const T* th = ST_Y1(stg);
             const T* tl = ST_Y2(stg);
+            if constexpr (F32) {
+                R::template stream<NGRP * NDB>([&](auto n) { return vrd.read(th, KW * (n / NDB), n % NDB); },
+                                               [&](auto n, const auto& cf, auto&& between) {
+                                                   R::mma_between(oacc[n % NDB], cf, xt[NGRP * tau + n / NDB], between);
+                                               });
+                continue;
+            }
             auto rd = [&](const T* tile, int g, int d) {
-                if constexpr (FAST_TR) return vrd.read(tile, KW * g, d);
+                if constexpr (FAST_TR || F32) return vrd.read(tile, KW * g, d);
                 else return swz_frag_transposed<T, D>(tile, KW * g, 32 * d, lane);
             };
             frag vf[2][NDB];
@@ -372,11 +405,11 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
                 for (int d = 0; d < NDB; d++) {
                     if constexpr (STRICT) vl[d] = rd(tl, g, d);
                     if (g + 1 < NGRP) vf[(g + 1) & 1][d] = rd(th, g + 1, d);
-                    R::mma(oacc[d], vf[g & 1][d], xf[NGRP * tau + g]);
+                    R::mma(oacc[d], vf[g & 1][d], xt[NGRP * tau + g]);
                 }
                 if constexpr (STRICT) {
 #pragma unroll
-                    for (int d = 0; d < NDB; d++) R::mma(oacc[d], vl[d], xf[NGRP * tau + g]);
+                    for (int d = 0; d < NDB; d++) R::mma(oacc[d], vl[d], xt[NGRP * tau + g]);
                 }
             }
         }
