@@ -4,6 +4,7 @@
 #include <utility>
 #include <vector>
 #include "mlstm_kernels.h"
+#include "mlstm_train.h"
 
 using namespace mlstm;
 
@@ -633,7 +634,7 @@ namespace {
 // the backward on a workspace of Sizes::bwd() bytes; arguments already validated
 int backward_impl(const void* dh, const void* q, const void* k, const void* v, const void* f, const void* i, const void* h, const float* m,
                   const float* b, void* dq, void* dk, void* dv, void* df, void* di, const Sizes& z, int D, int dtype, int gate_dtype,
-                  char* ws, hipStream_t st, const char* saved = nullptr, const Lay* h_layout = nullptr) {
+                  char* ws, hipStream_t st, const char* saved = nullptr, const Lay* h_layout = nullptr, char* gates_kept = nullptr) {
     if (z.scan_engine()) {   // (recomputes the forward it needs; h, m, b are not read)
         if (!is_dense(z.la, (long long)z.S, (long long)z.D) || !is_dense(z.lb, (long long)z.S, (long long)z.D) ||
             !is_dense(z.lg, (long long)z.S, 1) || z.gate_form != MLSTM_GATE_RAW || gate_dtype != MLSTM_F32)
@@ -671,6 +672,7 @@ int backward_impl(const void* dh, const void* q, const void* k, const void* v, c
         }
         h_lo = sv.h_lo;
     }
+    if (gates_kept && !reuse) w.gates_at(gates_kept, z);   // (a sequence that does not run in chunks: the forward's gate pre-pass)
     char* Ev = c.take<char>(z.state_elems() * z.el * z.parts());    // reverse states, value-major
     float* gvec = c.take<float>(z.BH * w.ncs * z.D);
     float* rowinter = c.take<float>(z.BH * z.S);
@@ -690,7 +692,7 @@ int backward_impl(const void* dh, const void* q, const void* k, const void* v, c
     if (have_fwd) {
         // gates only: alpha, beta, G (and m again, into the workspace) are cheap to rebuild; so are the chunk states
         G2 = w.G2; alpha2 = w.alpha2; beta2 = w.beta2; ek2 = w.ek2; amax2 = w.amax2; mm = w.mw;
-        if (reuse) {
+        if (reuse || gates_kept) {
             mm = const_cast<float*>(m);
         } else {
             Timed t(MLSTM_K_GATES, st);
@@ -769,7 +771,8 @@ int backward_impl(const void* dh, const void* q, const void* k, const void* v, c
 // the gated backward on a workspace of Sizes::bwd_gated() bytes; dense_out: dh_gated, o, h and d_o are dense tensors
 int backward_gated_impl(const void* dh_gated, const void* q, const void* k, const void* v, const void* f, const void* i, const void* o,
                         const void* h, const float* m, const float* b, void* dq, void* dk, void* dv, void* df, void* di, void* d_o, const Sizes& z,
-                        int NH, int D, int dtype, int gate_dtype, bool dense_out, char* ws, hipStream_t st) {
+                        int NH, int D, int dtype, int gate_dtype, bool dense_out, char* ws, hipStream_t st, const char* saved = nullptr,
+                        char* gates_kept = nullptr) {
     Carver c{ws, z.bwd()};
     char* dh = c.take<char>(z.BH * z.S * z.D * z.el);
     char* hown = c.take<char>(z.BH * z.S * z.D * z.el);
@@ -795,7 +798,7 @@ int backward_gated_impl(const void* dh_gated, const void* q, const void* k, cons
     // the ungated upstream gradient is the library's own, dense; h stays where it is
     Sizes zb = z;
     zb.lb = dense;
-    return backward_impl(dh, q, k, v, f, i, h, m, b, dq, dk, dv, df, di, zb, D, dtype, gate_dtype, ws, st, nullptr, &lh);
+    return backward_impl(dh, q, k, v, f, i, h, m, b, dq, dk, dv, df, di, zb, D, dtype, gate_dtype, ws, st, saved, &lh, gates_kept);
 }
 
 }  // namespace
@@ -954,3 +957,71 @@ int mlstm_scan_backward_saved_ex(const void* dh_gated, const void* q, const void
 }
 
 }  // extern "C"
+
+namespace {
+// the parts of a training step's buffer
+struct Kept {
+    float *m, *b;
+    char *saved = nullptr, *gates = nullptr;
+    size_t bytes;
+    Kept(char* p, const Sizes& z) {
+        Carver c{p, 0};
+        m = c.take<float>(z.BH * z.S);
+        b = c.take<float>(z.BH * z.S);
+        if (z.saved() > 0) saved = c.take<char>(z.saved());
+        if (!z.scan_engine() && z.n_states(z.chunk_len()) == 0) gates = c.take<char>(z.gates());
+        bytes = c.off;
+    }
+};
+}  // namespace
+
+namespace mlstm {
+
+size_t train_kept_bytes(int B, int NH, int S, int D, int dtype) { return Kept(nullptr, sizes_of(B, NH, S, D, dtype)).bytes; }
+
+int train_forward(const void* q, const void* k, const void* v, const void* f, const void* i, const void* o, void* h, void* h_gated, void* kept, size_t kept_bytes, int B,
+                  int NH, int S, int D, int dtype, int gate_dtype, const mlstm_layout* layout, void* workspace, size_t workspace_bytes, void* stream) {
+    const int dtype_arg = dtype;
+    dtype &= ~MLSTM_PRECISE;
+    if (!good_shape(D, dtype) || S > 131072) return MLSTM_ESHAPE;
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    Sizes z = sizes_of(B, NH, S, D, dtype_arg);
+    if (o && z.scan_engine()) return MLSTM_ESHAPE;
+    if (int rc = apply_layout(z, layout, NH, gate_dtype, {q, k, v, o, h, h_gated}, false, true, false)) return rc;
+    if (workspace_bytes < z.fwd()) return MLSTM_EWORKSPACE;
+    const Kept kp((char*)kept, z);
+    if (kept_bytes != kp.bytes) return MLSTM_EWORKSPACE;
+    SavedStamp stamp;
+    char *CstT = nullptr, *gates = kp.gates, *h_lo = nullptr;
+    float* Nst = nullptr;
+    if (kp.saved) {
+        SavedView sv(kp.saved, z);
+        stamp = saved_stamp_of(z);
+        stamp.dst = sv.header;
+        CstT = sv.CstT; Nst = sv.Nst; h_lo = sv.h_lo;
+        if (sv.gates) gates = sv.gates;
+    }
+    return forward_impl(q, k, v, f, i, h, kp.m, kp.b, z, D, dtype, gate_dtype, (char*)workspace, st, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr,
+                        nullptr, o, h_gated, CstT, Nst, gates, h_lo, kp.saved ? &stamp : nullptr);
+}
+
+int train_backward(const void* dh, const void* q, const void* k, const void* v, const void* f, const void* i, const void* o, const void* h,
+                   const void* kept, size_t kept_bytes, void* dq, void* dk, void* dv, void* df, void* di, void* d_o, int B, int NH, int S, int D, int dtype,
+                   int gate_dtype, const mlstm_layout* layout, void* workspace, size_t workspace_bytes, void* stream) {
+    const int dtype_arg = dtype;
+    dtype &= ~MLSTM_PRECISE;
+    if (!good_shape(D, dtype) || S > 131072) return MLSTM_ESHAPE;
+    hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    Sizes z = sizes_of(B, NH, S, D, dtype_arg);
+    if (o && z.scan_engine()) return MLSTM_ESHAPE;
+    if (int rc = apply_layout(z, layout, NH, gate_dtype, {dh, q, k, v, o, h, dq, dk, dv, d_o}, true, o != nullptr, true)) return rc;
+    if (workspace_bytes < (o ? z.bwd_gated() : z.bwd())) return MLSTM_EWORKSPACE;
+    const Kept kp((char*)const_cast<void*>(kept), z);
+    if (kept_bytes != kp.bytes) return MLSTM_EWORKSPACE;   // (a process-wide setting changed since the forward)
+    if (o)
+        return backward_gated_impl(dh, q, k, v, f, i, o, h, kp.m, kp.b, dq, dk, dv, df, di, d_o, z, NH, D, dtype, gate_dtype, layout == nullptr,
+                                   (char*)workspace, st, kp.saved, kp.gates);
+    return backward_impl(dh, q, k, v, f, i, h, kp.m, kp.b, dq, dk, dv, df, di, z, D, dtype, gate_dtype, (char*)workspace, st, kp.saved, nullptr, kp.gates);
+}
+
+}  // namespace mlstm

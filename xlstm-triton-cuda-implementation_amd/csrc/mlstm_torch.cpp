@@ -3,7 +3,7 @@
 // A call on a short sequence is bound by its host side: the GPU needs 18 us for a forward of one head of 640 positions and
 // 50-160 us for a training step of a small model, while the Python wrappers (tensor checks, a torch.empty per output, ctypes
 // with 20 arguments, autograd.Function in the engine's thread) took 36 and 230 us.  Here the checks read the tensors' fields,
-// the allocations go to torch's caching allocator directly, m, b and the saved states of a training step share one of them, and
+// the allocations go to torch's caching allocator directly, what a training step keeps for its backward shares one of them, and
 // the backward is a C++ node, which the autograd engine's thread runs without the interpreter lock.
 //
 // Every function takes the operator's tensors and returns its result, or None for whatever the fast path does not serve
@@ -21,7 +21,7 @@
 #include <torch/csrc/autograd/saved_variable.h>
 #include <algorithm>
 #include <vector>
-#include "../../include/mlstm_hip.h"
+#include "mlstm_train.h"
 
 namespace {
 
@@ -74,8 +74,6 @@ struct Buffer {
     Buffer() = default;
     void* get(size_t off = 0) const { return n ? static_cast<char*>(p.get()) + off : nullptr; }
 };
-size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
-
 Tensor new_tensor(at::IntArrayRef size, at::IntArrayRef stride, at::ScalarType type, const Tensor& like) {
     return Tensor(at::detail::empty_strided_cuda(size, stride, type, like.device()));
 }
@@ -117,7 +115,8 @@ struct Call {
     mlstm_layout layout(const Tensor& q, const Tensor& h, const Tensor& f) const {
         return mlstm_layout{q.stride(0), q.stride(1), q.stride(2), h.stride(0), h.stride(1), h.stride(2), f.stride(0), f.stride(1), f.stride(2), gate_form};
     }
-    size_t rows() const { return (size_t)B * NH * S; }
+    bool on_tiles() const { return D == 64 || D == 128; }   // scan form: the head dimensions that the tile kernels serve
+    Buffer kept() const { return Buffer(mlstm::train_kept_bytes(B, NH, S, D, dtype)); }
     Buffer workspace(int op) const { return Buffer(mlstm_workspace_bytes(op, B, NH, S, D, dtype)); }
 };
 
@@ -141,28 +140,13 @@ bool takes_matmul(const Tensor& q, const Tensor& k, const Tensor& v, const Tenso
     return true;
 }
 
-// What a training step keeps for its backward besides tensors: m, b and the library's saved states, in one allocation.
-struct Kept {
-    Buffer buf;
-    size_t b_off = 0, saved_off = 0, saved_bytes = 0;
-    explicit Kept(const Call& c) {
-        b_off = up256(c.rows() * 4);
-        saved_off = 2 * b_off;
-        saved_bytes = mlstm_saved_state_bytes(c.B, c.NH, c.S, c.D, c.dtype);
-        buf = Buffer(saved_off + saved_bytes);
-    }
-    Kept() = default;
-    float* m() const { return static_cast<float*>(buf.get()); }
-    float* b() const { return static_cast<float*>(buf.get(b_off)); }
-    void* saved() const { return saved_bytes ? buf.get(saved_off) : nullptr; }
-};
-
-// The nodes of the graph: the inputs (and an output the backward reads) under autograd's version checks, and a Kept.
+// The nodes of the graph: the inputs (and an output the backward reads) under autograd's version checks, and a buffer with what
+// else the backward reads.
 struct OpNode : torch::autograd::Node {
     Call c;
     std::vector<SavedVariable> vars;
     SavedVariable out;
-    Kept kept;
+    Buffer kept;
     void save(std::initializer_list<Tensor> ts) {
         vars.reserve(ts.size());
         for (const Tensor& t : ts) vars.emplace_back(t, false);
@@ -170,7 +154,7 @@ struct OpNode : torch::autograd::Node {
     void release_variables() override {
         for (auto& v : vars) v.reset_data();
         out.reset_data();
-        kept = Kept();
+        kept = Buffer();
     }
     std::vector<Tensor> inputs() {
         std::vector<Tensor> ts;
@@ -213,10 +197,9 @@ struct Triton_mLSTMBackward : OpNode {
         for (int n = 0; n < 5; n++) res[n] = new_like(in[n]);
         const mlstm_layout lay = c.layout(in[0], h, in[3]);
         Buffer ws = c.workspace(MLSTM_OP_BACKWARD);
-        check_rc(mlstm_backward_saved_lx(dh.data_ptr(), in[0].data_ptr(), in[1].data_ptr(), in[2].data_ptr(), in[3].data_ptr(), in[4].data_ptr(),
-                                         h.data_ptr(), kept.m(), kept.b(), kept.saved(), kept.saved_bytes, res[0].data_ptr(), res[1].data_ptr(),
-                                         res[2].data_ptr(), res[3].data_ptr(), res[4].data_ptr(), c.B, c.NH, c.S, c.D, c.dtype, c.gate_dtype, &lay,
-                                         ws.get(), ws.n, hip_stream()),
+        check_rc(mlstm::train_backward(dh.data_ptr(), in[0].data_ptr(), in[1].data_ptr(), in[2].data_ptr(), in[3].data_ptr(), in[4].data_ptr(), nullptr,
+                                       h.data_ptr(), kept.get(), kept.n, res[0].data_ptr(), res[1].data_ptr(), res[2].data_ptr(), res[3].data_ptr(),
+                                       res[4].data_ptr(), nullptr, c.B, c.NH, c.S, c.D, c.dtype, c.gate_dtype, &lay, ws.get(), ws.n, hip_stream()),
                  "mlstm_backward_saved_lx");
         return res;
     }
@@ -237,9 +220,9 @@ bool matmul(const Tensor* t, int precise, int gate_form, bool train, Tensor& h) 
     }
     auto node = make_node<Triton_mLSTMBackward>(q, k, v, f, i);
     node->c = c;
-    node->kept = Kept(c);
-    check_rc(mlstm_forward_save_lx(q.data_ptr(), k.data_ptr(), v.data_ptr(), f.data_ptr(), i.data_ptr(), h.data_ptr(), node->kept.m(), node->kept.b(),
-                                   node->kept.saved(), node->kept.saved_bytes, c.B, c.NH, c.S, c.D, c.dtype, c.gate_dtype, &lay, ws.get(), ws.n, hip_stream()),
+    node->kept = c.kept();
+    check_rc(mlstm::train_forward(q.data_ptr(), k.data_ptr(), v.data_ptr(), f.data_ptr(), i.data_ptr(), nullptr, h.data_ptr(), nullptr, node->kept.get(),
+                                  node->kept.n, c.B, c.NH, c.S, c.D, c.dtype, c.gate_dtype, &lay, ws.get(), ws.n, hip_stream()),
              "mlstm_forward_save_lx");
     node->save({q, k, v, f, i});
     torch::autograd::set_history(h, node);
@@ -267,10 +250,10 @@ struct Triton_mLSTM_gatedBackward : OpNode {
         res[5] = new_like(h);
         const mlstm_layout lay = c.layout(in[0], h, in[3]);
         Buffer ws = c.workspace(MLSTM_OP_BACKWARD_GATED);
-        check_rc(mlstm_backward_gated_lx(dh.data_ptr(), in[0].data_ptr(), in[1].data_ptr(), in[2].data_ptr(), in[3].data_ptr(), in[4].data_ptr(),
-                                         o.data_ptr(), h.data_ptr(), kept.m(), kept.b(), res[0].data_ptr(), res[1].data_ptr(), res[2].data_ptr(),
-                                         res[3].data_ptr(), res[4].data_ptr(), res[5].data_ptr(), c.B, c.NH, c.S, c.D, c.dtype, c.gate_dtype, &lay,
-                                         ws.get(), ws.n, hip_stream()),
+        check_rc(mlstm::train_backward(dh.data_ptr(), in[0].data_ptr(), in[1].data_ptr(), in[2].data_ptr(), in[3].data_ptr(), in[4].data_ptr(),
+                                       o.data_ptr(), h.data_ptr(), kept.get(), kept.n, res[0].data_ptr(), res[1].data_ptr(), res[2].data_ptr(), res[3].data_ptr(),
+                                       res[4].data_ptr(), res[5].data_ptr(), c.B, c.NH, c.S, c.D, c.dtype, c.gate_dtype, &lay, ws.get(), ws.n,
+                                       hip_stream()),
                  "mlstm_backward_gated_lx");
         return res;
     }
@@ -291,21 +274,21 @@ bool gated(const Tensor* t, bool train, Tensor& hg) {
     }
     const mlstm_layout lay = c.layout(q, h, f);
     Buffer ws = c.workspace(MLSTM_OP_FORWARD_GATED);
-    std::shared_ptr<Triton_mLSTM_gatedBackward> node;
-    if (keep) {
-        node = make_node<Triton_mLSTM_gatedBackward>(q, k, v, f, i, t[5]);
-        node->c = c;
-        node->kept = Kept(c);
+    if (!keep) {
+        check_rc(mlstm_forward_gated_lx(q.data_ptr(), k.data_ptr(), v.data_ptr(), f.data_ptr(), i.data_ptr(), o.data_ptr(), h.data_ptr(), hg.data_ptr(),
+                                        nullptr, nullptr, c.B, c.NH, c.S, c.D, c.dtype, c.gate_dtype, &lay, ws.get(), ws.n, hip_stream()),
+                 "mlstm_forward_gated_lx");
+        return true;
     }
-    check_rc(mlstm_forward_gated_lx(q.data_ptr(), k.data_ptr(), v.data_ptr(), f.data_ptr(), i.data_ptr(), o.data_ptr(), h.data_ptr(), hg.data_ptr(),
-                                    keep ? node->kept.m() : nullptr, keep ? node->kept.b() : nullptr, c.B, c.NH, c.S, c.D, c.dtype, c.gate_dtype, &lay,
-                                    ws.get(), ws.n, hip_stream()),
+    auto node = make_node<Triton_mLSTM_gatedBackward>(q, k, v, f, i, t[5]);
+    node->c = c;
+    node->kept = c.kept();
+    check_rc(mlstm::train_forward(q.data_ptr(), k.data_ptr(), v.data_ptr(), f.data_ptr(), i.data_ptr(), o.data_ptr(), h.data_ptr(), hg.data_ptr(),
+                                  node->kept.get(), node->kept.n, c.B, c.NH, c.S, c.D, c.dtype, c.gate_dtype, &lay, ws.get(), ws.n, hip_stream()),
              "mlstm_forward_gated_lx");
-    if (keep) {
-        node->save({q, k, v, f, i, t[5]});
-        node->h = h;
-        torch::autograd::set_history(hg, node);
-    }
+    node->save({q, k, v, f, i, t[5]});
+    node->h = h;
+    torch::autograd::set_history(hg, node);
     return true;
 }
 
@@ -326,9 +309,18 @@ struct Scan_mLSTMBackward : OpNode {
             in[n] = in[n].contiguous();
             res[n] = new_like(in[n]);
         }
+        if (c.on_tiles()) {
+            Buffer ws = c.workspace(MLSTM_OP_BACKWARD_GATED);
+            check_rc(mlstm::train_backward(dh.data_ptr(), in[0].data_ptr(), in[1].data_ptr(), in[2].data_ptr(), in[3].data_ptr(), in[4].data_ptr(),
+                                           in[5].data_ptr(), h_ungated.data_ptr(), kept.get(), kept.n, res[0].data_ptr(), res[1].data_ptr(), res[2].data_ptr(),
+                                           res[3].data_ptr(), res[4].data_ptr(), res[5].data_ptr(), c.B, c.NH, c.S, c.D, MLSTM_F32, MLSTM_F32, nullptr,
+                                           ws.get(), ws.n, hip_stream()),
+                     "mlstm_scan_backward_saved_ex");
+            return res;
+        }
         Buffer ws = c.workspace(MLSTM_OP_SCAN_BACKWARD);
         check_rc(mlstm_scan_backward_saved_ex(dh.data_ptr(), in[0].data_ptr(), in[1].data_ptr(), in[2].data_ptr(), in[3].data_ptr(), in[4].data_ptr(),
-                                              in[5].data_ptr(), h_ungated.data_ptr(), kept.b(), res[0].data_ptr(), res[1].data_ptr(), res[2].data_ptr(),
+                                              in[5].data_ptr(), h_ungated.data_ptr(), static_cast<float*>(kept.get()), res[0].data_ptr(), res[1].data_ptr(), res[2].data_ptr(),
                                               res[3].data_ptr(), res[4].data_ptr(), res[5].data_ptr(), c.B, c.NH, c.S, c.D, MLSTM_F32, ws.get(), ws.n,
                                               hip_stream()),
                  "mlstm_scan_backward_saved_ex");
@@ -352,8 +344,8 @@ bool scan(const Tensor* t, Tensor& h) {
         }
     }
     h = new_like(in[0]);
-    Buffer ws = c.workspace(MLSTM_OP_SCAN_FORWARD);
     if (!keep) {
+        Buffer ws = c.workspace(MLSTM_OP_SCAN_FORWARD);
         check_rc(mlstm_scan_forward_ex(in[0].data_ptr(), in[1].data_ptr(), in[2].data_ptr(), in[3].data_ptr(), in[4].data_ptr(), in[5].data_ptr(),
                                        h.data_ptr(), c.B, c.NH, c.S, c.D, MLSTM_F32, ws.get(), ws.n, hip_stream()),
                  "mlstm_scan_forward_ex");
@@ -361,12 +353,22 @@ bool scan(const Tensor* t, Tensor& h) {
     }
     auto node = make_node<Scan_mLSTMBackward>(t[0], t[1], t[2], t[3], t[4], t[5]);
     node->c = c;
-    node->kept.buf = Buffer(c.rows() * 4);   // (b alone, at offset 0)
     node->h_ungated = new_like(in[0]);
-    check_rc(mlstm_scan_forward_save_ex(in[0].data_ptr(), in[1].data_ptr(), in[2].data_ptr(), in[3].data_ptr(), in[4].data_ptr(), in[5].data_ptr(),
-                                        h.data_ptr(), node->h_ungated.data_ptr(), node->kept.b(), c.B, c.NH, c.S, c.D, MLSTM_F32, ws.get(), ws.n,
-                                        hip_stream()),
-             "mlstm_scan_forward_save_ex");
+    if (c.on_tiles()) {
+        node->kept = c.kept();
+        Buffer ws = c.workspace(MLSTM_OP_FORWARD_GATED);
+        check_rc(mlstm::train_forward(in[0].data_ptr(), in[1].data_ptr(), in[2].data_ptr(), in[3].data_ptr(), in[4].data_ptr(), in[5].data_ptr(),
+                                      node->h_ungated.data_ptr(), h.data_ptr(), node->kept.get(), node->kept.n, c.B, c.NH, c.S, c.D, MLSTM_F32, MLSTM_F32, nullptr,
+                                      ws.get(), ws.n, hip_stream()),
+                 "mlstm_scan_forward_save_ex");
+    } else {
+        node->kept = Buffer((size_t)c.B * c.NH * c.S * 4);   // the normaliser sums
+        Buffer ws = c.workspace(MLSTM_OP_SCAN_FORWARD);
+        check_rc(mlstm_scan_forward_save_ex(in[0].data_ptr(), in[1].data_ptr(), in[2].data_ptr(), in[3].data_ptr(), in[4].data_ptr(), in[5].data_ptr(),
+                                            h.data_ptr(), node->h_ungated.data_ptr(), static_cast<float*>(node->kept.get()), c.B, c.NH, c.S, c.D,
+                                            MLSTM_F32, ws.get(), ws.n, hip_stream()),
+                 "mlstm_scan_forward_save_ex");
+    }
     node->save({t[0], t[1], t[2], t[3], t[4], t[5]});
     torch::autograd::set_history(h, node);
     return true;
@@ -391,7 +393,7 @@ struct HIP_sLSTMBackward : OpNode {
         res[1] = new_like(r);
         res[2] = new_tensor(at::IntArrayRef(bs, 3), at::IntArrayRef(sb, 3), at::kFloat, h);
         Buffer ws(slstm_workspace_bytes(c.B, c.NH, c.S, c.D));
-        check_rc(slstm_backward_ex(dh.data_ptr<float>(), h.data_ptr<float>(), r.data_ptr<float>(), static_cast<const float*>(kept.saved()),
+        check_rc(slstm_backward_ex(dh.data_ptr<float>(), h.data_ptr<float>(), r.data_ptr<float>(), static_cast<const float*>(kept.get()),
                                    res[0].data_ptr<float>(), res[1].data_ptr<float>(), res[2].data_ptr<float>(), c.B, c.NH, c.S, c.D, forget_sigmoid,
                                    ws.get(), ws.n, hip_stream()),
                  "slstm_backward_ex");
@@ -416,11 +418,10 @@ bool slstm(const Tensor* t, int forget_sigmoid, Tensor& h) {
         node = make_node<HIP_sLSTMBackward>(wx, r, b);
         node->c = c;
         node->forget_sigmoid = forget_sigmoid;
-        node->kept.saved_bytes = slstm_saved_bytes(c.B, c.NH, c.S, c.D);
-        node->kept.buf = Buffer(node->kept.saved_bytes);
+        node->kept = Buffer(slstm_saved_bytes(c.B, c.NH, c.S, c.D));
     }
     check_rc(slstm_forward_ex(wx.data_ptr<float>(), r.data_ptr<float>(), b.data_ptr<float>(), h.data_ptr<float>(),
-                              keep ? static_cast<float*>(node->kept.saved()) : nullptr, c.B, c.NH, c.S, c.D, forget_sigmoid, hip_stream()),
+                              keep ? static_cast<float*>(node->kept.get()) : nullptr, c.B, c.NH, c.S, c.D, forget_sigmoid, hip_stream()),
              "slstm_forward_ex");
     if (keep) {
         node->save({r});
