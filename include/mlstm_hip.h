@@ -323,8 +323,8 @@ int mlstm_force_generic_kernels(int on);
 
 /*
  * Test and measurement aid with no counterpart in the reference.  The tile kernels (every type; D = 64, 128, and 256 in
- * 16 bits) cut sequences of 1024 positions and more (fp32: 320) into chunks -- 512 positions for the 16-bit types at
- * D = 128 / 256, 256 at D = 64, 128 for fp32 -- : a row walks the keys of its own chunk and takes everything
+ * 16 bits) cut long sequences into chunks -- the 16-bit types from about 1000 positions on, into 256 or 512 positions (D = 64:
+ * 128 or 256) by length and number of heads, fp32 from 320 on into 128 -- : a row walks the keys of its own chunk and takes everything
  * before it from the matrix state at the end of the previous chunk (the state of mlstm_scan.py:16-26; both forms are
  * the same function); the backward's keys likewise take the queries behind their chunk from a reverse state.  length > 0 (a multiple of 128) forces that chunk length, length < 0 switches chunking off,
  * 0 restores the default.  Process-wide; returns 0, or MLSTM_EINVAL for a length that is not a multiple of 128.
@@ -348,8 +348,8 @@ int mlstm_set_column_kernel(int variant);
  */
 int mlstm_set_state_kernel(int variant);
 /* The chunk length the entry points use for this shape under the current setting, 0 = the sequence is not cut
- * (measurement aid: the work a chunked kernel executes depends on it).  It speaks for sequences of 1024 positions and more;
- * below that fp32 sequences of at least 320 positions run in chunks of 128 as well, and 0 is returned for them. */
+ * (measurement aid: the work a chunked kernel executes depends on it).  It speaks for few heads and for sequences of 1024
+ * positions and more; shorter ones may run in chunks as well (fp32 from 320 positions on), and 0 is returned for them. */
 int mlstm_chunk_length_for(int S, int D, int dtype);
 
 /*
