@@ -149,6 +149,34 @@ template <> struct Tr<float> {
         return t;
     }
     static __device__ __forceinline__ terms split(const terms& t) { return t; }
+    // the same in five steps, for the gaps between MFMAs
+    struct Splitting {
+        float x[8];
+        bf16x2 p[4];
+        __device__ __forceinline__ void start(const frag& f) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) x[e] = f[e];
+        }
+        template <int I> __device__ __forceinline__ void step(terms& to) {
+            if constexpr (I % 2 == 0) {   // a term of every pair
+                bf16x8& t = I == 0 ? to.hi : (I == 2 ? to.mid : to.lo);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    p[e] = __builtin_convertvector(f32x2{x[2 * e], x[2 * e + 1]}, bf16x2);
+                    t[2 * e] = p[e][0];
+                    t[2 * e + 1] = p[e][1];
+                }
+            } else {                      // and what it leaves
+                int first_bits = 0x0000bf80, second_bits = (int)0xbf800000;   // (see split)
+                asm("" : "+s"(first_bits), "+s"(second_bits));
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    x[2 * e] = __builtin_amdgcn_fdot2_f32_bf16(p[e], __builtin_bit_cast(bf16x2, first_bits), x[2 * e], false);
+                    x[2 * e + 1] = __builtin_amdgcn_fdot2_f32_bf16(p[e], __builtin_bit_cast(bf16x2, second_bits), x[2 * e + 1], false);
+                }
+            }
+        }
+    };
     // the six products, smallest first, with something else between them (a vector instruction costs nothing while the matrix
     // unit works: six products keep it busy for 192 cycles, 48 instructions' worth)
     template <typename F>
@@ -181,30 +209,12 @@ template <> struct Tr<float> {
             constexpr int n = decltype(nc)::value;
             if constexpr (n + AHEAD + 1 < N) raw[(n + AHEAD + 1) % (AHEAD + 1)] = read(std::integral_constant<int, n + AHEAD + 1>{});
             terms next = cur;
-            float x[8];
-            bf16x2 p[4];
-            int first_bits = 0x0000bf80, second_bits = (int)0xbf800000;   // (see split)
-            asm("" : "+s"(first_bits), "+s"(second_bits));
+            Splitting sp;
             product(nc, cur, [&](auto ic) __attribute__((always_inline)) {
                 constexpr int i = decltype(ic)::value;
                 if constexpr (n + 1 < N) {
-                    if constexpr (i == 0) {
-#pragma unroll
-                        for (int e = 0; e < 8; e++) x[e] = raw[(n + 1) % (AHEAD + 1)][e];
-                    }
-                    if constexpr (i % 2 == 0) {   // a term of every pair
-#pragma unroll
-                        for (int e = 0; e < 4; e++) p[e] = __builtin_convertvector(f32x2{x[2 * e], x[2 * e + 1]}, bf16x2);
-                        bf16x8& t = i == 0 ? next.hi : (i == 2 ? next.mid : next.lo);
-#pragma unroll
-                        for (int e = 0; e < 4; e++) { t[2 * e] = p[e][0]; t[2 * e + 1] = p[e][1]; }
-                    } else {                      // and what it leaves
-#pragma unroll
-                        for (int e = 0; e < 4; e++) {
-                            x[2 * e] = __builtin_amdgcn_fdot2_f32_bf16(p[e], __builtin_bit_cast(bf16x2, first_bits), x[2 * e], false);
-                            x[2 * e + 1] = __builtin_amdgcn_fdot2_f32_bf16(p[e], __builtin_bit_cast(bf16x2, second_bits), x[2 * e + 1], false);
-                        }
-                    }
+                    if constexpr (i == 0) sp.start(raw[(n + 1) % (AHEAD + 1)]);
+                    sp.template step<i>(next);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             });

@@ -11,7 +11,7 @@
 //                       the chunk (the only place a q.k product is formed), its row sums, and the chunk's contribution
 //                       dn_c = sum_j exp(a_j - A_end) k_j / sqrt(D) to the vector state n~.
 //   scan_ncarry_kernel  n~ at every chunk end: n~_c = gamma_c n~_{c-1} + dn_c, in place, coalesced streaming.
-//   scan_state_kernel   one workgroup per (head, 32 value columns, key range) walks the chunks in order and keeps its
+//   scan_state_kernel   one workgroup per (head, value tile, key range) walks the chunks in order and keeps its
 //                       slice of C~ in MFMA accumulator registers for the whole sequence (the matrix carry never
 //                       leaves the chip): per chunk  num = decay_t (Q_c C~^T) + P_c V_c, then C~ = gamma C~ + (w V_c)^T K_c.
 //                       With more than one key range per value tile the partial numerators go to separate buffers.
@@ -183,15 +183,19 @@ __global__ __launch_bounds__(256) void scan_ncarry_kernel(ScanArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// The contraction over the 64 keys of a chunk runs in 32 MFMA steps; step s takes the keys {s, 32 + s} (lane half h
-// supplies key 32h + s), so that a lane's P operands and gate weights are contiguous in memory.  A wave's key columns
-// are interleaved over its NKB accumulator blocks (row rho of block kb is column kbase + NKB*rho + kb): one vector load
-// per key row then feeds all blocks.
-// Operands from memory are fetched one phase ahead into registers (one wave per SIMD has 512 of them): K of the chunk
-// before the read-out products, Q of the next chunk before the state update products.
-template <int N> struct FVec { typedef float type __attribute__((ext_vector_type(N))); };
-template <> struct FVec<1> { struct type { float x; __device__ float operator[](int) const { return x; } }; };
-
+// One workgroup: VT = 32 VB value columns, four waves of KPW = 32 NKB key columns each; a wave holds its [KPW x VT] piece of
+// C~ in accumulator registers.  The products are those of Tr<float>, three bf16 terms per operand: six 32x32x16 MFMAs per
+// block against eight 32x32x2 ones at twice the cycles, and the vector instructions of a split go between them.
+//
+// What bounds it: one wave per SIMD issues everything, about 1250 split instructions to 200 MFMAs per chunk (VB = NKB = 2),
+// so every operand is split as seldom as it can be.  64 value columns per workgroup and not 32 halve the splits (and the L2
+// traffic) of Q and K; a wave splits a quarter of the weighted values and the others read its terms from LDS; the state's
+// terms serve both query blocks.  Q comes with direct copies into a piece of LDS that belongs to the wave (its fragments want
+// one row per lane: 64 lines per load instruction from memory), K and V from memory into registers, 128 bytes per row.
+// Measured on 4 heads x 2048 x 1024, forward: 17,200 cycles per chunk (read-out 6400, update 5600) where the 32x32x2 kernel
+// took 27,900; whole call 393 -> 306 us.  Eight waves of half the tile each took 18,400: two waves per SIMD overlap splits and
+// MFMAs, and lose it again at twice the barriers.
+//
 // A sequence may also be cut into segments of seg_chunks chunks that run side by side (blockIdx.y), for the cases in
 // which heads x value tiles x key ranges alone leave most of the chip idle (one long sequence, small D):
 //   STATE_ONLY = true   every segment but the last walks its chunks from a zero state, updates only, and leaves the
@@ -200,19 +204,31 @@ template <> struct FVec<1> { struct type { float x; __device__ float operator[](
 //   STATE_ONLY = false  the walk proper: segment s > 0 starts from the state at the end of segment s - 1.
 // REV: q, k and v are walked from their last row (ScanArgs::rev).  A complete chunk's 64 rows then lie in front of the row of
 // its first position; the lane parts of the addresses stay non-negative by counting from the chunk's last position.
-template <int D, int KS, int NW, bool STATE_ONLY, bool REV>
-__global__ __launch_bounds__(NW * 64) void scan_state_kernel(ScanArgs a) {
-    constexpr int KPW = D / KS / NW, NKB = KPW / 32, NVT = D / 32;  // key columns per wave, in blocks of 32
-    constexpr int SH = 32 / (NW * KS);                              // in-chunk contraction steps per wave
-    static_assert(SH >= 1 && NW >= 1 && NW <= 8 && (NKB == 1 || NKB == 2 || NKB == 4) && NKB * 32 == KPW, "32, 64 or 128 key columns per wave");
-    using kvec = typename FVec<NKB>::type;
+constexpr int SCAN_NW = 4;   // waves per workgroup: one per SIMD, each wants the full register file
+template <int VB, int NKB> constexpr int scan_state_lds() {
+    return SCAN_NW * 64 * 32 * NKB * 4      // Q of a chunk, per wave
+         + SCAN_NW * 8 * VB * 64 * 16       // partial numerators
+         + 4 * VB * 3 * 64 * 16             // terms of the weighted values
+         + 3 * 2 * GRAN * 4;                // gate vectors
+}
+template <int D, int VB, int NKB, bool STATE_ONLY, bool REV>
+__global__ __launch_bounds__(SCAN_NW * 64) void scan_state_kernel(ScanArgs a) {
+    constexpr int NW = SCAN_NW, KPW = 32 * NKB, KS = D / KPW / NW, VT = 32 * VB, NVT = D / VT, NS = 2 * NKB;
+    static_assert(KS >= 1 && KS * NW * KPW == D && NVT * VT == D, "key ranges and value tiles must divide D");
+    typedef Tr<float> X;
+    typedef X::frag frag;
+    typedef X::terms terms;
+    typedef Swz<float, KPW> Z;
     extern __shared__ __align__(16) float lds[];
-    float (*red)[NW][32][64] = reinterpret_cast<float (*)[NW][32][64]>(lds);  // [chunk parity][wave][accumulator register][lane]
-    float (*sgate)[2][GRAN] = reinterpret_cast<float (*)[2][GRAN]>(lds + 2 * NW * 32 * 64);  // [chunk mod 3][0: key weights w_j, 1: query decays][position]
+    const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, c32 = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    float* const qst = lds + wave * 64 * KPW;                                      // [query][key column], swizzled
+    f32x4 (*red)[8 * VB][64] = reinterpret_cast<f32x4 (*)[8 * VB][64]>(lds + NW * 64 * KPW);   // [wave][(tb, vb, r / 4)][lane]
+    bf16x8 (*vterm)[VB][3][64] = reinterpret_cast<bf16x8 (*)[VB][3][64]>(lds + NW * 64 * KPW + NW * 8 * VB * 256);   // [16 positions][vb][term][lane]
+    float (*sgate)[2][GRAN] = reinterpret_cast<float (*)[2][GRAN]>(lds + NW * 64 * KPW + NW * 8 * VB * 256 + 4 * VB * 3 * 256);   // [chunk mod 3][0: key weights w_j, 1: query decays][position]
     const int bh = blockIdx.x % a.BH;
     const int rest = blockIdx.x / a.BH;
     const int vt = rest % NVT, ks = rest / NVT;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = lane >> 5, c32 = lane & 31;
     const int S = a.S, NC = a.NC;
     const int seg = blockIdx.y, c_begin = seg * a.seg_chunks, c_end = c_begin + a.seg_chunks < NC ? c_begin + a.seg_chunks : NC;
     const size_t hoff = (size_t)bh * S, poff = (size_t)bh * NC * GRAN;
@@ -221,215 +237,326 @@ __global__ __launch_bounds__(NW * 64) void scan_state_kernel(ScanArgs a) {
     const float* V = a.v + hoff * D;
     const double* G2 = a.G2 + (size_t)bh * NC;
     float* out = (ks == 0 ? a.h : a.hpart + (size_t)(ks - 1) * a.BH * S * D) + hoff * D;
-    const int kbase = (ks * NW + wave) * KPW, v0 = 32 * vt;
+    const int kbase = (ks * NW + wave) * KPW, v0 = VT * vt;
     const float log2scale = -0.5f * __log2f((float)D);
-    const int hrow = REV ? 32 * (1 - h) : 32 * h;         // the lane half's first row in a chunk's 64 rows as they lie in memory
+    // Position 16 s + 8 h + e of a chunk is contraction element e of lane half h in step s.
+    const int hrow = REV ? 8 * (1 - h) : 8 * h;           // the lane half's first row in 16 rows as they lie in memory
     const int v_lofs = hrow * D + v0 + c32;               // lane part of a value address (column v0 + c32)
-    const int k_lofs = hrow * D + kbase + NKB * c32;      // lane part of a key address
+    const int k_lofs = hrow * D + kbase + c32;            // lane part of a key address
     auto row_of = [&](int t) { return (size_t)(REV ? S - 1 - t : t); };   // the row that holds walk position t < S
+    auto row_in = [](int s, int e) { return (size_t)(REV ? 48 - 16 * s + 7 - e : 16 * s + e); };
 
     // Gate vectors of a chunk: weights of its keys, decays of its queries (from the previous chunk end).  The carried
     // state is kept as st = C~ / Gamma with a running power of two Gamma <= 1, so that the per-chunk decay gamma_c
     // multiplies into Gamma (folded into these vectors) and the registers are rescaled only when Gamma gets small.
-    constexpr int NI = (2 * GRAN + NW * 64 - 1) / (NW * 64);
     float lg = 0.f;  // log2 Gamma for the read-out of the next chunk to prepare
-    struct Gates { float x[NI]; float dec_add, w_add, rescale; };
-    auto gates_fetch = [&](int c) {  // the loads, and the scalars (identical in all lanes)
+    struct Gates { float x, bprev, bend; double g, gprev; };
+    int vzero = 0;   // (as vector loads: a scalar load in flight would make every wait for LDS a wait for it)
+    asm volatile("" : "+v"(vzero));
+    const float* const mygate = (tid < GRAN ? a.alpha2 : a.beta2) + poff + (tid & (GRAN - 1));
+    auto gates_fetch = [&](int c) {
         Gates g;
         const int cp = c > 0 ? c - 1 : 0;
-        const float bprev = a.beta2[poff + GRAN * cp + GRAN - 1], bend = a.beta2[poff + GRAN * c + GRAN - 1];
-        const float dG = (float)(G2[c] - G2[cp]);
-        const float lgam = c > 0 ? bprev - bend + dG : 0.f;
-        g.dec_add = c > 0 ? bprev + dG + lg : 0.f;
-        float lnew = lg + lgam;
-        g.rescale = 0.f;
-        if (lnew < -24.f) { g.rescale = lnew; lnew = 0.f; }
-        g.w_add = log2scale - bend - lnew;
-        lg = lnew;
-#pragma unroll
-        for (int n = 0; n < NI; n++) {
-            const int i = tid + n * NW * 64, pos = i & (GRAN - 1);
-            g.x[n] = i < GRAN ? a.alpha2[poff + GRAN * c + pos] : (i < 2 * GRAN ? a.beta2[poff + GRAN * c + pos] : 0.f);
-        }
+        g.bprev = a.beta2[poff + GRAN * cp + GRAN - 1 + vzero];
+        g.bend = a.beta2[poff + GRAN * c + GRAN - 1 + vzero];
+        g.g = G2[c + vzero];
+        g.gprev = G2[cp + vzero];
+        g.x = tid < 2 * GRAN ? mygate[(size_t)GRAN * c] : 0.f;
         return g;
     };
-    auto gates_store = [&](int c, const Gates& g) {
+    auto gates_store = [&](int c, const Gates& g) {   // returns the rescale before this chunk's update (0: none)
+        const float dG = (float)(g.g - g.gprev);
+        const float dec_add = g.bprev + dG + lg;
+        float lnew = lg + (c > 0 ? g.bprev - g.bend + dG : 0.f), rescale = 0.f;
+        if (lnew < -24.f) { rescale = lnew; lnew = 0.f; }
+        const float w_add = log2scale - g.bend - lnew;
+        lg = lnew;
+        const int pos = tid & (GRAN - 1);
+        if (tid < GRAN) sgate[c % 3][0][pos] = fast_exp2(g.x + w_add);
+        else if (tid < 2 * GRAN) sgate[c % 3][1][pos] = c > 0 ? fast_exp2(dec_add - g.x) : 1.0f;
+        return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, rescale)));
+    };
+    // Q of a chunk into the wave's LDS (rows clamped: the chunk may be the partial one)
+    const unsigned qst_off = __builtin_amdgcn_readfirstlane(lds_offset_of(qst));
+    constexpr int RPI = 64 / Z::CPR, QI = 64 / RPI, QP = 16 / RPI;   // rows per copy instruction, instructions, period of the swizzle key
+    unsigned q_lofs[QP];               // lane part of the source, in bytes
 #pragma unroll
-        for (int n = 0; n < NI; n++) {
-            const int i = tid + n * NW * 64, pos = i & (GRAN - 1);
-            if (i < GRAN) sgate[c % 3][0][pos] = fast_exp2(g.x[n] + g.w_add);
-            else if (i < 2 * GRAN) sgate[c % 3][1][pos] = c > 0 ? fast_exp2(g.dec_add - g.x[n]) : 1.0f;
+    for (int i = 0; i < QP; i++)
+        q_lofs[i] = (unsigned)(((REV ? RPI - 1 - lane / Z::CPR : lane / Z::CPR) * D + 4 * ((lane % Z::CPR) ^ Z::key(RPI * i + lane / Z::CPR))) * 4);
+    auto fetch_q_part = [&](int c, int part) {   // a quarter of a complete chunk
+        const float* base = Q + (REV ? (size_t)(S - GRAN - GRAN * c) : (size_t)(GRAN * c)) * D + kbase;
+#pragma unroll
+        for (int j = 0; j < QI / 4; j++) {
+            const int i = part * (QI / 4) + j;
+            dma16_s(base + (size_t)(REV ? GRAN - RPI - RPI * i : RPI * i) * D, q_lofs[i % QP], qst_off, 1024 * i);
         }
     };
-
-    f32x16 st[NKB];  // st[kb][r] = C~[v = v0 + c32][k = kbase + NKB*(8*(r/4) + 4h + r%4) + kb]
-    // a workgroup's state in seg_state: [segment][workgroup][wave][kb][r][lane]
-    const size_t seg_stride = (size_t)gridDim.x * NW * NKB * 16 * 64;
-    float* const seg_mine = a.seg_state + ((size_t)blockIdx.x * NW + wave) * NKB * 16 * 64 + lane;
-#pragma unroll
-    for (int kb = 0; kb < NKB; kb++)
-#pragma unroll
-        for (int r = 0; r < 16; r++) st[kb][r] = (!STATE_ONLY && seg > 0) ? seg_mine[(size_t)(seg - 1) * seg_stride + (kb * 16 + r) * 64] : 0.f;
-    kvec qreg[2][4][4];  // [query block][x][e]: Q[t][kbase + NKB*(8x + 4h + e) + 0..NKB-1]
-    auto load_q = [&](int c, int tb, int x, int e) {  // (row clamped: the chunk may be the partial one)
-        int t = GRAN * c + 32 * tb + c32;
-        t = t < S ? t : S - 1;
-        qreg[tb][x][e] = *reinterpret_cast<const kvec*>(Q + row_of(t) * D + kbase + 4 * NKB * h + NKB * (8 * x + e));
+    auto fetch_q_clamped = [&](int c) {
+#pragma unroll 1
+        for (int i = 0; i < QI; i++) {
+            const int r = RPI * i + lane / Z::CPR;
+            const int t = GRAN * c + r < S ? GRAN * c + r : S - 1;
+            dma16(Q + row_of(t) * D + kbase + 4 * ((lane % Z::CPR) ^ Z::key(r)), __builtin_amdgcn_readfirstlane(qst_off + 1024 * i));
+        }
     };
-    if constexpr (!STATE_ONLY) {
+    auto read_q = [&](int s, int tb) {   // key columns 16 s + 8 x + 4 h + e' of row 32 tb + c32, the order of from_acc
+        const char* base = reinterpret_cast<const char*>(qst);
+        const f32x4 x0 = *reinterpret_cast<const f32x4*>(base + Z::off(32 * tb + c32, 16 * s + 4 * h));
+        const f32x4 x1 = *reinterpret_cast<const f32x4*>(base + Z::off(32 * tb + c32, 16 * s + 8 + 4 * h));
+        return __builtin_shufflevector(x0, x1, 0, 1, 2, 3, 4, 5, 6, 7);
+    };
+
+    f32x16 st[NKB][VB];  // st[kb][vb][r] = C~[v = v0 + 32 vb + c32][k = kbase + 32 kb + 8*(r/4) + 4h + r%4]
+    // a workgroup's state in seg_state: [segment][workgroup][wave][kb][vb][r][lane]
+    const size_t seg_stride = (size_t)gridDim.x * NW * NKB * VB * 16 * 64;
+    float* const seg_mine = a.seg_state + ((size_t)blockIdx.x * NW + wave) * NKB * VB * 16 * 64 + lane;
 #pragma unroll
-        for (int i = 0; i < 32; i++) load_q(c_begin, i & 1, i >> 3, (i >> 1) & 3);
+    for (int b = 0; b < NKB * VB; b++)
+#pragma unroll
+        for (int r = 0; r < 16; r++) st[b / VB][b % VB][r] = 0.f;
+    if (!STATE_ONLY && seg > 0) {
+#pragma unroll
+        for (int b = 0; b < NKB * VB; b++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) st[b / VB][b % VB][r] = seg_mine[(size_t)(seg - 1) * seg_stride + (b * 16 + r) * 64];
     }
-    float rescale_cur;
+    if constexpr (!STATE_ONLY) fetch_q_clamped(c_begin);
     float lg_done = 0.f;   // log2 Gamma of the last chunk whose update is in st
-    {
-        const Gates g0 = gates_fetch(c_begin);
-        gates_store(c_begin, g0);
-        rescale_cur = g0.rescale;
-    }
+    float rescale_cur = gates_store(c_begin, gates_fetch(c_begin));
     __syncthreads();
 
-    // One chunk.  The memory operations are spread between the groups of matrix instructions that cover them (a wave
-    // issues in order, and four waves share the CU's one address path: a burst of loads would idle the matrix unit):
-    // values, pair weights and keys of this chunk during the read-out products, the next chunk's queries during the
-    // state update.  LAST: the final chunk of the sequence (possibly partial: rows clamped; no state update follows).
+    // One chunk.  LAST: the final chunk of a walk (possibly partial: rows clamped; no state update follows).
     auto chunk = [&](const int c, auto last_tag) {
         constexpr bool LAST = decltype(last_tag)::value;
         const int t0 = GRAN * c;
         const float* sw = sgate[c % 3][0];
         const float* sdec = sgate[c % 3][1];
-        float vraw[32];
-        float pa[2][SH];
-        float vin[SH];  // this wave's values for the in-chunk products (a register array takes no wave-dependent index)
-        kvec kreg[32];
         // uniform: the first of the chunk's 64 rows in memory (REV: the row of its last position; only complete chunks use it)
         const size_t r0 = LAST ? 0 : (REV ? (size_t)(S - GRAN - t0) : (size_t)t0);
         const float* vrow = V + r0 * D;
         const float* krow = K + r0 * D;
-        auto load_v = [&](int s) {   // position t0 + 32h + s
-            if constexpr (LAST) {
-                int j = t0 + 32 * h + s;
-                j = j < S ? j : S - 1;
-                vraw[s] = V[row_of(j) * D + v0 + c32];
-            } else {
-                vraw[s] = (vrow + (size_t)(REV ? 31 - s : s) * D)[v_lofs];
-            }
+        frag vraw[VB];          // this wave's 16 positions of the values (step `wave`)
+        frag kraw[4][NKB];
+        auto load_v = [&]() {
+#pragma unroll
+            for (int vb = 0; vb < VB; vb++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    if constexpr (LAST) {
+                        int j = t0 + 16 * wave + 8 * h + e;
+                        j = j < S ? j : S - 1;
+                        vraw[vb][e] = V[row_of(j) * D + v0 + 32 * vb + c32];
+                    } else {
+                        vraw[vb][e] = (vrow + row_in(wave, e) * D + 32 * vb)[v_lofs];
+                    }
+                }
         };
-        auto load_k = [&](int s) { kreg[s] = *reinterpret_cast<const kvec*>(krow + (size_t)(REV ? 31 - s : s) * D + k_lofs); };
-        // ---- read-out of the carried state: acc[tb] = decay_t * Q_c[32 tb.., k-range of this wave] . C~^T
-        f32x16 acc[2];
+        auto load_k = [&](int s) {
 #pragma unroll
-        for (int tb = 0; tb < 2; tb++)
+            for (int kb = 0; kb < NKB; kb++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) acc[tb][r] = 0.f;
+                for (int e = 0; e < 8; e++) kraw[s][kb][e] = (krow + row_in(s, e) * D + 32 * kb)[k_lofs];
+        };
+        // The pairs inside the chunk: 2 VB blocks of P V with four steps each, step `wave` of block (tb, vb) in key range
+        // (tb + 2 vb) mod KS.
+        auto pair_mine = [&](int tb, int vb) { return KS == 1 || (tb + 2 * vb) % KS == ks; };
+        frag praw[2];
+        if constexpr (!STATE_ONLY) {
+            dma_wait();   // Q of this chunk
+            const float* Pc = a.P + ((size_t)bh * NC + c) * GRAN * GRAN + 16 * wave + 8 * h;
+#pragma unroll
+            for (int tb = 0; tb < 2; tb++) praw[tb] = *reinterpret_cast<const frag*>(Pc + (32 * tb + c32) * GRAN);
+        }
+        load_v();
         Gates gn;
         lg_done = lg;
         if constexpr (!LAST) gn = gates_fetch(c + 1);
-        // the in-chunk products are split over all waves of all key ranges: SH contraction steps each
-        const int s0 = (ks * NW + wave) * SH;
-        auto load_p = [&]() {
-            const float* Pc = a.P + ((size_t)bh * NC + c) * GRAN * GRAN + 32 * h + s0;
-            using pvec = typename FVec<(SH < 4 ? SH : 4)>::type;
+
+        // N splits, step by step in the gaps of PN products: 5 PN gaps of 5 N steps
+        X::Splitting sp;
+        auto gap = [&](auto n_tag, auto pn_tag, auto g_tag, auto&& src, auto&& dst) __attribute__((always_inline)) {
+            constexpr int N = decltype(n_tag)::value, PN = decltype(pn_tag)::value, g = decltype(g_tag)::value;
+            constexpr int i0 = g * N / PN, i1 = (g + 1) * N / PN;
+            static_for<i1 - i0>([&](auto d) __attribute__((always_inline)) {
+                constexpr int job = (i0 + d) / 5, step = (i0 + d) % 5;
+                if constexpr (step == 0) sp.start(src(std::integral_constant<int, job>{}));
+                sp.template step<step>(dst(std::integral_constant<int, job>{}));
+            });
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        terms kt[2][NKB];
+        if constexpr (STATE_ONLY) {
 #pragma unroll
-            for (int tb = 0; tb < 2; tb++)
+            for (int s = 0; s < 4; s++) load_k(s);
 #pragma unroll
-                for (int x = 0; x < (SH + 3) / 4; x++) {
-                    const pvec pv = *reinterpret_cast<const pvec*>(Pc + (32 * tb + c32) * GRAN + 4 * x);
+            for (int kb = 0; kb < NKB; kb++) kt[0][kb] = X::split(kraw[0][kb]);
+        }
+        terms vt_mine[VB];   // this wave's share of the weighted values
+        auto weighted = [&](int vb) {
+            const f32x4 w0 = *reinterpret_cast<const f32x4*>(sw + 16 * wave + 8 * h), w1 = *reinterpret_cast<const f32x4*>(sw + 16 * wave + 8 * h + 4);
+            return vraw[vb] * __builtin_shufflevector(w0, w1, 0, 1, 2, 3, 4, 5, 6, 7);
+        };
+        if constexpr (STATE_ONLY) {
 #pragma unroll
-                    for (int e = 0; e < (SH < 4 ? SH : 4); e++) pa[tb][4 * x + e] = pv[e];
+            for (int vb = 0; vb < VB; vb++) vt_mine[vb] = X::split(weighted(vb));
+        }
+        const bool next_full = t0 + 2 * GRAN <= S;
+        // ---- read-out of the carried state: acc[tb][vb] = decay_t * Q_c[32 tb.., k-range of this wave] . C~^T
+        f32x16 acc[2][VB];
+        if constexpr (!STATE_ONLY) {
+#pragma unroll
+            for (int b = 0; b < 2 * VB; b++)
+#pragma unroll
+                for (int r = 0; r < 16; r++) acc[b / VB][b % VB][r] = 0.f;
+            terms qt[2][2], ct[2][VB];
+            frag qraw[2];
+#pragma unroll
+            for (int tb = 0; tb < 2; tb++) qraw[tb] = read_q(0, tb);
+#pragma unroll
+            for (int vb = 0; vb < VB; vb++) ct[0][vb] = X::split(X::from_acc(st[0][vb], 0));
+#pragma unroll
+            for (int tb = 0; tb < 2; tb++) qt[0][tb] = X::split(qraw[tb]);
+            static_for<NS>([&](auto s_tag) __attribute__((always_inline)) {
+                constexpr int s = decltype(s_tag)::value, PN = 2 * VB;
+                constexpr bool more = s + 1 < NS;
+                if constexpr (more) {
+#pragma unroll
+                    for (int tb = 0; tb < 2; tb++) qraw[tb] = read_q(s + 1, tb);
                 }
-        };
-        auto load_vin = [&]() {
+                if constexpr (!LAST) {
 #pragma unroll
-            for (int s = 0; s < SH; s++) {
-                int j = t0 + 32 * h + s0 + s;
-                if constexpr (LAST) j = j < S ? j : S - 1;
-                vin[s] = V[row_of(j) * D + v0 + c32];
-            }
-        };
-#pragma unroll
-        for (int g = 0; g < 16; g++) {  // g = 4x + e
-            if constexpr (!STATE_ONLY) {
-                if (g == 0) load_p();
-                if (g == 1) load_vin();
-            }
-            load_v(2 * g);
-            load_v(2 * g + 1);
-            if constexpr (!LAST) {
-                load_k(2 * g);
-                load_k(2 * g + 1);
-            }
-            if constexpr (!STATE_ONLY) {
-#pragma unroll
-                for (int kb = 0; kb < NKB; kb++) {
-                    acc[0] = mma_f32(qreg[0][g >> 2][g & 3][kb], st[kb][g], acc[0]);
-                    acc[1] = mma_f32(qreg[1][g >> 2][g & 3][kb], st[kb][g], acc[1]);
+                    for (int i = 0; i < 4 / NS; i++) load_k(s * (4 / NS) + i);
                 }
                 __builtin_amdgcn_sched_barrier(0);
+                static_for<PN>([&](auto p_tag) __attribute__((always_inline)) {
+                    constexpr int p = decltype(p_tag)::value, tb = p / VB, vb = p % VB;
+                    if constexpr (!more && !LAST) {   // (this wave's reads of its piece are over: queries of the next chunk)
+                        if (next_full) {
+#pragma unroll
+                            for (int j = 0; j < 4 / PN; j++) fetch_q_part(c + 1, p * (4 / PN) + j);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    X::mma_between(acc[tb][vb], qt[s & 1][tb], ct[s & 1][vb], [&](auto i_tag) __attribute__((always_inline)) {
+                        typedef std::integral_constant<int, 5 * p + decltype(i_tag)::value> G;
+                        typedef std::integral_constant<int, PN> P;
+                        if constexpr (more)   // the next step's state and queries
+                            gap(std::integral_constant<int, VB + 2>{}, P{}, G{},
+                                [&](auto j) __attribute__((always_inline)) {
+                                    if constexpr (j < VB) return X::from_acc(st[(s + 1) / 2][j < VB ? (int)j : 0], (s + 1) % 2);
+                                    else return qraw[j - VB];
+                                },
+                                [&](auto j) __attribute__((always_inline)) -> terms& {
+                                    if constexpr (j < VB) return ct[(s + 1) & 1][j < VB ? (int)j : 0];
+                                    else return qt[(s + 1) & 1][j - VB];
+                                });
+                        else if constexpr (!LAST)   // the first keys of the update and the weighted values
+                            gap(std::integral_constant<int, NKB + VB>{}, P{}, G{},
+                                [&](auto j) __attribute__((always_inline)) {
+                                    if constexpr (j < NKB) return kraw[0][j < NKB ? (int)j : 0];
+                                    else return weighted(j - NKB);
+                                },
+                                [&](auto j) __attribute__((always_inline)) -> terms& {
+                                    if constexpr (j < NKB) return kt[0][j < NKB ? (int)j : 0];
+                                    else return vt_mine[j - NKB];
+                                });
+                    });
+                });
+            });
+            if constexpr (!LAST) {
+                if (!next_full) fetch_q_clamped(c + 1);
             }
-        }
-        if constexpr (!STATE_ONLY) {
 #pragma unroll
             for (int tb = 0; tb < 2; tb++)
 #pragma unroll
                 for (int x = 0; x < 4; x++) {
                     const f32x4 dec = *reinterpret_cast<const f32x4*>(sdec + 32 * tb + 8 * x + 4 * h);
 #pragma unroll
-                    for (int e = 0; e < 4; e++) acc[tb][4 * x + e] *= dec[e];
+                    for (int vb = 0; vb < VB; vb++)
+#pragma unroll
+                        for (int e = 0; e < 4; e++) acc[tb][vb][4 * x + e] *= dec[e];
                 }
-            // ---- pairs inside the chunk: acc += P_c[:, this wave's keys] . V_c
+            // ---- pairs inside the chunk: acc += P_c[:, 16 wave ..] . V_c
 #pragma unroll
-            for (int s = 0; s < SH; s++) {
-                acc[0] = mma_f32(pa[0][s], vin[s], acc[0]);
-                acc[1] = mma_f32(pa[1][s], vin[s], acc[1]);
-            }
-            // ---- sum the partial numerators of the waves and store them (unnormalised)
+            for (int vb = 0; vb < VB; vb++)
 #pragma unroll
-            for (int tb = 0; tb < 2; tb++)
-#pragma unroll
-                for (int r = 0; r < 16; r++) red[c & 1][wave][16 * tb + r][lane] = acc[tb][r];
+                for (int tb = 0; tb < 2; tb++)
+                    if (pair_mine(tb, vb)) X::mma(acc[tb][vb], praw[tb], vraw[vb]);
         }
-        if constexpr (!LAST) gates_store(c + 1, gn);
-        // The only barrier of a chunk.  Between two barriers a wave is in the tail of one chunk or the head of the next:
-        // the partial sums alternate between two buffers, the gate vectors (written a chunk ahead) between three.
+        // ---- terms of the weighted values, partial numerators of the waves and the next gates, for all waves.  The first
+        // barrier: everybody is done with those of the chunk before.
+        float rescale_next = 0.f;
         __syncthreads();
-        auto sum_store = [&](int idx) {  // one accumulator register of the numerator: sum over the waves, store
-            float sum = 0.f;
+        if constexpr (!LAST) {
 #pragma unroll
-            for (int w = 0; w < NW; w++) sum += red[c & 1][w][idx][lane];
-            const int tl = 32 * (idx >> 4) + 8 * ((idx & 15) >> 2) + 4 * h + (idx & 3);
-            const int t = t0 + tl;
-            if (!LAST || t < S) out[(size_t)t * D + v0 + c32] = sum;
+            for (int vb = 0; vb < VB; vb++) {
+                vterm[wave][vb][0][lane] = vt_mine[vb].hi;
+                vterm[wave][vb][1][lane] = vt_mine[vb].mid;
+                vterm[wave][vb][2][lane] = vt_mine[vb].lo;
+            }
+            rescale_next = gates_store(c + 1, gn);
+        }
+        if constexpr (!STATE_ONLY) {
+#pragma unroll
+            for (int g = 0; g < 8 * VB; g++) {
+                const f32x16& x = acc[g / (4 * VB)][g / 4 % VB];
+                const int r = 4 * (g % 4);
+                red[wave][g][lane] = f32x4{x[r], x[r + 1], x[r + 2], x[r + 3]};
+            }
+        }
+        __syncthreads();
+        f32x4 part[NW];
+        auto sum_read = [&](int g) {   // four rows of the numerator: the waves' parts ...
+#pragma unroll
+            for (int w = 0; w < NW; w++) part[w] = red[w][g][lane];
+        };
+        auto sum_store = [&](int g) {  // ... their sum
+            f32x4 sum = part[0];
+#pragma unroll
+            for (int w = 1; w < NW; w++) sum += part[w];
+            const int t = t0 + 32 * (g / (4 * VB)) + 8 * (g % 4) + 4 * h;
+            float* o = out + (size_t)t * D + v0 + 32 * (g / 4 % VB) + c32;
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+                if (!LAST || t + e < S) o[e * D] = sum[e];
         };
         if constexpr (LAST) {
-            for (int idx = wave; idx < 32; idx += NW) sum_store(idx);
+            for (int g = wave; g < 8 * VB; g += NW) { sum_read(g); sum_store(g); }
         } else {
             // ---- state update: st += (w V_c)^T K_c (the weights carry 1/Gamma), rescaled first when Gamma got small
             if (rescale_cur != 0.f) {
                 const float f = fast_exp2(rescale_cur);
 #pragma unroll
-                for (int kb = 0; kb < NKB; kb++)
+                for (int b = 0; b < NKB * VB; b++)
 #pragma unroll
-                    for (int r = 0; r < 16; r++) st[kb][r] *= f;
+                    for (int r = 0; r < 16; r++) st[b / VB][b % VB][r] *= f;
             }
-            rescale_cur = gn.rescale;
-            __builtin_amdgcn_sched_barrier(0);
+            rescale_cur = rescale_next;
+            terms vt_s[2][VB];
+            auto read_v = [&](int s, terms (&t)[VB]) {
 #pragma unroll
-            for (int x = 0; x < 8; x++) {
-                const f32x4 w4 = *reinterpret_cast<const f32x4*>(sw + 32 * h + 4 * x);
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    const int i = 4 * x + e;
-                    if constexpr (!STATE_ONLY) {
-                        load_q(c + 1, i & 1, i >> 3, (i >> 1) & 3);
-                        if (i < 32 / NW) sum_store(wave + NW * i);
+                for (int vb = 0; vb < VB; vb++) t[vb] = terms{vterm[s][vb][0][lane], vterm[s][vb][1][lane], vterm[s][vb][2][lane]};
+            };
+            read_v(0, vt_s[0]);
+            static_for<4>([&](auto s_tag) __attribute__((always_inline)) {
+                constexpr int s = decltype(s_tag)::value, PN = NKB * VB;
+                if constexpr (s < 3) read_v(s + 1, vt_s[(s + 1) & 1]);
+                if constexpr (!STATE_ONLY && s < 2 * VB) sum_read(wave + NW * s);
+                __builtin_amdgcn_sched_barrier(0);
+                static_for<PN>([&](auto p_tag) __attribute__((always_inline)) {
+                    constexpr int p = decltype(p_tag)::value, kb = p / VB, vb = p % VB;
+                    X::mma_between(st[kb][vb], kt[s & 1][kb], vt_s[s & 1][vb], [&](auto i_tag) __attribute__((always_inline)) {
+                        if constexpr (s < 3)
+                            gap(std::integral_constant<int, NKB>{}, std::integral_constant<int, PN>{}, std::integral_constant<int, 5 * p + decltype(i_tag)::value>{},
+                                [&](auto j) __attribute__((always_inline)) { return kraw[s + 1][j]; },
+                                [&](auto j) __attribute__((always_inline)) -> terms& { return kt[(s + 1) & 1][j]; });
+                    });
+                    if constexpr (!STATE_ONLY && s < 2 * VB && p == PN / 2) {
+                        sum_store(wave + NW * s);
+                        __builtin_amdgcn_sched_barrier(0);
                     }
-                    const float wv = vraw[i] * w4[e];
-#pragma unroll
-                    for (int kb = 0; kb < NKB; kb++) st[kb] = mma_f32(kreg[i][kb], wv, st[kb]);  // rows = k, columns = v
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
+                });
+            });
         }
     };
     if constexpr (STATE_ONLY) {
@@ -437,9 +564,9 @@ __global__ __launch_bounds__(NW * 64) void scan_state_kernel(ScanArgs a) {
         for (int c = c_begin; c < c_end; c++) chunk(c, std::false_type{});
         const float f = fast_exp2(lg_done);   // st = C~ / Gamma
 #pragma unroll
-        for (int kb = 0; kb < NKB; kb++)
+        for (int b = 0; b < NKB * VB; b++)
 #pragma unroll
-            for (int r = 0; r < 16; r++) seg_mine[(size_t)seg * seg_stride + (kb * 16 + r) * 64] = st[kb][r] * f;
+            for (int r = 0; r < 16; r++) seg_mine[(size_t)seg * seg_stride + (b * 16 + r) * 64] = st[b / VB][b % VB][r] * f;
     } else {
         for (int c = c_begin; c + 1 < c_end; c++) chunk(c, std::false_type{});
         chunk(c_end - 1, std::true_type{});
@@ -549,28 +676,35 @@ __global__ __launch_bounds__(256) void scan_finish_kernel(ScanArgs a, int KS) {
     }
 }
 
-template <int D, int KS, int NW, bool REV>
+template <int D, int VB, int NKB, bool REV>
 static void launch_state(const ScanArgs& a, hipStream_t st) {
-    if constexpr ((D / KS / NW == 32 || D / KS / NW == 64 || D / KS / NW == 128) && NW * KS <= 32) {
-        constexpr int lds_bytes = (2 * NW * 32 * 64 + 3 * 2 * GRAN) * 4;
-        // (a failure here shows up as a launch error, which the caller reads with hipGetLastError)
-        (void)lds_limit_once<scan_state_kernel<D, KS, NW, false, REV>>(lds_bytes);
-        const int wgs = a.BH * (D / 32) * KS;
-        if (a.nseg > 1) {
-            (void)lds_limit_once<scan_state_kernel<D, KS, NW, true, REV>>(lds_bytes);
-            hipLaunchKernelGGL((scan_state_kernel<D, KS, NW, true, REV>), dim3(wgs, a.nseg - 1), dim3(NW * 64), lds_bytes, st, a);
-            const size_t elems = (size_t)wgs * NW * (D / KS / NW / 32) * 16 * 64;   // = BH * D * D
-            hipLaunchKernelGGL(scan_segcarry_kernel, dim3((unsigned)((elems + 255) / 256)), dim3(256), 0, st, a, elems,
-                               NW * (D / KS / NW / 32) * 16 * 64);
-        }
-        hipLaunchKernelGGL((scan_state_kernel<D, KS, NW, false, REV>), dim3(wgs, a.nseg), dim3(NW * 64), lds_bytes, st, a);
+    constexpr int lds_bytes = scan_state_lds<VB, NKB>(), wg_elems = SCAN_NW * NKB * VB * 16 * 64;
+    // (a failure here shows up as a launch error, which the caller reads with hipGetLastError)
+    (void)lds_limit_once<scan_state_kernel<D, VB, NKB, false, REV>>(lds_bytes);
+    const int wgs = a.BH * (D / (32 * VB)) * (D / (32 * NKB * SCAN_NW));
+    if (a.nseg > 1) {
+        (void)lds_limit_once<scan_state_kernel<D, VB, NKB, true, REV>>(lds_bytes);
+        hipLaunchKernelGGL((scan_state_kernel<D, VB, NKB, true, REV>), dim3(wgs, a.nseg - 1), dim3(SCAN_NW * 64), lds_bytes, st, a);
+        const size_t elems = (size_t)wgs * wg_elems;   // = BH * D * D
+        hipLaunchKernelGGL(scan_segcarry_kernel, dim3((unsigned)((elems + 255) / 256)), dim3(256), 0, st, a, elems, wg_elems);
     }
+    hipLaunchKernelGGL((scan_state_kernel<D, VB, NKB, false, REV>), dim3(wgs, a.nseg), dim3(SCAN_NW * 64), lds_bytes, st, a);
 }
 
-template <int D, int KS>
-static void launch_state_w(const ScanArgs& a, hipStream_t st) {
-    if (a.rev) launch_state<D, KS, 4, true>(a, st);
-    else launch_state<D, KS, 4, false>(a, st);
+template <int D, int VB, int NKB>
+static void launch_state_r(const ScanArgs& a, hipStream_t st) {
+    if (a.rev) launch_state<D, VB, NKB, true>(a, st);
+    else launch_state<D, VB, NKB, false>(a, st);
+}
+
+// Tile of a wave in blocks of 32: 64 value x 64 key columns while that gives every CU a workgroup, otherwise half of the key
+// columns, otherwise half of the value columns too.
+struct ScanTile { int vb, nkb; };
+static ScanTile scan_tile(int BH, int D) {
+    const int wgs = BH * (D / 64) * (D / 256);
+    if (wgs >= 256) return {2, 2};
+    if (2 * wgs >= 256) return {2, 1};
+    return {1, 1};
 }
 
 template <int D>
@@ -580,10 +714,10 @@ static int launch_scan_d(const ScanArgs& a, int KS, hipStream_t st, void (*mark)
     if (a.finish_mode != 2 || a.ep.vec) hipLaunchKernelGGL(scan_ncarry_kernel, dim3((D + 255) / 256, a.BH), dim3(256), 0, st, a);
     mark(MLSTM_K_SCAN_CARRY, st, false);
     mark(MLSTM_K_SCAN_STATE, st, true);
-    if (KS == 8) launch_state_w<D, 8>(a, st);
-    else if (KS == 4) launch_state_w<D, 4>(a, st);
-    else if (KS == 2) launch_state_w<D, 2>(a, st);
-    else launch_state_w<D, 1>(a, st);
+    const ScanTile tile = scan_tile(a.BH, D);
+    if (tile.nkb == 2) launch_state_r<D, 2, 2>(a, st);
+    else if (tile.vb == 2) launch_state_r<D, 2, 1>(a, st);
+    else launch_state_r<D, 1, 1>(a, st);
     mark(MLSTM_K_SCAN_STATE, st, false);
     mark(MLSTM_K_SCAN_OUT, st, true);
     const size_t rows = (size_t)a.BH * a.S;
@@ -598,17 +732,12 @@ void launch_scan_ncarry(const ScanArgs& a, hipStream_t st) {
 }
 
 // Key ranges per value tile.
-int scan_key_splits(int BH, int D) {
-    const int nw = 4;                          // waves per workgroup: one per SIMD (each wants the full register file)
-    int ks = D / nw > 128 ? D / nw / 128 : 1;  // at most 128 key columns per wave
-    while (D / ks / nw > 32 && BH * (D / 32) * ks < 256) ks *= 2;  // at least one workgroup per CU where D allows
-    return ks;
-}
+int scan_key_splits(int BH, int D) { return D / (32 * SCAN_NW * scan_tile(BH, D).nkb); }
 
 // Segments of a sequence that run side by side: none while heads x value tiles x key ranges fill the chip; otherwise
 // enough for about two workgroups per CU, of at least eight chunks each.
 void scan_segments(int BH, int S, int D, int* nseg, int* seg_chunks) {
-    const int NC = (S + GRAN - 1) / GRAN, wgs = BH * (D / 32) * scan_key_splits(BH, D);
+    const int NC = (S + GRAN - 1) / GRAN, wgs = BH * (D / (32 * scan_tile(BH, D).vb)) * scan_key_splits(BH, D);
     int n = 1;
     if (wgs < 256) {
         n = (512 + wgs - 1) / wgs;
@@ -633,8 +762,7 @@ int launch_scan(const ScanArgs& a_in, int KS, hipStream_t st, void (*mark)(int, 
                                (a.ep.dot_with && !a.ep.dot_out) || (a.ep.x_out && !(a.ep.dot_with && a.ep.dot_minus)) ||
                                (!a.ep.wd_alpha2 != !a.ep.wd_beta2)))
         return MLSTM_EINVAL;
-    const int kpw = a.D / KS / 4;
-    if (kpw * KS * 4 != a.D || (kpw != 32 && kpw != 64 && kpw != 128) || 4 * KS > 32) return MLSTM_ESHAPE;
+    if ((a.D != 256 && a.D != 512 && a.D != 1024) || KS != scan_key_splits(a.BH, a.D)) return MLSTM_ESHAPE;
     switch (a.D) {
         case 256: return launch_scan_d<256>(a, KS, st, mark);
         case 512: return launch_scan_d<512>(a, KS, st, mark);
