@@ -252,7 +252,8 @@ int launch_gate_backward_rows(int dtype, const void* dh_out, const void* o, cons
 struct ScanArgs {
     const float* q; const float* k; const float* v; const float* o;
     float* h;             // unnormalised numerator (first key range), then the output
-    float* hpart;         // [KS-1, BH, S, D] numerators of the other key ranges
+    float* hpart;         // [parts-1, BH, S, D] numerators of the other key ranges
+    int shared;           // key ranges 2p and 2p+1 add to one partial numerator p (parts = scan_key_parts)
     const float* alpha2; const float* beta2; const double* G2; const float* M;
     float* P;             // [BH, NC, 64, 64] in-chunk pair weights
     float* Nst;           // [BH, NC, D] vector state n~ at every chunk end
@@ -288,6 +289,9 @@ struct ScanArgs {
     int nseg, seg_chunks;
 };
 int scan_key_splits(int BH, int D);
+// Partial numerators of a walk: one per key range, or (shared) one per pair of them, where scan_can_share(BH, D)
+bool scan_can_share(int BH, int D);
+int scan_key_parts(int BH, int D, bool shared);
 void scan_segments(int BH, int S, int D, int* nseg, int* seg_chunks);
 size_t scan_segment_state_bytes(int BH, int S, int D);
 // mark(kernel id, stream, begin?) brackets groups of launches for the optional event timing

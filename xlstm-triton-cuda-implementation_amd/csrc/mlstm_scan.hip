@@ -236,7 +236,10 @@ __global__ __launch_bounds__(SCAN_NW * 64) void scan_state_kernel(ScanArgs a) {
     const float* K = a.k + hoff * D;
     const float* V = a.v + hoff * D;
     const double* G2 = a.G2 + (size_t)bh * NC;
-    float* out = (ks == 0 ? a.h : a.hpart + (size_t)(ks - 1) * a.BH * S * D) + hoff * D;
+    constexpr bool MAY_SHARE = KS >= 4 && NKB == 2;
+    const bool shared = MAY_SHARE && a.shared;
+    const int part_no = shared ? ks / 2 : ks;
+    float* out = (part_no == 0 ? a.h : a.hpart + (size_t)(part_no - 1) * a.BH * S * D) + hoff * D;
     const int kbase = (ks * NW + wave) * KPW, v0 = VT * vt;
     const float log2scale = -0.5f * __log2f((float)D);
     // Position 16 s + 8 h + e of a chunk is contraction element e of lane half h in step s.
@@ -518,7 +521,10 @@ __global__ __launch_bounds__(SCAN_NW * 64) void scan_state_kernel(ScanArgs a) {
             float* o = out + (size_t)t * D + v0 + 32 * (g / 4 % VB) + c32;
 #pragma unroll
             for (int e = 0; e < 4; e++)
-                if (!LAST || t + e < S) o[e * D] = sum[e];
+                if (!LAST || t + e < S) {
+                    if (MAY_SHARE && shared) unsafeAtomicAdd(o + e * D, sum[e]);   // (one hardware add, nothing returned)
+                    else o[e * D] = sum[e];
+                }
         };
         if constexpr (LAST) {
             for (int g = wave; g < 8 * VB; g += NW) { sum_read(g); sum_store(g); }
@@ -571,6 +577,13 @@ __global__ __launch_bounds__(SCAN_NW * 64) void scan_state_kernel(ScanArgs a) {
         for (int c = c_begin; c + 1 < c_end; c++) chunk(c, std::false_type{});
         chunk(c_end - 1, std::true_type{});
     }
+}
+
+// Shared partial numerators start from zero.  Two key ranges add to each element, and 0 + a + b is the same number in either
+// order, so results do not depend on which comes first.
+__global__ __launch_bounds__(256) void scan_zero_kernel(float* h, float* hpart, size_t n4, int parts) {
+    for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n4 * parts; e += (size_t)gridDim.x * 256)
+        *reinterpret_cast<f32x4*>((e < n4 ? h : hpart) + 4 * (e < n4 ? e : e - n4)) = f32x4{0.f, 0.f, 0.f, 0.f};
 }
 
 // States at the segment ends from the segments' own sums, in place: x_s = exp(A_{e(s-1)} - A_{e(s)}) x_{s-1} + x_s with
@@ -708,13 +721,17 @@ static ScanTile scan_tile(int BH, int D) {
 }
 
 template <int D>
-static int launch_scan_d(const ScanArgs& a, int KS, hipStream_t st, void (*mark)(int, hipStream_t, bool)) {
+static int launch_scan_d(const ScanArgs& a, int parts, hipStream_t st, void (*mark)(int, hipStream_t, bool)) {
     mark(MLSTM_K_SCAN_CARRY, st, true);
     hipLaunchKernelGGL(scan_intra_kernel<D>, dim3(a.BH * a.NC * 4), dim3(256), 0, st, a);
     if (a.finish_mode != 2 || a.ep.vec) hipLaunchKernelGGL(scan_ncarry_kernel, dim3((D + 255) / 256, a.BH), dim3(256), 0, st, a);
     mark(MLSTM_K_SCAN_CARRY, st, false);
     mark(MLSTM_K_SCAN_STATE, st, true);
     const ScanTile tile = scan_tile(a.BH, D);
+    if (a.shared) {
+        const size_t n4 = (size_t)a.BH * a.S * D / 4, want = (n4 * parts + 255) / 256;
+        hipLaunchKernelGGL(scan_zero_kernel, dim3((unsigned)(want < 8192 ? want : 8192)), dim3(256), 0, st, a.h, a.hpart, n4, parts);
+    }
     if (tile.nkb == 2) launch_state_r<D, 2, 2>(a, st);
     else if (tile.vb == 2) launch_state_r<D, 2, 1>(a, st);
     else launch_state_r<D, 1, 1>(a, st);
@@ -722,7 +739,7 @@ static int launch_scan_d(const ScanArgs& a, int KS, hipStream_t st, void (*mark)
     mark(MLSTM_K_SCAN_OUT, st, true);
     const size_t rows = (size_t)a.BH * a.S;
     const int blocks = (int)((rows + 3) / 4 < 16384 ? (rows + 3) / 4 : 16384);
-    hipLaunchKernelGGL(scan_finish_kernel, dim3(blocks), dim3(256), 0, st, a, KS);
+    hipLaunchKernelGGL(scan_finish_kernel, dim3(blocks), dim3(256), 0, st, a, parts);
     mark(MLSTM_K_SCAN_OUT, st, false);
     return (int)hipGetLastError();
 }
@@ -732,6 +749,8 @@ void launch_scan_ncarry(const ScanArgs& a, hipStream_t st) {
 }
 
 // Key ranges per value tile.
+bool scan_can_share(int BH, int D) { return scan_tile(BH, D).nkb == 2 && scan_key_splits(BH, D) >= 4; }
+int scan_key_parts(int BH, int D, bool shared) { return shared ? scan_key_splits(BH, D) / 2 : scan_key_splits(BH, D); }
 int scan_key_splits(int BH, int D) { return D / (32 * SCAN_NW * scan_tile(BH, D).nkb); }
 
 // Segments of a sequence that run side by side: none while heads x value tiles x key ranges fill the chip; otherwise
@@ -763,10 +782,12 @@ int launch_scan(const ScanArgs& a_in, int KS, hipStream_t st, void (*mark)(int, 
                                (!a.ep.wd_alpha2 != !a.ep.wd_beta2)))
         return MLSTM_EINVAL;
     if ((a.D != 256 && a.D != 512 && a.D != 1024) || KS != scan_key_splits(a.BH, a.D)) return MLSTM_ESHAPE;
+    if (a.shared && !scan_can_share(a.BH, a.D)) return MLSTM_EINVAL;
+    const int parts = scan_key_parts(a.BH, a.D, a.shared != 0);
     switch (a.D) {
-        case 256: return launch_scan_d<256>(a, KS, st, mark);
-        case 512: return launch_scan_d<512>(a, KS, st, mark);
-        case 1024: return launch_scan_d<1024>(a, KS, st, mark);
+        case 256: return launch_scan_d<256>(a, parts, st, mark);
+        case 512: return launch_scan_d<512>(a, parts, st, mark);
+        case 1024: return launch_scan_d<1024>(a, parts, st, mark);
     }
     return MLSTM_ESHAPE;
 }

@@ -144,9 +144,9 @@ Plan plan_of(char* ws, int BH_, int S_, int D_) {
     p.x = c.take<float>(BH * S);
     p.P = c.take<float>(BH * NG * GRAN * GRAN);
     p.Nst = c.take<float>(BH * NG * D);
-    const int KS = scan_key_splits(BH_, D_);
+    const int parts = scan_key_parts(BH_, D_, scan_can_share(BH_, D_));   // (see launch_scan_backward)
     p.hpart = nullptr;
-    for (int s = 1; s < KS; s++) { float* t = c.take<float>(N); if (s == 1) p.hpart = t; }
+    for (int s = 1; s < parts; s++) { float* t = c.take<float>(N); if (s == 1) p.hpart = t; }
     p.seg_state = c.take<float>(scan_segment_state_bytes(BH_, S_, D_) / 4);
     for (int t = 0; t < 2; t++) p.T[t] = c.take<float>(N);
     p.bytes = c.off;
@@ -179,6 +179,10 @@ int launch_scan_backward(const ScanBwdArgs& a, char* ws, hipStream_t st, void (*
     if (ge != hipSuccess) return (int)ge;
 
     ScanArgs base{};
+    // Where there are four key ranges (D = 1024), pairs of them share a partial numerator: with u and a numerator of its own this
+    // pass would otherwise need five tensors of workspace, not three.  It costs 8 % (4 heads x 2048 x 1024, forward + backward:
+    // 1248 us apart, 1345 shared), which a forward, whose workspace is smaller, does not pay.
+    base.shared = scan_can_share(BH, D) ? 1 : 0;
     base.hpart = p.hpart; base.P = p.P; base.Nst = p.Nst; base.M = p.m; base.o = a.o; base.seg_state = p.seg_state;
     base.BH = BH; base.S = S; base.D = D; base.NC = NG;
     auto fwd_gates = [&](ScanArgs& s) { s.alpha2 = p.alpha2; s.beta2 = p.beta2; s.G2 = p.G2; };
