@@ -234,6 +234,27 @@ struct Scratch {
     ~Scratch() { if (owned && p) (void)hipFreeAsync(p, st); }
 };
 
+// The row tensors of a scan-form call on 16-byte boundaries, where the kernels' copies into LDS want them: the caller's own
+// where they are, otherwise stream-ordered copies (a dense view that starts inside a tensor; such calls are rare and stay valid).
+struct AlignedRows {
+    static constexpr int MOST = 6;
+    Scratch copies[MOST];
+    int n = 0;
+    int take(const void** p, size_t bytes, hipStream_t st) {
+        if (!*p || !(reinterpret_cast<size_t>(*p) & 15)) return 0;
+        Scratch& s = copies[n++];
+        if (int rc = s.get(nullptr, 0, bytes, st)) return rc;
+        const hipError_t e = hipMemcpyAsync(s.p, *p, bytes, hipMemcpyDeviceToDevice, st);
+        *p = s.p;
+        return (int)e;
+    }
+    int take_all(std::initializer_list<const void**> ps, const Sizes& z, hipStream_t st) {
+        for (const void** p : ps)
+            if (int rc = take(p, z.BH * z.S * z.D * z.el, st)) return rc;
+        return 0;
+    }
+};
+
 // Scratch of mlstm_forward_noalloc_ex: the forward's workspace as a file-scope device array, for callers that cannot
 // allocate.  Every GPU the library runs on holds its own copy at its own address until the process ends; in host code
 // the array's name is only a handle for hipGetSymbolAddress, never a device address, so the address is looked up once
@@ -914,6 +935,8 @@ int mlstm_scan_forward_ex(const void* q, const void* k, const void* v, const voi
     const Sizes z = sizes_of(B, NH, S, D, MLSTM_F32);
     Scratch sc;
     if (int rc = sc.get(workspace, workspace_bytes, z.scan_form_fwd(), st)) return rc;
+    AlignedRows rows;
+    if (int rc = rows.take_all({&q, &k, &v, &o}, z, st)) return rc;
     if (scan_on_tiles(D)) return scan_forward_on_tiles(q, k, v, f, i, o, h, nullptr, nullptr, z, (char*)sc.p, st);
     return scan_forward_impl(q, k, v, f, i, o, h, nullptr, nullptr, z, MLSTM_F32, 0, (char*)sc.p, st);
 }
@@ -928,6 +951,8 @@ int mlstm_scan_forward_save_ex(const void* q, const void* k, const void* v, cons
     const Sizes z = sizes_of(B, NH, S, D, MLSTM_F32);
     Scratch sc;
     if (int rc = sc.get(workspace, workspace_bytes, z.scan_form_fwd(), st)) return rc;
+    AlignedRows rows;
+    if (int rc = rows.take_all({&q, &k, &v, &o}, z, st)) return rc;
     if (scan_on_tiles(D)) return scan_forward_on_tiles(q, k, v, f, i, o, h, h_ungated, b, z, (char*)sc.p, st);
     return scan_forward_impl(q, k, v, f, i, o, h, nullptr, b, z, MLSTM_F32, 0, (char*)sc.p, st, (float*)h_ungated);
 }
@@ -953,6 +978,8 @@ int mlstm_scan_backward_saved_ex(const void* dh_gated, const void* q, const void
     const size_t need = scan_on_tiles(D) ? z.bwd_gated() : scan_backward_workspace_bytes(B * NH, S, D);
     Scratch sc;
     if (int rc = sc.get(workspace, workspace_bytes, need, st)) return rc;
+    AlignedRows rows;
+    if (int rc = rows.take_all({&dh_gated, &q, &k, &v, &o, &h_ungated}, z, st)) return rc;
     if (scan_on_tiles(D))   // (m is formed again from the gates: b stands in for the pointer, which is not read)
         return backward_gated_impl(dh_gated, q, k, v, f, i, o, h_ungated, b, b, dq, dk, dv, df, di, d_o, z, NH, D, MLSTM_F32, MLSTM_F32, true,
                                    (char*)sc.p, st);

@@ -7,13 +7,16 @@
 // the backward is a C++ node, which the autograd engine's thread runs without the interpreter lock.
 //
 // Every function takes the operator's tensors and returns its result, or None for whatever the fast path does not serve
-// (unusual layouts, padded or widened head dimensions, arguments that are an error): the Python wrappers then do what they
-// always did, error messages included.
+// (unusual layouts, padded or widened head dimensions, arguments that are an error, calls under a function transform, a tracer,
+// a dispatch mode or with forward-mode tangents): the Python wrappers then do what they always did, error messages included.
 #include <Python.h>
 #include <ATen/ATen.h>
+#include <ATen/TracerMode.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
@@ -116,7 +119,10 @@ struct Call {
         return mlstm_layout{q.stride(0), q.stride(1), q.stride(2), h.stride(0), h.stride(1), h.stride(2), f.stride(0), f.stride(1), f.stride(2), gate_form};
     }
     bool on_tiles() const { return D == 64 || D == 128; }   // scan form: the head dimensions that the tile kernels serve
-    Buffer kept() const { return Buffer(mlstm::train_kept_bytes(B, NH, S, D, dtype)); }
+    bool operator==(const Call& x) const {
+        return B == x.B && NH == x.NH && S == x.S && D == x.D && dtype == x.dtype && gate_dtype == x.gate_dtype && gate_form == x.gate_form;
+    }
+    size_t kept_bytes() const { return mlstm::train_kept_bytes(B, NH, S, D, dtype); }
     Buffer workspace(int op) const { return Buffer(mlstm_workspace_bytes(op, B, NH, S, D, dtype)); }
 };
 
@@ -140,29 +146,43 @@ bool takes_matmul(const Tensor& q, const Tensor& k, const Tensor& v, const Tenso
     return true;
 }
 
-// The nodes of the graph: the inputs (and an output the backward reads) under autograd's version checks, and a buffer with what
-// else the backward reads.
+// The nodes of the graph: the inputs, what else the backward reads (`own`: a buffer of the library's, the ungated output) and
+// an output it reads, all as saved variables: under autograd's version checks and its saved-tensor hooks (checkpointing,
+// offloading), which may hand back other tensors of the same values.
 struct OpNode : torch::autograd::Node {
     Call c;
-    std::vector<SavedVariable> vars;
+    std::vector<SavedVariable> vars, own;
     SavedVariable out;
-    Buffer kept;
     void save(std::initializer_list<Tensor> ts) {
         vars.reserve(ts.size());
         for (const Tensor& t : ts) vars.emplace_back(t, false);
     }
+    void save_own(std::initializer_list<Tensor> ts) {
+        own.reserve(ts.size());
+        for (const Tensor& t : ts) own.emplace_back(t, false);
+    }
     void release_variables() override {
         for (auto& v : vars) v.reset_data();
+        for (auto& v : own) v.reset_data();
         out.reset_data();
-        kept = Buffer();
     }
-    std::vector<Tensor> inputs() {
+    static std::vector<Tensor> unpack(std::vector<SavedVariable>& from) {
         std::vector<Tensor> ts;
-        ts.reserve(vars.size());
-        for (auto& v : vars) ts.push_back(v.unpack());
+        ts.reserve(from.size());
+        for (auto& v : from) ts.push_back(v.unpack());
         return ts;
     }
+    std::vector<Tensor> inputs() { return unpack(vars); }
 };
+[[noreturn]] void saved_changed() { raise_python(PyExc_RuntimeError, "a tensor saved for the backward came back with another shape, type or device"); }
+// a tensor of these sizes and type, dense, on a 16-byte boundary, with the values of a saved one
+Tensor dense_saved(const Tensor& t, at::IntArrayRef sizes, at::ScalarType type, const at::Device& device) {
+    if (t.device() != device || t.scalar_type() != type || t.sizes() != sizes) saved_changed();
+    Tensor d = t.contiguous();
+    return reinterpret_cast<size_t>(d.data_ptr()) & 15 ? d.clone() : d;
+}
+Tensor bytes_tensor(size_t n, const Tensor& like) { return new_tensor({(int64_t)n}, {1}, at::kByte, like); }
+Tensor kept_saved(const Tensor& t, const Tensor& like) { return dense_saved(t, {t.dim() == 1 ? t.size(0) : -1}, at::kByte, like.device()); }
 template <typename N, typename... T>
 std::shared_ptr<N> make_node(const T&... inputs) {
     std::shared_ptr<N> node(new N(), torch::autograd::deleteNode);
@@ -180,6 +200,24 @@ void same_type(const Tensor& dh, const Tensor& q) {
     if (dh.scalar_type() != q.scalar_type()) raise_python(PyExc_TypeError, "dh must have q's dtype");
 }
 
+// the saved q, k, v, f, i of the matmul form: as they were, or dense copies where a hook changed their layouts
+void matmul_inputs(std::vector<Tensor>& in, const Call& c) {
+    for (const Tensor& t : in)
+        if (t.device() != in[0].device() || !t.is_cuda()) saved_changed();
+    Call now;
+    const int precise = c.dtype & MLSTM_PRECISE ? 1 : 0;
+    if (!takes_matmul(in[0], in[1], in[2], in[3], in[4], precise, c.gate_form, now)) {
+        for (int n = 0; n < 5; n++) in[n] = in[n].contiguous();
+        if (!takes_matmul(in[0], in[1], in[2], in[3], in[4], precise, c.gate_form, now)) saved_changed();
+    }
+    if (!(now == c)) saved_changed();
+}
+// the saved output (or ungated output), in its layout where that is one the kernels address
+Tensor rows_saved(const Tensor& h, const Tensor& q) {
+    if (h.device() != q.device() || h.scalar_type() != q.scalar_type() || h.sizes() != q.sizes()) saved_changed();
+    return h.stride(3) != 1 || overlaps(h) ? h.contiguous() : h;
+}
+
 // ---- matmul form ------------------------------------------------------------------------------------------------------
 
 struct Triton_mLSTMBackward : OpNode {
@@ -187,10 +225,10 @@ struct Triton_mLSTMBackward : OpNode {
     variable_list apply(variable_list&& grads) override {
         variable_list res(5);
         at::NoGradGuard no_grad;
-        Tensor dh = grads[0];
-        if (!dh.defined()) return res;
         auto in = inputs();
-        const Tensor h = out.unpack(getptr());
+        matmul_inputs(in, c);
+        const Tensor h = rows_saved(out.unpack(getptr()), in[0]), kept = kept_saved(own[0].unpack(), h);
+        Tensor dh = grads[0].defined() ? grads[0] : at::zeros_like(h);
         contiguous_head(dh);
         same_type(dh, in[0]);
         dh = like_layout(dh, h);
@@ -198,7 +236,7 @@ struct Triton_mLSTMBackward : OpNode {
         const mlstm_layout lay = c.layout(in[0], h, in[3]);
         Buffer ws = c.workspace(MLSTM_OP_BACKWARD);
         check_rc(mlstm::train_backward(dh.data_ptr(), in[0].data_ptr(), in[1].data_ptr(), in[2].data_ptr(), in[3].data_ptr(), in[4].data_ptr(), nullptr,
-                                       h.data_ptr(), kept.get(), kept.n, res[0].data_ptr(), res[1].data_ptr(), res[2].data_ptr(), res[3].data_ptr(),
+                                       h.data_ptr(), kept.data_ptr(), kept.numel(), res[0].data_ptr(), res[1].data_ptr(), res[2].data_ptr(), res[3].data_ptr(),
                                        res[4].data_ptr(), nullptr, c.B, c.NH, c.S, c.D, c.dtype, c.gate_dtype, &lay, ws.get(), ws.n, hip_stream()),
                  "mlstm_backward_saved_lx");
         return res;
@@ -220,11 +258,12 @@ bool matmul(const Tensor* t, int precise, int gate_form, bool train, Tensor& h) 
     }
     auto node = make_node<Triton_mLSTMBackward>(q, k, v, f, i);
     node->c = c;
-    node->kept = c.kept();
-    check_rc(mlstm::train_forward(q.data_ptr(), k.data_ptr(), v.data_ptr(), f.data_ptr(), i.data_ptr(), nullptr, h.data_ptr(), nullptr, node->kept.get(),
-                                  node->kept.n, c.B, c.NH, c.S, c.D, c.dtype, c.gate_dtype, &lay, ws.get(), ws.n, hip_stream()),
+    const Tensor kept = bytes_tensor(c.kept_bytes(), q);
+    check_rc(mlstm::train_forward(q.data_ptr(), k.data_ptr(), v.data_ptr(), f.data_ptr(), i.data_ptr(), nullptr, h.data_ptr(), nullptr, kept.data_ptr(),
+                                  kept.numel(), c.B, c.NH, c.S, c.D, c.dtype, c.gate_dtype, &lay, ws.get(), ws.n, hip_stream()),
              "mlstm_forward_save_lx");
     node->save({q, k, v, f, i});
+    node->save_own({kept});
     torch::autograd::set_history(h, node);
     node->out = SavedVariable(h, true);
     return true;
@@ -233,15 +272,15 @@ bool matmul(const Tensor* t, int precise, int gate_form, bool train, Tensor& h) 
 // ---- matmul form with the output gate ---------------------------------------------------------------------------------
 
 struct Triton_mLSTM_gatedBackward : OpNode {
-    Tensor h;   // the ungated output: never handed out, so no version to check
     std::string name() const override { return "Triton_mLSTM_gatedBackward"; }
-    void release_variables() override { OpNode::release_variables(); h.reset(); }
     variable_list apply(variable_list&& grads) override {
         variable_list res(6);
         at::NoGradGuard no_grad;
-        Tensor dh = grads[0];
-        if (!dh.defined()) return res;
         auto in = inputs();
+        matmul_inputs(in, c);
+        const Tensor h = rows_saved(own[1].unpack(), in[0]), kept = kept_saved(own[0].unpack(), h);
+        if (in[5].device() != h.device() || in[5].scalar_type() != h.scalar_type() || in[5].sizes() != h.sizes()) saved_changed();
+        Tensor dh = grads[0].defined() ? grads[0] : at::zeros_like(h);
         contiguous_head(dh);
         same_type(dh, in[0]);
         dh = like_layout(dh, h);
@@ -251,7 +290,7 @@ struct Triton_mLSTM_gatedBackward : OpNode {
         const mlstm_layout lay = c.layout(in[0], h, in[3]);
         Buffer ws = c.workspace(MLSTM_OP_BACKWARD_GATED);
         check_rc(mlstm::train_backward(dh.data_ptr(), in[0].data_ptr(), in[1].data_ptr(), in[2].data_ptr(), in[3].data_ptr(), in[4].data_ptr(),
-                                       o.data_ptr(), h.data_ptr(), kept.get(), kept.n, res[0].data_ptr(), res[1].data_ptr(), res[2].data_ptr(), res[3].data_ptr(),
+                                       o.data_ptr(), h.data_ptr(), kept.data_ptr(), kept.numel(), res[0].data_ptr(), res[1].data_ptr(), res[2].data_ptr(), res[3].data_ptr(),
                                        res[4].data_ptr(), res[5].data_ptr(), c.B, c.NH, c.S, c.D, c.dtype, c.gate_dtype, &lay, ws.get(), ws.n,
                                        hip_stream()),
                  "mlstm_backward_gated_lx");
@@ -282,12 +321,12 @@ bool gated(const Tensor* t, bool train, Tensor& hg) {
     }
     auto node = make_node<Triton_mLSTM_gatedBackward>(q, k, v, f, i, t[5]);
     node->c = c;
-    node->kept = c.kept();
+    const Tensor kept = bytes_tensor(c.kept_bytes(), q);
     check_rc(mlstm::train_forward(q.data_ptr(), k.data_ptr(), v.data_ptr(), f.data_ptr(), i.data_ptr(), o.data_ptr(), h.data_ptr(), hg.data_ptr(),
-                                  node->kept.get(), node->kept.n, c.B, c.NH, c.S, c.D, c.dtype, c.gate_dtype, &lay, ws.get(), ws.n, hip_stream()),
+                                  kept.data_ptr(), kept.numel(), c.B, c.NH, c.S, c.D, c.dtype, c.gate_dtype, &lay, ws.get(), ws.n, hip_stream()),
              "mlstm_forward_gated_lx");
     node->save({q, k, v, f, i, t[5]});
-    node->h = h;
+    node->save_own({kept, h});
     torch::autograd::set_history(hg, node);
     return true;
 }
@@ -295,32 +334,34 @@ bool gated(const Tensor* t, bool train, Tensor& hg) {
 // ---- scan form --------------------------------------------------------------------------------------------------------
 
 struct Scan_mLSTMBackward : OpNode {
-    Tensor h_ungated;
     std::string name() const override { return "Scan_mLSTMBackward"; }
-    void release_variables() override { OpNode::release_variables(); h_ungated.reset(); }
     variable_list apply(variable_list&& grads) override {
         variable_list res(6);
         at::NoGradGuard no_grad;
-        if (!grads[0].defined()) return res;
         auto in = inputs();
-        if (grads[0].scalar_type() != at::kFloat) raise_python(PyExc_TypeError, "dh must be float32");
-        const Tensor dh = grads[0].contiguous();
+        const at::Device device = in[0].device();
+        if (!device.is_cuda()) saved_changed();
+        const int64_t rows[4] = {c.B, c.NH, c.S, c.D};
         for (int n = 0; n < 6; n++) {
-            in[n] = in[n].contiguous();
+            in[n] = dense_saved(in[n], at::IntArrayRef(rows, n == 3 || n == 4 ? 3 : 4), at::kFloat, device);
             res[n] = new_like(in[n]);
         }
+        const Tensor kept = kept_saved(own[0].unpack(), in[0]), h_ungated = dense_saved(own[1].unpack(), at::IntArrayRef(rows, 4), at::kFloat, device);
+        if (grads[0].defined() && grads[0].scalar_type() != at::kFloat) raise_python(PyExc_TypeError, "dh must be float32");
+        const Tensor dh = grads[0].defined() ? dense_saved(grads[0], at::IntArrayRef(rows, 4), at::kFloat, device) : at::zeros_like(in[0]);
         if (c.on_tiles()) {
             Buffer ws = c.workspace(MLSTM_OP_BACKWARD_GATED);
             check_rc(mlstm::train_backward(dh.data_ptr(), in[0].data_ptr(), in[1].data_ptr(), in[2].data_ptr(), in[3].data_ptr(), in[4].data_ptr(),
-                                           in[5].data_ptr(), h_ungated.data_ptr(), kept.get(), kept.n, res[0].data_ptr(), res[1].data_ptr(), res[2].data_ptr(),
+                                           in[5].data_ptr(), h_ungated.data_ptr(), kept.data_ptr(), kept.numel(), res[0].data_ptr(), res[1].data_ptr(), res[2].data_ptr(),
                                            res[3].data_ptr(), res[4].data_ptr(), res[5].data_ptr(), c.B, c.NH, c.S, c.D, MLSTM_F32, MLSTM_F32, nullptr,
                                            ws.get(), ws.n, hip_stream()),
                      "mlstm_scan_backward_saved_ex");
             return res;
         }
+        if (kept.numel() != 4ll * c.B * c.NH * c.S) saved_changed();
         Buffer ws = c.workspace(MLSTM_OP_SCAN_BACKWARD);
         check_rc(mlstm_scan_backward_saved_ex(dh.data_ptr(), in[0].data_ptr(), in[1].data_ptr(), in[2].data_ptr(), in[3].data_ptr(), in[4].data_ptr(),
-                                              in[5].data_ptr(), h_ungated.data_ptr(), static_cast<float*>(kept.get()), res[0].data_ptr(), res[1].data_ptr(), res[2].data_ptr(),
+                                              in[5].data_ptr(), h_ungated.data_ptr(), static_cast<float*>(kept.data_ptr()), res[0].data_ptr(), res[1].data_ptr(), res[2].data_ptr(),
                                               res[3].data_ptr(), res[4].data_ptr(), res[5].data_ptr(), c.B, c.NH, c.S, c.D, MLSTM_F32, ws.get(), ws.n,
                                               hip_stream()),
                  "mlstm_scan_backward_saved_ex");
@@ -340,7 +381,8 @@ bool scan(const Tensor* t, Tensor& h) {
         for (int n = 0; n < 6; n++) {
             const bool gate = n == 3 || n == 4;
             if (t[n].scalar_type() != at::kFloat || (gate ? t[n].sizes() != q.sizes().slice(0, 3) : t[n].sizes() != q.sizes())) return false;
-            in[n] = t[n].contiguous();
+            in[n] = t[n].contiguous();   // (on a 16-byte boundary: the kernels copy whole rows of 16-byte pieces into LDS)
+            if (reinterpret_cast<size_t>(in[n].data_ptr()) & 15) in[n] = in[n].clone();
         }
     }
     h = new_like(in[0]);
@@ -353,23 +395,25 @@ bool scan(const Tensor* t, Tensor& h) {
     }
     auto node = make_node<Scan_mLSTMBackward>(t[0], t[1], t[2], t[3], t[4], t[5]);
     node->c = c;
-    node->h_ungated = new_like(in[0]);
+    const Tensor h_ungated = new_like(in[0]);
+    Tensor kept;
     if (c.on_tiles()) {
-        node->kept = c.kept();
+        kept = bytes_tensor(c.kept_bytes(), h);
         Buffer ws = c.workspace(MLSTM_OP_FORWARD_GATED);
         check_rc(mlstm::train_forward(in[0].data_ptr(), in[1].data_ptr(), in[2].data_ptr(), in[3].data_ptr(), in[4].data_ptr(), in[5].data_ptr(),
-                                      node->h_ungated.data_ptr(), h.data_ptr(), node->kept.get(), node->kept.n, c.B, c.NH, c.S, c.D, MLSTM_F32, MLSTM_F32, nullptr,
+                                      h_ungated.data_ptr(), h.data_ptr(), kept.data_ptr(), kept.numel(), c.B, c.NH, c.S, c.D, MLSTM_F32, MLSTM_F32, nullptr,
                                       ws.get(), ws.n, hip_stream()),
                  "mlstm_scan_forward_save_ex");
     } else {
-        node->kept = Buffer((size_t)c.B * c.NH * c.S * 4);   // the normaliser sums
+        kept = bytes_tensor((size_t)c.B * c.NH * c.S * 4, h);   // the normaliser sums
         Buffer ws = c.workspace(MLSTM_OP_SCAN_FORWARD);
         check_rc(mlstm_scan_forward_save_ex(in[0].data_ptr(), in[1].data_ptr(), in[2].data_ptr(), in[3].data_ptr(), in[4].data_ptr(), in[5].data_ptr(),
-                                            h.data_ptr(), node->h_ungated.data_ptr(), static_cast<float*>(node->kept.get()), c.B, c.NH, c.S, c.D,
+                                            h.data_ptr(), h_ungated.data_ptr(), static_cast<float*>(kept.data_ptr()), c.B, c.NH, c.S, c.D,
                                             MLSTM_F32, ws.get(), ws.n, hip_stream()),
                  "mlstm_scan_forward_save_ex");
     }
     node->save({t[0], t[1], t[2], t[3], t[4], t[5]});
+    node->save_own({kept, h_ungated});
     torch::autograd::set_history(h, node);
     return true;
 }
@@ -382,18 +426,23 @@ struct HIP_sLSTMBackward : OpNode {
     variable_list apply(variable_list&& grads) override {
         variable_list res(3);
         at::NoGradGuard no_grad;
-        if (!grads[0].defined()) return res;
         auto in = inputs();   // r alone: the pre-activations of wx are in the saved states
-        const Tensor h = out.unpack(getptr());
-        if (grads[0].scalar_type() != at::kFloat) raise_python(PyExc_TypeError, "dh must be float32");
-        const Tensor dh = grads[0].contiguous(), &r = in[0];
+        const Tensor h_saved = out.unpack(getptr());
+        const at::Device device = h_saved.device();
+        if (!device.is_cuda()) saved_changed();
+        const int64_t rows[4] = {c.B, c.S, c.NH, c.D}, mats[4] = {c.NH, 4, c.D, c.D};
+        const Tensor h = dense_saved(h_saved, at::IntArrayRef(rows, 4), at::kFloat, device), r = dense_saved(in[0], at::IntArrayRef(mats, 4), at::kFloat, device);
+        const Tensor kept = kept_saved(own[0].unpack(), h);
+        if ((size_t)kept.numel() != slstm_saved_bytes(c.B, c.NH, c.S, c.D)) saved_changed();
+        if (grads[0].defined() && grads[0].scalar_type() != at::kFloat) raise_python(PyExc_TypeError, "dh must be float32");
+        const Tensor dh = grads[0].defined() ? grads[0].contiguous() : at::zeros_like(h);
         const int64_t wx[5] = {c.B, c.S, 4, c.NH, c.D}, sx[5] = {4ll * c.S * c.NH * c.D, 4ll * c.NH * c.D, (int64_t)c.NH * c.D, c.D, 1};
         const int64_t bs[3] = {c.NH, 4, c.D}, sb[3] = {4ll * c.D, c.D, 1};
         res[0] = new_tensor(at::IntArrayRef(wx, 5), at::IntArrayRef(sx, 5), at::kFloat, h);
         res[1] = new_like(r);
         res[2] = new_tensor(at::IntArrayRef(bs, 3), at::IntArrayRef(sb, 3), at::kFloat, h);
         Buffer ws(slstm_workspace_bytes(c.B, c.NH, c.S, c.D));
-        check_rc(slstm_backward_ex(dh.data_ptr<float>(), h.data_ptr<float>(), r.data_ptr<float>(), static_cast<const float*>(kept.get()),
+        check_rc(slstm_backward_ex(dh.data_ptr<float>(), h.data_ptr<float>(), r.data_ptr<float>(), static_cast<const float*>(kept.data_ptr()),
                                    res[0].data_ptr<float>(), res[1].data_ptr<float>(), res[2].data_ptr<float>(), c.B, c.NH, c.S, c.D, forget_sigmoid,
                                    ws.get(), ws.n, hip_stream()),
                  "slstm_backward_ex");
@@ -414,17 +463,19 @@ bool slstm(const Tensor* t, int forget_sigmoid, Tensor& h) {
     h = new_tensor(at::IntArrayRef(hs, 4), at::IntArrayRef(sh, 4), at::kFloat, wx);
     const bool keep = wants_grad(wx, r, b);
     std::shared_ptr<HIP_sLSTMBackward> node;
+    Tensor kept;
     if (keep) {
         node = make_node<HIP_sLSTMBackward>(wx, r, b);
         node->c = c;
         node->forget_sigmoid = forget_sigmoid;
-        node->kept = Buffer(slstm_saved_bytes(c.B, c.NH, c.S, c.D));
+        kept = bytes_tensor(slstm_saved_bytes(c.B, c.NH, c.S, c.D), wx);
     }
     check_rc(slstm_forward_ex(wx.data_ptr<float>(), r.data_ptr<float>(), b.data_ptr<float>(), h.data_ptr<float>(),
-                              keep ? static_cast<float*>(node->kept.get()) : nullptr, c.B, c.NH, c.S, c.D, forget_sigmoid, hip_stream()),
+                              keep ? static_cast<float*>(kept.data_ptr()) : nullptr, c.B, c.NH, c.S, c.D, forget_sigmoid, hip_stream()),
              "slstm_forward_ex");
     if (keep) {
         node->save({r});
+        node->save_own({kept});
         torch::autograd::set_history(h, node);
         node->out = SavedVariable(h, true);
     }
@@ -434,12 +485,16 @@ bool slstm(const Tensor* t, int forget_sigmoid, Tensor& h) {
 // ---- Python -----------------------------------------------------------------------------------------------------------
 
 // The first `n` arguments as plain tensors on the current device (false: something else is among them).
+// Calls that a dispatch mode, a tracer or a function transform would have to see are not served here, nor forward-mode tangents.
 bool tensors(PyObject* const* args, Py_ssize_t nargs, int n, Tensor* t) {
-    if (nargs < n) return false;
+    if (nargs < n || c10::impl::dispatch_mode_enabled() || at::tracer::impl::is_dispatch_enabled() ||
+        c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode))
+        return false;
     for (int k = 0; k < n; k++) {
         if (!THPVariable_CheckExact(args[k])) return false;
         t[k] = THPVariable_Unpack(args[k]);
         if (!t[k].is_cuda() || t[k].layout() != at::kStrided) return false;
+        if (t[k]._fw_grad(0).defined()) return false;
     }
     const auto dev = t[0].device();
     if (dev.index() != c10::hip::current_device()) return false;

@@ -215,7 +215,8 @@ def mlstm_matmul(q, k, v, f, i, SB=16, num_warps=8):
 
 # Triton_mLSTM and its variants go to the native host path (csrc/mlstm_torch.cpp: checks, allocations, launches and the graph's
 # node in C++), which returns None for whatever it does not serve: padded and widened head dimensions, layouts that need a copy
-# first, arguments that are an error.  Those take the autograd functions below.
+# first, arguments that are an error, calls under torch.func, a tracer or with forward-mode tangents.  Those, and classes derived
+# from these, take the autograd functions below.
 def _native_matmul(q, k, v, f, i, precise, gate_form):
     form = _ffi.GATE_FORMS.get(gate_form)
     return None if form is None else _ffi.native().matmul_train(q, k, v, f, i, precise, form)
@@ -226,7 +227,7 @@ class Triton_mLSTM(torch.autograd.Function):
 
     @classmethod
     def apply(cls, q, k, v, f, i, SB=16, num_warps=8, gate_form="raw"):
-        h = _native_matmul(q, k, v, f, i, 0, gate_form)
+        h = _native_matmul(q, k, v, f, i, 0, gate_form) if cls is Triton_mLSTM else None
         return h if h is not None else super().apply(q, k, v, f, i, SB, num_warps, gate_form)
 
     @staticmethod
@@ -258,7 +259,7 @@ class Triton_mLSTM_precise(torch.autograd.Function):
 
     @classmethod
     def apply(cls, q, k, v, f, i, SB=16, num_warps=8, gate_form="raw"):
-        h = _native_matmul(q, k, v, f, i, 1, gate_form)
+        h = _native_matmul(q, k, v, f, i, 1, gate_form) if cls is Triton_mLSTM_precise else None
         return h if h is not None else super().apply(q, k, v, f, i, SB, num_warps, gate_form)
 
     @staticmethod
@@ -351,7 +352,7 @@ class Triton_mLSTM_gated(torch.autograd.Function):
 
     @classmethod
     def apply(cls, q, k, v, f, i, o, SB=16, num_warps=8):
-        h = _ffi.native().gated_train(q, k, v, f, i, o)
+        h = _ffi.native().gated_train(q, k, v, f, i, o) if cls is Triton_mLSTM_gated else None
         return h if h is not None else super().apply(q, k, v, f, i, o, SB, num_warps)
 
     @staticmethod
