@@ -118,3 +118,17 @@ def test_rejects_what_it_cannot_serve():
         slstm_forward_hip(wx.cuda().half(), r.cuda(), b.cuda())
     with pytest.raises(ValueError):
         slstm_forward_hip(wx.cuda(), r.cuda()[:, :3], b.cuda())
+
+
+@pytest.mark.parametrize("forget_sigmoid", [False, True])
+@pytest.mark.parametrize("B,NH,S,DH", [(1, 1, 2, 64), (1, 2, 3, 128), (2, 1, 5, 32), (1, 1, 6, 64), (1, 3, 10, 128), (2, 1, 15, 64)])
+def test_short_sequences_of_every_prologue_length(B, NH, S, DH, forget_sigmoid):
+    # a step's stores and loads are issued by its successor and the backward takes values two steps ahead: the first and last steps
+    from slstm import slstm_backward_hip, slstm_forward_hip
+    wx, r, b, dh = SO.make_inputs(B, NH, S, DH, seed=40 + S, f_mean=0.0)
+    h, saved = slstm_forward_hip(*gpu(wx, r, b), forget_sigmoid=forget_sigmoid)
+    assert_close(h, SO.slstm_forward(wx, r, b, forget_sigmoid), torch.float32, "h")
+    assert torch.equal(slstm_forward_hip(*gpu(wx, r, b), forget_sigmoid=forget_sigmoid, save=False)[0], h)
+    got = slstm_backward_hip(dh.cuda(), h, r.cuda(), saved, forget_sigmoid=forget_sigmoid)
+    for name, g, w in zip(("dwx", "dr", "db"), got, SO.slstm_backward(dh, wx, r, b, forget_sigmoid)):
+        assert_close(g, w, torch.float32, name)

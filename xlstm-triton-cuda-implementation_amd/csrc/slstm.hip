@@ -7,13 +7,13 @@
 //     c_t  = f'_t c_{t-1} + i'_t tanh(z~),  n_t = f'_t n_{t-1} + i'_t,  h_t = sigmoid(o~) c_t / n_t
 // The recurrence through h makes the cell sequential in t, so the kernels are latency machines, not throughput ones: one
 // workgroup per (batch, head) walks the sequence with the head's four recurrent matrices in registers.
-//   slstm_forward_kernel   four lanes per unit j, each with a quarter of row j of all four R_g: partial pre-activations from
-//                          h_{t-1} (LDS), summed over the four lanes; every lane then updates the cell of its unit.
-//                          Gate values and (c, n, m) are kept for the backward.
+//   slstm_forward_kernel   eight lanes per two units, each with an eighth of the units' rows of all four R_g: partial
+//                          pre-activations from h_{t-1} (LDS), one gate's sum per lane; every lane then updates the cell of its
+//                          unit.  Gate values and (c, n, m) are kept for the backward.
 //   slstm_backward_kernel  back through time: rows of 16 lanes form R^T delta_{t+1} for their four units (a sixteenth of the
-//                          gradient vector per lane, summed over the row), which is what step t+1 sent back to h_t; every
-//                          lane of a unit's quad turns (dh_t + that, dc, dn) into the four pre-activation gradients (= dWx_t).  The stabiliser m is a common scale of c and n that h
-//                          does not depend on, so it is held constant.
+//                          gradient vector per lane, summed over the row), which is what step t+1 sent back to h_t; the
+//                          lanes of a unit's quad turn (dh_t + that, dc, dn) into one pre-activation gradient each (= dWx_t).
+//                          The stabiliser m is a common scale of c and n that h does not depend on, so it is held constant.
 //   slstm_dr_kernel        dR_g = sum_{b,t} dWx_t[g] h_{t-1}^T and db_g = sum_{b,t} dWx_t[g]: off the sequential path, in
 //                          slices of (b, t) whose partial sums a second kernel adds in a fixed order.
 // Layouts: wx, dwx [B,S,4,NH,DH] (gates i, f, z, o); r, dr [NH,4,DH,DH] (r[h][g][j][k]: unit j from unit k); b, db [NH,4,DH];
@@ -32,16 +32,6 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 // on the critical path of every step of a sequential kernel.
 __device__ __forceinline__ float fast_exp(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896340736f); }
 __device__ __forceinline__ float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ __forceinline__ float sigmoid_fast(float x) { return fast_rcp(1.0f + fast_exp(-x)); }
-__device__ __forceinline__ float tanh_fast(float x) {
-    const float e = fast_exp(-2.0f * fabsf(x));   // in (0, 1]: no overflow
-    const float t = (1.0f - e) * fast_rcp(1.0f + e);
-    return x < 0.f ? -t : t;
-}
-__device__ __forceinline__ float log_sigmoid_fast(float x) {
-    // min(x, 0) - log(1 + exp(-|x|)); the log through the hardware log2
-    return fminf(x, 0.0f) - __builtin_amdgcn_logf(1.0f + fast_exp(-fabsf(x))) * 0.69314718055994530942f;
-}
 
 // Inputs of a step come from memory PF steps ahead of it, as direct-to-LDS loads into a ring (a trip to memory is several
 // steps long, and a step must not wait for one).  The loads are issued and waited for by hand: every wave issues the same
@@ -51,7 +41,11 @@ __device__ __forceinline__ float log_sigmoid_fast(float x) {
 // loads into a ring of registers ended in a wait for everything at every step.)  A lane only ever reads ring values that
 // its own wave loaded, so the wait needs no barrier behind it.
 constexpr int PF = 8;
-__device__ __forceinline__ void ring_load(const float* g, unsigned lds_off) {
+// (a row's address is uniform, the lane's place in it an offset in bytes)
+__device__ __forceinline__ void ring_load(const float* row, unsigned lane_off, unsigned lds_off) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(lane_off), "s"(row), "s"(lds_off) : "memory", "m0");
+}
+__device__ __forceinline__ void ring_load_lane(const float* g, unsigned lds_off) {   // an address of the lane's own
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "s"(lds_off) : "memory", "m0");
 }
 // (n is a constant once the step loops are unrolled; anything out of range waits for everything)
@@ -95,12 +89,6 @@ __device__ __forceinline__ float quad_sum(float x) {
     x += quad_perm<0x4E>(x);   // lanes 2, 3, 0, 1
     return x;
 }
-// Sum over the 16 lanes of a row (lanes 16a .. 16a+15), the same bits in all of them: rotations by 8 and 4, then the quad.
-__device__ __forceinline__ float row_sum(float x) {
-    x += quad_perm<0x128>(x);   // row_ror:8
-    x += quad_perm<0x124>(x);   // row_ror:4
-    return quad_sum(x);
-}
 // the value of lane q of a quad (three selects; is0..is2: q == 0, 1, 2)
 __device__ __forceinline__ float pick(bool is0, bool is1, bool is2, float a, float b, float c, float d) {
     float x = is2 ? c : d;
@@ -108,111 +96,146 @@ __device__ __forceinline__ float pick(bool is0, bool is1, bool is2, float a, flo
     return is0 ? a : x;
 }
 
-// A quad of lanes owns a unit j: lane q of it keeps, for all four gates, the quarter q of row j of R_g, forms its quarter of
-// the four pre-activations from its quarter of h_{t-1}, and after the sum over the quad every lane has all four and
-// updates the cell, all four alike (c, n, m are kept four times, the same bits).  So a step has no hand-over between
-// threads but h itself: one LDS write, one barrier (h in two buffers, taken in turns).  Lane q loads gate q's input of its
-// unit into the ring, and stores saved value q and value 4 + q (c, n, m; for q = 3, h itself).
+// A quad of lanes owns a unit j, an octet two of them: lane p of the octet keeps, for all four gates of both units, part p (an
+// eighth) of their rows of R_g and forms its part of the eight pre-activations from its part of h_{t-1}.  Lane q of a quad holds
+// gate q ^ s of its own unit, and q ^ 3 ^ s of the other, as its s-th, so that seven exchanges with an add each (the octet's mirror
+// image, then the quad) leave the whole sum of gate q in lane q; it applies that gate's nonlinearity (one exp2, one reciprocal,
+// one logarithm serve the three kinds side by side), the quad exchanges the four results, and every lane updates the cell, all
+// four alike (c, n, m are kept four times, the same bits).  A step has no hand-over between waves but h itself: one LDS write,
+// one barrier (h in two buffers, taken in turns).
+// What bounds it is the serial chain of a step, 340 ns or some 800 cycles (DH = 64): the trip of h through LDS and the barrier about
+// 300, 64 multiply-adds at 4 cycles on the one wave of a SIMD, the gates 160.  Eighths and not quarters because the LDS reads of
+// h (32 DH floats a step) were the longest part of that trip; whatever a step does not hand on -- its stores, the ring's refill,
+// its own input -- is done in the NEXT step, while that waits for h from LDS.  Row broadcasts in the place of wide LDS reads were
+// slower (DH = 128: 831 to 889 us): a broadcast, alone or as an operand of the multiply-add, costs as much as one.
+// Forward, B16 NH4, before (quarters, all four gates in every lane, stores ahead of the barrier) -> now: DH = 64, S = 2048 716 ->
+// 700 us; DH = 128, S = 1024 627 -> 559; DH = 32, S = 1024 285 -> 281.
 template <int DH, bool SAVE, bool FS>
 __global__ __launch_bounds__(4 * DH) void slstm_forward_kernel(const float* __restrict__ wx, const float* __restrict__ r,
                                                                const float* __restrict__ bias, float* __restrict__ h,
                                                                float* __restrict__ saved, int NH, int S) {
-    constexpr int KQ = DH / 4;
-    __shared__ __attribute__((aligned(16))) float hs[2][DH];
+    constexpr int KP = DH / 8, KS = KP < 16 ? KP : KP + 4;   // a part of h, and its place in LDS (eight parts, no bank twice)
+    __shared__ __attribute__((aligned(16))) float hs[2][8 * KS];
     __shared__ __attribute__((aligned(16))) float ring[PF][4 * DH];   // wx of the next PF steps: [slot][unit * 4 + gate]
     const int tid = threadIdx.x, j = tid >> 2, q = tid & 3, wave = tid >> 6;
     const bool is0 = q == 0, is1 = q == 1, is2 = q == 2;
     const int b = blockIdx.x / NH, hd = blockIdx.x % NH;
-    float rr[4][KQ], bq[4];
+    const int p = tid & 7;
+    float ro[4][KP], rx[4][KP];   // part p of the rows of the own unit, [s: gate q ^ s], and of the octet's other one, [s: gate q ^ 3 ^ s]
 #pragma unroll
-    for (int g = 0; g < 4; g++) {
-        const float* src = r + (((size_t)hd * 4 + g) * DH + j) * DH + q * KQ;
+    for (int s = 0; s < 4; s++) {
+        const float* own = r + (((size_t)hd * 4 + (q ^ s)) * DH + j) * DH + p * KP;
+        const float* oth = r + (((size_t)hd * 4 + (q ^ 3 ^ s)) * DH + (j ^ 1)) * DH + p * KP;
 #pragma unroll
-        for (int k = 0; k < KQ; k += 4) {
-            const f32x4 v = *reinterpret_cast<const f32x4*>(src + k);
-            rr[g][k] = v[0]; rr[g][k + 1] = v[1]; rr[g][k + 2] = v[2]; rr[g][k + 3] = v[3];
+        for (int k = 0; k < KP; k += 4) {
+            const f32x4 v = *reinterpret_cast<const f32x4*>(own + k), w = *reinterpret_cast<const f32x4*>(oth + k);
+#pragma unroll
+            for (int e = 0; e < 4; e++) { ro[s][k + e] = v[e]; rx[s][k + e] = w[e]; }
         }
-        bq[g] = bias[((size_t)hd * 4 + g) * DH + j];
     }
+    const float bq = bias[((size_t)hd * 4 + q) * DH + j];
     const size_t step_wx = (size_t)4 * NH * DH, step_h = (size_t)NH * DH, step_s = (size_t)7 * NH * DH;
-    // (pointers that walk with the steps: a lone wave per SIMD pays for every instruction of address arithmetic)
-    const float* wnext = wx + (size_t)b * S * step_wx + ((size_t)q * NH + hd) * DH + j;   // the row the ring takes next
-    float* own = SAVE ? saved + (size_t)b * S * step_s + ((size_t)q * NH + hd) * DH + j : nullptr;
+    // rows that walk with the steps (uniform), and the lane's place in them
+    const unsigned at_gate = (unsigned)((q * NH + hd) * DH + j);
+    const float* wnext = wx + (size_t)b * S * step_wx;   // the row the ring takes next
+    float* srow = SAVE ? saved + (size_t)b * S * step_s : nullptr;
+    // value 4 + q of the saved state; for q = 3, h itself
     float* out2 = q == 3 ? h + (size_t)b * S * step_h + (size_t)hd * DH + j
                          : (SAVE ? saved + (size_t)b * S * step_s + ((size_t)(4 + q) * NH + hd) * DH + j : nullptr);
     const size_t step2 = q == 3 ? step_h : step_s;
-    if (tid < DH) hs[0][tid] = 0.f;
+    // the gate's nonlinearity: e = exp2(coef |x|) (sigmoid: of x itself)
+    const float coef = is2 ? -2.0f * 1.44269504088896340736f : -1.44269504088896340736f;
+    const unsigned sign_off = q == 3 ? 0xffffffffu : 0x7fffffffu;
+    for (int e = tid; e < 8 * KS; e += 4 * DH) hs[0][e] = 0.f;
+    const int h_at = j / KP * KS + j % KP;
     // (the stabiliser starts at -inf rather than the paper's 0: with c_0 = n_0 = 0 it only sets the scale of the first
     // step, and this way the first input gate is exp(0) whatever the first forget gate says)
-    float c = 0.f, n = 0.f, m = -INFINITY;
+    float c = 0.f, n = 0.f, m = -INFINITY, hnew = 0.f, val = 0.f;
     // Memory operations per wave and step, the same in every wave: two stores (without the saved state one: every wave has
     // lanes with q = 3), then the ring load.
     constexpr int OPS = SAVE ? 3 : 2;
     const unsigned ring_base = __builtin_amdgcn_readfirstlane(mlstm::lds_offset_of(&ring[0][0]) + wave * 256);
 #pragma unroll
     for (int u = 0; u < PF; u++) {   // (past the end of the sequence the last row is loaded again)
-        ring_load(wnext, ring_base + u * (4 * DH * 4));
+        ring_load(wnext, 4 * at_gate, ring_base + u * (4 * DH * 4));
         if (u + 1 < S) wnext += step_wx;
     }
-    ring_wait(PF - 1);
-    f32x4 wv = *reinterpret_cast<const f32x4*>(&ring[0][4 * j]);   // the quad's four inputs: its own wave's loads
+    auto store = [&]() __attribute__((always_inline)) {   // what a step keeps, from the registers it left it in
+        if (SAVE) { *reinterpret_cast<float*>(reinterpret_cast<char*>(srow) + 4 * at_gate) = val; srow += step_s; }
+        if (SAVE || q == 3) { *out2 = pick(is0, is1, is2, c, n, m, hnew); out2 += step2; }
+    };
     __syncthreads();
-    // One step, u = t mod PF.  wait_n: how many of the wave's memory operations may still be under way when the NEXT
-    // step's inputs are taken from the ring, before the barrier rather than after it.
-    auto step = [&](int u, int t, int wait_n) __attribute__((always_inline)) {
-        const float* hcur = hs[u & 1] + q * KQ;   // (PF is even: the buffers alternate across rounds too)
-        f32x4 hv[KQ / 4];
+    // One step, u = t mod PF.  wait_n: how many of the wave's memory operations may still be under way when the step's input
+    // is taken from the ring.
+    auto step = [&](int u, int t, int wait_n, bool first) __attribute__((always_inline)) {
+        const float* hcur = hs[u & 1] + p * KS;   // (PF is even: the buffers alternate across rounds too)
+        f32x4 hv[KP / 4];
 #pragma unroll
-        for (int k = 0; k < KQ / 4; k++) hv[k] = *reinterpret_cast<const f32x4*>(hcur + 4 * k);
-        float a[4] = {0.f, 0.f, 0.f, 0.f};
+        for (int k = 0; k < KP / 4; k++) hv[k] = *reinterpret_cast<const f32x4*>(hcur + 4 * k);
+        __builtin_amdgcn_sched_barrier(0);
+        if (!first) {   // the step before: its results go out, and its ring slot takes the row PF steps on
+            store();
+            ring_load(wnext, 4 * at_gate, ring_base + ((u + PF - 1) % PF) * (4 * DH * 4));
+            if (t + PF < S) wnext += step_wx;
+        }
+        ring_wait(wait_n);
+        const float wv = ring[u][tid];   // (its own wave's load)
+        __builtin_amdgcn_sched_barrier(0);
+        float a[4] = {0.f, 0.f, 0.f, 0.f}, x4[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int k = 0; k < KQ / 4; k++)
+        for (int k = 0; k < KP / 4; k++)
 #pragma unroll
             for (int e = 0; e < 4; e++)
 #pragma unroll
-                for (int g = 0; g < 4; g++) a[g] += rr[g][4 * k + e] * hv[k][e];
-        const float it = quad_sum(a[0]) + (wv[0] + bq[0]);
-        const float ft = quad_sum(a[1]) + (wv[1] + bq[1]);
-        const float zt = quad_sum(a[2]) + (wv[2] + bq[2]);
-        const float ot = quad_sum(a[3]) + (wv[3] + bq[3]);
-        const float logf = FS ? log_sigmoid_fast(ft) : ft;
-        const float z = tanh_fast(zt), o = sigmoid_fast(ot);
-        const float mn = fmaxf(logf + m, it);
-        const float ip = fast_exp(it - mn), fp = fast_exp(logf + m - mn);
-        c = fp * c + ip * z;
+                for (int s = 0; s < 4; s++) {
+                    a[s] += ro[s][4 * k + e] * hv[k][e];
+                    x4[s] += rx[s][4 * k + e] * hv[k][e];
+                }
+        // own unit: what the octet's mirror lane (7 - p, of gate q ^ 3) has of it, then gate q from lanes q, q ^ 1, q ^ 2, q ^ 3
+#pragma unroll
+        for (int s = 0; s < 4; s++) a[s] += quad_perm<0x141>(x4[s]);   // row_half_mirror
+        const float x = ((a[0] + quad_perm<0xB1>(a[1])) + (quad_perm<0x4E>(a[2]) + quad_perm<0x1B>(a[3]))) + (wv + bq);
+        const float e = __builtin_amdgcn_exp2f(coef * __builtin_bit_cast(float, __builtin_bit_cast(unsigned, x) & sign_off));
+        const float d = 1.0f + e, rd = fast_rcp(d);
+        const float th = __builtin_copysignf((1.0f - e) * rd, x);                                             // tanh
+        const float ls = FS ? fminf(x, 0.0f) - __builtin_amdgcn_logf(d) * 0.69314718055994530942f : x;        // log sigmoid
+        val = pick(is0, is1, is2, x, ls, th, rd);   // i~, log f, z, o
+        const float it = quad_perm<0x00>(val), logf = quad_perm<0x55>(val), z = quad_perm<0xAA>(val), o = quad_perm<0xFF>(val);
+        const float fm = logf + m, mn = fmaxf(fm, it);
+        const float ip = fast_exp(it - mn), fp = fast_exp(fm - mn);
         n = fp * n + ip;
+        c = fp * c + ip * z;
         m = mn;
-        const float hnew = o * c * fast_rcp(n);
-        hs[(u & 1) ^ 1][j] = hnew;   // (the quad's four lanes write the same bits)
-        if (SAVE) { *own = pick(is0, is1, is2, it, logf, z, o); own += step_s; }
-        if (SAVE || q == 3) { *out2 = pick(is0, is1, is2, c, n, m, hnew); out2 += step2; }
-        // (the ring's values of this step went into the stores above: its slot takes the row PF steps on)
-        ring_load(wnext, ring_base + u * (4 * DH * 4));
-        if (t + PF + 1 < S) wnext += step_wx;
-        ring_wait(wait_n);
-        wv = *reinterpret_cast<const f32x4*>(&ring[(u + 1) % PF][4 * j]);
+        hnew = o * c * fast_rcp(n);
+        hs[(u & 1) ^ 1][h_at] = hnew;   // (the quad's four lanes write the same bits)
         __syncthreads();
     };
-    // The ring load of step t + 1 was issued at the end of step t + 1 - PF: when step t asks for it, the OPS operations of
-    // each of the PF - 1 steps since are younger (the wait allows one step's fewer).  In the first round the loads come
-    // from the prologue, and only the later slots' loads are counted as younger.
+    // The ring load of row t >= PF was issued in step t - PF + 1, as the last of its operations: when step t asks for it, the
+    // OPS operations of each of the PF - 1 steps since are younger (the wait allows one step's fewer).  The rows before come
+    // from the prologue, with the later slots' loads behind them and the operations of steps 1 .. t (one step's fewer again).
 #pragma unroll
     for (int u = 0; u < PF; u++)
-        if (u < S) step(u, u, u + 1 < PF ? PF - 2 - u : OPS * (PF - 2));
+        if (u < S) step(u, u, PF - 1 - u + (u > 0 ? OPS * (u - 1) : 0), u == 0);
     for (int t0 = PF; t0 < S; t0 += PF) {
 #pragma unroll
         for (int u = 0; u < PF; u++)
-            if (t0 + u < S) step(u, t0 + u, OPS * (PF - 2));
+            if (t0 + u < S) step(u, t0 + u, OPS * (PF - 2), false);
     }
+    store();
 }
 
 // Back through time with the same quads, but what step t + 1 sends back to h_t -- R^T delta_{t+1}, a vector of 4 DH gradients
 // against DH outputs -- is formed by rows of 16 lanes: the four quads of a row own four units k, and lane p of the row takes
 // a sixteenth of the gradient vector for all four of them (DH / 4 gradients x 4 columns of R: DH registers, DH multiply-adds,
 // but only DH / 4 floats of LDS reads where a lane that served one unit alone read DH: the LDS pipeline was what the step
-// waited for).  The four sums meet over the row in four DPP exchanges; every lane keeps its own unit's, and all four lanes
-// of a quad then form the unit's four pre-activation gradients alike; lane q hands on and stores gradient q (delta in two
+// waited for).  Quad Q of the row holds unit (Q + s) mod 4 as its s-th, so that three rotations with an add each bring a unit's
+// sums to its own quad, and the exchange inside the quad finishes them.
+// Everything else a step computes is linear in dh_t: with dc, dn what comes back to c_t and n_t, lane q of a quad needs
+//     dc = dh A + dc',  dn = dh B + dn',  its gradient = P dc + Q dn  (q = 3: O dh)
+// and A, B, P, Q, O are made of saved values only.  They are formed, like the stores and the ring's refill, while the step
+// waits for the gradients from LDS, so that five instructions lie between dh_t and the gradient that is handed on (delta in two
 // buffers, taken in turns: one barrier per step).  Lane q loads saved value q, and value 4 + q or, for q = 3, dh.
+// B16 NH4 S2048 DH64: 925 us with those formed behind the sum, 810 now.
 template <int DH, bool FS>
 __global__ __launch_bounds__(4 * DH) void slstm_backward_kernel(const float* __restrict__ dh, const float* __restrict__ r,
                                                                 const float* __restrict__ saved, float* __restrict__ dwx, int NH,
@@ -225,87 +248,104 @@ __global__ __launch_bounds__(4 * DH) void slstm_backward_kernel(const float* __r
     const bool is0 = q == 0, is1 = q == 1, is2 = q == 2;
     const int b = blockIdx.x / NH, hd = blockIdx.x % NH;
     const int part = tid & 15, k4 = (tid >> 4) * 4;   // the lane's part of the gradient vector; the first of its row's four units
-    float rc[PE][4];   // [gradient of the part][unit of the row]: R_g[j][k4 + u] for the part's (j, g)
+    const int urow = k & 3;                           // which of the row's units is this lane's own
+    float rc[PE][4];   // [gradient of the part][s]: R_g[j][k4 + (urow + s) mod 4] for the part's (j, g)
 #pragma unroll
     for (int e = 0; e < PE; e++) {
         const int f = part * PE + e, j = f >> 2, g = f & 3;
         const f32x4 v = *reinterpret_cast<const f32x4*>(r + (((size_t)hd * 4 + g) * DH + j) * DH + k4);
-        rc[e][0] = v[0]; rc[e][1] = v[1]; rc[e][2] = v[2]; rc[e][3] = v[3];
+#pragma unroll
+        for (int s = 0; s < 4; s++) rc[e][s] = pick(urow == 0, urow == 1, urow == 2, v[s], v[(s + 1) & 3], v[(s + 2) & 3], v[(s + 3) & 3]);
     }
-    const int urow = k & 3;   // which of the row's units is this lane's own
     const size_t step_wx = (size_t)4 * NH * DH, step_h = (size_t)NH * DH, step_s = (size_t)7 * NH * DH;
-    // (pointers that walk with the steps, from the last row down; f0, f1: the rows the ring takes next)
-    const float* f0 = saved + ((size_t)b * S + S - 1) * step_s + ((size_t)q * NH + hd) * DH + k;
+    // rows that walk with the steps, from the last one down (f0, f1: what the ring takes next; the second is saved values 4..6
+    // or dh, so its address is the lane's own)
+    const unsigned at_gate = (unsigned)((q * NH + hd) * DH + k);
+    const float* f0 = saved + ((size_t)b * S + S - 1) * step_s;
     const float* f1 = q < 3 ? saved + ((size_t)b * S + S - 1) * step_s + ((size_t)(4 + q) * NH + hd) * DH + k
                             : dh + ((size_t)b * S + S - 1) * step_h + (size_t)hd * DH + k;
     const size_t step1 = q < 3 ? step_s : step_h;
-    float* dwp = dwx + ((size_t)b * S + S - 1) * step_wx + ((size_t)q * NH + hd) * DH + k;
+    float* dwrow = dwx + ((size_t)b * S + S - 1) * step_wx;
     const int mine_at = ((4 * k + q) / PE) * PS + (4 * k + q) % PE;   // where this lane's gradient goes in a delta buffer
     const unsigned ring_base = __builtin_amdgcn_readfirstlane(mlstm::lds_offset_of(&ring[0][0][0]) + wave * 256);
     auto fetch = [&](int u, bool more) __attribute__((always_inline)) {   // (before the start of the sequence: row 0 again)
-        ring_load(f0, ring_base + (2 * u) * (4 * DH * 4));
-        ring_load(f1, ring_base + (2 * u + 1) * (4 * DH * 4));
+        ring_load(f0, 4 * at_gate, ring_base + (2 * u) * (4 * DH * 4));
+        ring_load_lane(f1, ring_base + (2 * u + 1) * (4 * DH * 4));
         if (more) { f0 -= step_s; f1 -= step1; }
     };
     constexpr int OPS = 3;   // per wave and step: the store of dwx, then two ring loads
 #pragma unroll
     for (int u = 0; u < PF; u++) fetch(u, S - 2 - u >= 0);
     for (int e = tid; e < 16 * PS; e += 4 * DH) delta[0][e] = 0.f;   // (nothing comes back to the last step)
-    float dc_next = 0.f, dn_next = 0.f;
+    float dc_next = 0.f, dn_next = 0.f, mine = 0.f;
+    f32x4 s0, s1, sp;   // i~, log f, z, o | c, n, m, dh of the step to come | c, n, m of the one before it in time
+    auto take = [&](int u) __attribute__((always_inline)) {
+        s0 = *reinterpret_cast<const f32x4*>(&ring[u % PF][0][4 * k]);
+        s1 = *reinterpret_cast<const f32x4*>(&ring[u % PF][1][4 * k]);
+        sp = *reinterpret_cast<const f32x4*>(&ring[(u + 1) % PF][1][4 * k]);
+    };
+    ring_wait(2 * (PF - 2));
+    take(0);
     __syncthreads();
-    // One step, the u-th of its round.  wait_n: how many of the wave's memory operations may still be under way when
-    // the step takes its values from the ring.
-    auto step = [&](int u, int t, int wait_n) __attribute__((always_inline)) {
+    // One step, the u-th of its round.  wait_n: how many of the wave's memory operations may still be under way when the
+    // next step's values are taken from the ring.
+    auto step = [&](int u, int t, int wait_n, bool first) __attribute__((always_inline)) {
         const float* dcur = delta[u & 1] + part * PS;
         f32x4 dl[PE / 4];
 #pragma unroll
         for (int e = 0; e < PE / 4; e++) dl[e] = *reinterpret_cast<const f32x4*>(dcur + 4 * e);
+        __builtin_amdgcn_sched_barrier(0);
+        if (!first) {   // the step before: its gradient goes out, its slot takes the row PF steps on
+            dwrow[at_gate] = mine;
+            dwrow -= step_wx;
+            fetch((u + PF - 1) % PF, t - PF >= 0);
+        }
+        if (t == 0) { sp[0] = 0.f; sp[1] = 0.f; sp[2] = -INFINITY; }
+        const float it = s0[0], logf = s0[1], z = s0[2], o = s0[3], ct = s1[0], nt = s1[1], mt = s1[2], dht = s1[3];
+        const float ip = fast_exp(it - mt);
+        float fp = fast_exp(logf + sp[2] - mt);
+        const float inv_n = fast_rcp(nt), psi = ct * inv_n;
+        float A = o * inv_n, B = -A * psi, O = psi * o * (1.0f - o);
+        // d i~ = (dc z + dn) i',  d f~ = (dc c_{t-1} + dn n_{t-1}) f' (sigmoid gate: sigmoid(-f~) = 1 - exp(log f)),  d z~ = dc i' (1 - z^2)
+        const float fs = FS ? fp * (1.0f - fast_exp(logf)) : fp;
+        float P = pick(is0, is1, true, z * ip, sp[0] * fs, ip * (1.0f - z * z), 0.f);
+        float Q = pick(is0, is1, true, ip, sp[1] * fs, 0.f, 0.f), dht_own = dht;
+        // (here, not among the multiply-adds below)
+        mlstm::pin(A); mlstm::pin(B); mlstm::pin(O); mlstm::pin(P); mlstm::pin(Q); mlstm::pin(fp); mlstm::pin(dht_own);
+        ring_wait(wait_n);
+        take(u + 1);
+        __builtin_amdgcn_sched_barrier(0);
         float a[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int e = 0; e < PE; e++)
 #pragma unroll
             for (int x = 0; x < 4; x++) a[x] += rc[e][x] * dl[e >> 2][e & 3];
-        const float r0 = row_sum(a[0]), r1 = row_sum(a[1]), r2 = row_sum(a[2]), r3 = row_sum(a[3]);
-        const float dhrec = urow == 0 ? r0 : urow == 1 ? r1 : urow == 2 ? r2 : r3;
-        ring_wait(wait_n);
-        const int un = (u + 1) % PF;
-        const f32x4 s0 = *reinterpret_cast<const f32x4*>(&ring[u][0][4 * k]);    // i~, log f, z, o
-        const f32x4 s1 = *reinterpret_cast<const f32x4*>(&ring[u][1][4 * k]);    // c, n, m, dh
-        f32x4 sp = *reinterpret_cast<const f32x4*>(&ring[un][1][4 * k]);         // c, n, m of step t - 1
-        if (t == 0) { sp[0] = 0.f; sp[1] = 0.f; sp[2] = -INFINITY; }
-        const float it = s0[0], logf = s0[1], z = s0[2], o = s0[3], ct = s1[0], nt = s1[1], mt = s1[2];
-        const float ip = fast_exp(it - mt), fp = fast_exp(logf + sp[2] - mt);
-        const float d_h = s1[3] + dhrec;
-        const float inv_n = fast_rcp(nt), psi = ct * inv_n;
-        const float d_o = d_h * psi * o * (1.0f - o);
-        const float dpsi = d_h * o;
-        const float dc = dpsi * inv_n + dc_next;
-        const float dn = -dpsi * psi * inv_n + dn_next;
-        const float d_z = dc * ip * (1.0f - z * z);
-        const float d_i = (dc * z + dn) * ip;
-        float d_f = (dc * sp[0] + dn * sp[1]) * fp;
-        if (FS) d_f *= 1.0f - fast_exp(logf);   // d logsigmoid(f~) / d f~ = sigmoid(-f~) = 1 - exp(log f)
+        // (row_ror: lane i takes from lane i - 4s of its row, whose s-th unit is this quad's own)
+        const float dhrec = quad_sum((a[0] + quad_perm<0x124>(a[1])) + (quad_perm<0x128>(a[2]) + quad_perm<0x12C>(a[3])));
+        const float d_h = dht_own + dhrec;
+        const float dc = d_h * A + dc_next, dn = d_h * B + dn_next;
+        const float lin = dc * P + dn * Q;
+        mine = q == 3 ? d_h * O : lin;
+        delta[(u & 1) ^ 1][mine_at] = mine;
         dc_next = dc * fp;
         dn_next = dn * fp;
-        const float mine = pick(is0, is1, is2, d_i, d_f, d_z, d_o);
-        delta[(u & 1) ^ 1][mine_at] = mine;
-        *dwp = mine;
-        dwp -= step_wx;
-        fetch(u, t - PF >= 1);   // (the slot's values of this step are in registers: the store took them)
+        mlstm::pin(sp);   // (its unused fourth value must not lend its register to the sums while the read is under way)
         __syncthreads();
     };
-    // Step t needs its own values (loaded PF steps ago) and c, n, m of step t - 1 (the next slot, loaded PF - 1 steps ago,
-    // as the last operations of that step): behind them lie the OPS operations of each of PF - 2 steps (the wait allows one
-    // step's fewer).  In the first round both come from the prologue, where only the later slots' loads are counted as
-    // younger; its last step's next slot is the first step's refill.  All of them are the quad's own wave's loads.
+    // Step n (of S, counted down in time) takes rows n + 1 and n + 2 for its successor.  Row m >= PF was loaded in step
+    // m - PF + 1, as the last of its operations: behind row n + 2 lie the OPS operations of each of PF - 3 steps (the wait
+    // allows one step's fewer).  The rows before come from the prologue, with the later slots' loads and the operations of
+    // steps 1 .. n (one step's fewer again) behind them.  All of them are the quad's own wave's loads.
 #pragma unroll
     for (int u = 0; u < PF; u++)
-        if (S - 1 - u >= 0) step(u, S - 1 - u, u + 1 < PF ? 2 * (PF - 2 - u) : OPS * (PF - 3));
+        if (S - 1 - u >= 0)
+            step(u, S - 1 - u, u < PF - 2 ? 2 * (PF - 3 - u) + (u > 0 ? OPS * (u - 1) : 0) : OPS * (PF - 4), u == 0);
     for (int t0 = S - 1 - PF; t0 >= 0; t0 -= PF) {
 #pragma unroll
         for (int u = 0; u < PF; u++)
-            if (t0 - u >= 0) step(u, t0 - u, OPS * (PF - 3));
+            if (t0 - u >= 0) step(u, t0 - u, OPS * (PF - 4), false);
     }
+    dwrow[at_gate] = mine;
 }
 
 constexpr int dr_parts(int DH) { return DH <= 64 ? 4 : 1; }   // partial sums per slice (slstm_dr_kernel's PARTS)
