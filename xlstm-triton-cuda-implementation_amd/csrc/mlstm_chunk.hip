@@ -575,7 +575,7 @@ __global__ __launch_bounds__(256) void chunk_carry_kernel(ChunkArgs a) {
     }
 }
 
-// The carry of the shapes of chunk_sum_small_kernel: a workgroup takes 32 keys x 32 values of a head's state, sixteen chunks'
+// The carry of the shapes of chunk_sum_small_kernel, and of the others where few workgroups would run (carry_in_small_blocks): a workgroup takes 32 keys x 32 values of a head's state, sixteen chunks'
 // sums at a time in registers (one trip to memory per sixteen steps, whatever the number of heads), writes either layout or
 // both -- the value-major one through LDS, in whole 64- or 128-byte pieces of a row -- and forms the contraction with another
 // set of states (ChunkArgs::dot_with) on the way.
@@ -701,8 +701,8 @@ __global__ __launch_bounds__(256, 4) void chunk_carry_t_kernel(ChunkArgs a) {
     float nrun = 0.f;
     __shared__ float red[4];
     const int lane = tid & 63, wave = tid >> 6;
-    // (the kernel moves 4 bytes in and 2 to 4 out per element and runs at memory speed: nothing to gain from requesting a
-    // step's chunk sums ahead of time)
+    // (the kernel moves 4 bytes in and 2 to 4 out per element and, where it is chosen, fills the chip and runs at memory speed:
+    // nothing to gain from requesting a step's chunk sums ahead of time)
     for (int step = 0; step < a.NCS; step++) {
         const int c = a.reverse ? a.NCS - 1 - step : step;
         const float gam = step > 0 ? carry_gamma(a, poff, goff, a.reverse ? c + 1 : c) : 0.f;
@@ -1163,6 +1163,25 @@ static int launch_chunk_sum(const ChunkArgs& a, hipStream_t st) {
     return 0;
 }
 
+// 16-bit D = 128 and 256: the carry in blocks of 32 x 32, sixteen steps per trip to memory, or in blocks of 64 x 64, a trip per
+// step but rows of 128 bytes.  The second moves memory faster once it fills the chip; below that it is its trips one after the
+// other.  Workgroups of the second form, chunks: training step in us, 64 x 64 / 32 x 32 (bf16):
+//   D = 128   4, 31: 253 / 159     32, 31: 427 / 339    64, 7 (gated): 135 / 119   128, 31: 1203 / 1107   192, 7: 219 / 227
+//             192, 31: 1727 / 1649   256, 7: 543 / 552   256, 31: 2187 / 2136
+//   D = 256   128, 7: 196 / 187    192, 7: 174 / 180    256, 7: 288 / 294          256, 31: 1206 / 1155    512, 15: 1073 / 1097
+static bool carry_in_small_blocks(const ChunkArgs& a, int D) {
+    const int wgs = a.BH * (D / 64) * (D / 64);
+    return wgs <= 128 || (wgs <= 256 && a.NCS >= 16);
+}
+
+template <typename T, int D>
+static int launch_chunk_carry_small(const ChunkArgs& a, hipStream_t st) {
+    const dim3 cgrid((D / 32) * (D / 32), a.BH);
+    if (a.dot_part) hipLaunchKernelGGL((chunk_carry_small_kernel<T, D, true>), cgrid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((chunk_carry_small_kernel<T, D, false>), cgrid, dim3(256), 0, st, a);
+    return (int)hipGetLastError();
+}
+
 template <typename T, int D>
 static int launch_chunk_t(const ChunkArgs& a, hipStream_t st) {
     if (a.precise && ((a.Cst && !a.Cst_lo) || (a.CstT && !a.CstT_lo))) return MLSTM_EINVAL;
@@ -1172,9 +1191,10 @@ static int launch_chunk_t(const ChunkArgs& a, hipStream_t st) {
     if (a.dot_part && !(a.CstT && a.dot_with)) return MLSTM_EINVAL;
     // (the variants of the value-major carry: with the contraction, with the key-major copy, with neither; both at once do
     // not fit the registers of four workgroups per CU, and nothing asks for both)
-    const dim3 cgrid((D / 64) * (D / 64), a.BH);
     if (a.CstT && a.dot_part && a.Cst) return MLSTM_EINVAL;
-    else if (a.CstT && a.dot_part) hipLaunchKernelGGL((chunk_carry_t_kernel<T, D, true, false>), cgrid, dim3(256), 0, st, a);
+    if (carry_in_small_blocks(a, D)) return launch_chunk_carry_small<T, D>(a, st);
+    const dim3 cgrid((D / 64) * (D / 64), a.BH);
+    if (a.CstT && a.dot_part) hipLaunchKernelGGL((chunk_carry_t_kernel<T, D, true, false>), cgrid, dim3(256), 0, st, a);
     else if (a.CstT && a.Cst) hipLaunchKernelGGL((chunk_carry_t_kernel<T, D, false, true>), cgrid, dim3(256), 0, st, a);
     else if (a.CstT) hipLaunchKernelGGL((chunk_carry_t_kernel<T, D, false, false>), cgrid, dim3(256), 0, st, a);
     else hipLaunchKernelGGL((chunk_carry_kernel<T, D>), dim3(D * D / 8 / 256, a.BH), dim3(256), 0, st, a);
@@ -1189,10 +1209,7 @@ static int launch_chunk_small(const ChunkArgs& a, hipStream_t st) {
     if (a.dot_part && !(a.CstT && a.dot_with)) return MLSTM_EINVAL;
     if (a.NCS > 1024) return MLSTM_ESHAPE;
     hipLaunchKernelGGL((chunk_sum_small_kernel<T, D>), dim3(a.BH * a.NCS * (D / 32)), dim3(256), 0, st, a);
-    const dim3 cgrid((D / 32) * (D / 32), a.BH);
-    if (a.dot_part) hipLaunchKernelGGL((chunk_carry_small_kernel<T, D, true>), cgrid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((chunk_carry_small_kernel<T, D, false>), cgrid, dim3(256), 0, st, a);
-    return (int)hipGetLastError();
+    return launch_chunk_carry_small<T, D>(a, st);
 }
 
 // Sum of dD over all pairs (query behind the end of chunk c, key up to it): the forward state at that boundary
@@ -1266,7 +1283,8 @@ int chunk_states_dot_parts(int dtype, int D, const ChunkArgs& a) {
     if (dtype == MLSTM_BF16 && D == 256) seq = chunk_seq_serves<__bf16, 256>(a);
     if (dtype == MLSTM_F16 && D == 128) seq = chunk_seq_serves<_Float16, 128>(a);
     if (dtype == MLSTM_F16 && D == 256) seq = chunk_seq_serves<_Float16, 256>(a);
-    return seq ? (D / 64) * 2 : (D / 64) * (D / 64);
+    if (seq) return (D / 64) * 2;
+    return carry_in_small_blocks(a, D) ? (D / 32) * (D / 32) : (D / 64) * (D / 64);
 }
 
 int set_state_kernel(int variant) {

@@ -211,7 +211,7 @@ template <int VB, int NKB> constexpr int scan_state_lds() {
          + 4 * VB * 3 * 64 * 16             // terms of the weighted values
          + 3 * 2 * GRAN * 4;                // gate vectors
 }
-template <int D, int VB, int NKB, bool STATE_ONLY, bool REV>
+template <int D, int VB, int NKB, bool STATE_ONLY, bool REV, bool SHARED>
 __global__ __launch_bounds__(SCAN_NW * 64) void scan_state_kernel(ScanArgs a) {
     constexpr int NW = SCAN_NW, KPW = 32 * NKB, KS = D / KPW / NW, VT = 32 * VB, NVT = D / VT, NS = 2 * NKB;
     static_assert(KS >= 1 && KS * NW * KPW == D && NVT * VT == D, "key ranges and value tiles must divide D");
@@ -236,9 +236,7 @@ __global__ __launch_bounds__(SCAN_NW * 64) void scan_state_kernel(ScanArgs a) {
     const float* K = a.k + hoff * D;
     const float* V = a.v + hoff * D;
     const double* G2 = a.G2 + (size_t)bh * NC;
-    constexpr bool MAY_SHARE = KS >= 4 && NKB == 2;
-    const bool shared = MAY_SHARE && a.shared;
-    const int part_no = shared ? ks / 2 : ks;
+    const int part_no = SHARED ? ks / 2 : ks;   // (ScanArgs::shared)
     float* out = (part_no == 0 ? a.h : a.hpart + (size_t)(part_no - 1) * a.BH * S * D) + hoff * D;
     const int kbase = (ks * NW + wave) * KPW, v0 = VT * vt;
     const float log2scale = -0.5f * __log2f((float)D);
@@ -522,7 +520,7 @@ __global__ __launch_bounds__(SCAN_NW * 64) void scan_state_kernel(ScanArgs a) {
 #pragma unroll
             for (int e = 0; e < 4; e++)
                 if (!LAST || t + e < S) {
-                    if (MAY_SHARE && shared) unsafeAtomicAdd(o + e * D, sum[e]);   // (one hardware add, nothing returned)
+                    if constexpr (SHARED) unsafeAtomicAdd(o + e * D, sum[e]);   // (one hardware add, nothing returned)
                     else o[e * D] = sum[e];
                 }
         };
@@ -689,25 +687,32 @@ __global__ __launch_bounds__(256) void scan_finish_kernel(ScanArgs a, int KS) {
     }
 }
 
-template <int D, int VB, int NKB, bool REV>
+template <int D, int VB, int NKB, bool REV, bool SHARED>
 static void launch_state(const ScanArgs& a, hipStream_t st) {
     constexpr int lds_bytes = scan_state_lds<VB, NKB>(), wg_elems = SCAN_NW * NKB * VB * 16 * 64;
     // (a failure here shows up as a launch error, which the caller reads with hipGetLastError)
-    (void)lds_limit_once<scan_state_kernel<D, VB, NKB, false, REV>>(lds_bytes);
+    (void)lds_limit_once<scan_state_kernel<D, VB, NKB, false, REV, SHARED>>(lds_bytes);
     const int wgs = a.BH * (D / (32 * VB)) * (D / (32 * NKB * SCAN_NW));
     if (a.nseg > 1) {
-        (void)lds_limit_once<scan_state_kernel<D, VB, NKB, true, REV>>(lds_bytes);
-        hipLaunchKernelGGL((scan_state_kernel<D, VB, NKB, true, REV>), dim3(wgs, a.nseg - 1), dim3(SCAN_NW * 64), lds_bytes, st, a);
+        (void)lds_limit_once<scan_state_kernel<D, VB, NKB, true, REV, false>>(lds_bytes);
+        hipLaunchKernelGGL((scan_state_kernel<D, VB, NKB, true, REV, false>), dim3(wgs, a.nseg - 1), dim3(SCAN_NW * 64), lds_bytes, st, a);
         const size_t elems = (size_t)wgs * wg_elems;   // = BH * D * D
         hipLaunchKernelGGL(scan_segcarry_kernel, dim3((unsigned)((elems + 255) / 256)), dim3(256), 0, st, a, elems, wg_elems);
     }
-    hipLaunchKernelGGL((scan_state_kernel<D, VB, NKB, false, REV>), dim3(wgs, a.nseg), dim3(SCAN_NW * 64), lds_bytes, st, a);
+    hipLaunchKernelGGL((scan_state_kernel<D, VB, NKB, false, REV, SHARED>), dim3(wgs, a.nseg), dim3(SCAN_NW * 64), lds_bytes, st, a);
 }
 
 template <int D, int VB, int NKB>
 static void launch_state_r(const ScanArgs& a, hipStream_t st) {
-    if (a.rev) launch_state<D, VB, NKB, true>(a, st);
-    else launch_state<D, VB, NKB, false>(a, st);
+    if constexpr (D / (32 * NKB * SCAN_NW) >= 2 && NKB == 2) {
+        if (a.shared) {
+            if (a.rev) launch_state<D, VB, NKB, true, true>(a, st);
+            else launch_state<D, VB, NKB, false, true>(a, st);
+            return;
+        }
+    }
+    if (a.rev) launch_state<D, VB, NKB, true, false>(a, st);
+    else launch_state<D, VB, NKB, false, false>(a, st);
 }
 
 // Tile of a wave in blocks of 32: 64 value x 64 key columns while that gives every CU a workgroup, otherwise half of the key
@@ -749,7 +754,7 @@ void launch_scan_ncarry(const ScanArgs& a, hipStream_t st) {
 }
 
 // Key ranges per value tile.
-bool scan_can_share(int BH, int D) { return scan_tile(BH, D).nkb == 2 && scan_key_splits(BH, D) >= 4; }
+bool scan_can_share(int BH, int D) { return scan_tile(BH, D).nkb == 2 && scan_key_splits(BH, D) >= 2; }
 int scan_key_parts(int BH, int D, bool shared) { return shared ? scan_key_splits(BH, D) / 2 : scan_key_splits(BH, D); }
 int scan_key_splits(int BH, int D) { return D / (32 * SCAN_NW * scan_tile(BH, D).nkb); }
 

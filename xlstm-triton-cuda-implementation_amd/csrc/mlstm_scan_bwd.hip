@@ -179,9 +179,9 @@ int launch_scan_backward(const ScanBwdArgs& a, char* ws, hipStream_t st, void (*
     if (ge != hipSuccess) return (int)ge;
 
     ScanArgs base{};
-    // Where there are four key ranges (D = 1024), pairs of them share a partial numerator: with u and a numerator of its own this
-    // pass would otherwise need five tensors of workspace, not three.  It costs 8 % (4 heads x 2048 x 1024, forward + backward:
-    // 1248 us apart, 1345 shared), which a forward, whose workspace is smaller, does not pay.
+    // Pairs of key ranges share a partial numerator where they can: with u and a numerator of its own this pass would otherwise
+    // need five tensors of workspace at D = 1024 and three at D = 512, not three and two.  It costs little (4 heads x 2048 x 1024,
+    // forward + backward: 1236 us apart, 1243 shared; 16 x 1024 x 512: 745, 749).
     base.shared = scan_can_share(BH, D) ? 1 : 0;
     base.hpart = p.hpart; base.P = p.P; base.Nst = p.Nst; base.M = p.m; base.o = a.o; base.seg_state = p.seg_state;
     base.BH = BH; base.S = S; base.D = D; base.NC = NG;
