@@ -1,0 +1,71 @@
+"""Edges of the dispatch rules: chunk lengths by length and heads, the two carries of the chunk states, fp32 operands as three
+bf16 terms, the scan form on the tile kernels and on its own, key ranges that share a partial numerator.  Forward and gradients
+against the float64 oracle: fp32 to the fp32 bound of tests/helpers.py, 16-bit types to the predicted rounding noise."""
+import pytest
+import torch
+
+from _mlstm_pkg import submodule
+from oracle import mlstm_oracle as O
+from tests.helpers import assert_close, assert_matches_oracle
+
+pytestmark = pytest.mark.gpu
+mm, ms = submodule("mlstm_matmul"), submodule("mlstm_scan")
+
+
+def _check(B, NH, S, D, dtype, seed, chunk_len=0):
+    q, k, v, f, i, dh = O.make_inputs(B, NH, S, D, dtype, seed=seed, f_mean=3.0)
+    ts = [t.cuda().requires_grad_(True) for t in (q, k, v, f, i)]
+    out = mm.Triton_mLSTM.apply(*ts)
+    assert_matches_oracle(dtype, q, k, v, f, i, dh=dh, h=out.detach(), grads=torch.autograd.grad(out, ts, dh.cuda()), chunk_len=chunk_len)
+
+
+# (16 bits: 959 / 960 and 1023 / 1024 are the first lengths in chunks, 1535 / 1536 where D = 64 and 128 change length; 8, 9 and 24,
+# 25 heads where D = 256 and 128 do; 128 workgroups of 64 x 64, 33 heads at D = 128 and 9 at D = 256, where the carry changes)
+# The last number is the chunk length the rule gives, which the noise prediction needs.
+@pytest.mark.parametrize("B,NH,S,D,L", [(1, 2, 959, 64, 0), (1, 2, 960, 64, 128), (1, 1, 1536, 64, 256), (1, 2, 960, 128, 256), (1, 1, 1023, 256, 0),
+                                        (1, 9, 1025, 256, 256), (1, 33, 1000, 128, 256), (25, 1, 1100, 128, 256), (1, 3, 1537, 128, 256)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_16_bit_chunk_lengths_and_carries(B, NH, S, D, L, dtype):
+    _check(B, NH, S, D, dtype, seed=S + NH, chunk_len=L)
+
+
+@pytest.mark.parametrize("B,NH,S,D", [(1, 2, 319, 64), (1, 2, 320, 64), (2, 1, 321, 128), (1, 1, 447, 128), (1, 3, 65, 128), (1, 1, 63, 64)])
+def test_fp32_short_chunks(B, NH, S, D):
+    _check(B, NH, S, D, torch.float32, seed=S)
+
+
+# (D = 64, 128: tile kernels; 256: one key range, 512: two that share, 1024: four in pairs and eight apart)
+@pytest.mark.parametrize("BH,S,D", [(2, 130, 64), (1, 400, 128), (3, 200, 256), (16, 70, 512), (4, 130, 1024), (1, 65, 1024)])
+def test_scan_form_every_key_split(BH, S, D):
+    q, k, v, f, i, dh = O.make_inputs(1, BH, S, D, torch.float32, seed=S + D, f_mean=3.0)
+    o = torch.randn(q.shape, generator=torch.Generator().manual_seed(D))
+    od, sg = o.double(), torch.sigmoid(o.double())
+    hd, _, _ = O.mlstm_forward_dense(q, k, v, f, i)
+    want = [hd * od * sg, *O.mlstm_backward_dense(dh.double() * od * sg, q.double(), k.double(), v.double(), f.double(), i.double(), zero_first_df=True),
+            dh.double() * hd * sg * (1 + od * (1 - sg))]
+    ts = [t.cuda().requires_grad_(True) for t in (q, k, v, f, i, o)]
+    out = ms.mlstm_scan(*ts)
+    got = [out.detach(), *torch.autograd.grad(out, ts, dh.cuda())]
+    again = ms.mlstm_scan(*ts)
+    for name, g, w, g2 in zip(("h", "dq", "dk", "dv", "df", "di", "do"), got, want, [again, *torch.autograd.grad(again, ts, dh.cuda())]):
+        assert_close(g, w, torch.float32, name)
+        assert torch.equal(g, g2), name   # (two contributions per shared element: the same bits in either order)
+
+
+# A product of three-term operands keeps fp32's range and precision over magnitudes; what is not finite stays not finite.
+@pytest.mark.parametrize("scale", [1e-12, 1.0, 1e12])
+def test_fp32_terms_over_magnitudes(scale):
+    q, k, v, f, i, _ = O.make_inputs(1, 1, 400, 64, torch.float32, seed=5, f_mean=3.0)
+    h, _, _ = O.mlstm_forward_dense(q, k, v * scale, f, i)
+    got = mm.mlstm_matmul(q.cuda(), k.cuda(), (v * scale).cuda(), f.cuda(), i.cuda())
+    assert_close(got / scale, h / scale, torch.float32, "h")
+
+
+@pytest.mark.parametrize("D", [64, 256])
+def test_fp32_terms_keep_what_is_not_finite(D):
+    q, k, v, f, i, _ = O.make_inputs(1, 1, 200, D, torch.float32, seed=6, f_mean=3.0)
+    v[0, 0, 150, 7] = float("inf")
+    got = mm.mlstm_matmul(q.cuda(), k.cuda(), v.cuda(), f.cuda(), i.cuda()).cpu()
+    assert not bool(torch.isfinite(got[0, 0, 150:, 7]).any())
+    keep = [d for d in range(D) if d != 7]
+    assert bool(torch.isfinite(got[..., keep]).all()) and bool(torch.isfinite(got[0, 0, :128]).all())
