@@ -2,8 +2,8 @@
 
 Mirror of the reference module mlstm_scan.py: ``mlstm_scan(q, k, v, f, i, o, reduce_block_size=4,
 value_block_size=4, num_warps=8)`` (:281-327), same positional order and defaults; fp32 in, fp32 out.  The three
-tuning arguments are accepted and ignored: the kernels fix their own tiling (chunks of 64 positions, 32 value columns
-per workgroup) and the result does not depend on them.
+tuning arguments are accepted and ignored: the kernels fix their own tiling (chunk length and columns
+per workgroup) and the result does not depend on the arguments.
 
 The reference's kernel path is forward only (its differentiable counterpart is the PyTorch loop mlstm_scan_pytorch,
 mlstm_scan.py:343-372).  Here ``mlstm_scan`` is differentiable: called on tensors that require a gradient it records
