@@ -351,11 +351,14 @@ __global__ __launch_bounds__(4 * DH) void slstm_backward_kernel(const float* __r
 constexpr int dr_parts(int DH) { return DH <= 64 ? 4 : 1; }   // partial sums per slice (slstm_dr_kernel's PARTS)
 // dR[h][g][j][k] and db[h][g][j] over one slice of the (b, t) pairs, on the matrix units: per head and gate this is the
 // product of dWx[g] ([pairs] x DH, taken transposed) with h_{t-1} ([pairs] x DH), the pairs being the inner dimension.
-// v_mfma_f32_32x32x2_f32 takes per lane one element of each operand -- row or column l % 32 at inner index l / 32 -- so both
+// Every fp32 operand is three bf16 terms (mlstm::Tr<float>: 24 significant bits); a lane holds row or column l % 32 at eight
+// successive pairs, 8 (l / 32) + e of a round's sixteen, so both
 // come straight from global memory, one dword per lane, rows of 128 bytes; nothing passes through LDS.  One workgroup per
 // (head, gate, slice), four waves: up to DH = 64 every wave forms the whole DH x DH block over a quarter of the slice's
 // pairs (chunks of 16, taken in turns) and leaves it as a partial sum of its own; at DH = 128 every wave forms one 64 x 64
 // quadrant over all the pairs.
+// B16 NH4 S2048 DH64: 70 us on v_mfma_f32_32x32x2_f32, bound by its 512 cycles per 32 x 32 x 16 block; 53 now (192, and the splits),
+// 134 MB of dWx and four readings of h (by gate, 34 MB each out of the caches).
 template <int DH>
 __global__ __launch_bounds__(256, 2) void slstm_dr_kernel(const float* __restrict__ dwx, const float* __restrict__ h, float* __restrict__ part_r,
                                                        float* __restrict__ part_b, int B, int NH, int S, int nslice) {
@@ -363,7 +366,8 @@ __global__ __launch_bounds__(256, 2) void slstm_dr_kernel(const float* __restric
     constexpr int W = DH < 64 ? DH : 64;   // a wave's block is W x W
     constexpr int T = W / 32;               // in T x T tiles
     constexpr int PARTS = dr_parts(DH);     // waves that share a block, each with its part of the pairs
-    constexpr int U = 8, CH = 2 * U;        // matrix instructions along the pairs per round, and the pairs they take
+    constexpr int U = 8, CH = 2 * U;        // pairs per lane and round, pairs per round
+    typedef mlstm::Tr<float> X;
     const int hg = blockIdx.x, hd = hg / 4, g = hg % 4, slice = blockIdx.y;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, hh = lane >> 5;
     const int part = PARTS > 1 ? wave : 0, quad = PARTS > 1 ? 0 : wave;
@@ -372,8 +376,8 @@ __global__ __launch_bounds__(256, 2) void slstm_dr_kernel(const float* __restric
     const long long lo = slice * per, hi = lo + per < total ? lo + per : total;
     const size_t step_wx = (size_t)4 * NH * DH, step_h = (size_t)NH * DH;
     // (a lane's place inside a pair of rows, as one 32-bit offset: the rows' own addresses are the same for the whole wave)
-    const unsigned la = (unsigned)(hh * step_wx + ((size_t)g * NH + hd) * DH + j0 + l32);
-    const unsigned lb = (unsigned)(hh * step_h + (size_t)hd * DH + k0 + l32);
+    const unsigned la = (unsigned)(U * hh * step_wx + ((size_t)g * NH + hd) * DH + j0 + l32);
+    const unsigned lb = (unsigned)(U * hh * step_h + (size_t)hd * DH + k0 + l32);
     f32x16 acc[T][T];
     float bsum[T];
 #pragma unroll
@@ -384,17 +388,17 @@ __global__ __launch_bounds__(256, 2) void slstm_dr_kernel(const float* __restric
 #pragma unroll
             for (int e = 0; e < 16; e++) acc[x][y][e] = 0.f;
     }
-    float a[2][T][U], bv[2][T][U];
-    // the operands of the round that starts at pair p0 (this lane's first pair: p0 + hh, t0 steps into its sequence)
+    X::frag a[2][T], bv[2][T];
+    // the operands of the round that starts at pair p0 (this lane's first pair: p0 + 8 hh, t0 steps into its sequence)
     auto load = [&](int set, long long p0, int t0) __attribute__((always_inline)) {
 #pragma unroll
         for (int e = 0; e < U; e++) {
-            const long long pp = p0 + 2 * e + hh;
-            int t = t0 + 2 * e;
+            const long long pp = p0 + U * hh + e;
+            int t = t0 + e;
             if (t >= S) t %= S;
             const bool in = pp < hi, prev = in && t != 0;   // (h_{-1} = 0: the first step of a sequence adds nothing to dR)
-            const float* ra = dwx + (p0 + 2 * e) * (long long)step_wx;
-            const float* rb = h + (p0 + 2 * e - 1) * (long long)step_h;
+            const float* ra = dwx + (p0 + e) * (long long)step_wx;
+            const float* rb = h + (p0 + e - 1) * (long long)step_h;
 #pragma unroll
             for (int x = 0; x < T; x++) {
                 a[set][x][e] = in ? ra[la + 32 * x] : 0.f;
@@ -403,7 +407,7 @@ __global__ __launch_bounds__(256, 2) void slstm_dr_kernel(const float* __restric
         }
     };
     long long p0 = lo + (long long)part * CH;
-    int t0 = (int)((p0 + hh) % S);
+    int t0 = (int)((p0 + U * hh) % S);
     if (p0 < hi) load(0, p0, t0);
     // one round on operand set `set` (a constant at each call); the next round's operands are under way while it multiplies
     auto round = [&](int set) __attribute__((always_inline)) {
@@ -411,15 +415,18 @@ __global__ __launch_bounds__(256, 2) void slstm_dr_kernel(const float* __restric
         int tn = t0 + PARTS * CH;
         if (tn >= S) tn %= S;
         if (pn < hi) load(set ^ 1, pn, tn);
+        X::terms ta[T], tb[T];
 #pragma unroll
-        for (int e = 0; e < U; e++) {
+        for (int x = 0; x < T; x++) {
 #pragma unroll
-            for (int x = 0; x < T; x++) {
-                bsum[x] += a[set][x][e];
-#pragma unroll
-                for (int y = 0; y < T; y++) acc[x][y] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[set][x][e], bv[set][y][e], acc[x][y], 0, 0, 0);
-            }
+            for (int e = 0; e < U; e++) bsum[x] += a[set][x][e];
+            ta[x] = X::split(a[set][x]);
+            tb[x] = X::split(bv[set][x]);
         }
+#pragma unroll
+        for (int x = 0; x < T; x++)
+#pragma unroll
+            for (int y = 0; y < T; y++) X::mma(acc[x][y], ta[x], tb[y]);
         p0 = pn;
         t0 = tn;
     };
