@@ -116,6 +116,8 @@ template <> struct Tr<_Float16> {
 // hi hi; what is left out (mid lo, lo mid, lo lo) is below 2^-26 of a product, a quarter of the rounding of ONE fp32 addition,
 // and the sums have a sixteenth of the roundings of 32x32x2 products.  Six bf16 products take 192 cycles per 32x32x16 block
 // where v_mfma_f32_32x32x2_f32 takes 512; splitting an operand is 44 vector instructions per fragment, which run beside them.
+// Outside the range of finite, normal terms: an infinite operand, or one beyond 3.39e38 (its hi rounds to infinity), makes the
+// sums it enters NaN where fp32 products could make them infinite; an operand below about 1e-33 loses its low terms.
 template <> struct Tr<float> {
     static constexpr int EPL = 8, KW = 16;
     static constexpr bool HALF = false;
