@@ -106,7 +106,9 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
         const T* hlo = nullptr;
         if constexpr (STRICT) { if (a.Hin_lo) hlo = reinterpret_cast<const T*>(a.Hin_lo) + (hoff + rowc) * D; }
         row_stats<T, NS>(xf, reinterpret_cast<const T*>(a.Hin) + offH + (size_t)rowc * rsH, h, a.Bin[hoff + rowc], a.M[hoff + rowc], inv_n, dbv, hlo);
-        if (row < S && h == 0) { a.inv_n[poff + row] = inv_n; a.db[poff + row] = dbv; }
+        // (the rows behind the sequence, up to the end of its last granule, as zeros: whoever reads whole granules multiplies
+        // them by a weight of zero, and what scratch memory holds need not be a number)
+        if (row < NG * GRAN && h == 0) { a.inv_n[poff + row] = row < S ? inv_n : 0.f; a.db[poff + row] = row < S ? dbv : 0.f; }
     }
 #pragma unroll
     for (int s = 0; s < NS; s++) pin(xf[s]);

@@ -367,7 +367,7 @@ __global__ __launch_bounds__(512) void row8_kernel(RowArgs a) {
             const int row = r0 + 32 * kh + c32;
             if (h == 0) {
                 *reinterpret_cast<float2*>(bex + ((rg * 2 + kh) * 32 + c32) * 2) = make_float2(inv, dbr);
-                if (row < S) { a.inv_n[poff + row] = inv; a.db[poff + row] = dbr; }
+                if (row < NG * GRAN) { a.inv_n[poff + row] = row < S ? inv : 0.f; a.db[poff + row] = row < S ? dbr : 0.f; }   // (see mlstm_row.hip)
             }
         }
 #pragma unroll
@@ -598,7 +598,7 @@ __global__ __launch_bounds__(512) void row8_kernel(RowArgs a) {
             const int row = r0 + 32 * dh + c32;
             if (h == 0) {
                 *reinterpret_cast<float2*>(bex + ((rg * 2 + dh) * 32 + c32) * 2) = make_float2(inv, dbr);
-                if (row < S) { a.inv_n[poff + row] = inv; a.db[poff + row] = dbr; }
+                if (row < NG * GRAN) { a.inv_n[poff + row] = row < S ? inv : 0.f; a.db[poff + row] = row < S ? dbr : 0.f; }   // (see mlstm_row.hip)
             }
         }
         const T* const Xc = reinterpret_cast<const T*>(a.X) + offX;
