@@ -207,7 +207,7 @@ def run_matmul(ffi, name, steps, warmup, precise=False, host=None):
     tflops = 7.0 * unit_flops / (ms_step * 1e-3) / 1e12
     peak = PEAK_TFLOPS[dtype]
     col_ms = kern["col"][0] / max(kern["col"][1], 1)
-    chunk = int(L.mlstm_chunk_length_for(S, D, dt_code))
+    chunk = int(L.mlstm_chunk_length(B, NH, S, D, dt_code))
     el = torch.empty(0, dtype=dtype).element_size()
     if chunk > 0 and (S + 63) // 64 <= 1024:
         executed, col_flops, col_bytes = chunk_work(S, D, BH, chunk, el, precise)

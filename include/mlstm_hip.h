@@ -348,8 +348,11 @@ int mlstm_set_column_kernel(int variant);
  */
 int mlstm_set_state_kernel(int variant);
 /* The chunk length the entry points use for this shape under the current setting, 0 = the sequence is not cut
- * (measurement aid: the work a chunked kernel executes depends on it).  It speaks for few heads and for sequences of 1024
- * positions and more; shorter ones may run in chunks as well (fp32 from 320 positions on), and 0 is returned for them. */
+ * (measurement aid: the work a chunked kernel executes depends on it).  The one exception is
+ * mlstm_forward_noalloc_ex, which takes longer chunks or none where the states do not fit its fixed workspace. */
+int mlstm_chunk_length(int B, int NH, int S, int D, int dtype);
+/* The same for one head and sequences of 1024 positions and more; 0 for every shorter one under the default setting, although fp32 runs in
+ * chunks from 320 positions on.  Kept for callers of before that: new ones ask mlstm_chunk_length. */
 int mlstm_chunk_length_for(int S, int D, int dtype);
 
 /*

@@ -46,6 +46,25 @@ def test_gradient_buffers_of_a_strided_view_keep_its_strides_and_do_not_alias():
     assert float(g.sum()) == B * NH * S * D
 
 
+def test_chunk_length_query_agrees_with_the_buffers_for_any_number_of_heads():
+    """mlstm_chunk_length against what the entry points size their buffers for: the states of a head in the buffer a
+    forward keeps for its backward (header, matrix and vector states, the gate pre-pass), on both sides of every length the rule
+    names and for few and many heads."""
+    L = ffi.lib()
+    up = lambda n: (n + 255) // 256 * 256  # noqa: E731
+    for code, el, dims in ((ffi.F32, 4, (64, 128)), (ffi.BF16, 2, (64, 128, 256)), (ffi.F16, 2, (64, 128, 256))):
+        for D in dims:
+            for S in (63, 319, 320, 500, 959, 960, 1023, 1024, 1100, 1535, 1536, 2048, 3071, 3072, 9000):
+                for BH in (1, 8, 9, 24, 25, 33, 64):
+                    length = int(L.mlstm_chunk_length(1, BH, S, D, code))
+                    assert length == int(L.mlstm_chunk_length(BH, 1, S, D, code))
+                    n = (S - 1) // length if length else 0
+                    NG = (S + 63) // 64
+                    gates = 3 * up(BH * NG * 256) + up(BH * NG * 8) + up((BH * NG * 2 + 64) * 4)
+                    want = 256 + up(BH * n * D * D * el) + up(BH * n * D * 4) + gates if n else 0
+                    assert int(L.mlstm_saved_state_bytes(1, BH, S, D, code)) == want, (code, D, S, BH, length)
+
+
 def test_tile_copy_index_arithmetic_stays_inside_the_tiles():
     """tests/harness/tile_bounds (the kernels' own offset functions, compiled for the host): every block of every tile shape
     is fetched exactly once, lands where the LDS readers expect it, and no fetch ends beyond the tile's last row -- for the

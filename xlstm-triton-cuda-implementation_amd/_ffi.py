@@ -100,6 +100,8 @@ def lib():
         L.mlstm_timing_select.argtypes = [ctypes.c_uint, ci]
         L.mlstm_set_chunk_length.restype = ci
         L.mlstm_set_chunk_length.argtypes = [ci]
+        L.mlstm_chunk_length.restype = ci
+        L.mlstm_chunk_length.argtypes = [ci] * 5
         L.mlstm_chunk_length_for.restype = ci
         L.mlstm_chunk_length_for.argtypes = [ci] * 3
         L.mlstm_kernel_error.restype = ci
@@ -140,7 +142,7 @@ def native():
 def exported_symbols():
     return ["mlstm_forward", "mlstm_backward", "mlstm_forward_ex", "mlstm_forward_noalloc_ex", "mlstm_backward_ex", "mlstm_scan_forward_ex",
             "mlstm_scan_backward_ex", "mlstm_scan_forward_save_ex", "mlstm_scan_backward_saved_ex", "slstm_saved_bytes", "slstm_workspace_bytes", "slstm_forward_ex", "slstm_backward_ex", "mlstm_forward_lx", "mlstm_backward_lx", "mlstm_forward_save_lx", "mlstm_backward_saved_lx",
-            "mlstm_forward_gated_ex", "mlstm_backward_gated_ex", "mlstm_forward_gated_lx", "mlstm_backward_gated_lx", "mlstm_set_chunk_length", "mlstm_chunk_length_for",
+            "mlstm_forward_gated_ex", "mlstm_backward_gated_ex", "mlstm_forward_gated_lx", "mlstm_backward_gated_lx", "mlstm_set_chunk_length", "mlstm_chunk_length", "mlstm_chunk_length_for",
             "mlstm_saved_state_bytes", "mlstm_forward_save_ex", "mlstm_backward_saved_ex",
             "mlstm_workspace_bytes", "mlstm_version", "mlstm_timing_enable", "mlstm_timing_select", "mlstm_timing_read",
             "mlstm_force_generic_kernels", "mlstm_kernel_error", "mlstm_set_spin_limit", "mlstm_init", "mlstm_set_column_kernel",

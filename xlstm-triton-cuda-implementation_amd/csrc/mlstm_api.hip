@@ -469,9 +469,14 @@ int mlstm_set_column_kernel(int variant) {
     return 0;
 }
 
+int mlstm_chunk_length(int B, int NH, int S, int D, int dtype) {
+    if (B <= 0 || NH <= 0 || S <= 0 || D <= 0 || !good_dtype_arg(dtype)) return 0;
+    return sizes_of(B, NH, S, D, dtype).chunk_len();
+}
+
 int mlstm_chunk_length_for(int S, int D, int dtype) {
     if (S <= 0 || D <= 0 || !good_dtype_arg(dtype)) return 0;
-    if (S < 1024 && g_chunk_override == 0) return 0;   // (shorter sequences are not reported: see the header)
+    if (S < 1024 && g_chunk_override == 0) return 0;   // (see the header)
     return chunk_len_for(dtype & ~MLSTM_PRECISE, D, (size_t)S, 1, false);
 }
 
