@@ -323,8 +323,8 @@ int mlstm_force_generic_kernels(int on);
 
 /*
  * Test and measurement aid with no counterpart in the reference.  The tile kernels (every type; D = 64, 128, and 256 in
- * 16 bits) cut long sequences into chunks -- the 16-bit types from about 1000 positions on, into 256 or 512 positions (D = 64:
- * 128 or 256) by length and number of heads, fp32 from 320 on into 128 -- : a row walks the keys of its own chunk and takes everything
+ * 16 bits) cut long sequences into chunks -- the 16-bit types from 1024 positions on into 512 positions (D = 64: 256), fp32
+ * from 320 on into 128 -- : a row walks the keys of its own chunk and takes everything
  * before it from the matrix state at the end of the previous chunk (the state of mlstm_scan.py:16-26; both forms are
  * the same function); the backward's keys likewise take the queries behind their chunk from a reverse state.  length > 0 (a multiple of 128) forces that chunk length, length < 0 switches chunking off,
  * 0 restores the default.  Process-wide; returns 0, or MLSTM_EINVAL for a length that is not a multiple of 128.
@@ -348,10 +348,11 @@ int mlstm_set_column_kernel(int variant);
  */
 int mlstm_set_state_kernel(int variant);
 /* The chunk length the entry points use for this shape under the current setting, 0 = the sequence is not cut
- * (measurement aid: the work a chunked kernel executes depends on it).  The one exception is
- * mlstm_forward_noalloc_ex, which takes longer chunks or none where the states do not fit its fixed workspace. */
+ * (measurement aid: the work a chunked kernel executes depends on it).  The default rule looks at one head, so that a head's
+ * results are the same bits alone and in any batch.  The one exception is mlstm_forward_noalloc_ex, which runs fp32 sequences of
+ * 320 to 1023 positions uncut where their chunk states do not fit its fixed workspace. */
 int mlstm_chunk_length(int B, int NH, int S, int D, int dtype);
-/* The same for one head and sequences of 1024 positions and more; 0 for every shorter one under the default setting, although fp32 runs in
+/* The same for sequences of 1024 positions and more; 0 for every shorter one under the default setting, although fp32 runs in
  * chunks from 320 positions on.  Kept for callers of before that: new ones ask mlstm_chunk_length. */
 int mlstm_chunk_length_for(int S, int D, int dtype);
 

@@ -1,4 +1,4 @@
-"""Edges of the dispatch rules: chunk lengths by length and heads, the two carries of the chunk states, fp32 operands as three
+"""Edges of the dispatch rules: chunk lengths, the two carries of the chunk states, fp32 operands as three
 bf16 terms, the scan form on the tile kernels and on its own, key ranges that share a partial numerator.  Forward and gradients
 against the float64 oracle: fp32 to the fp32 bound of tests/helpers.py, 16-bit types to the predicted rounding noise."""
 import pytest
@@ -9,7 +9,7 @@ from oracle import mlstm_oracle as O
 from tests.helpers import assert_close, assert_matches_oracle
 
 pytestmark = pytest.mark.gpu
-mm, ms = submodule("mlstm_matmul"), submodule("mlstm_scan")
+ffi, mm, ms = submodule("_ffi"), submodule("mlstm_matmul"), submodule("mlstm_scan")
 
 
 def _check(B, NH, S, D, dtype, seed, chunk_len=0):
@@ -19,14 +19,34 @@ def _check(B, NH, S, D, dtype, seed, chunk_len=0):
     assert_matches_oracle(dtype, q, k, v, f, i, dh=dh, h=out.detach(), grads=torch.autograd.grad(out, ts, dh.cuda()), chunk_len=chunk_len)
 
 
-# (16 bits: 959 / 960 and 1023 / 1024 are the first lengths in chunks, 1535 / 1536 where D = 64 and 128 change length; 8, 9 and 24,
-# 25 heads where D = 256 and 128 do; 128 workgroups of 64 x 64, 33 heads at D = 128 and 9 at D = 256, where the carry changes)
+# (16 bits: 1023 / 1024 are the last length that is not cut and the first in chunks; 128 and 132 workgroups of 64 x 64, 32 and 33
+# heads at D = 128, 8 and 9 at D = 256, are the edge of the two carries.)
 # The last number is the chunk length the rule gives, which the noise prediction needs.
-@pytest.mark.parametrize("B,NH,S,D,L", [(1, 2, 959, 64, 0), (1, 2, 960, 64, 128), (1, 1, 1536, 64, 256), (1, 2, 960, 128, 256), (1, 1, 1023, 256, 0),
-                                        (1, 9, 1025, 256, 256), (1, 33, 1000, 128, 256), (25, 1, 1100, 128, 256), (1, 3, 1537, 128, 256)])
+@pytest.mark.parametrize("B,NH,S,D,L", [(1, 2, 959, 64, 0), (1, 2, 1023, 64, 0), (1, 2, 1024, 64, 256), (1, 1, 1536, 64, 256), (1, 2, 1023, 128, 0),
+                                        (1, 1, 1023, 256, 0), (1, 9, 1025, 256, 512), (1, 33, 1024, 128, 512), (16, 2, 1100, 128, 512),
+                                        (1, 3, 1537, 128, 512)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_16_bit_chunk_lengths_and_carries(B, NH, S, D, L, dtype):
+    assert int(ffi.lib().mlstm_chunk_length(B, NH, S, D, ffi.dtype_code(dtype))) == L
     _check(B, NH, S, D, dtype, seed=S + NH, chunk_len=L)
+
+
+# A head's results are the same bits alone and in a batch, whatever the number of heads around it.
+@pytest.mark.parametrize("dtype,S,D", [(torch.bfloat16, 1000, 64), (torch.bfloat16, 1100, 128), (torch.float16, 2050, 128), (torch.bfloat16, 1500, 256),
+                                       (torch.float16, 1000, 128), (torch.float32, 400, 64), (torch.float32, 700, 128)])
+def test_a_head_is_the_same_bits_in_any_batch(dtype, S, D):
+    g = torch.Generator(device="cuda").manual_seed(S + D)
+    rnd = lambda *s: torch.randn(s, device="cuda", generator=g).to(dtype)  # noqa: E731
+    ins, dh = [rnd(1, 40, S, D), rnd(1, 40, S, D), rnd(1, 40, S, D), rnd(1, 40, S) + 3, rnd(1, 40, S)], rnd(1, 40, S, D)
+
+    def step(heads):
+        ts = [t[:, :heads].contiguous().requires_grad_(True) for t in ins]
+        out = mm.Triton_mLSTM.apply(*ts)
+        return [t[:, 0] for t in (out.detach(), *torch.autograd.grad(out, ts, dh[:, :heads].contiguous()))]
+    alone = step(1)
+    for heads in (9, 40):
+        for name, a, b in zip(("h", "dq", "dk", "dv"), alone, step(heads)):
+            assert torch.equal(a, b), (heads, name)
 
 
 @pytest.mark.parametrize("B,NH,S,D", [(1, 2, 319, 64), (1, 2, 320, 64), (2, 1, 321, 128), (1, 1, 447, 128), (1, 3, 65, 128), (1, 1, 63, 64)])

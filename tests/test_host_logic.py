@@ -57,7 +57,8 @@ def test_chunk_length_query_agrees_with_the_buffers_for_any_number_of_heads():
             for S in (63, 319, 320, 500, 959, 960, 1023, 1024, 1100, 1535, 1536, 2048, 3071, 3072, 9000):
                 for BH in (1, 8, 9, 24, 25, 33, 64):
                     length = int(L.mlstm_chunk_length(1, BH, S, D, code))
-                    assert length == int(L.mlstm_chunk_length(BH, 1, S, D, code))
+                    assert length == int(L.mlstm_chunk_length(BH, 1, S, D, code)) == int(L.mlstm_chunk_length(1, 1, S, D, code))
+                    assert S < 1024 or length == int(L.mlstm_chunk_length_for(S, D, code))
                     n = (S - 1) // length if length else 0
                     NG = (S + 63) // 64
                     gates = 3 * up(BH * NG * 256) + up(BH * NG * 8) + up((BH * NG * 2 + 64) * 4)

@@ -54,32 +54,30 @@ struct Carver {
 };
 
 // Chunk length for this shape, 0 = walk all the keys.  A chunk pays D/64 state tiles per row tile and saves the key tiles before
-// the chunk, and the states cost 2 S D^2 flops per head whatever the length.  `plain`: the lengths of a workspace that has to
-// stay small (the fixed array of mlstm_forward_noalloc_ex).
+// the chunk, and the states cost 2 S D^2 flops per head whatever the length.  The rule looks at one head, never at their number:
+// a head's results are then the same bits alone and in any batch.  `plain`: the lengths of a workspace that has to stay small
+// (the fixed array of mlstm_forward_noalloc_ex).
 int g_chunk_override = 0;   // test aid: > 0 forces this length, < 0 switches chunking off
-int chunk_len_for(int dtype, int D, size_t S, size_t BH, bool plain) {
+int chunk_len_for(int dtype, int D, size_t S, bool plain) {
     // (the chunk states are formed by 16-bit MFMA products at D = 128 and 256 and by fp32 ones at the smaller
     // shapes; every tile kernel knows chunks, the four-wave ones of fp32, of split mode and of the test switch included)
     const bool shape_ok = dtype == MLSTM_F32 ? (D == 64 || D == 128) : (D == 64 || D == 128 || D == 256);
     if (!shape_ok || g_chunk_override < 0) return 0;
     if (g_chunk_override > 0) return S > (size_t)g_chunk_override ? g_chunk_override : 0;
-    if (plain && S < 1024) return 0;
     // fp32 products run at a sixth of the 16-bit rate, so the key tiles a chunk saves weigh more against the states: the
     // shortest chunk wins at every length that has more than two of them (forward + backward, 8 heads, unchunked -> 128:
-    // D = 64 88 -> 85 us at S = 256, 142 -> 88 at 512, 469 -> 104 at 2048; D = 128 141 -> 144, 241 -> 151, 849 -> 180)
-    if (dtype == MLSTM_F32) return S >= 320 ? 128 : 0;
-    if (plain) return D == 64 ? 256 : 512;
-    // 16-bit types.  With few heads the chip is not full, a pass takes as long as its longest workgroup walks, and short chunks
-    // win; with many, what the states move through memory counts (D^2 per chunk) and long ones win.  Forward + backward in us,
-    // unchunked / 128 / 256 / 512:
-    //   D = 64    8 heads S = 1024  76 / 62 / 69 / 85     S = 4096 223 / 97 / 90 / 105    64 heads S = 1024 110 / 107 / 105 / 119
-    //   D = 128   8 heads S = 1024 105 / 91 / 85 / 99     S = 2048 182 / 127 / 108 / 113   S = 4096 335 / 199 / 151 / 138
-    //            64 heads S = 1024 194 / 165 / 140 / 138  S = 2048 475 / 330 / 270 / 258
-    //   D = 256   8 heads S = 1024 141 / 127 / 128 / 151  S = 2048 248 / 169 / 150 / 165   24 heads S = 1024 149 / 165 / 144 / 159
-    //            64 heads S = 1024 272 / 394 / 283 / 229
-    if (D == 64) return S < 960 ? 0 : (S < 1536 ? 128 : 256);
-    if (D == 128) return S < 960 ? 0 : (S < 1536 || (S < 3072 && BH <= 24) ? 256 : 512);
-    return S < 1024 ? 0 : ((S < 1536 && BH <= 24) || (S < 3072 && BH <= 8) ? 256 : 512);
+    // D = 64 88 -> 85 us at S = 256, 142 -> 88 at 512, 469 -> 104 at 2048; D = 128 141 -> 144, 241 -> 151, 849 -> 180).
+    // The states are fp32 there: errors against 64 bits at S = 384 and 700 (h, dQ, dK, dV; medians over the rows) are 0.79 to
+    // 0.91 of those of uncut sequences in 32x32x2 fp32 products.
+    if (dtype == MLSTM_F32) return S >= (plain ? 1024 : 320) ? 128 : 0;
+    // 16-bit types: what a row takes from a chunk state has been rounded to the tensor type once more, so the chunks are as
+    // long as they can be without walking most of the keys.  (Shorter ones are faster where heads are few -- training step, 8
+    // heads, 512 / 256: S = 2048 D = 128 113 / 108 us, D = 256 165 / 150 -- and less exact: dF at S = 1000, D = 128 in
+    // chunks of 256 is off by 1.06 to 1.09 times as much against 64 bits as uncut, at 1500 and 2048 in 256 instead of 512 by
+    // 1.00 to 1.03 times.)  Below two full chunks of 512 the state pass costs more than the skipped key tiles; at D = 64 256 is
+    // the measured best (B4 H8 S4096: 0.48 ms uncut, 0.24 / 0.22 / 0.25 in 128 / 256 / 512).
+    if (S < 1024) return 0;
+    return D == 64 ? 256 : 512;
 }
 
 // What mlstm_forward_save_* writes at the head of `saved` and mlstm_backward_saved_* checks on the device (no host
@@ -107,7 +105,7 @@ struct Sizes {
     bool precise = false;   // split mode (MLSTM_PRECISE): states as two terms, and the low-order part of h travels to the backward
     size_t parts() const { return precise ? 2 : 1; }   // terms per matrix state: hi, and lo directly behind it
     bool plain = false;     // see chunk_len_for
-    int chunk_len() const { return chunk_len_for(dtype_code, (int)D, S, BH, plain); }
+    int chunk_len() const { return chunk_len_for(dtype_code, (int)D, S, plain); }
     size_t state_elems() const { return BH * n_states(chunk_len()) * D * D; }             // one term of one set of states
     size_t states_t() const { return up256(state_elems() * el * parts()); }               // value-major copy for the dQ pass
     size_t saved_vec() const { return up256(BH * n_states(chunk_len()) * D * 4); }
@@ -477,7 +475,7 @@ int mlstm_chunk_length(int B, int NH, int S, int D, int dtype) {
 int mlstm_chunk_length_for(int S, int D, int dtype) {
     if (S <= 0 || D <= 0 || !good_dtype_arg(dtype)) return 0;
     if (S < 1024 && g_chunk_override == 0) return 0;   // (see the header)
-    return chunk_len_for(dtype & ~MLSTM_PRECISE, D, (size_t)S, 1, false);
+    return chunk_len_for(dtype & ~MLSTM_PRECISE, D, (size_t)S, false);
 }
 
 int mlstm_set_state_kernel(int variant) { return mlstm::set_state_kernel(variant); }
