@@ -31,21 +31,23 @@ def test_16_bit_chunk_lengths_and_carries(B, NH, S, D, L, dtype):
     _check(B, NH, S, D, dtype, seed=S + NH, chunk_len=L)
 
 
-# A head's results are the same bits alone and in a batch, whatever the number of heads around it.
+# A head's results are the same bits alone and in a batch, whatever the number of heads around it: with 40 heads the chunk states
+# of D = 128 and 256 come from the other carry, with another split of dF's sums over workgroups.
 @pytest.mark.parametrize("dtype,S,D", [(torch.bfloat16, 1000, 64), (torch.bfloat16, 1100, 128), (torch.float16, 2050, 128), (torch.bfloat16, 1500, 256),
-                                       (torch.float16, 1000, 128), (torch.float32, 400, 64), (torch.float32, 700, 128)])
-def test_a_head_is_the_same_bits_in_any_batch(dtype, S, D):
+                                       (torch.float16, 1000, 128), (torch.float32, 400, 64), (torch.float32, 700, 128), (torch.float32, 2048, 64)])
+@pytest.mark.parametrize("op", ["Triton_mLSTM", "Triton_mLSTM_precise"])
+def test_a_head_is_the_same_bits_in_any_batch(op, dtype, S, D):
     g = torch.Generator(device="cuda").manual_seed(S + D)
     rnd = lambda *s: torch.randn(s, device="cuda", generator=g).to(dtype)  # noqa: E731
     ins, dh = [rnd(1, 40, S, D), rnd(1, 40, S, D), rnd(1, 40, S, D), rnd(1, 40, S) + 3, rnd(1, 40, S)], rnd(1, 40, S, D)
 
     def step(heads):
         ts = [t[:, :heads].contiguous().requires_grad_(True) for t in ins]
-        out = mm.Triton_mLSTM.apply(*ts)
+        out = getattr(mm, op).apply(*ts)
         return [t[:, 0] for t in (out.detach(), *torch.autograd.grad(out, ts, dh[:, :heads].contiguous()))]
     alone = step(1)
     for heads in (9, 40):
-        for name, a, b in zip(("h", "dq", "dk", "dv"), alone, step(heads)):
+        for name, a, b in zip(("h", "dq", "dk", "dv", "df", "di"), alone, step(heads)):
             assert torch.equal(a, b), (heads, name)
 
 

@@ -575,6 +575,16 @@ __global__ __launch_bounds__(256) void chunk_carry_kernel(ChunkArgs a) {
     }
 }
 
+// Both carries leave the contraction of two sets of states (ChunkArgs::dot_with) as one sum per block of 32 values x 32 keys,
+// added up in one order -- the four elements of a group, the eight groups of a row, the 32 rows, each as a balanced tree -- so that
+// dF is the same bits whichever of them the number of heads selects.  (Nothing is contracted to a multiply-add here: the two
+// kernels would not agree on which.)
+__device__ __forceinline__ float dot_group(f32x4 x, f32x4 y) {
+#pragma clang fp contract(off)
+    const f32x4 p = x * y;
+    return (p[0] + p[1]) + (p[2] + p[3]);
+}
+
 // The carry of the shapes of chunk_sum_small_kernel, and of the others where few workgroups would run (carry_in_small_blocks): a workgroup takes 32 keys x 32 values of a head's state, sixteen chunks'
 // sums at a time in registers (one trip to memory per sixteen steps, whatever the number of heads), writes either layout or
 // both -- the value-major one through LDS, in whole 64- or 128-byte pieces of a row -- and forms the contraction with another
@@ -657,8 +667,7 @@ __global__ __launch_bounds__(256) void chunk_carry_small_kernel(ChunkArgs a) {
                     f32x4 xs = __builtin_convertvector(hi, f32x4), ys = __builtin_convertvector(y[u], f32x4);
                     if (split) xs += __builtin_convertvector(lo, f32x4);
                     if (a.dot_with_lo) ys += __builtin_convertvector(yl[u], f32x4);
-                    const f32x4 pr = xs * ys;
-                    const float dot = wave_reduce<OpAdd>((pr[0] + pr[1]) + (pr[2] + pr[3]));
+                    const float dot = wave_reduce<OpAdd>(dot_group(xs, ys));   // (a wave: eight rows of eight groups)
                     if (lane == 0) red[step & 1][wave] = dot;
                 }
             }
@@ -699,7 +708,7 @@ __global__ __launch_bounds__(256, 4) void chunk_carry_t_kernel(ChunkArgs a) {
     float* nst = a.Nst + (size_t)bh * a.NCS * D + tid;   // the vector states, in place, by the first workgroup of a head
     const bool vec = blockIdx.x == 0 && tid < D;
     float nrun = 0.f;
-    __shared__ float red[4];
+    __shared__ float red[4][2];
     const int lane = tid & 63, wave = tid >> 6;
     // (the kernel moves 4 bytes in and 2 to 4 out per element and, where it is chosen, fills the chip and runs at memory speed:
     // nothing to gain from requesting a step's chunk sums ahead of time)
@@ -769,10 +778,16 @@ __global__ __launch_bounds__(256, 4) void chunk_carry_t_kernel(ChunkArgs a) {
                 y0 += __builtin_convertvector(*reinterpret_cast<const V8*>(other_lo), f32x8);
                 y1 += __builtin_convertvector(*reinterpret_cast<const V8*>(other_lo + 8), f32x8);
             }
-            const f32x8 pr = x0 * y0 + x1 * y1;
-            float dot = ((pr[0] + pr[1]) + (pr[2] + pr[3])) + ((pr[4] + pr[5]) + (pr[6] + pr[7]));
-            dot = wave_scan_inclusive<OpAdd>(dot);
-            if (lane == 63) red[wave] = dot;
+            auto low = [](const f32x8& x) { return __builtin_shufflevector(x, x, 0, 1, 2, 3); };
+            auto high = [](const f32x8& x) { return __builtin_shufflevector(x, x, 4, 5, 6, 7); };
+            // a lane: four groups of a row; two lanes: the row of a block; a wave: sixteen rows of two blocks side by side
+            float dot = (dot_group(low(x0), low(y0)) + dot_group(high(x0), high(y0))) + (dot_group(low(x1), low(y1)) + dot_group(high(x1), high(y1)));
+            dot += dpp_f<0xb1>(0.f, dot);                 // quad_perm: the other lane of the pair
+            dot += dpp_f<0x114>(0.f, dot);                // row_shr:4, row_shr:8
+            dot += dpp_f<0x118>(0.f, dot);
+            auto at = [&](int l) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, dot), l)); };
+            const float left = (at(13) + at(29)) + (at(45) + at(61)), right = (at(15) + at(31)) + (at(47) + at(63));
+            if (lane == 0) { red[wave][0] = left; red[wave][1] = right; }
         }
         if (split) {
             T* dlo = reinterpret_cast<T*>(a.CstT_lo) + (dst - reinterpret_cast<T*>(a.CstT));
@@ -780,8 +795,11 @@ __global__ __launch_bounds__(256, 4) void chunk_carry_t_kernel(ChunkArgs a) {
             *reinterpret_cast<uint4*>(dlo + (size_t)c * D * D + 8) = *reinterpret_cast<const uint4*>(&tile[1][orow][16 * opiece + 8]);
         }
         __syncthreads();
-        if (DOT && tid == 0)   // (the waves' sums were written between the two barriers; the next ones follow the next barrier)
-            a.dot_part[((size_t)bh * a.NCS + c) * gridDim.x + blockIdx.x] = (red[0] + red[1]) + (red[2] + red[3]);
+        // (the waves' sums were written between the two barriers; the next ones follow the next barrier)
+        if (DOT && tid < 4) {   // block (values 32 (2 vb + tid / 2) .., keys 32 (2 kb + tid % 2) ..)
+            const int vh = tid >> 1, kh = tid & 1;
+            a.dot_part[((size_t)bh * a.NCS + c) * (D / 32) * (D / 32) + (2 * kb + kh) * (D / 32) + 2 * vb + vh] = red[2 * vh][kh] + red[2 * vh + 1][kh];
+        }
     }
 }
 
@@ -1283,8 +1301,7 @@ int chunk_states_dot_parts(int dtype, int D, const ChunkArgs& a) {
     if (dtype == MLSTM_BF16 && D == 256) seq = chunk_seq_serves<__bf16, 256>(a);
     if (dtype == MLSTM_F16 && D == 128) seq = chunk_seq_serves<_Float16, 128>(a);
     if (dtype == MLSTM_F16 && D == 256) seq = chunk_seq_serves<_Float16, 256>(a);
-    if (seq) return (D / 64) * 2;
-    return carry_in_small_blocks(a, D) ? (D / 32) * (D / 32) : (D / 64) * (D / 64);
+    return seq ? (D / 64) * 2 : (D / 32) * (D / 32);
 }
 
 int set_state_kernel(int variant) {
