@@ -125,7 +125,8 @@ int mlstm_forward_ex(const void* q, const void* k, const void* v, const void* f,
  * mlstm_forward_ex without the workspace: the scratch is a static device array of MLSTM_NOALLOC_MAX_WORKSPACE bytes
  * inside the library (each GPU the library runs on holds one until the process ends), and the call performs no
  * hipMalloc / hipFree, stream-ordered or otherwise.  Shapes whose mlstm_workspace_bytes(MLSTM_OP_FORWARD, ...) exceeds
- * that size are rejected with MLSTM_EWORKSPACE.  All calls on one GPU share the one array: two calls that overlap in
+ * that size are rejected with MLSTM_EWORKSPACE (fp32 at D >= 256 also where h is not ordinary memory of the current GPU, which
+ * then needs more).  All calls on one GPU share the one array: two calls that overlap in
  * time on the same GPU (different streams or threads) race; calls on one stream are ordered and safe.
  * (With mlstm_timing_enable on, events are created around the launches; leave it off in such callers.)
  * The first call on a device looks up the array's address (a mutex and a runtime query) and the first launch of each

@@ -83,6 +83,27 @@ def test_workspace_sizes_and_argument_errors_need_no_gpu():
     assert L.mlstm_scan_forward_ex(*([one] * 7), 1, 1, 64, 96, ffi.F32, null, 0, null) == -2
 
 
+@pytest.mark.parametrize("BH,D,more", [(1, 1024, 7), (2, 1024, 3), (3, 1024, 3), (4, 1024, 1), (40, 1024, 1), (1, 512, 3), (7, 512, 3), (8, 512, 1),
+                                       (15, 512, 1), (16, 512, 0), (128, 512, 0), (1, 256, 1), (31, 256, 1), (32, 256, 0), (63, 256, 0), (64, 256, 0)])
+def test_scan_workspace_holds_no_more_partial_numerators_than_key_ranges_need(BH, D, more):
+    """Tensors of [BH,S,D] beside the output: what two more positions per head add to the workspace (both lengths in one granule
+    and one segment, so that nothing but the [BH,S] and [BH,S,D] parts grows).  The shapes that the fixed array of
+    mlstm_forward_noalloc_ex has room for depend on it."""
+    ffi = submodule("_ffi")
+    L = ffi.lib()
+    up = lambda n: (n + 255) // 256 * 256  # noqa: E731
+    for op, own in ((ffi.OP_SCAN_FORWARD, 0), (ffi.OP_FORWARD, 0), (ffi.OP_SCAN_BACKWARD, 2)):
+        grows = int(L.mlstm_workspace_bytes(op, 1, BH, 130, D, ffi.F32)) - int(L.mlstm_workspace_bytes(op, 1, BH, 129, D, ffi.F32))
+        rows = up(BH * 130 * 4) - up(BH * 129 * 4)
+        assert grows - (more + own) * BH * D * 4 in ([2 * rows] if own == 0 else [5 * rows]), (op, grows)
+
+
+def test_shapes_the_fixed_workspace_serves():
+    ffi = submodule("_ffi")
+    for BH, S, D in ((16, 1024, 512), (16, 256, 512), (32, 512, 256)):
+        assert int(ffi.lib().mlstm_workspace_bytes(ffi.OP_FORWARD, 1, BH, S, D, ffi.F32)) <= ffi.NOALLOC_MAX_WORKSPACE, (BH, S, D)
+
+
 def test_python_wrappers_reject_bad_inputs_on_cpu():
     mm = submodule("mlstm_matmul")
     q = torch.zeros(1, 1, 8, 64)

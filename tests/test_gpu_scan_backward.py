@@ -99,6 +99,19 @@ def test_kept_forward_gives_the_same_bits(S, D):
         mlstm_scan_backward_hip(*dev, h_ungated, None)
 
 
+@pytest.mark.parametrize("BH,S,D", [(4, 130, 1024), (2, 130, 1024), (1, 70, 1024), (16, 70, 512), (8, 70, 512), (32, 65, 256)])
+def test_kept_forward_gives_the_same_bits_at_every_key_split(BH, S, D):
+    # pairs of key ranges that share a partial numerator (all but one head at 1024) and ranges apart: the forward that keeps its
+    # output and the backward's own forward add them up in the same order
+    from mlstm_scan import mlstm_scan_backward_hip, mlstm_scan_forward_save_hip
+    dev = [x.cuda() for x in O.make_inputs(1, BH, S, D, torch.float32, seed=S + D, with_o=True)]
+    q, k, v, f, i, dh, o = dev
+    _, h_ungated, b = mlstm_scan_forward_save_hip(q, k, v, f, i, o)
+    kept, plain = (mlstm_scan_backward_hip(dh, q, k, v, f, i, o, *more) for more in ((h_ungated, b), ()))
+    for name, x, y in zip(NAMES, kept, plain):
+        assert torch.equal(x, y), name
+
+
 def test_scan_backward_is_repeatable():
     q, k, v, f, i, dh, o = (x.cuda() for x in O.make_inputs(1, 4, 300, 256, torch.float32, seed=25, with_o=True))
     a = run_backward(dh, q, k, v, f, i, o)

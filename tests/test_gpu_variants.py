@@ -56,8 +56,10 @@ def test_fp32_short_chunks(B, NH, S, D):
     _check(B, NH, S, D, torch.float32, seed=S)
 
 
-# (D = 64, 128: tile kernels; 256: one key range, 512: two that share, 1024: four in pairs and eight apart)
-@pytest.mark.parametrize("BH,S,D", [(2, 130, 64), (1, 400, 128), (3, 200, 256), (16, 70, 512), (4, 130, 1024), (1, 65, 1024)])
+# (D = 64, 128: tile kernels.  Key ranges of the scan kernels by heads: 256 two apart, from 32 heads two that share, from 64 one;
+# 512 four apart, from 8 in two pairs, from 16 one pair; 1024 eight apart, from 2 heads in four pairs, from 4 in two)
+@pytest.mark.parametrize("BH,S,D", [(2, 130, 64), (1, 400, 128), (3, 200, 256), (32, 65, 256), (64, 70, 256), (3, 130, 512), (8, 70, 512), (16, 70, 512),
+                                    (1, 65, 1024), (2, 65, 1024), (4, 130, 1024)])
 def test_scan_form_every_key_split(BH, S, D):
     q, k, v, f, i, dh = O.make_inputs(1, BH, S, D, torch.float32, seed=S + D, f_mean=3.0)
     o = torch.randn(q.shape, generator=torch.Generator().manual_seed(D))
@@ -72,6 +74,18 @@ def test_scan_form_every_key_split(BH, S, D):
     for name, g, w, g2 in zip(("h", "dq", "dk", "dv", "df", "di", "do"), got, want, [again, *torch.autograd.grad(again, ts, dh.cuda())]):
         assert_close(g, w, torch.float32, name)
         assert torch.equal(g, g2), name   # (two contributions per shared element: the same bits in either order)
+
+
+# An output in host memory that the GPU can address: stores reach it, atomic adds may not, so shared partial numerators go elsewhere.
+def test_scan_kernels_with_an_output_in_pinned_host_memory():
+    q, k, v, f, i, _ = O.make_inputs(1, 16, 70, 512, torch.float32, seed=3, f_mean=3.0)
+    dev = [t.cuda() for t in (q, k, v, f, i)]
+    h = torch.zeros(q.shape, pin_memory=True)
+    null = ffi.ptr(None)
+    rc = ffi.lib().mlstm_forward_ex(*(ffi.ptr(t) for t in dev), ffi.ptr(h), null, null, 1, 16, 70, 512, ffi.F32, ffi.F32, null, 0, ffi.stream_ptr())
+    ffi.check_rc(rc, "mlstm_forward_ex")
+    torch.cuda.synchronize()
+    assert_close(h, O.mlstm_forward_dense(q, k, v, f, i)[0], torch.float32, "h")
 
 
 # A product of three-term operands keeps fp32's range and precision over magnitudes; what is not finite stays not finite.

@@ -44,6 +44,14 @@ def test_noalloc_forward_matches_forward_ex_on_two_calls_in_a_row():
         assert torch.equal(h0, h1) and torch.equal(m0, m1) and torch.equal(b0, b1), (S, D, dtype)
 
 
+@pytest.mark.parametrize("BH,S,D", [(16, 1024, 512), (16, 256, 512), (32, 512, 256), (9, 100, 512)])
+def test_noalloc_forward_of_fp32_at_large_head_dimensions(BH, S, D):
+    # (the scan form's kernels: key ranges that share a partial numerator, which is what lets these fit)
+    (h0, m0, b0), (h1, m1, b1) = forward_both(1, BH, S, D, torch.float32, S + D)
+    assert bool(torch.isfinite(h0).all()) and float(h0.abs().max()) > 0
+    assert torch.equal(h0, h1) and torch.equal(m0, m1) and torch.equal(b0, b1)
+
+
 def test_noalloc_forward_leaves_device_memory_as_it_found_it():
     """After one warm-up call per shape (which loads the kernels and looks up the scratch array), further calls must not
     change the device's free memory: nothing is allocated or freed, stream-ordered or otherwise."""

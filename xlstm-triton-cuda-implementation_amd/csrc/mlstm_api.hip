@@ -105,6 +105,7 @@ struct Sizes {
     bool precise = false;   // split mode (MLSTM_PRECISE): states as two terms, and the low-order part of h travels to the backward
     size_t parts() const { return precise ? 2 : 1; }   // terms per matrix state: hi, and lo directly behind it
     bool plain = false;     // see chunk_len_for
+    bool no_alloc = false;  // nothing may be allocated on the way (mlstm_forward_noalloc_ex)
     int chunk_len() const { return chunk_len_for(dtype_code, (int)D, S, plain); }
     size_t state_elems() const { return BH * n_states(chunk_len()) * D * D; }             // one term of one set of states
     size_t states_t() const { return up256(state_elems() * el * parts()); }               // value-major copy for the dQ pass
@@ -125,7 +126,7 @@ struct Sizes {
     // scan form: gates, m, row sums, in-chunk pairs, vector states, partial numerators of the other key ranges
     size_t scan_fwd() const {
         return gates() + stats() + up256(BH * NG * 64 * 64 * 4) + up256(BH * NG * D * 4) +
-               (size_t)(scan_key_splits((int)BH, (int)D) - 1) * up256(BH * S * D * 4) +
+               (size_t)(scan_key_parts((int)BH, (int)D, scan_can_share((int)BH, (int)D)) - 1) * up256(BH * S * D * 4) +
                up256(scan_segment_state_bytes((int)BH, (int)S, (int)D));
     }
     size_t fwd() const { return scan_engine() ? scan_fwd() : gates() + stats() + chunk_states(); }
@@ -363,6 +364,18 @@ int chunk_states_impl(const void* k, const void* v, const FwdWs& w, bool key_maj
     return launch_chunk_states(dtype, D, ca, st);
 }
 
+// Ordinary memory of the current GPU, where an fp32 atomic add of a kernel is sure to arrive (host memory that the GPU can address,
+// managed memory and another GPU's take its stores, not its adds).
+bool takes_atomics(const void* p) {
+    hipPointerAttribute_t at{};
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess || hipPointerGetAttributes(&at, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return at.type == hipMemoryTypeDevice && at.device == dev && !at.isManaged;
+}
+
 // The scan form's pipeline on a workspace of Sizes::scan_fwd() bytes: gate pre-pass, in-chunk pairs and vector carry,
 // matrix state walk, finish.  finish_mode as in ScanArgs; m_out / b_out (may be null) receive the stabiliser and the
 // normaliser sums.
@@ -379,8 +392,18 @@ int scan_forward_impl(const void* q, const void* k, const void* v, const void* f
     float* P = c.take<float>(z.BH * z.NG * 64 * 64);
     float* Nst = c.take<float>(z.BH * z.NG * z.D);
     const int KS = scan_key_splits((int)z.BH, (int)z.D);
+    // Pairs of key ranges share a numerator (the first: h) where the tile lets them; an h that atomics may not reach takes
+    // a numerator per range, from an allocation of its own.
+    bool share = scan_can_share((int)z.BH, (int)z.D);
     float* hpart = nullptr;
-    for (int p = 1; p < KS; p++) { float* x = c.take<float>(z.BH * z.S * z.D); if (p == 1) hpart = x; }
+    for (int p = 1; p < scan_key_parts((int)z.BH, (int)z.D, share); p++) { float* x = c.take<float>(z.BH * z.S * z.D); if (p == 1) hpart = x; }
+    Scratch apart;
+    if (share && !takes_atomics(h)) {
+        if (z.no_alloc) return MLSTM_EWORKSPACE;
+        if (int rc = apart.get(nullptr, 0, (size_t)(KS - 1) * z.BH * z.S * z.D * sizeof(float), st)) return rc;
+        share = false;
+        hpart = static_cast<float*>(apart.p);
+    }
     float* seg_state = c.take<float>(scan_segment_state_bytes((int)z.BH, (int)z.S, (int)z.D) / 4);
     if (m_out) m = m_out;
     (void)bw;
@@ -393,7 +416,7 @@ int scan_forward_impl(const void* q, const void* k, const void* v, const void* f
     a.q = (const float*)q; a.k = (const float*)k; a.v = (const float*)v; a.o = (const float*)o; a.h = (float*)h;
     a.alpha2 = alpha2; a.beta2 = beta2; a.G2 = G2; a.M = m; a.P = P; a.Nst = Nst; a.hpart = hpart;
     a.BH = (int)z.BH; a.S = (int)z.S; a.D = (int)z.D; a.NC = (int)z.NG;
-    a.finish_mode = finish_mode; a.Bout = b_out; a.Hun = h_ungated; a.seg_state = seg_state;
+    a.finish_mode = finish_mode; a.Bout = b_out; a.Hun = h_ungated; a.seg_state = seg_state; a.shared = share ? 1 : 0;
     return launch_scan(a, KS, st, scan_mark);
 }
 
@@ -592,7 +615,8 @@ int mlstm_forward_noalloc_ex(const void* q, const void* k, const void* v, const 
     if (!good_shape(D, dtype) || S > 131072) return MLSTM_ESHAPE;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     Sizes z = sizes_of(B, NH, S, D, dtype_arg);
-    if (z.fwd() > NOALLOC_SCRATCH_BYTES) z.plain = true;   // (chunk states of longer chunks, or none, may fit)
+    z.no_alloc = true;
+    if (z.fwd() > NOALLOC_SCRATCH_BYTES) z.plain = true;   // (no chunk states: they may not fit)
     if (z.fwd() > NOALLOC_SCRATCH_BYTES) return MLSTM_EWORKSPACE;   // the shape needs more scratch than the array holds
     char* ws = nullptr;
     if (int rc = symbols_of_current_device(&ws, nullptr)) return rc;

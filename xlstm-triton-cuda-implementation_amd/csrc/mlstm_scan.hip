@@ -704,7 +704,7 @@ static void launch_state(const ScanArgs& a, hipStream_t st) {
 
 template <int D, int VB, int NKB>
 static void launch_state_r(const ScanArgs& a, hipStream_t st) {
-    if constexpr (D / (32 * NKB * SCAN_NW) >= 2 && NKB == 2) {
+    if constexpr (D / (32 * NKB * SCAN_NW) >= 2 && VB == 2) {
         if (a.shared) {
             if (a.rev) launch_state<D, VB, NKB, true, true>(a, st);
             else launch_state<D, VB, NKB, false, true>(a, st);
@@ -753,8 +753,13 @@ void launch_scan_ncarry(const ScanArgs& a, hipStream_t st) {
     hipLaunchKernelGGL(scan_ncarry_kernel, dim3((a.D + 255) / 256, a.BH), dim3(256), 0, st, a);
 }
 
-// Key ranges per value tile.
-bool scan_can_share(int BH, int D) { return scan_tile(BH, D).nkb == 2 && scan_key_splits(BH, D) >= 2; }
+// Key ranges per value tile.  A walk with 64 value columns per workgroup has twice the key ranges that one with 32 would have; pairs
+// of them share a partial numerator, so that the workspace does not grow with them (in tensors beside the output: D = 1024 from 4
+// heads on one instead of three, D = 512 from 16 heads on none instead of one).  It costs a pass that writes zeros and adds in place of
+// stores, in us apart / shared: forward 4 heads x 2048 x 1024 306 / 311, 2 x 2048 x 1024 210 / 224, 16 x 1024 x 512 172 / 178,
+// 8 x 1024 x 512 118 / 129, 40 x 2048 x 256 456 / 474; forward + backward 2 x 2048 x 1024 868 / 905, 8 x 1024 x 512 482 / 521,
+// 40 x 2048 x 256 1902 / 2001.
+bool scan_can_share(int BH, int D) { return scan_tile(BH, D).vb == 2 && scan_key_splits(BH, D) >= 2; }
 int scan_key_parts(int BH, int D, bool shared) { return shared ? scan_key_splits(BH, D) / 2 : scan_key_splits(BH, D); }
 int scan_key_splits(int BH, int D) { return D / (32 * SCAN_NW * scan_tile(BH, D).nkb); }
 

@@ -179,9 +179,7 @@ int launch_scan_backward(const ScanBwdArgs& a, char* ws, hipStream_t st, void (*
     if (ge != hipSuccess) return (int)ge;
 
     ScanArgs base{};
-    // Pairs of key ranges share a partial numerator where they can: with u and a numerator of its own this pass would otherwise
-    // need five tensors of workspace at D = 1024 and three at D = 512, not three and two.  It costs little (4 heads x 2048 x 1024,
-    // forward + backward: 1236 us apart, 1243 shared; 16 x 1024 x 512: 745, 749).
+    // (as in the forward: a pass that is handed the forward's output and one that forms it again return the same bits)
     base.shared = scan_can_share(BH, D) ? 1 : 0;
     base.hpart = p.hpart; base.P = p.P; base.Nst = p.Nst; base.M = p.m; base.o = a.o; base.seg_state = p.seg_state;
     base.BH = BH; base.S = S; base.D = D; base.NC = NG;
@@ -204,7 +202,8 @@ int launch_scan_backward(const ScanBwdArgs& a, char* ws, hipStream_t st, void (*
     // dQ_t = N(u, v, k)_t + db_t n~_t, and rowdot_t = q_t . dQ_t
     {
         ScanArgs s = base; fwd_gates(s);
-        s.q = u; s.k = a.v; s.v = a.k; s.h = a.dq; s.finish_mode = 2;
+        s.q = u; s.k = a.v; s.v = a.k; s.h = num; s.finish_mode = 2;
+        s.ep.out = a.dq;   // (numerators stay in the workspace: shared ones are added up by atomics, which the caller's memory may not take)
         s.ep.vec = 1; s.ep.row_scale = p.db; s.ep.dot_with = a.q; s.ep.dot_out = p.rowdot;
         if (int rc = launch_scan(s, KS, st, mark)) return rc;
     }
