@@ -72,3 +72,46 @@ def test_forward_backward_in_a_hip_graph(D, dtype, S, save):
         torch.cuda.synchronize()
         for name, e, x in zip(("h", "m", "b", "dq", "dk", "dv", "df", "di"), eager, outs):
             assert torch.equal(e, x), (seed, name)
+
+
+@pytest.mark.parametrize("BH,S,D", [(16, 130, 512), (2, 130, 1024), (1, 1100, 256)])
+def test_scan_kernels_in_a_hip_graph(BH, S, D):
+    # fp32 at D >= 256: shared partial numerators (cleared and added to by kernels), segments, rows off a 16-byte boundary; the
+    # workspace is the caller's, nothing is allocated on the way
+    L, P, F32 = ffi.lib(), ffi.ptr, ffi.F32
+    shape = (1, BH, S, D, F32)
+    new = lambda: torch.empty(BH * S * D + 1, device="cuda")[1:].view(1, BH, S, D)  # noqa: E731
+    q, k, v, dh, h, dq, dk, dv = (new() for _ in range(8))
+    f, i, m, b, df, di = (torch.empty((1, BH, S), device="cuda") for _ in range(6))
+    ws, n = ffi.workspace(ffi.OP_BACKWARD, *shape, q.device)
+
+    def step():
+        st = ffi.stream_ptr()
+        ffi.check_rc(L.mlstm_forward_ex(P(q), P(k), P(v), P(f), P(i), P(h), P(m), P(b), *shape, F32, P(ws), n, st), "forward")
+        ffi.check_rc(L.mlstm_backward_ex(P(dh), P(q), P(k), P(v), P(f), P(i), P(h), P(m), P(b), P(dq), P(dk), P(dv), P(df), P(di), *shape, F32,
+                                         P(ws), n, st), "backward")
+
+    def load(seed):
+        for dst, x in zip((q, k, v, f, i, dh), O.make_inputs(1, BH, S, D, torch.float32, seed=seed, f_mean=2.0)):
+            dst.copy_(x)
+    outs = (h, m, b, dq, dk, dv, df, di)
+    load(7)
+    step()
+    torch.cuda.synchronize()
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        with torch.cuda.graph(graph, stream=side):
+            step()
+    torch.cuda.synchronize()
+    for seed in (8, 9, 10):
+        load(seed)
+        step()
+        torch.cuda.synchronize()
+        eager = [x.clone() for x in outs]
+        for x in outs:
+            x.zero_()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for name, e, x in zip(("h", "m", "b", "dq", "dk", "dv", "df", "di"), eager, outs):
+            assert torch.equal(e, x), (seed, name)

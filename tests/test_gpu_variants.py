@@ -76,6 +76,48 @@ def test_scan_form_every_key_split(BH, S, D):
         assert torch.equal(g, g2), name   # (two contributions per shared element: the same bits in either order)
 
 
+def _shifted(t, by):
+    buf = torch.zeros(t.numel() + by, dtype=t.dtype, device="cuda")
+    buf[by:] = t.flatten()
+    return buf[by:].view(t.shape)
+
+
+# Dense tensors that start off a 16-byte boundary, at the entry points that take no layout and therefore ask for no alignment: the
+# scan kernels behind the matmul form in fp32 at D >= 256, every entry point that reaches them; the same bits as on a boundary.
+@pytest.mark.parametrize("by", [1, 2])
+@pytest.mark.parametrize("BH,S,D", [(2, 300, 256), (32, 140, 256), (1, 1100, 256), (16, 130, 512), (2, 130, 1024), (4, 200, 1024)])
+def test_scan_kernels_on_rows_off_a_16_byte_boundary(BH, S, D, by):
+    g = torch.Generator(device="cuda").manual_seed(S + D)
+    rnd = lambda *s: torch.randn(s, device="cuda", generator=g)  # noqa: E731
+    q, k, v, dh, o = (rnd(1, BH, S, D) for _ in range(5))
+    f, i = rnd(1, BH, S) + 3, rnd(1, BH, S)
+    L, P, null, F32 = ffi.lib(), ffi.ptr, ffi.ptr(None), ffi.F32
+
+    def run(move):
+        q_, k_, v_, dh_, o_ = (move(t) for t in (q, k, v, dh, o))
+        new = lambda like: move(torch.zeros_like(like))  # noqa: E731
+        out, st, shape = [], ffi.stream_ptr(), (1, BH, S, D, F32)
+        h, m, b = new(q), torch.zeros_like(f), torch.zeros_like(f)
+        ins = (P(q_), P(k_), P(v_), P(f), P(i))
+        calls = [lambda: L.mlstm_forward_ex(*ins, P(h), P(m), P(b), *shape, F32, null, 0, st),
+                 lambda: L.mlstm_forward_save_ex(*ins, P(h), P(m), P(b), null, 0, *shape, F32, null, 0, st)]
+        if L.mlstm_workspace_bytes(ffi.OP_FORWARD, *shape) <= ffi.NOALLOC_MAX_WORKSPACE:
+            calls.append(lambda: L.mlstm_forward_noalloc_ex(*ins, P(h), P(m), P(b), *shape, F32, st))
+        calls.append(lambda: L.mlstm_scan_forward_ex(*ins, P(o_), P(h), *shape, null, 0, st))
+        for call in calls:
+            h.zero_()
+            ffi.check_rc(call(), "forward")
+            out += [h.clone(), m.clone(), b.clone()]
+        gr = [new(q), new(q), new(q), torch.zeros_like(f), torch.zeros_like(f)]
+        for call in (lambda: L.mlstm_backward_ex(P(dh_), *ins, null, null, null, *(P(t) for t in gr), *shape, F32, null, 0, st),
+                     lambda: L.mlstm_backward_saved_ex(P(dh_), *ins, P(h), P(m), P(b), null, 0, *(P(t) for t in gr), *shape, F32, null, 0, st)):
+            ffi.check_rc(call(), "backward")
+            out += [t.clone() for t in gr]
+        return out
+    for n, (a, w) in enumerate(zip(run(lambda t: _shifted(t, by)), run(lambda t: t.clone()))):
+        assert bool(torch.isfinite(a).all()) and torch.equal(a, w), n
+
+
 # An output in host memory that the GPU can address: stores reach it, atomic adds may not, so shared partial numerators go elsewhere.
 def test_scan_kernels_with_an_output_in_pinned_host_memory():
     q, k, v, f, i, _ = O.make_inputs(1, 16, 70, 512, torch.float32, seed=3, f_mean=3.0)

@@ -233,8 +233,9 @@ struct Scratch {
     ~Scratch() { if (owned && p) (void)hipFreeAsync(p, st); }
 };
 
-// The row tensors of a scan-form call on 16-byte boundaries, where the kernels' copies into LDS want them: the caller's own
-// where they are, otherwise stream-ordered copies (a dense view that starts inside a tensor; such calls are rare and stay valid).
+// The row tensors of a scan-form call on 16-byte boundaries, where the tile kernels' copies into LDS want them (the scan kernels
+// take any): the caller's own where they are, otherwise stream-ordered copies (a dense view that starts inside a tensor; such calls
+// are rare and stay valid).
 struct AlignedRows {
     static constexpr int MOST = 6;
     Scratch copies[MOST];
@@ -249,7 +250,8 @@ struct AlignedRows {
     }
     int take_all(std::initializer_list<const void**> ps, const Sizes& z, hipStream_t st) {
         for (const void** p : ps)
-            if (int rc = take(p, z.BH * z.S * z.D * z.el, st)) return rc;
+            if (scan_on_tiles((int)z.D))
+                if (int rc = take(p, z.BH * z.S * z.D * z.el, st)) return rc;
         return 0;
     }
 };

@@ -277,7 +277,8 @@ __global__ __launch_bounds__(SCAN_NW * 64) void scan_state_kernel(ScanArgs a) {
         else if (tid < 2 * GRAN) sgate[c % 3][1][pos] = c > 0 ? fast_exp2(dec_add - g.x) : 1.0f;
         return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, rescale)));
     };
-    // Q of a chunk into the wave's LDS (rows clamped: the chunk may be the partial one)
+    // Q of a chunk into the wave's LDS (rows clamped: the chunk may be the partial one).  The 16-byte copies want rows on 16-byte
+    // boundaries; every other access of these kernels takes any boundary of four bytes.
     const unsigned qst_off = __builtin_amdgcn_readfirstlane(lds_offset_of(qst));
     constexpr int RPI = 64 / Z::CPR, QI = 64 / RPI, QP = 16 / RPI;   // rows per copy instruction, instructions, period of the swizzle key
     unsigned q_lofs[QP];               // lane part of the source, in bytes
@@ -292,7 +293,17 @@ __global__ __launch_bounds__(SCAN_NW * 64) void scan_state_kernel(ScanArgs a) {
             dma16_s(base + (size_t)(REV ? GRAN - RPI - RPI * i : RPI * i) * D, q_lofs[i % QP], qst_off, 1024 * i);
         }
     };
+    const bool q16 = (reinterpret_cast<size_t>(a.q) & 15) == 0;   // (uniform; D is a multiple of four: one answer for all rows)
     auto fetch_q_clamped = [&](int c) {
+        if (!q16) {   // rows of a view that starts inside a tensor: the same places, four bytes at a time
+#pragma unroll 1
+            for (int i = 0; i < KPW; i++) {
+                const int w = 64 * i + lane, r = w / KPW, p = w % KPW;
+                const int t = GRAN * c + r < S ? GRAN * c + r : S - 1;
+                dma4(Q + row_of(t) * D + kbase + 4 * ((p / 4) ^ Z::key(r)) + p % 4, __builtin_amdgcn_readfirstlane(qst_off + 256 * i));
+            }
+            return;
+        }
 #pragma unroll 1
         for (int i = 0; i < QI; i++) {
             const int r = RPI * i + lane / Z::CPR;
@@ -401,7 +412,7 @@ __global__ __launch_bounds__(SCAN_NW * 64) void scan_state_kernel(ScanArgs a) {
 #pragma unroll
             for (int vb = 0; vb < VB; vb++) vt_mine[vb] = X::split(weighted(vb));
         }
-        const bool next_full = t0 + 2 * GRAN <= S;
+        const bool next_full = q16 && t0 + 2 * GRAN <= S;
         // ---- read-out of the carried state: acc[tb][vb] = decay_t * Q_c[32 tb.., k-range of this wave] . C~^T
         f32x16 acc[2][VB];
         if constexpr (!STATE_ONLY) {
