@@ -41,6 +41,32 @@ def test_sequences_around_the_prefetch_depth(B, NH, S, DH):
         assert_close(g, w, torch.float32, name)
 
 
+@pytest.mark.parametrize("DH", [32, 64, 128])
+def test_recurrent_gradient_of_what_is_not_finite(DH):
+    # one gradient of one step infinite, or beyond what rounds to a finite bf16, on the way into dR: the sums it enters are
+    # infinite or huge, as products in fp32 make them, and not NaN; every other element is as if it were not there
+    from slstm import slstm_backward_hip, slstm_forward_hip
+    wx, r, b, dh = SO.make_inputs(2, 2, 40, DH, seed=DH)
+    h, saved = slstm_forward_hip(*gpu(wx, r, b), forget_sigmoid=True)
+    clean = slstm_backward_hip(dh.cuda(), h, r.cuda(), saved, forget_sigmoid=True)
+    bad = dh.cuda()
+    bad[1, 0, 1, 5] = float("inf")    # (the first step of a sequence: its own gradients are not finite, nothing before it is)
+    dwx, dr, db = slstm_backward_hip(bad, h, r.cuda(), saved, forget_sigmoid=True)
+    for g, w in zip((dwx, dr, db), clean):
+        part = lambda t: t[:, :, :, 0] if t.dim() == 5 else t[0]  # noqa: E731  (head 0)
+        assert torch.equal(part(g), part(w))
+    assert_close(dr[1], clean[1][1], torch.float32, "dr")   # (h before the first step is zero: it adds nothing to dR)
+    assert not bool(torch.isfinite(dwx[1, 0, :, 1, 5]).all()) and not bool(torch.isfinite(db[1]).all())
+    # infinite at a later step: the rows of dR it enters are infinite with the sign of h, or NaN where its gradients are NaN
+    bad = dh.cuda()
+    bad[1, 39, 1, 5] = float("inf")
+    dwx, dr, _ = slstm_backward_hip(bad, h, r.cuda(), saved, forget_sigmoid=True)
+    last = dwx[1, 39, :, 1, 5]   # [gate]
+    for g in range(4):
+        if bool(torch.isinf(last[g])) and bool(torch.isfinite(dwx[1, :39, g, 1, 5]).all()):
+            assert torch.equal(dr[1, g, 5], torch.sign(last[g]) * torch.sign(h[1, 38, 1]) * float("inf"))
+
+
 def test_benchmark_shape_twice():
     # B16 NH4 S2048 DH64: two runs give the same bits (nothing depends on when a load lands), and match the oracle
     # (dR and db at a long sequence: test_long_sequence_and_many_heads)

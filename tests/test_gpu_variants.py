@@ -130,8 +130,8 @@ def test_scan_kernels_with_an_output_in_pinned_host_memory():
     assert_close(h, O.mlstm_forward_dense(q, k, v, f, i)[0], torch.float32, "h")
 
 
-# A product of three-term operands keeps fp32's range and precision over magnitudes; what is not finite stays not finite.
-@pytest.mark.parametrize("scale", [1e-12, 1.0, 1e12])
+# A product of three-term operands keeps fp32's range and precision over magnitudes.
+@pytest.mark.parametrize("scale", [1e-30, 1e-12, 1.0, 1e12, 1e30])
 def test_fp32_terms_over_magnitudes(scale):
     q, k, v, f, i, _ = O.make_inputs(1, 1, 400, 64, torch.float32, seed=5, f_mean=3.0)
     h, _, _ = O.mlstm_forward_dense(q, k, v * scale, f, i)
@@ -139,11 +139,75 @@ def test_fp32_terms_over_magnitudes(scale):
     assert_close(got / scale, h / scale, torch.float32, "h")
 
 
-@pytest.mark.parametrize("D", [64, 256])
-def test_fp32_terms_keep_what_is_not_finite(D):
-    q, k, v, f, i, _ = O.make_inputs(1, 1, 200, D, torch.float32, seed=6, f_mean=3.0)
-    v[0, 0, 150, 7] = float("inf")
+# An infinite operand makes infinite what it makes infinite in fp32 products, and nothing else: 150 of 200 is in a sequence that
+# is not cut, 150 of 400 in a chunk of 128 to 255 (the tile kernels take what lies before a row's chunk from a state, whose infinities
+# a row's products with it may turn into NaN, as they always could), 399 the last position.
+@pytest.mark.parametrize("value", [float("inf"), float("-inf")])
+@pytest.mark.parametrize("S,at", [(200, 150), (400, 150), (400, 399)])
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_fp32_terms_keep_what_is_not_finite(D, S, at, value):
+    q, k, v, f, i, dh = O.make_inputs(1, 1, S, D, torch.float32, seed=6, f_mean=3.0)
+    h, _, b = O.mlstm_forward_dense(q, k, v, f, i)
+    v[0, 0, at, 7] = value
     got = mm.mlstm_matmul(q.cuda(), k.cuda(), v.cuda(), f.cuda(), i.cuda()).cpu()
-    assert not bool(torch.isfinite(got[0, 0, 150:, 7]).any())
     keep = [d for d in range(D) if d != 7]
-    assert bool(torch.isfinite(got[..., keep]).all()) and bool(torch.isfinite(got[0, 0, :128]).all())
+    assert_close(got[..., keep], h[..., keep], torch.float32, "the other columns")
+    if at > 0:
+        assert_close(got[0, 0, :at], h[0, 0, :at], torch.float32, "the rows before")
+    own = min(S, (at // 128 + 1) * 128 if S > 320 and D <= 128 else S)
+    assert bool(torch.isinf(got[0, 0, at:own, 7]).all()) and not bool(torch.isfinite(got[0, 0, at:, 7]).any())
+    # in the output gradient: dV's column, for the keys up to that position; every other column is as if it were not there
+    v[0, 0, at, 7] = 0
+    dh[0, 0, at, 7] = value
+    ts = [t.cuda().requires_grad_(True) for t in (q, k, v, f, i)]
+    grads = torch.autograd.grad(mm.Triton_mLSTM.apply(*ts), ts, dh.cuda())
+    dh[0, 0, at, 7] = 0
+    want = O.mlstm_backward_dense(dh, q, k, v, f, i, zero_first_df=True)
+    assert_close(grads[2][..., keep], want[2][..., keep], torch.float32, "dv, the other columns")
+    if at + 1 < S:
+        assert_close(grads[2][0, 0, at + 1:], want[2][0, 0, at + 1:], torch.float32, "dv, the keys behind")
+    first = at // 128 * 128 if S > 320 and D <= 128 else 0
+    assert bool(torch.isinf(grads[2][0, 0, first:at + 1, 7]).all())
+    rows = [t for t in range(S) if t != at]
+    assert_close(grads[0][0, 0, rows], want[0][0, 0, rows], torch.float32, "dq, the other rows")
+
+
+# The lowest value of the type, as masks use it: it rounds to an infinite bf16.  As a value behind every row that is looked at it
+# changes nothing, not a bit.
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("S", [130, 200, 400])
+def test_fp32_terms_and_the_lowest_value(S, D):
+    q, k, v, f, i, _ = (t.cuda() for t in O.make_inputs(1, 2, S, D, torch.float32, seed=9, f_mean=3.0))
+    o = torch.randn(q.shape, generator=torch.Generator().manual_seed(S)).cuda()
+    for tail in (0.0, torch.finfo(torch.float32).min):
+        v[..., -3:, :] = tail
+        k[..., -1:, :] = tail
+        out = [mm.mlstm_matmul(q, k, v, f, i)[..., :-3, :], ms.mlstm_scan(q, k, v, f, i, o)[..., :-3, :]]
+        if tail == 0.0:
+            want = out
+    for a, w in zip(out, want):
+        assert bool(torch.isfinite(w).all())
+        assert_close(a, w, torch.float32, "the rows before")   # (a tile that had to be formed again: in another order)
+
+
+# One element of one key that rounds to an infinite bf16, where every query has a zero: scores, outputs and gradients are what
+# they are without it.  Every product with it goes wrong in terms, so all rows and keys that see it are formed again: forward, dQ, dK,
+# dV, dF and dI of those paths against the oracle, in the first chunk, behind it, and without chunks.
+@pytest.mark.parametrize("B,NH,S,D,at", [(1, 2, 200, 64, 0), (1, 1, 63, 64, 40), (1, 2, 400, 64, 3), (2, 1, 450, 64, 300), (1, 2, 200, 128, 100),
+                                         (1, 2, 450, 128, 3), (1, 1, 450, 128, 449), (1, 2, 200, 256, 3), (1, 16, 70, 512, 10)])
+def test_fp32_rows_and_keys_formed_again(B, NH, S, D, at):
+    q, k, v, f, i, dh = O.make_inputs(B, NH, S, D, torch.float32, seed=S + at, f_mean=3.0)
+    q[..., 7] = 0
+    k[..., at, 7] = 0
+    dh *= 1e-3   # (so that what the element itself contributes, to column 7 of dQ, stays finite)
+    want = [O.mlstm_forward_dense(q, k, v, f, i)[0], *O.mlstm_backward_dense(dh, q, k, v, f, i, zero_first_df=True)]
+    k[..., at, 7] = 3.4e38
+    ts = [t.cuda().requires_grad_(True) for t in (q, k, v, f, i)]
+    out = mm.Triton_mLSTM.apply(*ts)
+    got = [out.detach(), *torch.autograd.grad(out, ts, dh.cuda())]
+    keep = [d for d in range(D) if d != 7]
+    got[1], want[1] = got[1][..., keep], want[1][..., keep]
+    for name, g, w in zip(("h", "dq", "dk", "dv", "df", "di"), got, want):
+        assert_close(g, w, torch.float32, name)
+    o = torch.randn(q.shape, generator=torch.Generator().manual_seed(S)).cuda()
+    assert_close(ms.mlstm_scan(*(t.detach() for t in ts), o), want[0] * (o * torch.sigmoid(o)).cpu().double(), torch.float32, "scan form")

@@ -41,6 +41,77 @@ struct RowCfg {
     // plus one double per key tile of the head (the granule bases), appended at launch
 };
 
+// One row by one wave from its definition, in fp32 multiply-adds straight from memory (see not_finite in mlstm_device.h): the keys
+// of the row's own chunk one after the other and the state before it, columns lane and lane + 64.  Positions count from the
+// chunk's first one, as in the kernel.
+template <int D, int MODE>
+__device__ __forceinline__ void row_exact(const RowArgs& a, int bh, int chunk, int t, int S, size_t hoff, size_t poff, size_t goff, const float* x,
+                                          const float* Y1, const float* Y2, size_t rsA, size_t offA, size_t offO, size_t offB, size_t rsO, size_t rsB,
+                                          float inv_n, float db) {
+    constexpr int NC = D / 64;
+    const int lane = threadIdx.x & 63;
+    const double G = a.G2[goff + t / GRAN];
+    const float crow = -0.5f * __log2f((float)D) - a.beta2[poff + t];
+    float xv[NC], o[NC], b = 0.f;
+#pragma unroll
+    for (int n = 0; n < NC; n++) { xv[n] = x[lane + 64 * n]; o[n] = 0.f; }
+    if (chunk > 0) {
+        const size_t st = (size_t)bh * a.n_states + chunk - 1;
+        const float* C = reinterpret_cast<const float*>(a.Cst) + st * D * D;
+        const float* nst = a.Nst + st * D;
+        for (int k = 0; k < D; k++) {   // (row k of the state lies where the tile kernels' transposing reads want it: mlstm_chunk.hip)
+            const float xk = x[k];
+            const int at = (k & ~12) | ((k & 4) << 1) | ((k & 8) >> 1);
+#pragma unroll
+            for (int n = 0; n < NC; n++) o[n] += xk * C[(size_t)at * D + lane + 64 * n];
+            if constexpr (MODE == MODE_FWD) b += xk * nst[k];
+        }
+        const float dec = fast_exp2(a.beta2[poff - 1] - a.beta2[poff + t] + (float)(G - a.G2[goff - 1]));
+        if constexpr (MODE == MODE_FWD) {
+            b *= dec;
+#pragma unroll
+            for (int n = 0; n < NC; n++) o[n] *= dec;
+        } else {
+            const float* q = reinterpret_cast<const float*>(a.Qrow) + offA + (size_t)t * rsA;
+            float rp = 0.f;
+#pragma unroll
+            for (int n = 0; n < NC; n++) {
+                o[n] = o[n] * (dec * inv_n) + dec * db * nst[lane + 64 * n];
+                rp += o[n] * q[lane + 64 * n];
+            }
+            rp = wave_reduce<OpAdd>(rp);
+            if (lane == (t & 31)) a.rowinter[hoff + t] = rp;
+        }
+    }
+    for (int j = 0; j <= t; j++) {
+        float s = 0.f;
+#pragma unroll
+        for (int n = 0; n < NC; n++) s += xv[n] * Y1[(size_t)j * rsA + lane + 64 * n];
+        s = wave_reduce<OpAdd>(s);
+        const float e = fast_exp2(a.alpha2[poff + j] + (crow + (float)(G - a.G2[goff + j / GRAN])));
+        const float p = MODE == MODE_FWD ? s * e : (s * inv_n + db) * e;
+        b += p;
+#pragma unroll
+        for (int n = 0; n < NC; n++) o[n] += p * Y2[(size_t)j * rsA + lane + 64 * n];
+    }
+    float onorm = 1.0f;
+    if constexpr (MODE == MODE_FWD) {
+        onorm = 1.0f / (fmaxf(fabsf(b), __expf(-a.M[hoff + t])) + 1e-6f);
+        if (lane == (t & 31)) a.Bsum[hoff + t] = b;
+    }
+#pragma unroll
+    for (int n = 0; n < NC; n++) {
+        const int d = lane + 64 * n;
+        reinterpret_cast<float*>(a.out)[offO + (size_t)t * rsO + d] = o[n] * onorm;
+        if constexpr (MODE == MODE_FWD) {
+            if (a.O) {
+                const size_t at = offB + (size_t)t * rsB + d;
+                reinterpret_cast<float*>(a.out_gated)[at] = o[n] * onorm * silu(reinterpret_cast<const float*>(a.O)[at]);
+            }
+        }
+    }
+}
+
 // STRICT (16-bit types): split mode, see RowArgs::precise.
 template <typename T, int D, int MODE, bool STRICT>
 __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
@@ -542,15 +613,33 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
 #undef ST_Y1
 #undef ST_Y2
 #undef ST_AL
-    float onorm = 1.0f;
+    float onorm = 1.0f, brow = 0.f;
     if constexpr (MODE == MODE_FWD) {
-        const float b = sum_halves(bsum);
+        brow = sum_halves(bsum);
         const float m = a.M[hoff + rowc];
-        const float n = fmaxf(fabsf(b), __expf(-m)) + 1e-6f;
+        const float n = fmaxf(fabsf(brow), __expf(-m)) + 1e-6f;
         onorm = 1.0f / n;
-        if (row < S && h == 0) a.Bsum[hoff + row] = b;
     }
-    if (row < S) {
+    bool mine = row < S;   // (this lane writes its half of the row)
+    if constexpr (F32) {   // rows that are not finite, from their definition (see not_finite)
+        float seen = not_finite(0.f, brow);
+#pragma unroll
+        for (int d = 0; d < NDB; d++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) seen = not_finite(seen, oacc[d][r]);
+        const unsigned long long halves = __ballot(mine && seen != 0.f);
+        unsigned bad = (unsigned)halves | (unsigned)(halves >> 32);
+        mine = mine && !((bad >> c32) & 1);
+        for (; bad; bad &= bad - 1) {
+            const int b = __builtin_ctz(bad);
+            row_exact<D, MODE>(a, bh, chunk, r0 + b, S, hoff, poff, goff, X + (size_t)(r0 + b) * rsX, Y1, Y2, rsA, offA, offO, offB, rsO, rsB,
+                               __shfl(inv_n, b), __shfl(dbv, b));
+        }
+    }
+    if constexpr (MODE == MODE_FWD) {
+        if (mine && h == 0) a.Bsum[hoff + row] = brow;
+    }
+    if (mine) {
         T* out = reinterpret_cast<T*>(a.out) + offO + (size_t)row * rsO;
 #pragma unroll
         for (int d = 0; d < NDB; d++)

@@ -614,14 +614,71 @@ __global__ __launch_bounds__(256) void scan_segcarry_kernel(ScanArgs a, size_t e
 }
 
 // ---------------------------------------------------------------------------------------------------------------
+// The numerator of a row from its definition (see not_finite in mlstm_device.h): columns 4 lane + 256 n .. of
+//   sum_{j<=t} exp(a_j - A_t) / sqrt(D) (q_t . k_j) v_j,
+// the vector sum that may ride along (ScanArgs::Epilogue::vec) for the pairs inside the row's chunk only, as in P.
+template <int D>
+__device__ __forceinline__ void scan_numerator_exact(const ScanArgs& a, int bh, int t, f32x4 (&x)[D / 256]) {
+    constexpr int NB = D / 256;
+    const int lane = threadIdx.x & 63, S = a.S, c = t / GRAN;
+    const size_t hoff = (size_t)bh * S, poff = (size_t)bh * a.NC * GRAN;
+    auto row_of = [&](int j) { return (hoff + (a.rev ? S - 1 - j : j)) * D; };
+    const float log2scale = -0.5f * __log2f((float)D);
+    const bool vec = a.finish_mode == 2 && a.ep.vec;
+    const float rs = vec && a.ep.row_scale ? a.ep.row_scale[hoff + t] : 1.0f;
+    const double G = a.G2[(size_t)bh * a.NC + c];
+    const float beta = a.beta2[poff + t];
+    const float* q = a.q + row_of(t) + 4 * lane;
+#pragma unroll
+    for (int n = 0; n < NB; n++) x[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+    for (int j = 0; j <= t; j++) {
+        const size_t r = row_of(j);
+        float s = 0.f;
+#pragma unroll 1   // (as few registers as it takes: the kernel around this wants its waves)
+        for (int k = 0; k < D; k += 256) {
+            const f32x4 qv = *reinterpret_cast<const f32x4*>(q + k), kv = *reinterpret_cast<const f32x4*>(a.k + r + 4 * lane + k);
+            s += qv[0] * kv[0] + qv[1] * kv[1] + qv[2] * kv[2] + qv[3] * kv[3];
+        }
+        s = wave_reduce<OpAdd>(s);
+        if (vec && j / GRAN == c) s += rs * (a.col_scale ? a.col_scale[hoff + (a.rev ? S - 1 - j : j)] : 1.0f);
+        s *= fast_exp2(a.alpha2[poff + j] - beta + (float)(G - a.G2[(size_t)bh * a.NC + j / GRAN]) + log2scale);
+#pragma unroll
+        for (int n = 0; n < NB; n++) {
+            const int k = 4 * lane + 256 * n;
+            x[n] += s * *reinterpret_cast<const f32x4*>(a.v + r + k);
+        }
+        if ((j & 15) == 15) {   // (a row of nothing but NaN stays that)
+            bool number = false;
+#pragma unroll
+            for (int n = 0; n < NB; n++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) number = number || x[n][e] == x[n][e];
+            if (!__any(number)) break;
+        }
+    }
+}
+
 // one wave per row: normaliser sum, then the row of h
+template <int D>
 __global__ __launch_bounds__(256) void scan_finish_kernel(ScanArgs a, int KS) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    constexpr int NB = D / 256;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const size_t rows = (size_t)a.BH * a.S;
-    const int D = a.D;
     for (size_t row = (size_t)blockIdx.x * 4 + wave; row < rows; row += (size_t)gridDim.x * 4) {
         const int bh = (int)(row / a.S), t = (int)(row % a.S), c = t / GRAN;
         const size_t poff = (size_t)bh * a.NC * GRAN;
+        f32x4 num[NB];   // the row's numerator, columns 4 lane + 256 n ..
+        float seen = 0.f;
+#pragma unroll
+        for (int n = 0; n < NB; n++) {
+            const int k = 4 * lane + 256 * n;
+            num[n] = *reinterpret_cast<const f32x4*>(a.h + row * D + k);
+            for (int p = 1; p < KS; p++) num[n] += *reinterpret_cast<const f32x4*>(a.hpart + ((size_t)(p - 1) * rows + row) * D + k);
+#pragma unroll
+            for (int e = 0; e < 4; e++) seen = not_finite(seen, num[n][e]);
+        }
+        if (__any(seen != 0.f)) scan_numerator_exact<D>(a, bh, t, num);
         if (a.finish_mode == 2) {
             const ScanArgs::Epilogue& ep = a.ep;
             const size_t orow = ep.out_rev ? (size_t)bh * a.S + (a.S - 1 - t) : row;
@@ -634,9 +691,10 @@ __global__ __launch_bounds__(256) void scan_finish_kernel(ScanArgs a, int KS) {
             const float wd = ep.wd_alpha2 ? fast_exp2(ep.wd_alpha2[poff + (orow - (size_t)bh * a.S)] - ep.wd_beta2[poff + (orow - (size_t)bh * a.S)]) : 1.0f;
             float* const dst = (ep.out ? ep.out : a.h) + orow * D;
             float acc = 0.f;
-            for (int k = 4 * lane; k < D; k += 256) {
-                f32x4 x = *reinterpret_cast<const f32x4*>(a.h + row * D + k);
-                for (int p = 1; p < KS; p++) x += *reinterpret_cast<const f32x4*>(a.hpart + ((size_t)(p - 1) * rows + row) * D + k);
+#pragma unroll
+            for (int n = 0; n < NB; n++) {
+                const int k = 4 * lane + 256 * n;
+                f32x4 x = num[n];
                 if (carried) {
                     const f32x4 cv = *reinterpret_cast<const f32x4*>(cr + k);
 #pragma unroll
@@ -676,12 +734,10 @@ __global__ __launch_bounds__(256) void scan_finish_kernel(ScanArgs a, int KS) {
         const float b = dot + wave_reduce<OpAdd>(prow);
         const float inv = 1.0f / (fmaxf(fabsf(b), __expf(-a.M[row])) + 1e-6f);
         if (a.Bout && lane == 0) a.Bout[row] = b;
-        for (int k = 4 * lane; k < D; k += 256) {
-            f32x4 x = *reinterpret_cast<const f32x4*>(a.h + row * D + k);
-            for (int p = 1; p < KS; p++) {
-                const f32x4 y = *reinterpret_cast<const f32x4*>(a.hpart + ((size_t)(p - 1) * rows + row) * D + k);
-                x += y;
-            }
+#pragma unroll
+        for (int n = 0; n < NB; n++) {
+            const int k = 4 * lane + 256 * n;
+            f32x4 x = num[n];
             if (a.finish_mode == 0) {
                 const f32x4 ov = *reinterpret_cast<const f32x4*>(a.o + row * D + k);
 #pragma unroll
@@ -755,7 +811,7 @@ static int launch_scan_d(const ScanArgs& a, int parts, hipStream_t st, void (*ma
     mark(MLSTM_K_SCAN_OUT, st, true);
     const size_t rows = (size_t)a.BH * a.S;
     const int blocks = (int)((rows + 3) / 4 < 16384 ? (rows + 3) / 4 : 16384);
-    hipLaunchKernelGGL(scan_finish_kernel, dim3(blocks), dim3(256), 0, st, a, parts);
+    hipLaunchKernelGGL(scan_finish_kernel<D>, dim3(blocks), dim3(256), 0, st, a, parts);
     mark(MLSTM_K_SCAN_OUT, st, false);
     return (int)hipGetLastError();
 }

@@ -442,13 +442,34 @@ __global__ __launch_bounds__(256, 2) void slstm_dr_kernel(const float* __restric
     // (every wave's partial sum is a slice of its own for the kernel that adds the slices)
     const size_t sl = (size_t)slice * PARTS + part;
     float* out = part_r + ((sl * NH * 4 + hg) * DH) * DH;
+    float seen = 0.f;
 #pragma unroll
     for (int x = 0; x < T; x++)
 #pragma unroll
         for (int y = 0; y < T; y++)
 #pragma unroll
-            for (int e = 0; e < 16; e++)
-                out[(size_t)(j0 + 32 * x + 8 * (e / 4) + 4 * hh + e % 4) * DH + k0 + 32 * y + l32] = acc[x][y][e];
+            for (int e = 0; e < 16; e++) seen = mlstm::not_finite(seen, acc[x][y][e]);
+    if (__any(seen != 0.f)) {   // a block that is not finite, in fp32 multiply-adds straight from memory (see not_finite in mlstm_device.h)
+#pragma unroll 1
+        for (int n = lane; n < W * W; n += 64) {
+            const int j = j0 + n / W, k = k0 + n % W;
+            float sum = 0.f;
+#pragma unroll 1
+            for (long long c0 = lo + (long long)part * CH; c0 < hi; c0 += (long long)PARTS * CH)
+#pragma unroll 1
+                for (long long pp = c0; pp < c0 + CH && pp < hi; pp++)
+                    if (pp % S != 0) sum += dwx[pp * step_wx + ((size_t)g * NH + hd) * DH + j] * h[(pp - 1) * step_h + (size_t)hd * DH + k];
+            out[(size_t)j * DH + k] = sum;
+        }
+    } else {
+#pragma unroll
+        for (int x = 0; x < T; x++)
+#pragma unroll
+            for (int y = 0; y < T; y++)
+#pragma unroll
+                for (int e = 0; e < 16; e++)
+                    out[(size_t)(j0 + 32 * x + 8 * (e / 4) + 4 * hh + e % 4) * DH + k0 + 32 * y + l32] = acc[x][y][e];
+    }
     if (k0 == 0 && hh == 0) {
 #pragma unroll
         for (int x = 0; x < T; x++) part_b[(sl * NH * 4 + hg) * DH + j0 + 32 * x + l32] = bsum[x];
