@@ -130,6 +130,28 @@ def test_scan_kernels_with_an_output_in_pinned_host_memory():
     assert_close(h, O.mlstm_forward_dense(q, k, v, f, i)[0], torch.float32, "h")
 
 
+# Errors against 64 bits, medians over the rows of h, dQ, dK and dV, for inputs that the generator fixes: no larger than the same
+# operators had on v_mfma_f32_32x32x2_f32 (the scan form on the scan kernels), which gave the bounds below on these inputs.
+@pytest.mark.parametrize("form,S,D,bounds", [("scan", 1000, 64, (2.582e-7, 3.510e-7, 9.778e-7, 3.905e-7)),
+                                             ("scan", 1000, 128, (2.748e-7, 3.767e-7, 1.167e-6, 4.359e-7)),
+                                             ("matmul", 300, 128, (3.037e-7, 4.530e-7, 1.528e-6, 6.394e-7)),
+                                             ("matmul", 1000, 64, (2.720e-7, 3.847e-7, 1.217e-6, 5.665e-7)),
+                                             ("scan", 500, 256, (2.838e-7, 4.002e-7, 1.146e-6, 4.859e-7))])
+def test_fp32_errors_against_64_bits(form, S, D, bounds):
+    q, k, v, f, i, dh, o = O.make_inputs(1, 4, S, D, torch.float32, seed=S + D, f_mean=3.0, with_o=True)
+    if form == "scan":
+        ts = [t.cuda().requires_grad_(True) for t in (q, k, v, f, i, o)]
+        out = ms.mlstm_scan(*ts)
+        want = [O.mlstm_scan_dense(q, k, v, f, i, o), *O.mlstm_gated_backward_dense(dh, q, k, v, f, i, o, zero_first_df=True)]
+    else:
+        ts = [t.cuda().requires_grad_(True) for t in (q, k, v, f, i)]
+        out = mm.Triton_mLSTM.apply(*ts)
+        want = [O.mlstm_forward_dense(q, k, v, f, i)[0], *O.mlstm_backward_dense(dh, q, k, v, f, i, zero_first_df=True)]
+    got = [out.detach(), *torch.autograd.grad(out, ts, dh.cuda())]
+    errors = [float(((g.double().cpu() - w.double()).norm(dim=-1) / w.double().norm(dim=-1)).median()) for g, w in zip(got[:4], want[:4])]
+    assert all(e <= 1.01 * bound for e, bound in zip(errors, bounds)), (errors, bounds)   # (1.01: the bounds' own digits, and D = 256, level)
+
+
 # A product of three-term operands keeps fp32's range and precision over magnitudes.
 @pytest.mark.parametrize("scale", [1e-30, 1e-12, 1.0, 1e12, 1e30])
 def test_fp32_terms_over_magnitudes(scale):

@@ -67,8 +67,8 @@ int chunk_len_for(int dtype, int D, size_t S, bool plain) {
     // fp32 products run at a sixth of the 16-bit rate, so the key tiles a chunk saves weigh more against the states: the
     // shortest chunk wins at every length that has more than two of them (forward + backward, 8 heads, unchunked -> 128:
     // D = 64 88 -> 85 us at S = 256, 142 -> 88 at 512, 469 -> 104 at 2048; D = 128 141 -> 144, 241 -> 151, 849 -> 180).
-    // The states are fp32 there: errors against 64 bits at S = 384 and 700 (h, dQ, dK, dV; medians over the rows) are 0.79 to
-    // 0.91 of those of uncut sequences in 32x32x2 fp32 products.
+    // The states are fp32 there: errors against 64 bits at S = 384 and 700 (h, dQ, dK, dV; medians over the rows) are 0.63 to
+    // 0.78 of those of uncut sequences in 32x32x2 fp32 products.
     if (dtype == MLSTM_F32) return S >= (plain ? 1024 : 320) ? 128 : 0;
     // 16-bit types: what a row takes from a chunk state has been rounded to the tensor type once more, so the chunks are as
     // long as they can be without walking most of the keys.  (Shorter ones are faster where heads are few -- training step, 8

@@ -19,6 +19,7 @@
 // ahead of the query loop:  dK_j = w_j (E v_j + g),  dV_j = w_j E^T k_j,  w_j = exp(a_j - A_e), e the chunk's last
 // position, and k_j . dK_j of that part goes into the column sums.  In split mode E comes as two terms, hi + lo.
 #include <mutex>
+#include <algorithm>
 #include <type_traits>
 #include "mlstm_device.h"
 #include "mlstm_kernels.h"
@@ -35,6 +36,7 @@ struct ColCfg {
     static constexpr size_t TILE_ELEMS = (size_t)GRAN * D;
     static constexpr size_t STAGE_BYTES = 2 * TILE_ELEMS * sizeof(T) + 3 * GRAN * sizeof(float);  // Q, dH, (beta, 1/n, db)
     static constexpr size_t G_BYTES = (size_t)GRAN * LDG * sizeof(TG);
+    typedef typename std::conditional<Tr<T>::HALF, float, double>::type Base;   // granule bases (fp32: see Crow in mlstm_row.hip)
     // G, W (split mode: and their low-order terms), row-sum scratch.  With the two extra tiles the 16-bit D = 256 case
     // no longer fits two query stages and runs single-staged.
     static constexpr int PLANES = !Tr<T>::HALF ? 3 : (STRICT ? 2 : 1);
@@ -162,7 +164,8 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
     float* const rowtmp = reinterpret_cast<float*>(Gs + 2 * Cfg::PLANES * GRAN * LDG);  // [2][64]
     float* const cpart = rowtmp + 2 * GRAN;                                               // [4][64]
     // granule bases minus this key tile's (see row kernel)
-    float* const sG = reinterpret_cast<float*>(smem + Cfg::LDS_BYTES + (a.chunk_len > 0 ? Cfg::EXTRA_CHUNK_BYTES : 0));
+    typedef typename Cfg::Base Base;
+    Base* const sG = reinterpret_cast<Base*>(smem + Cfg::LDS_BYTES + (a.chunk_len > 0 ? Cfg::EXTRA_CHUNK_BYTES : 0));
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = lane >> 5, c32 = lane & 31;
     const int S = a.S, NG = a.NG;
@@ -238,7 +241,7 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
     }
     {
         const double gj = a.G2[(size_t)bh * a.NG + jt];
-        for (int g = threadIdx.x; g < a.NG; g += 256) sG[g] = (float)(a.G2[(size_t)bh * a.NG + g] - gj);
+        for (int g = threadIdx.x; g < a.NG; g += 256) sG[g] = (Base)(a.G2[(size_t)bh * a.NG + g] - gj);
     }
 
     const int kstartA = GRAN * jt + 32 * kbA;
@@ -456,14 +459,16 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
             // without the explicit interleave the reads of a batch and its MFMAs would take turns).
             constexpr int AHEAD = NS < 4 ? NS : 4;
             if constexpr (F32) {
+                f32x16 s2 = {}, d2 = {};
                 sacc = f32x16{}; dacc = f32x16{};
                 R::template stream<2 * NS>([&](auto n) { return n & 1 ? qrd.read(dHs, qbA, n >> 1) : qrd.read(Qs, qbA, n >> 1); },
                                            [&](auto n, const auto& f, auto&& between) {
                                                if constexpr (SPREAD && STAGES == 2) {
                                                    if (n % 4 == 0) tdma.issue_range(lq, gq, (n / 4) * PW / (NS / 2), (n / 4 + 1) * PW / (NS / 2), ra);
                                                }
-                                               R::mma_between(n & 1 ? dacc : sacc, n & 1 ? vt[n >> 1] : kt[n >> 1], f, between);
+                                               R::mma_between(n & 1 ? dacc : sacc, n & 1 ? d2 : s2, n & 1 ? vt[n >> 1] : kt[n >> 1], f, between);
                                            });
+                sacc += s2; dacc += d2;
             } else {
             frag qf[NS], hf[NS];
 #pragma unroll
@@ -483,10 +488,11 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
                 __builtin_amdgcn_sched_barrier(0);
             }
             }
-            const float crow = log2scale - srow[32 * qbA + c32] + sG[it];
+            const float nbeta = -srow[32 * qbA + c32];
+            const Base crow = F32 ? (Base)log2scale + sG[it] : (Base)(log2scale + nbeta + sG[it]);   // (fp32: without beta, see row_kernel)
             const float inv = srow[GRAN + 32 * qbA + c32], dbv = srow[2 * GRAN + 32 * qbA + c32];
             const bool qvalid = qrow < S;
-            const float er = qvalid ? fast_exp2(crow + amaxA) : 0.f;
+            const float er = !qvalid ? 0.f : (F32 ? fast_exp2((float)((Base)(amaxA + nbeta) + crow)) : fast_exp2((float)crow + amaxA));
             // below the diagonal E = ekr[key] * er[query]: the query factor goes into the per-lane scalars, which leaves
             // seven operations per element (G = dC~ E, W = C~ / n, dD = C~ dC~ with C~ = S E, dC~ = dC / n + db)
             const float inv_er = inv * er, dbv_er = dbv * er;
@@ -494,7 +500,7 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
             for (int r = 0; r < 16; r++) {
                 float dd;
                 if constexpr (FIRST) {
-                    float e = fast_exp2(al[r] + crow);
+                    float e = fast_exp2(F32 ? (al[r] + nbeta) + (float)crow : al[r] + (float)crow);
                     if (!qvalid || (diag && (8 * (r >> 2) + 4 * h + (r & 3) > c32))) e = 0.f;
                     const float ct = sacc[r] * e;
                     const float dct = dacc[r] * inv + dbv;
@@ -720,12 +726,12 @@ static int launch_col_ts(const ColArgs& a, hipStream_t st) {
     static hipError_t attr_rc = hipSuccess;
     std::call_once(once, [&] {
         attr_rc = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)(Cfg::LDS_BYTES + Cfg::EXTRA_CHUNK_BYTES + 2048 * sizeof(float)));
+                                      (int)std::min<size_t>(160 * 1024, Cfg::LDS_BYTES + Cfg::EXTRA_CHUNK_BYTES + 2048 * sizeof(typename Cfg::Base)));
     });
     if (attr_rc != hipSuccess) return (int)attr_rc;
     if (a.NG > 2048) return MLSTM_ESHAPE;
     if (a.chunk_len > 0 && (a.chunk_len % GRAN != 0 || (a.n_states > 0 && (!a.Ev || !a.gvec || (STRICT && !a.Ev_lo))))) return MLSTM_EINVAL;
-    const size_t lds = Cfg::LDS_BYTES + (a.chunk_len > 0 ? Cfg::EXTRA_CHUNK_BYTES : 0) + (size_t)a.NG * sizeof(float);
+    const size_t lds = Cfg::LDS_BYTES + (a.chunk_len > 0 ? Cfg::EXTRA_CHUNK_BYTES : 0) + (size_t)a.NG * sizeof(typename Cfg::Base);
     if (lds > 160 * 1024) return MLSTM_ESHAPE;
     hipLaunchKernelGGL(kern, dim3(a.BH * a.NG), dim3(256), lds, st, a);
     return (int)hipGetLastError();

@@ -114,9 +114,10 @@ template <> struct Tr<_Float16> {
 // fp32 operands run on the bf16 matrix units as three terms, x = hi + mid + lo with hi = bf16(x), mid = bf16(x - hi),
 // lo = bf16(x - hi - mid): 24 significant bits, all of an fp32 value.  A product is the six products of terms down to 2^-18 of
 // hi hi; what is left out (mid lo, lo mid, lo lo) is at most 2^-24 of a product, the rounding of one fp32 addition, and 2^-27 at its
-// root mean square.  A sum takes six roundings into the accumulator per 16 elements where 32x32x2 products take eight.  Errors
-// of the operators against 64 bits beside those of 32x32x2 products (median over the rows, ten seeds, S = 128 to 2048): h, dQ, dK,
-// dV of the matmul form at D = 64 and 128 0.79 to 0.97 times as large, of the scan form at D = 256 to 1024 0.97 to 1.00 times.
+// root mean square.  A sum takes six roundings into the accumulator per 16 elements where 32x32x2 products take eight, and one
+// where the small products have an accumulator of their own.  Errors of the operators against 64 bits beside those of 32x32x2
+// products (median over the rows, ten seeds, S = 128 to 2048): h, dQ, dK, dV of the matmul form at D = 64 and 128 0.63 to 0.91
+// times as large, of the scan form at D = 64 and 128 (then on the scan kernels) 0.84 to 1.00, at D = 256 to 1024 0.97 to 1.00 times.
 // Six bf16 products take 192 cycles per 32x32x16 block where v_mfma_f32_32x32x2_f32 takes 512; splitting an operand is 28 vector
 // instructions per fragment, which run beside them.
 // What the range of the terms does: an infinite operand, or one beyond 3.39e38 (its hi rounds to infinity), makes the sums it
@@ -186,16 +187,20 @@ template <> struct Tr<float> {
     // the six products, smallest first, with something else between them (a vector instruction costs nothing while the matrix
     // unit works: six products keep it busy for 192 cycles, 48 instructions' worth)
     template <typename F>
-    static __device__ __forceinline__ void mma_between(f32x16& c, const terms& a, const terms& b, F&& between) {
-        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.lo, b.hi, c, 0, 0, 0);
+    static __device__ __forceinline__ void mma_between(f32x16& c, const terms& a, const terms& b, F&& between) { mma_between(c, c, a, b, between); }
+    // the same with the five small products in an accumulator of their own (the caller adds the two in the end): the sum of the large
+    // ones then has one rounding per 16 elements, not six
+    template <typename F>
+    static __device__ __forceinline__ void mma_between(f32x16& c, f32x16& small, const terms& a, const terms& b, F&& between) {
+        small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.lo, b.hi, small, 0, 0, 0);
         between(std::integral_constant<int, 0>{});
-        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.hi, b.lo, c, 0, 0, 0);
+        small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.hi, b.lo, small, 0, 0, 0);
         between(std::integral_constant<int, 1>{});
-        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.mid, b.mid, c, 0, 0, 0);
+        small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.mid, b.mid, small, 0, 0, 0);
         between(std::integral_constant<int, 2>{});
-        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.mid, b.hi, c, 0, 0, 0);
+        small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.mid, b.hi, small, 0, 0, 0);
         between(std::integral_constant<int, 3>{});
-        c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.hi, b.mid, c, 0, 0, 0);
+        small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.hi, b.mid, small, 0, 0, 0);
         between(std::integral_constant<int, 4>{});
         c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.hi, b.hi, c, 0, 0, 0);
     }

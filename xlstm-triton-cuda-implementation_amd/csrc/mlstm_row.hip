@@ -120,6 +120,7 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
     using Cfg = RowCfg<T, D>;
     typedef typename R::frag frag;
     constexpr int KW = R::KW, NS = D / KW, NDB = D / 32, NSTEP32 = 32 / KW;
+    constexpr bool F32 = !R::HALF;
     extern __shared__ __attribute__((aligned(16))) char smem[];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = lane >> 5, c32 = lane & 31;
@@ -171,6 +172,12 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
     // vmcnt(0), which would also wait for the tile copies in flight
     double* const sG = reinterpret_cast<double*>(smem + Cfg::STAGES_BYTES);
     for (int g = tid; g < NG; g += 256) sG[g] = a.G2[goff + g];
+    // What a weight's exponent has beside alpha of the key.  fp32: its parts stay apart until they are added at the size of the
+    // result (alpha less beta of the row; the granules' distance and log2 of 1 / sqrt(D) in fp64): added up per row first they were
+    // rounded at the size of the parts, 3 % of the error of h and 6 % of that of dV.
+    typedef typename std::conditional<F32, double, float>::type Crow;
+    constexpr double LOG2_SCALE = D == 64 ? -3.0 : (D == 128 ? -3.5 : -4.0);
+    const float nbeta = -a.beta2[poff + rowc];
     float crow_base = -0.5f * __log2f((float)D) - a.beta2[poff + rowc];
     float inv_n = 0.f, dbv = 0.f;
     if constexpr (MODE == MODE_DQ) {
@@ -198,7 +205,6 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
     constexpr bool FAST_TR = R::HALF && Swz<T, D>::CPR >= 16;  // precomputed offsets for the transposing reads
     SwzRowReader<T, D> krd;
     krd.init(lane);
-    constexpr bool F32 = !R::HALF;
     typename std::conditional<F32, SwzTransReaderF32<D>, SwzTransReader<typename std::conditional<FAST_TR, T, __bf16>::type, FAST_TR ? D : 256>>::type vrd;
     if constexpr (FAST_TR || F32) vrd.init(lane);
 
@@ -233,11 +239,13 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
     // chains are interleaved so that consecutive MFMAs never depend on each other
     auto gemm1x2 = [&](const T* y1, f32x16& s0, f32x16& s1, auto&& hook) {
         if constexpr (F32) {
+            f32x16 t0 = {}, t1 = {};
             s0 = f32x16{}; s1 = f32x16{};
             R::template stream<2 * NS>([&](auto n) { return krd.read(y1, n & 1, n >> 1); }, [&](auto n, const auto& kf, auto&& between) {
                 if (n % 4 == 0) hook(n / 4, NS / 2);
-                R::mma_between(n & 1 ? s1 : s0, kf, xt[n >> 1], between);
+                R::mma_between(n & 1 ? s1 : s0, n & 1 ? t1 : t0, kf, xt[n >> 1], between);
             });
+            s0 += t0; s1 += t1;
             return;
         }
         constexpr int BATCH = NS < 4 ? NS : 4;  // fragments fetched ahead of the MFMAs that consume them
@@ -262,22 +270,26 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
 #pragma unroll
         for (int r = 0; r < 16; r++) sacc[r] = 0.f;
         if constexpr (F32) {
+            f32x16 small = {};
             R::template stream<NS>([&](auto n) { return krd.read(y1, kb, n); },
-                                   [&](auto n, const auto& kf, auto&& between) { R::mma_between(sacc, kf, xt[n], between); });
+                                   [&](auto n, const auto& kf, auto&& between) { R::mma_between(sacc, small, kf, xt[n], between); });
+            sacc += small;
         } else {
 #pragma unroll
             for (int s = 0; s < NS; s++) R::mma(sacc, krd.read(y1, kb, s), xt[s]);
         }
     };
     // gate weights; `diag` masks the keys above the diagonal of a diagonal block
-    auto weigh = [&](f32x16& sacc, const float* sal, int kb, float crow, bool diag) {
+    auto weigh = [&](f32x16& sacc, const float* sal, int kb, Crow crow, bool diag) {
 #pragma unroll
         for (int a4 = 0; a4 < 4; a4++) {
             const f32x4 al = *reinterpret_cast<const f32x4*>(sal + 32 * kb + 8 * a4 + 4 * h);
 #pragma unroll
             for (int c = 0; c < 4; c++) {
                 const int r = 4 * a4 + c;
-                float e = fast_exp2(al[c] + crow);
+                float e;
+                if constexpr (F32) e = fast_exp2((al[c] + nbeta) + (float)crow);
+                else e = fast_exp2(al[c] + crow);
                 if (diag && (8 * a4 + 4 * h + c > c32)) e = 0.f;
                 if constexpr (MODE == MODE_FWD) {
                     const float p = sacc[r] * e;
@@ -291,8 +303,10 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
     };
     // gate weights of a block entirely below the diagonal, factorised: exp2(alpha_j - c0) comes from the pre-pass
     // (sek), exp2(c0 - beta_i + dG) is one exponential per lane and block
-    auto weigh_fact = [&](f32x16& sacc, const float* sek, int kb, float crow) {
-        const float er = fast_exp2(crow + sek[GRAN + kb]);
+    auto weigh_fact = [&](f32x16& sacc, const float* sek, int kb, Crow crow) {
+        float er;
+        if constexpr (F32) er = fast_exp2((float)((double)(sek[GRAN + kb] + nbeta) + crow));
+        else er = fast_exp2(crow + sek[GRAN + kb]);
         float blk = 0.f;
 #pragma unroll
         for (int a4 = 0; a4 < 4; a4++) {
@@ -554,7 +568,9 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
         const T* y1 = ST_Y1(j & 1);
         const T* y2 = ST_Y2(j & 1);
         const float* sal = ST_AL(j & 1);
-        const float crow = crow_base + (float)(GI - sG[j]);
+        Crow crow;
+        if constexpr (F32) crow = LOG2_SCALE + (GI - sG[j]);
+        else crow = crow_base + (float)(GI - sG[j]);
         if constexpr (FAST_TR && NSTEP32 == 2) {
             tile_overlapped(y1, y2, sal + GRAN, crow, hook1, hook2);
         } else {
@@ -575,7 +591,9 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
         const T* y1 = ST_Y1(j & 1);
         const T* y2 = ST_Y2(j & 1);
         const float* sal = ST_AL(j & 1);
-        const float crow = crow_base + (float)(GI - sG[j]);
+        Crow crow;
+        if constexpr (F32) crow = LOG2_SCALE + (GI - sG[j]);
+        else crow = crow_base + (float)(GI - sG[j]);
         if constexpr (FAST_TR && NSTEP32 == 2) {
             tile_overlapped(y1, y2, sal + GRAN, crow, no_hook, no_hook);
         } else {
@@ -597,7 +615,9 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
         const T* y1 = ST_Y1(j & 1);
         const T* y2 = ST_Y2(j & 1);
         const float* sal = ST_AL(j & 1);
-        const float crow = crow_base + (float)(GI - sG[j]);
+        Crow crow;
+        if constexpr (F32) crow = LOG2_SCALE + (GI - sG[j]);
+        else crow = crow_base + (float)(GI - sG[j]);
 #pragma unroll
         for (int kb = 0; kb < 2; kb++) {
             const int kstart = GRAN * j + 32 * kb;
