@@ -139,3 +139,13 @@ def test_scan_form_on_views_that_start_off_a_16_byte_boundary(op, shift):
     plain = [t.detach() for t in views]
     h, hu, b = ms.mlstm_scan_forward_save_hip(*plain)
     _same([h, *ms.mlstm_scan_backward_hip(dh, *plain, h_ungated=shifted(hu), b=b)], want)
+
+
+@pytest.mark.parametrize("op", list(OPS))
+def test_the_same_bits_without_it(op, monkeypatch):
+    # the wrappers' own calls through ctypes, as where the extension has not been built for the torch at hand
+    ffi = submodule("_ffi")
+    ins = _inputs(op, S=1100 if op in ("matmul", "gated") else 100)
+    want = _step(op, ins)
+    monkeypatch.setattr(ffi, "_native", ffi._ServesNothing())
+    _same(_step(op, ins), want)

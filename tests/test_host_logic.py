@@ -1,4 +1,8 @@
 """Host-side logic of the ctypes layer that needs no GPU: layouts of gradient tensors, overlap detection."""
+import os
+import subprocess
+
+import pytest
 import torch
 
 from _mlstm_pkg import submodule
@@ -70,11 +74,37 @@ def test_tile_copy_index_arithmetic_stays_inside_the_tiles():
     """tests/harness/tile_bounds (the kernels' own offset functions, compiled for the host): every block of every tile shape
     is fetched exactly once, lands where the LDS readers expect it, and no fetch ends beyond the tile's last row -- for the
     last tile of the last head that is the end of the caller's tensor; the early touch of the dQ pass stays inside its half row."""
-    import os
-    import subprocess
     here = os.path.join(os.path.dirname(os.path.abspath(__file__)), "harness")
     exe = os.path.join(here, "tile_bounds")
     if not os.path.exists(exe):
         subprocess.check_call(["make", "-C", here, "tile_bounds"])
     out = subprocess.run([exe], capture_output=True, text=True)
     assert out.returncode == 0 and "tile_bounds: ok" in out.stdout, out.stdout + out.stderr
+
+
+def test_operators_do_without_the_native_host_path(monkeypatch):
+    """The extension belongs to one torch release; missing, or another release's, it is left out with a warning and the calls go
+    through ctypes (every function says that it serves nothing)."""
+    def missing():
+        raise ImportError("no such file")
+    monkeypatch.setattr(ffi, "_native", None)
+    monkeypatch.setattr(ffi, "_load_native", missing)
+    with pytest.warns(RuntimeWarning, match="native host path does not load"):
+        stand_in = ffi.native()
+    assert ffi.native() is stand_in
+    for name in ("matmul", "matmul_train", "gated", "gated_train", "scan", "slstm"):
+        assert getattr(stand_in, name)(1, 2, 3) is None
+    monkeypatch.undo()
+    monkeypatch.setattr(ffi, "_native", None)
+    monkeypatch.setattr(torch, "__version__", "1.0.0")
+    with pytest.warns(RuntimeWarning, match="built for torch"):
+        ffi.native()
+
+
+def test_library_target_needs_no_torch():
+    """The default target where Python has no torch: the library, and nothing that needs torch's headers."""
+    csrc = os.path.join(os.path.dirname(os.path.abspath(ffi.__file__)), "csrc")
+    for python, native in (("false", False), ("python3", True)):
+        plan = subprocess.run(["make", "-n", "-B", "-C", csrc, f"PYTHON={python}"], capture_output=True, text=True)
+        assert plan.returncode == 0 and "-o ../libmlstm_hip.so" in plan.stdout, plan.stderr
+        assert ("mlstm_torch.cpp" in plan.stdout) == native

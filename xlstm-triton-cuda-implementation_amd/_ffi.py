@@ -1,6 +1,7 @@
 """ctypes binding of libmlstm_hip.so (declared in include/mlstm_hip.h)."""
 import ctypes
 import os
+import warnings
 
 import torch
 
@@ -125,17 +126,33 @@ def lib():
 _native = None
 
 
+class _ServesNothing:
+    """In the place of the native host path: every call comes back with None, as for whatever that path leaves to the wrappers."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def _load_native():
+    from . import _native as module
+    if module.torch_version != torch.__version__.split("+")[0]:
+        raise ImportError(f"built for torch {module.torch_version}, this is {torch.__version__}")
+    return module
+
+
 def native():
-    """The operators' host path in native code (csrc/mlstm_torch.cpp).  Raises if it has not been built, like ``lib``."""
+    """The operators' host path in native code (csrc/mlstm_torch.cpp).  It is an extension of one torch release; where it has not been
+    built or is another release's, the wrappers make the same calls to the library through ctypes, with the same results and more
+    time on the host (a warning says so, once).  The library itself has no stand-in: see ``lib``."""
     global _native
     if _native is None:
         lib()
         try:
-            from . import _native as module
+            _native = _load_native()
         except ImportError as e:
-            raise ImportError(f"{os.path.join(_HERE, '_native.so')} is missing or does not load ({e}): build it with "
-                              f"`make -C {os.path.join(_HERE, 'csrc')}` (or __graft_entry__.build())") from None
-        _native = module
+            warnings.warn(f"the native host path does not load ({e}): calls go through ctypes, which costs 20 to 150 us each; build it "
+                          f"with `make -C {os.path.join(_HERE, 'csrc')}`", RuntimeWarning, stacklevel=3)
+            _native = _ServesNothing()
     return _native
 
 

@@ -22,6 +22,7 @@
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/version.h>
 #include <algorithm>
 #include <vector>
 #include "mlstm_train.h"
@@ -558,4 +559,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nu
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__native(void) { return PyModule_Create(&module); }
+// (torch_version: the release whose headers this was built with; a tensor's layout in memory belongs to one of them)
+PyMODINIT_FUNC PyInit__native(void) {
+    PyObject* m = PyModule_Create(&module);
+    if (m && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) < 0) Py_CLEAR(m);
+    return m;
+}
