@@ -30,8 +30,17 @@ def test_scan_gate_regimes(f_mean, i_mean):
     assert_close(h, O.mlstm_scan_dense(q, k, v, f, i, o), torch.float32, "h")
 
 
+@pytest.mark.parametrize("f_mean,i_mean", [(-3.0, 0.0), (0.0, 2.0), (8.0, -1.0)])
+@pytest.mark.parametrize("NH,S,D", [(2, 640, 256), (16, 320, 512), (4, 320, 1024)])
+def test_scan_gate_regimes_on_the_scan_kernels(NH, S, D, f_mean, i_mean):
+    # the same regimes where the state walk itself runs (D >= 256; the tile kernels serve the smaller head dimensions): its state is
+    # rescaled in every chunk, now and then, never; one walk per key tile shape
+    q, k, v, f, i, _, o = O.make_inputs(1, NH, S, D, torch.float32, seed=11, f_mean=f_mean, i_mean=i_mean, with_o=True)
+    assert_close(run_scan(q, k, v, f, i, o), O.mlstm_scan_dense(q, k, v, f, i, o), torch.float32, "h")
+
+
 def test_scan_many_heads_one_key_range():
-    # enough heads to fill the chip without splitting the key range of a value tile
+    # 16 heads of D = 512: one pair of key ranges per value tile, which shares a partial numerator
     q, k, v, f, i, _, o = O.make_inputs(4, 4, 200, 512, torch.float32, seed=12, with_o=True)
     h = run_scan(q, k, v, f, i, o)
     assert_close(h, O.mlstm_scan_dense(q, k, v, f, i, o), torch.float32, "h")
@@ -45,7 +54,7 @@ def test_scan_tuning_arguments_do_not_change_the_result():
 
 
 def test_scan_equals_gated_matmul_form():
-    # silu(o) * matmul-form h, both on the GPU
+    # silu(o) * matmul-form h, both on the GPU (D = 128: both on the tile kernels, one with the gate in the row kernel)
     from mlstm_matmul import mlstm_matmul
     q, k, v, f, i, _, o = O.make_inputs(2, 2, 320, 128, torch.float32, seed=9, with_o=True)
     h = run_scan(q, k, v, f, i, o)
@@ -72,7 +81,8 @@ def test_scan_against_committed_golden_vector():
 
 @pytest.mark.parametrize("S,D", [(8192, 64), (3000, 64), (4096, 128), (2048, 256)])
 def test_scan_one_long_sequence_in_segments(S, D):
-    # one head: the state walk runs in segments side by side (states at the segment ends from a pass of their own);
+    # one head: at D = 256 the state walk runs in segments side by side (states at the segment ends from a pass of their own), at
+    # D = 64 and 128 the tile kernels run in chunks;
     # checked against the step-by-step recurrence, and against the same head inside a batch that fills the chip and
     # therefore walks its chunks in one piece
     q, k, v, f, i, _, o = O.make_inputs(1, 1, S, D, torch.float32, seed=S + D, with_o=True)
@@ -84,6 +94,13 @@ def test_scan_one_long_sequence_in_segments(S, D):
     assert_close(h[0], hb[0].cpu(), torch.float32, "h against the unsegmented walk")
 
 
+@pytest.mark.parametrize("S,D", [(3000, 256), (2048, 512)])
+def test_scan_strong_forgetting_across_segments_of_the_walk(S, D):
+    q, k, v, f, i, _, o = O.make_inputs(1, 1, S, D, torch.float32, seed=78, f_mean=-3.0, with_o=True)
+    assert_close(run_scan(q, k, v, f, i, o), O.mlstm_recurrent(q, k, v, f, i, o), torch.float32, "h")
+
+
 def test_scan_strong_forgetting_across_segments():
+    # (D = 64: across the chunks of the tile kernels)
     q, k, v, f, i, _, o = O.make_inputs(1, 2, 4096, 64, torch.float32, seed=77, f_mean=-3.0, with_o=True)
     assert_close(run_scan(q, k, v, f, i, o), O.mlstm_recurrent(q, k, v, f, i, o), torch.float32, "h")

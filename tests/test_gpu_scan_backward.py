@@ -49,6 +49,22 @@ def test_scan_backward_gate_regimes(f_mean, i_mean):
     check(run_backward(dh, q, k, v, f, i, o), dh, q, k, v, f, i, o)
 
 
+@pytest.mark.parametrize("f_mean,i_mean", [(-3.0, 0.0), (0.0, 2.0), (8.0, -1.0), (3.0, -4.0)])
+@pytest.mark.parametrize("NH,S,D", [(2, 640, 256), (16, 200, 512)])
+def test_scan_backward_gate_regimes_on_the_scan_kernels(NH, S, D, f_mean, i_mean):
+    # the same where the state walk itself runs, from both ends (D >= 256)
+    q, k, v, f, i, dh, o = O.make_inputs(1, NH, S, D, torch.float32, seed=21, f_mean=f_mean, i_mean=i_mean, with_o=True)
+    check(run_backward(dh, q, k, v, f, i, o), dh, q, k, v, f, i, o)
+
+
+@pytest.mark.parametrize("S,D", [(2048, 256), (1500, 256), (1100, 512)])
+def test_scan_backward_one_long_sequence_in_segments(S, D):
+    # one head at D >= 256: every pass of the state walk runs in segments side by side, two of the passes from the end of the
+    # sequence (which at a ragged length begin inside a chunk)
+    q, k, v, f, i, dh, o = O.make_inputs(1, 1, S, D, torch.float32, seed=S + D, with_o=True)
+    check(run_backward(dh, q, k, v, f, i, o), dh, q, k, v, f, i, o)
+
+
 def test_scan_backward_many_heads():
     q, k, v, f, i, dh, o = O.make_inputs(4, 4, 200, 256, torch.float32, seed=22, with_o=True)
     check(run_backward(dh, q, k, v, f, i, o), dh, q, k, v, f, i, o)
@@ -68,7 +84,7 @@ def test_scan_autograd_path():
 
 
 def test_scan_backward_equals_gated_matmul_backward():
-    # both backward paths on the GPU, at a head dimension both serve in fp32
+    # both backward entry points on the GPU, at a head dimension where both run on the tile kernels
     from mlstm_matmul import mlstm_backward_gated_hip, mlstm_forward_gated_hip
     q, k, v, f, i, dh, o = (x.cuda() for x in O.make_inputs(2, 2, 320, 128, torch.float32, seed=24, with_o=True))
     got = run_backward(dh, q, k, v, f, i, o)
@@ -168,6 +184,6 @@ def test_matmul_form_fp32_large_head_dimension_limits():
 
 @pytest.mark.parametrize("S,D", [(4096, 128), (2500, 64)])
 def test_scan_backward_one_long_sequence(S, D):
-    # one head: every pass of the state kernel runs in segments (two of them from the end of the sequence backwards)
+    # one head at the head dimensions of the tile kernels: chunks of 128 (the state walk in segments: the test above)
     q, k, v, f, i, dh, o = O.make_inputs(1, 1, S, D, torch.float32, seed=S + D, with_o=True)
     check(run_backward(dh, q, k, v, f, i, o), dh, q, k, v, f, i, o)
