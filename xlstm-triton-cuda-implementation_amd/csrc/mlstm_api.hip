@@ -130,7 +130,7 @@ struct Sizes {
                up256(scan_segment_state_bytes((int)BH, (int)S, (int)D));
     }
     size_t fwd() const { return scan_engine() ? scan_fwd() : gates() + stats() + chunk_states(); }
-    size_t anchor_parts() const { return D >= 32 ? (D / 32) * (D / 32) : 1; }   // workgroups per head of the value-major carry, at most
+    size_t anchor_parts() const { return D >= 32 ? (D / 32) * (D / 32) : 1; }   // one per 32 x 32 block
     size_t fwd_fixed() const { return gates() + stats(); }   // offset of the chunk states inside fwd()
     size_t bwd() const {
         if (scan_engine()) return scan_backward_workspace_bytes((int)BH, (int)S, (int)D);

@@ -1,4 +1,4 @@
-// Chunk states for the matmul-form forward of long sequences (16-bit types).
+// Chunk states for the matmul form of long sequences.
 //
 // The forward of a row i only needs the keys of its own chunk of L positions one by one; everything before the chunk
 // enters through the state the scan form carries (mlstm_scan.py:16-26; the two forms are the same function):
@@ -14,6 +14,7 @@
 //                       into LDS), fp32 result; and dn_c = sum_j w_j k_j.  Eight waves: four multiply, four bring the tiles.
 //   chunk_carry_kernel  C~_c = gamma_c C~_{c-1} + dC_c over the chunks of a head (gamma_c = exp(A_{e_{c-1}} - A_{e_c})),
 //                       element-wise, written in the element type; n~_c likewise, in place, fp32.
+//   chunk_sum_small_kernel, chunk_carry_small_kernel  the same two steps for fp32 and for 16-bit types at D = 64 (fp32 MFMA).
 // State rows are stored in the order in which the row kernel's second product contracts them (see PERM16 below).
 #include "mlstm_device.h"
 #include "mlstm_kernels.h"

@@ -237,8 +237,9 @@ int chunk_states_dot_parts(int dtype, int D, const ChunkArgs& a);
 // 2 = the one-pass kernel wherever it can serve
 int set_state_kernel(int variant);
 
-// anchor[bh][c] = <A_c, B_c> + va_c . vb_c over two sets of states in the same layout; A_lo, B_lo (both or neither):
-// their low-order terms (split mode)
+// anchor[bh][c] = <A_c, B_c> + va_c . vb_c over two sets of states in the same layout; A_lo, B_lo (both or neither): their low-order
+// terms (split mode).  Only for chunks of more than 1024 positions, which mlstm_set_chunk_length alone asks for: with shorter ones the
+// reverse carry leaves the anchors in parts.
 int launch_anchor(int dtype, int D, const void* A, const void* B, const void* A_lo, const void* B_lo, const float* va, const float* vb,
                   float* anchor, int BH, int NCS, hipStream_t st);
 

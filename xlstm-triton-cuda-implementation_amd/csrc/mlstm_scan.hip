@@ -193,7 +193,7 @@ __global__ __launch_bounds__(256) void scan_ncarry_kernel(ScanArgs a) {
 // terms serve both query blocks.  Q comes with direct copies into a piece of LDS that belongs to the wave (its fragments want
 // one row per lane: 64 lines per load instruction from memory), K and V from memory into registers, 128 bytes per row.
 // Measured on 4 heads x 2048 x 1024, forward: 17,200 cycles per chunk (read-out 6400, update 5600) where the 32x32x2 kernel
-// took 27,900; whole call 393 -> 306 us.  Eight waves of half the tile each took 18,400: two waves per SIMD overlap splits and
+// took 27,900; whole call 393 -> 308 us.  Eight waves of half the tile each took 18,400: two waves per SIMD overlap splits and
 // MFMAs, and lose it again at twice the barriers.
 //
 // A sequence may also be cut into segments of seg_chunks chunks that run side by side (blockIdx.y), for the cases in
