@@ -1,0 +1,40 @@
+"""The kernel for launches that would leave the chip part empty (chunk_sum_narrow_kernel) against the one that
+serves larger launches: the same products in the same order, so a head alone and the same head in a batch that is large enough for the
+other kernel give the same bits.  Lengths at the edges of the chunks."""
+import pytest
+import torch
+
+from _mlstm_pkg import submodule
+
+pytestmark = pytest.mark.gpu
+mm = submodule("mlstm_matmul")
+
+
+def _inputs(heads, S, D, dtype, layout):
+    g = torch.Generator(device="cuda").manual_seed(S + D)
+    shape = (1, heads, S, D) if layout == "bnsd" else (1, S, heads, D)
+    rows = [torch.randn(shape, device="cuda", generator=g).to(dtype) for _ in range(5)]
+    if layout == "bsnd":
+        rows = [t.transpose(1, 2) for t in rows]
+    return rows, [(torch.randn(1, heads, S, device="cuda", generator=g) + m).to(dtype) for m in (3, 0)]
+
+
+def _step(op, rows, gates, heads):
+    q, k, v, dh, o = [t[:, :heads] for t in rows]
+    f, i = [t[:, :heads].contiguous() for t in gates]
+    if op == "gated":
+        hg, h, m, b = mm.mlstm_forward_gated_hip(q, k, v, f, i, o)
+        return [hg, h, m, b, *mm.mlstm_backward_gated_hip(dh, q, k, v, f, i, o, h, m, b)]
+    h, m, b, saved = mm.mlstm_forward_save_hip(q, k, v, f, i, precise=op == "precise")
+    return [h, m, b, *mm.mlstm_backward_saved_hip(dh, q, k, v, f, i, h, m, b, saved, precise=op == "precise")]
+
+
+# heads: enough for more than 768 blocks of 64 x 64
+@pytest.mark.parametrize("op,S,D,heads,layout", [
+    ("plain", 1023, 256, 17, "bsnd"), ("plain", 1023, 128, 17, "bnsd"), ("plain", 1024, 256, 49, "bnsd"), ("gated", 1025, 128, 65, "bnsd"),
+    ("plain", 1601, 256, 25, "bsnd"), ("plain", 2048, 128, 22, "bnsd"), ("precise", 1100, 256, 26, "bnsd"), ("precise", 1537, 128, 30, "bsnd")])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_a_head_alone_is_the_head_of_a_full_chip(op, S, D, heads, layout, dtype):
+    rows, gates = _inputs(heads, S, D, dtype, layout)
+    for name, a, b in zip(range(10), _step(op, rows, gates, 1), _step(op, rows, gates, heads)):
+        assert bool(torch.isfinite(b.float()).all()) and torch.equal(a[:, :1], b[:, :1]), name

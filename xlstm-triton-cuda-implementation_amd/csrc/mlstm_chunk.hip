@@ -12,6 +12,7 @@
 //                       w_j = exp(a_j - A_{e_c}) / sqrt(D), as a bf16 / fp16 MFMA product over the chunk's positions (both
 //                       operands are contracted over positions: transposing LDS reads; V is scaled by w on its way
 //                       into LDS), fp32 result; and dn_c = sum_j w_j k_j.  Eight waves: four multiply, four bring the tiles.
+//   chunk_sum_narrow_kernel  the same sums, bit for bit, on 64 x 64 blocks, for few heads.
 //   chunk_carry_kernel  C~_c = gamma_c C~_{c-1} + dC_c over the chunks of a head (gamma_c = exp(A_{e_{c-1}} - A_{e_c})),
 //                       element-wise, written in the element type; n~_c likewise, in place, fp32.
 //   chunk_sum_small_kernel, chunk_carry_small_kernel  the same two steps for fp32 and for 16-bit types at D = 64 (fp32 MFMA).
@@ -159,7 +160,7 @@ __global__ __launch_bounds__(512) void chunk_sum_kernel(ChunkArgs a) {
                 unpack8<T>(kset[P][it], x);
                 const float w2 = sw2[GRAN * j + pc / ZK::CPR];
 #pragma unroll
-                for (int e = 0; e < 8; e++) nacc[e] += x[e] * w2;
+                for (int e = 0; e < 8; e++) nacc[e] = fmaf(x[e], w2, nacc[e]);
             }
         }
 #pragma unroll
@@ -366,6 +367,200 @@ __global__ __launch_bounds__(512) void chunk_sum_kernel(ChunkArgs a) {
 
     if (feeder) feed();
     else multiply();
+#endif
+}
+
+// The chunk sums of chunk_sum_kernel -- the same products in the same order, hence the same bits -- where few workgroups would run:
+// one workgroup per (head, chunk, 64 keys, 64 values), a wave per 32 x 32 block.  With 48 workgroups that kernel takes as long as its
+// eight tiles one after the other (D = 256 17 us, split mode 24, D = 128 12, whatever the number of heads); here a workgroup's
+// 64 columns of K and V are 64 KB each, V's requested at once, K's in two parts, and two trips to memory, 32 products and the
+// write-out remain: 8 to 10 us.  K and V are read D / 64 times over, which is what the larger workgroups save where there are enough of them.
+template <typename T, bool STRICT>
+struct ChunkNarrowCfg {
+    static constexpr int L = 512, W = 64, PART = 256;               // positions per chunk, columns per workgroup, positions per part
+    static constexpr size_t PART_BYTES = (size_t)PART * W * sizeof(T);
+    // One part of K and V at a time, so that two workgroups fit a CU (both at once: level up to 256 workgroups, 15.4 us instead of
+    // 11.9 at 384).  Split mode: V's part as hi and lo, next to all of K.  And the positions' weights of the two sums.
+    static constexpr int KPARTS = STRICT ? 2 : 1, VPARTS = STRICT ? 2 : 1;
+    static constexpr size_t LDS_BYTES = (KPARTS + VPARTS) * PART_BYTES + 2 * L * sizeof(float);
+};
+template <typename T, int D, bool STRICT>
+__global__ __launch_bounds__(256) void chunk_sum_narrow_kernel(ChunkArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    using R = Tr<T>;
+    using Cfg = ChunkNarrowCfg<T, STRICT>;
+    using Z = Swz<T, Cfg::W>;
+    typedef typename R::frag frag;
+    constexpr int L = Cfg::L, W = Cfg::W, PART = Cfg::PART, KW = R::KW, NBK = (D / W) * (D / W);
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    auto kpart = [&](int p) { return smem + (STRICT ? p : 0) * Cfg::PART_BYTES; };
+    char* const vt = smem + Cfg::KPARTS * Cfg::PART_BYTES;   // (split mode: the lo tile behind it)
+    float* const sw = reinterpret_cast<float*>(smem + (Cfg::KPARTS + Cfg::VPARTS) * Cfg::PART_BYTES);
+    float* const sw2 = sw + L;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5, c32 = lane & 31;
+    int pair, blk;   // (head, chunk) and block of its sum: with a multiple of 8 pairs a pair's workgroups run on one XCD
+    if (((a.BH * a.NCS) & 7) == 0) { pair = (blockIdx.x & 7) | ((blockIdx.x >> 3) / NBK << 3); blk = (blockIdx.x >> 3) % NBK; }
+    else { pair = blockIdx.x / NBK; blk = blockIdx.x % NBK; }
+    const int cc = pair % a.NCS, bh = pair / a.NCS, kcol = W * (blk / (D / W)), vcol = W * (blk % (D / W));
+    const int S = a.S;
+    const size_t poff = (size_t)bh * a.NG * GRAN, goff = (size_t)bh * a.NG;
+    const int p0 = (a.reverse ? cc + 1 : cc) * L, pe = a.reverse ? p0 - 1 : p0 + L - 1;   // (see chunk_sum_kernel)
+    const size_t rsK = (size_t)a.lk.ss, rsV = (size_t)a.lv.ss;
+    const T* Kh = reinterpret_cast<const T*>(a.K) + a.lk.head(bh) + (size_t)p0 * rsK + kcol;
+    const T* Vh = reinterpret_cast<const T*>(a.V) + a.lv.head(bh) + (size_t)p0 * rsV + vcol;
+
+    // what the weights need, then K straight into LDS and V into registers, all positions at once
+    float x0[2], x1[2] = {0.f, 0.f}, x2[2] = {0.f, 0.f};
+    double xg[2];
+    const float bend = a.beta2[poff + pe];
+    const double Gend = a.G2[goff + pe / GRAN];
+#pragma unroll
+    for (int n = 0; n < 2; n++) {
+        const int pos = p0 + tid + 256 * n < S ? p0 + tid + 256 * n : S - 1;
+        xg[n] = a.G2[goff + pos / GRAN];
+        x0[n] = a.reverse ? a.beta2[poff + pos] : a.alpha2[poff + pos];
+        if (a.reverse) { x1[n] = a.inv_n[poff + pos]; x2[n] = a.db[poff + pos]; }
+    }
+    constexpr int NP = 2 * PART * Z::CPR / 256;   // a thread's 16-byte pieces of V: row vrow + 32 i, piece vch
+    const int vrow = tid / Z::CPR, vch = tid % Z::CPR;
+    u32x4 vset[NP];
+    const bool whole = p0 + L <= S;
+    auto row_of = [&](int r) { return whole || p0 + r < S ? r : S - 1 - p0; };   // (rows past the end, with weights of 0, become its last)
+#pragma unroll
+    for (int i = 0; i < NP; i++) vset[i] = *reinterpret_cast<const u32x4*>(Vh + (size_t)row_of(vrow + 32 * i) * rsV + Z::EPC * vch);
+    // K: 1 KB (eight rows) per load of a wave; piece c of row r at piece c ^ key(r) of the row
+    auto copy_k = [&](int p) __attribute__((always_inline)) {
+        const unsigned kbase = lds_offset_of(kpart(p));
+        const int kr = lane / Z::CPR, kc = lane % Z::CPR;
+#pragma unroll
+        for (int i = 0; i < PART / 32; i++) {
+            const int r = 32 * i + 8 * wave;
+            dma16(Kh + (size_t)row_of(PART * p + r + kr) * rsK + Z::EPC * (kc ^ Z::key(r + kr)), __builtin_amdgcn_readfirstlane(kbase + r * Z::ROW_BYTES));
+        }
+    };
+    copy_k(0);
+    if constexpr (STRICT) copy_k(1);
+    const float log2scale = -0.5f * __log2f((float)D);
+#pragma unroll
+    for (int n = 0; n < 2; n++) {
+        float w = 0.f, w2 = 0.f;
+        if (p0 + tid + 256 * n < S) {
+            if (a.reverse) {
+                const float rho = fast_exp2(bend - x0[n] + (float)(xg[n] - Gend) + log2scale);
+                w = rho * x1[n];
+                w2 = rho * x2[n];
+            } else {
+                w = w2 = fast_exp2(x0[n] - bend + (float)(Gend - xg[n]) + log2scale);
+            }
+        }
+        sw[tid + 256 * n] = w;
+        sw2[tid + 256 * n] = w2;
+    }
+    __syncthreads();   // the weights are there
+    auto commit = [&](auto part_tag) __attribute__((always_inline)) {   // V times the weights, rounded
+        constexpr int P = decltype(part_tag)::value;
+        typedef typename R::vec4 V4;
+        struct Pair { V4 lo, hi; };
+#pragma unroll
+        for (int i = 0; i < NP / 2; i++) {
+            const int row = vrow + 32 * i;
+            const float w = sw[PART * P + row];
+            float x[8];
+            unpack8<T>(vset[P * (NP / 2) + i], x);
+            Pair out;
+            if constexpr (STRICT) {
+                Pair rest;
+                R::cvt4_split(f32x4{x[0] * w, x[1] * w, x[2] * w, x[3] * w}, out.lo, rest.lo);
+                R::cvt4_split(f32x4{x[4] * w, x[5] * w, x[6] * w, x[7] * w}, out.hi, rest.hi);
+                *reinterpret_cast<Pair*>(vt + Cfg::PART_BYTES + Z::off(row, Z::EPC * vch)) = rest;
+            } else {
+                out.lo = R::cvt4(f32x4{x[0] * w, x[1] * w, x[2] * w, x[3] * w});
+                out.hi = R::cvt4(f32x4{x[4] * w, x[5] * w, x[6] * w, x[7] * w});
+            }
+            *reinterpret_cast<Pair*>(vt + Z::off(row, Z::EPC * vch)) = out;
+        }
+    };
+    // per-lane offsets of the transposing reads (see frag_transposed): rows 16 apart meet the same swizzle
+    const int kb = wave & 1, vb = wave >> 1;
+    const int j16 = lane & 15, sub = (lane >> 4) & 1, trow = 4 * h + (j16 >> 2), tcol = 16 * sub + 4 * (j16 & 3);
+    const int ko0 = Z::off(trow, 32 * kb + tcol), ko1 = Z::off(trow + 8, 32 * kb + tcol);
+    const int vo0 = Z::off(trow, 32 * vb + tcol), vo1 = Z::off(trow + 8, 32 * vb + tcol);
+    auto read = [&](const char* tile, int o0, int o1) __attribute__((always_inline)) {
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_PTR(s16x4))(tile + o0));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_PTR(s16x4))(tile + o1));
+        return __builtin_bit_cast(frag, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+    f32x16 acc;
+#pragma unroll
+    for (int x = 0; x < 16; x++) acc[x] = 0.f;
+    auto compute = [&](int p) __attribute__((always_inline)) {
+        constexpr int NSTEP = PART / KW, AHEAD = 4;
+        const char* kt = kpart(p);
+        frag af[NSTEP], bf[NSTEP], bl[STRICT ? NSTEP : 1];
+        auto rd = [&](int n) __attribute__((always_inline)) {
+            const int at = KW * n * Z::ROW_BYTES;
+            af[n] = read(kt + at, ko0, ko1);
+            bf[n] = read(vt + at, vo0, vo1);
+            if constexpr (STRICT) bl[n] = read(vt + Cfg::PART_BYTES + at, vo0, vo1);
+        };
+#pragma unroll
+        for (int n = 0; n < AHEAD; n++) rd(n);
+#pragma unroll
+        for (int n = 0; n < NSTEP; n++) {
+            if (n + AHEAD < NSTEP) rd(n + AHEAD);
+            R::mma(acc, af[n], bf[n]);
+            if constexpr (STRICT) R::mma(acc, af[n], bl[n]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    // the vector state of the workgroup's keys (the workgroups of the first values), added up as the feeders of chunk_sum_kernel do:
+    // position modulo NPG, then over those sums; a thread takes two keys of a row
+    constexpr int NPG = 256 / (D / 8), NH = NPG / 8;
+    float n0[NH], n1[NH];
+    const int k2 = tid & 31, pg = tid >> 5;
+#pragma unroll
+    for (int u = 0; u < NH; u++) { n0[u] = 0.f; n1[u] = 0.f; }
+    auto vector_part = [&](int p) __attribute__((always_inline)) {
+        if (vcol != 0) return;
+#pragma unroll
+        for (int u = 0; u < NH; u++)
+#pragma unroll 8
+            for (int r = pg + 8 * u; r < PART; r += NPG) {
+                typedef T T2 __attribute__((ext_vector_type(2)));
+                const T2 kv = *reinterpret_cast<const T2*>(kpart(p) + Z::off(r, 2 * k2));
+                const float w2 = sw2[PART * p + r];
+                n0[u] = fmaf((float)kv[0], w2, n0[u]);
+                n1[u] = fmaf((float)kv[1], w2, n1[u]);
+            }
+    };
+    commit(std::integral_constant<int, 0>{});
+    dma_wait();
+    __syncthreads();
+    compute(0);
+    vector_part(0);
+    __syncthreads();
+    if constexpr (!STRICT) copy_k(1);
+    commit(std::integral_constant<int, 1>{});
+    dma_wait();
+    __syncthreads();
+    compute(1);
+    vector_part(1);
+    float* out = a.dC + ((size_t)bh * a.NCS + cc) * D * D + (size_t)(kcol + 32 * kb) * D + vcol + 32 * vb + c32;
+#pragma unroll
+    for (int r = 0; r < 16; r++) out[(size_t)(8 * (r >> 2) + 4 * h + (r & 3)) * D] = acc[r];
+    if (vcol == 0) {
+        float* const red = reinterpret_cast<float*>(vt);   // [NPG][W]
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < NH; u++) *reinterpret_cast<float2*>(red + (pg + 8 * u) * W + 2 * k2) = make_float2(n0[u], n1[u]);
+        __syncthreads();
+        if (tid < W) {
+            float sum = 0.f;
+#pragma unroll
+            for (int g = 0; g < NPG; g++) sum += red[g * W + tid];
+            a.Nst[((size_t)bh * a.NCS + cc) * D + kcol + tid] = sum;
+        }
+    }
 #endif
 }
 
@@ -1168,6 +1363,17 @@ static int launch_chunk_sum(const ChunkArgs& a, hipStream_t st) {
     using Cfg = ChunkCfg<T, D, STRICT>;
     if (a.L > Cfg::MAX_L) return MLSTM_ESHAPE;
     const dim3 grid(a.BH * a.NCS * (D / Cfg::VW));
+    // Workgroups of the narrow kernel up to which it is the faster one (us, bf16, chunk_sum_kernel / narrow):
+    //   D = 256   32: 15.5 / 7.9   128: 16.2 / 8.4   384: 17.6 / 11.9   640: 18.0 / 16.5   768: 18.3 / 16.9   896: 18.6 / 19.7
+    //   D = 128   96: 10.7 / 8.0   192: 11.2 / 8.2   384: 11.3 / 11.8   768: 13.1 / 17.1
+    //   D = 256 in split mode   128: 23.2 / 9.8   256: 24.2 / 11.4   512: 24.2 / 19.1   768: 24.9 / 26.7
+    using N = ChunkNarrowCfg<T, STRICT>;
+    const int narrow = a.BH * a.NCS * (D / N::W) * (D / N::W);
+    if (a.L == N::L && narrow <= (D == 128 ? 256 : (STRICT ? 512 : 768))) {
+        if (hipError_t e = lds_limit_once<chunk_sum_narrow_kernel<T, D, STRICT>>((int)N::LDS_BYTES); e != hipSuccess) return (int)e;
+        hipLaunchKernelGGL((chunk_sum_narrow_kernel<T, D, STRICT>), dim3(narrow), dim3(256), N::LDS_BYTES, st, a);
+        return 0;
+    }
     const size_t lds = Cfg::TILE_BYTES + 2 * (size_t)a.L * sizeof(float);
     // (the unrolled variant of split mode at D = 256 does not fit the 256 registers of a wave and would spill)
     constexpr bool UNROLLED_FITS = !(STRICT && D == 256);
