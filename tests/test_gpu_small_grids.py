@@ -1,6 +1,6 @@
-"""The kernel for launches that would leave the chip part empty (chunk_sum_narrow_kernel) against the one that
-serves larger launches: the same products in the same order, so a head alone and the same head in a batch that is large enough for the
-other kernel give the same bits.  Lengths at the edges of the chunks."""
+"""Kernels for launches that would leave the chip part empty (roww_kernel, chunk_sum_narrow_kernel) against the ones that
+serve larger launches: the same products in the same order, so a head alone and the same head in a batch that is large enough for the
+other kernels give the same bits.  Lengths at the edges of the 64-row tiles, of the pairs of key tiles and of the chunks."""
 import pytest
 import torch
 
@@ -29,8 +29,10 @@ def _step(op, rows, gates, heads):
     return [h, m, b, *mm.mlstm_backward_saved_hip(dh, q, k, v, f, i, h, m, b, saved, precise=op == "precise")]
 
 
-# heads: enough for more than 768 blocks of 64 x 64
+# heads: enough for more than 256 workgroups of 64 rows, and from 1024 positions on for more than 768 blocks of 64 x 64
 @pytest.mark.parametrize("op,S,D,heads,layout", [
+    ("plain", 1, 128, 264, "bnsd"), ("plain", 63, 256, 258, "bnsd"), ("plain", 64, 128, 260, "bsnd"), ("plain", 65, 256, 130, "bnsd"),
+    ("gated", 127, 128, 131, "bnsd"), ("plain", 129, 128, 90, "bsnd"), ("gated", 200, 256, 70, "bsnd"), ("plain", 640, 128, 27, "bnsd"),
     ("plain", 1023, 256, 17, "bsnd"), ("plain", 1023, 128, 17, "bnsd"), ("plain", 1024, 256, 49, "bnsd"), ("gated", 1025, 128, 65, "bnsd"),
     ("plain", 1601, 256, 25, "bsnd"), ("plain", 2048, 128, 22, "bnsd"), ("precise", 1100, 256, 26, "bnsd"), ("precise", 1537, 128, 30, "bsnd")])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

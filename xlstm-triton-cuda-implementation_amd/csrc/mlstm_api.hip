@@ -289,7 +289,6 @@ int symbols_of_current_device(char** scratch_out, int** err_out) {
     return 0;
 }
 int g_spin_limit = 0;   // test aid (mlstm_set_spin_limit): 0 = the default bound
-constexpr int DEFAULT_SPIN_LIMIT = 1 << 22;   // iterations of 64 cycles and an LDS read each: a fraction of a second
 // error word and wait bound of the eight-wave row kernel
 int arm_row_args(RowArgs& a) {
     if (int rc = symbols_of_current_device(nullptr, &a.err)) return rc;

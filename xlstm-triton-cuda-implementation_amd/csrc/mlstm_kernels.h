@@ -72,6 +72,7 @@ inline hipError_t launch_gates(int gate_dtype, const void* F, const void* I, flo
 }
 
 extern bool g_force_generic;  // see mlstm_force_generic_kernels
+constexpr int DEFAULT_SPIN_LIMIT = 1 << 22;   // iterations of 64 cycles and an LDS read each: a fraction of a second
 
 struct RowArgs {
     const void* X;    // row operand held in registers: Q (forward) or dH (dQ pass)      [BH,S,D]
@@ -125,10 +126,18 @@ struct RowArgs {
 int launch_row_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t st);
 // eight waves (producer / consumer pairs per SIMD); 16-bit types and D in {128, 256} only
 int launch_row8_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t st);
+// the same bits on 64 rows per workgroup, for launches that leave the chip part empty; 16-bit types and D in {128, 256} only
+int launch_roww_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t st);
 // (the four-wave kernel serves every other case: fp32, D = 64, split mode -- in chunks too -- and the test switch)
 inline int launch_row_best(int mode, int dtype, int D, const RowArgs& a, hipStream_t st) {
     if (dtype != MLSTM_F32 && (D == 128 || D == 256) && !g_force_generic && !a.precise) {
-        int rc = launch_row8_kernel(mode, dtype, D, a, st);
+        // While its workgroups (64 rows) number no more than the chip's CUs, roww_kernel: row8_kernel / roww_kernel, forward, us --
+        // D = 128   10: 13.3 / 11.2   80: 14.6 / 12.1   240 (uncut, 1001 positions): 21.3 / 19.0   256: 13.0 / 10.9   384: 13.8 / 14.0
+        // D = 256   10: 17.2 / 13.4   224 (chunks of 512): 23.1 / 17.4   256: 15.4 / 13.0   384: 19.9 / 19.2   512: 25.9 / 27.2
+        int rc = MLSTM_ESHAPE;
+        // (a wait bound of the caller's asks for the kernel that has the wait: mlstm_set_spin_limit)
+        if ((long long)a.BH * a.NG <= 256 && a.spin_limit == DEFAULT_SPIN_LIMIT) rc = launch_roww_kernel(mode, dtype, D, a, st);
+        if (rc == MLSTM_ESHAPE) rc = launch_row8_kernel(mode, dtype, D, a, st);
         if (rc != MLSTM_ESHAPE) return rc;  // extremely long sequences do not fit its LDS budget
     }
     return launch_row_kernel(mode, dtype, D, a, st);

@@ -272,7 +272,7 @@ __global__ __launch_bounds__(512) void row8_kernel(RowArgs a) {
                     }
                 }
             }
-            if constexpr (MODE == R8_FWD) { bsum[0] += blk0 * er0; bsum[1] += blk1 * er1; }
+            if constexpr (MODE == R8_FWD) { bsum[0] = fmaf(blk0, er0, bsum[0]); bsum[1] = fmaf(blk1, er1, bsum[1]); }
         };
         // One 32 x 32 block of a tile that the diagonal crosses.  mode (the same in all lanes) 0: the block lies above the
         // diagonal (P = 0), 1: below it (the factorised weights of weigh_fact), 2: on it (one exp2 per element, masked).
@@ -302,9 +302,10 @@ __global__ __launch_bounds__(512) void row8_kernel(RowArgs a) {
                         }
                     }
                 }
-                if constexpr (MODE == R8_FWD) bs += blk * er;
+                if constexpr (MODE == R8_FWD) bs = fmaf(blk, er, bs);
                 return;
             }
+            float blk = 0.f;
 #pragma unroll
             for (int a4 = 0; a4 < 4; a4++) {
                 const f32x4 al = *reinterpret_cast<const f32x4*>(sal + 32 * kh + 8 * a4 + 4 * h);
@@ -314,14 +315,14 @@ __global__ __launch_bounds__(512) void row8_kernel(RowArgs a) {
                     float e = fast_exp2(al[c] + crow);
                     if (8 * a4 + 4 * h + c > c32) e = 0.f;
                     if constexpr (MODE == R8_FWD) {
-                        const float p = sacc[x] * e;
-                        bs += p;
-                        sacc[x] = p;
+                        sacc[x] *= e;
+                        blk += sacc[x];
                     } else {
                         sacc[x] = (sacc[x] * invn + dbr) * e;
                     }
                 }
             }
+            if constexpr (MODE == R8_FWD) bs += blk;
         };
         // hand the fragments of tile j to the consumers of the same rows; they have copied tile j-1's long ago
         bool expired = false;
@@ -466,14 +467,14 @@ __global__ __launch_bounds__(512) void row8_kernel(RowArgs a) {
                         for (int r = 0; r < 2; r++) {
                             const f32x8 qv = __builtin_convertvector(xf[r][s], f32x8);
 #pragma unroll
-                            for (int e = 0; e < 4; e++) part[r] += qv[e] * n0[e] + qv[4 + e] * n1[e];
+                            for (int e = 0; e < 4; e++) part[r] = fmaf(qv[4 + e], n1[e], fmaf(qv[e], n0[e], part[r]));
                         }
                     }
                 };
                 if (kh == 0) half_dot(std::integral_constant<int, 0>{});
                 else half_dot(std::integral_constant<int, NS / 2>{});
 #pragma unroll
-                for (int r = 0; r < 2; r++) bsum[r] += part[r] * dec_rows[r];
+                for (int r = 0; r < 2; r++) bsum[r] = fmaf(part[r], dec_rows[r], bsum[r]);
             }
         }
         dma_wait();
@@ -670,7 +671,10 @@ __global__ __launch_bounds__(512) void row8_kernel(RowArgs a) {
                         f32x4 nv = {0.f, 0.f, 0.f, 0.f};
                         if constexpr (MODE == R8_DQ) nv = *reinterpret_cast<const f32x4*>(nst + 32 * d + 8 * a4);
 #pragma unroll
-                        for (int c = 0; c < 4; c++) oacc[r][d][4 * a4 + c] = oacc[r][d][4 * a4 + c] * dec + rank1 * nv[c];
+                        for (int c = 0; c < 4; c++) {
+                            if constexpr (MODE == R8_FWD) oacc[r][d][4 * a4 + c] *= dec;
+                            else oacc[r][d][4 * a4 + c] = fmaf(oacc[r][d][4 * a4 + c], dec, rank1 * nv[c]);
+                        }
                     }
             }
             if constexpr (MODE == R8_DQ) {
@@ -688,7 +692,9 @@ __global__ __launch_bounds__(512) void row8_kernel(RowArgs a) {
                 const char* Qh = reinterpret_cast<const char*>(reinterpret_cast<const T*>(a.Qrow) + offA + (size_t)dh * (D / 2));
 #pragma unroll
                 for (int r = 0; r < 2; r++) {
-                    float rp = 0.f;
+                    float rpd[NDH];   // (per column block, then in their order: the order of mlstm_roww.hip, which splits a row by columns)
+#pragma unroll
+                    for (int d = 0; d < NDH; d++) rpd[d] = 0.f;
                     i32x4 wq[NP];
 #pragma unroll
                     for (int i = 0; i < NP; i++)
@@ -703,9 +709,12 @@ __global__ __launch_bounds__(512) void row8_kernel(RowArgs a) {
                             const f32x4 qv = __builtin_convertvector(__builtin_bit_cast(typename R::vec4, i32x2{(int)s0[u], (int)s1[u]}), f32x4);
                             const int pc = NP * u + i, d = pc / 4, a4 = pc % 4;   // column block and group of four registers
 #pragma unroll
-                            for (int c = 0; c < 4; c++) rp += oacc[r][d][4 * a4 + c] * qv[c];
+                            for (int c = 0; c < 4; c++) rpd[d] = fmaf(oacc[r][d][4 * a4 + c], qv[c], rpd[d]);
                         }
                     }
+                    float rp = 0.f;
+#pragma unroll
+                    for (int d = 0; d < NDH; d++) rp += rpd[d];
                     rp = sum_halves(rp);
                     if (h == 0) rix[((rg * 2 + dh) * 2 + r) * 32 + c32] = rp;
                 }

@@ -1,0 +1,494 @@
+// Row-parallel tile kernel for the 16-bit types at D >= 128 where few workgroups would run: the same math and, element by
+// element, the same order of operations as mlstm_row8.hip, hence the same bits, on half as many rows per workgroup and with every
+// key tile's work spread over all eight waves.
+//
+// What bounds a small call is one workgroup's walk of its key tiles, and in the eight-wave producer / consumer kernel that walk
+// takes 1.2 us per 64 keys (products, weights, hand-over, products, one tile after the other) whatever the number of workgroups.
+// There is no online maximum (the row maximum is a prefix maximum of the gates), so the weights of several tiles can be formed
+// side by side; only the accumulation over the keys is a chain.  A workgroup here owns one granule of 64 rows and takes 128 keys
+// at a time in two phases:
+//   phase 1   wave (rb, kb) = (row block of 32, key block of 32):  S^T = K Q^T (dQ pass: dC^T = V dH^T) for its 32 x 32 block, gate
+//             weights, the 16-bit weights and the block's share of the row sums to LDS;
+//   phase 2   wave (rb, c) = (row block, D / 4 of the output columns):  H^T += V^T P^T (dQ^T += K^T G^T) over the 128 keys.
+// Phase 2's chain of products per accumulator is that of the consumers of mlstm_row8.hip, phase 1's blocks are those of its
+// producers, and the row sums are added up in its order.  In chunks the state of the previous chunk goes first, as there.
+// Replaces, like mlstm_row8.hip, mlstm_matmul_kernel (mlstm_matmul.py:38-101) and the dQ loop of mlstm_matmul_kernel_backward
+// (mlstm_matmul.py:239-267).
+#include <type_traits>
+#include "mlstm_device.h"
+#include "mlstm_kernels.h"
+
+namespace mlstm {
+
+constexpr int RW_FWD = 0, RW_DQ = 1;
+constexpr int RW_MOST_KEYS = 1024;   // keys a row may meet: their scalars stay in LDS for the whole kernel
+
+template <typename T, int D>
+struct RowwCfg {
+    static constexpr size_t TILE_BYTES = (size_t)GRAN * D * sizeof(T);
+    static constexpr int NST = D == 256 ? 1 : 2;                       // stages of 128 keys for each of Y1 and Y2: 128 KB in all
+    static constexpr size_t POOL_BYTES = 4 * NST * TILE_BYTES;
+    static constexpr size_t P_BYTES = 4 * 2 * 2 * 64 * 16;             // [key block][row block][16 keys][lane] x 16 B
+    static constexpr size_t PART_BYTES = 4 * 2 * 64 * 8;               // [key block][row block][lane] x {sum, row factor}; dQ pass: [column block][row block][lane]
+    static constexpr size_t MISC_FLOATS = 2 * 2 * 32 + 2 * 32 * 2 + D + RW_MOST_KEYS / GRAN;   // row sums, 1/n and db, vector state, granule distances
+    static size_t lds_bytes(int keys) { return POOL_BYTES + P_BYTES + PART_BYTES + MISC_FLOATS * 4 + (size_t)keys * 8 + GRAN * 4; }
+};
+
+template <typename T, int D, int MODE>
+__global__ __launch_bounds__(512) void roww_kernel(RowArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    using R = Tr<T>;
+    using Cfg = RowwCfg<T, D>;
+    typedef typename R::frag frag;
+    static_assert(R::HALF && (D == 128 || D == 256), "16-bit types, D = 128 or 256");
+    constexpr int KW = R::KW, NS = D / KW, NC = D / 128, NST = Cfg::NST;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    frag* const pbuf = reinterpret_cast<frag*>(smem + Cfg::POOL_BYTES);
+    float* const part = reinterpret_cast<float*>(smem + Cfg::POOL_BYTES + Cfg::P_BYTES);
+    float* const bex = part + Cfg::PART_BYTES / 4;         // [rb][kh][32]
+    float* const stat = bex + 2 * 2 * 32;                  // [rb][32] x {1/n, db}
+    float* const nvl = stat + 2 * 32 * 2;                  // [D]
+    float* const sdg = nvl + D;                            // granule of the rows minus granule j
+    float* const sek = sdg + RW_MOST_KEYS / GRAN;          // ek of the keys, then alpha, then the block maxima
+
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = lane >> 5, c32 = lane & 31;
+    const int rb = wave >> 2, kb = wave & 3;               // phase 1: key block kb; phase 2: column blocks NC * kb ...
+    int S = a.S, NG = a.NG;
+    int bh, qt;
+    {
+        // heaviest row tiles first over all heads; with a multiple of 8 heads a head's tiles run on one XCD
+        const int bid = blockIdx.x, nQT = NG;
+        if ((a.BH & 7) == 0) {
+            const int rest = bid >> 3, ngrp = a.BH >> 3;
+            bh = (rest % ngrp) * 8 + (bid & 7);
+            qt = nQT - 1 - rest / ngrp;
+        } else {
+            bh = bid % a.BH;
+            qt = nQT - 1 - bid / a.BH;
+        }
+    }
+    size_t hoff = (size_t)bh * S, poff = (size_t)bh * NG * GRAN, goff = (size_t)bh * NG;
+    const size_t rsA = (size_t)a.la.ss, rsB = (size_t)a.lb.ss, rsH = (size_t)a.lh.ss;
+    size_t offA = a.la.head(bh), offB = a.lb.head(bh), offH = MODE == RW_DQ ? a.lh.head(bh) : 0;
+    int chunk = 0;   // in chunks positions count from the chunk's first one (see mlstm_row8.hip)
+    if (a.chunk_len > 0) {
+        chunk = (qt * GRAN) / a.chunk_len;
+        const int p0 = chunk * a.chunk_len;
+        hoff += p0; poff += p0; goff += p0 / GRAN;
+        offA += (size_t)p0 * rsA; offB += (size_t)p0 * rsB; offH += (size_t)p0 * rsH;
+        S -= p0; qt -= p0 / GRAN;
+    }
+    const int r0 = GRAN * qt;
+    const int nJ = qt + 1;                                  // key tiles; the last one is the rows' own
+    const int row = r0 + 32 * rb + c32, rowc = row < S ? row : S - 1;
+    const size_t rsX = MODE == RW_FWD ? rsA : rsB, offX = MODE == RW_FWD ? offA : offB;
+    const size_t rsO = MODE == RW_FWD ? rsB : rsA, offO = MODE == RW_FWD ? offB : offA;
+    const T* X = reinterpret_cast<const T*>(a.X) + offX;
+    const T* Y1 = reinterpret_cast<const T*>(a.Y1) + offA;
+    const T* Y2 = reinterpret_cast<const T*>(a.Y2) + offA;
+    const int full_tiles = S / GRAN;
+    const int keys = GRAN * nJ;
+    float* const sal = sek + keys;
+    float* const sam = sal + keys;
+
+    // tiles of 64 rows in the pool: Y1 of stage st at 2 st + t, Y2 behind all of those
+    auto tile_at = [&](int n) { return reinterpret_cast<T*>(smem + (size_t)n * Cfg::TILE_BYTES); };
+    auto y1_at = [&](int r, int t) { return tile_at(2 * (r & (NST - 1)) + t); };
+    auto y2_at = [&](int r, int t) { return tile_at(2 * NST + 2 * (r & (NST - 1)) + t); };
+    TileDma<T, D, GRAN, 512> tdma;
+    tdma.init(tid);
+    const auto ra = tdma.rows(tid, (unsigned)(rsA * sizeof(T)));
+    auto copy_tile = [&](T* dst, const T* src, int j) {
+        if (j < full_tiles) tdma.issue(dst, src + (size_t)GRAN * j * rsA, ra);
+        else tile_dma_rolled<T, D, GRAN, 512>(dst, src, GRAN * j, S, tid, rsA);
+    };
+    auto copy_y1 = [&](int r) {
+        copy_tile(y1_at(r, 0), Y1, 2 * r);
+        if (2 * r + 1 < nJ) copy_tile(y1_at(r, 1), Y1, 2 * r + 1);
+    };
+    auto copy_y2 = [&](int r) {
+        copy_tile(y2_at(r, 0), Y2, 2 * r);
+        if (2 * r + 1 < nJ) copy_tile(y2_at(r, 1), Y2, 2 * r + 1);
+    };
+    // (plain loads first: what they bring is used behind the copies' issue)
+    const double g_rows = a.G2[goff + qt], g_mine = a.G2[goff + (tid < nJ ? tid : 0)], g_end = chunk > 0 ? a.G2[goff - 1] : 0.0;
+    const float beta_row = a.beta2[poff + rowc], beta_end = chunk > 0 ? a.beta2[poff - 1] : 0.f;
+    const float n_mine = chunk > 0 && tid < D ? a.Nst[((size_t)bh * a.n_states + chunk - 1) * D + tid] : 0.f;
+    const float m_row = MODE == RW_FWD || kb == 0 ? a.M[hoff + rowc] : 0.f;
+    const float b_row = MODE == RW_DQ && kb == 0 ? a.Bin[hoff + rowc] : 0.f;
+    // piece i of a pair of complete tiles j, j + 1
+    auto copy_piece = [&](const T* src, T* d0, T* d1, int j, int i) {
+        constexpr int PW = TileDma<T, D, GRAN, 512>::PER_WAVE;
+        const int t = i / PW, n = i % PW;
+        tdma.issue_range(t ? d1 : d0, src + (size_t)GRAN * (j + t) * rsA, n, n + 1, ra);
+    };
+    // ---- prologue.  The rows' own operand, the state of the previous chunk and the first keys are requested at once, as far as the
+    // pool holds them.  D = 256: X in tile 3 (then the last state tile), state tiles in 0, 1, 2; D = 128: X in tile 3 (Y1's second
+    // stage), the state in Y2's second stage, the first keys in the first stages.
+    const T* const xtile = tile_at(3);
+    {
+        const auto rx = tdma.rows(tid, (unsigned)(rsX * sizeof(T)));
+        if (r0 + GRAN <= S) tdma.issue(tile_at(3), X + (size_t)r0 * rsX, rx);
+        else tile_dma_rolled<T, D, GRAN, 512>(tile_at(3), X, r0, S, tid, rsX);
+    }
+    const T* const Cst = chunk > 0 ? reinterpret_cast<const T*>(a.Cst) + ((size_t)bh * a.n_states + chunk - 1) * D * D : nullptr;
+    if (chunk > 0) {
+        if constexpr (NST == 1) {
+#pragma unroll
+            for (int t = 0; t < 3; t++) tdma.issue(tile_at(t), Cst + (size_t)GRAN * t * D);
+        } else {
+#pragma unroll
+            for (int t = 0; t < 2; t++) tdma.issue(tile_at(6 + t), Cst + (size_t)GRAN * t * D);
+        }
+    }
+    if (NST == 2 || chunk == 0) copy_y1(0);
+    if (NST == 2) copy_y2(0);
+    for (int t = tdma.wave_s; t < nJ; t += 8) {
+        dma4(a.ek2 + poff + GRAN * t + lane, __builtin_amdgcn_readfirstlane(lds_offset_of(sek + GRAN * t)));
+        dma4(a.alpha2 + poff + GRAN * t + lane, __builtin_amdgcn_readfirstlane(lds_offset_of(sal + GRAN * t)));
+    }
+    if (tid < GRAN) dma4(a.amax2 + goff * 2 + tid, __builtin_amdgcn_readfirstlane(lds_offset_of(sam)));   // (2 nJ of them count; padded array)
+    const float crow_base = -0.5f * __log2f((float)D) - beta_row;
+    float dec = 0.f;   // the row's decay since the end of the previous chunk
+    if (chunk > 0) dec = fast_exp2(beta_end - beta_row + (float)(g_rows - g_end));
+    if (tid < nJ) sdg[tid] = (float)(g_rows - g_mine);
+    if (chunk > 0 && tid < D) nvl[tid] = n_mine;
+    frag hfr[NS];
+    if constexpr (MODE == RW_DQ) {
+        if (kb == 0) {
+            const T* hrow = reinterpret_cast<const T*>(a.Hin) + offH + (size_t)rowc * rsH;
+#pragma unroll
+            for (int s = 0; s < NS; s++) hfr[s] = frag_rowmajor<T>(hrow, s, h);
+        }
+    }
+    SwzRowReaderX<T, D> rrd;
+    rrd.init(lane);
+    SwzTransReader<T, D> vrd;
+    vrd.init(lane, NC * kb);
+    f32x16 acc[NC];
+#pragma unroll
+    for (int c = 0; c < NC; c++)
+#pragma unroll
+        for (int x = 0; x < 16; x++) acc[c][x] = 0.f;
+    dma_wait();
+    __syncthreads();
+    frag xf[NS];
+#pragma unroll
+    for (int s = 0; s < NS; s++) xf[s] = rrd.read(xtile, rb, s);
+    if constexpr (MODE == RW_DQ) {   // 1/n and db of the rows (see row_stats), for this kernel and for the column kernel
+        if (kb == 0) {
+            float dot = 0.f;
+#pragma unroll
+            for (int s = 0; s < NS; s++)
+#pragma unroll
+                for (int e = 0; e < R::EPL; e++) dot += (float)xf[s][e] * (float)hfr[s][e];
+            float inv = 0.f, dbr = 0.f;
+            row_stats_of(sum_halves(dot), b_row, m_row, inv, dbr);
+            if (h == 0) {
+                *reinterpret_cast<float2*>(stat + (32 * rb + c32) * 2) = make_float2(inv, dbr);
+                a.inv_n[poff + row] = row < S ? inv : 0.f;   // (rows behind the sequence: zeros, see mlstm_row.hip)
+                a.db[poff + row] = row < S ? dbr : 0.f;
+            }
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < NS; s++) pin(xf[s]);
+    __syncthreads();   // X's tile is free; the rows' scalars are there
+
+    // G groups of 16 contraction rows out of consecutive tiles, times the fragments operand(g)
+    auto chain = [&](auto groups_tag, auto&& tile, auto&& operand, auto&& hook) {
+        constexpr int G = decltype(groups_tag)::value;
+        frag vf[2][NC], pf[2];
+#pragma unroll
+        for (int c = 0; c < NC; c++) vf[0][c] = vrd.read(tile(0), 0, c);
+        pf[0] = operand(std::integral_constant<int, 0>{});
+        static_for<G>([&](auto gc) __attribute__((always_inline)) {
+            constexpr int g = decltype(gc)::value;
+            if constexpr (g + 1 < G) {
+#pragma unroll
+                for (int c = 0; c < NC; c++) vf[(g + 1) & 1][c] = vrd.read(tile((g + 1) / 4), KW * ((g + 1) % 4), c);
+                pf[(g + 1) & 1] = operand(std::integral_constant<int, g + 1>{});
+            }
+#pragma unroll
+            for (int c = 0; c < NC; c++) R::mma(acc[c], vf[g & 1][c], pf[g & 1]);
+            hook(gc);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    typedef std::integral_constant<int, 8> Eight;
+    typedef std::integral_constant<int, 4> Four;
+    float inv_n = 0.f, dbv = 0.f;
+    if constexpr (MODE == RW_DQ) {
+        const float2 st = *reinterpret_cast<const float2*>(stat + (32 * rb + c32) * 2);
+        inv_n = st.x; dbv = st.y;
+    }
+    if (chunk > 0) {
+        if constexpr (NST == 1) {
+            tdma.issue(tile_at(3), Cst + (size_t)GRAN * 3 * D);
+            chain(std::integral_constant<int, 12>{}, [&](int t) { return tile_at(t); }, [&](auto g) { return xf[decltype(g)::value]; }, [](auto) {});
+            dma_wait();
+            __syncthreads();
+            copy_y1(0);
+            chain(Four{}, [&](int) { return tile_at(3); }, [&](auto g) { return xf[12 + decltype(g)::value]; }, [](auto) {});
+        } else {
+            chain(Eight{}, [&](int t) { return tile_at(6 + t); }, [&](auto g) { return xf[decltype(g)::value]; }, [](auto) {});
+        }
+        if constexpr (MODE == RW_FWD) {
+#pragma unroll
+            for (int c = 0; c < NC; c++)
+#pragma unroll
+                for (int x = 0; x < 16; x++) acc[c][x] *= dec;
+        } else {
+            const float rank1 = dec * dbv, decn = dec * inv_n;
+            const T* qrow = reinterpret_cast<const T*>(a.Qrow) + offA + (size_t)rowc * rsA;
+#pragma unroll
+            for (int c = 0; c < NC; c++) {
+                float rp = 0.f;   // q_i . dQ_i of the state part: the row sums of dD over the keys before the chunk
+#pragma unroll
+                for (int a4 = 0; a4 < 4; a4++) {
+                    const int col = 32 * (NC * kb + c) + 8 * a4 + 4 * h;
+                    const f32x4 nv = *reinterpret_cast<const f32x4*>(nvl + col);
+                    const f32x4 qv = __builtin_convertvector(*reinterpret_cast<const typename R::vec4*>(qrow + col), f32x4);
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        acc[c][4 * a4 + e] = fmaf(acc[c][4 * a4 + e], decn, rank1 * nv[e]);
+                        rp = fmaf(acc[c][4 * a4 + e], qv[e], rp);
+                    }
+                }
+                part[((NC * kb + c) * 2 + rb) * 64 + lane] = rp;
+            }
+        }
+    }
+
+    // ---- the key tiles, two at a time
+    const int nR = (nJ + 1) / 2;
+    float bsum = 0.f;   // waves kb < 2: the row sums over the key blocks of parity kb, in the order of the keys
+    for (int r = 0; r < nR; r++) {
+        const bool two = 2 * r + 1 < nJ;
+        dma_wait();
+        __syncthreads();   // this round's Y1 (NST == 2: and Y2) has landed; phase 2 of the previous round is over
+        // The copies under phase 1: NST == 1 this round's Y2, NST == 2 both of the next round's.  A wave that issues its loads back
+        // to back waits for the memory pipeline (64 KB: 0.5 us per round, measured), so they go between the products.
+        const int rc = NST == 1 ? r : r + 1;
+        const bool copies = rc < nR, spread1 = copies && 2 * rc + 1 < nJ && 2 * rc + 1 < full_tiles;
+        const int j = 2 * r + (kb >> 1);
+        if (copies && !(spread1 && j < nJ)) {
+            if constexpr (NST == 2) copy_y1(rc);
+            copy_y2(rc);
+        }
+        auto phase1 = [&](auto spread_tag) __attribute__((always_inline)) {
+            constexpr bool SPREAD = decltype(spread_tag)::value;
+            f32x16 s;
+            const int k0 = GRAN * j + 32 * (kb & 1), rr = r0 + 32 * rb;
+            const T* y1 = y1_at(r, kb >> 1);
+            const float crow = crow_base + sdg[j];
+            constexpr int AHEAD = 4;
+            frag kf[NS];
+#pragma unroll
+            for (int n = 0; n < AHEAD; n++) kf[n] = rrd.read(y1, kb & 1, n);
+#pragma unroll
+            for (int n = 0; n < NS; n++) {
+                if (n + AHEAD < NS) kf[n + AHEAD] = rrd.read(y1, kb & 1, n + AHEAD);
+                if (n == 0) {
+#pragma unroll
+                    for (int x = 0; x < 16; x++) s[x] = 0.f;
+                }
+                R::mma(s, kf[n], xf[n]);
+                if constexpr (SPREAD) {
+                    if constexpr (NST == 1) {
+                        if (n % 2 == 0) copy_piece(Y2, y2_at(r, 0), y2_at(r, 1), 2 * r, n / 2);
+                    } else {
+                        if (n < 4) copy_piece(Y1, y1_at(rc, 0), y1_at(rc, 1), 2 * rc, n);
+                        else copy_piece(Y2, y2_at(rc, 0), y2_at(rc, 1), 2 * rc, n - 4);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            float blk = 0.f, er = 0.f;
+            if (k0 > rr) {             // above the diagonal
+#pragma unroll
+                for (int x = 0; x < 16; x++) s[x] = 0.f;
+            } else if (k0 < rr) {      // below it: factorised weights
+                er = fast_exp2(crow + sam[k0 / 32]);
+                const float sc = inv_n * er, of = dbv * er;
+#pragma unroll
+                for (int a4 = 0; a4 < 4; a4++) {
+                    const f32x4 ek = *reinterpret_cast<const f32x4*>(sek + k0 + 8 * a4 + 4 * h);
+#pragma unroll
+                    for (int c = 0; c < 4; c++) {
+                        const int x = 4 * a4 + c;
+                        if constexpr (MODE == RW_FWD) {
+                            const float t = s[x] * ek[c];
+                            blk += t;
+                            s[x] = t * er;
+                        } else {
+                            s[x] = (s[x] * sc + of) * ek[c];
+                        }
+                    }
+                }
+            } else {                   // on it
+#pragma unroll
+                for (int a4 = 0; a4 < 4; a4++) {
+                    const f32x4 al = *reinterpret_cast<const f32x4*>(sal + k0 + 8 * a4 + 4 * h);
+#pragma unroll
+                    for (int c = 0; c < 4; c++) {
+                        const int x = 4 * a4 + c;
+                        float e = fast_exp2(al[c] + crow);
+                        if (8 * a4 + 4 * h + c > c32) e = 0.f;
+                        if constexpr (MODE == RW_FWD) {
+                            s[x] *= e;
+                            blk += s[x];
+                        } else {
+                            s[x] = (s[x] * inv_n + dbv) * e;
+                        }
+                    }
+                }
+                er = 1.f;
+            }
+            frag* const p = pbuf + (kb * 2 + rb) * 2 * 64 + lane;
+            p[0] = R::from_acc(s, 0);
+            p[64] = R::from_acc(s, 1);
+            if constexpr (MODE == RW_FWD) *reinterpret_cast<float2*>(part + ((kb * 2 + rb) * 64 + lane) * 2) = make_float2(blk, er);
+        };
+        if (j < nJ) {
+            if (spread1) phase1(std::true_type{});
+            else phase1(std::false_type{});
+        }
+        if constexpr (NST == 1) dma_wait();
+        __syncthreads();
+        if constexpr (MODE == RW_FWD) {
+            if (kb < 2) {
+#pragma unroll
+                for (int t = 0; t < 2; t++)
+                    if (t == 0 || two) {
+                        const float2 be = *reinterpret_cast<const float2*>(part + (((2 * t + kb) * 2 + rb) * 64 + lane) * 2);
+                        bsum = fmaf(be.x, be.y, bsum);
+                    }
+            }
+        }
+        const frag* const p = pbuf + rb * 2 * 64 + lane;
+        auto weights = [&](auto g) { return p[((decltype(g)::value >> 1) * 2 * 2 + (decltype(g)::value & 1)) * 64]; };
+        auto y2 = [&](int t) { return y2_at(r, t); };
+        auto none = [](auto) {};
+        const bool spread2 = NST == 1 && r + 1 < nR && 2 * r + 3 < nJ && 2 * r + 3 < full_tiles;   // the next round's Y1 under phase 2
+        if constexpr (NST == 1) {
+            if (r + 1 < nR && !spread2) copy_y1(r + 1);
+        }
+        if (spread2) chain(Eight{}, y2, weights, [&](auto g) { copy_piece(Y1, y1_at(r + 1, 0), y1_at(r + 1, 1), 2 * r + 2, decltype(g)::value); });
+        else if (two) chain(Eight{}, y2, weights, none);
+        else chain(Four{}, y2, weights, none);
+    }
+    // ---- epilogue
+    uint4 og[D / 64];   // output gate: this thread's pieces, requested ahead of the barriers
+    constexpr int CPR = D * (int)sizeof(T) / 16, RB = D * (int)sizeof(T) + 16, NP = 64 * CPR / 512;
+    static_assert(NP == D / 64, "pieces per thread");
+    if constexpr (MODE == RW_FWD) {
+        if (a.O) {
+            const char* go = reinterpret_cast<const char*>(a.O) + (offB + (size_t)r0 * rsB) * sizeof(T);
+#pragma unroll
+            for (int i = 0; i < NP; i++) {
+                const int c = tid + 512 * i, rr = c / CPR, cc = c % CPR;
+                og[i] = r0 + rr < S ? *reinterpret_cast<const uint4*>(go + (size_t)rr * rsB * sizeof(T) + 16 * cc) : uint4{0, 0, 0, 0};
+            }
+        }
+        if (kb < 2) {
+            if (chunk > 0) {   // what lies before the chunk: decay (q . n~), half of the contraction each
+                const float* nst = nvl + 8 * h;
+                float pt = 0.f;
+                auto half_dot = [&](auto first_tag) {
+                    constexpr int S0 = decltype(first_tag)::value;
+#pragma unroll
+                    for (int s = S0; s < S0 + NS / 2; s++) {
+                        const f32x4 n0 = *reinterpret_cast<const f32x4*>(nst + KW * s), n1 = *reinterpret_cast<const f32x4*>(nst + KW * s + 4);
+                        const f32x8 qv = __builtin_convertvector(xf[s], f32x8);
+#pragma unroll
+                        for (int e = 0; e < 4; e++) pt = fmaf(qv[4 + e], n1[e], fmaf(qv[e], n0[e], pt));
+                    }
+                };
+                if (kb == 0) half_dot(std::integral_constant<int, 0>{});
+                else half_dot(std::integral_constant<int, NS / 2>{});
+                bsum = fmaf(pt, dec, bsum);
+            }
+            const float b = sum_halves(bsum);
+            if (h == 0) bex[(rb * 2 + kb) * 32 + c32] = b;
+        }
+    }
+    __syncthreads();   // the row sums are there; every wave is done with the pool
+    float onorm = 1.0f;
+    if constexpr (MODE == RW_FWD) {
+        const float b = bex[(rb * 2 + 0) * 32 + c32] + bex[(rb * 2 + 1) * 32 + c32];
+        onorm = 1.0f / (fmaxf(fabsf(b), __expf(-m_row)) + 1e-6f);
+        if (kb == 0 && h == 0 && row < S) a.Bsum[hoff + row] = b;
+    } else {
+        if (a.chunk_len > 0 && kb == 0) {
+            float v = 0.f;
+            if (chunk > 0) {
+#pragma unroll
+                for (int half = 0; half < 2; half++) {
+                    float rp = 0.f;
+#pragma unroll
+                    for (int d = 0; d < D / 64; d++) rp += part[((half * (D / 64) + d) * 2 + rb) * 64 + lane];
+                    rp = sum_halves(rp);
+                    v = half ? v + rp : rp;
+                }
+            }
+            if (h == 0 && row < S) a.rowinter[hoff + row] = v;
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < NC; c++)
+#pragma unroll
+        for (int a4 = 0; a4 < 4; a4++) {
+            f32x4 v;
+#pragma unroll
+            for (int e = 0; e < 4; e++) v[e] = acc[c][4 * a4 + e] * onorm;
+            *reinterpret_cast<typename R::vec4*>(smem + (32 * rb + c32) * RB + (32 * (NC * kb + c) + 8 * a4 + 4 * h) * (int)sizeof(T)) = R::cvt4(v);
+        }
+    __syncthreads();
+    {
+        char* const gout = reinterpret_cast<char*>(a.out) + (offO + (size_t)r0 * rsO) * sizeof(T);
+        char* const gg = MODE == RW_FWD ? reinterpret_cast<char*>(a.out_gated) + (offB + (size_t)r0 * rsB) * sizeof(T) : nullptr;
+#pragma unroll
+        for (int i = 0; i < NP; i++) {
+            const int c = tid + 512 * i, rr = c / CPR, cc = c % CPR;
+            const uint4 v = *reinterpret_cast<const uint4*>(smem + rr * RB + 16 * cc);
+            if (r0 + rr < S) {
+                *reinterpret_cast<uint4*>(gout + (size_t)rr * rsO * sizeof(T) + 16 * cc) = v;
+                if constexpr (MODE == RW_FWD) {
+                    if (a.O) {
+                        typedef typename R::vec4 V4;
+                        struct Pair { V4 lo, hi; };
+                        const Pair hv = __builtin_bit_cast(Pair, v), ov = __builtin_bit_cast(Pair, og[i]);
+                        Pair res;
+                        res.lo = gate4<T>(hv.lo, ov.lo);
+                        res.hi = gate4<T>(hv.hi, ov.hi);
+                        *reinterpret_cast<Pair*>(gg + (size_t)rr * rsB * sizeof(T) + 16 * cc) = res;
+                    }
+                }
+            }
+        }
+    }
+#endif
+}
+
+template <typename T, int D, int MODE>
+static int launch_roww_t(const RowArgs& a, hipStream_t st) {
+    using Cfg = RowwCfg<T, D>;
+    const int most = a.chunk_len > 0 && a.chunk_len < a.NG * GRAN ? a.chunk_len : a.NG * GRAN;   // keys a row may meet
+    if (most > RW_MOST_KEYS) return MLSTM_ESHAPE;
+    if (hipError_t e = lds_limit_once<roww_kernel<T, D, MODE>>((int)Cfg::lds_bytes(RW_MOST_KEYS)); e != hipSuccess) return (int)e;
+    hipLaunchKernelGGL((roww_kernel<T, D, MODE>), dim3(a.BH * a.NG), dim3(512), Cfg::lds_bytes(most), st, a);
+    return (int)hipGetLastError();
+}
+
+template <typename T>
+static int launch_roww_m(int mode, int D, const RowArgs& a, hipStream_t st) {
+    if (mode == RW_FWD) return D == 128 ? launch_roww_t<T, 128, RW_FWD>(a, st) : launch_roww_t<T, 256, RW_FWD>(a, st);
+    return D == 128 ? launch_roww_t<T, 128, RW_DQ>(a, st) : launch_roww_t<T, 256, RW_DQ>(a, st);
+}
+
+int launch_roww_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t st) {
+    return dtype == MLSTM_F16 ? launch_roww_m<_Float16>(mode, D, a, st) : launch_roww_m<__bf16>(mode, D, a, st);
+}
+
+}  // namespace mlstm
