@@ -1,6 +1,6 @@
-"""Kernels for launches that would leave the chip part empty (roww_kernel, chunk_sum_narrow_kernel) against the ones that
+"""Kernels for launches that would leave the chip part empty (roww_kernel, chunk_sum_narrow_kernel; fp32: rowf_kernel) against the ones that
 serve larger launches: the same products in the same order, so a head alone and the same head in a batch that is large enough for the
-other kernels give the same bits.  Lengths at the edges of the 64-row tiles, of the pairs of key tiles and of the chunks."""
+other kernels give the same bits.  Lengths at the edges of the 64-row tiles, of the pairs of key tiles, of the 32-row blocks and of the chunks."""
 import pytest
 import torch
 
@@ -40,3 +40,12 @@ def test_a_head_alone_is_the_head_of_a_full_chip(op, S, D, heads, layout, dtype)
     rows, gates = _inputs(heads, S, D, dtype, layout)
     for name, a, b in zip(range(10), _step(op, rows, gates, 1), _step(op, rows, gates, heads)):
         assert bool(torch.isfinite(b.float()).all()) and torch.equal(a[:, :1], b[:, :1]), name
+
+
+# fp32: more than 512 workgroups of 32 rows.
+@pytest.mark.parametrize("op,S,D,heads,layout", [
+    ("plain", 1, 64, 260, "bnsd"), ("plain", 31, 128, 260, "bnsd"), ("plain", 33, 64, 260, "bsnd"), ("plain", 64, 128, 260, "bnsd"),
+    ("gated", 97, 128, 130, "bnsd"), ("plain", 129, 64, 90, "bnsd"), ("plain", 319, 64, 52, "bnsd"), ("gated", 319, 128, 52, "bsnd"),
+    ("plain", 320, 64, 52, "bnsd"), ("gated", 450, 64, 33, "bsnd"), ("plain", 700, 128, 24, "bnsd"), ("plain", 1000, 64, 17, "bnsd")])
+def test_a_head_alone_is_the_head_of_a_full_chip_fp32(op, S, D, heads, layout):
+    test_a_head_alone_is_the_head_of_a_full_chip(op, S, D, heads, layout, torch.float32)

@@ -124,6 +124,8 @@ struct RowArgs {
 };
 // mode 0 = forward (H, b), mode 1 = dQ
 int launch_row_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t st);
+// fp32 on 32 rows per workgroup, the same bits, for launches that leave the chip part empty; D in {64, 128}
+int launch_rowf_kernel(int mode, int D, const RowArgs& a, hipStream_t st);
 // eight waves (producer / consumer pairs per SIMD); 16-bit types and D in {128, 256} only
 int launch_row8_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t st);
 // the same bits on 64 rows per workgroup, for launches that leave the chip part empty; 16-bit types and D in {128, 256} only
@@ -165,6 +167,7 @@ struct ColArgs {
     Lay la, lb;              // layouts of Q, K, V, dK, dV (la) and of dH (lb)
 };
 int launch_col_kernel(int dtype, int D, const ColArgs& a, hipStream_t st);
+int launch_colf_kernel(int D, const ColArgs& a, hipStream_t st);
 // phase A as 16x16x32 products on two query halves, the element-wise part of the first between the MFMAs of the second;
 // 16-bit types at D = 128 and 256 only
 int launch_col16_kernel(int dtype, int D, const ColArgs& a, hipStream_t st);

@@ -27,10 +27,11 @@
 #include <type_traits>
 #include "mlstm_device.h"
 #include "mlstm_kernels.h"
+#include "mlstm_row_exact.h"
 
 namespace mlstm {
 
-constexpr int MODE_FWD = 0, MODE_DQ = 1;
+constexpr int MODE_FWD = ROW_MODE_FWD, MODE_DQ = ROW_MODE_DQ;
 constexpr int ROW_BQ = 128;
 
 template <typename T, int D>
@@ -40,77 +41,6 @@ struct RowCfg {
     static constexpr size_t STAGES_BYTES = 2 * STAGE_BYTES;
     // plus one double per key tile of the head (the granule bases), appended at launch
 };
-
-// One row by one wave from its definition, in fp32 multiply-adds straight from memory (see not_finite in mlstm_device.h): the keys
-// of the row's own chunk one after the other and the state before it, columns lane and lane + 64.  Positions count from the
-// chunk's first one, as in the kernel.
-template <int D, int MODE>
-__device__ __forceinline__ void row_exact(const RowArgs& a, int bh, int chunk, int t, int S, size_t hoff, size_t poff, size_t goff, const float* x,
-                                          const float* Y1, const float* Y2, size_t rsA, size_t offA, size_t offO, size_t offB, size_t rsO, size_t rsB,
-                                          float inv_n, float db) {
-    constexpr int NC = D / 64;
-    const int lane = threadIdx.x & 63;
-    const double G = a.G2[goff + t / GRAN];
-    const float crow = -0.5f * __log2f((float)D) - a.beta2[poff + t];
-    float xv[NC], o[NC], b = 0.f;
-#pragma unroll
-    for (int n = 0; n < NC; n++) { xv[n] = x[lane + 64 * n]; o[n] = 0.f; }
-    if (chunk > 0) {
-        const size_t st = (size_t)bh * a.n_states + chunk - 1;
-        const float* C = reinterpret_cast<const float*>(a.Cst) + st * D * D;
-        const float* nst = a.Nst + st * D;
-        for (int k = 0; k < D; k++) {   // (row k of the state lies where the tile kernels' transposing reads want it: mlstm_chunk.hip)
-            const float xk = x[k];
-            const int at = (k & ~12) | ((k & 4) << 1) | ((k & 8) >> 1);
-#pragma unroll
-            for (int n = 0; n < NC; n++) o[n] += xk * C[(size_t)at * D + lane + 64 * n];
-            if constexpr (MODE == MODE_FWD) b += xk * nst[k];
-        }
-        const float dec = fast_exp2(a.beta2[poff - 1] - a.beta2[poff + t] + (float)(G - a.G2[goff - 1]));
-        if constexpr (MODE == MODE_FWD) {
-            b *= dec;
-#pragma unroll
-            for (int n = 0; n < NC; n++) o[n] *= dec;
-        } else {
-            const float* q = reinterpret_cast<const float*>(a.Qrow) + offA + (size_t)t * rsA;
-            float rp = 0.f;
-#pragma unroll
-            for (int n = 0; n < NC; n++) {
-                o[n] = o[n] * (dec * inv_n) + dec * db * nst[lane + 64 * n];
-                rp += o[n] * q[lane + 64 * n];
-            }
-            rp = wave_reduce<OpAdd>(rp);
-            if (lane == (t & 31)) a.rowinter[hoff + t] = rp;
-        }
-    }
-    for (int j = 0; j <= t; j++) {
-        float s = 0.f;
-#pragma unroll
-        for (int n = 0; n < NC; n++) s += xv[n] * Y1[(size_t)j * rsA + lane + 64 * n];
-        s = wave_reduce<OpAdd>(s);
-        const float e = fast_exp2(a.alpha2[poff + j] + (crow + (float)(G - a.G2[goff + j / GRAN])));
-        const float p = MODE == MODE_FWD ? s * e : (s * inv_n + db) * e;
-        b += p;
-#pragma unroll
-        for (int n = 0; n < NC; n++) o[n] += p * Y2[(size_t)j * rsA + lane + 64 * n];
-    }
-    float onorm = 1.0f;
-    if constexpr (MODE == MODE_FWD) {
-        onorm = 1.0f / (fmaxf(fabsf(b), __expf(-a.M[hoff + t])) + 1e-6f);
-        if (lane == (t & 31)) a.Bsum[hoff + t] = b;
-    }
-#pragma unroll
-    for (int n = 0; n < NC; n++) {
-        const int d = lane + 64 * n;
-        reinterpret_cast<float*>(a.out)[offO + (size_t)t * rsO + d] = o[n] * onorm;
-        if constexpr (MODE == MODE_FWD) {
-            if (a.O) {
-                const size_t at = offB + (size_t)t * rsB + d;
-                reinterpret_cast<float*>(a.out_gated)[at] = o[n] * onorm * silu(reinterpret_cast<const float*>(a.O)[at]);
-            }
-        }
-    }
-}
 
 // STRICT (16-bit types): split mode, see RowArgs::precise.
 template <typename T, int D, int MODE, bool STRICT>
@@ -281,6 +211,7 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
     };
     // gate weights; `diag` masks the keys above the diagonal of a diagonal block
     auto weigh = [&](f32x16& sacc, const float* sal, int kb, Crow crow, bool diag) {
+        float blk = 0.f;
 #pragma unroll
         for (int a4 = 0; a4 < 4; a4++) {
             const f32x4 al = *reinterpret_cast<const f32x4*>(sal + 32 * kb + 8 * a4 + 4 * h);
@@ -292,14 +223,14 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
                 else e = fast_exp2(al[c] + crow);
                 if (diag && (8 * a4 + 4 * h + c > c32)) e = 0.f;
                 if constexpr (MODE == MODE_FWD) {
-                    const float p = sacc[r] * e;
-                    bsum += p;
-                    sacc[r] = p;
+                    sacc[r] *= e;
+                    blk += sacc[r];
                 } else {
                     sacc[r] = (sacc[r] * inv_n + dbv) * e;
                 }
             }
         }
+        if constexpr (MODE == MODE_FWD) bsum += blk;
     };
     // gate weights of a block entirely below the diagonal, factorised: exp2(alpha_j - c0) comes from the pre-pass
     // (sek), exp2(c0 - beta_i + dG) is one exponential per lane and block
@@ -323,7 +254,7 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
                 }
             }
         }
-        if constexpr (MODE == MODE_FWD) bsum += blk * er;
+        if constexpr (MODE == MODE_FWD) bsum = fmaf(blk, er, bsum);
     };
     // second product: accumulate this key block into the output
     auto gemm2 = [&](const T* y2, const f32x16& sacc, int kb, auto&& hook) {
@@ -440,7 +371,7 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
             if (g == 1) take_p(s1, 0);
             if (g == 2) take_p(s1, 1);
         }
-        if constexpr (MODE == MODE_FWD) bsum += blk0 * er0 + blk1 * er1;
+        if constexpr (MODE == MODE_FWD) bsum = fmaf(blk1, er1, fmaf(blk0, er0, bsum));
       }
     };
 
@@ -507,8 +438,8 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
 #pragma unroll
             for (int s2 = 0; s2 < NS; s2++)
 #pragma unroll
-                for (int e = 0; e < R::EPL; e++) part += to_f32(xf[s2][e]) * nst[KW * s2 + R::EPL * h + e];
-            bsum += dec * part;
+                for (int e = 0; e < R::EPL; e++) part = fmaf(to_f32(xf[s2][e]), nst[KW * s2 + R::EPL * h + e], part);
+            bsum = fmaf(dec, part, bsum);
 #pragma unroll
             for (int d = 0; d < NDB; d++)
 #pragma unroll
@@ -516,9 +447,10 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
         } else {
             const float decn = dec * inv_n, rank1 = dec * dbv;
             const T* qrow = reinterpret_cast<const T*>(a.Qrow) + offA + (size_t)rowc * rsA;
-            float rp = 0.f;
+            float rp = 0.f;   // (summed per block of 32 columns, as mlstm_rowf.hip, which splits a row by columns, has to)
 #pragma unroll
-            for (int d = 0; d < NDB; d++)
+            for (int d = 0; d < NDB; d++) {
+                float rpd = 0.f;
 #pragma unroll
                 for (int a4 = 0; a4 < 4; a4++) {
                     const int col = 32 * d + 8 * a4 + 4 * h;
@@ -526,11 +458,13 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
                     const f32x4 qv = __builtin_convertvector(*reinterpret_cast<const typename R::vec4*>(qrow + col), f32x4);
 #pragma unroll
                     for (int c = 0; c < 4; c++) {
-                        const float v = oacc[d][4 * a4 + c] * decn + rank1 * nv[c];
+                        const float v = fmaf(oacc[d][4 * a4 + c], decn, rank1 * nv[c]);
                         oacc[d][4 * a4 + c] = v;
-                        rp += v * qv[c];
+                        rpd = fmaf(v, qv[c], rpd);
                     }
                 }
+                rp += rpd;
+            }
             // row sums of dD over the keys before the chunk: q_i . dQ_i of what the accumulators hold now
             rp = sum_halves(rp);
             if (row < S && h == 0) a.rowinter[hoff + row] = rp;
@@ -735,6 +669,9 @@ static int launch_row_d(int D, const RowArgs& a, hipStream_t st) {
 }
 
 int launch_row_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t st) {
+    // fp32 up to one (D = 64) or two (D = 128) workgroups of 32 rows per CU: row_kernel / rowf_kernel, forward, us, in chunks of 128 --
+    //   D = 64    256: 15.7 / 10.3   384: 16.0 / 17.4     D = 128   256: 27.8 / 13.7   512: 28.9 / 25.4   640 (uncut): 36.7 / 36.6   1024: 32.5 / 45.1
+    if (dtype == MLSTM_F32 && D <= 128 && 2ll * a.BH * a.NG <= (D == 64 ? 256 : 512)) return launch_rowf_kernel(mode, D, a, st);
     if (mode == MODE_FWD) {
         switch (dtype) {
             case MLSTM_F32: return launch_row_d<float, MODE_FWD>(D, a, st);
