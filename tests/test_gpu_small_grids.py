@@ -1,4 +1,4 @@
-"""Kernels for launches that would leave the chip part empty (roww_kernel, chunk_sum_narrow_kernel; fp32: rowf_kernel) against the ones that
+"""Kernels for launches that would leave the chip part empty (roww_kernel, chunk_sum_narrow_kernel; fp32: rowf_kernel, colf_kernel) against the ones that
 serve larger launches: the same products in the same order, so a head alone and the same head in a batch that is large enough for the
 other kernels give the same bits.  Lengths at the edges of the 64-row tiles, of the pairs of key tiles, of the 32-row blocks and of the chunks."""
 import pytest
@@ -42,7 +42,7 @@ def test_a_head_alone_is_the_head_of_a_full_chip(op, S, D, heads, layout, dtype)
         assert bool(torch.isfinite(b.float()).all()) and torch.equal(a[:, :1], b[:, :1]), name
 
 
-# fp32: more than 512 workgroups of 32 rows.
+# fp32: more than 512 workgroups of 32 rows.  (colf_kernel serves chunks of 128 at D = 128 whatever the number of heads.)
 @pytest.mark.parametrize("op,S,D,heads,layout", [
     ("plain", 1, 64, 260, "bnsd"), ("plain", 31, 128, 260, "bnsd"), ("plain", 33, 64, 260, "bsnd"), ("plain", 64, 128, 260, "bnsd"),
     ("gated", 97, 128, 130, "bnsd"), ("plain", 129, 64, 90, "bnsd"), ("plain", 319, 64, 52, "bnsd"), ("gated", 319, 128, 52, "bsnd"),

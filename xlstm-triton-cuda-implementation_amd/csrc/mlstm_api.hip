@@ -812,12 +812,14 @@ int backward_impl(const void* dh, const void* q, const void* k, const void* v, c
     ca.BH = (int)z.BH; ca.S = (int)z.S; ca.NG = (int)z.NG;
     ca.precise = z.precise ? 1 : 0; ca.RS = (int)z.row_slices();
     if (col_chunks) { ca.chunk_len = w.L; ca.n_states = (int)w.ncs; ca.Ev = Ev; ca.Ev_lo = z.precise ? Ev + lo_off : nullptr; ca.gvec = gvec; }
+    // (the rows of h have been read by the dQ pass: their buffer takes a second array of row partials, of no more than D slices)
+    if (colf_serves(dtype, D, ca)) ca.rowpart2 = reinterpret_cast<float*>(hbuf);
     {
         Timed t(MLSTM_K_COL, st);
         if (int rc = launch_col_best(dtype, D, ca, st)) return rc;
     }
 
-    DfArgs da{f, colsum, rowpart, df, di, (int)z.BH, (int)z.S, (int)z.NG, (int)z.row_slices(), col_chunks ? w.L : 0, rowinter, anchor, (int)w.ncs};
+    DfArgs da{f, colsum, rowpart, df, di, (int)z.BH, (int)z.S, (int)z.NG, (int)z.row_slices(), ca.rowpart2, col_chunks ? w.L : 0, rowinter, anchor, (int)w.ncs};
     da.lg = z.lg; da.gate_form = z.gate_form; da.stamp = stamp;
     if (col_chunks && fused_anchor) {
         da.anchor = nullptr; da.anchor_part = anchor; da.anchor_parts = anchor_parts; da.anchor_va = Nst; da.anchor_vb = gvec; da.D = D;

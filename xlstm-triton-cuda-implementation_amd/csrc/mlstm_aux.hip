@@ -96,7 +96,7 @@ __global__ __launch_bounds__(1024) void dfscan_kernel(const TG* __restrict__ F, 
 // per head, a thread per position (twice, beyond 1024): a position has at most 32 row partials.  As two kernels (rowreduce,
 // dfscan) the pair took 4.7 + 4.0 us at B1 H2 S300 and a launch more, in steps of 50 to 100 us.
 template <typename TG>
-__global__ __launch_bounds__(1024) void dfhead_kernel(const TG* __restrict__ F, const float* __restrict__ colsum, const float* __restrict__ rowpart,
+__global__ __launch_bounds__(1024) void dfhead_kernel(const TG* __restrict__ F, const float* __restrict__ colsum, const float* __restrict__ rowpart, const float* __restrict__ rowpart2,
                                                       TG* __restrict__ dF, TG* __restrict__ dI, int S, int RS, Lay lg, int form, SavedStamp stamp) {
     __shared__ float wt[2][16];
     const int bh = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = blockDim.x >> 6;
@@ -113,6 +113,11 @@ __global__ __launch_bounds__(1024) void dfhead_kernel(const TG* __restrict__ F, 
                 float part[16];   // (the loads leave together)
 #pragma unroll
                 for (int j = 0; j < 16; j++) part[j] = j0 + j <= g ? rp[(size_t)(j0 + j) * S] : 0.f;
+                if (rowpart2) {   // (the tiles' second halves)
+                    const float* rp2 = rowpart2 + (rp - rowpart);
+#pragma unroll
+                    for (int j = 0; j < 16; j++) part[j] += j0 + j <= g ? rp2[(size_t)(j0 + j) * S] : 0.f;
+                }
 #pragma unroll
                 for (int j = 0; j < 16; j++) row += part[j];
             }
@@ -142,7 +147,7 @@ __global__ __launch_bounds__(1024) void dfhead_kernel(const TG* __restrict__ F, 
 // position has at most chunk_len / 64 row partials.  chunk_len <= 1024; as many threads as positions (or as the anchors' sums
 // take), whole waves: with 1024 whatever the chunk, most of a workgroup's waves had nothing to do but arrive at the barrier.
 template <typename TG>
-__global__ __launch_bounds__(1024) void dfchunk_kernel(const TG* __restrict__ F, const float* __restrict__ colsum, const float* __restrict__ rowpart,
+__global__ __launch_bounds__(1024) void dfchunk_kernel(const TG* __restrict__ F, const float* __restrict__ colsum, const float* __restrict__ rowpart, const float* __restrict__ rowpart2,
                                                        const float* __restrict__ rowinter, const float* __restrict__ anchor,
                                                        TG* __restrict__ dF, TG* __restrict__ dI, int S, int RS, int chunk_len, int n_states,
                                                        Lay lg, int form, const float* __restrict__ anchor_part, int anchor_parts,
@@ -179,6 +184,11 @@ __global__ __launch_bounds__(1024) void dfchunk_kernel(const TG* __restrict__ F,
         float part[16];   // (a fixed count, so that the loads leave together: chunk_len <= 1024 is at most 16 slices)
 #pragma unroll
         for (int j = 0; j < 16; j++) part[j] = j <= g - g0 ? rp[(size_t)j * S] : 0.f;
+        if (rowpart2) {   // (the tiles' second halves)
+            const float* rp2 = rowpart2 + (rp - rowpart);
+#pragma unroll
+            for (int j = 0; j < 16; j++) part[j] += j <= g - g0 ? rp2[(size_t)j * S] : 0.f;
+        }
 #pragma unroll
         for (int j = 0; j < 16; j++) row += part[j];
         col = colsum[(size_t)bh * S + t];
@@ -219,14 +229,14 @@ static int launch_df_t(const DfArgs& a, hipStream_t st) {
         if (a.anchor_part) threads = threads > a.D ? threads : a.D;
         if (threads < a.anchor_parts) threads = a.anchor_parts;
         hipLaunchKernelGGL(dfchunk_kernel<TG>, dim3((a.S + a.chunk_len - 1) / a.chunk_len, a.BH), dim3((threads + 63) / 64 * 64), 0, st, reinterpret_cast<const TG*>(a.F),
-                           a.colsum, a.rowpart, a.rowinter, a.anchor, reinterpret_cast<TG*>(a.dF), reinterpret_cast<TG*>(a.dI), a.S, a.RS,
+                           a.colsum, a.rowpart, a.rowpart2, a.rowinter, a.anchor, reinterpret_cast<TG*>(a.dF), reinterpret_cast<TG*>(a.dI), a.S, a.RS,
                            a.chunk_len, a.n_states, a.lg, a.gate_form, a.anchor_part, a.anchor_parts, a.anchor_va, a.anchor_vb, a.D, a.stamp);
         return (int)hipGetLastError();
     }
     if (a.anchor_part) return MLSTM_EINVAL;   // (only the one-kernel form adds the parts up)
     if (a.chunk_len == 0 && a.S <= 2048) {
         const int threads = a.S < 1024 ? (a.S + 63) / 64 * 64 : 1024;
-        hipLaunchKernelGGL(dfhead_kernel<TG>, dim3(a.BH), dim3(threads), 0, st, reinterpret_cast<const TG*>(a.F), a.colsum, a.rowpart,
+        hipLaunchKernelGGL(dfhead_kernel<TG>, dim3(a.BH), dim3(threads), 0, st, reinterpret_cast<const TG*>(a.F), a.colsum, a.rowpart, a.rowpart2,
                            reinterpret_cast<TG*>(a.dF), reinterpret_cast<TG*>(a.dI), a.S, a.RS, a.lg, a.gate_form, a.stamp);
         return (int)hipGetLastError();
     }

@@ -23,6 +23,7 @@
 #include <type_traits>
 #include "mlstm_device.h"
 #include "mlstm_kernels.h"
+#include "mlstm_col_exact.h"
 
 namespace mlstm {
 
@@ -55,85 +56,6 @@ struct ColCfg {
 // 32 consecutive rows per instruction (all 16 residues of q spread over both 128-byte bank windows x 8 chunks);
 // phase B gathers 4 consecutive rows x 64 bytes (rows q and q+2 land in different halves of the row).
 __device__ __forceinline__ int gkey(int q) { return (((q >> 1) & 1) << 2) | ((q >> 2) & 3); }
-
-// A key tile by its workgroup from the definitions, in fp32 multiply-adds straight from memory (see not_finite in mlstm_device.h):
-// dK, dV and the column sums a key per wave, over the queries of the key's own chunk and the reverse state behind it, columns
-// lane and lane + 64; then the row partials a query per wave and a key per lane.
-template <int D>
-__device__ __forceinline__ void col_exact(const ColArgs& a, int bh, int jt, int chunk, int NGe, bool has_state, const float* Q, const float* dH, const float* K,
-                                          const float* V, size_t rsA, size_t rsB, size_t offA) {
-    constexpr int NC = D / 64;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, S = a.S, end = GRAN * NGe < S ? GRAN * NGe : S;
-    const size_t hoff = (size_t)bh * S, poff = (size_t)bh * a.NG * GRAN, goff = (size_t)bh * a.NG;
-    const double gj = a.G2[goff + jt];
-    const float log2scale = -0.5f * __log2f((float)D);
-    auto gate = [&](int t) { return log2scale - a.beta2[poff + t] + (float)(a.G2[goff + t / GRAN] - gj); };   // plus alpha2 of the key
-    for (int j = GRAN * jt + wave; j < GRAN * (jt + 1) && j < S; j += 4) {
-        const float al = a.alpha2[poff + j];
-        float k[NC], v[NC], dk[NC], dv[NC], col = 0.f;
-#pragma unroll
-        for (int n = 0; n < NC; n++) { k[n] = K[(size_t)j * rsA + lane + 64 * n]; v[n] = V[(size_t)j * rsA + lane + 64 * n]; dk[n] = dv[n] = 0.f; }
-        if (has_state) {   // (rows of the state: see row_exact)
-            const size_t st = (size_t)bh * a.n_states + chunk;
-            const float* E = reinterpret_cast<const float*>(a.Ev) + st * D * D;
-            const float* g = a.gvec + st * D;
-            auto at = [](int u) { return (size_t)((u & ~12) | ((u & 4) << 1) | ((u & 8) >> 1)) * D; };
-            for (int u = 0; u < D; u++) {
-                const float vu = V[(size_t)j * rsA + u], ku = K[(size_t)j * rsA + u];
-#pragma unroll
-                for (int n = 0; n < NC; n++) {
-                    dk[n] += vu * E[at(u) + lane + 64 * n];
-                    dv[n] += ku * E[at(lane + 64 * n) + u];
-                }
-            }
-            const int pe = (chunk + 1) * a.chunk_len - 1;
-            const float w = fast_exp2(al - a.beta2[poff + pe] + (float)(a.G2[goff + pe / GRAN] - gj));
-#pragma unroll
-            for (int n = 0; n < NC; n++) {
-                dk[n] = (dk[n] + g[lane + 64 * n]) * w;
-                dv[n] *= w;
-                col += dk[n] * k[n];
-            }
-            col = wave_reduce<OpAdd>(col);
-        }
-        for (int t = j; t < end; t++) {
-            float q[NC], u[NC], s = 0.f, dc = 0.f;
-#pragma unroll
-            for (int n = 0; n < NC; n++) {
-                q[n] = Q[(size_t)t * rsA + lane + 64 * n];
-                u[n] = dH[(size_t)t * rsB + lane + 64 * n];
-                s += q[n] * k[n];
-                dc += u[n] * v[n];
-            }
-            const float e = fast_exp2(al + gate(t)), inv = a.inv_n[poff + t];
-            const float ct = wave_reduce<OpAdd>(s) * e, dct = wave_reduce<OpAdd>(dc) * inv + a.db[poff + t];
-            col += ct * dct;
-#pragma unroll
-            for (int n = 0; n < NC; n++) {
-                dk[n] += dct * e * q[n];
-                dv[n] += ct * inv * u[n];
-            }
-        }
-#pragma unroll
-        for (int n = 0; n < NC; n++) {
-            const size_t at = offA + (size_t)j * rsA + lane + 64 * n;
-            reinterpret_cast<float*>(a.dK)[at] = dk[n];
-            reinterpret_cast<float*>(a.dV)[at] = dv[n];
-        }
-        if (lane == 0) a.colsum[hoff + j] = col;
-    }
-    const int j = GRAN * jt + lane, jc = j < S ? j : S - 1;
-    for (int t = GRAN * jt + wave; t < end; t += 4) {
-        float s = 0.f, dc = 0.f;
-        for (int u = 0; u < D; u++) {
-            s += Q[(size_t)t * rsA + u] * K[(size_t)jc * rsA + u];
-            dc += dH[(size_t)t * rsB + u] * V[(size_t)jc * rsA + u];
-        }
-        const float ct = s * fast_exp2(a.alpha2[poff + j] + gate(t)), dd = ct * (dc * a.inv_n[poff + t] + a.db[poff + t]);
-        const float sum = wave_reduce<OpAdd>(j <= t ? dd : 0.f);
-        if (lane == 0) a.rowpart[((size_t)bh * a.RS + (a.RS == a.NG ? jt : jt % a.RS)) * S + t] = sum;
-    }
-}
 
 // STRICT (16-bit types): split mode, see ColArgs::precise.
 template <typename T, int D, bool STRICT>
@@ -385,7 +307,7 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
                         const float dkv = (dkacc[kb][x][4 * a4 + c] + g4v[c]) * wk[kb];
                         dkacc[kb][x][4 * a4 + c] = dkv;
                         dvacc[kb][x][4 * a4 + c] *= wk[kb];
-                        cp += dkv * kv[c];
+                        cp = fmaf(dkv, kv[c], cp);
                     }
                 }
             cp = sum_halves(cp);
@@ -498,17 +420,18 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
             const float inv_er = inv * er, dbv_er = dbv * er;
 #pragma unroll
             for (int r = 0; r < 16; r++) {
+#pragma clang fp contract(off)   // (dD is rounded before it is added anywhere: mlstm_colf.hip hands it from wave to wave)
                 float dd;
                 if constexpr (FIRST) {
                     float e = fast_exp2(F32 ? (al[r] + nbeta) + (float)crow : al[r] + (float)crow);
                     if (!qvalid || (diag && (8 * (r >> 2) + 4 * h + (r & 3) > c32))) e = 0.f;
                     const float ct = sacc[r] * e;
-                    const float dct = dacc[r] * inv + dbv;
+                    const float dct = fmaf(dacc[r], inv, dbv);
                     dd = ct * dct;
                     g[r] = dct * e;
                     w[r] = ct * inv;
                 } else {
-                    const float dct_er = dacc[r] * inv_er + dbv_er;
+                    const float dct_er = fmaf(dacc[r], inv_er, dbv_er);
                     const float sk = sacc[r] * ekr[r];
                     g[r] = dct_er * ekr[r];
                     w[r] = sk * inv_er;
@@ -665,7 +588,8 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
         if (lane == 0) rowtmp[wave] = any ? 1.f : 0.f;
         __syncthreads();
         if (rowtmp[0] + rowtmp[1] + rowtmp[2] + rowtmp[3] > 0.f) {
-            col_exact<D>(a, bh, jt, chunk, NGe, has_state, Q, dH, K, V, rsA, rsB, offA);
+            col_exact<D, GRAN>(a, bh, GRAN * jt, chunk, NGe, has_state, Q, dH, K, V, rsA, rsB, offA,
+                               a.rowpart + ((size_t)bh * a.RS + (a.RS == NG ? jt : jt % a.RS)) * S);
             return;
         }
     }
@@ -757,7 +681,17 @@ static int launch_col_d(int D, const ColArgs& a, hipStream_t st) {
     return MLSTM_ESHAPE;
 }
 
+// col_kernel / colf_kernel, fp32, workgroups of 32 keys, us: D = 64, chunks of 128   128: 23.9 / 16.7   256: 25.6 / 18.1   320: 26.1 / 30.0
+//   uncut (300 positions)   240: 34.5 / 26.7   480: 36.8 / 38.1     D = 128, chunks of 128   256: 46.5 / 25.7   512: 50.0 / 45.3
+//   2048: 198 / 170   8192: 748 / 655   uncut   480: 60 / 50   1000: 101 / 105
+bool colf_serves(int dtype, int D, const ColArgs& a) {
+    if (dtype != MLSTM_F32 || D > 128 || a.RS > D || (a.chunk_len > 0 ? a.chunk_len > 1024 : a.S > 2048)) return false;
+    const long long wgs = 2ll * a.BH * a.NG;
+    return D == 64 ? wgs <= 256 : (wgs <= 512 || a.chunk_len == 128);
+}
+
 int launch_col_kernel(int dtype, int D, const ColArgs& a, hipStream_t st) {
+    if (a.rowpart2) return launch_colf_kernel(D, a, st);
     switch (dtype) {
         case MLSTM_F32: return launch_col_d<float>(D, a, st);
         case MLSTM_F16: return launch_col_d<_Float16>(D, a, st);

@@ -739,6 +739,18 @@ __device__ __forceinline__ float sum_halves(float v) {
     return __builtin_bit_cast(float, (int)r[0]) + __builtin_bit_cast(float, (int)r[1]);
 }
 
+// Sum over the 32 lanes of a wave's half, pairs of neighbours first, in every lane (the tree of five __shfl_xor steps, which take an
+// LDS round trip each).
+__device__ __forceinline__ float sum_half_wave(float v) {
+    v += dpp_f<0xB1>(0.f, v);    // quad_perm 1 0 3 2
+    v += dpp_f<0x4E>(0.f, v);    // quad_perm 2 3 0 1
+    v += dpp_f<0x141>(0.f, v);   // row_half_mirror: the other quad of eight
+    v += dpp_f<0x140>(0.f, v);   // row_mirror: the other eight of sixteen
+    const int x = __builtin_bit_cast(int, v);
+    const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);   // the other row of sixteen
+    return __builtin_bit_cast(float, (int)r[0]) + __builtin_bit_cast(float, (int)r[1]);
+}
+
 template <typename T> __device__ __forceinline__ float to_f32(T x) { return (float)x; }
 
 // Per-row scalars of the backward, computed by the lanes that already hold the row's dh fragments (xf):

@@ -152,6 +152,7 @@ struct ColArgs {
     float* rowpart;   // [BH,RS,S] fp32 partial row sums of dD, one slice per key tile (RS = NG), or, in chunks, per key
                       // tile of the position's own chunk (RS = chunk_len / 64: slice = key tile modulo RS)
     int RS;
+    float* rowpart2 = nullptr;   // may be null: a second array of partials, for the kernel that keeps a tile's halves apart (colf_serves)
     const float* alpha2; const float* beta2; const double* G2;
     const float* inv_n; const float* db;
     int BH, S, NG;
@@ -167,6 +168,9 @@ struct ColArgs {
     Lay la, lb;              // layouts of Q, K, V, dK, dV (la) and of dH (lb)
 };
 int launch_col_kernel(int dtype, int D, const ColArgs& a, hipStream_t st);
+// fp32 on 32 keys per workgroup, the same bits, for launches that leave the chip part empty; D in {64, 128}.  The row partials of a
+// tile's first and second 32 keys go to rowpart and rowpart2 (launch_df adds them): launch_col_kernel takes it where rowpart2 is given
+bool colf_serves(int dtype, int D, const ColArgs& a);
 int launch_colf_kernel(int D, const ColArgs& a, hipStream_t st);
 // phase A as 16x16x32 products on two query halves, the element-wise part of the first between the MFMAs of the second;
 // 16-bit types at D = 128 and 256 only
@@ -192,6 +196,7 @@ struct DfArgs {
     void* dF; void* dI;
     int BH, S, NG;
     int RS;                  // row-partial slices per head (see ColArgs)
+    const float* rowpart2;   // may be null: the partials of the tiles' second halves (see ColArgs)
     // in chunks: rowpart holds the slices of the key tiles of the position's own chunk only, rowinter the rest
     int chunk_len;
     const float* rowinter;
