@@ -75,6 +75,11 @@ int main() {
     check_tile<__bf16, 256, 32, 256>("32-row tile");
     check_tile<__bf16, 128, 128, 256>("128-row tile");
     check_tile<__bf16, 256, 128, 256>("128-row tile");
+    // the same by eight waves (roww_kernel's tiles, colw_kernel's key tiles and state pieces)
+    check_tile<__bf16, 128, 64, 512>("64-row tile, eight waves");
+    check_tile<__bf16, 256, 64, 512>("64-row tile, eight waves");
+    check_tile<__bf16, 128, 32, 512>("32-row tile, eight waves");
+    check_tile<__bf16, 256, 32, 512>("32-row tile, eight waves");
     // half rows of the dQ pass: the pieces its row sums load, D = 128 and 256, 16-bit
     check_pieces<128>();
     check_pieces<256>();

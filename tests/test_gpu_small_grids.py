@@ -49,3 +49,24 @@ def test_a_head_alone_is_the_head_of_a_full_chip(op, S, D, heads, layout, dtype)
     ("plain", 320, 64, 52, "bnsd"), ("gated", 450, 64, 33, "bsnd"), ("plain", 700, 128, 24, "bnsd"), ("plain", 1000, 64, 17, "bnsd")])
 def test_a_head_alone_is_the_head_of_a_full_chip_fp32(op, S, D, heads, layout):
     test_a_head_alone_is_the_head_of_a_full_chip(op, S, D, heads, layout, torch.float32)
+
+
+# colw_kernel (few workgroups) against cold_kernel (selected by hand): lengths at the edges of its 32-query tiles, of the pipeline's first and
+# last steps, of the 64-key tiles and of the chunks; 1024 queries are the most that a key may meet without chunks
+@pytest.mark.parametrize("op,S,D,heads,layout", [
+    ("plain", 1, 128, 2, "bnsd"), ("plain", 32, 256, 1, "bnsd"), ("plain", 33, 128, 1, "bsnd"), ("plain", 63, 256, 3, "bsnd"), ("gated", 65, 128, 1, "bnsd"),
+    ("precise", 95, 256, 2, "bnsd"), ("precise", 97, 128, 8, "bsnd"), ("plain", 129, 256, 2, "bnsd"), ("precise", 161, 256, 1, "bnsd"),
+    ("plain", 1000, 256, 1, "bnsd"), ("precise", 1001, 128, 1, "bnsd"), ("plain", 1025, 256, 3, "bnsd"), ("precise", 1057, 256, 2, "bsnd"),
+    ("plain", 1089, 128, 8, "bnsd"), ("precise", 1500, 128, 2, "bnsd"), ("gated", 2047, 256, 2, "bnsd"), ("plain", 2600, 128, 1, "bnsd")])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_few_key_tiles_give_the_bits_of_many(op, S, D, heads, layout, dtype):
+    rows, gates = _inputs(heads, S, D, dtype, layout)
+    ours = _step(op, rows, gates, heads)
+    ffi = submodule("_ffi")
+    ffi.set_column_kernel(2)
+    try:
+        theirs = _step(op, rows, gates, heads)
+    finally:
+        ffi.set_column_kernel(0)
+    for name, a, b in zip(range(10), ours, theirs):
+        assert bool(torch.isfinite(a.float()).all()) and torch.equal(a, b), name

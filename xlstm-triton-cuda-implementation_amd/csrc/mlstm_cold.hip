@@ -13,7 +13,7 @@
 //              and dV outright (256 accumulator registers at D = 256), nothing is exchanged between waves.
 // A lane holds one key and 16 queries of a block, so the key's scalars are one register each and the column sums of dD one
 // accumulating register; the queries' scalars (beta, 1/n, db) come from LDS four at a time, and the row sums of dD are
-// reduced across the lanes (v_permlane16_swap folds register pairs, DPP row shifts add up 16 lanes) between the MFMAs of
+// reduced across the lanes (row_sums8) between the MFMAs of
 // phase B.  A query tile is 32 rows so that two stages of Q and dH (64 KB at D = 256) and the V tile (64 KB) fit the LDS.
 // In chunks (ColArgs::chunk_len) a state phase precedes the query loop:  dK_j = w_j (E v_j + g),  dV_j = w_j E^T k_j  with the
 // chunk's reverse state E, which streams through the (then idle) query stages.
@@ -33,23 +33,9 @@ struct ColdCfg {
     static constexpr size_t QT_BYTES = (size_t)CD_QT * D * sizeof(T);                  // a 32-row tile of Q or dH
     static constexpr size_t STAGES_BYTES = 4 * QT_BYTES;                               // two stages of (Q, dH); the state tiles before them
     static constexpr size_t ROW_BYTES = 2 * 3 * GRAN * sizeof(float);                  // per stage: beta, 1/n, db (64 floats copied, 32 used)
-    static constexpr size_t MISC_BYTES = (2 * 4 * CD_QT + 64 + D) * sizeof(float);     // row sums [2 parities][4 key blocks][32], 64 sink words, the vector state
+    static constexpr size_t MISC_BYTES = (2 * 4 * CD_QT + D) * sizeof(float);     // row sums [2 parities][4 key blocks][32], the vector state
     static constexpr size_t LDS_BYTES = V_BYTES + STAGES_BYTES + ROW_BYTES + MISC_BYTES;   // plus one float per 64-position granule
 };
-
-// v_permlane16_swap exchanges the odd 16-lane rows of its first operand with the even rows of its second: one swap and one
-// add fold a pair of registers (a, b) into one that holds a(l) + a(l ^ 16) in the even rows and b(l) + b(l ^ 16) in the odd ones.
-__device__ __forceinline__ float fold_pair(float a, float b) {
-    auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(int, a), __builtin_bit_cast(int, b), false, false);
-    return __builtin_bit_cast(float, (int)r[0]) + __builtin_bit_cast(float, (int)r[1]);
-}
-__device__ __forceinline__ float row_total(float v) {   // lane 15 of each 16-lane row: the row's sum
-    v += dpp_f<0x111>(0.f, v);
-    v += dpp_f<0x112>(0.f, v);
-    v += dpp_f<0x114>(0.f, v);
-    v += dpp_f<0x118>(0.f, v);
-    return v;
-}
 
 // 32x32x16 MFMA whose accumulator is held in ordinary vector registers, for D = 256.  With a budget of 512 registers per
 // lane the compiler gives every MFMA it emits an accumulator in the second half of the register file (AGPRs), which this
@@ -112,7 +98,7 @@ __global__ __launch_bounds__(256, 1) void cold_kernel(ColArgs a) {
 #define ST_DH(st) (reinterpret_cast<T*>(stg + (size_t)(2 * (st) + 1) * Cfg::QT_BYTES))
 #define ST_ROW(st) (reinterpret_cast<float*>(tail) + (st) * 3 * GRAN)
     float* const rowtmp = reinterpret_cast<float*>(tail + Cfg::ROW_BYTES);   // [2][4][32]
-    float* const gvl = rowtmp + 2 * 4 * CD_QT + 64;   // (behind the sink words) the chunk's vector state g
+    float* const gvl = rowtmp + 2 * 4 * CD_QT;   // the chunk's vector state g
     float* const sG = gvl + D;                         // granule bases minus that of the tile's first granule
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = lane >> 5, c32 = lane & 31;
@@ -306,9 +292,10 @@ __global__ __launch_bounds__(256, 1) void cold_kernel(ColArgs a) {
         // k_j . (E v_j + g) w_j, the column sums of dD over the queries behind the chunk (and, for fp16, the scaling itself).
         // The K values a lane needs (its accumulators' rows 8 a4 + 4 h + c of every block) are in the K fragments of the two
         // lanes of its key (which hold columns 16 s + 8 h + 0..7): one v_permlane32_swap per register pair sorts them out.
-        float cp = 0.f;
+        float cp = 0.f, cpx = 0.f;   // (per block of 32 columns, then over the blocks)
 #pragma unroll
         for (int s = 0; s < NS; s++) {
+            if (s % 2 == 0) cpx = 0.f;
             const int x = s >> 1, a4a = 2 * (s & 1);
             const i32x4 w = __builtin_bit_cast(i32x4, kf[s]);
             const auto r0 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
@@ -326,30 +313,31 @@ __global__ __launch_bounds__(256, 1) void cold_kernel(ColArgs a) {
                 for (int c = 0; c < 4; c++) {
                     const float kval = u ? kc[c] : ka[c];
                     if constexpr (END_SCALE) {
-                        cp += (dkacc[x][4 * a4 + c] + g4v[c]) * kval;
+                        cpx = fmaf(dkacc[x][4 * a4 + c] + g4v[c], kval, cpx);
                     } else {
                         const float dkv = (dkacc[x][4 * a4 + c] + g4v[c]) * wk;
                         dkacc[x][4 * a4 + c] = dkv;
                         dvacc[x][4 * a4 + c] *= wk;
-                        cp += dkv * kval;
+                        cpx = fmaf(dkv, kval, cpx);
                     }
                 }
             }
+            if (s % 2 == 1) cp += cpx;
             if (s % 2 == 1) __builtin_amdgcn_sched_barrier(0);   // (one block of the accumulators at a time through the vector registers)
         }
-        colacc = END_SCALE ? cp * wk : cp;   // (starts the lane's column accumulator: the two halves of the wave meet in the epilogue)
+        colacc = END_SCALE ? rounded_product(cp, wk) : cp;   // (starts the lane's column accumulator: the two halves of the wave meet in the epilogue)
         CP_STAMP(2);
     }
     const float log2scale = -0.5f * __log2f((float)D);
 
-    // row sums go to the slice of the 64-key tile of the workgroup's first keys (the dF pass adds up one slice per 64 keys),
-    // zeros to the slice of its second half wherever that pass reads it
+    // row sums: one slice per 64 keys (the dF pass adds them up), that of the second half where that pass reads it
     const int j64 = 2 * jt;
     float* const rowpart_slice = a.rowpart + ((size_t)bh * a.RS + (a.RS == NG ? j64 : j64 % a.RS)) * S;
     // One step = one 32-query tile.  A lane computes E = exp2(alpha_key + crow_query) per element (a lane holds one key and
     // 16 queries: the factorised form of the other kernels would need one exponential per query and lane as well) and
     // masks it where the key lies behind the query, so diagonal tiles need no code of their own.
     constexpr int PW = TileDma<T, D, CD_QT, 256>::PER_WAVE;
+    const int rt_own = (lane & 4) * 2 + 4 * h + ((lane >> 2) & 2) + ((lane >> 4) & 1);   // the query whose row sum row_sums8 leaves in this lane
     auto step = [&](auto spread_tag, int it) {
         constexpr bool SPREAD = decltype(spread_tag)::value;  // copy of tile it+1 interleaved with this step's MFMAs
         const int qi0 = CD_QT * it;
@@ -367,8 +355,8 @@ __global__ __launch_bounds__(256, 1) void cold_kernel(ColArgs a) {
         if (it > it0 && tid < CD_QT && qi0 - CD_QT + tid < S) {
             const float* rt = rowtmp + ((it - 1) & 1) * 4 * CD_QT;
             float* rp = rowpart_slice + qi0 - CD_QT + tid;
-            rp[0] = (rt[tid] + rt[CD_QT + tid]) + (rt[2 * CD_QT + tid] + rt[3 * CD_QT + tid]);
-            if (j64 + 1 < NG && (qi0 - CD_QT) / GRAN >= j64 + 1) rp[S] = 0.f;
+            rp[0] = rt[tid] + rt[CD_QT + tid];
+            if (j64 + 1 < NG && (qi0 - CD_QT) / GRAN >= j64 + 1) rp[S] = rt[2 * CD_QT + tid] + rt[3 * CD_QT + tid];
         }
         const T* gq = Q + (size_t)CD_QT * (it + 1) * rsA;
         const T* gdh = dH + (size_t)CD_QT * (it + 1) * rsB;
@@ -420,7 +408,7 @@ __global__ __launch_bounds__(256, 1) void cold_kernel(ColArgs a) {
             const float argbase = al + (sG[it >> 1] + gcorr + log2scale) - log2_s;   // (weights over s_j: see END_SCALE)
             const unsigned span = (unsigned)(S - key);    // query q takes part iff 0 <= q - key < S - key (unsigned compare)
             const int dq0 = qi0 + 4 * h - key;            // q - key of register r: dq0 + 8 (r / 4) + r % 4
-            float dd[16];
+            float dd[16], csum0 = 0.f, csum1 = 0.f;   // (column sums: per half of a block, then over the blocks, the order of mlstm_colw.hip)
             f32x4 beta4[2], inv4[2], db4[2];   // the scalars of the half's eight queries (two groups of four registers)
             auto ew_scalars = [&](int t) {
 #pragma unroll
@@ -436,28 +424,17 @@ __global__ __launch_bounds__(256, 1) void cold_kernel(ColArgs a) {
                 const bool live = (unsigned)(dq0 + 8 * (r >> 2) + c) < span;
                 const float e = fast_exp2(live ? argbase - beta4[u][c] : -INFINITY);
                 const float ct = wacc[r] * e;
-                const float dct = gacc[r] * inv4[u][c] + db4[u][c];
-                dd[r] = END_SCALE ? (ct * scale_s) * dct : ct * dct;
-                gacc[r] = dct * e;
-                wacc[r] = ct * inv4[u][c];
-                colacc += dd[r];
-            };
-            // lane 15 of a 16-lane row holds the row's total: rows 0 / 2 (h = 0 / 1) carry register 2p, rows 1 / 3 register
-            // 2p + 1 of the folded pair; the other lanes write to a word of their own that nobody reads
-            float* const sink = rowtmp + 2 * 4 * CD_QT + lane;
-            auto row_sum_out = [&](int p, float folded) {
-                const float tot = row_total(folded);
-                const int r = 2 * p + ((lane >> 4) & 1);
-                float* dst = (lane & 15) == 15 ? rt + (8 * (r >> 2) + 4 * h + (r & 3)) : sink;
-                *dst = tot;
+                const float dct = fmaf(gacc[r], inv4[u][c], db4[u][c]);
+                dd[r] = rounded_product(END_SCALE ? ct * scale_s : ct, dct);
+                gacc[r] = STRICT ? rounded_product(dct, e) : dct * e;   // (their low-order terms are what these values lose)
+                wacc[r] = STRICT ? rounded_product(ct, inv4[u][c]) : ct * inv4[u][c];
+                if (r < 8) csum0 += dd[r];
+                else csum1 += dd[r];
             };
             ew_scalars(0);
 #pragma unroll
             for (int r = 0; r < 8; r++) ew_one(r);
             ew_scalars(1);   // (for the second half, whose work rides on phase B below)
-            float rs[8];
-#pragma unroll
-            for (int p = 0; p < 4; p++) rs[p] = fold_pair(dd[2 * p], dd[2 * p + 1]);
             CP_STAMP(5);
 #pragma unroll
             for (int t = 0; t < 2; t++) {
@@ -483,20 +460,15 @@ __global__ __launch_bounds__(256, 1) void cold_kernel(ColArgs a) {
                         R::mma(dkacc[x], qa[x & 1], glo);
                         R::mma(dvacc[x], ha[x & 1], wlo);
                     }
-                    // behind the MFMAs: 8 / NXD registers of the second half's element-wise work (t = 0 only) and 4 / NXD
-                    // folded row sums of this half
+                    // behind the MFMAs: 8 / NXD registers of the second half's element-wise work (t = 0 only) and this half's row sums
                     if (t == 0) {
 #pragma unroll
                         for (int u = 0; u < 8 / NXD; u++) ew_one(8 + x * (8 / NXD) + u);
                     }
-                    if constexpr (NXD == 8) { if (x % 2 == 1) row_sum_out(4 * t + x / 2, rs[4 * t + x / 2]); }
-                    else row_sum_out(4 * t + x, rs[4 * t + x]);
+                    if (x == 1 - t) rt[rt_own + 16 * t] = row_sums8(dd + 8 * t, lane & 8, lane & 4);
                     __builtin_amdgcn_sched_barrier(0);
                 }
-                if (t == 0) {
-#pragma unroll
-                    for (int p = 4; p < 8; p++) rs[p] = fold_pair(dd[2 * p], dd[2 * p + 1]);
-                }
+                if (t == 0) colacc += csum0 + csum1;
             }
             CP_STAMP(6);
         } else {
@@ -521,8 +493,8 @@ __global__ __launch_bounds__(256, 1) void cold_kernel(ColArgs a) {
         if (tid < CD_QT && CD_QT * last + tid < S) {
             const float* rt = rowtmp + (last & 1) * 4 * CD_QT;
             float* rp = rowpart_slice + CD_QT * last + tid;
-            rp[0] = (rt[tid] + rt[CD_QT + tid]) + (rt[2 * CD_QT + tid] + rt[3 * CD_QT + tid]);
-            if (j64 + 1 < NG && (CD_QT * last) / GRAN >= j64 + 1) rp[S] = 0.f;
+            rp[0] = rt[tid] + rt[CD_QT + tid];
+            if (j64 + 1 < NG && (CD_QT * last) / GRAN >= j64 + 1) rp[S] = rt[2 * CD_QT + tid] + rt[3 * CD_QT + tid];
         }
     }
     {
@@ -542,7 +514,11 @@ __global__ __launch_bounds__(256, 1) void cold_kernel(ColArgs a) {
                     for (int c = 0; c < 4; c++) v[c] = which ? dvacc[x][4 * a4 + c] : dkacc[x][4 * a4 + c];
                     if constexpr (END_SCALE) {   // the keys' weights: see the state phase
                         v *= scale_s;
-                        if (!which && has_state) v += *reinterpret_cast<const f32x4*>(gvl + d) * wkg;
+                        if (!which && has_state) {
+                            const f32x4 g4 = *reinterpret_cast<const f32x4*>(gvl + d);
+#pragma unroll
+                            for (int c = 0; c < 4; c++) v[c] = fmaf(g4[c], wkg, v[c]);
+                        }
                     }
                     const int chunk16 = (d * (int)sizeof(T)) >> 4, within = (d * (int)sizeof(T)) & 15;
                     *reinterpret_cast<typename R::vec4*>(out + row * ROWB + (((chunk16 ^ (row & 31)) & (CPR - 1)) << 4) + within) = R::cvt4(v);

@@ -681,6 +681,35 @@ __device__ __forceinline__ float dpp_f(float old, float src) {
                                                                  CTRL, ROW_MASK, BANK_MASK, BOUND));
 }
 
+// A product that is rounded before it is added up, for kernels that must give the same bits: left to itself the compiler contracts it
+// with one sum in one of them and with another in the other.
+__device__ __forceinline__ float rounded_product(float a, float b) {
+#pragma clang fp contract(off)
+    float p = a * b;
+    asm("" : "+v"(p));
+    return p;
+}
+// v_permlane16_swap exchanges the odd 16-lane rows of its first operand with the even rows of its second: one swap and one
+// add fold a pair of registers (a, b) into one that holds a(l) + a(l ^ 16) in the even rows and b(l) + b(l ^ 16) in the odd ones.
+__device__ __forceinline__ float fold_pair(float a, float b) {
+    auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(int, a), __builtin_bit_cast(int, b), false, false);
+    return __builtin_bit_cast(float, (int)r[0]) + __builtin_bit_cast(float, (int)r[1]);
+}
+// Sums of eight registers over the 32 lanes of either half of a wave: registers and lanes are folded together, 16, 8 and 4 lanes
+// apart, then the four lanes of a quad add up.  Lane l returns the sum of register k = 4 (l / 4 % 2) + 2 (l / 8 % 2) + l / 16 % 2 of
+// its half; hi8, hi4: l & 8, l & 4.  (Eight chains of one swap, an add and four row shifts take 2.5 times the instructions, and each waits for
+// its own.)
+__device__ __forceinline__ float row_sums8(const float* x, bool hi8, bool hi4) {
+    float f[4], g[2];
+#pragma unroll
+    for (int p = 0; p < 4; p++) f[p] = fold_pair(x[2 * p], x[2 * p + 1]);
+#pragma unroll
+    for (int p = 0; p < 2; p++) g[p] = (hi8 ? f[2 * p + 1] : f[2 * p]) + dpp_f<0x128>(0.f, hi8 ? f[2 * p] : f[2 * p + 1]);   // row_ror:8
+    float s = (hi4 ? g[1] : g[0]) + dpp_f<0x141>(0.f, hi4 ? g[0] : g[1]);   // row_half_mirror: lane 7 - l of eight
+    s += dpp_f<0x4e>(0.f, s);   // quad_perm: two lanes away, then one
+    s += dpp_f<0xb1>(0.f, s);
+    return s;
+}
 struct OpAdd { static __device__ __forceinline__ float id() { return 0.0f; } static __device__ __forceinline__ float f(float a, float b) { return a + b; } };
 struct OpMax { static __device__ __forceinline__ float id() { return -INFINITY; } static __device__ __forceinline__ float f(float a, float b) { return fmaxf(a, b); } };
 

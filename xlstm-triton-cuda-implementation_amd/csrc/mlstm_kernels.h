@@ -177,12 +177,26 @@ int launch_colf_kernel(int D, const ColArgs& a, hipStream_t st);
 int launch_col16_kernel(int dtype, int D, const ColArgs& a, hipStream_t st);
 // weights kept in registers between the two phases (no G / W tiles in LDS); 16-bit types at D = 128 and 256, split mode included
 int launch_cold_kernel(int dtype, int D, const ColArgs& a, hipStream_t st);
+// the same on 64 keys per workgroup and eight waves, the same bits, for launches of few workgroups; keys that meet up to 1024 queries
+int launch_colw_kernel(int dtype, int D, const ColArgs& a, hipStream_t st);
 extern int g_col_variant;   // see mlstm_set_column_kernel: 0 = the library's choice, 1 = col16_kernel, 2 = cold_kernel, 3 = col_kernel
 inline int launch_col_best(int dtype, int D, const ColArgs& a, hipStream_t st) {
     const bool half_big = dtype != MLSTM_F32 && (D == 128 || D == 256);
     int variant = g_force_generic ? 3 : g_col_variant;
     if (!half_big || variant < 0 || variant > 3) variant = 3;
-    if (variant == 0) variant = 2;   // (measured faster than col16_kernel at D = 128 and 256, chunked and not)
+    if (variant == 0) {
+        // Workgroups of 64 keys up to which colw_kernel is the faster one; cold_kernel / colw_kernel, us (bf16, workgroups of 64 keys):
+        //   D = 128, S = 1000 (not in chunks)   64: 50 / 27   256: 52 / 30   512: 54 / 39   768: 82 / 58
+        //   D = 128 in chunks of 512            64: 32 / 20   256: 35 / 23   512: 37 / 34   768: 51 / 48   1024: 52 / 59
+        //   D = 256, S = 1000                   64: 69 / 40   256: 72 / 45   512: 76 / 57
+        //   D = 256 in chunks                  128: 51 / 33   256: 53 / 36   512: 56 / 54   768: 82 / 82
+        //   D = 256 in split mode              128: 65 / 42   256: 67 / 47   512: 72 / 70   768: 108 / 103
+        if ((long long)a.BH * a.NG <= 768) {
+            const int rc = launch_colw_kernel(dtype, D, a, st);
+            if (rc != MLSTM_ESHAPE) return rc;
+        }
+        variant = 2;   // (measured faster than col16_kernel at D = 128 and 256, chunked and not)
+    }
     if (variant == 1 && a.precise) variant = 2;   // (col16_kernel has no split mode)
     if (variant == 1 || variant == 2) {
         int rc = variant == 1 ? launch_col16_kernel(dtype, D, a, st) : launch_cold_kernel(dtype, D, a, st);
