@@ -70,3 +70,23 @@ def test_few_key_tiles_give_the_bits_of_many(op, S, D, heads, layout, dtype):
         ffi.set_column_kernel(0)
     for name, a, b in zip(range(10), ours, theirs):
         assert bool(torch.isfinite(a.float()).all()) and torch.equal(a, b), name
+
+
+# split mode: rowx_kernel against row_kernel (force_generic_kernels), edges of the 64-key tiles, the 32-row blocks, the walk's first steps and the
+# chunks' state
+@pytest.mark.parametrize("S,D,heads,layout", [
+    (1, 128, 1, "bnsd"), (32, 256, 2, "bnsd"), (33, 128, 8, "bsnd"), (64, 256, 1, "bnsd"), (65, 128, 2, "bnsd"), (127, 256, 3, "bsnd"), (130, 256, 1, "bnsd"),
+    (200, 128, 1, "bnsd"), (257, 128, 2, "bnsd"), (1000, 256, 2, "bnsd"), (1023, 128, 3, "bsnd"), (1025, 256, 1, "bnsd"), (1089, 128, 2, "bnsd"),
+    (1100, 256, 8, "bsnd"), (1665, 256, 2, "bnsd"), (2048, 128, 1, "bnsd")])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_split_mode_few_row_tiles_give_the_bits_of_many(S, D, heads, layout, dtype):
+    rows, gates = _inputs(heads, S, D, dtype, layout)
+    ours = _step("precise", rows, gates, heads)
+    ffi = submodule("_ffi")
+    ffi.force_generic_kernels(True)
+    try:
+        theirs = _step("precise", rows, gates, heads)
+    finally:
+        ffi.force_generic_kernels(False)
+    for name, a, b in zip(range(4), ours, theirs):   # h, m, b, dq
+        assert bool(torch.isfinite(a.float()).all()) and torch.equal(a, b), name

@@ -130,16 +130,22 @@ int launch_rowf_kernel(int mode, int D, const RowArgs& a, hipStream_t st);
 int launch_row8_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t st);
 // the same bits on 64 rows per workgroup, for launches that leave the chip part empty; 16-bit types and D in {128, 256} only
 int launch_roww_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t st);
+// split mode on 64 rows per workgroup, the bits of the four-wave kernel, for the same launches; not with an output gate
+int launch_rowx_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t st);
 // (the four-wave kernel serves every other case: fp32, D = 64, split mode -- in chunks too -- and the test switch)
 inline int launch_row_best(int mode, int dtype, int D, const RowArgs& a, hipStream_t st) {
-    if (dtype != MLSTM_F32 && (D == 128 || D == 256) && !g_force_generic && !a.precise) {
+    if (dtype != MLSTM_F32 && (D == 128 || D == 256) && !g_force_generic) {
         // While its workgroups (64 rows) number no more than the chip's CUs, roww_kernel: row8_kernel / roww_kernel, forward, us --
         // D = 128   10: 13.3 / 11.2   80: 14.6 / 12.1   240 (uncut, 1001 positions): 21.3 / 19.0   256: 13.0 / 10.9   384: 13.8 / 14.0
         // D = 256   10: 17.2 / 13.4   224 (chunks of 512): 23.1 / 17.4   256: 15.4 / 13.0   384: 19.9 / 19.2   512: 25.9 / 27.2
         int rc = MLSTM_ESHAPE;
         // (a wait bound of the caller's asks for the kernel that has the wait: mlstm_set_spin_limit)
-        if ((long long)a.BH * a.NG <= 256 && a.spin_limit == DEFAULT_SPIN_LIMIT) rc = launch_roww_kernel(mode, dtype, D, a, st);
-        if (rc == MLSTM_ESHAPE) rc = launch_row8_kernel(mode, dtype, D, a, st);
+        if ((long long)a.BH * a.NG <= 256 && !a.precise && a.spin_limit == DEFAULT_SPIN_LIMIT) rc = launch_roww_kernel(mode, dtype, D, a, st);
+        // Split mode: row_kernel / rowx_kernel, forward and dQ pass, us --
+        // D = 128   64: 21.3, 23.2 / 13.5, 15.7   256: 23.4, 24.9 / 16.1, 18.4   384: 23.9, 26.5 / 22.6, 27.0   512: 24.8, 27.6 / 26.2, 29.8
+        // D = 256   64: 39.3, 43.8 / 22.6, 26.9   256: 41.8, 47.3 / 26.0, 30.2   384: 42.9, 47.6 / 36.9, 42.4   512: 44.1, 49.0 / 40.8, 46.8
+        if ((long long)a.BH * a.NG <= (D == 128 ? 256 : 512) && a.precise) rc = launch_rowx_kernel(mode, dtype, D, a, st);
+        if (rc == MLSTM_ESHAPE && !a.precise) rc = launch_row8_kernel(mode, dtype, D, a, st);
         if (rc != MLSTM_ESHAPE) return rc;  // extremely long sequences do not fit its LDS budget
     }
     return launch_row_kernel(mode, dtype, D, a, st);

@@ -133,6 +133,12 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
     float bsum = 0.f;
 
     constexpr bool FAST_TR = R::HALF && Swz<T, D>::CPR >= 16;  // precomputed offsets for the transposing reads
+    // Split mode at D >= 128 shares its order of operations with mlstm_rowx.hip, which spreads a row over waves: the row sums over the key
+    // blocks of either parity and over either half of the state's rows apart, the factorised weights wherever a block lies below the
+    // diagonal, and products that enter a low-order term or a sum rounded first (rounded_product).
+    constexpr bool SPLIT = STRICT && FAST_TR;
+    float bpar[2] = {0.f, 0.f}, bfar[2] = {0.f, 0.f}, dec_far = 0.f;
+    auto product = [](float x, float y) { return SPLIT ? rounded_product(x, y) : x * y; };
     SwzRowReader<T, D> krd;
     krd.init(lane);
     typename std::conditional<F32, SwzTransReaderF32<D>, SwzTransReader<typename std::conditional<FAST_TR, T, __bf16>::type, FAST_TR ? D : 256>>::type vrd;
@@ -223,14 +229,17 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
                 else e = fast_exp2(al[c] + crow);
                 if (diag && (8 * a4 + 4 * h + c > c32)) e = 0.f;
                 if constexpr (MODE == MODE_FWD) {
-                    sacc[r] *= e;
+                    sacc[r] = product(sacc[r], e);
                     blk += sacc[r];
+                } else if constexpr (SPLIT) {
+                    sacc[r] = product(fmaf(sacc[r], inv_n, dbv), e);
                 } else {
                     sacc[r] = (sacc[r] * inv_n + dbv) * e;
                 }
             }
         }
-        if constexpr (MODE == MODE_FWD) bsum += blk;
+        if constexpr (MODE == MODE_FWD && SPLIT) bpar[kb] += blk;
+        else if constexpr (MODE == MODE_FWD) bsum += blk;
     };
     // gate weights of a block entirely below the diagonal, factorised: exp2(alpha_j - c0) comes from the pre-pass
     // (sek), exp2(c0 - beta_i + dG) is one exponential per lane and block
@@ -246,15 +255,18 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
             for (int c = 0; c < 4; c++) {
                 const int r = 4 * a4 + c;
                 if constexpr (MODE == MODE_FWD) {
-                    const float t = sacc[r] * ek[c];
+                    const float t = product(sacc[r], ek[c]);
                     blk += t;
-                    sacc[r] = t * er;
+                    sacc[r] = product(t, er);
+                } else if constexpr (SPLIT) {
+                    sacc[r] = product(fmaf(sacc[r], inv_n * er, dbv * er), ek[c]);
                 } else {
                     sacc[r] = (sacc[r] * inv_n + dbv) * (ek[c] * er);
                 }
             }
         }
-        if constexpr (MODE == MODE_FWD) bsum = fmaf(blk, er, bsum);
+        if constexpr (MODE == MODE_FWD && SPLIT) bpar[kb] = fmaf(blk, er, bpar[kb]);
+        else if constexpr (MODE == MODE_FWD) bsum = fmaf(blk, er, bsum);
     };
     // second product: accumulate this key block into the output
     auto gemm2 = [&](const T* y2, const f32x16& sacc, int kb, auto&& hook) {
@@ -300,9 +312,11 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
         // one accumulator register of a block below the diagonal: see weigh_fact
         auto weigh_reg = [&](f32x16& sacc, int r, const f32x4 (&ek)[4], float er, float& blk) {
             if constexpr (MODE == MODE_FWD) {
-                const float t = sacc[r] * ek[r >> 2][r & 3];
+                const float t = product(sacc[r], ek[r >> 2][r & 3]);
                 blk += t;
-                sacc[r] = t * er;
+                sacc[r] = product(t, er);
+            } else if constexpr (SPLIT) {
+                sacc[r] = product(fmaf(sacc[r], inv_n * er, dbv * er), ek[r >> 2][r & 3]);
             } else {
                 sacc[r] = (sacc[r] * inv_n + dbv) * (ek[r >> 2][r & 3] * er);
             }
@@ -371,7 +385,8 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
             if (g == 1) take_p(s1, 0);
             if (g == 2) take_p(s1, 1);
         }
-        if constexpr (MODE == MODE_FWD) bsum = fmaf(blk1, er1, fmaf(blk0, er0, bsum));
+        if constexpr (MODE == MODE_FWD && SPLIT) { bpar[0] = fmaf(blk0, er0, bpar[0]); bpar[1] = fmaf(blk1, er1, bpar[1]); }
+        else if constexpr (MODE == MODE_FWD) bsum = fmaf(blk1, er1, fmaf(blk0, er0, bsum));
       }
     };
 
@@ -434,12 +449,24 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
         const float* nst = a.Nst + ((size_t)bh * a.n_states + chunk - 1) * D;
         if constexpr (MODE == MODE_FWD) {
             // row sums: decay_i (q_i . n~); the lane's half of the row (the halves meet in the epilogue)
-            float part = 0.f;
+            if constexpr (SPLIT) {
+                dec_far = dec;
 #pragma unroll
-            for (int s2 = 0; s2 < NS; s2++)
+                for (int s2 = 0; s2 < NS; s2++)
 #pragma unroll
-                for (int e = 0; e < R::EPL; e++) part = fmaf(to_f32(xf[s2][e]), nst[KW * s2 + R::EPL * h + e], part);
-            bsum = fmaf(dec, part, bsum);
+                    for (int e = 0; e < 4; e++) {
+                        float& part = bfar[s2 / (NS / 2)];
+                        const float* const n8 = nst + KW * s2 + R::EPL * h;
+                        part = fmaf(to_f32(xf[s2][4 + e]), n8[4 + e], fmaf(to_f32(xf[s2][e]), n8[e], part));
+                    }
+            } else {
+                float part = 0.f;
+#pragma unroll
+                for (int s2 = 0; s2 < NS; s2++)
+#pragma unroll
+                    for (int e = 0; e < R::EPL; e++) part = fmaf(to_f32(xf[s2][e]), nst[KW * s2 + R::EPL * h + e], part);
+                bsum = fmaf(dec, part, bsum);
+            }
 #pragma unroll
             for (int d = 0; d < NDB; d++)
 #pragma unroll
@@ -447,7 +474,7 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
         } else {
             const float decn = dec * inv_n, rank1 = dec * dbv;
             const T* qrow = reinterpret_cast<const T*>(a.Qrow) + offA + (size_t)rowc * rsA;
-            float rp = 0.f;   // (summed per block of 32 columns, as mlstm_rowf.hip, which splits a row by columns, has to)
+            float rp = 0.f, rp_first = 0.f;   // (summed per block of 32 columns, as mlstm_rowf.hip, which splits a row by columns, has to; split mode: and per half of them)
 #pragma unroll
             for (int d = 0; d < NDB; d++) {
                 float rpd = 0.f;
@@ -464,9 +491,11 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
                     }
                 }
                 rp += rpd;
+                if (SPLIT && d == NDB / 2 - 1) { rp_first = rp; rp = 0.f; }
             }
             // row sums of dD over the keys before the chunk: q_i . dQ_i of what the accumulators hold now
             rp = sum_halves(rp);
+            if constexpr (SPLIT) rp = sum_halves(rp_first) + rp;
             if (row < S && h == 0) a.rowinter[hoff + row] = rp;
         }
     } else {
@@ -558,7 +587,8 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
             if (kstart <= r0) {
                 f32x16 s0;
                 gemm1(y1, kb, s0);
-                weigh(s0, sal, kb, crow, kstart == r0);
+                if (SPLIT && kstart < r0) weigh_fact(s0, sal + GRAN, kb, crow);
+                else weigh(s0, sal, kb, crow, kstart == r0);
                 gemm2(y2, s0, kb, no_hook);
             }
         }
@@ -569,7 +599,12 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
 #undef ST_AL
     float onorm = 1.0f, brow = 0.f;
     if constexpr (MODE == MODE_FWD) {
-        brow = sum_halves(bsum);
+        if constexpr (SPLIT) {
+            if (chunk > 0) { bpar[0] = fmaf(bfar[0], dec_far, bpar[0]); bpar[1] = fmaf(bfar[1], dec_far, bpar[1]); }
+            brow = sum_halves(bpar[0]) + sum_halves(bpar[1]);
+        } else {
+            brow = sum_halves(bsum);
+        }
         const float m = a.M[hoff + rowc];
         const float n = fmaxf(fabsf(brow), __expf(-m)) + 1e-6f;
         onorm = 1.0f / n;
@@ -601,7 +636,7 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
             for (int a4 = 0; a4 < 4; a4++) {
                 f32x4 v;
 #pragma unroll
-                for (int c = 0; c < 4; c++) v[c] = oacc[d][4 * a4 + c] * onorm;
+                for (int c = 0; c < 4; c++) v[c] = product(oacc[d][4 * a4 + c], onorm);
                 if constexpr (STRICT && MODE == MODE_FWD) {
                     typename R::vec4 hi, lo;
                     R::cvt4_split(v, hi, lo);
