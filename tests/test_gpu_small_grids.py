@@ -90,3 +90,12 @@ def test_split_mode_few_row_tiles_give_the_bits_of_many(S, D, heads, layout, dty
         ffi.force_generic_kernels(False)
     for name, a, b in zip(range(4), ours, theirs):   # h, m, b, dq
         assert bool(torch.isfinite(a.float()).all()) and torch.equal(a, b), name
+
+
+# the carry in blocks of 32 x 32 against the one in blocks of 64 x 64 (more than 192, from 6 states on 384, from 12 on 512 of them), and groups of
+# four steps: 1 to 5 states, 6, 7, 12, 13 (D = 128 in chunks of 512), 16 and 17 (the edge of what is requested at once)
+@pytest.mark.parametrize("op,S,D,heads", [("plain", 1024, 128, 49), ("plain", 1537, 128, 49), ("precise", 2049, 256, 13), ("plain", 2561, 256, 13),
+                                          ("plain", 3073, 128, 97), ("precise", 3600, 256, 25), ("plain", 6145, 128, 129), ("plain", 6700, 256, 33),
+                                          ("plain", 8193, 128, 129), ("plain", 8705, 128, 129)])
+def test_either_carry_gives_a_head_the_same_bits(op, S, D, heads):
+    test_a_head_alone_is_the_head_of_a_full_chip(op, S, D, heads, "bnsd", torch.bfloat16)

@@ -19,8 +19,7 @@ def _check(B, NH, S, D, dtype, seed, chunk_len=0):
     assert_matches_oracle(dtype, q, k, v, f, i, dh=dh, h=out.detach(), grads=torch.autograd.grad(out, ts, dh.cuda()), chunk_len=chunk_len)
 
 
-# (16 bits: 1023 / 1024 are the last length that is not cut and the first in chunks; 128 and 132 workgroups of 64 x 64, 32 and 33
-# heads at D = 128, 8 and 9 at D = 256, are the edge of the two carries.)
+# (16 bits: 1023 / 1024 are the last length that is not cut and the first in chunks.  The edges of the two carries: test_gpu_small_grids.)
 # The last number is the chunk length the rule gives, which the noise prediction needs.
 @pytest.mark.parametrize("B,NH,S,D,L", [(1, 2, 959, 64, 0), (1, 2, 1023, 64, 0), (1, 2, 1024, 64, 256), (1, 1, 1536, 64, 256), (1, 2, 1023, 128, 0),
                                         (1, 1, 1023, 256, 0), (1, 9, 1025, 256, 512), (1, 33, 1024, 128, 512), (16, 2, 1100, 128, 512),

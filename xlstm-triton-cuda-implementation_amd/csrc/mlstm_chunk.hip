@@ -785,15 +785,19 @@ __device__ __forceinline__ float dot_group(f32x4 x, f32x4 y) {
 // sums at a time in registers (one trip to memory per sixteen steps, whatever the number of heads), writes either layout or
 // both -- the value-major one through LDS, in whole 64- or 128-byte pieces of a row -- and forms the contraction with another
 // set of states (ChunkArgs::dot_with) on the way.
+// Four steps share a barrier: their states go to LDS one after the other and come back turned round side by side.  With a barrier per
+// step it was a chain of LDS round trips and lane reductions: with the contraction 91 us -> 60 at 64 heads x 31 states x 128 x 128 (16 bits),
+// 10.1 -> 7.5 at 8 x 2 x 256 x 256 in split mode, 8.8 -> 6.7 at 8 x 7 x 128 x 128 (fp32).
 // (Before: 2 to 8 workgroups per head, four steps at a time, the value-major copy element by element, and a kernel of its own
 // for the contraction: 14.6 + 4.7 us at B1 H4 S2048 D64 fp32.)
-template <typename T, int D, bool DOT>
+// DOT: 0 no contraction, 1 with states of one term, 2 of two (their fragments cost registers, and registers workgroups per CU)
+template <typename T, int D, int DOT>
 __global__ __launch_bounds__(256) void chunk_carry_small_kernel(ChunkArgs a) {
-    constexpr int AHEAD = 16, MAXC = 1024;   // (S <= 131072 in chunks of at least 128)
+    constexpr int AHEAD = 16, GROUP = 4, MAXC = 1024;   // (S <= 131072 in chunks of at least 128)
     typedef typename Tr<T>::vec4 V4;
-    __shared__ __attribute__((aligned(16))) float tile[2][32][36];
+    __shared__ __attribute__((aligned(16))) float tile[2][GROUP][32][36];   // [parity of the group][step]
     __shared__ float gams[MAXC];
-    __shared__ float red[2][4];
+    __shared__ float red[2][GROUP][4];
     const int bh = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int kb = blockIdx.x / (D / 32), vb = blockIdx.x % (D / 32);
     const int row = tid >> 3, c4 = 4 * (tid & 7);   // row of the block (key; value in the turned one) and first of four columns
@@ -805,7 +809,7 @@ __global__ __launch_bounds__(256) void chunk_carry_small_kernel(ChunkArgs a) {
     const bool vec = blockIdx.x == 0 && tid < D;
     auto chunk_of = [&](int step) { return a.reverse ? a.NCS - 1 - step : step; };
     f32x4 d[AHEAD];
-    V4 y[DOT ? AHEAD : 1], yl[DOT ? AHEAD : 1];
+    V4 y[DOT ? AHEAD : 1], yl[DOT == 2 ? AHEAD : 1];
     float nin[AHEAD];
     auto request = [&](int step0) __attribute__((always_inline)) {
 #pragma unroll
@@ -813,9 +817,9 @@ __global__ __launch_bounds__(256) void chunk_carry_small_kernel(ChunkArgs a) {
             const int c = chunk_of(step0 + u < a.NCS ? step0 + u : a.NCS - 1);
             const size_t co = (size_t)c * D * D;
             d[u] = *reinterpret_cast<const f32x4*>(src + co);
-            if constexpr (DOT) {
+            if constexpr (DOT > 0) {
                 y[u] = *reinterpret_cast<const V4*>(reinterpret_cast<const T*>(a.dot_with) + voff + co);
-                if (a.dot_with_lo) yl[u] = *reinterpret_cast<const V4*>(reinterpret_cast<const T*>(a.dot_with_lo) + voff + co);
+                if constexpr (DOT == 2) yl[u] = *reinterpret_cast<const V4*>(reinterpret_cast<const T*>(a.dot_with_lo) + voff + co);
             }
             nin[u] = vec ? nst[(size_t)c * D] : 0.f;
         }
@@ -833,50 +837,65 @@ __global__ __launch_bounds__(256) void chunk_carry_small_kernel(ChunkArgs a) {
         if (hi_base) *reinterpret_cast<V4*>(reinterpret_cast<T*>(hi_base) + off) = hi;
         if (lo_base) *reinterpret_cast<V4*>(reinterpret_cast<T*>(lo_base) + off) = lo;
     };
-    auto put_dot = [&](int step) {   // (behind the barrier that follows the step's partial sums)
-        if (DOT && tid == 0)
-            a.dot_part[((size_t)bh * a.NCS + chunk_of(step)) * gridDim.x + blockIdx.x] =
-                (red[step & 1][0] + red[step & 1][1]) + (red[step & 1][2] + red[step & 1][3]);
+    auto put_dots = [&](int first) {   // of a group's steps, behind the barrier that follows their partial sums
+        if constexpr (DOT > 0) {
+            if (tid < GROUP && first + tid < a.NCS) {
+                const float* const r = red[(first / GROUP) & 1][tid];
+                a.dot_part[((size_t)bh * a.NCS + chunk_of(first + tid)) * gridDim.x + blockIdx.x] = (r[0] + r[1]) + (r[2] + r[3]);
+            }
+        }
     };
     for (int step0 = 0; step0 < a.NCS; step0 += AHEAD) {
         if (step0 > 0) request(step0);
 #pragma unroll
-        for (int u = 0; u < AHEAD; u++) {
-            const int step = step0 + u;
-            if (step < a.NCS) {
-            const size_t co = (size_t)chunk_of(step) * D * D;
-            const float gam = gams[step];
-            run = run * gam + d[u];
-#pragma unroll
-            for (int e = 0; e < 4; e++) asm volatile("" : "+v"(run[e]));   // (see chunk_carry_t_kernel)
+        for (int u0 = 0; u0 < AHEAD; u0 += GROUP) {
+            const int first = step0 + u0, par = (first / GROUP) & 1;
+            if (first < a.NCS) {
             V4 hi, lo;
-            if (a.Cst) put(a.Cst, a.Cst_lo, koff + co, run, hi, lo);
-            if (a.CstT) {   // (uniform) turned round in LDS
-                float (*t)[36] = tile[step & 1];
 #pragma unroll
-                for (int e = 0; e < 4; e++) t[c4 + e][row] = run[e];
-                __syncthreads();
-                if (step > 0) put_dot(step - 1);
-                const f32x4 x = *reinterpret_cast<const f32x4*>(&t[row][c4]);
-                put(a.CstT, a.CstT_lo, voff + co, x, hi, lo);
-                if constexpr (DOT) {   // the state as it is written (the sum of its terms in split mode)
-                    f32x4 xs = __builtin_convertvector(hi, f32x4), ys = __builtin_convertvector(y[u], f32x4);
-                    if (split) xs += __builtin_convertvector(lo, f32x4);
-                    if (a.dot_with_lo) ys += __builtin_convertvector(yl[u], f32x4);
-                    const float dot = wave_reduce<OpAdd>(dot_group(xs, ys));   // (a wave: eight rows of eight groups)
-                    if (lane == 0) red[step & 1][wave] = dot;
+            for (int g = 0; g < GROUP; g++) {
+                const int step = first + g;
+                if (step < a.NCS) {
+                    const float gam = gams[step];
+                    run = run * gam + d[u0 + g];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) asm volatile("" : "+v"(run[e]));   // (see chunk_carry_t_kernel)
+                    if (a.Cst) put(a.Cst, a.Cst_lo, koff + (size_t)chunk_of(step) * D * D, run, hi, lo);
+                    if (a.CstT) {
+#pragma unroll
+                        for (int e = 0; e < 4; e++) tile[par][g][c4 + e][row] = run[e];
+                    }
+                    if (vec) {
+                        nrun = nrun * gam + nin[u0 + g];
+                        nst[(size_t)chunk_of(step) * D] = nrun;
+                    }
                 }
             }
-            if (vec) {
-                nrun = nrun * gam + nin[u];
-                nst[(size_t)chunk_of(step) * D] = nrun;
+            if (a.CstT) {   // (uniform) turned round in LDS
+                __syncthreads();
+                if (first > 0) put_dots(first - GROUP);
+#pragma unroll
+                for (int g = 0; g < GROUP; g++) {
+                    const int step = first + g;
+                    if (step < a.NCS) {
+                        const f32x4 x = *reinterpret_cast<const f32x4*>(&tile[par][g][row][c4]);
+                        put(a.CstT, a.CstT_lo, voff + (size_t)chunk_of(step) * D * D, x, hi, lo);
+                        if constexpr (DOT > 0) {   // the state as it is written (the sum of its terms in split mode)
+                            f32x4 xs = __builtin_convertvector(hi, f32x4), ys = __builtin_convertvector(y[u0 + g], f32x4);
+                            if (split) xs += __builtin_convertvector(lo, f32x4);
+                            if constexpr (DOT == 2) ys += __builtin_convertvector(yl[u0 + g], f32x4);
+                            const float dot = wave_reduce<OpAdd>(dot_group(xs, ys));   // (a wave: eight rows of eight groups)
+                            if (lane == 0) red[par][g][wave] = dot;
+                        }
+                    }
+                }
             }
             }
         }
     }
-    if constexpr (DOT) {
+    if constexpr (DOT > 0) {
         __syncthreads();
-        put_dot(a.NCS - 1);
+        put_dots((a.NCS - 1) / GROUP * GROUP);
     }
 }
 
@@ -1048,8 +1067,6 @@ struct SeqCfg {
 #define SQ_DUMP(kind) do {} while (0)
 #endif
 
-template <int N> __device__ __forceinline__ void dma_wait_all_but() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-
 template <typename T, int D, bool DOT>
 __global__ __launch_bounds__(512) void chunk_seq_kernel(ChunkArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -1172,11 +1189,11 @@ __global__ __launch_bounds__(512) void chunk_seq_kernel(ChunkArgs a) {
 #pragma unroll
         for (int p = 0; p < PF; p++)
             if (p < NTOT) { issue(ci, p % NS); advance(ci); }
-        if (NTOT >= PF) dma_wait_all_but<(PF - 1) * NI>(); else dma_wait();
+        if (NTOT >= PF) dma_wait_but<(PF - 1) * NI>(); else dma_wait();
         __syncthreads();   // tile 0 has landed
         prepare(ct, 0);
         advance(ct);
-        if (NTOT >= PF) dma_wait_all_but<(PF - 2) * NI>(); else dma_wait();
+        if (NTOT >= PF) dma_wait_but<(PF - 2) * NI>(); else dma_wait();
         __syncthreads();   // tile 1 has landed
         SQ_DECL;
         for (int t = 0; t < NTOT; t++) {
@@ -1184,7 +1201,7 @@ __global__ __launch_bounds__(512) void chunk_seq_kernel(ChunkArgs a) {
             SQ_STAMP(0);
             if (t + 1 < NTOT) { prepare(ct, (t + 1) % NS); advance(ct); }
             SQ_STAMP(1);
-            if (t + PF < NTOT) dma_wait_all_but<(PF - 2) * NI>(); else dma_wait();
+            if (t + PF < NTOT) dma_wait_but<(PF - 2) * NI>(); else dma_wait();
             SQ_STAMP(2);
             __syncthreads();
             SQ_STAMP(3);
@@ -1389,21 +1406,23 @@ static int launch_chunk_sum(const ChunkArgs& a, hipStream_t st) {
 }
 
 // 16-bit D = 128 and 256: the carry in blocks of 32 x 32, sixteen steps per trip to memory, or in blocks of 64 x 64, a trip per
-// step but rows of 128 bytes.  The second moves memory faster once it fills the chip; below that it is its trips one after the
-// other.  Workgroups of the second form, chunks: training step in us, 64 x 64 / 32 x 32 (bf16):
-//   D = 128   4, 31: 253 / 159     32, 31: 427 / 339    64, 7 (gated): 135 / 119   128, 31: 1203 / 1107   192, 7: 219 / 227
-//             192, 31: 1727 / 1649   256, 7: 543 / 552   256, 31: 2187 / 2136
-//   D = 256   128, 7: 196 / 187    192, 7: 174 / 180    256, 7: 288 / 294          256, 31: 1206 / 1155    512, 15: 1073 / 1097
+// step but rows of 128 bytes.  The second moves memory faster where it fills the chip and the states are few; otherwise it is its trips
+// one after the other.  Workgroups of the second form, states: both carries of a training step in us, 64 x 64 / 32 x 32 (bf16):
+//   D = 128   64, 4: 21.3 / 11.1    128, 7: 33.8 / 20.8   192, 7: 37.7 / 24.9   256, 4: 24.4 / 25.1   256, 7: 39.0 / 31.2   256, 15: 99.8 / 54.1
+//             256, 31: 207 / 118    512, 7: 61.2 / 53.7   512, 15: 122 / 112    512, 31: 240 / 213
+//   D = 256   192, 3: 16.3 / 13.8   256, 3: 16.6 / 17.9   256, 7: 35.6 / 30.0   256, 15: 72.9 / 52.2  384, 7: 45.5 / 42.9   512, 3: 22.5 / 33.8
+//             512, 7: 50.8 / 52.6   512, 15: 128 / 116    512, 31: 248 / 236    1024, 15: 195 / 228
 static bool carry_in_small_blocks(const ChunkArgs& a, int D) {
     const int wgs = a.BH * (D / 64) * (D / 64);
-    return wgs <= 128 || (wgs <= 256 && a.NCS >= 16);
+    return wgs <= 192 || (wgs <= 384 && a.NCS >= 6) || (wgs <= 512 && a.NCS >= 12);
 }
 
 template <typename T, int D>
 static int launch_chunk_carry_small(const ChunkArgs& a, hipStream_t st) {
     const dim3 cgrid((D / 32) * (D / 32), a.BH);
-    if (a.dot_part) hipLaunchKernelGGL((chunk_carry_small_kernel<T, D, true>), cgrid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((chunk_carry_small_kernel<T, D, false>), cgrid, dim3(256), 0, st, a);
+    if (a.dot_part && a.dot_with_lo) hipLaunchKernelGGL((chunk_carry_small_kernel<T, D, 2>), cgrid, dim3(256), 0, st, a);
+    else if (a.dot_part) hipLaunchKernelGGL((chunk_carry_small_kernel<T, D, 1>), cgrid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL((chunk_carry_small_kernel<T, D, 0>), cgrid, dim3(256), 0, st, a);
     return (int)hipGetLastError();
 }
 

@@ -23,8 +23,6 @@ namespace mlstm {
 constexpr int CW_QT = 32;                // queries per tile
 constexpr int CW_MOST_QUERIES = 1024;    // queries a key may meet: their scalars stay in LDS for the whole kernel
 
-template <int N> __device__ __forceinline__ void dma_wait_but() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-
 template <typename T, int D, bool STRICT>
 struct ColwCfg {
     static constexpr size_t QT_BYTES = (size_t)CW_QT * D * sizeof(T), SLOT_BYTES = 2 * QT_BYTES;   // a tile of Q, one of dH

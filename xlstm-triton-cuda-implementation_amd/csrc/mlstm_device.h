@@ -367,6 +367,8 @@ __device__ __forceinline__ void dma4(const void* g, unsigned lds_off) {
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "s"(lds_off) : "memory", "m0");
 }
 __device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// everything but the N newest of the wave's memory operations (others than the counted loads among them, a spill's, only make it wait longer)
+template <int N> __device__ __forceinline__ void dma_wait_but() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 // The compiler does not know about the direct loads in flight, so a wait it places inside the main loop for a value
 // that was loaded from global memory before the loop would, every iteration, also wait for the tile copy just
 // issued.  pin() makes a prologue value "used" at the point of the call, which moves that wait out of the loop.

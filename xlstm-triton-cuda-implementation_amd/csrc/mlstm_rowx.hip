@@ -32,8 +32,6 @@ struct RowxCfg {
     static size_t lds_bytes(int keys) { return POOL_BYTES + P_BYTES + MISC_FLOATS * 4 + (size_t)keys * 8 + GRAN * 4; }
 };
 
-template <int N> __device__ __forceinline__ void dma_wait_but() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-
 template <typename T, int D, int MODE>
 __global__ __launch_bounds__(512) void rowx_kernel(RowArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
