@@ -33,7 +33,7 @@ struct ColdCfg {
     static constexpr size_t QT_BYTES = (size_t)CD_QT * D * sizeof(T);                  // a 32-row tile of Q or dH
     static constexpr size_t STAGES_BYTES = 4 * QT_BYTES;                               // two stages of (Q, dH); the state tiles before them
     static constexpr size_t ROW_BYTES = 2 * 3 * GRAN * sizeof(float);                  // per stage: beta, 1/n, db (64 floats copied, 32 used)
-    static constexpr size_t MISC_BYTES = (2 * 4 * CD_QT + D) * sizeof(float);     // row sums [2 parities][4 key blocks][32], the vector state
+    static constexpr size_t MISC_BYTES = (2 * 4 * CD_QT + D + (D == 128 ? 3 * CD_KEYS : 0)) * sizeof(float);     // row sums [2 parities][4 key blocks][32], the vector state
     static constexpr size_t LDS_BYTES = V_BYTES + STAGES_BYTES + ROW_BYTES + MISC_BYTES;   // plus one float per 64-position granule
 };
 
@@ -66,9 +66,26 @@ template <> struct MmaV<_Float16> {
 };
 __device__ __forceinline__ void settle(f32x16& c0, f32x16& c1) { asm volatile("s_nop 15\n\ts_nop 15" : "+v"(c0), "+v"(c1)); }
 
+// SwzTransReader from two offsets: column block d meets the swizzle's upper bits in an XOR
+template <typename T, int D>
+struct TransX {
+    int off[2];
+    __device__ __forceinline__ void init(int lane, int) {
+        const int h = lane >> 5, j = lane & 15, sub = (lane >> 4) & 1;
+#pragma unroll
+        for (int hi = 0; hi < 2; hi++) off[hi] = Swz<T, D>::off(4 * h + (j >> 2) + 8 * hi, 16 * sub + 4 * (j & 3));
+    }
+    __device__ __forceinline__ typename Tr<T>::frag read(const T* tile, int kr, int d) const {
+        const char* base = reinterpret_cast<const char*>(tile) + kr * Swz<T, D>::ROW_BYTES + (d / 4) * 256;
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_PTR(s16x4))(base + (off[0] ^ ((d % 4) << 6))));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_PTR(s16x4))(base + (off[1] ^ ((d % 4) << 6))));
+        return __builtin_bit_cast(typename Tr<T>::frag, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    }
+};
+
 // Profiling builds (-DMLSTM_COLD_PROF): waves 0 and 3 add up the shader-clock cycles they spend in each part of the
 // kernel and leave the sums, as floats, in the first two rows of the workgroup's dK tile (the results are then wrong, the
-// timing is what the build is for).  s_memtime is only trustworthy with one wave per SIMD, which this kernel has.
+// timing is what the build is for).  s_memtime is only trustworthy with one wave per SIMD (D = 256, split mode).
 #ifdef MLSTM_COLD_PROF
 #define CP_DECL float prof_[12] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}; long long last_ = (long long)__builtin_amdgcn_s_memtime()
 #define CP_STAMP(k) do { const long long now_ = (long long)__builtin_amdgcn_s_memtime(); prof_[k] += (float)(now_ - last_); last_ = now_; } while (0)
@@ -80,7 +97,7 @@ __device__ __forceinline__ void settle(f32x16& c0, f32x16& c1) { asm volatile("s
 #endif
 
 template <typename T, int D, bool STRICT, bool DENSE>
-__global__ __launch_bounds__(256, 1) void cold_kernel(ColArgs a) {
+__global__ __launch_bounds__(256, D == 128 && !STRICT ? 2 : 1) void cold_kernel(ColArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the body uses device-only builtins; the host pass only needs the stub
     CP_DECL;
     using R = Tr<T>;
@@ -89,6 +106,12 @@ __global__ __launch_bounds__(256, 1) void cold_kernel(ColArgs a) {
     typedef typename R::frag frag;
     static_assert(R::HALF && (D == 128 || D == 256), "16-bit types, D = 128 or 256");
     constexpr int KW = R::KW, NS = D / KW, NXD = D / 32;
+    // D = 128: two workgroups per CU, 256 registers per lane, so that one of them multiplies while the other waits for its first tiles (HBM: all
+    // CUs ask at once) or writes out -- 15000 of a workgroup's 38000 cycles on average -- instead of one per CU with the element-wise part of a
+    // half tile between the products of the other half.  64 heads x 16384 x 128: 789 us -> 613.  What a register less costs: with three spilled
+    // values per step 700 us, with twelve 932 (a reload waits for the copies in front of it).
+    // (Split mode keeps one: 32 heads x 2048 x 128 64 us against 73, 64 heads 121 against 114.)
+    constexpr bool LEAN = D == 128 && !STRICT;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     // The stages come first: their tiles are read with instruction offsets (16 bits), which reach the first 64 KB only
     char* const stg = smem;
@@ -99,7 +122,8 @@ __global__ __launch_bounds__(256, 1) void cold_kernel(ColArgs a) {
 #define ST_ROW(st) (reinterpret_cast<float*>(tail) + (st) * 3 * GRAN)
     float* const rowtmp = reinterpret_cast<float*>(tail + Cfg::ROW_BYTES);   // [2][4][32]
     float* const gvl = rowtmp + 2 * 4 * CD_QT;   // the chunk's vector state g
-    float* const sG = gvl + D;                         // granule bases minus that of the tile's first granule
+    float* const keyvals = gvl + D;                    // D = 128: [alpha, log2 s, s][key]
+    float* const sG = keyvals + (LEAN ? 3 * CD_KEYS : 0);                         // granule bases minus that of the tile's first granule
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = lane >> 5, c32 = lane & 31;
     const int kb = wave;
@@ -158,14 +182,18 @@ __global__ __launch_bounds__(256, 1) void cold_kernel(ColArgs a) {
     const int NQe = a.chunk_len > 0 ? ((chunk + 1) * (a.chunk_len / CD_QT) < NQ ? (chunk + 1) * (a.chunk_len / CD_QT) : NQ) : NQ;
     const bool has_state = a.chunk_len > 0 && chunk < a.n_states;   // (uniform over the workgroup)
     const int it0 = jt * (CD_KEYS / CD_QT);        // the first query tile: the keys' own
+    auto last_tile = [&](T* tile, const T* g, int row0, size_t rs) __attribute__((always_inline)) {
+        if constexpr (LEAN) tile_dma_rolled<T, D, CD_QT, 256>(tile, g, row0, S, tid, rs);
+        else tile_dma<T, D, CD_QT, 256>(tile, g, row0, S, tid, rs);
+    };
 #define COLD_DMA(it, st)                                                          \
     do {                                                                          \
         if ((it) < full_q) {                                                      \
             qdma.issue(ST_Q(st), Q + (size_t)CD_QT * (it) * rsA, ra);              \
             qdma.issue(ST_DH(st), dH + (size_t)CD_QT * (it) * rsB, rb);            \
         } else {                                                                  \
-            tile_dma<T, D, CD_QT, 256>(ST_Q(st), Q, CD_QT * (it), S, tid, rsA);    \
-            tile_dma<T, D, CD_QT, 256>(ST_DH(st), dH, CD_QT * (it), S, tid, rsB);  \
+            last_tile(ST_Q(st), Q, CD_QT * (it), rsA);                             \
+            last_tile(ST_DH(st), dH, CD_QT * (it), rsB);                           \
         }                                                                         \
         rvdma.issue(ST_ROW(st), (it));                                             \
     } while (0)
@@ -205,14 +233,24 @@ __global__ __launch_bounds__(256, 1) void cold_kernel(ColArgs a) {
     for (int x = 0; x < NXD; x++)
 #pragma unroll
         for (int r = 0; r < 16; r++) { dkacc[x][r] = 0.f; dvacc[x][r] = 0.f; }
-    SwzTransReader<T, D> trd;
+    typename std::conditional<LEAN, TransX<T, D>, SwzTransReader<T, D>>::type trd;
     trd.init(lane, 0);
     SwzRowReaderX<T, D> rrd;
     rrd.init(lane);
 
     if (has_state && tid < D) gvl[tid] = a.gvec[((size_t)bh * a.n_states + chunk) * D + tid];
-    if (tid < NG) sG[tid] = (float)(g_first - gbase);
-    for (int g = tid + 256; g < NG; g += 256) sG[g] = (float)(a.G2[goff + g] - gbase);
+    if constexpr (LEAN) {
+        // for either granule of keys with what else the exponent of a weight has
+        const float corr0 = (float)(gbase - a.G2[goff + g0]), corr1 = (float)(gbase - a.G2[goff + (g0 + 1 < NG ? g0 + 1 : NG - 1)]), l2s = -0.5f * __log2f((float)D);
+        for (int g = tid; g < NG; g += 256) {
+            const float d = (float)((g == tid ? g_first : a.G2[goff + g]) - gbase);
+            sG[g] = d + corr0 + l2s;
+            sG[NG + g] = d + corr1 + l2s;
+        }
+    } else {
+        if (tid < NG) sG[tid] = (float)(g_first - gbase);
+        for (int g = tid + 256; g < NG; g += 256) sG[g] = (float)(a.G2[goff + g] - gbase);
+    }
     const float gcorr = (float)(gbase - gkey);   // granule base of the tile's first granule minus that of the wave's keys
 #pragma unroll
     for (int s = 0; s < NS; s++) pin(kf[s]);
@@ -329,6 +367,11 @@ __global__ __launch_bounds__(256, 1) void cold_kernel(ColArgs a) {
         CP_STAMP(2);
     }
     const float log2scale = -0.5f * __log2f((float)D);
+    // (two workgroups per CU leave no register for a key's scalars, and a spilled one would be waited for behind the copies under way)
+    if constexpr (LEAN) {
+        if (h == 0) { keyvals[32 * kb + c32] = al; keyvals[CD_KEYS + 32 * kb + c32] = log2_s; keyvals[2 * CD_KEYS + 32 * kb + c32] = scale_s; }
+        __builtin_amdgcn_wave_barrier();
+    }
 
     // row sums: one slice per 64 keys (the dF pass adds them up), that of the second half where that pass reads it
     const int j64 = 2 * jt;
@@ -337,16 +380,14 @@ __global__ __launch_bounds__(256, 1) void cold_kernel(ColArgs a) {
     // 16 queries: the factorised form of the other kernels would need one exponential per query and lane as well) and
     // masks it where the key lies behind the query, so diagonal tiles need no code of their own.
     constexpr int PW = TileDma<T, D, CD_QT, 256>::PER_WAVE;
-    const int rt_own = (lane & 4) * 2 + 4 * h + ((lane >> 2) & 2) + ((lane >> 4) & 1);   // the query whose row sum row_sums8 leaves in this lane
-    auto step = [&](auto spread_tag, int it) {
-        constexpr bool SPREAD = decltype(spread_tag)::value;  // copy of tile it+1 interleaved with this step's MFMAs
+    auto step = [&](auto spread, int it) __attribute__((always_inline)) {   // spread: copy of tile it+1 interleaved with this step's MFMAs
         const int qi0 = CD_QT * it;
         const int stage = (it - it0) & 1, stn = stage ^ 1;
         dma_wait();
         __syncthreads();   // tile `it` has landed and every wave is past phase B of the previous step
         CP_STAMP(3);
         CP_COUNT(8);
-        if constexpr (SPREAD) {
+        if (spread) {
             rvdma.issue(ST_ROW(stn), it + 1);
         } else {
             if (it + 1 < NQe) { if (stage) COLD_DMA(it + 1, 0); else COLD_DMA(it + 1, 1); }
@@ -366,24 +407,29 @@ __global__ __launch_bounds__(256, 1) void cold_kernel(ColArgs a) {
         const T* dHs = ST_DH(stage);
         const float* srow = ST_ROW(stage);
         float* const rt = rowtmp + (it & 1) * 4 * CD_QT + kb * CD_QT;
+        int l = lane;
+        auto rr = rrd;
+        auto tr = trd;
+        if constexpr (LEAN) asm volatile("" : "+v"(l), "+v"(rr.off0), "+v"(tr.off[0]), "+v"(tr.off[1]));   // (addresses are formed anew in every step: see keyvals)
+        const int rt_own = (l & 4) * 2 + ((l >> 3) & 4) + ((l >> 2) & 2) + ((l >> 4) & 1);   // the query whose row sum row_sums8 leaves in this lane
 
         const bool active = key0 <= qi0 + CD_QT - 1;   // some key of the wave lies at or before some query of the tile
         f32x16 gacc, wacc;   // dC, then G = dC~ E;  S, then W = C~ / n   (rows = queries 8 (r / 4) + 4 h + r % 4, column = key c32)
         if (active) {
             // ---- phase A
-            constexpr int AHEAD = 4;
+            constexpr int AHEAD = LEAN ? 1 : 4;
             frag qf[NS], hf[NS], vf[NS];
 #pragma unroll
-            for (int s = 0; s < AHEAD; s++) { qf[s] = rrd.read(Qs, 0, s); hf[s] = rrd.read(dHs, 0, s); vf[s] = rrd.read(Vt, kb, s); }
+            for (int s = 0; s < AHEAD; s++) { qf[s] = rr.read(Qs, 0, s); hf[s] = rr.read(dHs, 0, s); vf[s] = rr.read(Vt, kb, s); }
 #pragma unroll
             for (int s = 0; s < NS; s++) {
-                if constexpr (SPREAD) {
-                    if (s % AHEAD == 0) qdma.issue_range(lq, gq, (s / AHEAD) * PW / (NS / AHEAD), (s / AHEAD + 1) * PW / (NS / AHEAD), ra);
+                if (spread) {
+                    if (s % 4 == 0) qdma.issue_range(lq, gq, (s / 4) * PW / (NS / 4), (s / 4 + 1) * PW / (NS / 4), ra);
                 }
                 if (s + AHEAD < NS) {
-                    qf[s + AHEAD] = rrd.read(Qs, 0, s + AHEAD);
-                    hf[s + AHEAD] = rrd.read(dHs, 0, s + AHEAD);
-                    vf[s + AHEAD] = rrd.read(Vt, kb, s + AHEAD);
+                    qf[s + AHEAD] = rr.read(Qs, 0, s + AHEAD);
+                    hf[s + AHEAD] = rr.read(dHs, 0, s + AHEAD);
+                    vf[s + AHEAD] = rr.read(Vt, kb, s + AHEAD);
                 }
                 if constexpr (D == 256) {   // (accumulators in vector registers: see MmaV)
                     if (s == 0) { MmaV<T>::first(wacc, qf[s], kf[s]); MmaV<T>::first(gacc, hf[s], vf[s]); }
@@ -405,7 +451,8 @@ __global__ __launch_bounds__(256, 1) void cold_kernel(ColArgs a) {
             // queries of contraction step t of phase B, so the second half's element-wise work, and all the lane reductions
             // of the row sums, are placed between the MFMAs of phase B.  Everything is branch-free: a masked element (key
             // behind the query, or a query past the end) gets the exponent -inf.
-            const float argbase = al + (sG[it >> 1] + gcorr + log2scale) - log2_s;   // (weights over s_j: see END_SCALE)
+            const float argbase = (LEAN ? keyvals[32 * kb + c32] : al) + (LEAN ? sG[(kb >> 1) * NG + (it >> 1)] : sG[it >> 1] + gcorr + log2scale) - (LEAN ? keyvals[CD_KEYS + 32 * kb + c32] : log2_s);
+            const float scale_k = LEAN ? keyvals[2 * CD_KEYS + 32 * kb + c32] : scale_s;   // (weights over s_j: see END_SCALE)
             const unsigned span = (unsigned)(S - key);    // query q takes part iff 0 <= q - key < S - key (unsigned compare)
             const int dq0 = qi0 + 4 * h - key;            // q - key of register r: dq0 + 8 (r / 4) + r % 4
             float dd[16], csum0 = 0.f, csum1 = 0.f;   // (column sums: per half of a block, then over the blocks, the order of mlstm_colw.hip)
@@ -425,7 +472,7 @@ __global__ __launch_bounds__(256, 1) void cold_kernel(ColArgs a) {
                 const float e = fast_exp2(live ? argbase - beta4[u][c] : -INFINITY);
                 const float ct = wacc[r] * e;
                 const float dct = fmaf(gacc[r], inv4[u][c], db4[u][c]);
-                dd[r] = rounded_product(END_SCALE ? ct * scale_s : ct, dct);
+                dd[r] = rounded_product(END_SCALE ? ct * scale_k : ct, dct);
                 gacc[r] = STRICT ? rounded_product(dct, e) : dct * e;   // (their low-order terms are what these values lose)
                 wacc[r] = STRICT ? rounded_product(ct, inv4[u][c]) : ct * inv4[u][c];
                 if (r < 8) csum0 += dd[r];
@@ -434,26 +481,35 @@ __global__ __launch_bounds__(256, 1) void cold_kernel(ColArgs a) {
             ew_scalars(0);
 #pragma unroll
             for (int r = 0; r < 8; r++) ew_one(r);
-            ew_scalars(1);   // (for the second half, whose work rides on phase B below)
+            if constexpr (!LEAN) ew_scalars(1);   // (for the second half, whose work rides on phase B below)
             CP_STAMP(5);
 #pragma unroll
             for (int t = 0; t < 2; t++) {
+                if constexpr (LEAN) {
+                    if (t == 1) {
+                        ew_scalars(1);
+#pragma unroll
+                        for (int r = 8; r < 16; r++) ew_one(r);
+                    }
+                    rt[rt_own + 16 * t] = row_sums8(dd + 8 * t, lane & 8, lane & 4);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
                 frag ghi, glo, whi, wlo;
                 if constexpr (STRICT) { R::from_acc_split(gacc, t, ghi, glo); R::from_acc_split(wacc, t, whi, wlo); }
                 else { ghi = R::from_acc(gacc, t); whi = R::from_acc(wacc, t); }
                 frag qa[2], ha[2];
-                qa[0] = trd.read(Qs, KW * t, 0);
-                ha[0] = trd.read(dHs, KW * t, 0);
+                qa[0] = tr.read(Qs, KW * t, 0);
+                ha[0] = tr.read(dHs, KW * t, 0);
 #pragma unroll
                 for (int x = 0; x < NXD; x++) {
-                    if constexpr (SPREAD) {
+                    if (spread) {
                         constexpr int HOOKS = 2 * NXD / 2;   // one hook per two column blocks, over both halves
                         if (x % 2 == 0) {
                             const int k = t * (NXD / 2) + x / 2;
                             qdma.issue_range(ldh, gdh, k * PW / HOOKS, (k + 1) * PW / HOOKS, rb);
                         }
                     }
-                    if (x + 1 < NXD) { qa[(x + 1) & 1] = trd.read(Qs, KW * t, x + 1); ha[(x + 1) & 1] = trd.read(dHs, KW * t, x + 1); }
+                    if (x + 1 < NXD) { qa[(x + 1) & 1] = tr.read(Qs, KW * t, x + 1); ha[(x + 1) & 1] = tr.read(dHs, KW * t, x + 1); }
                     R::mma(dkacc[x], qa[x & 1], ghi);
                     R::mma(dvacc[x], ha[x & 1], whi);
                     if constexpr (STRICT) {
@@ -461,25 +517,29 @@ __global__ __launch_bounds__(256, 1) void cold_kernel(ColArgs a) {
                         R::mma(dvacc[x], ha[x & 1], wlo);
                     }
                     // behind the MFMAs: 8 / NXD registers of the second half's element-wise work (t = 0 only) and this half's row sums
-                    if (t == 0) {
+                    if (!LEAN && t == 0) {
 #pragma unroll
                         for (int u = 0; u < 8 / NXD; u++) ew_one(8 + x * (8 / NXD) + u);
                     }
-                    if (x == 1 - t) rt[rt_own + 16 * t] = row_sums8(dd + 8 * t, lane & 8, lane & 4);
+                    if (!LEAN && x == 1 - t) rt[rt_own + 16 * t] = row_sums8(dd + 8 * t, lane & 8, lane & 4);
                     __builtin_amdgcn_sched_barrier(0);
                 }
-                if (t == 0) colacc += csum0 + csum1;
             }
+            colacc += csum0 + csum1;
             CP_STAMP(6);
         } else {
-            if constexpr (SPREAD) { qdma.issue(lq, gq, ra); qdma.issue(ldh, gdh, rb); }
+            if (spread) { qdma.issue(lq, gq, ra); qdma.issue(ldh, gdh, rb); }
             if (lane < CD_QT) rt[lane] = 0.f;
         }
     };
     const int lim = (NQe < full_q ? NQe : full_q) - 1;   // last step index that may spread is lim - 1
     int it = it0;
-    for (; it < lim; it++) step(std::true_type{}, it);
-    for (; it < NQe; it++) step(std::false_type{}, it);
+    if constexpr (LEAN) {
+        for (; it < NQe; it++) step(it < lim, it);
+    } else {
+        for (; it < lim; it++) step(std::true_type{}, it);
+        for (; it < NQe; it++) step(std::false_type{}, it);
+    }
 #undef COLD_DMA
 
     // ---- epilogue: column sums, the last step's row sums, then dK and dV through LDS (the V tile and the stages are free
@@ -513,7 +573,7 @@ __global__ __launch_bounds__(256, 1) void cold_kernel(ColArgs a) {
 #pragma unroll
                     for (int c = 0; c < 4; c++) v[c] = which ? dvacc[x][4 * a4 + c] : dkacc[x][4 * a4 + c];
                     if constexpr (END_SCALE) {   // the keys' weights: see the state phase
-                        v *= scale_s;
+                        v *= LEAN ? keyvals[2 * CD_KEYS + 32 * kb + c32] : scale_s;
                         if (!which && has_state) {
                             const f32x4 g4 = *reinterpret_cast<const f32x4*>(gvl + d);
 #pragma unroll
@@ -557,11 +617,11 @@ template <typename T, int D, bool STRICT, bool DENSE>
 static int launch_cold_t(const ColArgs& a, hipStream_t st) {
     using Cfg = ColdCfg<T, D>;
     auto kern = cold_kernel<T, D, STRICT, DENSE>;
-    if (hipError_t e = lds_limit_once<cold_kernel<T, D, STRICT, DENSE>>((int)(Cfg::LDS_BYTES + 2048 * sizeof(float))); e != hipSuccess) return (int)e;
+    if (hipError_t e = lds_limit_once<cold_kernel<T, D, STRICT, DENSE>>((int)(Cfg::LDS_BYTES + 2048 * sizeof(float) * (D == 128 ? 2 : 1))); e != hipSuccess) return (int)e;
     if (a.NG > 2048) return MLSTM_ESHAPE;
     if (a.chunk_len > 0 && (a.chunk_len % CD_KEYS != 0 || (a.n_states > 0 && (!a.Ev || !a.gvec || (STRICT && !a.Ev_lo))))) return MLSTM_EINVAL;
     const int NK = (a.S + CD_KEYS - 1) / CD_KEYS;
-    hipLaunchKernelGGL(kern, dim3(a.BH * NK), dim3(256), Cfg::LDS_BYTES + (size_t)a.NG * sizeof(float), st, a);
+    hipLaunchKernelGGL(kern, dim3(a.BH * NK), dim3(256), Cfg::LDS_BYTES + (size_t)a.NG * sizeof(float) * (D == 128 ? 2 : 1), st, a);
     return (int)hipGetLastError();
 }
 

@@ -192,12 +192,12 @@ inline int launch_col_best(int dtype, int D, const ColArgs& a, hipStream_t st) {
     if (!half_big || variant < 0 || variant > 3) variant = 3;
     if (variant == 0) {
         // Workgroups of 64 keys up to which colw_kernel is the faster one; cold_kernel / colw_kernel, us (bf16, workgroups of 64 keys):
-        //   D = 128, S = 1000 (not in chunks)   64: 50 / 27   256: 52 / 30   512: 54 / 39   768: 82 / 58
-        //   D = 128 in chunks of 512            64: 32 / 20   256: 35 / 23   512: 37 / 34   768: 51 / 48   1024: 52 / 59
+        //   D = 128, S = 1000 (not in chunks)  256: 57 / 30   512: 61 / 39   768: 80 / 60
+        //   D = 128 in chunks of 512           256: 37 / 22   512: 39 / 32   768: 44 / 48    in split mode   128: 38 / 26   256: 40 / 28   512: 43 / 41   768: 61 / 60
         //   D = 256, S = 1000                   64: 69 / 40   256: 72 / 45   512: 76 / 57
         //   D = 256 in chunks                  128: 51 / 33   256: 53 / 36   512: 56 / 54   768: 82 / 82
         //   D = 256 in split mode              128: 65 / 42   256: 67 / 47   512: 72 / 70   768: 108 / 103
-        if ((long long)a.BH * a.NG <= 768) {
+        if ((long long)a.BH * a.NG <= (D == 128 && a.chunk_len > 0 && !a.precise ? 512 : 768)) {
             const int rc = launch_colw_kernel(dtype, D, a, st);
             if (rc != MLSTM_ESHAPE) return rc;
         }
