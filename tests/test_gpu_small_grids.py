@@ -99,3 +99,14 @@ def test_split_mode_few_row_tiles_give_the_bits_of_many(S, D, heads, layout, dty
                                           ("plain", 8193, 128, 129), ("plain", 8705, 128, 129)])
 def test_either_carry_gives_a_head_the_same_bits(op, S, D, heads):
     test_a_head_alone_is_the_head_of_a_full_chip(op, S, D, heads, "bnsd", torch.bfloat16)
+
+
+# D = 128 with more than 512 workgroups of 64 rows (row_kernel, two workgroups per CU) and more than 768 of 64 keys (cold_kernel, likewise; in
+# chunks 512): edges of the 128-row and 128-key tiles, of the 64- and 32-row tiles that they walk, and of the chunks
+@pytest.mark.parametrize("op,S,heads,layout", [
+    ("plain", 1, 772, "bnsd"), ("gated", 32, 770, "bnsd"), ("plain", 33, 769, "bsnd"), ("plain", 64, 776, "bnsd"), ("gated", 65, 390, "bsnd"),
+    ("plain", 127, 388, "bnsd"), ("plain", 129, 260, "bnsd"), ("plain", 200, 200, "bsnd"), ("plain", 640, 80, "bnsd"), ("gated", 1023, 50, "bnsd"),
+    ("plain", 1024, 41, "bnsd"), ("gated", 1025, 40, "bsnd"), ("plain", 1153, 33, "bnsd"), ("plain", 1601, 24, "bnsd")])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_pairs_of_workgroups_per_cu_give_the_same_bits(op, S, heads, layout, dtype):
+    test_a_head_alone_is_the_head_of_a_full_chip(op, S, 128, heads, layout, dtype)

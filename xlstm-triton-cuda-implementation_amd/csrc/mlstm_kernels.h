@@ -132,7 +132,7 @@ int launch_row8_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t
 int launch_roww_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t st);
 // split mode on 64 rows per workgroup, the bits of the four-wave kernel, for the same launches; not with an output gate
 int launch_rowx_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t st);
-// (the four-wave kernel serves every other case: fp32, D = 64, split mode -- in chunks too -- and the test switch)
+// (the four-wave kernel serves every other case: fp32, D = 64, split mode -- in chunks too --, large launches at D = 128 and the test switch)
 inline int launch_row_best(int mode, int dtype, int D, const RowArgs& a, hipStream_t st) {
     if (dtype != MLSTM_F32 && (D == 128 || D == 256) && !g_force_generic) {
         // While its workgroups (64 rows) number no more than the chip's CUs, roww_kernel: row8_kernel / roww_kernel, forward, us --
@@ -145,7 +145,11 @@ inline int launch_row_best(int mode, int dtype, int D, const RowArgs& a, hipStre
         // D = 128   64: 21.3, 23.2 / 13.5, 15.7   256: 23.4, 24.9 / 16.1, 18.4   384: 23.9, 26.5 / 22.6, 27.0   512: 24.8, 27.6 / 26.2, 29.8
         // D = 256   64: 39.3, 43.8 / 22.6, 26.9   256: 41.8, 47.3 / 26.0, 30.2   384: 42.9, 47.6 / 36.9, 42.4   512: 44.1, 49.0 / 40.8, 46.8
         if ((long long)a.BH * a.NG <= (D == 128 ? 256 : 512) && a.precise) rc = launch_rowx_kernel(mode, dtype, D, a, st);
-        if (rc == MLSTM_ESHAPE && !a.precise) rc = launch_row8_kernel(mode, dtype, D, a, st);
+        // D = 128 beyond 512 of them, row_kernel, whose workgroups share a CU in pairs: row8_kernel / row_kernel, forward and dQ pass, us --
+        //   512: 18.2, 21.1 / 19.0, 22.6   768: 26.9, 30.8 / 23.6, 27.6   1024: 31.6, 36.4 / 25.4, 30.8   2048: 49.7, 59.3 / 41.0, 48.9
+        //   8192: 224, 259 / 180, 224      16384: 416, 482 / 334, 420     not in chunks, 1024: 40.7, 43.0 / 29.4, 33.1
+        const bool pairs = D == 128 && (long long)a.BH * a.NG > 512 && a.spin_limit == DEFAULT_SPIN_LIMIT;
+        if (rc == MLSTM_ESHAPE && !a.precise && !pairs) rc = launch_row8_kernel(mode, dtype, D, a, st);
         if (rc != MLSTM_ESHAPE) return rc;  // extremely long sequences do not fit its LDS budget
     }
     return launch_row_kernel(mode, dtype, D, a, st);

@@ -23,6 +23,10 @@
 //   dQ pass  dQ^T += C~-tiles (value-major) x dH^T, then decay / n_i, the rank-one term decay db_i n~, and the row sums
 //            q_i . dQ_i of dD over the keys before the chunk.
 // In split mode the state comes as two terms, hi + lo (one tile each per stage), and takes two MFMAs per fragment.
+//
+// 16-bit tensors at D = 128: two workgroups per CU (256 registers per lane, 66 KB of LDS), so that one of them multiplies while the other waits
+// for its first tiles or writes out.  64 heads x 16384 x 128, forward and dQ pass: 334 and 420 us, one eight-wave workgroup per CU
+// (mlstm_row8.hip) 416 and 482.
 #include <mutex>
 #include <type_traits>
 #include "mlstm_device.h"
@@ -44,7 +48,7 @@ struct RowCfg {
 
 // STRICT (16-bit types): split mode, see RowArgs::precise.
 template <typename T, int D, int MODE, bool STRICT>
-__global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
+__global__ __launch_bounds__(256, (Tr<T>::HALF && D == 128 && !STRICT) ? 2 : 1) void row_kernel(RowArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the body uses device-only builtins; the host pass only needs the stub
     using R = Tr<T>;
     using Cfg = RowCfg<T, D>;
@@ -133,12 +137,13 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
     float bsum = 0.f;
 
     constexpr bool FAST_TR = R::HALF && Swz<T, D>::CPR >= 16;  // precomputed offsets for the transposing reads
-    // Split mode at D >= 128 shares its order of operations with mlstm_rowx.hip, which spreads a row over waves: the row sums over the key
-    // blocks of either parity and over either half of the state's rows apart, the factorised weights wherever a block lies below the
-    // diagonal, and products that enter a low-order term or a sum rounded first (rounded_product).
-    constexpr bool SPLIT = STRICT && FAST_TR;
+    // The 16-bit types at D >= 128 share their order of operations with mlstm_roww.hip (split mode: mlstm_rowx.hip), which spreads a row
+    // over waves: the row sums over the key blocks of either parity and over either half of the state's rows apart, the factorised
+    // weights wherever a block lies below the diagonal, and in split mode products that enter a low-order term or a sum rounded
+    // first (rounded_product).
+    constexpr bool SPLIT = FAST_TR;
     float bpar[2] = {0.f, 0.f}, bfar[2] = {0.f, 0.f}, dec_far = 0.f;
-    auto product = [](float x, float y) { return SPLIT ? rounded_product(x, y) : x * y; };
+    auto product = [](float x, float y) { return STRICT && SPLIT ? rounded_product(x, y) : x * y; };
     SwzRowReader<T, D> krd;
     krd.init(lane);
     typename std::conditional<F32, SwzTransReaderF32<D>, SwzTransReader<typename std::conditional<FAST_TR, T, __bf16>::type, FAST_TR ? D : 256>>::type vrd;
@@ -657,6 +662,12 @@ __global__ __launch_bounds__(256, 1) void row_kernel(RowArgs a) {
                         const int col = 32 * d + 8 * a4 + 4 * h;
                         const f32x4 of = __builtin_convertvector(*reinterpret_cast<const typename R::vec4*>(og + col), f32x4);
                         f32x4 v;
+                        if constexpr (SPLIT && !STRICT) {   // (from h as it is written, like the other row kernels)
+#pragma unroll
+                            for (int c = 0; c < 4; c++) v[c] = oacc[d][4 * a4 + c] * onorm;
+                            *reinterpret_cast<typename R::vec4*>(outg + col) = gate4<T>(R::cvt4(v), *reinterpret_cast<const typename R::vec4*>(og + col));
+                            continue;
+                        }
 #pragma unroll
                         for (int c = 0; c < 4; c++) v[c] = oacc[d][4 * a4 + c] * onorm * silu(of[c]);
                         *reinterpret_cast<typename R::vec4*>(outg + col) = R::cvt4(v);
