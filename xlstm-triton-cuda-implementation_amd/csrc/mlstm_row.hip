@@ -27,6 +27,10 @@
 // 16-bit tensors at D = 128: two workgroups per CU (256 registers per lane, 66 KB of LDS), so that one of them multiplies while the other waits
 // for its first tiles or writes out.  64 heads x 16384 x 128, forward and dQ pass: 334 and 420 us, one eight-wave workgroup per CU
 // (mlstm_row8.hip) 416 and 482.
+// D = 64, dQ pass: three (168 registers) instead of two, us before / after: 18 heads x 1000 21.2 / 17.9, 64 x 1000 25.4 / 21.6,
+// 59 x 3008 40.0 / 34.0, 64 x 8192 117 / 101.  The forward pass stays at two: three lose where the sequence is not cut (18 x 1000:
+// 17.9 / 19.6, 64 x 1000: 20.4 / 22.4; in chunks 64 x 8192: 89 / 77), in split mode too (18 x 1000: 21.4 / 23.5); its dQ pass measures
+// the same.
 #include <mutex>
 #include <type_traits>
 #include "mlstm_device.h"
@@ -44,11 +48,17 @@ struct RowCfg {
     static constexpr size_t STAGE_BYTES = 2 * TILE_ELEMS * sizeof(T) + 3 * GRAN * sizeof(float);  // Y1, Y2, alpha, ek, amax
     static constexpr size_t STAGES_BYTES = 2 * STAGE_BYTES;
     // plus one double per key tile of the head (the granule bases), appended at launch
+    // workgroups per CU that the register budget is cut for
+    static constexpr int per_cu(int mode, bool strict) {
+        if (!Tr<T>::HALF) return 1;
+        if (D == 128) return strict ? 1 : 2;
+        return D == 64 && mode == ROW_MODE_DQ && !strict ? 3 : 1;
+    }
 };
 
 // STRICT (16-bit types): split mode, see RowArgs::precise.
 template <typename T, int D, int MODE, bool STRICT>
-__global__ __launch_bounds__(256, (Tr<T>::HALF && D == 128 && !STRICT) ? 2 : 1) void row_kernel(RowArgs a) {
+__global__ __launch_bounds__(256, (RowCfg<T, D>::per_cu(MODE, STRICT))) void row_kernel(RowArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the body uses device-only builtins; the host pass only needs the stub
     using R = Tr<T>;
     using Cfg = RowCfg<T, D>;
