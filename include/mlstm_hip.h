@@ -34,8 +34,8 @@ extern "C" {
  * (two MFMAs per fragment), and the forward hands the low-order part of h to the backward (the `saved` buffer of
  * mlstm_forward_save_ex, or a recomputation), which makes the results agree with an fp32 evaluation of the
  * reference's formulas (mlstm_matmul.py:104-118, :336-365) to rtol 2e-2 / atol 2e-3 element by element.  Long
- * sequences run in chunks in this mode too, with every chunk state kept as two terms.  Price: the four-wave kernels
- * instead of the eight-wave ones, and half as many MFMAs again.
+ * sequences run in chunks in this mode too, with every chunk state kept as two terms.  Price: half as many MFMAs again, and
+ * for large launches the four-wave row kernel instead of the eight-wave one.
  */
 #define MLSTM_PRECISE 0x100
 
@@ -315,8 +315,8 @@ int mlstm_timing_select(unsigned mask, int every);
 int mlstm_timing_read(int kernel, double* total_ms, int* launches);
 
 /*
- * Test aid with no counterpart in the reference: the 16-bit types at D >= 128 are normally served by an eight-wave
- * row kernel and fall back to the generic four-wave kernel only when a sequence is too long for its LDS budget.  With
+ * Test aid with no counterpart in the reference: the 16-bit types at D >= 128 are served by one of several kernels per pass, by type, D and
+ * number of workgroups, and fall back to the generic four-wave ones when a sequence is too long for their LDS budget.  With
  * `on` != 0 every shape goes through the generic kernels, so that the fallback can be tested at sizes the CPU oracle
  * can check.  Process-wide; returns the previous setting.
  */
@@ -334,7 +334,7 @@ int mlstm_force_generic_kernels(int on);
 int mlstm_set_chunk_length(int length);
 /*
  * Measurement and test aid: which column kernel (dK, dV, dI) serves the 16-bit types at D = 128 and 256.
- * 0 = the library's choice, 1 = col16_kernel (G / W through LDS, 16x16 MFMA chains), 2 = cold_kernel (G / W stay in
+ * 0 = the library's choice (few workgroups: colw_kernel, else cold_kernel), 1 = col16_kernel (G / W through LDS, 16x16 MFMA chains), 2 = cold_kernel (G / W stay in
  * registers; the only one of the two with a split mode), 3 = the generic four-wave col_kernel.  Process-wide; returns 0,
  * or MLSTM_EINVAL.  No counterpart in the reference.
  */

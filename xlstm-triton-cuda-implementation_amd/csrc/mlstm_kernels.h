@@ -83,7 +83,7 @@ struct RowArgs {
     // backward needs, still goes to out)
     const void* O;
     void* out_gated;
-    // long sequences in chunks (eight-wave kernel only): with chunk_len = L > 0 a row takes the keys of its own chunk of
+    // long sequences in chunks: with chunk_len = L > 0 a row takes the keys of its own chunk of
     // L positions from Y1 / Y2 and everything before the chunk from the state at the end of the previous chunk
     // (launch_chunk_states).  L is a multiple of 128.
     int chunk_len;
@@ -108,7 +108,7 @@ struct RowArgs {
     float* inv_n;
     float* db;
     int BH, S, NG;
-    // Split mode (16-bit types, generic kernel only): the weights of the second product enter it as two terms, hi + lo,
+    // Split mode (16-bit types; rowx_kernel and row_kernel): the weights of the second product enter it as two terms, hi + lo,
     // each in the element type (two MFMAs per fragment), so that their rounding no longer limits the result.  The
     // forward then also leaves h - (h rounded) in out_lo; the dQ pass reads it back through Hin_lo for dh . h.
     int precise;
@@ -166,7 +166,7 @@ struct ColArgs {
     const float* alpha2; const float* beta2; const double* G2;
     const float* inv_n; const float* db;
     int BH, S, NG;
-    // long sequences in chunks (col16_kernel only): with chunk_len > 0 the keys walk the queries of their own chunk and
+    // long sequences in chunks: with chunk_len > 0 the keys walk the queries of their own chunk and
     // take the contribution of the queries behind it from the chunk's reverse states (ChunkArgs::reverse); rowpart is then
     // written for the key tiles of the query's own chunk only
     int chunk_len;
