@@ -110,3 +110,23 @@ def test_either_carry_gives_a_head_the_same_bits(op, S, D, heads):
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_pairs_of_workgroups_per_cu_give_the_same_bits(op, S, heads, layout, dtype):
     test_a_head_alone_is_the_head_of_a_full_chip(op, S, 128, heads, layout, dtype)
+
+
+# split mode at D = 128 on row_kernel with two workgroups per CU (more than 256 of 64 rows) against rowx_kernel (one head), the same edges
+@pytest.mark.parametrize("S,heads,layout", [(1, 258, "bnsd"), (33, 257, "bsnd"), (65, 130, "bnsd"), (129, 90, "bsnd"), (640, 27, "bnsd"), (1023, 17, "bnsd"),
+                                            (1025, 16, "bsnd"), (1601, 25, "bnsd")])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_split_mode_pairs_of_workgroups_per_cu_give_the_same_bits(S, heads, layout, dtype):
+    test_a_head_alone_is_the_head_of_a_full_chip("precise", S, 128, heads, layout, dtype)
+
+
+# D = 64: the forward in chunks of 256 (three workgroups per CU) against the uncut one (two) on the first chunk alone, whose rows take no state
+@pytest.mark.parametrize("S,heads,layout", [(1024, 1, "bnsd"), (1025, 9, "bsnd"), (1100, 3, "bnsd"), (1919, 40, "bsnd")])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_the_first_chunk_at_head_dimension_64_is_the_uncut_sequence(S, heads, layout, dtype):
+    rows, gates = _inputs(heads, S, 64, dtype, layout)
+    L = submodule("_ffi").lib().mlstm_chunk_length_for(S, 64, submodule("_ffi").dtype_code(dtype))
+    whole = mm.mlstm_forward_hip(*rows[:3], *gates)
+    first = mm.mlstm_forward_hip(*[t[:, :, :L] for t in rows[:3]], *[t[:, :, :L].contiguous() for t in gates])
+    for name, a, b in zip(("h", "m", "b"), first, whole):
+        assert bool(torch.isfinite(a.float()).all()) and torch.equal(a, b[:, :, :L]), name

@@ -27,10 +27,13 @@
 // 16-bit tensors at D = 128: two workgroups per CU (256 registers per lane, 66 KB of LDS), so that one of them multiplies while the other waits
 // for its first tiles or writes out.  64 heads x 16384 x 128, forward and dQ pass: 334 and 420 us, one eight-wave workgroup per CU
 // (mlstm_row8.hip) 416 and 482.
+// Split mode at D = 128: two as well (246 to 256 registers, before 271 to 280 and hence one), forward and dQ pass, us before / after, by workgroups:
+// 384: 34.8, 34.9 / 33.0, 33.9   512: 44.8, 48.6 / 34.7, 37.2   2048: 156, 176 / 121, 132.  At D = 64 its forward missed two by two
+// registers: 432: 21.4 / 16.0   512: 31.8 / 25.2   1416: 54.0 / 38.6   4096: 160 / 116; its dQ pass on registers of one kind 137 / 127.
 // D = 64, dQ pass: three (168 registers) instead of two, us before / after: 18 heads x 1000 21.2 / 17.9, 64 x 1000 25.4 / 21.6,
-// 59 x 3008 40.0 / 34.0, 64 x 8192 117 / 101.  The forward pass stays at two: three lose where the sequence is not cut (18 x 1000:
-// 17.9 / 19.6, 64 x 1000: 20.4 / 22.4; in chunks 64 x 8192: 89 / 77), in split mode too (18 x 1000: 21.4 / 23.5); its dQ pass measures
-// the same.
+// 59 x 3008 40.0 / 34.0, 64 x 8192 117 / 101.  The forward pass takes three in chunks (432 workgroups: 13.7 / 11.6, 4096: 81 / 69, on fewer
+// than one per CU the same) and stays at two where the sequence is not cut, where three lose (18 x 1000: 17.9 / 19.6, 64 x 1000:
+// 20.4 / 22.4); in split mode they lose too (18 x 1000: 21.4 / 23.5).
 #include <mutex>
 #include <type_traits>
 #include "mlstm_device.h"
@@ -48,17 +51,18 @@ struct RowCfg {
     static constexpr size_t STAGE_BYTES = 2 * TILE_ELEMS * sizeof(T) + 3 * GRAN * sizeof(float);  // Y1, Y2, alpha, ek, amax
     static constexpr size_t STAGES_BYTES = 2 * STAGE_BYTES;
     // plus one double per key tile of the head (the granule bases), appended at launch
-    // workgroups per CU that the register budget is cut for
-    static constexpr int per_cu(int mode, bool strict) {
-        if (!Tr<T>::HALF) return 1;
-        if (D == 128) return strict ? 1 : 2;
-        return D == 64 && mode == ROW_MODE_DQ && !strict ? 3 : 1;
+    // workgroups per CU that the register budget is cut for (the head of this file has the figures)
+    static constexpr int per_cu(int mode, bool strict, bool chunks) {
+        if (!Tr<T>::HALF || D > 128) return 1;
+        if (D == 64 && !strict) return mode == ROW_MODE_DQ || chunks ? 3 : 1;   // (1: 252 registers, two have room)
+        return 2;
     }
 };
 
 // STRICT (16-bit types): split mode, see RowArgs::precise.
-template <typename T, int D, int MODE, bool STRICT>
-__global__ __launch_bounds__(256, (RowCfg<T, D>::per_cu(MODE, STRICT))) void row_kernel(RowArgs a) {
+// PER_CU: workgroups per CU that the register budget is cut for.
+template <typename T, int D, int MODE, bool STRICT, int PER_CU>
+__global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the body uses device-only builtins; the host pass only needs the stub
     using R = Tr<T>;
     using Cfg = RowCfg<T, D>;
@@ -688,10 +692,10 @@ __global__ __launch_bounds__(256, (RowCfg<T, D>::per_cu(MODE, STRICT))) void row
 #endif
 }
 
-template <typename T, int D, int MODE, bool STRICT>
+template <typename T, int D, int MODE, bool STRICT, bool CHUNKS>
 static int launch_row_ts(const RowArgs& a, hipStream_t st) {
     using Cfg = RowCfg<T, D>;
-    auto kern = row_kernel<T, D, MODE, STRICT>;
+    auto kern = row_kernel<T, D, MODE, STRICT, Cfg::per_cu(MODE, STRICT, CHUNKS)>;
     static std::once_flag once;
     static hipError_t attr_rc = hipSuccess;
     std::call_once(once, [&] {
@@ -707,9 +711,10 @@ static int launch_row_ts(const RowArgs& a, hipStream_t st) {
 template <typename T, int D, int MODE>
 static int launch_row_t(const RowArgs& a, hipStream_t st) {
     if constexpr (Tr<T>::HALF) {
-        if (a.precise) return launch_row_ts<T, D, MODE, true>(a, st);
+        if (a.precise) return launch_row_ts<T, D, MODE, true, false>(a, st);
+        if (D == 64 && a.chunk_len > 0) return launch_row_ts<T, D, MODE, false, true>(a, st);
     }
-    return launch_row_ts<T, D, MODE, false>(a, st);
+    return launch_row_ts<T, D, MODE, false, false>(a, st);
 }
 
 template <typename T, int MODE>
