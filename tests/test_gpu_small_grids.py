@@ -130,3 +130,10 @@ def test_the_first_chunk_at_head_dimension_64_is_the_uncut_sequence(S, heads, la
     first = mm.mlstm_forward_hip(*[t[:, :, :L] for t in rows[:3]], *[t[:, :, :L].contiguous() for t in gates])
     for name, a, b in zip(("h", "m", "b"), first, whole):
         assert bool(torch.isfinite(a.float()).all()) and torch.equal(a, b[:, :, :L]), name
+
+
+# fp32 at D = 64 on row_kernel with two workgroups per CU (more than 256 of 128 rows) against rowf_kernel (one head)
+@pytest.mark.parametrize("op,S,heads,layout", [("plain", 1, 520, "bnsd"), ("plain", 97, 514, "bsnd"), ("gated", 129, 260, "bnsd"), ("plain", 320, 176, "bnsd"),
+                                               ("plain", 1025, 60, "bsnd")])
+def test_fp32_pairs_of_workgroups_per_cu_give_the_same_bits(op, S, heads, layout):
+    test_a_head_alone_is_the_head_of_a_full_chip(op, S, 64, heads, layout, torch.float32)

@@ -34,6 +34,8 @@
 // 59 x 3008 40.0 / 34.0, 64 x 8192 117 / 101.  The forward pass takes three in chunks (432 workgroups: 13.7 / 11.6, 4096: 81 / 69, on fewer
 // than one per CU the same) and stays at two where the sequence is not cut, where three lose (18 x 1000: 17.9 / 19.6, 64 x 1000:
 // 20.4 / 22.4); in split mode they lose too (18 x 1000: 21.4 / 23.5).
+// fp32 at D = 64: two (256 registers, before 319 and hence one).  A training step, us before / after: 16 heads x 1000 98.7 / 95.7,
+// 64 x 300 104 / 103, 16 x 4096 240 / 224, 48 x 4096 618 / 555.  At D = 128 the 131 KB of LDS leave room for one.
 #include <mutex>
 #include <type_traits>
 #include "mlstm_device.h"
@@ -53,7 +55,8 @@ struct RowCfg {
     // plus one double per key tile of the head (the granule bases), appended at launch
     // workgroups per CU that the register budget is cut for (the head of this file has the figures)
     static constexpr int per_cu(int mode, bool strict, bool chunks) {
-        if (!Tr<T>::HALF || D > 128) return 1;
+        if (!Tr<T>::HALF) return D == 64 ? 2 : 1;
+        if (D > 128) return 1;
         if (D == 64 && !strict) return mode == ROW_MODE_DQ || chunks ? 3 : 1;   // (1: 252 registers, two have room)
         return 2;
     }
