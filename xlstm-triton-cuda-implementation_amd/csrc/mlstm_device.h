@@ -77,6 +77,15 @@ template <> struct Tr<__bf16> {
         hi = __builtin_convertvector(x, vec4);
         lo = __builtin_convertvector(x - __builtin_convertvector(hi, f32x4), vec4);
     }
+    // the same of x y, the low-order term from the product as it is before it is rounded to fp32
+    static __device__ __forceinline__ void split_products(f32x4 x, f32x4 y, vec4& hi, vec4& lo) {
+        hi = __builtin_convertvector(x * y, vec4);
+        const f32x4 up = __builtin_convertvector(hi, f32x4);
+        f32x4 rest;
+#pragma unroll
+        for (int e = 0; e < 4; e++) rest[e] = fmaf(x[e], y[e], -up[e]);
+        lo = __builtin_convertvector(rest, vec4);
+    }
 };
 
 template <> struct Tr<_Float16> {
@@ -108,6 +117,15 @@ template <> struct Tr<_Float16> {
     static __device__ __forceinline__ void cvt4_split(f32x4 x, vec4& hi, vec4& lo) {
         hi = __builtin_convertvector(x, vec4);
         lo = __builtin_convertvector(x - __builtin_convertvector(hi, f32x4), vec4);
+    }
+    // the same of x y, the low-order term from the product as it is before it is rounded to fp32
+    static __device__ __forceinline__ void split_products(f32x4 x, f32x4 y, vec4& hi, vec4& lo) {
+        hi = __builtin_convertvector(x * y, vec4);
+        const f32x4 up = __builtin_convertvector(hi, f32x4);
+        f32x4 rest;
+#pragma unroll
+        for (int e = 0; e < 4; e++) rest[e] = fmaf(x[e], y[e], -up[e]);
+        lo = __builtin_convertvector(rest, vec4);
     }
 };
 
@@ -242,6 +260,7 @@ template <> struct Tr<float> {
     // (there is no split mode for fp32 tensors; these keep the shared templates well-formed)
     static __device__ __forceinline__ void from_acc_split(const f32x16& c, int t, frag& hi, frag& lo) { hi = from_acc(c, t); lo = frag{}; }
     static __device__ __forceinline__ void cvt4_split(f32x4 x, vec4& hi, vec4& lo) { hi = x; lo = vec4{0.f, 0.f, 0.f, 0.f}; }
+    static __device__ __forceinline__ void split_products(f32x4 x, f32x4 y, vec4& hi, vec4& lo) { cvt4_split(x * y, hi, lo); }
 };
 
 // What a product of terms (Tr<float>) cannot say: an infinite operand, or a finite one that rounds to an infinite bf16, makes the

@@ -25,10 +25,10 @@
 // In split mode the state comes as two terms, hi + lo (one tile each per stage), and takes two MFMAs per fragment.
 //
 // 16-bit tensors at D = 128: two workgroups per CU (256 registers per lane, 66 KB of LDS), so that one of them multiplies while the other waits
-// for its first tiles or writes out.  64 heads x 16384 x 128, forward and dQ pass: 334 and 420 us, one eight-wave workgroup per CU
+// for its first tiles or writes out.  64 heads x 16384 x 128, forward and dQ pass: 330 and 412 us, one eight-wave workgroup per CU
 // (mlstm_row8.hip) 416 and 482.
-// Split mode at D = 128: two as well (246 to 256 registers, before 271 to 280 and hence one), forward and dQ pass, us before / after, by workgroups:
-// 384: 34.8, 34.9 / 33.0, 33.9   512: 44.8, 48.6 / 34.7, 37.2   2048: 156, 176 / 121, 132.  At D = 64 its forward missed two by two
+// Split mode at D = 128: two as well (244 to 256 registers, before 271 to 280 and hence one), forward and dQ pass, us before / after, by workgroups:
+// 384: 34.8, 34.9 / 35.2, 35.7   512: 44.8, 48.6 / 36.5, 38.5   2048: 156, 176 / 125, 136.  At D = 64 its forward missed two by two
 // registers: 432: 21.4 / 16.0   512: 31.8 / 25.2   1416: 54.0 / 38.6   4096: 160 / 116; its dQ pass on registers of one kind 137 / 127.
 // D = 64, dQ pass: three (168 registers) instead of two, us before / after: 18 heads x 1000 21.2 / 17.9, 64 x 1000 25.4 / 21.6,
 // 59 x 3008 40.0 / 34.0, 64 x 8192 117 / 101.  The forward pass takes three in chunks (432 workgroups: 13.7 / 11.6, 4096: 81 / 69, on fewer
@@ -154,13 +154,11 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
     float bsum = 0.f;
 
     constexpr bool FAST_TR = R::HALF && Swz<T, D>::CPR >= 16;  // precomputed offsets for the transposing reads
-    // The 16-bit types at D >= 128 share their order of operations with mlstm_roww.hip (split mode: mlstm_rowx.hip), which spreads a row
-    // over waves: the row sums over the key blocks of either parity and over either half of the state's rows apart, the factorised
-    // weights wherever a block lies below the diagonal, and in split mode products that enter a low-order term or a sum rounded
-    // first (rounded_product).
-    constexpr bool SPLIT = FAST_TR;
+    // The 16-bit types at D >= 128 outside split mode share their order of operations with mlstm_row8.hip and mlstm_roww.hip, which spread a
+    // row over waves: the row sums over the key blocks of either parity and over either half of the state's rows apart, and the
+    // factorised weights wherever a block lies below the diagonal.
+    constexpr bool PARITY = FAST_TR && !STRICT;
     float bpar[2] = {0.f, 0.f}, bfar[2] = {0.f, 0.f}, dec_far = 0.f;
-    auto product = [](float x, float y) { return STRICT && SPLIT ? rounded_product(x, y) : x * y; };
     SwzRowReader<T, D> krd;
     krd.init(lane);
     typename std::conditional<F32, SwzTransReaderF32<D>, SwzTransReader<typename std::conditional<FAST_TR, T, __bf16>::type, FAST_TR ? D : 256>>::type vrd;
@@ -187,8 +185,10 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
             tdma.issue(ST_Y1(st), Y1 + (size_t)GRAN * (j) * rsA, ra);                     \
             tdma.issue(ST_Y2(st), Y2 + (size_t)GRAN * (j) * rsA, ra);                     \
         } else {                                                                         \
-            tile_dma<T, D, GRAN, 256>(ST_Y1(st), Y1, GRAN * (j), S, tid, rsA);            \
-            tile_dma<T, D, GRAN, 256>(ST_Y2(st), Y2, GRAN * (j), S, tid, rsA);            \
+            int t = tid;   /* (formed anew: addresses kept for a tile that rarely comes were spilled) */ \
+            if constexpr (R::HALF && D == 128) asm volatile("" : "+v"(t));                 \
+            tile_dma<T, D, GRAN, 256>(ST_Y1(st), Y1, GRAN * (j), S, t, rsA);              \
+            tile_dma<T, D, GRAN, 256>(ST_Y2(st), Y2, GRAN * (j), S, t, rsA);              \
         }                                                                                \
         rvdma.issue(ST_AL(st), (j));                                                     \
     } while (0)
@@ -237,12 +237,16 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
             for (int s = 0; s < NS; s++) R::mma(sacc, krd.read(y1, kb, s), xt[s]);
         }
     };
+    // Split mode: the weights of a block as they enter the second product, formed four at a time where they are weighed.  They come as factors,
+    // x y, of which the low-order term takes what rounding the product would lose; factors kept until the product is due cost 16 registers.
+    struct Terms { typename R::vec4 hi[4], lo[4]; };
+    auto terms_of = [](const typename R::vec4* x, int t) { return __builtin_shufflevector(x[2 * t], x[2 * t + 1], 0, 1, 2, 3, 4, 5, 6, 7); };
     // gate weights; `diag` masks the keys above the diagonal of a diagonal block
-    auto weigh = [&](f32x16& sacc, const float* sal, int kb, Crow crow, bool diag) {
-        float blk = 0.f;
+    auto weigh = [&](f32x16& sacc, Terms& w, const float* sal, int kb, Crow crow, bool diag) {
 #pragma unroll
         for (int a4 = 0; a4 < 4; a4++) {
             const f32x4 al = *reinterpret_cast<const f32x4*>(sal + 32 * kb + 8 * a4 + 4 * h);
+            f32x4 wx, wy;
 #pragma unroll
             for (int c = 0; c < 4; c++) {
                 const int r = 4 * a4 + c;
@@ -251,21 +255,24 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
                 else e = fast_exp2(al[c] + crow);
                 if (diag && (8 * a4 + 4 * h + c > c32)) e = 0.f;
                 if constexpr (MODE == MODE_FWD) {
-                    sacc[r] = product(sacc[r], e);
-                    blk += sacc[r];
-                } else if constexpr (SPLIT) {
-                    sacc[r] = product(fmaf(sacc[r], inv_n, dbv), e);
+                    float& b = PARITY ? bpar[kb] : bsum;
+                    b = fmaf(sacc[r], e, b);
+                    wx[c] = sacc[r];
                 } else {
-                    sacc[r] = (sacc[r] * inv_n + dbv) * e;
+                    wx[c] = fmaf(sacc[r], inv_n, dbv);
                 }
+                wy[c] = e;
+                sacc[r] = wx[c] * e;
+            }
+            if constexpr (STRICT) {
+                R::split_products(wx, wy, w.hi[a4], w.lo[a4]);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
-        if constexpr (MODE == MODE_FWD && SPLIT) bpar[kb] += blk;
-        else if constexpr (MODE == MODE_FWD) bsum += blk;
     };
     // gate weights of a block entirely below the diagonal, factorised: exp2(alpha_j - c0) comes from the pre-pass
     // (sek), exp2(c0 - beta_i + dG) is one exponential per lane and block
-    auto weigh_fact = [&](f32x16& sacc, const float* sek, int kb, Crow crow) {
+    auto weigh_fact = [&](f32x16& sacc, Terms& w, const float* sek, int kb, Crow crow) {
         float er;
         if constexpr (F32) er = fast_exp2((float)((double)(sek[GRAN + kb] + nbeta) + crow));
         else er = fast_exp2(crow + sek[GRAN + kb]);
@@ -273,25 +280,32 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
 #pragma unroll
         for (int a4 = 0; a4 < 4; a4++) {
             const f32x4 ek = *reinterpret_cast<const f32x4*>(sek + 32 * kb + 8 * a4 + 4 * h);
+            f32x4 wx, wy;
 #pragma unroll
             for (int c = 0; c < 4; c++) {
                 const int r = 4 * a4 + c;
                 if constexpr (MODE == MODE_FWD) {
-                    const float t = product(sacc[r], ek[c]);
-                    blk += t;
-                    sacc[r] = product(t, er);
-                } else if constexpr (SPLIT) {
-                    sacc[r] = product(fmaf(sacc[r], inv_n * er, dbv * er), ek[c]);
+                    blk = fmaf(sacc[r], ek[c], blk);
+                    wx[c] = sacc[r] * ek[c];
+                    wy[c] = er;
+                    sacc[r] = wx[c] * er;
+                } else if constexpr (PARITY) {
+                    sacc[r] = fmaf(sacc[r], inv_n * er, dbv * er) * ek[c];
                 } else {
-                    sacc[r] = (sacc[r] * inv_n + dbv) * (ek[c] * er);
+                    wx[c] = fmaf(sacc[r], inv_n, dbv);
+                    wy[c] = ek[c] * er;
+                    sacc[r] = wx[c] * wy[c];
                 }
             }
+            if constexpr (STRICT) R::split_products(wx, wy, w.hi[a4], w.lo[a4]);
         }
-        if constexpr (MODE == MODE_FWD && SPLIT) bpar[kb] = fmaf(blk, er, bpar[kb]);
-        else if constexpr (MODE == MODE_FWD) bsum = fmaf(blk, er, bsum);
+        if constexpr (MODE == MODE_FWD) {
+            float& b = PARITY ? bpar[kb] : bsum;
+            b = fmaf(blk, er, b);
+        }
     };
     // second product: accumulate this key block into the output
-    auto gemm2 = [&](const T* y2, const f32x16& sacc, int kb, auto&& hook) {
+    auto gemm2 = [&](const T* y2, const f32x16& sacc, const Terms& w, int kb, auto&& hook) {
         if constexpr (F32) {
             const typename R::terms p[2] = {R::split(R::from_acc(sacc, 0)), R::split(R::from_acc(sacc, 1))};
             R::template stream<2 * NDB>([&](auto n) { return vrd.read(y2, 32 * kb + KW * (n / NDB), n % NDB); },
@@ -305,7 +319,7 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
         for (int t = 0; t < NSTEP32; t++) {
             hook(kb * NSTEP32 + t, 2 * NSTEP32);
             frag pf, pl;
-            if constexpr (STRICT) R::from_acc_split(sacc, t, pf, pl);
+            if constexpr (STRICT) { pf = terms_of(w.hi, t); pl = terms_of(w.lo, t); }
             else pf = R::from_acc(sacc, t);
             frag vf[NDB];
 #pragma unroll
@@ -332,17 +346,22 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
         constexpr int AH = NS < 4 ? NS : 4;
         f32x16 s0, s1;
         // one accumulator register of a block below the diagonal: see weigh_fact
-        auto weigh_reg = [&](f32x16& sacc, int r, const f32x4 (&ek)[4], float er, float& blk) {
+        auto weigh_reg = [&](f32x16& sacc, Terms& w, int r, const f32x4 (&ek)[4], float er, float& blk) {
             if constexpr (MODE == MODE_FWD) {
-                const float t = product(sacc[r], ek[r >> 2][r & 3]);
-                blk += t;
-                sacc[r] = product(t, er);
-            } else if constexpr (SPLIT) {
-                sacc[r] = product(fmaf(sacc[r], inv_n * er, dbv * er), ek[r >> 2][r & 3]);
+                blk = fmaf(sacc[r], ek[r >> 2][r & 3], blk);
+                sacc[r] *= ek[r >> 2][r & 3];
+                if constexpr (!STRICT) sacc[r] *= er;
+            } else if constexpr (PARITY) {
+                sacc[r] = fmaf(sacc[r], inv_n * er, dbv * er) * ek[r >> 2][r & 3];
             } else {
-                sacc[r] = (sacc[r] * inv_n + dbv) * (ek[r >> 2][r & 3] * er);
+                sacc[r] = fmaf(sacc[r], inv_n, dbv);
+                if constexpr (!STRICT) sacc[r] *= ek[r >> 2][r & 3] * er;
+            }
+            if constexpr (STRICT && MODE == MODE_DQ) {
+                if ((r & 3) == 3) R::split_products(f32x4{sacc[r - 3], sacc[r - 2], sacc[r - 1], sacc[r]}, ek[r >> 2] * er, w.hi[r >> 2], w.lo[r >> 2]);
             }
         };
+        Terms w0, w1;
         f32x4 ek0[4], ek1[4];
 #pragma unroll
         for (int a4 = 0; a4 < 4; a4++) {
@@ -376,7 +395,7 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
             if (s + AH < NS) kr[s + AH] = krd.read(y1, 1, s + AH);
             R::mma(s1, kr[s], xt[s]);
 #pragma unroll
-            for (int r = s * 16 / NS; r < (s + 1) * 16 / NS; r++) weigh_reg(s0, r, ek0, er0, blk0);
+            for (int r = s * 16 / NS; r < (s + 1) * 16 / NS; r++) weigh_reg(s0, w0, r, ek0, er0, blk0);
             __builtin_amdgcn_sched_barrier(0);
         }
         // ---- H += V^T P^T: groups g = 2*kb + t of 16 keys; the weighing of S1 rides on the groups of key block 0
@@ -384,11 +403,20 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
 #pragma unroll
         for (int d = 0; d < NDB; d++) vf[0][d] = vrd.read(y2, 0, d);
         frag pf, pl;
-        auto take_p = [&](const f32x16& sacc, int t) {
-            if constexpr (STRICT) R::from_acc_split(sacc, t, pf, pl);
-            else pf = R::from_acc(sacc, t);
+        auto take_p = [&](const f32x16& sacc, Terms& w, float er, int t) {
+            if constexpr (STRICT) {
+                if constexpr (MODE == MODE_FWD) {
+#pragma unroll
+                    for (int a4 = 2 * t; a4 < 2 * t + 2; a4++)
+                        R::split_products(f32x4{sacc[4 * a4], sacc[4 * a4 + 1], sacc[4 * a4 + 2], sacc[4 * a4 + 3]}, f32x4{er, er, er, er}, w.hi[a4], w.lo[a4]);
+                }
+                pf = terms_of(w.hi, t);
+                pl = terms_of(w.lo, t);
+            } else {
+                pf = R::from_acc(sacc, t);
+            }
         };
-        take_p(s0, 0);
+        take_p(s0, w0, er0, 0);
 #pragma unroll
         for (int g = 0; g < 4; g++) {
             hook2(g, 4);
@@ -399,16 +427,16 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
                 if constexpr (STRICT) R::mma(oacc[d], vf[g & 1][d], pl);
                 if (g < 2) {
 #pragma unroll
-                    for (int r = (g * NDB + d) * 16 / (2 * NDB); r < (g * NDB + d + 1) * 16 / (2 * NDB); r++) weigh_reg(s1, r, ek1, er1, blk1);
+                    for (int r = (g * NDB + d) * 16 / (2 * NDB); r < (g * NDB + d + 1) * 16 / (2 * NDB); r++) weigh_reg(s1, w1, r, ek1, er1, blk1);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
-            if (g == 0) take_p(s0, 1);
-            if (g == 1) take_p(s1, 0);
-            if (g == 2) take_p(s1, 1);
+            if (g == 0) take_p(s0, w0, er0, 1);
+            if (g == 1) take_p(s1, w1, er1, 0);
+            if (g == 2) take_p(s1, w1, er1, 1);
         }
-        if constexpr (MODE == MODE_FWD && SPLIT) { bpar[0] = fmaf(blk0, er0, bpar[0]); bpar[1] = fmaf(blk1, er1, bpar[1]); }
-        else if constexpr (MODE == MODE_FWD) bsum = fmaf(blk1, er1, fmaf(blk0, er0, bsum));
+        if constexpr (MODE == MODE_FWD && PARITY) { bpar[0] = fmaf(blk0, er0, bpar[0]); bpar[1] = fmaf(blk1, er1, bpar[1]); }
+        else if constexpr (MODE == MODE_FWD) bsum += fmaf(blk0, er0, blk1 * er1);
       }
     };
 
@@ -471,7 +499,7 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
         const float* nst = a.Nst + ((size_t)bh * a.n_states + chunk - 1) * D;
         if constexpr (MODE == MODE_FWD) {
             // row sums: decay_i (q_i . n~); the lane's half of the row (the halves meet in the epilogue)
-            if constexpr (SPLIT) {
+            if constexpr (PARITY) {
                 dec_far = dec;
 #pragma unroll
                 for (int s2 = 0; s2 < NS; s2++)
@@ -479,7 +507,7 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
                     for (int e = 0; e < 4; e++) {
                         float& part = bfar[s2 / (NS / 2)];
                         const float* const n8 = nst + KW * s2 + R::EPL * h;
-                        part = fmaf(to_f32(xf[s2][4 + e]), n8[4 + e], fmaf(to_f32(xf[s2][e]), n8[e], part));
+                        part += fmaf(to_f32(xf[s2][e]), n8[e], to_f32(xf[s2][4 + e]) * n8[4 + e]);
                     }
             } else {
                 float part = 0.f;
@@ -496,28 +524,40 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
         } else {
             const float decn = dec * inv_n, rank1 = dec * dbv;
             const T* qrow = reinterpret_cast<const T*>(a.Qrow) + offA + (size_t)rowc * rsA;
-            float rp = 0.f, rp_first = 0.f;   // (summed per block of 32 columns, as mlstm_rowf.hip, which splits a row by columns, has to; split mode: and per half of them)
-#pragma unroll
-            for (int d = 0; d < NDB; d++) {
-                float rpd = 0.f;
+            // (summed per block of 32 columns, as mlstm_rowf.hip, mlstm_roww.hip and mlstm_rowx.hip, which split a row by columns, have to;
+            // 16 bits at D >= 128: and per half of them.  At D = 64 they are one sum.)
+            float rp = 0.f, rp_first = 0.f, rpd = 0.f;
+            f32x4 nv[2][4];   // a column block's values, requested a block ahead (left to the compiler: sixteen loads, each waited for)
+            typename R::vec4 qv[2][4];
+            auto request = [&](int d) {
 #pragma unroll
                 for (int a4 = 0; a4 < 4; a4++) {
-                    const int col = 32 * d + 8 * a4 + 4 * h;
-                    const f32x4 nv = *reinterpret_cast<const f32x4*>(nst + col);
-                    const f32x4 qv = __builtin_convertvector(*reinterpret_cast<const typename R::vec4*>(qrow + col), f32x4);
+                    nv[d & 1][a4] = *reinterpret_cast<const f32x4*>(nst + 32 * d + 8 * a4 + 4 * h);
+                    qv[d & 1][a4] = *reinterpret_cast<const typename R::vec4*>(qrow + 32 * d + 8 * a4 + 4 * h);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            request(0);
+#pragma unroll
+            for (int d = 0; d < NDB; d++) {
+                if (d + 1 < NDB) request(d + 1);
+                if (F32 || FAST_TR) rpd = 0.f;
+#pragma unroll
+                for (int a4 = 0; a4 < 4; a4++) {
+                    const f32x4 q4 = __builtin_convertvector(qv[d & 1][a4], f32x4);
 #pragma unroll
                     for (int c = 0; c < 4; c++) {
-                        const float v = fmaf(oacc[d][4 * a4 + c], decn, rank1 * nv[c]);
+                        const float v = fmaf(rank1, nv[d & 1][a4][c], oacc[d][4 * a4 + c] * decn);
                         oacc[d][4 * a4 + c] = v;
-                        rpd = fmaf(v, qv[c], rpd);
+                        rpd = fmaf(v, q4[c], rpd);
                     }
                 }
-                rp += rpd;
-                if (SPLIT && d == NDB / 2 - 1) { rp_first = rp; rp = 0.f; }
+                if (F32 || FAST_TR || d == NDB - 1) rp += rpd;
+                if (FAST_TR && d == NDB / 2 - 1) { rp_first = rp; rp = 0.f; }
             }
             // row sums of dD over the keys before the chunk: q_i . dQ_i of what the accumulators hold now
             rp = sum_halves(rp);
-            if constexpr (SPLIT) rp = sum_halves(rp_first) + rp;
+            if constexpr (FAST_TR) rp = sum_halves(rp_first) + rp;
             if (row < S && h == 0) a.rowinter[hoff + row] = rp;
         }
     } else {
@@ -561,10 +601,11 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
         } else {
             f32x16 s0, s1;
             gemm1x2(y1, s0, s1, hook1);
-            weigh_fact(s0, sal + GRAN, 0, crow);
-            gemm2(y2, s0, 0, hook2);
-            weigh_fact(s1, sal + GRAN, 1, crow);
-            gemm2(y2, s1, 1, hook2);
+            Terms w;
+            weigh_fact(s0, w, sal + GRAN, 0, crow);
+            gemm2(y2, s0, w, 0, hook2);
+            weigh_fact(s1, w, sal + GRAN, 1, crow);
+            gemm2(y2, s1, w, 1, hook2);
         }
     }
     for (; j < jfull; j++) {
@@ -584,10 +625,11 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
         } else {
             f32x16 s0, s1;
             gemm1x2(y1, s0, s1, no_hook);
-            weigh_fact(s0, sal + GRAN, 0, crow);
-            gemm2(y2, s0, 0, no_hook);
-            weigh_fact(s1, sal + GRAN, 1, crow);
-            gemm2(y2, s1, 1, no_hook);
+            Terms w;
+            weigh_fact(s0, w, sal + GRAN, 0, crow);
+            gemm2(y2, s0, w, 0, no_hook);
+            weigh_fact(s1, w, sal + GRAN, 1, crow);
+            gemm2(y2, s1, w, 1, no_hook);
         }
     }
     for (; j < nJ; j++) {
@@ -609,9 +651,10 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
             if (kstart <= r0) {
                 f32x16 s0;
                 gemm1(y1, kb, s0);
-                if (SPLIT && kstart < r0) weigh_fact(s0, sal + GRAN, kb, crow);
-                else weigh(s0, sal, kb, crow, kstart == r0);
-                gemm2(y2, s0, kb, no_hook);
+                Terms w;
+                if (PARITY && kstart < r0) weigh_fact(s0, w, sal + GRAN, kb, crow);
+                else weigh(s0, w, sal, kb, crow, kstart == r0);
+                gemm2(y2, s0, w, kb, no_hook);
             }
         }
     }
@@ -621,7 +664,7 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
 #undef ST_AL
     float onorm = 1.0f, brow = 0.f;
     if constexpr (MODE == MODE_FWD) {
-        if constexpr (SPLIT) {
+        if constexpr (PARITY) {
             if (chunk > 0) { bpar[0] = fmaf(bfar[0], dec_far, bpar[0]); bpar[1] = fmaf(bfar[1], dec_far, bpar[1]); }
             brow = sum_halves(bpar[0]) + sum_halves(bpar[1]);
         } else {
@@ -658,7 +701,7 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
             for (int a4 = 0; a4 < 4; a4++) {
                 f32x4 v;
 #pragma unroll
-                for (int c = 0; c < 4; c++) v[c] = product(oacc[d][4 * a4 + c], onorm);
+                for (int c = 0; c < 4; c++) v[c] = STRICT ? rounded_product(oacc[d][4 * a4 + c], onorm) : oacc[d][4 * a4 + c] * onorm;
                 if constexpr (STRICT && MODE == MODE_FWD) {
                     typename R::vec4 hi, lo;
                     R::cvt4_split(v, hi, lo);
@@ -679,7 +722,7 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
                         const int col = 32 * d + 8 * a4 + 4 * h;
                         const f32x4 of = __builtin_convertvector(*reinterpret_cast<const typename R::vec4*>(og + col), f32x4);
                         f32x4 v;
-                        if constexpr (SPLIT && !STRICT) {   // (from h as it is written, like the other row kernels)
+                        if constexpr (PARITY) {   // (from h as it is written, like the other row kernels)
 #pragma unroll
                             for (int c = 0; c < 4; c++) v[c] = oacc[d][4 * a4 + c] * onorm;
                             *reinterpret_cast<typename R::vec4*>(outg + col) = gate4<T>(R::cvt4(v), *reinterpret_cast<const typename R::vec4*>(og + col));

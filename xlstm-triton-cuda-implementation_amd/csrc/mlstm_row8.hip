@@ -305,7 +305,6 @@ __global__ __launch_bounds__(512) void row8_kernel(RowArgs a) {
                 if constexpr (MODE == R8_FWD) bs = fmaf(blk, er, bs);
                 return;
             }
-            float blk = 0.f;
 #pragma unroll
             for (int a4 = 0; a4 < 4; a4++) {
                 const f32x4 al = *reinterpret_cast<const f32x4*>(sal + 32 * kh + 8 * a4 + 4 * h);
@@ -315,14 +314,13 @@ __global__ __launch_bounds__(512) void row8_kernel(RowArgs a) {
                     float e = fast_exp2(al[c] + crow);
                     if (8 * a4 + 4 * h + c > c32) e = 0.f;
                     if constexpr (MODE == R8_FWD) {
+                        bs = fmaf(sacc[x], e, bs);
                         sacc[x] *= e;
-                        blk += sacc[x];
                     } else {
                         sacc[x] = (sacc[x] * invn + dbr) * e;
                     }
                 }
             }
-            if constexpr (MODE == R8_FWD) bs += blk;
         };
         // hand the fragments of tile j to the consumers of the same rows; they have copied tile j-1's long ago
         bool expired = false;
@@ -467,7 +465,7 @@ __global__ __launch_bounds__(512) void row8_kernel(RowArgs a) {
                         for (int r = 0; r < 2; r++) {
                             const f32x8 qv = __builtin_convertvector(xf[r][s], f32x8);
 #pragma unroll
-                            for (int e = 0; e < 4; e++) part[r] = fmaf(qv[4 + e], n1[e], fmaf(qv[e], n0[e], part[r]));
+                            for (int e = 0; e < 4; e++) part[r] += fmaf(qv[e], n0[e], qv[4 + e] * n1[e]);
                         }
                     }
                 };
@@ -673,7 +671,7 @@ __global__ __launch_bounds__(512) void row8_kernel(RowArgs a) {
 #pragma unroll
                         for (int c = 0; c < 4; c++) {
                             if constexpr (MODE == R8_FWD) oacc[r][d][4 * a4 + c] *= dec;
-                            else oacc[r][d][4 * a4 + c] = fmaf(oacc[r][d][4 * a4 + c], dec, rank1 * nv[c]);
+                            else oacc[r][d][4 * a4 + c] = fmaf(rank1, nv[c], oacc[r][d][4 * a4 + c] * dec);
                         }
                     }
             }

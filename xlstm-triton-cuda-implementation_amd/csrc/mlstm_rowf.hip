@@ -23,7 +23,8 @@ struct RowfCfg {
     static constexpr int ROWS = 32, KEYS = 128;
     static constexpr size_t X_BYTES = (size_t)ROWS * D * 4, K_BYTES = (size_t)KEYS * D * 4;
     static constexpr size_t P_BYTES = 4 * 2 * 3 * 64 * 16;   // [key block][16 keys][term][lane] x 16 B
-    static constexpr size_t LDS_BYTES = X_BYTES + K_BYTES + P_BYTES + (4 * 64 * 2 + 32 * 2 + 4 * 64 + 4 + D) * sizeof(float);
+    static constexpr size_t HAND_BYTES = 2 * 16 * 64 * 8;     // forward: [key block of the rows' granule][register][lane] x {product, weight}
+    static constexpr size_t LDS_BYTES = X_BYTES + K_BYTES + P_BYTES + HAND_BYTES + (4 * 64 * 2 + 32 * 2 + 4 * 64 + 4 + D) * sizeof(float);
 };
 
 template <int D, int MODE>
@@ -37,7 +38,8 @@ __global__ __launch_bounds__(256, 1) void rowf_kernel(RowArgs a) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     T* const xtile = reinterpret_cast<T*>(smem);
     char* const pbuf = smem + Cfg::X_BYTES + Cfg::K_BYTES;
-    float* const part = reinterpret_cast<float*>(pbuf + Cfg::P_BYTES);   // [key block][lane] x {sum, row factor}
+    float2* const hand = reinterpret_cast<float2*>(pbuf + Cfg::P_BYTES);
+    float* const part = reinterpret_cast<float*>(pbuf + Cfg::P_BYTES + Cfg::HAND_BYTES);   // [key block][lane] x {sum, row factor}
     float* const stat = part + 4 * 64 * 2;                               // [row] x {1/n, db}; then (forward) {1/n, b}
     float* const rix = stat + 32 * 2;                                    // [column block][lane]
     unsigned* const bads = reinterpret_cast<unsigned*>(rix + 4 * 64);    // [wave]
@@ -79,6 +81,7 @@ __global__ __launch_bounds__(256, 1) void rowf_kernel(RowArgs a) {
     const T* Y1 = reinterpret_cast<const T*>(a.Y1) + offA;
     const T* Y2 = reinterpret_cast<const T*>(a.Y2) + offA;
     const bool second = wave < NCB;   // the wave has a column block
+    constexpr int SUMS = 3;           // the wave of the row sums (D = 64: it has none)
     const int col = 32 * wave + c32;
 
     // ---- requests: the rows' operand, the wave's first key block, its columns of the state and of the first keys
@@ -166,7 +169,7 @@ __global__ __launch_bounds__(256, 1) void rowf_kernel(RowArgs a) {
                                    [&](auto n, const auto& c, auto&& between) { R::mma_between(acc, c, xt[n], between); });
         }
         if constexpr (MODE == ROW_MODE_FWD) {
-            if (wave == 0) {
+            if (wave == SUMS) {
                 float pt = 0.f;
 #pragma unroll
                 for (int s = 0; s < NS; s++)
@@ -186,7 +189,7 @@ __global__ __launch_bounds__(256, 1) void rowf_kernel(RowArgs a) {
                 const f32x4 nv = *reinterpret_cast<const f32x4*>(nvl + c0), qv = *reinterpret_cast<const f32x4*>(qrow + c0);
 #pragma unroll
                 for (int c = 0; c < 4; c++) {
-                    acc[4 * a4 + c] = fmaf(acc[4 * a4 + c], decn, rank1 * nv[c]);
+                    acc[4 * a4 + c] = fmaf(rank1, nv[c], acc[4 * a4 + c] * decn);
                     rp = fmaf(acc[4 * a4 + c], qv[c], rp);
                 }
             }
@@ -221,9 +224,8 @@ __global__ __launch_bounds__(256, 1) void rowf_kernel(RowArgs a) {
                 for (int x = 0; x < 16; x++) {
                     const float ek = wk[x >> 2][x & 3];
                     if constexpr (MODE == ROW_MODE_FWD) {
-                        const float t = s[x] * ek;
-                        blk += t;
-                        s[x] = t * er;
+                        blk = fmaf(s[x], ek, blk);
+                        s[x] = (s[x] * ek) * er;
                     } else {
                         s[x] = (s[x] * inv_n + dbv) * (ek * er);
                     }
@@ -234,8 +236,8 @@ __global__ __launch_bounds__(256, 1) void rowf_kernel(RowArgs a) {
                     float e = fast_exp2((wk[x >> 2][x & 3] + nbeta) + (float)crow);
                     if (k0 == r0 && 8 * (x >> 2) + 4 * h + (x & 3) > c32) e = 0.f;
                     if constexpr (MODE == ROW_MODE_FWD) {
+                        hand[((kb & 1) * 16 + x) * 64 + lane] = make_float2(s[x], e);
                         s[x] *= e;
-                        blk += s[x];
                     } else {
                         s[x] = (s[x] * inv_n + dbv) * e;
                     }
@@ -251,11 +253,14 @@ __global__ __launch_bounds__(256, 1) void rowf_kernel(RowArgs a) {
         }
         __syncthreads();
         const int nb = nkb - 4 * r < 4 ? nkb - 4 * r : 4;   // key blocks of this round
+        float2 be[4], own[32];
         if constexpr (MODE == ROW_MODE_FWD) {
-            if (wave == 0) {
-                for (int t = 0; t < nb; t++) {
-                    const float2 be = *reinterpret_cast<const float2*>(part + (t * 64 + lane) * 2);
-                    bsum = fmaf(be.x, be.y, bsum);
+            if (wave == SUMS) {   // (requested ahead of the products, added up behind them)
+#pragma unroll
+                for (int t = 0; t < 4; t++) be[t] = *reinterpret_cast<const float2*>(part + (t * 64 + lane) * 2);
+                if (r == nR - 1) {
+#pragma unroll
+                    for (int x = 0; x < 32; x++) own[x] = hand[x * 64 + lane];
                 }
             }
         }
@@ -275,10 +280,28 @@ __global__ __launch_bounds__(256, 1) void rowf_kernel(RowArgs a) {
             }
             if (r + 1 < nR) load_v(r + 1);
         }
+        if constexpr (MODE == ROW_MODE_FWD) {
+            if (wave == SUMS) {
+                const int before = r0 / GRAN * 2 - 4 * r;   // the round's key blocks before the rows' own granule
+#pragma unroll
+                for (int t = 0; t < 4; t++) {
+                    if (t < before) bsum = fmaf(be[t].x, be[t].y, bsum);
+                }
+                // the own granule's element by element onto the sum over the keys before it, as a wave of row_kernel does that holds all of them
+                if (r == nR - 1) {
+#pragma unroll
+                    for (int x = 0; x < 16; x++) bsum = fmaf(own[x].x, own[x].y, bsum);
+                    if (rt & 1) {
+#pragma unroll
+                        for (int x = 16; x < 32; x++) bsum = fmaf(own[x].x, own[x].y, bsum);
+                    }
+                }
+            }
+        }
     }
     // ---- epilogue: the normaliser, rows that are not finite from their definition (see not_finite), the wave's columns
     float seen = 0.f;
-    if (MODE == ROW_MODE_FWD && wave == 0) {
+    if (MODE == ROW_MODE_FWD && wave == SUMS) {
         const float b = sum_halves(bsum);
         seen = not_finite(seen, b);
         const float n = fmaxf(fabsf(b), __expf(-m_row)) + 1e-6f;
@@ -287,7 +310,7 @@ __global__ __launch_bounds__(256, 1) void rowf_kernel(RowArgs a) {
 #pragma unroll
     for (int x = 0; x < 16; x++) seen = not_finite(seen, acc[x]);
     {
-        const unsigned long long halves = __ballot(second && row < S && seen != 0.f);
+        const unsigned long long halves = __ballot((second || wave == SUMS) && row < S && seen != 0.f);
         if (lane == 0) bads[wave] = (unsigned)halves | (unsigned)(halves >> 32);
     }
     __syncthreads();

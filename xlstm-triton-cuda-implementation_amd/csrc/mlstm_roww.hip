@@ -251,7 +251,7 @@ __global__ __launch_bounds__(512) void roww_kernel(RowArgs a) {
                     const f32x4 qv = __builtin_convertvector(*reinterpret_cast<const typename R::vec4*>(qrow + col), f32x4);
 #pragma unroll
                     for (int e = 0; e < 4; e++) {
-                        acc[c][4 * a4 + e] = fmaf(acc[c][4 * a4 + e], decn, rank1 * nv[e]);
+                        acc[c][4 * a4 + e] = fmaf(rank1, nv[e], acc[c][4 * a4 + e] * decn);
                         rp = fmaf(acc[c][4 * a4 + e], qv[e], rp);
                     }
                 }
@@ -318,9 +318,8 @@ __global__ __launch_bounds__(512) void roww_kernel(RowArgs a) {
                     for (int c = 0; c < 4; c++) {
                         const int x = 4 * a4 + c;
                         if constexpr (MODE == RW_FWD) {
-                            const float t = s[x] * ek[c];
-                            blk += t;
-                            s[x] = t * er;
+                            blk = fmaf(s[x], ek[c], blk);
+                            s[x] = (s[x] * ek[c]) * er;
                         } else {
                             s[x] = (s[x] * sc + of) * ek[c];
                         }
@@ -336,14 +335,12 @@ __global__ __launch_bounds__(512) void roww_kernel(RowArgs a) {
                         float e = fast_exp2(al[c] + crow);
                         if (8 * a4 + 4 * h + c > c32) e = 0.f;
                         if constexpr (MODE == RW_FWD) {
-                            s[x] *= e;
-                            blk += s[x];
+                            s[x] *= e;     // (its share of the row sums: behind the loop)
                         } else {
                             s[x] = (s[x] * inv_n + dbv) * e;
                         }
                     }
                 }
-                er = 1.f;
             }
             frag* const p = pbuf + (kb * 2 + rb) * 2 * 64 + lane;
             p[0] = R::from_acc(s, 0);
@@ -357,7 +354,7 @@ __global__ __launch_bounds__(512) void roww_kernel(RowArgs a) {
         if constexpr (NST == 1) dma_wait();
         __syncthreads();
         if constexpr (MODE == RW_FWD) {
-            if (kb < 2) {
+            if (kb < 2) {   // (a block on the diagonal or above it has left zeros)
 #pragma unroll
                 for (int t = 0; t < 2; t++)
                     if (t == 0 || two) {
@@ -377,6 +374,30 @@ __global__ __launch_bounds__(512) void roww_kernel(RowArgs a) {
         if (spread2) chain(Eight{}, y2, weights, [&](auto g) { copy_piece(Y1, y1_at(r + 1, 0), y1_at(r + 1, 1), 2 * r + 2, decltype(g)::value); });
         else if (two) chain(Eight{}, y2, weights, none);
         else chain(Four{}, y2, weights, none);
+    }
+    if constexpr (MODE == RW_FWD) {
+        // The elements of the block on the diagonal go one by one onto the sum over the blocks before it.  They are formed once more here, where
+        // that sum is, from tiles that are still in LDS: kept from phase 1 on, products and weights cost 64 moves in every round, and the
+        // kernel 1 us of 11 (640 x 128).
+        if (kb == rb) {
+            const T* const y1 = y1_at(nR - 1, (nJ - 1) & 1);
+            f32x16 s;
+#pragma unroll
+            for (int x = 0; x < 16; x++) s[x] = 0.f;
+#pragma unroll
+            for (int n = 0; n < NS; n++) R::mma(s, rrd.read(y1, rb, n), xf[n]);
+            const float crow = crow_base + sdg[qt];
+#pragma unroll
+            for (int a4 = 0; a4 < 4; a4++) {
+                const f32x4 al = *reinterpret_cast<const f32x4*>(sal + r0 + 32 * rb + 8 * a4 + 4 * h);
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    float e = fast_exp2(al[c] + crow);
+                    if (8 * a4 + 4 * h + c > c32) e = 0.f;
+                    bsum = fmaf(s[4 * a4 + c], e, bsum);
+                }
+            }
+        }
     }
     // ---- epilogue
     uint4 og[D / 64];   // output gate: this thread's pieces, requested ahead of the barriers
@@ -402,7 +423,7 @@ __global__ __launch_bounds__(512) void roww_kernel(RowArgs a) {
                         const f32x4 n0 = *reinterpret_cast<const f32x4*>(nst + KW * s), n1 = *reinterpret_cast<const f32x4*>(nst + KW * s + 4);
                         const f32x8 qv = __builtin_convertvector(xf[s], f32x8);
 #pragma unroll
-                        for (int e = 0; e < 4; e++) pt = fmaf(qv[4 + e], n1[e], fmaf(qv[e], n0[e], pt));
+                        for (int e = 0; e < 4; e++) pt += fmaf(qv[e], n0[e], qv[4 + e] * n1[e]);
                     }
                 };
                 if (kb == 0) half_dot(std::integral_constant<int, 0>{});

@@ -5,7 +5,7 @@
 // row_kernel gives a wave 32 rows with all of their work: 3 us per 64 keys at D = 256, with half the chip idle at 96 workgroups.  A
 // workgroup here owns one granule of 64 rows; its walk is a pipeline of 64-key tiles with one barrier per tile:
 //   step v      four producer waves, (row block of 32, key block of 32):  S^T = K Q^T (dQ pass: dC^T = V dH^T) of tile v, gate weights, the
-//               weights' two terms to LDS; the row sums stay in their registers;
+//               weights' two terms to LDS; the row sums go from wave to wave, one sum per row;
 //   step v + 1  four consumer waves, (row block, half of the columns):  H^T += V^T P^T (dQ^T += K^T G^T), both terms.
 // The state of the previous chunk goes through the consumers first, while the producers are at tile 0.  A step takes 2300 cycles at D = 256:
 // the 64 KB of a tile pair at what a CU gets out of L2 with all of them asking, 26 bytes per cycle.  (The form without terms, measured on
@@ -28,7 +28,7 @@ struct RowxCfg {
     static constexpr size_t POOL_BYTES = 2 * NB * TILE_BYTES;
     static constexpr size_t BLOCK_BYTES = 2 * 2 * 64 * 16, P_BYTES = 4 * BLOCK_BYTES;   // [key block][row block][16 keys][hi, lo][lane]; one buffer (two and the tiles are all of LDS)
     static constexpr int E_ROWS = 32, NE = D / E_ROWS;                 // the state in pieces of a tile's size, hi, then lo
-    static constexpr size_t MISC_FLOATS = 2 * 2 * 32 + 2 * 2 * 32 + 2 * 32 * 2 + D + RX_MOST_KEYS / GRAN;   // row sums, far row sums, 1/n and db, vector state, granule distances
+    static constexpr size_t MISC_FLOATS = 2 * 64 * 2 + 2 * 32 + 2 * 2 * 32 + 2 * 32 * 2 + D + RX_MOST_KEYS / GRAN;   // what producers hand over, row sums, far row sums, 1/n and db, vector state, granule distances
     static size_t lds_bytes(int keys) { return POOL_BYTES + P_BYTES + MISC_FLOATS * 4 + (size_t)keys * 8 + GRAN * 4; }
 };
 
@@ -42,8 +42,9 @@ __global__ __launch_bounds__(512) void rowx_kernel(RowArgs a) {
     constexpr int KW = R::KW, NS = D / KW, NC = D / 64, NB = Cfg::NB, AHEAD = Cfg::AHEAD;   // NC: column blocks of a consumer
     extern __shared__ __attribute__((aligned(16))) char smem[];
     char* const pbuf = smem + Cfg::POOL_BYTES;
-    float* const bex = reinterpret_cast<float*>(pbuf + Cfg::P_BYTES);   // [rb][kb][32]
-    float* const rpx = bex + 2 * 2 * 32;                   // [rb][column half][32]
+    float* const handed = reinterpret_cast<float*>(pbuf + Cfg::P_BYTES);   // [rb][lane] x {sum, row factor} of the second key block; then {row sum so far}
+    float* const bex = handed + 2 * 64 * 2;                // [rb][32]
+    float* const rpx = bex + 2 * 32;                       // [rb][column half][32]
     float* const stat = rpx + 2 * 2 * 32;                  // [rb][32] x {1/n, db}
     float* const nvl = stat + 2 * 32 * 2;                  // [D]
     float* const sdg = nvl + D;                            // granule of the rows minus granule j
@@ -208,12 +209,26 @@ __global__ __launch_bounds__(512) void rowx_kernel(RowArgs a) {
         for (int s = 0; s < NS; s++) pin(xf[s]);
         __syncthreads();   // X's tile is free; the rows' scalars are there
         row_scalars();
-        float bsum = 0.f;   // the row sums over the key blocks of parity kb, in the order of the keys
+        // Row sums: one sum per row in the order of the keys, the state part first, as a wave of row_kernel keeps it.  The waves of the first key
+        // blocks have it; the others hand their blocks' shares to them, a tile behind, and take it over for the block on the diagonal.
+        float bsum = 0.f, blk_was = 0.f, er_was = 0.f;
+        float* const mine = handed + (rb * 64 + lane) * 2;
+        float s_own[16], e_own[16];   // products and weights of the rows' own granule
+        auto add_own = [&] {
+#pragma unroll
+            for (int x = 0; x < 16; x++) bsum = fmaf(s_own[x], e_own[x], bsum);
+        };
         auto weigh_tile = [&](int j) __attribute__((always_inline)) {
             f32x16 s;
             const int k0 = GRAN * j + 32 * kb, rr = r0 + 32 * rb;
             const T* const y1 = y1_at(j);
             const float crow = crow_base + sdg[j];
+            if constexpr (MODE == RX_FWD) {
+                if (kb == 0 && j > 0) {   // the tile before this one
+                    const float2 other = *reinterpret_cast<const float2*>(mine);
+                    bsum += fmaf(blk_was, er_was, other.x * other.y);
+                }
+            }
             constexpr int PRE = 4;
             frag kf[NS];
 #pragma unroll
@@ -227,14 +242,15 @@ __global__ __launch_bounds__(512) void rowx_kernel(RowArgs a) {
                 __builtin_amdgcn_sched_barrier(0);
                 if (n == NS / 2 && j > 0) __syncthreads();   // (the consumers have read the tile before)
             }
-            // (products that enter the low-order terms or a sum are rounded first: see rounded_product)
+            // The weights as factors x y, of which the low-order terms take what rounding the product would lose
             float blk = 0.f, er = 0.f;
+            f32x4 wx, wy;
+            typename R::vec4 hi[4], lo[4];
             if (k0 > rr) {             // above the diagonal
 #pragma unroll
-                for (int x = 0; x < 16; x++) s[x] = 0.f;
-            } else if (k0 < rr) {      // below it: factorised weights
+                for (int a4 = 0; a4 < 4; a4++) hi[a4] = lo[a4] = typename R::vec4{};
+            } else if (j < nJ - 1) {   // factorised weights, as long as the keys' granule lies before the rows'
                 er = fast_exp2(crow + sam[k0 / 32]);
-                const float sc = inv_n * er, of = dbv * er;
 #pragma unroll
                 for (int a4 = 0; a4 < 4; a4++) {
                     const f32x4 ek = *reinterpret_cast<const f32x4*>(sek + k0 + 8 * a4 + 4 * h);
@@ -242,15 +258,17 @@ __global__ __launch_bounds__(512) void rowx_kernel(RowArgs a) {
                     for (int c = 0; c < 4; c++) {
                         const int x = 4 * a4 + c;
                         if constexpr (MODE == RX_FWD) {
-                            const float t = rounded_product(s[x], ek[c]);
-                            blk += t;
-                            s[x] = rounded_product(t, er);
+                            blk = fmaf(s[x], ek[c], blk);
+                            wx[c] = s[x] * ek[c];
+                            wy[c] = er;
                         } else {
-                            s[x] = rounded_product(fmaf(s[x], sc, of), ek[c]);
+                            wx[c] = fmaf(s[x], inv_n, dbv);
+                            wy[c] = ek[c] * er;
                         }
                     }
+                    R::split_products(wx, wy, hi[a4], lo[a4]);
                 }
-            } else {                   // on it
+            } else {                   // the rows' own granule, on the diagonal or below it
 #pragma unroll
                 for (int a4 = 0; a4 < 4; a4++) {
                     const f32x4 al = *reinterpret_cast<const f32x4*>(sal + k0 + 8 * a4 + 4 * h);
@@ -258,35 +276,52 @@ __global__ __launch_bounds__(512) void rowx_kernel(RowArgs a) {
                     for (int c = 0; c < 4; c++) {
                         const int x = 4 * a4 + c;
                         float e = fast_exp2(al[c] + crow);
-                        if (8 * a4 + 4 * h + c > c32) e = 0.f;
+                        if (k0 == rr && 8 * a4 + 4 * h + c > c32) e = 0.f;
                         if constexpr (MODE == RX_FWD) {
-                            s[x] = rounded_product(s[x], e);
-                            blk += s[x];
+                            wx[c] = s[x];
+                            s_own[x] = s[x];
+                            e_own[x] = e;
                         } else {
-                            s[x] = rounded_product(fmaf(s[x], inv_n, dbv), e);
+                            wx[c] = fmaf(s[x], inv_n, dbv);
                         }
+                        wy[c] = e;
                     }
+                    R::split_products(wx, wy, hi[a4], lo[a4]);
                 }
-                er = 1.f;
             }
             frag* const p = reinterpret_cast<frag*>(p_block(kb)) + lane;
 #pragma unroll
             for (int t = 0; t < 2; t++) {
-                frag hi, lo;
-                R::from_acc_split(s, t, hi, lo);
-                p[128 * t] = hi;
-                p[128 * t + 64] = lo;
+                p[128 * t] = __builtin_shufflevector(hi[2 * t], hi[2 * t + 1], 0, 1, 2, 3, 4, 5, 6, 7);
+                p[128 * t + 64] = __builtin_shufflevector(lo[2 * t], lo[2 * t + 1], 0, 1, 2, 3, 4, 5, 6, 7);
             }
-            if constexpr (MODE == RX_FWD) bsum = fmaf(blk, er, bsum);
+            if constexpr (MODE == RX_FWD) {
+                blk_was = blk;
+                er_was = er;
+                if (kb == 1 && j < nJ - 1) *reinterpret_cast<float2*>(mine) = make_float2(blk, er);
+            }
         };
         weigh_tile(0);
         if (chunk > 0) {
+            float pt = 0.f;   // q . n~ of what lies before the chunk, a piece at a time
 #pragma unroll
             for (int n = 0; n < Cfg::NE; n++) {
                 state_wait(n);
                 __syncthreads();
                 if (D == 256) piece(n + 3);
+                if constexpr (MODE == RX_FWD) {
+                    if (kb == 0) {
+#pragma unroll
+                        for (int s = NS / Cfg::NE * n; s < NS / Cfg::NE * (n + 1); s++) {
+                            const f32x4 n0 = *reinterpret_cast<const f32x4*>(nvl + 8 * h + KW * s), n1 = *reinterpret_cast<const f32x4*>(nvl + 8 * h + KW * s + 4);
+                            const f32x8 qv = __builtin_convertvector(xf[s], f32x8);
+#pragma unroll
+                            for (int e = 0; e < 8; e++) pt = fmaf(qv[e], e < 4 ? n0[e] : n1[e - 4], pt);
+                        }
+                    }
+                }
             }
+            bsum = dec * pt;
         } else {
             __syncthreads();
         }
@@ -294,29 +329,24 @@ __global__ __launch_bounds__(512) void rowx_kernel(RowArgs a) {
             weigh_tile(v);
             __syncthreads();
         }
-        __syncthreads();
+        if constexpr (MODE == RX_FWD) {
+            if (kb == 0) {
+                add_own();
+                if (rb == 1) mine[0] = bsum;
+            }
+        }
         __syncthreads();
         if constexpr (MODE == RX_FWD) {
-            if (chunk > 0) {   // what lies before the chunk: decay (q . n~), half of the contraction each
-                const float* nst = nvl + 8 * h;
-                float pt = 0.f;
-                auto half_dot = [&](auto first_tag) {
-                    constexpr int S0 = decltype(first_tag)::value;
-#pragma unroll
-                    for (int s = S0; s < S0 + NS / 2; s++) {
-                        const f32x4 n0 = *reinterpret_cast<const f32x4*>(nst + KW * s), n1 = *reinterpret_cast<const f32x4*>(nst + KW * s + 4);
-                        const f32x8 qv = __builtin_convertvector(xf[s], f32x8);
-#pragma unroll
-                        for (int e = 0; e < 4; e++) pt = fmaf(qv[4 + e], n1[e], fmaf(qv[e], n0[e], pt));
-                    }
-                };
-                if (kb == 0) half_dot(std::integral_constant<int, 0>{});
-                else half_dot(std::integral_constant<int, NS / 2>{});
-                bsum = fmaf(pt, dec, bsum);
+            if (kb == rb) {
+                if (kb == 1) {   // the block on the diagonal, onto what the first block's wave has
+                    bsum = mine[0];
+                    add_own();
+                }
+                const float b = sum_halves(bsum);
+                if (h == 0) bex[rb * 32 + c32] = b;
             }
-            const float b = sum_halves(bsum);
-            if (h == 0) bex[(rb * 2 + kb) * 32 + c32] = b;
         }
+        __syncthreads();
     } else {
         dma_wait();
         __syncthreads();
@@ -399,7 +429,7 @@ __global__ __launch_bounds__(512) void rowx_kernel(RowArgs a) {
                         const f32x4 qv = __builtin_convertvector(*reinterpret_cast<const typename R::vec4*>(qrow + col), f32x4);
 #pragma unroll
                         for (int e = 0; e < 4; e++) {
-                            acc[c][4 * a4 + e] = fmaf(acc[c][4 * a4 + e], decn, rank1 * nv[e]);
+                            acc[c][4 * a4 + e] = fmaf(rank1, nv[e], acc[c][4 * a4 + e] * decn);
                             rp = fmaf(acc[c][4 * a4 + e], qv[e], rp);
                         }
                     }
@@ -458,7 +488,7 @@ __global__ __launch_bounds__(512) void rowx_kernel(RowArgs a) {
     constexpr int CPR = D * (int)sizeof(T) / 16, RB = D * (int)sizeof(T) + 16, NP = 64 * CPR / 512;
     __syncthreads();   // the row sums are there; every wave is done with the pool
     if constexpr (MODE == RX_FWD) {
-        const float b = bex[(rb * 2 + 0) * 32 + c32] + bex[(rb * 2 + 1) * 32 + c32];
+        const float b = bex[rb * 32 + c32];
         onorm = 1.0f / (fmaxf(fabsf(b), __expf(-m_row)) + 1e-6f);
         if (producer && kb == 0 && h == 0 && row < S) a.Bsum[hoff + row] = b;
     } else {
