@@ -51,3 +51,10 @@ def copies_of(case, many):   # one head: the kernels for few workgroups; more th
 @pytest.mark.parametrize("case", sorted(GOLDEN))
 def test_row_pass(case, many):
     check(case, ("b", "h", "dq"), copies_of(case, many))
+
+
+# fp32 and D = 64: col_kernel and colf_kernel; the products of dD enter the row sums unrounded
+@pytest.mark.parametrize("many", [False, True])
+@pytest.mark.parametrize("case", [c for c in sorted(GOLDEN) if "f32" in c or c.endswith("D64")])
+def test_column_pass_of_fp32_and_of_head_dimension_64(case, many):
+    check(case, [n for n in ("dk", "dv", "di", "df") if n in GOLDEN[case]], copies_of(case, many))

@@ -420,14 +420,15 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
             const float inv_er = inv * er, dbv_er = dbv * er;
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-#pragma clang fp contract(off)   // (dD is rounded before it is added anywhere: mlstm_colf.hip hands it from wave to wave)
+                // dD: the column sums add it up as it is rounded (mlstm_colf.hip hands it from wave to wave), the row sums before it is
                 float dd;
                 if constexpr (FIRST) {
                     float e = fast_exp2(F32 ? (al[r] + nbeta) + (float)crow : al[r] + (float)crow);
                     if (!qvalid || (diag && (8 * (r >> 2) + 4 * h + (r & 3) > c32))) e = 0.f;
                     const float ct = sacc[r] * e;
                     const float dct = fmaf(dacc[r], inv, dbv);
-                    dd = ct * dct;
+                    dd = product_apart(ct, dct);
+                    rsum = fmaf(ct, dct, rsum);
                     g[r] = dct * e;
                     w[r] = ct * inv;
                 } else {
@@ -435,9 +436,9 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
                     const float sk = sacc[r] * ekr[r];
                     g[r] = dct_er * ekr[r];
                     w[r] = sk * inv_er;
-                    dd = sk * dct_er;
+                    dd = product_apart(sk, dct_er);
+                    rsum = fmaf(sk, dct_er, rsum);
                 }
-                rsum += dd;
                 colacc[r] += dd;
             }
         } else {

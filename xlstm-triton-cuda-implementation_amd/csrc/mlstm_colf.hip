@@ -239,13 +239,13 @@ __global__ __launch_bounds__(256, 1) void colf_kernel(ColArgs a) {
             const float er = !qvalid ? 0.f : fast_exp2((float)((double)(amaxA + nbeta) + crow));
             const float inv_er = inv * er, dbv_er = dbv * er;
             auto element = [&](auto first_tag, int x) __attribute__((always_inline)) {
-#pragma clang fp contract(off)   // (as in col_kernel)
                 if constexpr (decltype(first_tag)::value) {
                     float e = fast_exp2((al[x] + nbeta) + (float)crow);
                     if (!qvalid || (diag && (8 * (x >> 2) + 4 * h + (x & 3) > c32))) e = 0.f;
                     const float ct = s[x] * e;
                     const float dct = fmaf(d[x], inv, dbv);
-                    dd[x] = ct * dct;
+                    dd[x] = product_apart(ct, dct);   // (as in col_kernel)
+                    rsum = fmaf(ct, dct, rsum);
                     g[x] = dct * e;
                     w[x] = ct * inv;
                 } else {
@@ -253,9 +253,9 @@ __global__ __launch_bounds__(256, 1) void colf_kernel(ColArgs a) {
                     const float sk = s[x] * ekr[x];
                     g[x] = dct_er * ekr[x];
                     w[x] = sk * inv_er;
-                    dd[x] = sk * dct_er;
+                    dd[x] = product_apart(sk, dct_er);
+                    rsum = fmaf(sk, dct_er, rsum);
                 }
-                rsum += dd[x];
             };
             if (first) {
 #pragma unroll

@@ -710,6 +710,11 @@ __device__ __forceinline__ float rounded_product(float a, float b) {
     asm("" : "+v"(p));
     return p;
 }
+// The same where nothing but the compiler's own contraction is to be kept out.
+__device__ __forceinline__ float product_apart(float a, float b) {
+#pragma clang fp contract(off)
+    return a * b;
+}
 // v_permlane16_swap exchanges the odd 16-lane rows of its first operand with the even rows of its second: one swap and one
 // add fold a pair of registers (a, b) into one that holds a(l) + a(l ^ 16) in the even rows and b(l) + b(l ^ 16) in the odd ones.
 __device__ __forceinline__ float fold_pair(float a, float b) {
