@@ -58,3 +58,11 @@ def test_row_pass(case, many):
 @pytest.mark.parametrize("case", [c for c in sorted(GOLDEN) if "f32" in c or c.endswith("D64")])
 def test_column_pass_of_fp32_and_of_head_dimension_64(case, many):
     check(case, [n for n in ("dk", "dv", "di", "df") if n in GOLDEN[case]], copies_of(case, many))
+
+
+# 16 bits at D = 128 and 256: cold_kernel and colw_kernel; one column sum per key, products of dD unrounded in it, and those of G and W in their
+# low-order terms
+@pytest.mark.parametrize("many", [False, True])
+@pytest.mark.parametrize("case", [c for c in sorted(GOLDEN) if "f32" not in c and not c.endswith("D64")])
+def test_column_pass_of_16_bits(case, many):
+    check(case, [n for n in ("dk", "dv", "di", "df") if n in GOLDEN[case]], copies_of(case, many))

@@ -819,7 +819,7 @@ int backward_impl(const void* dh, const void* q, const void* k, const void* v, c
         if (int rc = launch_col_best(dtype, D, ca, st)) return rc;
     }
 
-    DfArgs da{f, colsum, rowpart, df, di, (int)z.BH, (int)z.S, (int)z.NG, (int)z.row_slices(), ca.rowpart2, col_chunks ? w.L : 0, rowinter, anchor, (int)w.ncs};
+    DfArgs da{f, colsum, rowpart, df, di, (int)z.BH, (int)z.S, (int)z.NG, (int)z.row_slices(), ca.rowpart2, colw_serves(dtype, D, ca), col_chunks ? w.L : 0, rowinter, anchor, (int)w.ncs};
     da.lg = z.lg; da.gate_form = z.gate_form; da.stamp = stamp;
     if (col_chunks && fused_anchor) {
         da.anchor = nullptr; da.anchor_part = anchor; da.anchor_parts = anchor_parts; da.anchor_va = Nst; da.anchor_vb = gvec; da.D = D;

@@ -92,11 +92,22 @@ __global__ __launch_bounds__(1024) void dfscan_kernel(const TG* __restrict__ F, 
     }
 }
 
+__device__ __forceinline__ float add_slices(float row, const float (&part)[16], bool pairs) {   // pairs: see DfArgs
+    if (pairs) {
+#pragma unroll
+        for (int j = 0; j < 16; j += 2) row += part[j] + part[j + 1];
+    } else {
+#pragma unroll
+        for (int j = 0; j < 16; j++) row += part[j];
+    }
+    return row;
+}
+
 // Row reduction and dF scan of a sequence of up to 2048 positions that did not run in chunks, in one kernel and one workgroup
 // per head, a thread per position (twice, beyond 1024): a position has at most 32 row partials.  As two kernels (rowreduce,
 // dfscan) the pair took 4.7 + 4.0 us at B1 H2 S300 and a launch more, in steps of 50 to 100 us.
 template <typename TG>
-__global__ __launch_bounds__(1024) void dfhead_kernel(const TG* __restrict__ F, const float* __restrict__ colsum, const float* __restrict__ rowpart, const float* __restrict__ rowpart2,
+__global__ __launch_bounds__(1024) void dfhead_kernel(const TG* __restrict__ F, const float* __restrict__ colsum, const float* __restrict__ rowpart, const float* __restrict__ rowpart2, bool pairs,
                                                       TG* __restrict__ dF, TG* __restrict__ dI, int S, int RS, Lay lg, int form, SavedStamp stamp) {
     __shared__ float wt[2][16];
     const int bh = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = blockDim.x >> 6;
@@ -118,8 +129,7 @@ __global__ __launch_bounds__(1024) void dfhead_kernel(const TG* __restrict__ F, 
 #pragma unroll
                     for (int j = 0; j < 16; j++) part[j] += j0 + j <= g ? rp2[(size_t)(j0 + j) * S] : 0.f;
                 }
-#pragma unroll
-                for (int j = 0; j < 16; j++) row += part[j];
+                row = add_slices(row, part, pairs);
             }
             col = colsum[(size_t)bh * S + t];
             f = (float)F[lg.head(bh) + (size_t)t * lg.ss];
@@ -147,7 +157,7 @@ __global__ __launch_bounds__(1024) void dfhead_kernel(const TG* __restrict__ F, 
 // position has at most chunk_len / 64 row partials.  chunk_len <= 1024; as many threads as positions (or as the anchors' sums
 // take), whole waves: with 1024 whatever the chunk, most of a workgroup's waves had nothing to do but arrive at the barrier.
 template <typename TG>
-__global__ __launch_bounds__(1024) void dfchunk_kernel(const TG* __restrict__ F, const float* __restrict__ colsum, const float* __restrict__ rowpart, const float* __restrict__ rowpart2,
+__global__ __launch_bounds__(1024) void dfchunk_kernel(const TG* __restrict__ F, const float* __restrict__ colsum, const float* __restrict__ rowpart, const float* __restrict__ rowpart2, bool pairs,
                                                        const float* __restrict__ rowinter, const float* __restrict__ anchor,
                                                        TG* __restrict__ dF, TG* __restrict__ dI, int S, int RS, int chunk_len, int n_states,
                                                        Lay lg, int form, const float* __restrict__ anchor_part, int anchor_parts,
@@ -189,8 +199,7 @@ __global__ __launch_bounds__(1024) void dfchunk_kernel(const TG* __restrict__ F,
 #pragma unroll
             for (int j = 0; j < 16; j++) part[j] += j <= g - g0 ? rp2[(size_t)j * S] : 0.f;
         }
-#pragma unroll
-        for (int j = 0; j < 16; j++) row += part[j];
+        row = add_slices(row, part, pairs);
         col = colsum[(size_t)bh * S + t];
         f = (float)F[lg.head(bh) + (size_t)t * lg.ss];
         v = col - row;
@@ -229,14 +238,14 @@ static int launch_df_t(const DfArgs& a, hipStream_t st) {
         if (a.anchor_part) threads = threads > a.D ? threads : a.D;
         if (threads < a.anchor_parts) threads = a.anchor_parts;
         hipLaunchKernelGGL(dfchunk_kernel<TG>, dim3((a.S + a.chunk_len - 1) / a.chunk_len, a.BH), dim3((threads + 63) / 64 * 64), 0, st, reinterpret_cast<const TG*>(a.F),
-                           a.colsum, a.rowpart, a.rowpart2, a.rowinter, a.anchor, reinterpret_cast<TG*>(a.dF), reinterpret_cast<TG*>(a.dI), a.S, a.RS,
+                           a.colsum, a.rowpart, a.rowpart2, a.pairs, a.rowinter, a.anchor, reinterpret_cast<TG*>(a.dF), reinterpret_cast<TG*>(a.dI), a.S, a.RS,
                            a.chunk_len, a.n_states, a.lg, a.gate_form, a.anchor_part, a.anchor_parts, a.anchor_va, a.anchor_vb, a.D, a.stamp);
         return (int)hipGetLastError();
     }
     if (a.anchor_part) return MLSTM_EINVAL;   // (only the one-kernel form adds the parts up)
     if (a.chunk_len == 0 && a.S <= 2048) {
         const int threads = a.S < 1024 ? (a.S + 63) / 64 * 64 : 1024;
-        hipLaunchKernelGGL(dfhead_kernel<TG>, dim3(a.BH), dim3(threads), 0, st, reinterpret_cast<const TG*>(a.F), a.colsum, a.rowpart, a.rowpart2,
+        hipLaunchKernelGGL(dfhead_kernel<TG>, dim3(a.BH), dim3(threads), 0, st, reinterpret_cast<const TG*>(a.F), a.colsum, a.rowpart, a.rowpart2, a.pairs,
                            reinterpret_cast<TG*>(a.dF), reinterpret_cast<TG*>(a.dI), a.S, a.RS, a.lg, a.gate_form, a.stamp);
         return (int)hipGetLastError();
     }

@@ -330,10 +330,9 @@ __global__ __launch_bounds__(256, D == 128 && !STRICT ? 2 : 1) void cold_kernel(
         // k_j . (E v_j + g) w_j, the column sums of dD over the queries behind the chunk (and, for fp16, the scaling itself).
         // The K values a lane needs (its accumulators' rows 8 a4 + 4 h + c of every block) are in the K fragments of the two
         // lanes of its key (which hold columns 16 s + 8 h + 0..7): one v_permlane32_swap per register pair sorts them out.
-        float cp = 0.f, cpx = 0.f;   // (per block of 32 columns, then over the blocks)
+        float cp = 0.f;
 #pragma unroll
         for (int s = 0; s < NS; s++) {
-            if (s % 2 == 0) cpx = 0.f;
             const int x = s >> 1, a4a = 2 * (s & 1);
             const i32x4 w = __builtin_bit_cast(i32x4, kf[s]);
             const auto r0 = __builtin_amdgcn_permlane32_swap(w[0], w[2], false, false);
@@ -351,16 +350,15 @@ __global__ __launch_bounds__(256, D == 128 && !STRICT ? 2 : 1) void cold_kernel(
                 for (int c = 0; c < 4; c++) {
                     const float kval = u ? kc[c] : ka[c];
                     if constexpr (END_SCALE) {
-                        cpx = fmaf(dkacc[x][4 * a4 + c] + g4v[c], kval, cpx);
+                        cp = fmaf(dkacc[x][4 * a4 + c] + g4v[c], kval, cp);
                     } else {
                         const float dkv = (dkacc[x][4 * a4 + c] + g4v[c]) * wk;
                         dkacc[x][4 * a4 + c] = dkv;
                         dvacc[x][4 * a4 + c] *= wk;
-                        cpx = fmaf(dkv, kval, cpx);
+                        cp = fmaf(dkv, kval, cp);
                     }
                 }
             }
-            if (s % 2 == 1) cp += cpx;
             if (s % 2 == 1) __builtin_amdgcn_sched_barrier(0);   // (one block of the accumulators at a time through the vector registers)
         }
         colacc = END_SCALE ? rounded_product(cp, wk) : cp;   // (starts the lane's column accumulator: the two halves of the wave meet in the epilogue)
@@ -373,7 +371,8 @@ __global__ __launch_bounds__(256, D == 128 && !STRICT ? 2 : 1) void cold_kernel(
         __builtin_amdgcn_wave_barrier();
     }
 
-    // row sums: one slice per 64 keys (the dF pass adds them up), that of the second half where that pass reads it
+    // row sums go to the slice of the 64-key tile of the workgroup's first keys (the dF pass adds up one slice per 64 keys),
+    // zeros to the slice of its second half wherever that pass reads it
     const int j64 = 2 * jt;
     float* const rowpart_slice = a.rowpart + ((size_t)bh * a.RS + (a.RS == NG ? j64 : j64 % a.RS)) * S;
     // One step = one 32-query tile.  A lane computes E = exp2(alpha_key + crow_query) per element (a lane holds one key and
@@ -392,12 +391,17 @@ __global__ __launch_bounds__(256, D == 128 && !STRICT ? 2 : 1) void cold_kernel(
         } else {
             if (it + 1 < NQe) { if (stage) COLD_DMA(it + 1, 0); else COLD_DMA(it + 1, 1); }
         }
+        int l = lane;
+        auto rr = rrd;
+        auto tr = trd;
+        if constexpr (LEAN) asm volatile("" : "+v"(l), "+v"(rr.off0), "+v"(tr.off[0]), "+v"(tr.off[1]));   // (addresses are formed anew in every step: see keyvals)
         // row sums of the previous step: the four key blocks' shares are in LDS
-        if (it > it0 && tid < CD_QT && qi0 - CD_QT + tid < S) {
+        const unsigned q = LEAN ? 64 * kb + l : tid;
+        if (it > it0 && q < CD_QT && qi0 - CD_QT + (int)q < S) {
             const float* rt = rowtmp + ((it - 1) & 1) * 4 * CD_QT;
-            float* rp = rowpart_slice + qi0 - CD_QT + tid;
-            rp[0] = rt[tid] + rt[CD_QT + tid];
-            if (j64 + 1 < NG && (qi0 - CD_QT) / GRAN >= j64 + 1) rp[S] = rt[2 * CD_QT + tid] + rt[3 * CD_QT + tid];
+            float* const rp = rowpart_slice + (qi0 - CD_QT);
+            rp[q] = (rt[q] + rt[CD_QT + q]) + (rt[2 * CD_QT + q] + rt[3 * CD_QT + q]);
+            if (j64 + 1 < NG && (qi0 - CD_QT) / GRAN >= j64 + 1) rp[S + q] = 0.f;
         }
         const T* gq = Q + (size_t)CD_QT * (it + 1) * rsA;
         const T* gdh = dH + (size_t)CD_QT * (it + 1) * rsB;
@@ -407,11 +411,7 @@ __global__ __launch_bounds__(256, D == 128 && !STRICT ? 2 : 1) void cold_kernel(
         const T* dHs = ST_DH(stage);
         const float* srow = ST_ROW(stage);
         float* const rt = rowtmp + (it & 1) * 4 * CD_QT + kb * CD_QT;
-        int l = lane;
-        auto rr = rrd;
-        auto tr = trd;
-        if constexpr (LEAN) asm volatile("" : "+v"(l), "+v"(rr.off0), "+v"(tr.off[0]), "+v"(tr.off[1]));   // (addresses are formed anew in every step: see keyvals)
-        const int rt_own = (l & 4) * 2 + ((l >> 3) & 4) + ((l >> 2) & 2) + ((l >> 4) & 1);   // the query whose row sum row_sums8 leaves in this lane
+        const int rt_own = (l & 2) * 4 + ((l >> 3) & 4) + (l & 1) * 2 + ((l >> 4) & 1);   // the query whose row sum row_sums8 leaves in this lane
 
         const bool active = key0 <= qi0 + CD_QT - 1;   // some key of the wave lies at or before some query of the tile
         f32x16 gacc, wacc;   // dC, then G = dC~ E;  S, then W = C~ / n   (rows = queries 8 (r / 4) + 4 h + r % 4, column = key c32)
@@ -453,9 +453,12 @@ __global__ __launch_bounds__(256, D == 128 && !STRICT ? 2 : 1) void cold_kernel(
             // behind the query, or a query past the end) gets the exponent -inf.
             const float argbase = (LEAN ? keyvals[32 * kb + c32] : al) + (LEAN ? sG[(kb >> 1) * NG + (it >> 1)] : sG[it >> 1] + gcorr + log2scale) - (LEAN ? keyvals[CD_KEYS + 32 * kb + c32] : log2_s);
             const float scale_k = LEAN ? keyvals[2 * CD_KEYS + 32 * kb + c32] : scale_s;   // (weights over s_j: see END_SCALE)
-            const unsigned span = (unsigned)(S - key);    // query q takes part iff 0 <= q - key < S - key (unsigned compare)
-            const int dq0 = qi0 + 4 * h - key;            // q - key of register r: dq0 + 8 (r / 4) + r % 4
-            float dd[16], csum0 = 0.f, csum1 = 0.f;   // (column sums: per half of a block, then over the blocks, the order of mlstm_colw.hip)
+            const int key_l = LEAN ? key0 + (l & 31) : key;
+            const unsigned span = (unsigned)(S - key_l);  // query q takes part iff 0 <= q - key < S - key (unsigned compare)
+            const int dq0 = qi0 + 4 * h - key_l;          // q - key of register r: dq0 + 8 (r / 4) + r % 4
+            float dd[16];
+            typename R::vec4 gw[STRICT ? 4 : 1][4];   // split mode: terms of G and W, [four registers][G hi, G lo, W hi, W lo]
+            float e4[4];
             f32x4 beta4[2], inv4[2], db4[2];   // the scalars of the half's eight queries (two groups of four registers)
             auto ew_scalars = [&](int t) {
 #pragma unroll
@@ -472,11 +475,23 @@ __global__ __launch_bounds__(256, D == 128 && !STRICT ? 2 : 1) void cold_kernel(
                 const float e = fast_exp2(live ? argbase - beta4[u][c] : -INFINITY);
                 const float ct = wacc[r] * e;
                 const float dct = fmaf(gacc[r], inv4[u][c], db4[u][c]);
-                dd[r] = rounded_product(END_SCALE ? ct * scale_k : ct, dct);
-                gacc[r] = STRICT ? rounded_product(dct, e) : dct * e;   // (their low-order terms are what these values lose)
-                wacc[r] = STRICT ? rounded_product(ct, inv4[u][c]) : ct * inv4[u][c];
-                if (r < 8) csum0 += dd[r];
-                else csum1 += dd[r];
+                const float cs = END_SCALE ? ct * scale_k : ct;
+                dd[r] = cs * dct;
+                colacc = fmaf(cs, dct, colacc);
+                if constexpr (LEAN) asm volatile("" : "+v"(colacc));   // (here and now: put off, the sum keeps its factors in registers that are short)
+                if constexpr (STRICT) {   // (as factors: the low-order terms take what rounding the products would lose)
+                    gacc[r] = dct;
+                    wacc[r] = ct;
+                    e4[c] = e;
+                    if (c == 3) {
+                        auto four = [&](const f32x16& x) { return f32x4{x[r - 3], x[r - 2], x[r - 1], x[r]}; };
+                        R::split_products(four(gacc), f32x4{e4[0], e4[1], e4[2], e4[3]}, gw[r >> 2][0], gw[r >> 2][1]);
+                        R::split_products(four(wacc), inv4[u], gw[r >> 2][2], gw[r >> 2][3]);
+                    }
+                } else {
+                    gacc[r] = dct * e;
+                    wacc[r] = ct * inv4[u][c];
+                }
             };
             ew_scalars(0);
 #pragma unroll
@@ -491,12 +506,17 @@ __global__ __launch_bounds__(256, D == 128 && !STRICT ? 2 : 1) void cold_kernel(
 #pragma unroll
                         for (int r = 8; r < 16; r++) ew_one(r);
                     }
-                    rt[rt_own + 16 * t] = row_sums8(dd + 8 * t, lane & 8, lane & 4);
+                    rt[rt_own + 16 * t] = row_sums8(dd + 8 * t, lane & 1, lane & 2);
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 frag ghi, glo, whi, wlo;
-                if constexpr (STRICT) { R::from_acc_split(gacc, t, ghi, glo); R::from_acc_split(wacc, t, whi, wlo); }
-                else { ghi = R::from_acc(gacc, t); whi = R::from_acc(wacc, t); }
+                if constexpr (STRICT) {
+                    auto terms = [&](int n) { return __builtin_shufflevector(gw[2 * t][n], gw[2 * t + 1][n], 0, 1, 2, 3, 4, 5, 6, 7); };
+                    ghi = terms(0); glo = terms(1); whi = terms(2); wlo = terms(3);
+                } else {
+                    ghi = R::from_acc(gacc, t);
+                    whi = R::from_acc(wacc, t);
+                }
                 frag qa[2], ha[2];
                 qa[0] = tr.read(Qs, KW * t, 0);
                 ha[0] = tr.read(dHs, KW * t, 0);
@@ -521,11 +541,10 @@ __global__ __launch_bounds__(256, D == 128 && !STRICT ? 2 : 1) void cold_kernel(
 #pragma unroll
                         for (int u = 0; u < 8 / NXD; u++) ew_one(8 + x * (8 / NXD) + u);
                     }
-                    if (!LEAN && x == 1 - t) rt[rt_own + 16 * t] = row_sums8(dd + 8 * t, lane & 8, lane & 4);
+                    if (!LEAN && x == 1 - t) rt[rt_own + 16 * t] = row_sums8(dd + 8 * t, lane & 1, lane & 2);
                     __builtin_amdgcn_sched_barrier(0);
                 }
             }
-            colacc += csum0 + csum1;
             CP_STAMP(6);
         } else {
             if (spread) { qdma.issue(lq, gq, ra); qdma.issue(ldh, gdh, rb); }
@@ -553,8 +572,8 @@ __global__ __launch_bounds__(256, D == 128 && !STRICT ? 2 : 1) void cold_kernel(
         if (tid < CD_QT && CD_QT * last + tid < S) {
             const float* rt = rowtmp + (last & 1) * 4 * CD_QT;
             float* rp = rowpart_slice + CD_QT * last + tid;
-            rp[0] = rt[tid] + rt[CD_QT + tid];
-            if (j64 + 1 < NG && (CD_QT * last) / GRAN >= j64 + 1) rp[S] = rt[2 * CD_QT + tid] + rt[3 * CD_QT + tid];
+            rp[0] = (rt[tid] + rt[CD_QT + tid]) + (rt[2 * CD_QT + tid] + rt[3 * CD_QT + tid]);
+            if (j64 + 1 < NG && (CD_QT * last) / GRAN >= j64 + 1) rp[S] = 0.f;
         }
     }
     {

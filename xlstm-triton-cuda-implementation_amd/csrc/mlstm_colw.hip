@@ -21,7 +21,6 @@
 namespace mlstm {
 
 constexpr int CW_QT = 32;                // queries per tile
-constexpr int CW_MOST_QUERIES = 1024;    // queries a key may meet: their scalars stay in LDS for the whole kernel
 
 template <typename T, int D, bool STRICT>
 struct ColwCfg {
@@ -32,7 +31,7 @@ struct ColwCfg {
     static constexpr int PBUF = STRICT ? 1 : 2;                        // (twice 16 KB and the slots are all of LDS)
     static constexpr size_t P_BYTES = PBUF * 4 * HALF_BYTES;
     static constexpr int E_ROWS = STRICT ? 32 : 64, NE = D / E_ROWS;   // the state in pieces of a slot (split mode: hi, then lo)
-    static constexpr size_t MISC_FLOATS = 2 * 2 * 32 + 2 * 2 * 64 + D;   // row sums, column sums, the vector state
+    static constexpr size_t MISC_FLOATS = 2 * 2 * 32 + 2 * 64 + D;   // row sums, column sums, the vector state
     static size_t lds_bytes(int granules) { return POOL_BYTES + P_BYTES + (MISC_FLOATS + (size_t)granules * (3 * GRAN + 1)) * sizeof(float); }
 };
 
@@ -50,8 +49,8 @@ __global__ __launch_bounds__(512) void colw_kernel(ColArgs a) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     char* const pbuf = smem + Cfg::POOL_BYTES;                                // [buffer][key block][half]
     float* const rowtmp = reinterpret_cast<float*>(pbuf + Cfg::P_BYTES);      // [tile parity][key block][32]
-    float* const colp = rowtmp + 2 * 2 * 32;                                  // [tile parity][key block][lane]
-    float* const gvl = colp + 2 * 2 * 64;                                     // [D] the chunk's vector state g
+    float* const colp = rowtmp + 2 * 2 * 32;                                  // [key block][lane]: the column sums so far
+    float* const gvl = colp + 2 * 64;                                         // [D] the chunk's vector state g
     float* const rowvec = gvl + D;                                            // [granule][beta, 1/n, db][64] of the queries
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5, c32 = lane & 31;
@@ -220,24 +219,29 @@ __global__ __launch_bounds__(512) void colw_kernel(ColArgs a) {
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
-        auto hand_over = [&](int v) __attribute__((always_inline)) {
+        auto hand_over = [&](int v, const f32x4 (&inv4)[4]) __attribute__((always_inline)) {
             char* const block = pbuf + (size_t)((Cfg::PBUF == 2 ? (v & 1) * 2 : 0) + kb) * 2 * Cfg::HALF_BYTES;
 #pragma unroll
             for (int t = 0; t < 2; t++) {
                 frag* const out = reinterpret_cast<frag*>(block + t * Cfg::HALF_BYTES) + lane;
                 if constexpr (STRICT) {
-                    frag hi, lo;
-                    R::from_acc_split(gacc, t, hi, lo);
-                    out[0] = hi; out[128] = lo;
-                    R::from_acc_split(wacc, t, hi, lo);
-                    out[64] = hi; out[192] = lo;
+                    // (the low-order terms take what rounding the products would lose)
+                    typename R::vec4 hi[2], lo[2];
+                    auto terms = [](const typename R::vec4 (&x)[2]) { return __builtin_shufflevector(x[0], x[1], 0, 1, 2, 3, 4, 5, 6, 7); };
+                    auto four = [&](const auto& x, int a4) { return f32x4{x[4 * a4], x[4 * a4 + 1], x[4 * a4 + 2], x[4 * a4 + 3]}; };
+#pragma unroll
+                    for (int u = 0; u < 2; u++) R::split_products(four(gacc, 2 * t + u), four(wt, 2 * t + u), hi[u], lo[u]);
+                    out[0] = terms(hi); out[128] = terms(lo);
+#pragma unroll
+                    for (int u = 0; u < 2; u++) R::split_products(four(wacc, 2 * t + u), inv4[2 * t + u], hi[u], lo[u]);
+                    out[64] = terms(hi); out[192] = terms(lo);
                 } else {
                     out[0] = R::from_acc(gacc, t);
                     out[64] = R::from_acc(wacc, t);
                 }
             }
         };
-        const bool hi8 = lane & 8, hi4 = lane & 4;
+        const bool hi1 = lane & 1, hi2 = lane & 2;
         auto weigh = [&](int v) __attribute__((always_inline)) {
             const float* const srow = rowvec + (v >> 1) * 3 * GRAN + 32 * (v & 1) + 4 * h;
             f32x4 inv4[4], db4[4];   // 1/n and db of the tile's queries
@@ -246,7 +250,7 @@ __global__ __launch_bounds__(512) void colw_kernel(ColArgs a) {
                 inv4[a4] = *reinterpret_cast<const f32x4*>(srow + GRAN + 8 * a4);
                 db4[a4] = *reinterpret_cast<const f32x4*>(srow + 2 * GRAN + 8 * a4);
             }
-            float dd[16], csum0 = 0.f, csum1 = 0.f;
+            float dd[16], colsum = colp[kb * 64 + lane];   // (one sum over all queries, as a wave of cold_kernel keeps it: from weighing wave to weighing wave)
 #pragma unroll
             for (int a4 = 0; a4 < 4; a4++) {
 #pragma unroll
@@ -255,19 +259,19 @@ __global__ __launch_bounds__(512) void colw_kernel(ColArgs a) {
                     const float e = wt[r];
                     const float ct = wacc[r] * e;
                     const float dct = fmaf(gacc[r], inv4[a4][c], db4[a4][c]);
-                    dd[r] = rounded_product(END_SCALE ? ct * scale_s : ct, dct);
-                    gacc[r] = STRICT ? rounded_product(dct, e) : dct * e;   // (their low-order terms are what these values lose)
-                    wacc[r] = STRICT ? rounded_product(ct, inv4[a4][c]) : ct * inv4[a4][c];
-                    if (r < 8) csum0 += dd[r];
-                    else csum1 += dd[r];
+                    const float cs = END_SCALE ? ct * scale_s : ct;
+                    dd[r] = cs * dct;
+                    colsum = fmaf(cs, dct, colsum);
+                    gacc[r] = STRICT ? dct : dct * e;   // (split mode: with wt and 1/n, the factors of G and W)
+                    wacc[r] = STRICT ? ct : ct * inv4[a4][c];
                 }
             }
-            colp[((v & 1) * 2 + kb) * 64 + lane] = csum0 + csum1;
+            colp[kb * 64 + lane] = colsum;
             // (a lane's sum is that of its register: see row_sums8)
-            float* const rt = rowtmp + ((v & 1) * 2 + kb) * 32 + (lane & 4) * 2 + 4 * h + ((lane >> 2) & 2) + ((lane >> 4) & 1);
-            rt[0] = row_sums8(dd, hi8, hi4);
-            rt[16] = row_sums8(dd + 8, hi8, hi4);
-            hand_over(v);
+            float* const rt = rowtmp + ((v & 1) * 2 + kb) * 32 + (lane & 2) * 4 + 4 * h + (lane & 1) * 2 + ((lane >> 4) & 1);
+            rt[0] = row_sums8(dd, hi1, hi2);
+            rt[16] = row_sums8(dd + 8, hi1, hi2);
+            hand_over(v, inv4);
         };
         if (role == 1) {   // the second pair is one step behind
             if constexpr (Cfg::PBUF == 1) __syncthreads();
@@ -369,7 +373,6 @@ __global__ __launch_bounds__(512) void colw_kernel(ColArgs a) {
                 float cp = 0.f;
 #pragma unroll
                 for (int x = 0; x < NXD; x++) {
-                    float cpx = 0.f;
 #pragma unroll
                     for (int a4 = 0; a4 < 4; a4++) {
                         const f32x4 kv = __builtin_convertvector(*reinterpret_cast<const typename R::vec4*>(krow + 32 * x + 8 * a4), f32x4);
@@ -377,15 +380,14 @@ __global__ __launch_bounds__(512) void colw_kernel(ColArgs a) {
 #pragma unroll
                         for (int c = 0; c < 4; c++) {
                             if constexpr (END_SCALE) {
-                                cpx = fmaf(acc[x][4 * a4 + c] + g4[c], kv[c], cpx);
+                                cp = fmaf(acc[x][4 * a4 + c] + g4[c], kv[c], cp);
                             } else {
                                 const float dkv = (acc[x][4 * a4 + c] + g4[c]) * wk;
                                 acc[x][4 * a4 + c] = dkv;
-                                cpx = fmaf(dkv, kv[c], cpx);
+                                cp = fmaf(dkv, kv[c], cp);
                             }
                         }
                     }
-                    cp += cpx;
                 }
                 colacc = END_SCALE ? rounded_product(cp, wk) : cp;
             } else if constexpr (!END_SCALE) {
@@ -395,6 +397,7 @@ __global__ __launch_bounds__(512) void colw_kernel(ColArgs a) {
                     for (int r = 0; r < 16; r++) acc[x][r] *= wk;
             }
         }
+        if (role == 0) colp[kb * 64 + lane] = colacc;   // (the weighing waves take it on from here)
         // row sums: the slice of these 64 keys
         float* const rowpart_slice = a.rowpart + ((size_t)bh * a.RS + (a.RS == NG ? jt : jt % a.RS)) * S + CW_QT * it0;
         constexpr int PF = 4, N = 2 * NXD;   // fragments under way, products per tile
@@ -441,7 +444,6 @@ __global__ __launch_bounds__(512) void colw_kernel(ColArgs a) {
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
-                if (role == 0) colacc += colp[((u & 1) * 2 + kb) * 64 + lane];
             }
             // the next step's tile has landed: everything but the newest AHEAD - 1 tiles (2 PW loads each; a row sum's store
             // counts as one more and makes the wait a little longer)
@@ -451,7 +453,7 @@ __global__ __launch_bounds__(512) void colw_kernel(ColArgs a) {
         }
         // ---- epilogue: column sums, dK and dV through LDS in whole rows (16-byte chunk c of row r at chunk c ^ (r & 31))
         if (role == 0) {
-            colacc = sum_halves(colacc);
+            colacc = sum_halves(colp[kb * 64 + lane]);
             if (h == 0 && key < S) a.colsum[hoff + key] = colacc;
         }
         constexpr int ROWB = D * (int)sizeof(T), CPR = ROWB / 16;

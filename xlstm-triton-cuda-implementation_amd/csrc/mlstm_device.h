@@ -721,19 +721,19 @@ __device__ __forceinline__ float fold_pair(float a, float b) {
     auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(int, a), __builtin_bit_cast(int, b), false, false);
     return __builtin_bit_cast(float, (int)r[0]) + __builtin_bit_cast(float, (int)r[1]);
 }
-// Sums of eight registers over the 32 lanes of either half of a wave: registers and lanes are folded together, 16, 8 and 4 lanes
-// apart, then the four lanes of a quad add up.  Lane l returns the sum of register k = 4 (l / 4 % 2) + 2 (l / 8 % 2) + l / 16 % 2 of
-// its half; hi8, hi4: l & 8, l & 4.  (Eight chains of one swap, an add and four row shifts take 2.5 times the instructions, and each waits for
-// its own.)
-__device__ __forceinline__ float row_sums8(const float* x, bool hi8, bool hi4) {
+// Sums of eight registers over the 32 lanes of either half of a wave: registers and lanes are folded together, 16, 1 and 2 lanes
+// apart, then the four quads of a row add up (in the order of four row shifts by 1, 2, 4 and 8).  Lane l returns the sum of register
+// k = 4 (l / 2 % 2) + 2 (l % 2) + l / 16 % 2 of its half; hi1, hi2: l & 1, l & 2.  (Eight chains of one swap, an add and four row shifts
+// take 2.5 times the instructions, and each waits for its own.)
+__device__ __forceinline__ float row_sums8(const float* x, bool hi1, bool hi2) {
     float f[4], g[2];
 #pragma unroll
     for (int p = 0; p < 4; p++) f[p] = fold_pair(x[2 * p], x[2 * p + 1]);
 #pragma unroll
-    for (int p = 0; p < 2; p++) g[p] = (hi8 ? f[2 * p + 1] : f[2 * p]) + dpp_f<0x128>(0.f, hi8 ? f[2 * p] : f[2 * p + 1]);   // row_ror:8
-    float s = (hi4 ? g[1] : g[0]) + dpp_f<0x141>(0.f, hi4 ? g[0] : g[1]);   // row_half_mirror: lane 7 - l of eight
-    s += dpp_f<0x4e>(0.f, s);   // quad_perm: two lanes away, then one
-    s += dpp_f<0xb1>(0.f, s);
+    for (int p = 0; p < 2; p++) g[p] = (hi1 ? f[2 * p + 1] : f[2 * p]) + dpp_f<0xB1>(0.f, hi1 ? f[2 * p] : f[2 * p + 1]);   // quad_perm 1 0 3 2
+    float s = (hi2 ? g[1] : g[0]) + dpp_f<0x4E>(0.f, hi2 ? g[0] : g[1]);   // quad_perm 2 3 0 1
+    s += dpp_f<0x141>(0.f, dpp_f<0x1B>(0.f, s));   // quad_perm 3 2 1 0, row_half_mirror: the other quad of eight, lane by lane
+    s += dpp_f<0x128>(0.f, s);                     // row_ror:8
     return s;
 }
 struct OpAdd { static __device__ __forceinline__ float id() { return 0.0f; } static __device__ __forceinline__ float f(float a, float b) { return a + b; } };

@@ -190,21 +190,24 @@ int launch_cold_kernel(int dtype, int D, const ColArgs& a, hipStream_t st);
 // the same on 64 keys per workgroup and eight waves, the same bits, for launches of few workgroups; keys that meet up to 1024 queries
 int launch_colw_kernel(int dtype, int D, const ColArgs& a, hipStream_t st);
 extern int g_col_variant;   // see mlstm_set_column_kernel: 0 = the library's choice, 1 = col16_kernel, 2 = cold_kernel, 3 = col_kernel
+constexpr int CW_MOST_QUERIES = 1024;    // queries a key of colw_kernel may meet: their scalars stay in LDS for the whole kernel
+inline bool colw_serves(int dtype, int D, const ColArgs& a) {
+    if (dtype == MLSTM_F32 || (D != 128 && D != 256) || g_force_generic || g_col_variant != 0) return false;
+    if ((a.chunk_len > 0 && a.chunk_len < a.NG * GATE_GRANULE ? a.chunk_len : a.NG * GATE_GRANULE) > CW_MOST_QUERIES) return false;
+    // Workgroups of 64 keys up to which colw_kernel is the faster one; cold_kernel / colw_kernel, us (bf16, workgroups of 64 keys):
+    //   D = 128, S = 1000 (not in chunks)  256: 57 / 30   512: 61 / 39   768: 80 / 60
+    //   D = 128 in chunks of 512           256: 37 / 22   512: 39 / 32   768: 44 / 48    in split mode   128: 38 / 26   256: 40 / 28   512: 43 / 41   768: 61 / 60
+    //   D = 256, S = 1000                   64: 69 / 40   256: 72 / 45   512: 76 / 57
+    //   D = 256 in chunks                  128: 51 / 33   256: 53 / 36   512: 56 / 54   768: 82 / 82
+    //   D = 256 in split mode              128: 65 / 42   256: 67 / 47   512: 72 / 70   768: 108 / 103
+    return (long long)a.BH * a.NG <= (D == 128 && a.chunk_len > 0 && !a.precise ? 512 : 768);
+}
 inline int launch_col_best(int dtype, int D, const ColArgs& a, hipStream_t st) {
     const bool half_big = dtype != MLSTM_F32 && (D == 128 || D == 256);
     int variant = g_force_generic ? 3 : g_col_variant;
     if (!half_big || variant < 0 || variant > 3) variant = 3;
     if (variant == 0) {
-        // Workgroups of 64 keys up to which colw_kernel is the faster one; cold_kernel / colw_kernel, us (bf16, workgroups of 64 keys):
-        //   D = 128, S = 1000 (not in chunks)  256: 57 / 30   512: 61 / 39   768: 80 / 60
-        //   D = 128 in chunks of 512           256: 37 / 22   512: 39 / 32   768: 44 / 48    in split mode   128: 38 / 26   256: 40 / 28   512: 43 / 41   768: 61 / 60
-        //   D = 256, S = 1000                   64: 69 / 40   256: 72 / 45   512: 76 / 57
-        //   D = 256 in chunks                  128: 51 / 33   256: 53 / 36   512: 56 / 54   768: 82 / 82
-        //   D = 256 in split mode              128: 65 / 42   256: 67 / 47   512: 72 / 70   768: 108 / 103
-        if ((long long)a.BH * a.NG <= (D == 128 && a.chunk_len > 0 && !a.precise ? 512 : 768)) {
-            const int rc = launch_colw_kernel(dtype, D, a, st);
-            if (rc != MLSTM_ESHAPE) return rc;
-        }
+        if (colw_serves(dtype, D, a)) return launch_colw_kernel(dtype, D, a, st);
         variant = 2;   // (measured faster than col16_kernel at D = 128 and 256, chunked and not)
     }
     if (variant == 1 && a.precise) variant = 2;   // (col16_kernel has no split mode)
@@ -221,6 +224,7 @@ struct DfArgs {
     int BH, S, NG;
     int RS;                  // row-partial slices per head (see ColArgs)
     const float* rowpart2;   // may be null: the partials of the tiles' second halves (see ColArgs)
+    bool pairs;              // the slices are added up in pairs first (the order of a kernel whose tiles are twice as wide: see colw_serves)
     // in chunks: rowpart holds the slices of the key tiles of the position's own chunk only, rowinter the rest
     int chunk_len;
     const float* rowinter;
