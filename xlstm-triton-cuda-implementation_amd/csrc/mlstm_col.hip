@@ -686,7 +686,7 @@ static int launch_col_d(int D, const ColArgs& a, hipStream_t st) {
 //   uncut (300 positions)   240: 34.5 / 26.7   480: 36.8 / 38.1     D = 128, chunks of 128   256: 46.5 / 25.7   512: 50.0 / 45.3
 //   2048: 198 / 170   8192: 748 / 655   uncut   480: 60 / 50   1000: 101 / 105
 bool colf_serves(int dtype, int D, const ColArgs& a) {
-    if (dtype != MLSTM_F32 || D > 128 || a.RS > D || (a.chunk_len > 0 ? a.chunk_len > 1024 : a.S > 2048)) return false;
+    if (dtype != MLSTM_F32 || D > 128 || g_force_generic || a.RS > D || (a.chunk_len > 0 ? a.chunk_len > 1024 : a.S > 2048)) return false;
     const long long wgs = 2ll * a.BH * a.NG;
     return D == 64 ? wgs <= 256 : (wgs <= 512 || a.chunk_len == 128);
 }

@@ -778,7 +778,7 @@ static int launch_row_d(int D, const RowArgs& a, hipStream_t st) {
 int launch_row_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t st) {
     // fp32 up to one (D = 64) or two (D = 128) workgroups of 32 rows per CU: row_kernel / rowf_kernel, forward, us, in chunks of 128 --
     //   D = 64    256: 15.7 / 10.3   384: 16.0 / 17.4     D = 128   256: 27.8 / 13.7   512: 28.9 / 25.4   640 (uncut): 36.7 / 36.6   1024: 32.5 / 45.1
-    if (dtype == MLSTM_F32 && D <= 128 && 2ll * a.BH * a.NG <= (D == 64 ? 256 : 512)) return launch_rowf_kernel(mode, D, a, st);
+    if (dtype == MLSTM_F32 && D <= 128 && !g_force_generic && 2ll * a.BH * a.NG <= (D == 64 ? 256 : 512)) return launch_rowf_kernel(mode, D, a, st);
     if (mode == MODE_FWD) {
         switch (dtype) {
             case MLSTM_F32: return launch_row_d<float, MODE_FWD>(D, a, st);
