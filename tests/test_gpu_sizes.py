@@ -71,6 +71,27 @@ def test_single_sequences_beyond_the_dense_oracle(S):
         assert frac <= 0.12 and rel <= REL_RMS[dtype], (name, frac, rel)
 
 
+# tables of granules in LDS at the lengths where they are longest: the forward's rows are those of the sequence's beginning alone, bit by bit,
+# and the gradients close to those of split mode, whose column kernel is another
+@pytest.mark.parametrize("S", [94784, 119297, 131072])
+def test_the_longest_sequences(S):
+    dtype = torch.bfloat16
+    g = torch.Generator(device="cuda").manual_seed(S)
+    q, k, v, dh = (torch.randn(1, 1, S, 128, device="cuda", generator=g).to(dtype) for _ in range(4))
+    f, i = (torch.randn(1, 1, S, device="cuda", generator=g) + mean for mean in (3, 0))
+    out = []
+    for precise in (False, True):
+        h, m, b, saved = mm.mlstm_forward_save_hip(q, k, v, f, i, precise=precise)
+        out.append([h, *mm.mlstm_backward_saved_hip(dh, q, k, v, f, i, h, m, b, saved, precise=precise)])
+        n = 20000
+        begin = mm.mlstm_forward_hip(*(t[:, :, :n].contiguous() for t in (q, k, v, f, i)), precise=precise)
+        for name, a_, w_ in zip(("h", "m", "b"), begin, (h, m, b)):
+            assert torch.equal(a_, w_[:, :, :n]), name
+    for name, fast, prec in zip(["h"] + GRADS, *out):
+        frac, rel = literal_violations(fast, prec.float())
+        assert frac <= 0.12 and rel <= REL_RMS[dtype], (name, frac, rel)
+
+
 def test_backward_at_the_headline_shape_is_repeatable():
     """B4 H8 S4096 D256 bf16: two runs of forward + backward on the same buffers give the same bits (no kernel adds
     across workgroups in launch order; the asynchronous tile copies are waited for before their data is read)."""

@@ -33,7 +33,7 @@ struct ColdCfg {
     static constexpr size_t QT_BYTES = (size_t)CD_QT * D * sizeof(T);                  // a 32-row tile of Q or dH
     static constexpr size_t STAGES_BYTES = 4 * QT_BYTES;                               // two stages of (Q, dH); the state tiles before them
     static constexpr size_t ROW_BYTES = 2 * 3 * GRAN * sizeof(float);                  // per stage: beta, 1/n, db (64 floats copied, 32 used)
-    static constexpr size_t MISC_BYTES = (2 * 4 * CD_QT + D + (D == 128 ? 3 * CD_KEYS : 0)) * sizeof(float);     // row sums [2 parities][4 key blocks][32], the vector state
+    static constexpr size_t MISC_BYTES = (2 * 4 * CD_QT + D + (D == 128 ? 3 * CD_KEYS + 2 : 0)) * sizeof(float);     // row sums [2 parities][4 key blocks][32], the vector state
     static constexpr size_t LDS_BYTES = V_BYTES + STAGES_BYTES + ROW_BYTES + MISC_BYTES;   // plus one float per 64-position granule
 };
 
@@ -122,8 +122,8 @@ __global__ __launch_bounds__(256, D == 128 && !STRICT ? 2 : 1) void cold_kernel(
 #define ST_ROW(st) (reinterpret_cast<float*>(tail) + (st) * 3 * GRAN)
     float* const rowtmp = reinterpret_cast<float*>(tail + Cfg::ROW_BYTES);   // [2][4][32]
     float* const gvl = rowtmp + 2 * 4 * CD_QT;   // the chunk's vector state g
-    float* const keyvals = gvl + D;                    // D = 128: [alpha, log2 s, s][key]
-    float* const sG = keyvals + (LEAN ? 3 * CD_KEYS : 0);                         // granule bases minus that of the tile's first granule
+    float* const keyvals = gvl + D;                    // D = 128: [alpha, log2 s, s][key], the tile's first granule minus either granule of keys
+    float* const sG = keyvals + (D == 128 ? 3 * CD_KEYS + 2 : 0);                 // granule bases minus that of the tile's first granule
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = lane >> 5, c32 = lane & 31;
     const int kb = wave;
@@ -239,18 +239,11 @@ __global__ __launch_bounds__(256, D == 128 && !STRICT ? 2 : 1) void cold_kernel(
     rrd.init(lane);
 
     if (has_state && tid < D) gvl[tid] = a.gvec[((size_t)bh * a.n_states + chunk) * D + tid];
-    if constexpr (LEAN) {
-        // for either granule of keys with what else the exponent of a weight has
-        const float corr0 = (float)(gbase - a.G2[goff + g0]), corr1 = (float)(gbase - a.G2[goff + (g0 + 1 < NG ? g0 + 1 : NG - 1)]), l2s = -0.5f * __log2f((float)D);
-        for (int g = tid; g < NG; g += 256) {
-            const float d = (float)((g == tid ? g_first : a.G2[goff + g]) - gbase);
-            sG[g] = d + corr0 + l2s;
-            sG[NG + g] = d + corr1 + l2s;
-        }
-    } else {
-        if (tid < NG) sG[tid] = (float)(g_first - gbase);
-        for (int g = tid + 256; g < NG; g += 256) sG[g] = (float)(a.G2[goff + g] - gbase);
-    }
+    // (one table whatever the length: with one for either granule of keys, two workgroups shared a CU up to 94208 positions only, 64 more cost
+    // 6000 -> 7900 us)
+    if (tid < NG) sG[tid] = (float)(g_first - gbase);
+    for (int g = tid + 256; g < NG; g += 256) sG[g] = (float)(a.G2[goff + g] - gbase);
+    if (LEAN && tid < 2) keyvals[3 * CD_KEYS + tid] = (float)(gbase - a.G2[goff + (g0 + tid < NG ? g0 + tid : NG - 1)]);
     const float gcorr = (float)(gbase - gkey);   // granule base of the tile's first granule minus that of the wave's keys
 #pragma unroll
     for (int s = 0; s < NS; s++) pin(kf[s]);
@@ -451,7 +444,7 @@ __global__ __launch_bounds__(256, D == 128 && !STRICT ? 2 : 1) void cold_kernel(
             // queries of contraction step t of phase B, so the second half's element-wise work, and all the lane reductions
             // of the row sums, are placed between the MFMAs of phase B.  Everything is branch-free: a masked element (key
             // behind the query, or a query past the end) gets the exponent -inf.
-            const float argbase = (LEAN ? keyvals[32 * kb + c32] : al) + (LEAN ? sG[(kb >> 1) * NG + (it >> 1)] : sG[it >> 1] + gcorr + log2scale) - (LEAN ? keyvals[CD_KEYS + 32 * kb + c32] : log2_s);
+            const float argbase = (LEAN ? keyvals[32 * kb + c32] : al) + (sG[it >> 1] + (LEAN ? keyvals[3 * CD_KEYS + (kb >> 1)] : gcorr) + log2scale) - (LEAN ? keyvals[CD_KEYS + 32 * kb + c32] : log2_s);
             const float scale_k = LEAN ? keyvals[2 * CD_KEYS + 32 * kb + c32] : scale_s;   // (weights over s_j: see END_SCALE)
             const int key_l = LEAN ? key0 + (l & 31) : key;
             const unsigned span = (unsigned)(S - key_l);  // query q takes part iff 0 <= q - key < S - key (unsigned compare)
@@ -636,11 +629,11 @@ template <typename T, int D, bool STRICT, bool DENSE>
 static int launch_cold_t(const ColArgs& a, hipStream_t st) {
     using Cfg = ColdCfg<T, D>;
     auto kern = cold_kernel<T, D, STRICT, DENSE>;
-    if (hipError_t e = lds_limit_once<cold_kernel<T, D, STRICT, DENSE>>((int)(Cfg::LDS_BYTES + 2048 * sizeof(float) * (D == 128 ? 2 : 1))); e != hipSuccess) return (int)e;
+    if (hipError_t e = lds_limit_once<cold_kernel<T, D, STRICT, DENSE>>((int)(Cfg::LDS_BYTES + 2048 * sizeof(float))); e != hipSuccess) return (int)e;
     if (a.NG > 2048) return MLSTM_ESHAPE;
     if (a.chunk_len > 0 && (a.chunk_len % CD_KEYS != 0 || (a.n_states > 0 && (!a.Ev || !a.gvec || (STRICT && !a.Ev_lo))))) return MLSTM_EINVAL;
     const int NK = (a.S + CD_KEYS - 1) / CD_KEYS;
-    hipLaunchKernelGGL(kern, dim3(a.BH * NK), dim3(256), Cfg::LDS_BYTES + (size_t)a.NG * sizeof(float) * (D == 128 ? 2 : 1), st, a);
+    hipLaunchKernelGGL(kern, dim3(a.BH * NK), dim3(256), Cfg::LDS_BYTES + (size_t)a.NG * sizeof(float), st, a);
     return (int)hipGetLastError();
 }
 

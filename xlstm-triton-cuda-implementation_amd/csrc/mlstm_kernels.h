@@ -148,7 +148,8 @@ inline int launch_row_best(int mode, int dtype, int D, const RowArgs& a, hipStre
         // D = 128 beyond 512 of them, row_kernel, whose workgroups share a CU in pairs: row8_kernel / row_kernel, forward and dQ pass, us --
         //   512: 18.2, 21.1 / 19.0, 22.6   768: 26.9, 30.8 / 23.6, 27.6   1024: 31.6, 36.4 / 25.4, 30.8   2048: 49.7, 59.3 / 41.0, 48.9
         //   8192: 224, 259 / 180, 224      16384: 416, 482 / 334, 420     not in chunks, 1024: 40.7, 43.0 / 29.4, 33.1
-        const bool pairs = D == 128 && (long long)a.BH * a.NG > 512 && a.spin_limit == DEFAULT_SPIN_LIMIT;
+        // (and as long as the granules a row may meet leave the LDS for two: uncut sequences of up to 118784 positions)
+        const bool pairs = D == 128 && (long long)a.BH * a.NG > 512 && a.spin_limit == DEFAULT_SPIN_LIMIT && (a.chunk_len > 0 || a.NG <= 1856);
         if (rc == MLSTM_ESHAPE && !a.precise && !pairs) rc = launch_row8_kernel(mode, dtype, D, a, st);
         if (rc != MLSTM_ESHAPE) return rc;  // extremely long sequences do not fit its LDS budget
     }
