@@ -35,7 +35,7 @@ extern "C" {
  * mlstm_forward_save_ex, or a recomputation), which makes the results agree with an fp32 evaluation of the
  * reference's formulas (mlstm_matmul.py:104-118, :336-365) to rtol 2e-2 / atol 2e-3 element by element.  Long
  * sequences run in chunks in this mode too, with every chunk state kept as two terms.  Price: half as many MFMAs again, and
- * for large launches the four-wave row kernel instead of the eight-wave one.
+ * for large launches at D = 256 the four-wave row kernel instead of the eight-wave one.
  */
 #define MLSTM_PRECISE 0x100
 

@@ -108,7 +108,7 @@ __global__ __launch_bounds__(256, D == 128 && !STRICT ? 2 : 1) void cold_kernel(
     constexpr int KW = R::KW, NS = D / KW, NXD = D / 32;
     // D = 128: two workgroups per CU, 256 registers per lane, so that one of them multiplies while the other waits for its first tiles (HBM: all
     // CUs ask at once) or writes out -- 15000 of a workgroup's 38000 cycles on average -- instead of one per CU with the element-wise part of a
-    // half tile between the products of the other half.  64 heads x 16384 x 128: 789 us -> 613.  What a register less costs: with three spilled
+    // half tile between the products of the other half.  64 heads x 16384 x 128: 789 us -> 561.  What a register less costs: with three spilled
     // values per step 700 us, with twelve 932 (a reload waits for the copies in front of it).
     // (Split mode keeps one: 32 heads x 2048 x 128 64 us against 73, 64 heads 121 against 114.)
     constexpr bool LEAN = D == 128 && !STRICT;

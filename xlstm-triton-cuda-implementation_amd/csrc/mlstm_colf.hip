@@ -1,5 +1,6 @@
 // Column kernel of the fp32 tensors where few workgroups would run: the math of mlstm_col.hip and its order of operations, hence its
-// bits, on 32 keys per workgroup with four waves on them.
+// bits, on 32 keys per workgroup with four waves on them.  (Where something is not finite, keys are formed again in fp32 multiply-adds:
+// a workgroup's 32 here, 64 there.  Finite keys beside such a one can then differ in their last places.)
 //
 // As in mlstm_rowf.hip nothing but the accumulation over the queries is a chain:
 //   phase A   wave w = block of 32 queries:  S^T = K Q^T, dC^T = V dH^T, the element-wise part, the terms of G and W to LDS;
@@ -136,7 +137,7 @@ __global__ __launch_bounds__(256, 1) void colf_kernel(ColArgs a) {
     __syncthreads();   // K and V (and each wave's own blocks) are there
     SwzRowReader<T, D> rrd;
     rrd.init(lane);
-    SwzTransReaderF32<D> trd;   // (block cb & ~1 and the next)
+    SwzTransReaderF32<D> trd;   // (block cb & ~1 and the next; which of the two is known at run time only, so its offsets lie in 64 bytes of scratch)
     trd.init(lane, cb & ~1);
     __builtin_amdgcn_sched_barrier(0);
     f32x16 dk, dv;

@@ -15,10 +15,11 @@ inline hipError_t lds_limit_once(int bytes) {
     static const hipError_t rc = hipFuncSetAttribute(reinterpret_cast<const void*>(KERN), hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     return rc;
 }
-// For kernels whose waits for memory are counted by hand (s_waitcnt vmcnt(n) with n derived from the operations the SOURCE
-// issues): a register spill adds memory operations of the compiler's that the count does not know, and the wait would then
-// let a load pass as landed that has not.  Asked once per process and kernel: the launch is refused (MLSTM_EBUILD) if the
-// compiled kernel uses any scratch memory at all.
+// For kernels that wait in every step for memory that is counted by hand (s_waitcnt vmcnt(n) with n the operations the SOURCE issues behind the
+// ones it waits for).  Operations that the count does not know, the compiler's own for a spilled register among them, never let a load pass
+// as landed that has not: they only push counted ones out of the newest n, and the wait takes in copies that were meant to stay under
+// way.  In a step that is all latency that is its whole point gone, so the launch is refused (MLSTM_EBUILD) if the compiled kernel uses any
+// scratch memory at all.  Asked once per process and kernel.
 template <auto KERN>
 inline int no_scratch_once() {
     static const int rc = [] {
@@ -138,6 +139,7 @@ inline int launch_row_best(int mode, int dtype, int D, const RowArgs& a, hipStre
         // While its workgroups (64 rows) number no more than the chip's CUs, roww_kernel: row8_kernel / roww_kernel, forward, us --
         // D = 128   10: 13.3 / 11.2   80: 14.6 / 12.1   240 (uncut, 1001 positions): 21.3 / 19.0   256: 13.0 / 10.9   384: 13.8 / 14.0
         // D = 256   10: 17.2 / 13.4   224 (chunks of 512): 23.1 / 17.4   256: 15.4 / 13.0   384: 19.9 / 19.2   512: 25.9 / 27.2
+        // (bf16; fp16, in chunks of 512, forward and dQ pass, 256: D = 128 17.5, 18.8 / 15.0, 16.7, D = 256 25.6, 29.2 / 21.1, 23.4)
         int rc = MLSTM_ESHAPE;
         // (a wait bound of the caller's asks for the kernel that has the wait: mlstm_set_spin_limit)
         if ((long long)a.BH * a.NG <= 256 && !a.precise && a.spin_limit == DEFAULT_SPIN_LIMIT) rc = launch_roww_kernel(mode, dtype, D, a, st);
@@ -147,7 +149,7 @@ inline int launch_row_best(int mode, int dtype, int D, const RowArgs& a, hipStre
         if ((long long)a.BH * a.NG <= (D == 128 ? 256 : 512) && a.precise) rc = launch_rowx_kernel(mode, dtype, D, a, st);
         // D = 128 beyond 512 of them, row_kernel, whose workgroups share a CU in pairs: row8_kernel / row_kernel, forward and dQ pass, us --
         //   512: 18.2, 21.1 / 19.0, 22.6   768: 26.9, 30.8 / 23.6, 27.6   1024: 31.6, 36.4 / 25.4, 30.8   2048: 49.7, 59.3 / 41.0, 48.9
-        //   8192: 224, 259 / 180, 224      16384: 416, 482 / 334, 420     not in chunks, 1024: 40.7, 43.0 / 29.4, 33.1
+        //   8192: 224, 259 / 180, 224      16384: 416, 482 / 330, 412     not in chunks, 1024: 40.7, 43.0 / 29.4, 33.1
         // (and as long as the granules a row may meet leave the LDS for two: uncut sequences of up to 118784 positions)
         const bool pairs = D == 128 && (long long)a.BH * a.NG > 512 && a.spin_limit == DEFAULT_SPIN_LIMIT && (a.chunk_len > 0 || a.NG <= 1856);
         if (rc == MLSTM_ESHAPE && !a.precise && !pairs) rc = launch_row8_kernel(mode, dtype, D, a, st);
@@ -201,6 +203,8 @@ inline bool colw_serves(int dtype, int D, const ColArgs& a) {
     //   D = 256, S = 1000                   64: 69 / 40   256: 72 / 45   512: 76 / 57
     //   D = 256 in chunks                  128: 51 / 33   256: 53 / 36   512: 56 / 54   768: 82 / 82
     //   D = 256 in split mode              128: 65 / 42   256: 67 / 47   512: 72 / 70   768: 108 / 103
+    //   fp16 (at D = 256 with 50 registers spilled where bf16 has 8, one or two reloads per tile of a weighing wave): D = 128, S = 1000  768: 74 / 54   in chunks 512: 37 / 30   768: 49 / 49
+    //     in split mode 768: 57 / 53      D = 256, S = 1000  768: 131 / 89   in chunks 512: 68 / 58   768: 107 / 86   in split mode 768: 128 / 104
     return (long long)a.BH * a.NG <= (D == 128 && a.chunk_len > 0 && !a.precise ? 512 : 768);
 }
 inline int launch_col_best(int dtype, int D, const ColArgs& a, hipStream_t st) {
