@@ -846,6 +846,28 @@ __device__ __forceinline__ void row_stats(const typename Tr<T>::frag (&xf)[NS], 
     row_stats_of(sum_halves(acc), b, m, inv_n, db);
 }
 
+// the same from h's fragments; `low`: hlo holds those of the remainder
+template <typename T, int NS, int NLO>
+__device__ __forceinline__ void row_stats_of_frags(const typename Tr<T>::frag (&xf)[NS], const typename Tr<T>::frag (&hf)[NS],
+                                                   const typename Tr<T>::frag (&hlo)[NLO], bool low, float b, float m, float& inv_n, float& db) {
+    float acc = 0.f;
+#pragma unroll
+    for (int s = 0; s < NS; s++)
+#pragma unroll
+        for (int e = 0; e < Tr<T>::EPL; e++) acc += (float)xf[s][e] * (float)hf[s][e];
+    if constexpr (NLO == NS) {
+        if (low) {
+            float acc_lo = 0.f;
+#pragma unroll
+            for (int s = 0; s < NS; s++)
+#pragma unroll
+                for (int e = 0; e < Tr<T>::EPL; e++) acc_lo += (float)xf[s][e] * (float)hlo[s][e];
+            acc += acc_lo;
+        }
+    }
+    row_stats_of(sum_halves(acc), b, m, inv_n, db);
+}
+
 __device__ __forceinline__ float log_sigmoid(float x) {
     // log(sigmoid(x)) = min(x, 0) - log1p(exp(-|x|))
     return fminf(x, 0.0f) - log1pf(__expf(-fabsf(x)));

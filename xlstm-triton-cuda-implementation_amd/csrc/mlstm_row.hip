@@ -26,7 +26,7 @@
 //
 // 16-bit tensors at D = 128: two workgroups per CU (256 registers per lane, 66 KB of LDS), so that one of them multiplies while the other waits
 // for its first tiles or writes out.  64 heads x 16384 x 128, forward and dQ pass: 330 and 412 us, one eight-wave workgroup per CU
-// (mlstm_row8.hip) 416 and 482.
+// (mlstm_row8.hip) 416 and 482; with what a workgroup does once in whole lines and one trip to memory 283 and 378.  (The figures below are from before that.)
 // Split mode at D = 128: two as well (244 to 256 registers, before 271 to 280 and hence one), forward and dQ pass, us before / after, by workgroups:
 // 384: 34.8, 34.9 / 35.2, 35.7   512: 44.8, 48.6 / 36.5, 38.5   2048: 156, 176 / 125, 136.  At D = 64 its forward missed two by two
 // registers: 432: 21.4 / 16.0   512: 31.8 / 25.2   1416: 54.0 / 38.6   4096: 160 / 116; its dQ pass on registers of one kind 137 / 127.
@@ -115,34 +115,119 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
     const T* Y1 = reinterpret_cast<const T*>(a.Y1) + offA;
     const T* Y2 = reinterpret_cast<const T*>(a.Y2) + offA;
 
-    frag xf[NS];
+    // ---- one trip to memory for all that is needed before the first key tile: the rows of X, as two 64-row tiles in whole lines, and with them
+    // the state of the previous chunk or, in the first one, key tile 0 (a row per lane straight into registers asks for 32 bytes of 32 lines per
+    // instruction, and the state and the first keys came one trip after the other: 64 heads x 16384 x 128,
+    // forward 334 -> 297 us, dQ pass 422 -> 400).  Where all state tiles fit one
+    // stage, in up to 32 KB (64 KB are no longer one trip: fp32 at D = 128 143 -> 147 us), they lie in stage 1 and X in stage 0; otherwise the first
+    // one lies in stage NTL % 2, as below, and X in the other.
+    constexpr int NTL = D / GRAN;
+    constexpr bool AT_ONCE = !STRICT && NTL <= 2 && NTL * Cfg::TILE_ELEMS * sizeof(T) <= 32 * 1024;
+    const bool far = chunk > 0;
+#define ST_Y1(st) (reinterpret_cast<T*>(smem + (st) * Cfg::STAGE_BYTES))
+#define ST_Y2(st) (ST_Y1(st) + Cfg::TILE_ELEMS)
+#define ST_AL(st) (reinterpret_cast<float*>(ST_Y2(st) + Cfg::TILE_ELEMS))
+    double* const sG = reinterpret_cast<double*>(smem + Cfg::STAGES_BYTES);   // granule bases of this head
+    const int met = a.chunk_len > 0 && a.chunk_len / GRAN < NG ? a.chunk_len / GRAN : NG;   // granules a row may meet
+    float* const nvl = reinterpret_cast<float*>(sG + ((met + 1) & ~1));       // in chunks: the vector state of the previous one, [D]
+    // (plain loads first: what they bring is used behind the copies' issue)
+    const float beta_row = a.beta2[poff + rowc], m_row = a.M[hoff + rowc];
+    const float b_row = MODE == MODE_DQ ? a.Bin[hoff + rowc] : 0.f;
+    const float beta_end = far ? a.beta2[poff - 1] : 0.f;
+    const double g_row = far ? a.G2[goff + rowc / GRAN] : 0.0, g_end = far ? a.G2[goff - 1] : 0.0;
+    frag hfr[NS], hlr[STRICT ? NS : 1];
+    bool h_low = false;
+    if constexpr (MODE == MODE_DQ) {
+        const T* hrow = reinterpret_cast<const T*>(a.Hin) + offH + (size_t)rowc * rsH;
 #pragma unroll
-    for (int s = 0; s < NS; s++) xf[s] = frag_rowmajor<T>(X + (size_t)rowc * rsX, s, h);
-
+        for (int s = 0; s < NS; s++) hfr[s] = frag_rowmajor<T>(hrow, s, h);
+        if constexpr (STRICT) {
+            h_low = a.Hin_lo != nullptr;
+            if (h_low) {
+                const T* hlo = reinterpret_cast<const T*>(a.Hin_lo) + (hoff + rowc) * D;
+#pragma unroll
+                for (int s = 0; s < NS; s++) hlr[s] = frag_rowmajor<T>(hlo, s, h);
+            }
+        }
+    }
+    TileDma<T, D, GRAN, 256> tdma;
+    tdma.init(tid);
+    const auto ra = tdma.rows(tid, (unsigned)(rsA * sizeof(T)));
+    RowVec3Dma rvdma;   // alpha, ek (64 per tile) and the two block maxima of a tile (padded arrays: always readable)
+    rvdma.init(tid, a.alpha2 + poff, a.ek2 + poff, a.amax2 + goff * 2, 64, 64, 2);
+    const int full_tiles = S / GRAN;  // key tiles whose 64 rows all exist
+#define ROW_DMA(j, st)                                                                   \
+    do {                                                                                 \
+        if ((j) < full_tiles) {                                                          \
+            tdma.issue(ST_Y1(st), Y1 + (size_t)GRAN * (j) * rsA, ra);                     \
+            tdma.issue(ST_Y2(st), Y2 + (size_t)GRAN * (j) * rsA, ra);                     \
+        } else {                                                                         \
+            int t = tid;   /* (formed anew: addresses kept for a tile that rarely comes were spilled) */ \
+            if constexpr (R::HALF && D == 128) asm volatile("" : "+v"(t));                 \
+            tile_dma<T, D, GRAN, 256>(ST_Y1(st), Y1, GRAN * (j), S, t, rsA);              \
+            tile_dma<T, D, GRAN, 256>(ST_Y2(st), Y2, GRAN * (j), S, t, rsA);              \
+        }                                                                                \
+        rvdma.issue(ST_AL(st), (j));                                                     \
+    } while (0)
+    const size_t sbase = far ? ((size_t)bh * a.n_states + chunk - 1) * D * D : 0;
+    const T* const Cs = reinterpret_cast<const T*>(a.Cst) + sbase;
+    const T* const Cl = STRICT ? reinterpret_cast<const T*>(a.Cst_lo) + sbase : nullptr;
+    auto issue_state = [&](int tau) {
+        if constexpr (AT_ONCE) {
+            tdma.issue(tau == 0 ? ST_Y1(1) : ST_Y2(1), Cs + (size_t)GRAN * tau * D);
+        } else {
+            const int stg = (tau + (NTL & 1)) & 1;
+            tdma.issue(ST_Y1(stg), Cs + (size_t)GRAN * tau * D);
+            if constexpr (STRICT) tdma.issue(ST_Y2(stg), Cl + (size_t)GRAN * tau * D);
+        }
+    };
+    T* const xtile = ST_Y1(far && (AT_ONCE || (NTL & 1)) ? 0 : 1);
+    {
+        const auto rx = tdma.rows(tid, (unsigned)(rsX * sizeof(T)));
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            if (q0 + GRAN * (t + 1) <= S) tdma.issue(xtile + t * Cfg::TILE_ELEMS, X + (size_t)(q0 + GRAN * t) * rsX, rx);
+            else tile_dma_rolled<T, D, GRAN, 256>(xtile + t * Cfg::TILE_ELEMS, X, q0 + GRAN * t, S, tid, rsX);
+        }
+    }
+    if (far) {
+        issue_state(0);
+        if constexpr (AT_ONCE && NTL == 2) issue_state(1);
+        if (tdma.wave_s < D / 64)
+            dma4(a.Nst + ((size_t)bh * a.n_states + chunk - 1) * D + 64 * tdma.wave_s + lane, __builtin_amdgcn_readfirstlane(lds_offset_of(nvl + 64 * tdma.wave_s)));
+    } else {
+        ROW_DMA(0, 0);
+    }
     // granule bases of this head in LDS: a global load inside the main loop would have to be waited for with
     // vmcnt(0), which would also wait for the tile copies in flight
-    double* const sG = reinterpret_cast<double*>(smem + Cfg::STAGES_BYTES);
-    const int met = a.chunk_len > 0 && a.chunk_len / GRAN < NG ? a.chunk_len / GRAN : NG;   // granules a row may meet
     for (int g = tid; g < met; g += 256) sG[g] = a.G2[goff + g];
     // What a weight's exponent has beside alpha of the key.  fp32: its parts stay apart until they are added at the size of the
     // result (alpha less beta of the row; the granules' distance and log2 of 1 / sqrt(D) in fp64): added up per row first they were
     // rounded at the size of the parts, 3 % of the error of h and 6 % of that of dV.
     typedef typename std::conditional<F32, double, float>::type Crow;
     constexpr double LOG2_SCALE = D == 64 ? -3.0 : (D == 128 ? -3.5 : -4.0);
-    const float nbeta = -a.beta2[poff + rowc];
-    float crow_base = -0.5f * __log2f((float)D) - a.beta2[poff + rowc];
+    const float nbeta = -beta_row;
+    float crow_base = -0.5f * __log2f((float)D) - beta_row;
+    // the rows' decay since the end of the previous chunk
+    float dec = far ? fast_exp2(beta_end - beta_row + (float)(g_row - g_end)) : 0.f;
+    SwzRowReader<T, D> krd;
+    krd.init(lane);
+    dma_wait();
+    __syncthreads();   // X, what came with it and sG are there
+    frag xf[NS];
+#pragma unroll
+    for (int s = 0; s < NS; s++) xf[s] = krd.read(xtile + (wave >> 1) * Cfg::TILE_ELEMS, wave & 1, s);
     float inv_n = 0.f, dbv = 0.f;
     if constexpr (MODE == MODE_DQ) {
-        const T* hlo = nullptr;
-        if constexpr (STRICT) { if (a.Hin_lo) hlo = reinterpret_cast<const T*>(a.Hin_lo) + (hoff + rowc) * D; }
-        row_stats<T, NS>(xf, reinterpret_cast<const T*>(a.Hin) + offH + (size_t)rowc * rsH, h, a.Bin[hoff + rowc], a.M[hoff + rowc], inv_n, dbv, hlo);
+        row_stats_of_frags<T, NS>(xf, hfr, hlr, h_low, b_row, m_row, inv_n, dbv);
         // (the rows behind the sequence, up to the end of its last granule, as zeros: whoever reads whole granules multiplies
         // them by a weight of zero, and what scratch memory holds need not be a number)
         if (row < NG * GRAN && h == 0) { a.inv_n[poff + row] = row < S ? inv_n : 0.f; a.db[poff + row] = row < S ? dbv : 0.f; }
     }
 #pragma unroll
     for (int s = 0; s < NS; s++) pin(xf[s]);
-    pin(crow_base); pin(inv_n); pin(dbv);
+    pin(crow_base); pin(inv_n); pin(dbv); pin(dec);
+    if (far) __syncthreads();   // X's stage is free
     typename R::terms xt[NS];   // the rows' operand of every first product
 #pragma unroll
     for (int s = 0; s < NS; s++) xt[s] = R::split(xf[s]);
@@ -160,39 +245,11 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
     // factorised weights wherever a block lies below the diagonal.
     constexpr bool PARITY = FAST_TR && !STRICT;
     float bpar[2] = {0.f, 0.f}, bfar[2] = {0.f, 0.f}, dec_far = 0.f;
-    SwzRowReader<T, D> krd;
-    krd.init(lane);
     typename std::conditional<F32, SwzTransReaderF32<D>, SwzTransReader<typename std::conditional<FAST_TR, T, __bf16>::type, FAST_TR ? D : 256>>::type vrd;
     if constexpr (FAST_TR || F32) vrd.init(lane);
 
     const int last_row = (q0 + ROW_BQ - 1 < S - 1) ? q0 + ROW_BQ - 1 : S - 1;
     const int nJ = last_row / GRAN + 1;
-
-#define ST_Y1(st) (reinterpret_cast<T*>(smem + (st) * Cfg::STAGE_BYTES))
-#define ST_Y2(st) (ST_Y1(st) + Cfg::TILE_ELEMS)
-#define ST_AL(st) (reinterpret_cast<float*>(ST_Y2(st) + Cfg::TILE_ELEMS))
-    const float* const alpha_head = a.alpha2 + poff;
-    const float* const ek_head = a.ek2 + poff;
-    const float* const amax_head = a.amax2 + goff * 2;
-    TileDma<T, D, GRAN, 256> tdma;
-    tdma.init(tid);
-    const auto ra = tdma.rows(tid, (unsigned)(rsA * sizeof(T)));
-    RowVec3Dma rvdma;   // alpha, ek (64 per tile) and the two block maxima of a tile (padded arrays: always readable)
-    rvdma.init(tid, alpha_head, ek_head, amax_head, 64, 64, 2);
-    const int full_tiles = S / GRAN;  // key tiles whose 64 rows all exist
-#define ROW_DMA(j, st)                                                                   \
-    do {                                                                                 \
-        if ((j) < full_tiles) {                                                          \
-            tdma.issue(ST_Y1(st), Y1 + (size_t)GRAN * (j) * rsA, ra);                     \
-            tdma.issue(ST_Y2(st), Y2 + (size_t)GRAN * (j) * rsA, ra);                     \
-        } else {                                                                         \
-            int t = tid;   /* (formed anew: addresses kept for a tile that rarely comes were spilled) */ \
-            if constexpr (R::HALF && D == 128) asm volatile("" : "+v"(t));                 \
-            tile_dma<T, D, GRAN, 256>(ST_Y1(st), Y1, GRAN * (j), S, t, rsA);              \
-            tile_dma<T, D, GRAN, 256>(ST_Y2(st), Y2, GRAN * (j), S, t, rsA);              \
-        }                                                                                \
-        rvdma.issue(ST_AL(st), (j));                                                     \
-    } while (0)
 
     // first product of both 32-key blocks of a tile, S^T (or dC^T) in accumulator layout; the two accumulation
     // chains are interleaved so that consecutive MFMAs never depend on each other
@@ -441,32 +498,38 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
       }
     };
 
-    __syncthreads();  // sG visible; every plain global load above has been waited for (pin)
     const double GI = sG[(wave_active ? r0 : S - 1) / GRAN];
-    if (chunk > 0) {
+    if (far) {
         // ---- what lies before the chunk: the state at the end of the previous chunk, as D/64 tiles of 64 rows in the order
-        // in which this product contracts them (mlstm_chunk.hip), hi tile in a stage's Y1 slot and, in split mode, the lo
-        // tile in its Y2 slot.  The last state tile sits in stage 1, so that key tile 0 can follow into stage 0 under it.
-        constexpr int NTL = D / GRAN, NGRP = GRAN / KW;
-        const size_t sbase = ((size_t)bh * a.n_states + chunk - 1) * D * D;
-        const T* const Cs = reinterpret_cast<const T*>(a.Cst) + sbase;
-        const T* const Cl = STRICT ? reinterpret_cast<const T*>(a.Cst_lo) + sbase : nullptr;
-        auto issue_state = [&](int tau) {
-            const int stg = (tau + (NTL & 1)) & 1;
-            tdma.issue(ST_Y1(stg), Cs + (size_t)GRAN * tau * D);
-            if constexpr (STRICT) tdma.issue(ST_Y2(stg), Cl + (size_t)GRAN * tau * D);
-        };
-        issue_state(0);
-        // the rows' decay since the end of the previous chunk: requested now, used behind the tiles
-        const float dec = fast_exp2(a.beta2[poff - 1] - a.beta2[poff + rowc] + (float)(a.G2[goff + rowc / GRAN] - a.G2[goff - 1]));
+        // in which this product contracts them (mlstm_chunk.hip), in split mode each as a hi and a lo tile.  One tile at a time (not
+        // AT_ONCE) they go through the stages in turns, hi tile in the Y1 slot and lo tile in the Y2 slot, the last one in stage 1, so that
+        // key tile 0 can follow into stage 0 under it.
+        constexpr int NGRP = GRAN / KW;
+        // dQ pass: the rows of Q for q_i . dQ_i below, requested ahead of the state's products.  A lane holds four columns of every eight, 8 bytes of
+        // a 16-byte piece; 16-bit rows are loaded in whole pieces, half of them by either lane of a row, which exchange the halves
+        // (64 heads x 16384 x 128 400 -> 394 us).
+        constexpr bool QPIECES = MODE == MODE_DQ && R::HALF && D <= 128;
+        constexpr int QP = QPIECES ? D / 16 : 1;
+        uint4 qpiece[QP];
+        if constexpr (QPIECES) {
+            const T* qrow = reinterpret_cast<const T*>(a.Qrow) + offA + (size_t)rowc * rsA;
+#pragma unroll
+            for (int p = 0; p < QP; p++) qpiece[p] = *reinterpret_cast<const uint4*>(qrow + 8 * (QP * h + p));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (AT_ONCE) ROW_DMA(0, 0);
 #pragma unroll
         for (int tau = 0; tau < NTL; tau++) {
-            const int stg = (tau + (NTL & 1)) & 1;
-            dma_wait();
-            __syncthreads();   // tile tau has landed; the other stage is free
-            if (tau + 1 < NTL) issue_state(tau + 1);
-            else ROW_DMA(0, 0);
-            const T* th = ST_Y1(stg);
+            const int stg = AT_ONCE ? 1 : (tau + (NTL & 1)) & 1;
+            if constexpr (!AT_ONCE) {
+                if (tau > 0) {
+                    dma_wait();
+                    __syncthreads();   // tile tau has landed; the other stage is free
+                }
+                if (tau + 1 < NTL) issue_state(tau + 1);
+                else ROW_DMA(0, 0);
+            }
+            const T* th = AT_ONCE && tau == 1 ? ST_Y2(stg) : ST_Y1(stg);
             const T* tl = ST_Y2(stg);
             if constexpr (F32) {
                 R::template stream<NGRP * NDB>([&](auto n) { return vrd.read(th, KW * (n / NDB), n % NDB); },
@@ -497,7 +560,7 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
                 }
             }
         }
-        const float* nst = a.Nst + ((size_t)bh * a.n_states + chunk - 1) * D;
+        const float* const nst = nvl;
         if constexpr (MODE == MODE_FWD) {
             // row sums: decay_i (q_i . n~); the lane's half of the row (the halves meet in the epilogue)
             if constexpr (PARITY) {
@@ -524,37 +587,51 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
                 for (int r = 0; r < 16; r++) oacc[d][r] *= dec;
         } else {
             const float decn = dec * inv_n, rank1 = dec * dbv;
-            const T* qrow = reinterpret_cast<const T*>(a.Qrow) + offA + (size_t)rowc * rsA;
             // (summed per block of 32 columns, as mlstm_rowf.hip, mlstm_roww.hip and mlstm_rowx.hip, which split a row by columns, have to;
             // 16 bits at D >= 128: and per half of them.  At D = 64 they are one sum.)
             float rp = 0.f, rp_first = 0.f, rpd = 0.f;
-            f32x4 nv[2][4];   // a column block's values, requested a block ahead (left to the compiler: sixteen loads, each waited for)
-            typename R::vec4 qv[2][4];
-            auto request = [&](int d) {
-#pragma unroll
-                for (int a4 = 0; a4 < 4; a4++) {
-                    nv[d & 1][a4] = *reinterpret_cast<const f32x4*>(nst + 32 * d + 8 * a4 + 4 * h);
-                    qv[d & 1][a4] = *reinterpret_cast<const typename R::vec4*>(qrow + 32 * d + 8 * a4 + 4 * h);
-                }
-                __builtin_amdgcn_sched_barrier(0);
-            };
-            request(0);
-#pragma unroll
-            for (int d = 0; d < NDB; d++) {
-                if (d + 1 < NDB) request(d + 1);
+            auto block = [&](int d, auto&& n_of, auto&& q_of) {
                 if (F32 || FAST_TR) rpd = 0.f;
 #pragma unroll
                 for (int a4 = 0; a4 < 4; a4++) {
-                    const f32x4 q4 = __builtin_convertvector(qv[d & 1][a4], f32x4);
+                    const f32x4 n4 = n_of(a4), q4 = __builtin_convertvector(q_of(a4), f32x4);
 #pragma unroll
                     for (int c = 0; c < 4; c++) {
-                        const float v = fmaf(rank1, nv[d & 1][a4][c], oacc[d][4 * a4 + c] * decn);
+                        const float v = fmaf(rank1, n4[c], oacc[d][4 * a4 + c] * decn);
                         oacc[d][4 * a4 + c] = v;
                         rpd = fmaf(v, q4[c], rpd);
                     }
                 }
                 if (F32 || FAST_TR || d == NDB - 1) rp += rpd;
                 if (FAST_TR && d == NDB / 2 - 1) { rp_first = rp; rp = 0.f; }
+            };
+            auto n_at = [&](int d, int a4) { return *reinterpret_cast<const f32x4*>(nst + 32 * d + 8 * a4 + 4 * h); };
+            if constexpr (QPIECES) {
+                // pieces p (lanes h = 0) and QP + p (h = 1) of the row: the low halves to h = 0, the high ones to h = 1
+                uint2 qh[2 * QP];
+#pragma unroll
+                for (int p = 0; p < QP; p++) {
+                    const auto x = __builtin_amdgcn_permlane32_swap((int)qpiece[p].x, (int)qpiece[p].z, false, false);
+                    const auto y = __builtin_amdgcn_permlane32_swap((int)qpiece[p].y, (int)qpiece[p].w, false, false);
+                    qh[p] = make_uint2(x[0], y[0]);
+                    qh[QP + p] = make_uint2(x[1], y[1]);
+                }
+#pragma unroll
+                for (int d = 0; d < NDB; d++) block(d, [&](int a4) { return n_at(d, a4); }, [&](int a4) { return __builtin_bit_cast(typename R::vec4, qh[4 * d + a4]); });
+            } else {
+                const T* qrow = reinterpret_cast<const T*>(a.Qrow) + offA + (size_t)rowc * rsA;
+                typename R::vec4 qv[2][4];   // a column block's values, requested a block ahead (left to the compiler: loads one by one, each waited for)
+                auto request = [&](int d) {
+#pragma unroll
+                    for (int a4 = 0; a4 < 4; a4++) qv[d & 1][a4] = *reinterpret_cast<const typename R::vec4*>(qrow + 32 * d + 8 * a4 + 4 * h);
+                    __builtin_amdgcn_sched_barrier(0);
+                };
+                request(0);
+#pragma unroll
+                for (int d = 0; d < NDB; d++) {
+                    if (d + 1 < NDB) request(d + 1);
+                    block(d, [&](int a4) { return n_at(d, a4); }, [&](int a4) { return qv[d & 1][a4]; });
+                }
             }
             // row sums of dD over the keys before the chunk: q_i . dQ_i of what the accumulators hold now
             rp = sum_halves(rp);
@@ -565,7 +642,6 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
         if constexpr (MODE == MODE_DQ) {
             if (a.chunk_len > 0 && row < S && h == 0) a.rowinter[hoff + row] = 0.f;
         }
-        ROW_DMA(0, 0);
     }
     // Tiles strictly below this wave's rows take the mask-free path; the last one or two tiles of the workgroup are
     // diagonal, or entirely above the diagonal, for this wave.  Two loops with one code path each keep the output
@@ -671,11 +747,11 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
         } else {
             brow = sum_halves(bsum);
         }
-        const float m = a.M[hoff + rowc];
-        const float n = fmaxf(fabsf(brow), __expf(-m)) + 1e-6f;
+        const float n = fmaxf(fabsf(brow), __expf(-m_row)) + 1e-6f;
         onorm = 1.0f / n;
     }
-    bool mine = row < S;   // (this lane writes its half of the row)
+    const bool mine = row < S;
+    unsigned left_out = 0;   // rows that row_exact writes
     if constexpr (F32) {   // rows that are not finite, from their definition (see not_finite)
         float seen = not_finite(0.f, brow);
 #pragma unroll
@@ -683,57 +759,99 @@ __global__ __launch_bounds__(256, PER_CU) void row_kernel(RowArgs a) {
 #pragma unroll
             for (int r = 0; r < 16; r++) seen = not_finite(seen, oacc[d][r]);
         const unsigned long long halves = __ballot(mine && seen != 0.f);
-        unsigned bad = (unsigned)halves | (unsigned)(halves >> 32);
-        mine = mine && !((bad >> c32) & 1);
-        for (; bad; bad &= bad - 1) {
+        left_out = (unsigned)halves | (unsigned)(halves >> 32);
+        for (unsigned bad = left_out; bad; bad &= bad - 1) {
             const int b = __builtin_ctz(bad);
             row_exact<D, MODE>(a, bh, chunk, r0 + b, S, hoff, poff, goff, X + (size_t)(r0 + b) * rsX, Y1, Y2, rsA, offA, offO, offB, rsO, rsB,
                                __shfl(inv_n, b), __shfl(dbv, b));
         }
     }
     if constexpr (MODE == MODE_FWD) {
-        if (mine && h == 0) a.Bsum[hoff + row] = brow;
+        if (mine && h == 0 && !((left_out >> c32) & 1)) a.Bsum[hoff + row] = brow;
     }
-    if (mine) {
-        T* out = reinterpret_cast<T*>(a.out) + offO + (size_t)row * rsO;
+    // A lane holds four columns of every eight of its row; stored from there that is 8 or 16 bytes of 32 rows per instruction.  The wave's 32 rows go through
+    // LDS (rows padded by 16 bytes; the stages are free behind the barrier) and leave in whole lines: 64 heads x 16384 x 128, forward
+    // 297 -> 283 us, dQ pass 394 -> 378; up to two workgroups per CU level (64 x 1000 x 64 20.6 and 22.2 either way, 8 x 1000 x 64, dQ pass, 16.9 -> 17.2).
+    constexpr int RB = D * (int)sizeof(T) + 16, CPR = D * (int)sizeof(T) / 16, NPC = 32 * CPR / 64;
+    static_assert(4 * 32 * RB <= (int)Cfg::STAGES_BYTES, "the rows fit the stages");
+    char* const stage = smem + wave * 32 * RB;
+    auto put = [&](int d, int a4, const typename R::vec4& v) {
+        *reinterpret_cast<typename R::vec4*>(stage + c32 * RB + (32 * d + 8 * a4 + 4 * h) * (int)sizeof(T)) = v;
+    };
+    auto pieces = [&](auto&& f) {   // f(row of the wave, piece of the row, piece number) for the rows to write
 #pragma unroll
-        for (int d = 0; d < NDB; d++)
+        for (int i = 0; i < NPC; i++) {
+            const int c = lane + 64 * i, rr = c / CPR;
+            if (r0 + rr < S && !((left_out >> rr) & 1)) f(rr, c % CPR, i);
+        }
+    };
+    auto piece_at = [&](int rr, int cc) { return *reinterpret_cast<const uint4*>(stage + rr * RB + 16 * cc); };
+    uint4 og[PARITY && MODE == MODE_FWD ? NPC : 1];   // output gate, ahead of the barrier
+    if constexpr (PARITY && MODE == MODE_FWD) {
+        if (a.O) {
+            const char* go = reinterpret_cast<const char*>(a.O) + (offB + (size_t)r0 * rsB) * sizeof(T);
+            pieces([&](int rr, int cc, int i) { og[i] = *reinterpret_cast<const uint4*>(go + (size_t)rr * rsB * sizeof(T) + 16 * cc); });
+        }
+    }
+    __syncthreads();
+    typename R::vec4 low[STRICT && MODE == MODE_FWD ? NDB : 1][4];
 #pragma unroll
-            for (int a4 = 0; a4 < 4; a4++) {
-                f32x4 v;
+    for (int d = 0; d < NDB; d++)
 #pragma unroll
-                for (int c = 0; c < 4; c++) v[c] = STRICT ? rounded_product(oacc[d][4 * a4 + c], onorm) : oacc[d][4 * a4 + c] * onorm;
-                if constexpr (STRICT && MODE == MODE_FWD) {
-                    typename R::vec4 hi, lo;
-                    R::cvt4_split(v, hi, lo);
-                    *reinterpret_cast<typename R::vec4*>(out + 32 * d + 8 * a4 + 4 * h) = hi;
-                    if (a.out_lo) *reinterpret_cast<typename R::vec4*>(reinterpret_cast<T*>(a.out_lo) + (hoff + row) * D + 32 * d + 8 * a4 + 4 * h) = lo;
-                } else {
-                    *reinterpret_cast<typename R::vec4*>(out + 32 * d + 8 * a4 + 4 * h) = R::cvt4(v);
+        for (int a4 = 0; a4 < 4; a4++) {
+            f32x4 v;
+#pragma unroll
+            for (int c = 0; c < 4; c++) v[c] = STRICT ? rounded_product(oacc[d][4 * a4 + c], onorm) : oacc[d][4 * a4 + c] * onorm;
+            if constexpr (STRICT && MODE == MODE_FWD) {
+                typename R::vec4 hi;
+                R::cvt4_split(v, hi, low[d][a4]);
+                put(d, a4, hi);
+            } else {
+                put(d, a4, R::cvt4(v));
+            }
+        }
+    {
+        char* const gout = reinterpret_cast<char*>(a.out) + (offO + (size_t)r0 * rsO) * sizeof(T);
+        pieces([&](int rr, int cc, int) { *reinterpret_cast<uint4*>(gout + (size_t)rr * rsO * sizeof(T) + 16 * cc) = piece_at(rr, cc); });
+        if constexpr (PARITY && MODE == MODE_FWD) {
+            if (a.O) {   // (from h as it is written, like the other row kernels)
+                char* const gg = reinterpret_cast<char*>(a.out_gated) + (offB + (size_t)r0 * rsB) * sizeof(T);
+                pieces([&](int rr, int cc, int i) {
+                    struct Pair { typename R::vec4 lo, hi; };
+                    const Pair hv = __builtin_bit_cast(Pair, piece_at(rr, cc)), ov = __builtin_bit_cast(Pair, og[i]);
+                    Pair res;
+                    res.lo = gate4<T>(hv.lo, ov.lo);
+                    res.hi = gate4<T>(hv.hi, ov.hi);
+                    *reinterpret_cast<Pair*>(gg + (size_t)rr * rsB * sizeof(T) + 16 * cc) = res;
+                });
+            }
+        }
+    }
+    if constexpr (STRICT && MODE == MODE_FWD) {
+        if (a.out_lo) {
+#pragma unroll
+            for (int d = 0; d < NDB; d++)
+#pragma unroll
+                for (int a4 = 0; a4 < 4; a4++) put(d, a4, low[d][a4]);
+            char* const gl = reinterpret_cast<char*>(a.out_lo) + (hoff + r0) * D * sizeof(T);
+            pieces([&](int rr, int cc, int) { *reinterpret_cast<uint4*>(gl + (size_t)rr * D * sizeof(T) + 16 * cc) = piece_at(rr, cc); });
+        }
+    }
+    if constexpr (MODE == MODE_FWD && !PARITY) {
+        if (a.O && mine && !((left_out >> c32) & 1)) {  // gated copy from the fp32 accumulators
+            const T* og = reinterpret_cast<const T*>(a.O) + offB + (size_t)row * rsB;
+            T* outg = reinterpret_cast<T*>(a.out_gated) + offB + (size_t)row * rsB;
+#pragma unroll
+            for (int d = 0; d < NDB; d++)
+#pragma unroll
+                for (int a4 = 0; a4 < 4; a4++) {
+                    const int col = 32 * d + 8 * a4 + 4 * h;
+                    const f32x4 of = __builtin_convertvector(*reinterpret_cast<const typename R::vec4*>(og + col), f32x4);
+                    f32x4 v;
+#pragma unroll
+                    for (int c = 0; c < 4; c++) v[c] = oacc[d][4 * a4 + c] * onorm * silu(of[c]);
+                    *reinterpret_cast<typename R::vec4*>(outg + col) = R::cvt4(v);
                 }
-            }
-        if constexpr (MODE == MODE_FWD) {
-            if (a.O) {  // gated copy from the fp32 accumulators
-                const T* og = reinterpret_cast<const T*>(a.O) + offB + (size_t)row * rsB;
-                T* outg = reinterpret_cast<T*>(a.out_gated) + offB + (size_t)row * rsB;
-#pragma unroll
-                for (int d = 0; d < NDB; d++)
-#pragma unroll
-                    for (int a4 = 0; a4 < 4; a4++) {
-                        const int col = 32 * d + 8 * a4 + 4 * h;
-                        const f32x4 of = __builtin_convertvector(*reinterpret_cast<const typename R::vec4*>(og + col), f32x4);
-                        f32x4 v;
-                        if constexpr (PARITY) {   // (from h as it is written, like the other row kernels)
-#pragma unroll
-                            for (int c = 0; c < 4; c++) v[c] = oacc[d][4 * a4 + c] * onorm;
-                            *reinterpret_cast<typename R::vec4*>(outg + col) = gate4<T>(R::cvt4(v), *reinterpret_cast<const typename R::vec4*>(og + col));
-                            continue;
-                        }
-#pragma unroll
-                        for (int c = 0; c < 4; c++) v[c] = oacc[d][4 * a4 + c] * onorm * silu(of[c]);
-                        *reinterpret_cast<typename R::vec4*>(outg + col) = R::cvt4(v);
-                    }
-            }
         }
     }
 #endif
@@ -747,14 +865,14 @@ static int launch_row_ts(const RowArgs& a, hipStream_t st) {
     static hipError_t attr_rc = hipSuccess;
     std::call_once(once, [&] {
         attr_rc = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      (int)(Cfg::STAGES_BYTES + 2048 * sizeof(double)));
+                                      (int)(Cfg::STAGES_BYTES + 2048 * sizeof(double) + sizeof(double) + D * sizeof(float)));
     });
     if (attr_rc != hipSuccess) return (int)attr_rc;
     const int nQT = (a.S + ROW_BQ - 1) / ROW_BQ;
     // (the table is as long as what a row may meet: with the whole sequence's, two workgroups shared a CU up to 118784 positions only, 64 more cost
     // 55 -> 74 us in chunks)
     const int met = a.chunk_len > 0 && a.chunk_len / GRAN < a.NG ? a.chunk_len / GRAN : a.NG;
-    hipLaunchKernelGGL(kern, dim3(a.BH * nQT), dim3(256), Cfg::STAGES_BYTES + (size_t)met * sizeof(double), st, a);
+    hipLaunchKernelGGL(kern, dim3(a.BH * nQT), dim3(256), Cfg::STAGES_BYTES + (size_t)met * sizeof(double) + (a.chunk_len > 0 ? sizeof(double) + D * sizeof(float) : 0), st, a);
     return (int)hipGetLastError();
 }
 
