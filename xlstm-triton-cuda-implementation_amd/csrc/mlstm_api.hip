@@ -407,10 +407,9 @@ int scan_forward_impl(const void* q, const void* k, const void* v, const void* f
     }
     float* seg_state = c.take<float>(scan_segment_state_bytes((int)z.BH, (int)z.S, (int)z.D) / 4);
     if (m_out) m = m_out;
-    (void)bw;
     {
         Timed t(MLSTM_K_GATES, st);
-        hipError_t e = launch_gates(gate_dtype, f, i, alpha2, beta2, G2, m, ek2, amax2, (int)z.BH, (int)z.S, st, z.lg, z.gate_form);
+        hipError_t e = launch_gates(gate_dtype, f, i, alpha2, beta2, G2, m, ek2, amax2, bw, (int)z.BH, (int)z.S, st, z.lg, z.gate_form);
         if (e != hipSuccess) return (int)e;
     }
     ScanArgs a{};
@@ -440,7 +439,7 @@ int forward_impl(const void* q, const void* k, const void* v, const void* f, con
     if (!b) b = w.bw;
     {
         Timed t(MLSTM_K_GATES, st);
-        hipError_t e = launch_gates(gate_dtype, f, i, alpha2, beta2, G2, m, ek2, amax2, (int)z.BH, (int)z.S, st, z.lg, z.gate_form, stamp);
+        hipError_t e = launch_gates(gate_dtype, f, i, alpha2, beta2, G2, m, ek2, amax2, w.bw, (int)z.BH, (int)z.S, st, z.lg, z.gate_form, stamp);
         if (e != hipSuccess) return (int)e;
     }
     RowArgs a{};
@@ -754,7 +753,7 @@ int backward_impl(const void* dh, const void* q, const void* k, const void* v, c
             mm = const_cast<float*>(m);
         } else {
             Timed t(MLSTM_K_GATES, st);
-            hipError_t e = launch_gates(gate_dtype, f, i, alpha2, beta2, G2, mm, ek2, amax2, (int)z.BH, (int)z.S, st, z.lg, z.gate_form);
+            hipError_t e = launch_gates(gate_dtype, f, i, alpha2, beta2, G2, mm, ek2, amax2, w.bw, (int)z.BH, (int)z.S, st, z.lg, z.gate_form);
             if (e != hipSuccess) return (int)e;
         }
         bb = const_cast<float*>(b);

@@ -18,178 +18,250 @@
 namespace mlstm {
 
 constexpr int GATES_MAX_GRANULES = 2048;  // S <= 131072
+constexpr int GATES_WAVES = 16;           // waves per workgroup, a granule each at a time
 
-// fp64 prefix over granules by the first wave, 64 granules at a time: exclusive sum G of the totals (sT), then the running
-// maximum R of (P - G) over EARLIER granules (sP), by log-step lane shuffles (a serial loop of one lane costs a dependent
-// LDS round trip per granule)
-__device__ __forceinline__ void granule_prefix(double* sT, double* sP, int NG, int wave, int lane) {
-    if (wave == 0) {
-        double run = 0.0, rmax = -INFINITY;
-        for (int g0 = 0; g0 < NG; g0 += 64) {
-            const int g = g0 + lane;
-            const double tot = g < NG ? sT[g] : 0.0, p = g < NG ? sP[g] : -INFINITY;
-            double incl = tot;
-#pragma unroll
-            for (int d = 1; d < 64; d <<= 1) {
-                const double up = __shfl_up(incl, d);
-                if (lane >= d) incl += up;
-            }
-            const double excl = run + (incl - tot);       // G of this granule
-            double mx = p - excl;                          // this granule's candidate for later granules
-#pragma unroll
-            for (int d = 1; d < 64; d <<= 1) {
-                const double up = __shfl_up(mx, d);
-                if (lane >= d) mx = fmax(mx, up);
-            }
-            double before = __shfl_up(mx, 1);              // maximum over earlier granules of this chunk
-            if (lane == 0) before = -INFINITY;
-            if (g < NG) { sT[g] = excl; sP[g] = fmax(rmax, before); }
-            run += __shfl(incl, 63);
-            rmax = fmax(rmax, __shfl(mx, 63));
-        }
-    }
+// the DPP scans of mlstm_device.h on doubles, two moves per step
+template <int CTRL>
+__device__ __forceinline__ double dpp_d(double old, double src) {
+    const long long o = __builtin_bit_cast(long long, old), x = __builtin_bit_cast(long long, src);
+    const int lo = __builtin_amdgcn_update_dpp((int)o, (int)x, CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp((int)(o >> 32), (int)(x >> 32), CTRL, 0xf, 0xf, false);
+    return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+}
+__device__ __forceinline__ double readlane_d(double v, int lane) {
+    const long long x = __builtin_bit_cast(long long, v);
+    const int lo = __builtin_amdgcn_readlane((int)x, lane), hi = __builtin_amdgcn_readlane((int)(x >> 32), lane);
+    return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
+}
+struct AddD { static __device__ __forceinline__ double id() { return 0.0; } static __device__ __forceinline__ double f(double a, double b) { return a + b; } };
+struct MaxD { static __device__ __forceinline__ double id() { return -INFINITY; } static __device__ __forceinline__ double f(double a, double b) { return fmax(a, b); } };
+template <typename Op>
+__device__ __forceinline__ double wave_scan_inclusive_d(double v, int lane) {
+    v = Op::f(v, dpp_d<0x111>(Op::id(), v));
+    v = Op::f(v, dpp_d<0x112>(Op::id(), v));
+    v = Op::f(v, dpp_d<0x114>(Op::id(), v));
+    v = Op::f(v, dpp_d<0x118>(Op::id(), v));
+    const double r0 = readlane_d(v, 15), r1 = Op::f(r0, readlane_d(v, 31)), r2 = Op::f(r1, readlane_d(v, 47));
+    double c = Op::id();
+    if (lane >= 16) c = r0;
+    if (lane >= 32) c = r1;
+    if (lane >= 48) c = r2;
+    return Op::f(c, v);
 }
 
-// per-position outputs of one granule from the in-granule cumulative sum c and alpha (natural units)
-__device__ __forceinline__ void gates_outputs(float c, float al, bool ok, double Gg, double Rg, size_t pos, size_t mpos, size_t gidx, int lane,
-                                              float* alpha2, float* beta2, double* G2, float* M, float* ek2, float* amax2) {
+// fp64 prefix over up to 64 granules, one per lane: exclusive sum G of the totals behind `run`, and the running maximum R of (P - G) over
+// EARLIER granules, `rmax` those before the 64.  The totals of 64 logarithms are floats: their sums are exact in fp64, in any order, unless they
+// lie 2^18 apart.  (By log-step lane shuffles, an LDS round trip each, the two scans took 0.9 us; these take 0.2.)
+__device__ __forceinline__ void granule_scan(double tot, double p, double run, int lane, double& incl, double& excl, double& mx) {
+    incl = wave_scan_inclusive_d<AddD>(tot, lane);
+    excl = run + (incl - tot);                               // G of this granule
+    mx = wave_scan_inclusive_d<MaxD>(p - excl, lane);        // with this granule's candidate for later ones
+}
+__device__ __forceinline__ double before_lane(double mx, int lane) {   // maximum over the earlier granules of these 64
+    double x = dpp_d<0x111>(-INFINITY, mx);
+    const double r0 = readlane_d(mx, 15), r1 = readlane_d(mx, 31), r2 = readlane_d(mx, 47);
+    if (lane == 16) x = r0;
+    if (lane == 32) x = r1;
+    if (lane == 48) x = r2;
+    return x;
+}
+
+// what a position's outputs need beside the granules before its own, from the in-granule cumulative sum c and alpha (natural units): the
+// prefix maximum of alpha; written here: alpha2 (rows padded to whole granules: alpha = -inf there, so padded keys weigh nothing) and the
+// factorised weights for blocks of 32 keys that lie entirely below the diagonal: with c0 the block maximum of
+// alpha, exp2(alpha_j - beta_i + dG) = exp2(alpha_j - c0) * exp2(c0 - beta_i + dG); both factors are <= 1 there,
+// so the product under- or overflows only where the weight itself does.
+__device__ __forceinline__ float gates_local(float al, bool ok, size_t pos, size_t gidx, int lane, float* alpha2, float* ek2, float* amax2) {
     const float loc = wave_scan_inclusive<OpMax>(al);
+    const float al2 = product_apart(al, LOG2E);   // (rounded, also where the block maximum is taken off it)
+    alpha2[pos] = ok ? al2 : -INFINITY;
+    float lo, hi;
+    wave_half_max(al2, lo, hi);
+    const float c0 = lane < 32 ? lo : hi;
+    ek2[pos] = (ok && c0 > -INFINITY) ? fast_exp2(al2 - c0) : 0.0f;
+    if ((lane & 31) == 0) amax2[gidx * 2 + (lane >> 5)] = c0;
+    return loc;
+}
+// and with G and R of the granule
+__device__ __forceinline__ void gates_global(float c, float loc, bool ok, double Gg, double Rg, size_t pos, size_t mpos, size_t gidx, int lane,
+                                             float* beta2, double* G2, float* M) {
     const float carry = (float)(Rg + Gg);  // max over earlier granules of (alpha_j - G_g(j)) + G_g ; -inf for g == 0
     const float be = fmaxf(loc, carry);
-    // alpha2 / beta2 rows are padded to whole granules: alpha = -inf there, so padded keys weigh nothing
-    alpha2[pos] = ok ? al * LOG2E : -INFINITY;
     beta2[pos] = ok ? be * LOG2E : 0.0f;
     if (ok) M[mpos] = c + be;
-    // Factorised weights for blocks of 32 keys that lie entirely below the diagonal: with c0 the block maximum of
-    // alpha, exp2(alpha_j - beta_i + dG) = exp2(alpha_j - c0) * exp2(c0 - beta_i + dG); both factors are <= 1 there,
-    // so the product under- or overflows only where the weight itself does.
-    float lo, hi;
-    wave_half_max(al * LOG2E, lo, hi);
-    const float c0 = lane < 32 ? lo : hi;
-    ek2[pos] = (ok && c0 > -INFINITY) ? fast_exp2(al * LOG2E - c0) : 0.0f;
-    if ((lane & 31) == 0) amax2[gidx * 2 + (lane >> 5)] = c0;
     if (lane == 0) G2[gidx] = Gg * LOG2E_D;
 }
 
 // log-sigmoid of the forget gate at position t from what the caller's F holds (see launch_gates): the pre-activation,
 // the log-sigmoid itself, or its cumulative sum over the head (then the difference of two neighbours)
+struct GateIn { float x, before, i; };
 template <typename TG>
-__device__ __forceinline__ float forget_log(const TG* f, size_t ss, int t, int form) {
-    const float x = (float)f[(size_t)t * ss];
-    if (form == MLSTM_GATE_RAW) return log_sigmoid(x);
-    if (form == MLSTM_GATE_LOGSIGMOID) return x;
-    return t > 0 ? x - (float)f[(size_t)(t - 1) * ss] : x;
+__device__ __forceinline__ GateIn gate_in(const TG* f, const TG* ig, size_t ss, int t, int S, int form) {   // (positions past the end: the last one's)
+    t = t < S ? t : S - 1;
+    GateIn v;
+    v.x = (float)f[(size_t)t * ss];
+    v.i = (float)ig[(size_t)t * ss];
+    v.before = form == MLSTM_GATE_CUMSUM && t > 0 ? (float)f[(size_t)(t - 1) * ss] : 0.f;
+    return v;
 }
+__device__ __forceinline__ float forget_log(const GateIn& v, int t, int form) {
+    if (form == MLSTM_GATE_RAW) return log_sigmoid(v.x);
+    if (form == MLSTM_GATE_LOGSIGMOID) return v.x;
+    return t > 0 ? v.x - v.before : v.x;
+}
+__device__ __forceinline__ float last_lane(float v) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63)); }
 
-// Sequences of up to 16 * GPW granules (GPW = 4, 8, 16: S <= 16384): every wave keeps its granules' cumulative sums and alphas in registers
-// between the two passes, and issues all its loads before the first scan (one memory round trip instead of one per granule
-// and pass).
+// Sequences of up to 16 * GPW granules (GPW = 1, 2, 4: S <= 4096) in one launch: a workgroup writes `per` granules (a power of two of up to 16) and
+// forms the totals of all granules up to those by itself, one per wave and turn.  What bounds it is instruction issue on one CU, some 90
+// instructions per granule for the totals and as many for the outputs; all loads are issued before the first scan.  us, one
+// workgroup of 16 waves per head with GPW = 4 whatever the length, and the prefix by lane shuffles / now, one head: S = 64 3.9 / 2.8, 640 4.6 / 3.3,
+// 1000 5.0 / 3.4; eight: 2048 7.4 / 5.7, 4096 10.9 / 8.0.  With as many workgroups as CUs the totals formed several times over cost more than
+// the outputs saved, hence per = 16 there (32 heads x 4096 10.0 / 8.2; 256 x 1000 6.4 / 5.3 on 16, 5.8 on 4).
 template <typename TG, int GPW>
 __global__ __launch_bounds__(1024) void gates_kernel_reg(const TG* __restrict__ F, const TG* __restrict__ I, float* __restrict__ alpha2,
                                                         float* __restrict__ beta2, double* __restrict__ G2, float* __restrict__ M,
-                                                        float* __restrict__ ek2, float* __restrict__ amax2, int S, int NG, Lay lg, int form,
+                                                        float* __restrict__ ek2, float* __restrict__ amax2, int S, int NG, int per, Lay lg, int form,
                                                         SavedStamp stamp) {
-    stamp_apply(stamp, blockIdx.x == 0, threadIdx.x);
-    __shared__ double sT[16 * GPW];
-    __shared__ double sP[16 * GPW];
-    const int bh = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    stamp_apply(stamp, blockIdx.x == 0 && blockIdx.y == 0, threadIdx.x);
+    __shared__ double sT[GATES_WAVES * GPW];
+    __shared__ double sP[GATES_WAVES * GPW];
+    // (the last granules first: they take longest)
+    const int bh = blockIdx.x, first = per * (int)(gridDim.y - 1 - blockIdx.y), seg = first / GATES_WAVES, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const size_t gs = (size_t)lg.ss;
     const TG* f = F + lg.head(bh);
     const TG* ig = I + lg.head(bh);
-    float fv[GPW], iv[GPW], c[GPW], al[GPW];
+    GateIn in[GPW];
+    float c = 0.f, al = -INFINITY;
+#pragma unroll
+    for (int k = 0; k < GPW; k++) in[k] = gate_in(f, ig, gs, (wave + GATES_WAVES * k) * GRAN + lane, S, form);
 #pragma unroll
     for (int k = 0; k < GPW; k++) {
-        const int t = (wave + 16 * k) * GRAN + lane;
-        const bool ok = t < S;
-        fv[k] = ok ? forget_log(f, gs, t, form) : 0.0f;
-        iv[k] = ok ? (float)ig[(size_t)t * gs] : 0.0f;
+        const int g = wave + GATES_WAVES * k, t = g * GRAN + lane;
+        if (g < first + per && g < NG) {
+            c = wave_scan_inclusive<OpAdd>(t < S ? forget_log(in[k], t, form) : 0.0f);
+            al = t < S ? in[k].i - c : -INFINITY;
+            const float p = wave_reduce<OpMax>(al);
+            const float tot = last_lane(c);
+            if (lane == 0) { sT[g] = (double)tot; sP[g] = (double)p; }
+        }
     }
-#pragma unroll
-    for (int k = 0; k < GPW; k++) {
-        const int g = wave + 16 * k, t = g * GRAN + lane;
-        const bool ok = t < S;
-        const float lf = ok ? fv[k] : 0.0f;
-        c[k] = wave_scan_inclusive<OpAdd>(lf);
-        al[k] = ok ? iv[k] - c[k] : -INFINITY;
-        const float p = wave_reduce<OpMax>(al[k]);
-        const float tot = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, c[k]), 63));
-        if (lane == 0 && g < NG) { sT[g] = (double)tot; sP[g] = (double)p; }
-    }
+    // (c and al are now those of the last granule passed, the wave's own)
+    const int g = wave + GATES_WAVES * seg, t = g * GRAN + lane;
+    const bool mine = g >= first && g < first + per && g < NG, ok = t < S;
+    const size_t pos = (size_t)bh * NG * GRAN + t, gidx = (size_t)bh * NG + g;
+    const float loc = mine ? gates_local(al, ok, pos, gidx, lane, alpha2, ek2, amax2) : 0.f;
     __syncthreads();
-    granule_prefix(sT, sP, NG, wave, lane);
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < GPW; k++) {
-        const int g = wave + 16 * k, t = g * GRAN + lane;
-        if (g < NG)
-            gates_outputs(c[k], al[k], t < S, sT[g], sP[g], (size_t)bh * NG * GRAN + t, (size_t)bh * S + t, (size_t)bh * NG + g, lane, alpha2,
-                          beta2, G2, M, ek2, amax2);
+    if (!mine) return;
+    {   // the prefix, by every wave for itself (a wave alone, with the others waiting for it, takes as long, and a barrier)
+        const int ng = g + 1;
+        double incl, excl, mx;
+        granule_scan(lane < ng ? sT[lane] : 0.0, lane < ng ? sP[lane] : -INFINITY, 0.0, lane, incl, excl, mx);
+        const double before = before_lane(mx, lane);
+        gates_global(c, loc, ok, readlane_d(excl, g), readlane_d(before, g), pos, (size_t)bh * S + t, gidx, lane, beta2, G2, M);
     }
 }
 
+// Longer sequences in two launches of a workgroup per 16 granules, each granule's totals formed once.  us, one workgroup per
+// head / now: one head of 8192 positions 16.6 / 8.0, 64 heads of 8192 20.1 / 12.0, of 16384 37.5 / 17.2 (at 4096 one launch of 8 is level with these two):
+//   gates_local_kernel   alpha2 and the key weights, which need no other granule; in beta2 the prefix maxima of alpha, in M the cumulative
+//                        sums, both of the granule alone and in natural units; totals: sum of the log-sigmoids and maximum of alpha per granule
+//   gates_carry_kernel   the granules before, and with them beta2, M and G2
 template <typename TG>
-__global__ __launch_bounds__(1024) void gates_kernel(const TG* __restrict__ F, const TG* __restrict__ I, float* __restrict__ alpha2,
-                                                    float* __restrict__ beta2, double* __restrict__ G2, float* __restrict__ M,
-                                                    float* __restrict__ ek2, float* __restrict__ amax2, int S, int NG, Lay lg, int form,
-                                                    SavedStamp stamp) {
-    stamp_apply(stamp, blockIdx.x == 0, threadIdx.x);
-    __shared__ double sT[GATES_MAX_GRANULES];  // granule totals of lf, then exclusive prefix G
-    __shared__ double sP[GATES_MAX_GRANULES];  // granule maxima of alpha, then running max R of (P - G) over earlier granules
-    const int bh = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+__global__ __launch_bounds__(1024) void gates_local_kernel(const TG* __restrict__ F, const TG* __restrict__ I, float* __restrict__ alpha2,
+                                                          float* __restrict__ beta2, float2* __restrict__ totals, float* __restrict__ M,
+                                                          float* __restrict__ ek2, float* __restrict__ amax2, int S, int NG, Lay lg, int form,
+                                                          SavedStamp stamp) {
+    stamp_apply(stamp, blockIdx.x == 0 && blockIdx.y == 0, threadIdx.x);
+    const int bh = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    const int g = blockIdx.y * GATES_WAVES + __builtin_amdgcn_readfirstlane(tid >> 6), t = g * GRAN + lane;
+    if (g >= NG) return;
     const size_t gs = (size_t)lg.ss;
-    const TG* f = F + lg.head(bh);
-    const TG* ig = I + lg.head(bh);
-
-    // pass 1: per-granule total of lf and maximum of alpha
-    for (int g = wave; g < NG; g += 16) {
-        int t = g * GRAN + lane;
-        bool ok = t < S;
-        float lf = ok ? forget_log(f, gs, t, form) : 0.0f;
-        float c = wave_scan_inclusive<OpAdd>(lf);
-        float al = ok ? (float)ig[(size_t)t * gs] - c : -INFINITY;
-        float p = wave_reduce<OpMax>(al);
-        float tot = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, c), 63));
-        if (lane == 0) { sT[g] = (double)tot; sP[g] = (double)p; }
+    const bool ok = t < S;
+    const GateIn in = gate_in(F + lg.head(bh), I + lg.head(bh), gs, t, S, form);
+    const float c = wave_scan_inclusive<OpAdd>(ok ? forget_log(in, t, form) : 0.0f), al = ok ? in.i - c : -INFINITY;
+    const float p = wave_reduce<OpMax>(al), tot = last_lane(c);
+    const size_t pos = (size_t)bh * NG * GRAN + t, gidx = (size_t)bh * NG + g;
+    if (lane == 0) totals[gidx] = make_float2(tot, p);
+    beta2[pos] = gates_local(al, ok, pos, gidx, lane, alpha2, ek2, amax2);
+    if (ok) M[(size_t)bh * S + t] = c;
+}
+__global__ __launch_bounds__(1024) void gates_carry_kernel(const float2* __restrict__ totals, float* __restrict__ beta2, double* __restrict__ G2,
+                                                          float* __restrict__ M, int S, int NG) {
+    constexpr int GROUPS = GATES_MAX_GRANULES / 64;   // of 64 granules
+    __shared__ double sSum[GROUPS], sMax[GROUPS], sG[GATES_WAVES], sR[GATES_WAVES];
+    const int bh = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int first = blockIdx.y * GATES_WAVES, mygroup = first / 64;   // (the workgroup's granules lie in one group)
+    const float2* tp = totals + (size_t)bh * NG;
+    const int g = first + wave, t = g * GRAN + lane;
+    const bool mine = g < NG, ok = mine && t < S;
+    const size_t pos = (size_t)bh * NG * GRAN + t, mpos = (size_t)bh * S + t;
+    const float loc = mine ? beta2[pos] : 0.f, c = ok ? M[mpos] : 0.f;
+    double tot[2], p[2];   // of groups wave and wave + 16
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const int n = 64 * (wave + GATES_WAVES * k) + lane;
+        const bool there = wave + GATES_WAVES * k <= mygroup && n < NG;
+        const float2 x = there ? tp[n] : make_float2(0.f, -INFINITY);
+        tot[k] = (double)x.x;
+        p[k] = (double)x.y;
+    }
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+        if (wave + GATES_WAVES * k <= mygroup) {
+            const double incl = wave_scan_inclusive_d<AddD>(tot[k], lane);
+            if (lane == 63) sSum[wave + GATES_WAVES * k] = incl;
+        }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        const int group = wave + GATES_WAVES * k;
+        if (group <= mygroup) {
+            double run = 0.0, incl, excl, mx;
+            for (int n = 0; n < group; n++) run += sSum[n];
+            granule_scan(tot[k], p[k], run, lane, incl, excl, mx);
+            if (lane == 63) sMax[group] = mx;
+            const int own = 64 * group + lane - first;
+            const double before = before_lane(mx, lane);
+            if (group == mygroup && own >= 0 && own < GATES_WAVES) { sG[own] = excl; sR[own] = before; }
+        }
     }
     __syncthreads();
-    granule_prefix(sT, sP, NG, wave, lane);
-    __syncthreads();
-    // pass 2: per-position outputs
-    for (int g = wave; g < NG; g += 16) {
-        int t = g * GRAN + lane;
-        bool ok = t < S;
-        float lf = ok ? forget_log(f, gs, t, form) : 0.0f;
-        float c = wave_scan_inclusive<OpAdd>(lf);
-        float al = ok ? (float)ig[(size_t)t * gs] - c : -INFINITY;
-        gates_outputs(c, al, ok, sT[g], sP[g], (size_t)bh * NG * GRAN + t, (size_t)bh * S + t, (size_t)bh * NG + g, lane, alpha2, beta2, G2, M,
-                      ek2, amax2);
-    }
+    if (!mine) return;
+    double rmax = -INFINITY;
+    for (int n = 0; n < mygroup; n++) rmax = fmax(rmax, sMax[n]);
+    gates_global(c, loc, ok, sG[wave], fmax(rmax, sR[wave]), pos, mpos, (size_t)bh * NG + g, lane, beta2, G2, M);
 }
 
 template <typename TG>
 static hipError_t launch_gates_t(const void* F, const void* I, float* alpha2, float* beta2, double* G2, float* M, float* ek2,
-                                 float* amax2, int BH, int S, hipStream_t st, const Lay& lg, int form, const SavedStamp& stamp) {
-    int NG = (S + GRAN - 1) / GRAN;
-    if (NG <= 16 * 4)
-        hipLaunchKernelGGL((gates_kernel_reg<TG, 4>), dim3(BH), dim3(1024), 0, st, (const TG*)F, (const TG*)I, alpha2, beta2, G2, M, ek2, amax2, S, NG, lg, form, stamp);
-    else if (NG <= 16 * 8)
-        hipLaunchKernelGGL((gates_kernel_reg<TG, 8>), dim3(BH), dim3(1024), 0, st, (const TG*)F, (const TG*)I, alpha2, beta2, G2, M, ek2, amax2, S, NG, lg, form, stamp);
-    else if (NG <= 16 * 16)
-        hipLaunchKernelGGL((gates_kernel_reg<TG, 16>), dim3(BH), dim3(1024), 0, st, (const TG*)F, (const TG*)I, alpha2, beta2, G2, M, ek2, amax2, S, NG, lg, form, stamp);
-    else
-        hipLaunchKernelGGL(gates_kernel<TG>, dim3(BH), dim3(1024), 0, st, (const TG*)F, (const TG*)I, alpha2, beta2, G2, M, ek2, amax2, S, NG, lg, form, stamp);
+                                 float* amax2, void* scratch, int BH, int S, hipStream_t st, const Lay& lg, int form, const SavedStamp& stamp) {
+    const int NG = (S + GRAN - 1) / GRAN;
+    const TG *f = (const TG*)F, *i = (const TG*)I;
+    const int per = (long long)BH * ((NG + 3) / 4) <= 256 ? 4 : GATES_WAVES, parts = (NG + per - 1) / per;
+    if (NG <= GATES_WAVES)
+        hipLaunchKernelGGL((gates_kernel_reg<TG, 1>), dim3(BH, parts), dim3(1024), 0, st, f, i, alpha2, beta2, G2, M, ek2, amax2, S, NG, per, lg, form, stamp);
+    else if (NG <= 2 * GATES_WAVES)
+        hipLaunchKernelGGL((gates_kernel_reg<TG, 2>), dim3(BH, parts), dim3(1024), 0, st, f, i, alpha2, beta2, G2, M, ek2, amax2, S, NG, per, lg, form, stamp);
+    else if (NG <= 4 * GATES_WAVES)
+        hipLaunchKernelGGL((gates_kernel_reg<TG, 4>), dim3(BH, parts), dim3(1024), 0, st, f, i, alpha2, beta2, G2, M, ek2, amax2, S, NG, per, lg, form, stamp);
+    else {
+        const dim3 grid(BH, (NG + GATES_WAVES - 1) / GATES_WAVES);
+        float2* const totals = static_cast<float2*>(scratch);
+        hipLaunchKernelGGL(gates_local_kernel<TG>, grid, dim3(1024), 0, st, f, i, alpha2, beta2, totals, M, ek2, amax2, S, NG, lg, form, stamp);
+        hipLaunchKernelGGL(gates_carry_kernel, grid, dim3(1024), 0, st, totals, beta2, G2, M, S, NG);
+    }
     return hipGetLastError();
 }
 
 hipError_t launch_gates(int gate_dtype, const void* F, const void* I, float* alpha2, float* beta2, double* G2, float* M, float* ek2,
-                        float* amax2, int BH, int S, hipStream_t st, const Lay& lg, int form, const SavedStamp* stamp_in) {
+                        float* amax2, void* scratch, int BH, int S, hipStream_t st, const Lay& lg, int form, const SavedStamp* stamp_in) {
     const SavedStamp stamp = stamp_in ? *stamp_in : SavedStamp{};
     if ((S + GRAN - 1) / GRAN > GATES_MAX_GRANULES) return hipErrorInvalidValue;
     if (form == MLSTM_GATE_CUMSUM && gate_dtype != MLSTM_F32) return hipErrorInvalidValue;   // (16-bit types cannot hold the sum)
     switch (gate_dtype) {
-        case MLSTM_F32: return launch_gates_t<float>(F, I, alpha2, beta2, G2, M, ek2, amax2, BH, S, st, lg, form, stamp);
-        case MLSTM_F16: return launch_gates_t<_Float16>(F, I, alpha2, beta2, G2, M, ek2, amax2, BH, S, st, lg, form, stamp);
-        case MLSTM_BF16: return launch_gates_t<__bf16>(F, I, alpha2, beta2, G2, M, ek2, amax2, BH, S, st, lg, form, stamp);
+        case MLSTM_F32: return launch_gates_t<float>(F, I, alpha2, beta2, G2, M, ek2, amax2, scratch, BH, S, st, lg, form, stamp);
+        case MLSTM_F16: return launch_gates_t<_Float16>(F, I, alpha2, beta2, G2, M, ek2, amax2, scratch, BH, S, st, lg, form, stamp);
+        case MLSTM_BF16: return launch_gates_t<__bf16>(F, I, alpha2, beta2, G2, M, ek2, amax2, scratch, BH, S, st, lg, form, stamp);
     }
     return hipErrorInvalidValue;
 }

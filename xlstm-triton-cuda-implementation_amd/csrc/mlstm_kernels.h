@@ -65,11 +65,12 @@ __device__ __forceinline__ void stamp_apply(const SavedStamp& s, bool first_bloc
 // ek2 [BH, NG*64] = exp2(alpha2 - block max), amax2 [BH, NG*2] = the maxima of alpha2 over blocks of 32 positions.
 // lg: layout of F and I.  gate_form: what F holds (MLSTM_GATE_RAW: the forget gate's pre-activation, _LOGSIGMOID: its
 // log-sigmoid, _CUMSUM: the cumulative sum of that over the positions of a head).
+// scratch: 8 BH NG bytes (on an 8-byte boundary), written and read where S > 4096.
 hipError_t launch_gates(int gate_dtype, const void* F, const void* I, float* alpha2, float* beta2, double* G2, float* M, float* ek2,
-                        float* amax2, int BH, int S, hipStream_t st, const Lay& lg, int gate_form, const SavedStamp* stamp = nullptr);
+                        float* amax2, void* scratch, int BH, int S, hipStream_t st, const Lay& lg, int gate_form, const SavedStamp* stamp = nullptr);
 inline hipError_t launch_gates(int gate_dtype, const void* F, const void* I, float* alpha2, float* beta2, double* G2, float* M, float* ek2,
-                               float* amax2, int BH, int S, hipStream_t st) {
-    return launch_gates(gate_dtype, F, I, alpha2, beta2, G2, M, ek2, amax2, BH, S, st, dense_layout(BH, S, 1), MLSTM_GATE_RAW);
+                               float* amax2, void* scratch, int BH, int S, hipStream_t st) {
+    return launch_gates(gate_dtype, F, I, alpha2, beta2, G2, M, ek2, amax2, scratch, BH, S, st, dense_layout(BH, S, 1), MLSTM_GATE_RAW);
 }
 
 extern bool g_force_generic;  // see mlstm_force_generic_kernels

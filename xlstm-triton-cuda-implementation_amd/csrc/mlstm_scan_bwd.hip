@@ -174,7 +174,7 @@ int launch_scan_backward(const ScanBwdArgs& a, char* ws, hipStream_t st, void (*
     const float* bsum = a.h_kept ? a.b_kept : p.b;
 
     mark(MLSTM_K_GATES, st, true);
-    const hipError_t ge = launch_gates(MLSTM_F32, a.f, a.i, p.alpha2, p.beta2, p.G2, p.m, p.ek2, p.amax2, BH, S, st);
+    const hipError_t ge = launch_gates(MLSTM_F32, a.f, a.i, p.alpha2, p.beta2, p.G2, p.m, p.ek2, p.amax2, p.b, BH, S, st);
     mark(MLSTM_K_GATES, st, false);
     if (ge != hipSuccess) return (int)ge;
 
