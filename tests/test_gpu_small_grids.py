@@ -137,3 +137,19 @@ def test_the_first_chunk_at_head_dimension_64_is_the_uncut_sequence(S, heads, la
                                                ("plain", 1025, 60, "bsnd")])
 def test_fp32_pairs_of_workgroups_per_cu_give_the_same_bits(op, S, heads, layout):
     test_a_head_alone_is_the_head_of_a_full_chip(op, S, 64, heads, layout, torch.float32)
+
+
+# roww_kernel on 32 rows per workgroup (up to 128 granules of 64 rows) and on 64 (up to 256, uncut sequences a few more) against row8_kernel: rows that end in
+# either half of a granule, one to five rounds of 128 keys, diagonal blocks in either half of a round, and the chunks' state in front of them
+@pytest.mark.parametrize("op,S,layout", [("plain", 1, "bnsd"), ("gated", 31, "bsnd"), ("plain", 32, "bnsd"), ("plain", 33, "bsnd"), ("plain", 96, "bnsd"),
+                                         ("gated", 129, "bnsd"), ("plain", 160, "bsnd"), ("plain", 193, "bnsd"), ("plain", 257, "bnsd"), ("gated", 321, "bnsd"),
+                                         ("plain", 385, "bsnd"), ("plain", 450, "bnsd"), ("plain", 545, "bnsd"), ("plain", 990, "bsnd"), ("plain", 1024, "bnsd"),
+                                         ("gated", 1025, "bsnd"), ("plain", 1185, "bnsd"), ("plain", 1700, "bnsd")])
+@pytest.mark.parametrize("D", [128, 256])
+def test_row_workgroups_of_every_size_give_the_same_bits(op, S, D, layout):
+    NG = (S + 63) // 64
+    sizes = (1, 128 // NG + 1, (256 if S >= 1024 else 256 + 8 * NG) // NG + 1)
+    rows, gates = _inputs(sizes[-1], S, D, torch.bfloat16, layout)
+    small, middle, large = [_step(op, rows, gates, heads) for heads in sizes]
+    for name, a, b, c in zip(range(10), small, middle, large):
+        assert bool(torch.isfinite(c.float()).all()) and torch.equal(a, c[:, :1]) and torch.equal(b, c[:, :sizes[1]]), name

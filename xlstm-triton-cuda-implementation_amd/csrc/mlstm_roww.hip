@@ -1,12 +1,12 @@
 // Row-parallel tile kernel for the 16-bit types at D >= 128 where few workgroups would run: the same math and, element by
 // element, the same order of operations as mlstm_row8.hip, hence the same bits, on half as many rows per workgroup and with every
-// key tile's work spread over all eight waves.
+// key tile's work spread over all waves.
 //
 // What bounds a small call is one workgroup's walk of its key tiles, and in the eight-wave producer / consumer kernel that walk
 // takes 1.2 us per 64 keys (products, weights, hand-over, products, one tile after the other) whatever the number of workgroups.
 // There is no online maximum (the row maximum is a prefix maximum of the gates), so the weights of several tiles can be formed
-// side by side; only the accumulation over the keys is a chain.  A workgroup here owns one granule of 64 rows and takes 128 keys
-// at a time in two phases:
+// side by side; only the accumulation over the keys is a chain.  A workgroup here owns 64 rows (RB = 2: eight waves) or 32 (RB = 1: four) and takes
+// 128 keys at a time in two phases:
 //   phase 1   wave (rb, kb) = (row block of 32, key block of 32):  S^T = K Q^T (dQ pass: dC^T = V dH^T) for its 32 x 32 block, gate
 //             weights, the 16-bit weights and the block's share of the row sums to LDS;
 //   phase 2   wave (rb, c) = (row block, D / 4 of the output columns):  H^T += V^T P^T (dQ^T += K^T G^T) over the 128 keys.
@@ -23,22 +23,23 @@ namespace mlstm {
 constexpr int RW_FWD = 0, RW_DQ = 1;
 constexpr int RW_MOST_KEYS = 1024;   // keys a row may meet: their scalars stay in LDS for the whole kernel
 
-template <typename T, int D>
+template <typename T, int D, int RB>
 struct RowwCfg {
     static constexpr size_t TILE_BYTES = (size_t)GRAN * D * sizeof(T);
     static constexpr int NST = D == 256 ? 1 : 2;                       // stages of 128 keys for each of Y1 and Y2: 128 KB in all
     static constexpr size_t POOL_BYTES = 4 * NST * TILE_BYTES;
-    static constexpr size_t P_BYTES = 4 * 2 * 2 * 64 * 16;             // [key block][row block][16 keys][lane] x 16 B
-    static constexpr size_t PART_BYTES = 4 * 2 * 64 * 8;               // [key block][row block][lane] x {sum, row factor}; dQ pass: [column block][row block][lane]
-    static constexpr size_t MISC_FLOATS = 2 * 2 * 32 + 2 * 32 * 2 + D + RW_MOST_KEYS / GRAN;   // row sums, 1/n and db, vector state, granule distances
+    static constexpr size_t P_BYTES = 4 * RB * 2 * 64 * 16;            // [key block][row block][16 keys][lane] x 16 B
+    static constexpr size_t PART_BYTES = 4 * RB * 64 * 8;              // [key block][row block][lane] x {sum, row factor}; dQ pass: [column block][row block][lane]
+    static constexpr size_t MISC_FLOATS = RB * 2 * 32 + RB * 32 * 2 + D + RW_MOST_KEYS / GRAN;   // row sums, 1/n and db, vector state, granule distances
     static size_t lds_bytes(int keys) { return POOL_BYTES + P_BYTES + PART_BYTES + MISC_FLOATS * 4 + (size_t)keys * 8 + GRAN * 4; }
 };
 
-template <typename T, int D, int MODE>
-__global__ __launch_bounds__(512) void roww_kernel(RowArgs a) {
+template <typename T, int D, int MODE, int RB>
+__global__ __launch_bounds__(256 * RB) void roww_kernel(RowArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using R = Tr<T>;
-    using Cfg = RowwCfg<T, D>;
+    using Cfg = RowwCfg<T, D, RB>;
+    constexpr int NT = 256 * RB, ROWS = 32 * RB;
     typedef typename R::frag frag;
     static_assert(R::HALF && (D == 128 || D == 256), "16-bit types, D = 128 or 256");
     constexpr int KW = R::KW, NS = D / KW, NC = D / 128, NST = Cfg::NST;
@@ -46,8 +47,8 @@ __global__ __launch_bounds__(512) void roww_kernel(RowArgs a) {
     frag* const pbuf = reinterpret_cast<frag*>(smem + Cfg::POOL_BYTES);
     float* const part = reinterpret_cast<float*>(smem + Cfg::POOL_BYTES + Cfg::P_BYTES);
     float* const bex = part + Cfg::PART_BYTES / 4;         // [rb][kh][32]
-    float* const stat = bex + 2 * 2 * 32;                  // [rb][32] x {1/n, db}
-    float* const nvl = stat + 2 * 32 * 2;                  // [D]
+    float* const stat = bex + RB * 2 * 32;                 // [rb][32] x {1/n, db}
+    float* const nvl = stat + RB * 32 * 2;                 // [D]
     float* const sdg = nvl + D;                            // granule of the rows minus granule j
     float* const sek = sdg + RW_MOST_KEYS / GRAN;          // ek of the keys, then alpha, then the block maxima
 
@@ -57,7 +58,7 @@ __global__ __launch_bounds__(512) void roww_kernel(RowArgs a) {
     int bh, qt;
     {
         // heaviest row tiles first over all heads; with a multiple of 8 heads a head's tiles run on one XCD
-        const int bid = blockIdx.x, nQT = NG;
+        const int bid = blockIdx.x, nQT = NG * (GRAN / ROWS);
         if ((a.BH & 7) == 0) {
             const int rest = bid >> 3, ngrp = a.BH >> 3;
             bh = (rest % ngrp) * 8 + (bid & 7);
@@ -72,14 +73,14 @@ __global__ __launch_bounds__(512) void roww_kernel(RowArgs a) {
     size_t offA = a.la.head(bh), offB = a.lb.head(bh), offH = MODE == RW_DQ ? a.lh.head(bh) : 0;
     int chunk = 0;   // in chunks positions count from the chunk's first one (see mlstm_row8.hip)
     if (a.chunk_len > 0) {
-        chunk = (qt * GRAN) / a.chunk_len;
+        chunk = (qt * ROWS) / a.chunk_len;
         const int p0 = chunk * a.chunk_len;
         hoff += p0; poff += p0; goff += p0 / GRAN;
         offA += (size_t)p0 * rsA; offB += (size_t)p0 * rsB; offH += (size_t)p0 * rsH;
-        S -= p0; qt -= p0 / GRAN;
+        S -= p0; qt -= p0 / ROWS;
     }
-    const int r0 = GRAN * qt;
-    const int nJ = qt + 1;                                  // key tiles; the last one is the rows' own
+    const int r0 = ROWS * qt, gt = r0 / GRAN;
+    const int nJ = gt + 1;                                  // key tiles; the last one is the rows' own
     const int row = r0 + 32 * rb + c32, rowc = row < S ? row : S - 1;
     const size_t rsX = MODE == RW_FWD ? rsA : rsB, offX = MODE == RW_FWD ? offA : offB;
     const size_t rsO = MODE == RW_FWD ? rsB : rsA, offO = MODE == RW_FWD ? offB : offA;
@@ -95,12 +96,12 @@ __global__ __launch_bounds__(512) void roww_kernel(RowArgs a) {
     auto tile_at = [&](int n) { return reinterpret_cast<T*>(smem + (size_t)n * Cfg::TILE_BYTES); };
     auto y1_at = [&](int r, int t) { return tile_at(2 * (r & (NST - 1)) + t); };
     auto y2_at = [&](int r, int t) { return tile_at(2 * NST + 2 * (r & (NST - 1)) + t); };
-    TileDma<T, D, GRAN, 512> tdma;
+    TileDma<T, D, GRAN, NT> tdma;
     tdma.init(tid);
     const auto ra = tdma.rows(tid, (unsigned)(rsA * sizeof(T)));
     auto copy_tile = [&](T* dst, const T* src, int j) {
         if (j < full_tiles) tdma.issue(dst, src + (size_t)GRAN * j * rsA, ra);
-        else tile_dma_rolled<T, D, GRAN, 512>(dst, src, GRAN * j, S, tid, rsA);
+        else tile_dma_rolled<T, D, GRAN, NT>(dst, src, GRAN * j, S, tid, rsA);
     };
     auto copy_y1 = [&](int r) {
         copy_tile(y1_at(r, 0), Y1, 2 * r);
@@ -111,25 +112,34 @@ __global__ __launch_bounds__(512) void roww_kernel(RowArgs a) {
         if (2 * r + 1 < nJ) copy_tile(y2_at(r, 1), Y2, 2 * r + 1);
     };
     // (plain loads first: what they bring is used behind the copies' issue)
-    const double g_rows = a.G2[goff + qt], g_mine = a.G2[goff + (tid < nJ ? tid : 0)], g_end = chunk > 0 ? a.G2[goff - 1] : 0.0;
+    const double g_rows = a.G2[goff + gt], g_mine = a.G2[goff + (tid < nJ ? tid : 0)], g_end = chunk > 0 ? a.G2[goff - 1] : 0.0;
     const float beta_row = a.beta2[poff + rowc], beta_end = chunk > 0 ? a.beta2[poff - 1] : 0.f;
     const float n_mine = chunk > 0 && tid < D ? a.Nst[((size_t)bh * a.n_states + chunk - 1) * D + tid] : 0.f;
     const float m_row = MODE == RW_FWD || kb == 0 ? a.M[hoff + rowc] : 0.f;
     const float b_row = MODE == RW_DQ && kb == 0 ? a.Bin[hoff + rowc] : 0.f;
     // piece i of a pair of complete tiles j, j + 1
     auto copy_piece = [&](const T* src, T* d0, T* d1, int j, int i) {
-        constexpr int PW = TileDma<T, D, GRAN, 512>::PER_WAVE;
+        constexpr int PW = TileDma<T, D, GRAN, NT>::PER_WAVE;
         const int t = i / PW, n = i % PW;
         tdma.issue_range(t ? d1 : d0, src + (size_t)GRAN * (j + t) * rsA, n, n + 1, ra);
+    };
+    // the share of slot n of `slots` in the copy of a pair of tiles
+    auto pieces = [&](int n, int slots, auto&& f) __attribute__((always_inline)) {
+        constexpr int PP = 2 * TileDma<T, D, GRAN, NT>::PER_WAVE;
+#pragma unroll
+        for (int i = 0; i < PP; i++)
+            if (i >= n * PP / slots && i < (n + 1) * PP / slots) f(i);
     };
     // ---- prologue.  The rows' own operand, the state of the previous chunk and the first keys are requested at once, as far as the
     // pool holds them.  D = 256: X in tile 3 (then the last state tile), state tiles in 0, 1, 2; D = 128: X in tile 3 (Y1's second
     // stage), the state in Y2's second stage, the first keys in the first stages.
     const T* const xtile = tile_at(3);
     {
-        const auto rx = tdma.rows(tid, (unsigned)(rsX * sizeof(T)));
-        if (r0 + GRAN <= S) tdma.issue(tile_at(3), X + (size_t)r0 * rsX, rx);
-        else tile_dma_rolled<T, D, GRAN, 512>(tile_at(3), X, r0, S, tid, rsX);
+        TileDma<T, D, ROWS, NT> xdma;
+        xdma.init(tid);
+        const auto rx = xdma.rows(tid, (unsigned)(rsX * sizeof(T)));
+        if (r0 + ROWS <= S) xdma.issue(tile_at(3), X + (size_t)r0 * rsX, rx);
+        else tile_dma_rolled<T, D, ROWS, NT>(tile_at(3), X, r0, S, tid, rsX);
     }
     const T* const Cst = chunk > 0 ? reinterpret_cast<const T*>(a.Cst) + ((size_t)bh * a.n_states + chunk - 1) * D * D : nullptr;
     if (chunk > 0) {
@@ -143,7 +153,7 @@ __global__ __launch_bounds__(512) void roww_kernel(RowArgs a) {
     }
     if (NST == 2 || chunk == 0) copy_y1(0);
     if (NST == 2) copy_y2(0);
-    for (int t = tdma.wave_s; t < nJ; t += 8) {
+    for (int t = tdma.wave_s; t < nJ; t += NT / 64) {
         dma4(a.ek2 + poff + GRAN * t + lane, __builtin_amdgcn_readfirstlane(lds_offset_of(sek + GRAN * t)));
         dma4(a.alpha2 + poff + GRAN * t + lane, __builtin_amdgcn_readfirstlane(lds_offset_of(sal + GRAN * t)));
     }
@@ -194,6 +204,9 @@ __global__ __launch_bounds__(512) void roww_kernel(RowArgs a) {
 #pragma unroll
     for (int s = 0; s < NS; s++) pin(xf[s]);
     __syncthreads();   // X's tile is free; the rows' scalars are there
+    if constexpr (NST == 2) {
+        if (nJ > 2) copy_y1(1);
+    }
 
     // G groups of 16 contraction rows out of consecutive tiles, times the fragments operand(g)
     auto chain = [&](auto groups_tag, auto&& tile, auto&& operand, auto&& hook) {
@@ -255,138 +268,207 @@ __global__ __launch_bounds__(512) void roww_kernel(RowArgs a) {
                         rp = fmaf(acc[c][4 * a4 + e], qv[e], rp);
                     }
                 }
-                part[((NC * kb + c) * 2 + rb) * 64 + lane] = rp;
+                part[((NC * kb + c) * RB + rb) * 64 + lane] = rp;
             }
         }
     }
 
     // ---- the key tiles, two at a time
-    const int nR = (nJ + 1) / 2;
+    const int nR = (nJ + 1) / 2, rr = r0 + 32 * rb;
     float bsum = 0.f;   // waves kb < 2: the row sums over the key blocks of parity kb, in the order of the keys
-    for (int r = 0; r < nR; r++) {
-        const bool two = 2 * r + 1 < nJ;
-        dma_wait();
-        __syncthreads();   // this round's Y1 (NST == 2: and Y2) has landed; phase 2 of the previous round is over
-        // The copies under phase 1: NST == 1 this round's Y2, NST == 2 both of the next round's.  A wave that issues its loads back
-        // to back waits for the memory pipeline (64 KB: 0.5 us per round, measured), so they go between the products.
-        const int rc = NST == 1 ? r : r + 1;
-        const bool copies = rc < nR, spread1 = copies && 2 * rc + 1 < nJ && 2 * rc + 1 < full_tiles;
-        const int j = 2 * r + (kb >> 1);
-        if (copies && !(spread1 && j < nJ)) {
-            if constexpr (NST == 2) copy_y1(rc);
-            copy_y2(rc);
+    const frag* const p = pbuf + rb * 2 * 64 + lane;
+    auto weights = [&](auto g) { return p[((decltype(g)::value >> 1) * RB * 2 + (decltype(g)::value & 1)) * 64]; };
+    auto none = [](auto) {};
+    // weights of a block whose products are in s, by where it lies; blk, er: its share of the row sums
+    auto weigh_element = [&](f32x16& s, int x, float ek, float er, float sc, float of, float& blk) __attribute__((always_inline)) {
+        if constexpr (MODE == RW_FWD) {
+            blk = fmaf(s[x], ek, blk);
+            s[x] = (s[x] * ek) * er;
+        } else {
+            s[x] = (s[x] * sc + of) * ek;
         }
-        auto phase1 = [&](auto spread_tag) __attribute__((always_inline)) {
-            constexpr bool SPREAD = decltype(spread_tag)::value;
-            f32x16 s;
-            const int k0 = GRAN * j + 32 * (kb & 1), rr = r0 + 32 * rb;
-            const T* y1 = y1_at(r, kb >> 1);
-            const float crow = crow_base + sdg[j];
-            constexpr int AHEAD = 4;
-            frag kf[NS];
+    };
+    auto weigh = [&](f32x16& s, int k0, float crow, float& blk, float& er) __attribute__((always_inline)) {
+        blk = 0.f; er = 0.f;
+        if (k0 > rr) {             // above the diagonal
 #pragma unroll
-            for (int n = 0; n < AHEAD; n++) kf[n] = rrd.read(y1, kb & 1, n);
+            for (int x = 0; x < 16; x++) s[x] = 0.f;
+        } else if (k0 < rr) {      // below it: factorised weights
+            er = fast_exp2(crow + sam[k0 / 32]);
+            const float sc = inv_n * er, of = dbv * er;
 #pragma unroll
-            for (int n = 0; n < NS; n++) {
-                if (n + AHEAD < NS) kf[n + AHEAD] = rrd.read(y1, kb & 1, n + AHEAD);
-                if (n == 0) {
+            for (int a4 = 0; a4 < 4; a4++) {
+                const f32x4 ek = *reinterpret_cast<const f32x4*>(sek + k0 + 8 * a4 + 4 * h);
 #pragma unroll
-                    for (int x = 0; x < 16; x++) s[x] = 0.f;
-                }
-                R::mma(s, kf[n], xf[n]);
-                if constexpr (SPREAD) {
-                    if constexpr (NST == 1) {
-                        if (n % 2 == 0) copy_piece(Y2, y2_at(r, 0), y2_at(r, 1), 2 * r, n / 2);
+                for (int c = 0; c < 4; c++) weigh_element(s, 4 * a4 + c, ek[c], er, sc, of, blk);
+            }
+        } else {                   // on it
+#pragma unroll
+            for (int a4 = 0; a4 < 4; a4++) {
+                const f32x4 al = *reinterpret_cast<const f32x4*>(sal + k0 + 8 * a4 + 4 * h);
+#pragma unroll
+                for (int c = 0; c < 4; c++) {
+                    const int x = 4 * a4 + c;
+                    float e = fast_exp2(al[c] + crow);
+                    if (8 * a4 + 4 * h + c > c32) e = 0.f;
+                    if constexpr (MODE == RW_FWD) {
+                        s[x] *= e;     // (its share of the row sums: behind the loop)
                     } else {
-                        if (n < 4) copy_piece(Y1, y1_at(rc, 0), y1_at(rc, 1), 2 * rc, n);
-                        else copy_piece(Y2, y2_at(rc, 0), y2_at(rc, 1), 2 * rc, n - 4);
+                        s[x] = (s[x] * inv_n + dbv) * e;
                     }
                 }
-                __builtin_amdgcn_sched_barrier(0);
             }
-            float blk = 0.f, er = 0.f;
-            if (k0 > rr) {             // above the diagonal
+        }
+    };
+    auto put_weights = [&](const f32x16& s, float blk, float er) __attribute__((always_inline)) {
+        frag* const q = pbuf + (kb * RB + rb) * 2 * 64 + lane;
+        q[0] = R::from_acc(s, 0);
+        q[64] = R::from_acc(s, 1);
+        if constexpr (MODE == RW_FWD) *reinterpret_cast<float2*>(part + ((kb * RB + rb) * 64 + lane) * 2) = make_float2(blk, er);
+    };
+    // S^T of the wave's block of round r, with something between the products
+    auto products = [&](f32x16& s, int r, auto&& hook) __attribute__((always_inline)) {
+        const T* y1 = y1_at(r, kb >> 1);
+        constexpr int AHEAD = 4;
+        frag kf[NS];
+#pragma unroll
+        for (int n = 0; n < AHEAD; n++) kf[n] = rrd.read(y1, kb & 1, n);
+        static_for<NS>([&](auto nc) __attribute__((always_inline)) {
+            constexpr int n = decltype(nc)::value;
+            if constexpr (n + AHEAD < NS) kf[n + AHEAD] = rrd.read(y1, kb & 1, n + AHEAD);
+            if constexpr (n == 0) {
 #pragma unroll
                 for (int x = 0; x < 16; x++) s[x] = 0.f;
-            } else if (k0 < rr) {      // below it: factorised weights
-                er = fast_exp2(crow + sam[k0 / 32]);
-                const float sc = inv_n * er, of = dbv * er;
-#pragma unroll
-                for (int a4 = 0; a4 < 4; a4++) {
-                    const f32x4 ek = *reinterpret_cast<const f32x4*>(sek + k0 + 8 * a4 + 4 * h);
-#pragma unroll
-                    for (int c = 0; c < 4; c++) {
-                        const int x = 4 * a4 + c;
-                        if constexpr (MODE == RW_FWD) {
-                            blk = fmaf(s[x], ek[c], blk);
-                            s[x] = (s[x] * ek[c]) * er;
-                        } else {
-                            s[x] = (s[x] * sc + of) * ek[c];
-                        }
-                    }
-                }
-            } else {                   // on it
-#pragma unroll
-                for (int a4 = 0; a4 < 4; a4++) {
-                    const f32x4 al = *reinterpret_cast<const f32x4*>(sal + k0 + 8 * a4 + 4 * h);
-#pragma unroll
-                    for (int c = 0; c < 4; c++) {
-                        const int x = 4 * a4 + c;
-                        float e = fast_exp2(al[c] + crow);
-                        if (8 * a4 + 4 * h + c > c32) e = 0.f;
-                        if constexpr (MODE == RW_FWD) {
-                            s[x] *= e;     // (its share of the row sums: behind the loop)
-                        } else {
-                            s[x] = (s[x] * inv_n + dbv) * e;
-                        }
-                    }
-                }
             }
-            frag* const p = pbuf + (kb * 2 + rb) * 2 * 64 + lane;
-            p[0] = R::from_acc(s, 0);
-            p[64] = R::from_acc(s, 1);
-            if constexpr (MODE == RW_FWD) *reinterpret_cast<float2*>(part + ((kb * 2 + rb) * 64 + lane) * 2) = make_float2(blk, er);
-        };
-        if (j < nJ) {
-            if (spread1) phase1(std::true_type{});
-            else phase1(std::false_type{});
-        }
-        if constexpr (NST == 1) dma_wait();
-        __syncthreads();
+            R::mma(s, kf[n], xf[n]);
+            hook(nc);
+            __builtin_amdgcn_sched_barrier(0);
+        });
+    };
+    auto add_row_sums = [&](bool two) __attribute__((always_inline)) {
         if constexpr (MODE == RW_FWD) {
             if (kb < 2) {   // (a block on the diagonal or above it has left zeros)
 #pragma unroll
                 for (int t = 0; t < 2; t++)
                     if (t == 0 || two) {
-                        const float2 be = *reinterpret_cast<const float2*>(part + (((2 * t + kb) * 2 + rb) * 64 + lane) * 2);
+                        const float2 be = *reinterpret_cast<const float2*>(part + (((2 * t + kb) * RB + rb) * 64 + lane) * 2);
                         bsum = fmaf(be.x, be.y, bsum);
                     }
             }
         }
-        const frag* const p = pbuf + rb * 2 * 64 + lane;
-        auto weights = [&](auto g) { return p[((decltype(g)::value >> 1) * 2 * 2 + (decltype(g)::value & 1)) * 64]; };
-        auto y2 = [&](int t) { return y2_at(r, t); };
-        auto none = [](auto) {};
-        const bool spread2 = NST == 1 && r + 1 < nR && 2 * r + 3 < nJ && 2 * r + 3 < full_tiles;   // the next round's Y1 under phase 2
-        if constexpr (NST == 1) {
+    };
+    if constexpr (NST == 1) {
+        for (int r = 0; r < nR; r++) {
+            const bool two = 2 * r + 1 < nJ;
+            dma_wait();
+            __syncthreads();   // this round's Y1 has landed; phase 2 of the previous round is over
+            // This round's Y2 is copied under phase 1.  A wave that issues its loads back to back waits for the memory pipeline (64 KB: 0.5 us
+            // per round, measured), so they go between the products.
+            const bool spread1 = two && 2 * r + 1 < full_tiles;
+            const int j = 2 * r + (kb >> 1);
+            if (!(spread1 && j < nJ)) copy_y2(r);
+            auto phase1 = [&](auto spread_tag) __attribute__((always_inline)) {
+                constexpr bool SPREAD = decltype(spread_tag)::value;
+                f32x16 s;
+                products(s, r, [&](auto n) {
+                    if constexpr (SPREAD) pieces(decltype(n)::value, NS, [&](int i) { copy_piece(Y2, y2_at(r, 0), y2_at(r, 1), 2 * r, i); });
+                });
+                float blk, er;
+                weigh(s, GRAN * j + 32 * (kb & 1), crow_base + sdg[j], blk, er);
+                put_weights(s, blk, er);
+            };
+            if (j < nJ) {
+                if (spread1) phase1(std::true_type{});
+                else phase1(std::false_type{});
+            }
+            dma_wait();
+            __syncthreads();
+            add_row_sums(two);
+            auto y2 = [&](int t) { return y2_at(r, t); };
+            const bool spread2 = r + 1 < nR && 2 * r + 3 < nJ && 2 * r + 3 < full_tiles;   // the next round's Y1 under phase 2
             if (r + 1 < nR && !spread2) copy_y1(r + 1);
+            if (spread2) chain(Eight{}, y2, weights, [&](auto g) { pieces(decltype(g)::value, 8, [&](int i) { copy_piece(Y1, y1_at(r + 1, 0), y1_at(r + 1, 1), 2 * r + 2, i); }); });
+            else if (two) chain(Eight{}, y2, weights, none);
+            else chain(Four{}, y2, weights, none);
         }
-        if (spread2) chain(Eight{}, y2, weights, [&](auto g) { copy_piece(Y1, y1_at(r + 1, 0), y1_at(r + 1, 1), 2 * r + 2, decltype(g)::value); });
-        else if (two) chain(Eight{}, y2, weights, none);
-        else chain(Four{}, y2, weights, none);
+    } else {
+        // D = 128 holds two stages of either operand: phase 1 of a round runs with phase 2 of the one before, its element-wise part between those
+        // products, and only the 16-bit weights wait (in 8 registers) until every wave has read the ones before them.  A round is then bound by
+        // its LDS traffic (192 KB and 64 KB of copies on 64 rows, 96 and 64 on 32) instead of by the chain products, weights, hand-over, products.
+        // Forward, us, before / now: 1 x 640 x 128 on 32 rows 10.6 / 9.9, 8 x 1000 16.1 / 14.9, on 64 rows 15 x 1001 19.1 / 17.9, 4 x 4096 in chunks 13.2 / 12.5.
+        f32x16 s;
+        float blk = 0.f, er = 0.f;
+        auto alone = [&](int r) __attribute__((always_inline)) {   // phase 1 by itself
+            const int j = 2 * r + (kb >> 1);
+            if (j < nJ) {
+                products(s, r, none);
+                weigh(s, GRAN * j + 32 * (kb & 1), crow_base + sdg[j], blk, er);
+            }
+        };
+        alone(0);
+        if (kb >> 1 < nJ) put_weights(s, blk, er);
+        dma_wait();
+        __syncthreads();   // the first weights, and Y1 of the second round
+        for (int r = 0; r < nR; r++) {
+            const bool two = 2 * r + 1 < nJ, next = r + 1 < nR;
+            const int j = 2 * r + 2 + (kb >> 1), k0 = GRAN * j + 32 * (kb & 1);
+            const bool mine = next && j < nJ;
+            auto y2 = [&](int t) { return y2_at(r, t); };
+            add_row_sums(two);
+            // the copies of this round: Y1 two rounds ahead, Y2 one ahead, into the stages that are free since the last barrier
+            auto with_next = [&](auto spread_tag) __attribute__((always_inline)) {
+                constexpr bool SPREAD = decltype(spread_tag)::value;
+                const float crow = crow_base + sdg[j], cmax = sam[k0 / 32];
+                f32x4 ek[4];
+#pragma unroll
+                for (int a4 = 0; a4 < 4; a4++) ek[a4] = *reinterpret_cast<const f32x4*>(sek + k0 + 8 * a4 + 4 * h);
+                products(s, r + 1, [&](auto n) {
+                    if constexpr (SPREAD) pieces(decltype(n)::value, NS, [&](int i) { copy_piece(Y1, y1_at(r, 0), y1_at(r, 1), 2 * r + 4, i); });
+                });
+                er = fast_exp2(crow + cmax);
+                blk = 0.f;
+                const float sc = inv_n * er, of = dbv * er;
+                chain(Eight{}, y2, weights, [&](auto gc) {
+                    constexpr int g = decltype(gc)::value;
+                    weigh_element(s, 2 * g, ek[g / 2][2 * (g % 2)], er, sc, of, blk);
+                    weigh_element(s, 2 * g + 1, ek[g / 2][2 * (g % 2) + 1], er, sc, of, blk);
+                    if constexpr (SPREAD) pieces(g, 8, [&](int i) { copy_piece(Y2, y2_at(r + 1, 0), y2_at(r + 1, 1), 2 * r + 2, i); });
+                });
+            };
+            const bool below = mine && k0 < rr, spread = below && r + 2 < nR && 2 * r + 5 < nJ && 2 * r + 5 < full_tiles;
+            if (spread) {
+                with_next(std::true_type{});
+            } else {
+                if (r + 2 < nR) copy_y1(r + 2);
+                if (next) copy_y2(r + 1);
+                if (below) {
+                    with_next(std::false_type{});
+                } else {
+                    if (next) alone(r + 1);
+                    if (two) chain(Eight{}, y2, weights, none);
+                    else chain(Four{}, y2, weights, none);
+                }
+            }
+            if (!next) break;
+            __syncthreads();   // every wave has read this round's weights
+            if (mine) put_weights(s, blk, er);
+            dma_wait();
+            __syncthreads();   // the next ones are there, and the tiles requested above
+        }
     }
     if constexpr (MODE == RW_FWD) {
         // The elements of the block on the diagonal go one by one onto the sum over the blocks before it.  They are formed once more here, where
         // that sum is, from tiles that are still in LDS: kept from phase 1 on, products and weights cost 64 moves in every round, and the
         // kernel 1 us of 11 (640 x 128).
-        if (kb == rb) {
+        const int own = (r0 / 32 + rb) & 1;   // the block's place in its tile
+        if (kb == own) {
             const T* const y1 = y1_at(nR - 1, (nJ - 1) & 1);
             f32x16 s;
 #pragma unroll
             for (int x = 0; x < 16; x++) s[x] = 0.f;
 #pragma unroll
-            for (int n = 0; n < NS; n++) R::mma(s, rrd.read(y1, rb, n), xf[n]);
-            const float crow = crow_base + sdg[qt];
+            for (int n = 0; n < NS; n++) R::mma(s, rrd.read(y1, own, n), xf[n]);
+            const float crow = crow_base + sdg[gt];
 #pragma unroll
             for (int a4 = 0; a4 < 4; a4++) {
                 const f32x4 al = *reinterpret_cast<const f32x4*>(sal + r0 + 32 * rb + 8 * a4 + 4 * h);
@@ -401,14 +483,14 @@ __global__ __launch_bounds__(512) void roww_kernel(RowArgs a) {
     }
     // ---- epilogue
     uint4 og[D / 64];   // output gate: this thread's pieces, requested ahead of the barriers
-    constexpr int CPR = D * (int)sizeof(T) / 16, RB = D * (int)sizeof(T) + 16, NP = 64 * CPR / 512;
+    constexpr int CPR = D * (int)sizeof(T) / 16, ROWB = D * (int)sizeof(T) + 16, NP = ROWS * CPR / NT;
     static_assert(NP == D / 64, "pieces per thread");
     if constexpr (MODE == RW_FWD) {
         if (a.O) {
             const char* go = reinterpret_cast<const char*>(a.O) + (offB + (size_t)r0 * rsB) * sizeof(T);
 #pragma unroll
             for (int i = 0; i < NP; i++) {
-                const int c = tid + 512 * i, rr = c / CPR, cc = c % CPR;
+                const int c = tid + NT * i, rr = c / CPR, cc = c % CPR;
                 og[i] = r0 + rr < S ? *reinterpret_cast<const uint4*>(go + (size_t)rr * rsB * sizeof(T) + 16 * cc) : uint4{0, 0, 0, 0};
             }
         }
@@ -448,7 +530,7 @@ __global__ __launch_bounds__(512) void roww_kernel(RowArgs a) {
                 for (int half = 0; half < 2; half++) {
                     float rp = 0.f;
 #pragma unroll
-                    for (int d = 0; d < D / 64; d++) rp += part[((half * (D / 64) + d) * 2 + rb) * 64 + lane];
+                    for (int d = 0; d < D / 64; d++) rp += part[((half * (D / 64) + d) * RB + rb) * 64 + lane];
                     rp = sum_halves(rp);
                     v = half ? v + rp : rp;
                 }
@@ -463,7 +545,7 @@ __global__ __launch_bounds__(512) void roww_kernel(RowArgs a) {
             f32x4 v;
 #pragma unroll
             for (int e = 0; e < 4; e++) v[e] = acc[c][4 * a4 + e] * onorm;
-            *reinterpret_cast<typename R::vec4*>(smem + (32 * rb + c32) * RB + (32 * (NC * kb + c) + 8 * a4 + 4 * h) * (int)sizeof(T)) = R::cvt4(v);
+            *reinterpret_cast<typename R::vec4*>(smem + (32 * rb + c32) * ROWB + (32 * (NC * kb + c) + 8 * a4 + 4 * h) * (int)sizeof(T)) = R::cvt4(v);
         }
     __syncthreads();
     {
@@ -471,8 +553,8 @@ __global__ __launch_bounds__(512) void roww_kernel(RowArgs a) {
         char* const gg = MODE == RW_FWD ? reinterpret_cast<char*>(a.out_gated) + (offB + (size_t)r0 * rsB) * sizeof(T) : nullptr;
 #pragma unroll
         for (int i = 0; i < NP; i++) {
-            const int c = tid + 512 * i, rr = c / CPR, cc = c % CPR;
-            const uint4 v = *reinterpret_cast<const uint4*>(smem + rr * RB + 16 * cc);
+            const int c = tid + NT * i, rr = c / CPR, cc = c % CPR;
+            const uint4 v = *reinterpret_cast<const uint4*>(smem + rr * ROWB + 16 * cc);
             if (r0 + rr < S) {
                 *reinterpret_cast<uint4*>(gout + (size_t)rr * rsO * sizeof(T) + 16 * cc) = v;
                 if constexpr (MODE == RW_FWD) {
@@ -492,24 +574,29 @@ __global__ __launch_bounds__(512) void roww_kernel(RowArgs a) {
 #endif
 }
 
-template <typename T, int D, int MODE>
+template <typename T, int D, int MODE, int RB>
 static int launch_roww_t(const RowArgs& a, hipStream_t st) {
-    using Cfg = RowwCfg<T, D>;
+    using Cfg = RowwCfg<T, D, RB>;
     const int most = a.chunk_len > 0 && a.chunk_len < a.NG * GRAN ? a.chunk_len : a.NG * GRAN;   // keys a row may meet
     if (most > RW_MOST_KEYS) return MLSTM_ESHAPE;
-    if (hipError_t e = lds_limit_once<roww_kernel<T, D, MODE>>((int)Cfg::lds_bytes(RW_MOST_KEYS)); e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL((roww_kernel<T, D, MODE>), dim3(a.BH * a.NG), dim3(512), Cfg::lds_bytes(most), st, a);
+    if (hipError_t e = lds_limit_once<roww_kernel<T, D, MODE, RB>>((int)Cfg::lds_bytes(RW_MOST_KEYS)); e != hipSuccess) return (int)e;
+    hipLaunchKernelGGL((roww_kernel<T, D, MODE, RB>), dim3(a.BH * a.NG * (2 / RB)), dim3(256 * RB), Cfg::lds_bytes(most), st, a);
     return (int)hipGetLastError();
 }
 
-template <typename T>
+template <typename T, int RB>
 static int launch_roww_m(int mode, int D, const RowArgs& a, hipStream_t st) {
-    if (mode == RW_FWD) return D == 128 ? launch_roww_t<T, 128, RW_FWD>(a, st) : launch_roww_t<T, 256, RW_FWD>(a, st);
-    return D == 128 ? launch_roww_t<T, 128, RW_DQ>(a, st) : launch_roww_t<T, 256, RW_DQ>(a, st);
+    if (mode == RW_FWD) return D == 128 ? launch_roww_t<T, 128, RW_FWD, RB>(a, st) : launch_roww_t<T, 256, RW_FWD, RB>(a, st);
+    return D == 128 ? launch_roww_t<T, 128, RW_DQ, RB>(a, st) : launch_roww_t<T, 256, RW_DQ, RB>(a, st);
 }
 
 int launch_roww_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t st) {
-    return dtype == MLSTM_F16 ? launch_roww_m<_Float16>(mode, D, a, st) : launch_roww_m<__bf16>(mode, D, a, st);
+    // 32 rows and four waves per workgroup as long as there is a CU for each: a round's LDS traffic, which bounds it, is half of that of 64 rows but for the
+    // tiles' copies.  64 / 32 rows, forward and dQ pass, us, D = 128   1 x 64: 5.1, 6.1 / 5.2, 5.7   1 x 256: 7.1, 8.1 / 6.8, 7.6   1 x 640: 10.9, 12 / 9.9, 10.6
+    // 2 x 2048: 11.1, 12.8 / 10.5, 11.8   D = 256   1 x 64: 6.0, 7.8 / 5.9, 7.1   1 x 640: 13.9, 15.6 / 12.6, 13.7   8 x 1000: 22.2, 23.3 / 20.4, 21.4
+    // (two workgroups of 32 rows one after the other on a CU: 15 x 1001 x 128 18.0, 19.2 / 21.7, 22.2; 8 x 1777 x 256 18.4, 21.4 / 23.9, 27.0)
+    if ((long long)a.BH * a.NG <= 128) return dtype == MLSTM_F16 ? launch_roww_m<_Float16, 1>(mode, D, a, st) : launch_roww_m<__bf16, 1>(mode, D, a, st);
+    return dtype == MLSTM_F16 ? launch_roww_m<_Float16, 2>(mode, D, a, st) : launch_roww_m<__bf16, 2>(mode, D, a, st);
 }
 
 }  // namespace mlstm
