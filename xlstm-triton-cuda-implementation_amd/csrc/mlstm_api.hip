@@ -437,11 +437,6 @@ int forward_impl(const void* q, const void* k, const void* v, const void* f, con
     const size_t ncs = w.ncs;
     if (!m) m = w.mw;
     if (!b) b = w.bw;
-    {
-        Timed t(MLSTM_K_GATES, st);
-        hipError_t e = launch_gates(gate_dtype, f, i, alpha2, beta2, G2, m, ek2, amax2, w.bw, (int)z.BH, (int)z.S, st, z.lg, z.gate_form, stamp);
-        if (e != hipSuccess) return (int)e;
-    }
     RowArgs a{};
     a.la = z.la; a.lb = z.lb; a.lh = z.lb;
     a.X = q; a.Y1 = k; a.Y2 = v; a.out = h; a.alpha2 = alpha2; a.beta2 = beta2; a.G2 = G2; a.M = m; a.Bsum = b;
@@ -449,6 +444,13 @@ int forward_impl(const void* q, const void* k, const void* v, const void* f, con
     a.BH = (int)z.BH; a.S = (int)z.S; a.NG = (int)z.NG;
     a.precise = z.precise ? 1 : 0; a.out_lo = h_lo;
     if (int rc = arm_row_args(a)) return rc;
+    if (ncs == 0 && !stamp && z.gate_form != MLSTM_GATE_CUMSUM && roww_serves(dtype, D, a)) {   // one launch for both
+        a.gate_F = f; a.gate_I = i; a.gate_dtype = gate_dtype; a.gate_form = z.gate_form; a.lg = z.lg;
+    } else {
+        Timed t(MLSTM_K_GATES, st);
+        hipError_t e = launch_gates(gate_dtype, f, i, alpha2, beta2, G2, m, ek2, amax2, w.bw, (int)z.BH, (int)z.S, st, z.lg, z.gate_form, stamp);
+        if (e != hipSuccess) return (int)e;
+    }
     if (ncs > 0) {   // long sequence: the states at the chunk ends first, then every row tile stays inside its chunk
         float* Nst = Nst_ext ? Nst_ext : w.Nst;
         if (int e = chunk_states_impl(k, v, w, true, CstT, Nst, z, D, dtype, st)) return e;

@@ -711,7 +711,8 @@ __device__ __forceinline__ float rounded_product(float a, float b) {
     return p;
 }
 // The same where nothing but the compiler's own contraction is to be kept out.
-__device__ __forceinline__ float product_apart(float a, float b) {
+template <typename F>
+__device__ __forceinline__ F product_apart(F a, F b) {
 #pragma clang fp contract(off)
     return a * b;
 }

@@ -12,104 +12,12 @@
 // whence  a_j - A_i = alpha_j - beta_i + (G_g(i) - G_g(j))  with one fp64 subtraction per tile pair.
 // alpha, beta and G are stored pre-multiplied by log2(e) (the kernels use exp2); m in natural units.
 // alpha and beta have a row stride of ceil(S/64)*64 per head (padded to whole granules).
-#include "mlstm_device.h"
-#include "mlstm_kernels.h"
+#include "mlstm_gates.h"
 
 namespace mlstm {
 
 constexpr int GATES_MAX_GRANULES = 2048;  // S <= 131072
 constexpr int GATES_WAVES = 16;           // waves per workgroup, a granule each at a time
-
-// the DPP scans of mlstm_device.h on doubles, two moves per step
-template <int CTRL>
-__device__ __forceinline__ double dpp_d(double old, double src) {
-    const long long o = __builtin_bit_cast(long long, old), x = __builtin_bit_cast(long long, src);
-    const int lo = __builtin_amdgcn_update_dpp((int)o, (int)x, CTRL, 0xf, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp((int)(o >> 32), (int)(x >> 32), CTRL, 0xf, 0xf, false);
-    return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
-}
-__device__ __forceinline__ double readlane_d(double v, int lane) {
-    const long long x = __builtin_bit_cast(long long, v);
-    const int lo = __builtin_amdgcn_readlane((int)x, lane), hi = __builtin_amdgcn_readlane((int)(x >> 32), lane);
-    return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
-}
-struct AddD { static __device__ __forceinline__ double id() { return 0.0; } static __device__ __forceinline__ double f(double a, double b) { return a + b; } };
-struct MaxD { static __device__ __forceinline__ double id() { return -INFINITY; } static __device__ __forceinline__ double f(double a, double b) { return fmax(a, b); } };
-template <typename Op>
-__device__ __forceinline__ double wave_scan_inclusive_d(double v, int lane) {
-    v = Op::f(v, dpp_d<0x111>(Op::id(), v));
-    v = Op::f(v, dpp_d<0x112>(Op::id(), v));
-    v = Op::f(v, dpp_d<0x114>(Op::id(), v));
-    v = Op::f(v, dpp_d<0x118>(Op::id(), v));
-    const double r0 = readlane_d(v, 15), r1 = Op::f(r0, readlane_d(v, 31)), r2 = Op::f(r1, readlane_d(v, 47));
-    double c = Op::id();
-    if (lane >= 16) c = r0;
-    if (lane >= 32) c = r1;
-    if (lane >= 48) c = r2;
-    return Op::f(c, v);
-}
-
-// fp64 prefix over up to 64 granules, one per lane: exclusive sum G of the totals behind `run`, and the running maximum R of (P - G) over
-// EARLIER granules, `rmax` those before the 64.  The totals of 64 logarithms are floats: their sums are exact in fp64, in any order, unless they
-// lie 2^18 apart.  (By log-step lane shuffles, an LDS round trip each, the two scans took 0.9 us; these take 0.2.)
-__device__ __forceinline__ void granule_scan(double tot, double p, double run, int lane, double& incl, double& excl, double& mx) {
-    incl = wave_scan_inclusive_d<AddD>(tot, lane);
-    excl = run + (incl - tot);                               // G of this granule
-    mx = wave_scan_inclusive_d<MaxD>(p - excl, lane);        // with this granule's candidate for later ones
-}
-__device__ __forceinline__ double before_lane(double mx, int lane) {   // maximum over the earlier granules of these 64
-    double x = dpp_d<0x111>(-INFINITY, mx);
-    const double r0 = readlane_d(mx, 15), r1 = readlane_d(mx, 31), r2 = readlane_d(mx, 47);
-    if (lane == 16) x = r0;
-    if (lane == 32) x = r1;
-    if (lane == 48) x = r2;
-    return x;
-}
-
-// what a position's outputs need beside the granules before its own, from the in-granule cumulative sum c and alpha (natural units): the
-// prefix maximum of alpha; written here: alpha2 (rows padded to whole granules: alpha = -inf there, so padded keys weigh nothing) and the
-// factorised weights for blocks of 32 keys that lie entirely below the diagonal: with c0 the block maximum of
-// alpha, exp2(alpha_j - beta_i + dG) = exp2(alpha_j - c0) * exp2(c0 - beta_i + dG); both factors are <= 1 there,
-// so the product under- or overflows only where the weight itself does.
-__device__ __forceinline__ float gates_local(float al, bool ok, size_t pos, size_t gidx, int lane, float* alpha2, float* ek2, float* amax2) {
-    const float loc = wave_scan_inclusive<OpMax>(al);
-    const float al2 = product_apart(al, LOG2E);   // (rounded, also where the block maximum is taken off it)
-    alpha2[pos] = ok ? al2 : -INFINITY;
-    float lo, hi;
-    wave_half_max(al2, lo, hi);
-    const float c0 = lane < 32 ? lo : hi;
-    ek2[pos] = (ok && c0 > -INFINITY) ? fast_exp2(al2 - c0) : 0.0f;
-    if ((lane & 31) == 0) amax2[gidx * 2 + (lane >> 5)] = c0;
-    return loc;
-}
-// and with G and R of the granule
-__device__ __forceinline__ void gates_global(float c, float loc, bool ok, double Gg, double Rg, size_t pos, size_t mpos, size_t gidx, int lane,
-                                             float* beta2, double* G2, float* M) {
-    const float carry = (float)(Rg + Gg);  // max over earlier granules of (alpha_j - G_g(j)) + G_g ; -inf for g == 0
-    const float be = fmaxf(loc, carry);
-    beta2[pos] = ok ? be * LOG2E : 0.0f;
-    if (ok) M[mpos] = c + be;
-    if (lane == 0) G2[gidx] = Gg * LOG2E_D;
-}
-
-// log-sigmoid of the forget gate at position t from what the caller's F holds (see launch_gates): the pre-activation,
-// the log-sigmoid itself, or its cumulative sum over the head (then the difference of two neighbours)
-struct GateIn { float x, before, i; };
-template <typename TG>
-__device__ __forceinline__ GateIn gate_in(const TG* f, const TG* ig, size_t ss, int t, int S, int form) {   // (positions past the end: the last one's)
-    t = t < S ? t : S - 1;
-    GateIn v;
-    v.x = (float)f[(size_t)t * ss];
-    v.i = (float)ig[(size_t)t * ss];
-    v.before = form == MLSTM_GATE_CUMSUM && t > 0 ? (float)f[(size_t)(t - 1) * ss] : 0.f;
-    return v;
-}
-__device__ __forceinline__ float forget_log(const GateIn& v, int t, int form) {
-    if (form == MLSTM_GATE_RAW) return log_sigmoid(v.x);
-    if (form == MLSTM_GATE_LOGSIGMOID) return v.x;
-    return t > 0 ? v.x - v.before : v.x;
-}
-__device__ __forceinline__ float last_lane(float v) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63)); }
 
 // Sequences of up to 16 * GPW granules (GPW = 1, 2, 4: S <= 4096) in one launch: a workgroup writes `per` granules (a power of two of up to 16) and
 // forms the totals of all granules up to those by itself, one per wave and turn.  What bounds it is instruction issue on one CU, some 90
@@ -131,33 +39,41 @@ __global__ __launch_bounds__(1024) void gates_kernel_reg(const TG* __restrict__ 
     const TG* f = F + lg.head(bh);
     const TG* ig = I + lg.head(bh);
     GateIn in[GPW];
-    float c = 0.f, al = -INFINITY;
+    const int gown = wave + GATES_WAVES * seg, t = gown * GRAN + lane;
+    const bool mine = gown >= first && gown < first + per && gown < NG, ok = t < S;
+    const size_t pos = (size_t)bh * NG * GRAN + t, gidx = (size_t)bh * NG + gown;
+    float c = 0.f, loc = 0.f;
 #pragma unroll
     for (int k = 0; k < GPW; k++) in[k] = gate_in(f, ig, gs, (wave + GATES_WAVES * k) * GRAN + lane, S, form);
 #pragma unroll
     for (int k = 0; k < GPW; k++) {
-        const int g = wave + GATES_WAVES * k, t = g * GRAN + lane;
+        const int g = wave + GATES_WAVES * k, tk = g * GRAN + lane;
         if (g < first + per && g < NG) {
-            c = wave_scan_inclusive<OpAdd>(t < S ? forget_log(in[k], t, form) : 0.0f);
-            al = t < S ? in[k].i - c : -INFINITY;
-            const float p = wave_reduce<OpMax>(al);
+            c = wave_scan_inclusive<OpAdd>(tk < S ? forget_log(in[k], tk, form) : 0.0f);
+            const float al = tk < S ? in[k].i - c : -INFINITY;
             const float tot = last_lane(c);
+            float p;
+            if (mine && k == seg) {
+                const GateLocal v = gates_local(al, ok, lane);
+                store_local(v, pos, gidx, lane, alpha2, ek2, amax2);
+                loc = v.loc;
+                p = v.p;
+            } else {
+                p = wave_reduce<OpMax>(al);
+            }
             if (lane == 0) { sT[g] = (double)tot; sP[g] = (double)p; }
         }
     }
-    // (c and al are now those of the last granule passed, the wave's own)
-    const int g = wave + GATES_WAVES * seg, t = g * GRAN + lane;
-    const bool mine = g >= first && g < first + per && g < NG, ok = t < S;
-    const size_t pos = (size_t)bh * NG * GRAN + t, gidx = (size_t)bh * NG + g;
-    const float loc = mine ? gates_local(al, ok, pos, gidx, lane, alpha2, ek2, amax2) : 0.f;
+    // (c is now that of the last granule passed, the wave's own)
     __syncthreads();
     if (!mine) return;
     {   // the prefix, by every wave for itself (a wave alone, with the others waiting for it, takes as long, and a barrier)
-        const int ng = g + 1;
+        const int ng = gown + 1;
         double incl, excl, mx;
         granule_scan(lane < ng ? sT[lane] : 0.0, lane < ng ? sP[lane] : -INFINITY, 0.0, lane, incl, excl, mx);
         const double before = before_lane(mx, lane);
-        gates_global(c, loc, ok, readlane_d(excl, g), readlane_d(before, g), pos, (size_t)bh * S + t, gidx, lane, beta2, G2, M);
+        const double Gg = readlane_d(excl, gown);
+        store_global(gates_global(c, loc, ok, Gg, readlane_d(before, gown)), ok, Gg, pos, (size_t)bh * S + t, gidx, lane, beta2, G2, M);
     }
 }
 
@@ -179,10 +95,12 @@ __global__ __launch_bounds__(1024) void gates_local_kernel(const TG* __restrict_
     const bool ok = t < S;
     const GateIn in = gate_in(F + lg.head(bh), I + lg.head(bh), gs, t, S, form);
     const float c = wave_scan_inclusive<OpAdd>(ok ? forget_log(in, t, form) : 0.0f), al = ok ? in.i - c : -INFINITY;
-    const float p = wave_reduce<OpMax>(al), tot = last_lane(c);
+    const float tot = last_lane(c);
     const size_t pos = (size_t)bh * NG * GRAN + t, gidx = (size_t)bh * NG + g;
-    if (lane == 0) totals[gidx] = make_float2(tot, p);
-    beta2[pos] = gates_local(al, ok, pos, gidx, lane, alpha2, ek2, amax2);
+    const GateLocal v = gates_local(al, ok, lane);
+    if (lane == 0) totals[gidx] = make_float2(tot, v.p);
+    store_local(v, pos, gidx, lane, alpha2, ek2, amax2);
+    beta2[pos] = v.loc;
     if (ok) M[(size_t)bh * S + t] = c;
 }
 __global__ __launch_bounds__(1024) void gates_carry_kernel(const float2* __restrict__ totals, float* __restrict__ beta2, double* __restrict__ G2,
@@ -229,7 +147,8 @@ __global__ __launch_bounds__(1024) void gates_carry_kernel(const float2* __restr
     if (!mine) return;
     double rmax = -INFINITY;
     for (int n = 0; n < mygroup; n++) rmax = fmax(rmax, sMax[n]);
-    gates_global(c, loc, ok, sG[wave], fmax(rmax, sR[wave]), pos, mpos, (size_t)bh * NG + g, lane, beta2, G2, M);
+    const double Gg = sG[wave];
+    store_global(gates_global(c, loc, ok, Gg, fmax(rmax, sR[wave])), ok, Gg, pos, mpos, (size_t)bh * NG + g, lane, beta2, G2, M);
 }
 
 template <typename TG>

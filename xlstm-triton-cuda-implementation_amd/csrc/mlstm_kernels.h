@@ -123,6 +123,12 @@ struct RowArgs {
     // layouts of the caller's tensors: la for q, k, v (forward: X, Y1, Y2; dQ pass: Y1, Y2, Qrow and out),
     // lb for h, dh, o (forward: out, O, out_gated; dQ pass: X), lh for Hin (the caller's h, or a dense recomputed one)
     Lay la, lb, lh;
+    // forward of a sequence that is not cut, where roww_kernel serves it (roww_serves): with gate_F set it forms the gates of its head by itself, from
+    // F and I in layout lg, and leaves in alpha2, beta2, G2, ek2, amax2 and M what launch_gates would have
+    const void* gate_F = nullptr;
+    const void* gate_I = nullptr;
+    int gate_dtype = 0, gate_form = 0;
+    Lay lg{};
 };
 // mode 0 = forward (H, b), mode 1 = dQ
 int launch_row_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t st);
@@ -134,23 +140,29 @@ int launch_row8_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t
 int launch_roww_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t st);
 // split mode on 64 rows per workgroup, the bits of the four-wave kernel, for the same launches; not with an output gate
 int launch_rowx_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t st);
+constexpr int RW_MOST_KEYS = 1024;   // keys a row of roww_kernel may meet: their scalars stay in LDS for the whole kernel
+inline bool roww_serves(int dtype, int D, const RowArgs& a) {
+    // (a wait bound of the caller's asks for the kernel that has the wait: mlstm_set_spin_limit)
+    if (dtype == MLSTM_F32 || (D != 128 && D != 256) || a.precise || g_force_generic || a.spin_limit != DEFAULT_SPIN_LIMIT) return false;
+    if ((a.chunk_len > 0 && a.chunk_len < a.NG * GATE_GRANULE ? a.chunk_len : a.NG * GATE_GRANULE) > RW_MOST_KEYS) return false;
+    // While its workgroups (64 rows) number no more than the chip's CUs, roww_kernel: row8_kernel / roww_kernel, forward, us --
+    // D = 128   10: 13.3 / 9.9   128 (uncut, 1000 positions): 20 / 14.9   256 (chunks of 512): 15.6 / 12.9
+    // D = 256   10: 17.2 / 12.6   224 (chunks of 512): 23.1 / 18.4   256: 15.4 / 13.0
+    // and beyond them, where sequences are not cut, as long as the workgroups left over, which are the lightest, end before the longest walk,
+    // forward and dQ pass --
+    // D = 128   320: 128 positions 8.2, 10.6 / 11.2, 13.0   256: 10.6, 12.6 / 11.8, 13.4   512: 13.6, 16.0 / 13.2, 15.7   1000: 21.1, 22.8 / 16.8, 18.7
+    //           384: 512 positions 14.1, 16.1 / 14.8, 16.7   1000: 20.9, 22.3 / 18.6, 20.7   448: 1000 positions 21.0, 22.8 / 21.4, 23.4
+    // D = 256   320: 256 positions 14.4, 19.2 / 14.5, 19.1   512: 18.9, 23.7 / 17.5, 21.4   1000: 28.4, 32.5 / 24.7, 26.5   384: 1000 28.5, 32.7 / 25.5, 28.8
+    //           (in chunks of 512, 320: D = 128 16.4, 18.5 / 19.8, 23.6   D = 256 25.8, 30.4 / 29.2, 36.9)
+    // (bf16; fp16, in chunks of 512, forward and dQ pass, 256: D = 128 17.5, 18.8 / 15.0, 16.7, D = 256 25.6, 29.2 / 21.1, 23.4)
+    const long long roww_most = a.chunk_len > 0 ? 256 : 256 + 8 * a.NG;
+    return (long long)a.BH * a.NG <= roww_most;
+}
 // (the four-wave kernel serves every other case: fp32, D = 64, split mode -- in chunks too --, large launches at D = 128 and the test switch)
 inline int launch_row_best(int mode, int dtype, int D, const RowArgs& a, hipStream_t st) {
     if (dtype != MLSTM_F32 && (D == 128 || D == 256) && !g_force_generic) {
-        // While its workgroups (64 rows) number no more than the chip's CUs, roww_kernel: row8_kernel / roww_kernel, forward, us --
-        // D = 128   10: 13.3 / 9.9   128 (uncut, 1000 positions): 20 / 14.9   256 (chunks of 512): 15.6 / 12.9
-        // D = 256   10: 17.2 / 12.6   224 (chunks of 512): 23.1 / 18.4   256: 15.4 / 13.0
-        // and beyond them, where sequences are not cut, as long as the workgroups left over, which are the lightest, end before the longest walk,
-        // forward and dQ pass --
-        // D = 128   320: 128 positions 8.2, 10.6 / 11.2, 13.0   256: 10.6, 12.6 / 11.8, 13.4   512: 13.6, 16.0 / 13.2, 15.7   1000: 21.1, 22.8 / 16.8, 18.7
-        //           384: 512 positions 14.1, 16.1 / 14.8, 16.7   1000: 20.9, 22.3 / 18.6, 20.7   448: 1000 positions 21.0, 22.8 / 21.4, 23.4
-        // D = 256   320: 256 positions 14.4, 19.2 / 14.5, 19.1   512: 18.9, 23.7 / 17.5, 21.4   1000: 28.4, 32.5 / 24.7, 26.5   384: 1000 28.5, 32.7 / 25.5, 28.8
-        //           (in chunks of 512, 320: D = 128 16.4, 18.5 / 19.8, 23.6   D = 256 25.8, 30.4 / 29.2, 36.9)
-        // (bf16; fp16, in chunks of 512, forward and dQ pass, 256: D = 128 17.5, 18.8 / 15.0, 16.7, D = 256 25.6, 29.2 / 21.1, 23.4)
-        const long long roww_most = a.chunk_len > 0 ? 256 : 256 + 8 * a.NG;
         int rc = MLSTM_ESHAPE;
-        // (a wait bound of the caller's asks for the kernel that has the wait: mlstm_set_spin_limit)
-        if ((long long)a.BH * a.NG <= roww_most && !a.precise && a.spin_limit == DEFAULT_SPIN_LIMIT) rc = launch_roww_kernel(mode, dtype, D, a, st);
+        if (roww_serves(dtype, D, a)) rc = launch_roww_kernel(mode, dtype, D, a, st);
         // Split mode: row_kernel / rowx_kernel, forward and dQ pass, us --
         // D = 128   64: 21.3, 23.2 / 13.5, 15.7   256: 23.4, 24.9 / 16.1, 18.4   384: 23.9, 26.5 / 22.6, 27.0   512: 24.8, 27.6 / 26.2, 29.8
         // D = 256   64: 39.3, 43.8 / 22.6, 26.9   256: 41.8, 47.3 / 26.0, 30.2   384: 42.9, 47.6 / 36.9, 42.4   512: 44.1, 49.0 / 40.8, 46.8

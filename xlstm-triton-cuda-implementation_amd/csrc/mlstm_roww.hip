@@ -15,13 +15,11 @@
 // Replaces, like mlstm_row8.hip, mlstm_matmul_kernel (mlstm_matmul.py:38-101) and the dQ loop of mlstm_matmul_kernel_backward
 // (mlstm_matmul.py:239-267).
 #include <type_traits>
-#include "mlstm_device.h"
-#include "mlstm_kernels.h"
+#include "mlstm_gates.h"
 
 namespace mlstm {
 
 constexpr int RW_FWD = 0, RW_DQ = 1;
-constexpr int RW_MOST_KEYS = 1024;   // keys a row may meet: their scalars stay in LDS for the whole kernel
 
 template <typename T, int D, int RB>
 struct RowwCfg {
@@ -34,7 +32,8 @@ struct RowwCfg {
     static size_t lds_bytes(int keys) { return POOL_BYTES + P_BYTES + PART_BYTES + MISC_FLOATS * 4 + (size_t)keys * 8 + GRAN * 4; }
 };
 
-template <typename T, int D, int MODE, int RB>
+// FUSED (forward, uncut sequences): the gates too, see RowArgs::gate_F
+template <typename T, int D, int MODE, int RB, bool FUSED>
 __global__ __launch_bounds__(256 * RB) void roww_kernel(RowArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using R = Tr<T>;
@@ -111,11 +110,31 @@ __global__ __launch_bounds__(256 * RB) void roww_kernel(RowArgs a) {
         copy_tile(y2_at(r, 0), Y2, 2 * r);
         if (2 * r + 1 < nJ) copy_tile(y2_at(r, 1), Y2, 2 * r + 1);
     };
+    // The gates of the head's granules up to the rows' own, granule wave + NW k in turn k, are requested first: copies into LDS (the places of
+    // their key weights), so that a counted wait can leave the tiles behind them under way while the gates are formed.  16-bit values come as the
+    // dword that holds them.  Two launches / one, forward, us: 1 x 64 x 128 7.9 / 6.3, 1 x 320 10.5 / 9.6, 1 x 640 12.9 / 12.9 (a granule is 250
+    // instructions, 100 of them its logarithms, and a workgroup forms all of its head's: 2 us of a CU for ten), 8 x 1000 19.5 / 18.1, 15 x 1001
+    // 22.7 / 19.2, 16 x 256 10.7 / 9.0; D = 256, 1 x 640 15.6 / 15.0, 8 x 1000 24.5 / 22.8, 24 x 1000 31.5 / 29.3, 100 x 128 12.3 / 9.5.
+    constexpr int NW = NT / 64, TURNS = FUSED ? RW_MOST_KEYS / GRAN / NW : 1;
+    if constexpr (FUSED) {
+        const size_t off = a.lg.head(bh), ss = (size_t)a.lg.ss, el = a.gate_dtype == MLSTM_F32 ? 4 : 2;
+#pragma unroll
+        for (int k = 0; k < TURNS; k++) {
+            const int g = tid / 64 + NW * k;
+            if (g < nJ) {
+                const int t = g * GRAN + lane;
+                const size_t at = (off + (size_t)(t < S ? t : S - 1) * ss) * el;
+                dma4((const void*)(((size_t)a.gate_F + at) & ~(size_t)3), __builtin_amdgcn_readfirstlane(lds_offset_of(sek + GRAN * g)));
+                dma4((const void*)(((size_t)a.gate_I + at) & ~(size_t)3), __builtin_amdgcn_readfirstlane(lds_offset_of(sal + GRAN * g)));
+            }
+        }
+    }
     // (plain loads first: what they bring is used behind the copies' issue)
-    const double g_rows = a.G2[goff + gt], g_mine = a.G2[goff + (tid < nJ ? tid : 0)], g_end = chunk > 0 ? a.G2[goff - 1] : 0.0;
-    const float beta_row = a.beta2[poff + rowc], beta_end = chunk > 0 ? a.beta2[poff - 1] : 0.f;
+    const double g_rows = FUSED ? 0.0 : a.G2[goff + gt], g_mine = FUSED ? 0.0 : a.G2[goff + (tid < nJ ? tid : 0)], g_end = chunk > 0 ? a.G2[goff - 1] : 0.0;
+    float beta_row = FUSED ? 0.f : a.beta2[poff + rowc];
+    const float beta_end = chunk > 0 ? a.beta2[poff - 1] : 0.f;
     const float n_mine = chunk > 0 && tid < D ? a.Nst[((size_t)bh * a.n_states + chunk - 1) * D + tid] : 0.f;
-    const float m_row = MODE == RW_FWD || kb == 0 ? a.M[hoff + rowc] : 0.f;
+    float m_row = !FUSED && (MODE == RW_FWD || kb == 0) ? a.M[hoff + rowc] : 0.f;
     const float b_row = MODE == RW_DQ && kb == 0 ? a.Bin[hoff + rowc] : 0.f;
     // piece i of a pair of complete tiles j, j + 1
     auto copy_piece = [&](const T* src, T* d0, T* d1, int j, int i) {
@@ -153,15 +172,96 @@ __global__ __launch_bounds__(256 * RB) void roww_kernel(RowArgs a) {
     }
     if (NST == 2 || chunk == 0) copy_y1(0);
     if (NST == 2) copy_y2(0);
-    for (int t = tdma.wave_s; t < nJ; t += NT / 64) {
-        dma4(a.ek2 + poff + GRAN * t + lane, __builtin_amdgcn_readfirstlane(lds_offset_of(sek + GRAN * t)));
-        dma4(a.alpha2 + poff + GRAN * t + lane, __builtin_amdgcn_readfirstlane(lds_offset_of(sal + GRAN * t)));
+    GateLocal gown{};     // of the rows' granule, in the wave that forms it
+    GateGlobal gbeta{};
+    double gbase = 0.0;
+    if constexpr (FUSED) {
+        // (in the row sums' place until those need it: totals and maxima of the granules, beta and m of the rows' own)
+        double* const sT = reinterpret_cast<double*>(part);
+        double* const sP = sT + RW_MOST_KEYS / GRAN;
+        float* const own = reinterpret_cast<float*>(sP + RW_MOST_KEYS / GRAN);   // [beta, m][64]
+        float c = 0.f;
+        // all but the copies behind the gates': the rows of X and one or two tiles of Y1 (NST == 2: and of Y2), as many of a wave whatever their rows
+        constexpr int PX = TileDma<T, D, ROWS, NT>::PER_WAVE, PT = NST * TileDma<T, D, GRAN, NT>::PER_WAVE;
+        if (nJ > 1) dma_wait_but<PX + 2 * PT>();
+        else dma_wait_but<PX + PT>();
+        // N turns side by side: a granule's 180 instructions are one chain of 1800 cycles
+        auto turns = [&](auto n_tag) __attribute__((always_inline)) {
+            constexpr int N = decltype(n_tag)::value;
+            float lf[N], ig[N], cs[N], al[N];
+            GateLocal vs[N];
+            const size_t off = a.lg.head(bh), ss = (size_t)a.lg.ss;
+#pragma unroll
+            for (int k = 0; k < N; k++) {
+                const int t = (wave + NW * k) * GRAN + lane, tr = (wave + NW * k < nJ ? t : lane);   // (a turn too many: some place that is there)
+                unsigned x = __builtin_bit_cast(unsigned, sek[tr]), y = __builtin_bit_cast(unsigned, sal[tr]);
+                if (a.gate_dtype != MLSTM_F32) {
+                    const size_t e = off + (size_t)(t < S ? t : S - 1) * ss;
+                    x >>= (((size_t)a.gate_F >> 1) + e) & 1 ? 16 : 0;
+                    y >>= (((size_t)a.gate_I >> 1) + e) & 1 ? 16 : 0;
+                    if (a.gate_dtype == MLSTM_F16) {
+                        x = __builtin_bit_cast(unsigned, (float)__builtin_bit_cast(_Float16, (unsigned short)x));
+                        y = __builtin_bit_cast(unsigned, (float)__builtin_bit_cast(_Float16, (unsigned short)y));
+                    } else {
+                        x <<= 16;
+                        y <<= 16;
+                    }
+                }
+                const GateIn in{__builtin_bit_cast(float, x), 0.f, __builtin_bit_cast(float, y)};
+                lf[k] = forget_log(in, t, a.gate_form);
+                ig[k] = in.i;
+            }
+#pragma unroll
+            for (int k = 0; k < N; k++) cs[k] = wave_scan_inclusive<OpAdd>((wave + NW * k) * GRAN + lane < S ? lf[k] : 0.0f);
+#pragma unroll
+            for (int k = 0; k < N; k++) {
+                const bool ok = (wave + NW * k) * GRAN + lane < S;
+                al[k] = ok ? ig[k] - cs[k] : -INFINITY;
+                vs[k] = gates_local(al[k], ok, lane);
+            }
+#pragma unroll
+            for (int k = 0; k < N; k++) {
+                const int g = wave + NW * k, t = g * GRAN + lane;
+                if (g < nJ) {
+                    const float tot = last_lane(cs[k]);
+                    if (lane == 0) { sT[g] = (double)tot; sP[g] = (double)vs[k].p; }
+                    sek[t] = vs[k].ek2;
+                    sal[t] = vs[k].alpha2;
+                    if ((lane & 31) == 0) sam[2 * g + (lane >> 5)] = vs[k].c0;
+                    c = cs[k];
+                    gown = vs[k];
+                }
+            }
+        };
+        if (nJ <= NW) turns(std::integral_constant<int, 1>{});
+        else if (TURNS == 2 || nJ <= 2 * NW) turns(std::integral_constant<int, 2>{});
+        else turns(std::integral_constant<int, TURNS>{});
+        __syncthreads();
+        if (wave == (gt & (NW - 1)) || wave == ((gt + 1) & (NW - 1))) {   // (the wave that holds the rows' granule, and another)
+            double incl, excl, mx;
+            granule_scan(lane < nJ ? sT[lane] : 0.0, lane < nJ ? sP[lane] : -INFINITY, 0.0, lane, incl, excl, mx);
+            const double before = before_lane(mx, lane), Gg = readlane_d(excl, gt);
+            if (wave == (gt & (NW - 1))) {
+                const int t = gt * GRAN + lane;
+                gbeta = gates_global(c, gown.loc, t < S, Gg, readlane_d(before, gt));
+                gbase = Gg;
+                own[lane] = gbeta.beta2;
+                own[GRAN + lane] = gbeta.m;
+            } else if (lane < nJ) {
+                sdg[lane] = (float)(product_apart(Gg, LOG2E_D) - product_apart(excl, LOG2E_D));
+            }
+        }
+    } else {
+        for (int t = tdma.wave_s; t < nJ; t += NT / 64) {
+            dma4(a.ek2 + poff + GRAN * t + lane, __builtin_amdgcn_readfirstlane(lds_offset_of(sek + GRAN * t)));
+            dma4(a.alpha2 + poff + GRAN * t + lane, __builtin_amdgcn_readfirstlane(lds_offset_of(sal + GRAN * t)));
+        }
+        if (tid < GRAN) dma4(a.amax2 + goff * 2 + tid, __builtin_amdgcn_readfirstlane(lds_offset_of(sam)));   // (2 nJ of them count; padded array)
     }
-    if (tid < GRAN) dma4(a.amax2 + goff * 2 + tid, __builtin_amdgcn_readfirstlane(lds_offset_of(sam)));   // (2 nJ of them count; padded array)
-    const float crow_base = -0.5f * __log2f((float)D) - beta_row;
+    float crow_base = -0.5f * __log2f((float)D) - beta_row;
     float dec = 0.f;   // the row's decay since the end of the previous chunk
     if (chunk > 0) dec = fast_exp2(beta_end - beta_row + (float)(g_rows - g_end));
-    if (tid < nJ) sdg[tid] = (float)(g_rows - g_mine);
+    if (!FUSED && tid < nJ) sdg[tid] = (float)(g_rows - g_mine);
     if (chunk > 0 && tid < D) nvl[tid] = n_mine;
     frag hfr[NS];
     if constexpr (MODE == RW_DQ) {
@@ -182,6 +282,18 @@ __global__ __launch_bounds__(256 * RB) void roww_kernel(RowArgs a) {
         for (int x = 0; x < 16; x++) acc[c][x] = 0.f;
     dma_wait();
     __syncthreads();
+    if constexpr (FUSED) {
+        const float* const own = part + 4 * (RW_MOST_KEYS / GRAN);
+        beta_row = own[rowc - GRAN * gt];
+        m_row = own[GRAN + rowc - GRAN * gt];
+        crow_base = -0.5f * __log2f((float)D) - beta_row;
+        // (of two workgroups with rows of a granule the first one writes its gates)
+        if (wave == (gt & (NW - 1)) && (r0 & (GRAN - 1)) == 0) {
+            const int t = gt * GRAN + lane;
+            store_local(gown, poff + t, goff + gt, lane, const_cast<float*>(a.alpha2), const_cast<float*>(a.ek2), const_cast<float*>(a.amax2));
+            store_global(gbeta, t < S, gbase, poff + t, hoff + t, goff + gt, lane, const_cast<float*>(a.beta2), const_cast<double*>(a.G2), const_cast<float*>(a.M));
+        }
+    }
     frag xf[NS];
 #pragma unroll
     for (int s = 0; s < NS; s++) xf[s] = rrd.read(xtile, rb, s);
@@ -574,14 +686,22 @@ __global__ __launch_bounds__(256 * RB) void roww_kernel(RowArgs a) {
 #endif
 }
 
-template <typename T, int D, int MODE, int RB>
-static int launch_roww_t(const RowArgs& a, hipStream_t st) {
+template <typename T, int D, int MODE, int RB, bool FUSED>
+static int launch_roww_f(const RowArgs& a, hipStream_t st) {
     using Cfg = RowwCfg<T, D, RB>;
     const int most = a.chunk_len > 0 && a.chunk_len < a.NG * GRAN ? a.chunk_len : a.NG * GRAN;   // keys a row may meet
     if (most > RW_MOST_KEYS) return MLSTM_ESHAPE;
-    if (hipError_t e = lds_limit_once<roww_kernel<T, D, MODE, RB>>((int)Cfg::lds_bytes(RW_MOST_KEYS)); e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL((roww_kernel<T, D, MODE, RB>), dim3(a.BH * a.NG * (2 / RB)), dim3(256 * RB), Cfg::lds_bytes(most), st, a);
+    if (hipError_t e = lds_limit_once<roww_kernel<T, D, MODE, RB, FUSED>>((int)Cfg::lds_bytes(RW_MOST_KEYS)); e != hipSuccess) return (int)e;
+    hipLaunchKernelGGL((roww_kernel<T, D, MODE, RB, FUSED>), dim3(a.BH * a.NG * (2 / RB)), dim3(256 * RB), Cfg::lds_bytes(most), st, a);
     return (int)hipGetLastError();
+}
+
+template <typename T, int D, int MODE, int RB>
+static int launch_roww_t(const RowArgs& a, hipStream_t st) {
+    if constexpr (MODE == RW_FWD) {
+        if (a.gate_F) return a.chunk_len > 0 ? MLSTM_EINVAL : launch_roww_f<T, D, MODE, RB, true>(a, st);
+    }
+    return launch_roww_f<T, D, MODE, RB, false>(a, st);
 }
 
 template <typename T, int RB>
