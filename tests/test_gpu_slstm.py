@@ -158,3 +158,23 @@ def test_short_sequences_of_every_prologue_length(B, NH, S, DH, forget_sigmoid):
     got = slstm_backward_hip(dh.cuda(), h, r.cuda(), saved, forget_sigmoid=forget_sigmoid)
     for name, g, w in zip(("dwx", "dr", "db"), got, SO.slstm_backward(dh, wx, r, b, forget_sigmoid)):
         assert_close(g, w, torch.float32, name)
+
+
+@pytest.mark.parametrize("DH", [32, 64, 128])
+@pytest.mark.parametrize("S", [1, 2, 3, 4, 5, 6, 7, 8, 9, 16, 17, 18, 19, 21])
+def test_backward_at_every_turn_of_the_helpers(S, DH):
+    # The waves beside a step's own serve every second or fourth step and keep four of these under way: sequences that end at each
+    # of their intervals.  A saved state off a 16-byte boundary is loaded a float a lane: the same values, so the same bits.
+    from slstm import slstm_backward_hip, slstm_forward_hip
+    B, NH = 2, 3
+    wx, r, b, dh = SO.make_inputs(B, NH, S, DH, seed=70 + S, f_mean=0.5)
+    h, saved = slstm_forward_hip(*gpu(wx, r, b), forget_sigmoid=True)
+    got = slstm_backward_hip(dh.cuda(), h, r.cuda(), saved, forget_sigmoid=True)
+    for name, g, w in zip(("dwx", "dr", "db"), got, SO.slstm_backward(dh, wx, r, b, True)):
+        assert_close(g, w, torch.float32, name)
+    for off in (1, 2):
+        def away(x):
+            skip = 4 * off // x.element_size()
+            return torch.empty(x.numel() + skip, dtype=x.dtype, device="cuda")[skip:].view(x.shape).copy_(x)
+        for g, w in zip(slstm_backward_hip(away(dh), h, r.cuda(), away(saved), forget_sigmoid=True), got):
+            assert torch.equal(g, w)

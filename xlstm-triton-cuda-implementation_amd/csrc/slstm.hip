@@ -13,6 +13,7 @@
 //   slstm_backward_kernel  back through time: rows of 16 lanes form R^T delta_{t+1} for their four units (a sixteenth of the
 //                          gradient vector per lane, summed over the row), which is what step t+1 sent back to h_t; the
 //                          lanes of a unit's quad turn (dh_t + that, dc, dn) into one pre-activation gradient each (= dWx_t).
+//                          Helper waves form the factors of that from the saved values and write dWx out.
 //                          The stabiliser m is a common scale of c and n that h does not depend on, so it is held constant.
 //   slstm_dr_kernel        dR_g = sum_{b,t} dWx_t[g] h_{t-1}^T and db_g = sum_{b,t} dWx_t[g]: off the sequential path, in
 //                          slices of (b, t) whose partial sums a second kernel adds in a fixed order.
@@ -44,9 +45,6 @@ constexpr int PF = 8;
 // (a row's address is uniform, the lane's place in it an offset in bytes)
 __device__ __forceinline__ void ring_load(const float* row, unsigned lane_off, unsigned lds_off) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(lane_off), "s"(row), "s"(lds_off) : "memory", "m0");
-}
-__device__ __forceinline__ void ring_load_lane(const float* g, unsigned lds_off) {   // an address of the lane's own
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "s"(lds_off) : "memory", "m0");
 }
 // (n is a constant once the step loops are unrolled; anything out of range waits for everything)
 __device__ __forceinline__ void ring_wait(int n) {
@@ -232,120 +230,245 @@ __global__ __launch_bounds__(4 * DH) void slstm_forward_kernel(const float* __re
 // sums to its own quad, and the exchange inside the quad finishes them.
 // Everything else a step computes is linear in dh_t: with dc, dn what comes back to c_t and n_t, lane q of a quad needs
 //     dc = dh A + dc',  dn = dh B + dn',  its gradient = P dc + Q dn  (q = 3: O dh)
-// and A, B, P, Q, O are made of saved values only.  They are formed, like the stores and the ring's refill, while the step
-// waits for the gradients from LDS, so that five instructions lie between dh_t and the gradient that is handed on (delta in two
-// buffers, taken in turns: one barrier per step).  Lane q loads saved value q, and value 4 + q or, for q = 3, dh.
-// B16 NH4 S2048 DH64: 925 us with those formed behind the sum, 810 now.
-template <int DH, bool FS>
-__global__ __launch_bounds__(4 * DH) void slstm_backward_kernel(const float* __restrict__ dh, const float* __restrict__ r,
-                                                                const float* __restrict__ saved, float* __restrict__ dwx, int NH,
-                                                                int S) {
+// and A, B, P, Q, O are made of saved values only, so that five instructions lie between dh_t and the gradient that is handed on
+// (delta in two buffers, taken in turns: one barrier per step).
+// What bounded a step was instruction issue: 157 instructions on the one wave of a SIMD, 4 to 5 cycles each, of which only 100 are on
+// the chain; the rest -- the factors, the ring of their inputs, the stores -- do not fit behind a trip to LDS of 130 cycles.  They
+// belong to waves of their own: helper group g of NGRP, a lane per unit, serves every NGRP-th step, its work spread over the
+// intervals between as many barriers, and leaves a step's factors in LDS ahead of it.  (A lane per unit, where each of the quad's
+// lanes formed the same factors: the helpers issue a fraction of what they replace.  Work of more than some 250 ns in one
+// interval makes the step wait for it: addresses that walk, and 16-byte loads of several rows at a time.)
+// Now a step is bounded by R^T delta alone: the same kernel whose helpers only met the barriers took 515 of its 519 us.
+// Backward, us, without / with the helpers: B16 NH4, DH = 64, S = 2048 824 / 519; DH = 32, S = 1024 317 / 209; DH = 128, S = 1024
+// 682 / 528; 256 and 512 workgroups (DH = 64, S = 500; S = 300) 212 / 144, 172 / 125; DH = 32 at 1024 workgroups and S = 200, where
+// 3.6 TB/s are moved, 86.6 / 88.7.
+constexpr int BWD_SAVED = 10;   // rows of the saved state that a step's factors are made of: i~, log f, z, o, c, n, m of the step, c, n, m of the one before it in time
+template <int DH>
+struct BwdCfg {
+    static constexpr int UW = DH > 64 ? DH / 64 : 1;      // waves per helper group
+    static constexpr int NGRP = DH > 64 ? 2 : 4;
+    static constexpr int THREADS = 4 * DH + NGRP * UW * 64;
+    static constexpr int RING = 4;                         // jobs of a group under way
+    static constexpr int SLOTS = 4;                        // steps whose factors are in LDS
+};
+
+// WIDE: saved is on a 16-byte boundary (its rows then are, too): four floats per lane and load
+template <int DH, bool FS, bool WIDE>
+__global__ __launch_bounds__(BwdCfg<DH>::THREADS) void slstm_backward_kernel(const float* __restrict__ dh, const float* __restrict__ r,
+                                                                             const float* __restrict__ saved, float* __restrict__ dwx, int NH,
+                                                                             int S) {
+    using Cfg = BwdCfg<DH>;
     constexpr int PE = DH / 4;       // gradients per lane: a sixteenth of the 4 DH (in the order unit * 4 + gate)
     constexpr int PS = PE + 4;       // ... and four floats, so that the 16 parts of a row's read start in different banks
-    __shared__ __attribute__((aligned(16))) float delta[2][16 * PS];       // [buffer][part][unit * 4 + gate within the part]
-    __shared__ __attribute__((aligned(16))) float ring[PF][2][4 * DH];     // [slot][0: saved 0..3 | 1: saved 4..6, dh][unit * 4 + q]
-    const int tid = threadIdx.x, k = tid >> 2, q = tid & 3, wave = tid >> 6;
-    const bool is0 = q == 0, is1 = q == 1, is2 = q == 2;
+    constexpr int UW = Cfg::UW, NGRP = Cfg::NGRP, RING = Cfg::RING, SLOTS = Cfg::SLOTS, UL = DH < 64 ? DH : 64;   // UL: units per helper wave
+    constexpr int RPL = WIDE ? 256 / UL : 1, NLOAD = (BWD_SAVED + RPL - 1) / RPL;   // rows per load, loads per job
+    struct Lds {   // (what the steps read comes first: within an offset of the instructions)
+        float delta[2][16 * PS];             // [buffer][part][unit * 4 + gate within the part]
+        float shared_of[SLOTS][DH][4];       // A, B, f', dh of a unit
+        float own_of[SLOTS][DH][4][2];       // P, Q of gates 0..2; O
+        float ring[NGRP * UW][RING][(BWD_SAVED + 1) * UL];   // of a job: ten rows of the saved state, dh
+    };
+    __shared__ __attribute__((aligned(16))) Lds lds;
+    auto& delta = lds.delta;
+    auto& shared_of = lds.shared_of;
+    auto& own_of = lds.own_of;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int b = blockIdx.x / NH, hd = blockIdx.x % NH;
-    const int part = tid & 15, k4 = (tid >> 4) * 4;   // the lane's part of the gradient vector; the first of its row's four units
-    const int urow = k & 3;                           // which of the row's units is this lane's own
-    float rc[PE][4];   // [gradient of the part][s]: R_g[j][k4 + (urow + s) mod 4] for the part's (j, g)
-#pragma unroll
-    for (int e = 0; e < PE; e++) {
-        const int f = part * PE + e, j = f >> 2, g = f & 3;
-        const f32x4 v = *reinterpret_cast<const f32x4*>(r + (((size_t)hd * 4 + g) * DH + j) * DH + k4);
-#pragma unroll
-        for (int s = 0; s < 4; s++) rc[e][s] = pick(urow == 0, urow == 1, urow == 2, v[s], v[(s + 1) & 3], v[(s + 2) & 3], v[(s + 3) & 3]);
-    }
     const size_t step_wx = (size_t)4 * NH * DH, step_h = (size_t)NH * DH, step_s = (size_t)7 * NH * DH;
-    // rows that walk with the steps, from the last one down (f0, f1: what the ring takes next; the second is saved values 4..6
-    // or dh, so its address is the lane's own)
-    const unsigned at_gate = (unsigned)((q * NH + hd) * DH + k);
-    const float* f0 = saved + ((size_t)b * S + S - 1) * step_s;
-    const float* f1 = q < 3 ? saved + ((size_t)b * S + S - 1) * step_s + ((size_t)(4 + q) * NH + hd) * DH + k
-                            : dh + ((size_t)b * S + S - 1) * step_h + (size_t)hd * DH + k;
-    const size_t step1 = q < 3 ? step_s : step_h;
-    float* dwrow = dwx + ((size_t)b * S + S - 1) * step_wx;
-    const int mine_at = ((4 * k + q) / PE) * PS + (4 * k + q) % PE;   // where this lane's gradient goes in a delta buffer
-    const unsigned ring_base = __builtin_amdgcn_readfirstlane(mlstm::lds_offset_of(&ring[0][0][0]) + wave * 256);
-    auto fetch = [&](int u, bool more) __attribute__((always_inline)) {   // (before the start of the sequence: row 0 again)
-        ring_load(f0, 4 * at_gate, ring_base + (2 * u) * (4 * DH * 4));
-        ring_load_lane(f1, ring_base + (2 * u + 1) * (4 * DH * 4));
-        if (more) { f0 -= step_s; f1 -= step1; }
-    };
-    constexpr int OPS = 3;   // per wave and step: the store of dwx, then two ring loads
+    for (int e = tid; e < 16 * PS; e += Cfg::THREADS) delta[0][e] = 0.f;   // (nothing comes back to the last step)
+    // step n (of S, counted down in time) is row S - 1 - n; its gradients go to buffer (n & 1) ^ 1, its factors lie in slot n % SLOTS
+    if (wave < 4 * DH / 64) {
+        const int k = tid >> 2, q = tid & 3;
+        const int part = tid & 15, k4 = (tid >> 4) * 4;   // the lane's part of the gradient vector; the first of its row's four units
+        const int urow = k & 3;                           // which of the row's units is this lane's own
+        float rc[PE][4];   // [gradient of the part][s]: R_g[j][k4 + (urow + s) mod 4] for the part's (j, g)
 #pragma unroll
-    for (int u = 0; u < PF; u++) fetch(u, S - 2 - u >= 0);
-    for (int e = tid; e < 16 * PS; e += 4 * DH) delta[0][e] = 0.f;   // (nothing comes back to the last step)
-    float dc_next = 0.f, dn_next = 0.f, mine = 0.f;
-    f32x4 s0, s1, sp;   // i~, log f, z, o | c, n, m, dh of the step to come | c, n, m of the one before it in time
-    auto take = [&](int u) __attribute__((always_inline)) {
-        s0 = *reinterpret_cast<const f32x4*>(&ring[u % PF][0][4 * k]);
-        s1 = *reinterpret_cast<const f32x4*>(&ring[u % PF][1][4 * k]);
-        sp = *reinterpret_cast<const f32x4*>(&ring[(u + 1) % PF][1][4 * k]);
-    };
-    ring_wait(2 * (PF - 2));
-    take(0);
-    __syncthreads();
-    // One step, the u-th of its round.  wait_n: how many of the wave's memory operations may still be under way when the
-    // next step's values are taken from the ring.
-    auto step = [&](int u, int t, int wait_n, bool first) __attribute__((always_inline)) {
-        const float* dcur = delta[u & 1] + part * PS;
-        f32x4 dl[PE / 4];
+        for (int e = 0; e < PE; e++) {
+            const int f = part * PE + e, j = f >> 2, g = f & 3;
+            const f32x4 v = *reinterpret_cast<const f32x4*>(r + (((size_t)hd * 4 + g) * DH + j) * DH + k4);
 #pragma unroll
-        for (int e = 0; e < PE / 4; e++) dl[e] = *reinterpret_cast<const f32x4*>(dcur + 4 * e);
-        __builtin_amdgcn_sched_barrier(0);
-        if (!first) {   // the step before: its gradient goes out, its slot takes the row PF steps on
-            dwrow[at_gate] = mine;
-            dwrow -= step_wx;
-            fetch((u + PF - 1) % PF, t - PF >= 0);
+            for (int s = 0; s < 4; s++) rc[e][s] = pick(urow == 0, urow == 1, urow == 2, v[s], v[(s + 1) & 3], v[(s + 2) & 3], v[(s + 3) & 3]);
         }
-        if (t == 0) { sp[0] = 0.f; sp[1] = 0.f; sp[2] = -INFINITY; }
-        const float it = s0[0], logf = s0[1], z = s0[2], o = s0[3], ct = s1[0], nt = s1[1], mt = s1[2], dht = s1[3];
+        const int mine_at = ((4 * k + q) / PE) * PS + (4 * k + q) % PE;   // where this lane's gradient goes in a delta buffer
+        float dc_next = 0.f, dn_next = 0.f;
+        __syncthreads();
+        auto step = [&](auto u_tag) __attribute__((always_inline)) {
+            constexpr int u = decltype(u_tag)::value;
+            const float* dcur = delta[u & 1] + part * PS;
+            constexpr int AHEAD = PE / 4 < 4 ? PE / 4 : 4;   // (reads under way: DH = 128 has registers for no more)
+            f32x4 dl[PE / 4];
+#pragma unroll
+            for (int e = 0; e < AHEAD; e++) dl[e] = *reinterpret_cast<const f32x4*>(dcur + 4 * e);
+            const f32x4 sh = *reinterpret_cast<const f32x4*>(shared_of[u % SLOTS][k]);   // (a quad reads one address)
+            const float2 pq = *reinterpret_cast<const float2*>(own_of[u % SLOTS][k][q]);
+            __builtin_amdgcn_sched_barrier(0);
+            float a[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int e = 0; e < PE / 4; e++) {
+#pragma unroll
+                for (int f = 0; f < 4; f++)
+#pragma unroll
+                    for (int x = 0; x < 4; x++) a[x] += rc[4 * e + f][x] * dl[e][f];
+                if (e + AHEAD < PE / 4) {   // (the sums so far are formed before the next read is issued)
+                    asm volatile("" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]));
+                    __builtin_amdgcn_sched_barrier(0);
+                    dl[e + AHEAD] = *reinterpret_cast<const f32x4*>(dcur + 4 * (e + AHEAD));
+                }
+            }
+            // (row_ror: lane i takes from lane i - 4s of its row, whose s-th unit is this quad's own)
+            const float dhrec = quad_sum((a[0] + quad_perm<0x124>(a[1])) + (quad_perm<0x128>(a[2]) + quad_perm<0x12C>(a[3])));
+            const float d_h = sh[3] + dhrec;
+            const float dc = fmaf(d_h, sh[0], dc_next), dn = fmaf(d_h, sh[1], dn_next);   // (the shorter way from d_h)
+            const float lin = fmaf(dc, pq.x, dn * pq.y);
+            delta[(u & 1) ^ 1][mine_at] = q == 3 ? d_h * pq.x : lin;
+            dc_next = dc * sh[2];
+            dn_next = dn * sh[2];
+            mlstm::pin(dc_next); mlstm::pin(dn_next);
+            __syncthreads();
+        };
+        static_assert(SLOTS == 4, "the steps are unrolled by the slots");
+        int n = 0;
+        for (; n + 4 <= S; n += 4) {
+            step(std::integral_constant<int, 0>{});
+            step(std::integral_constant<int, 1>{});
+            step(std::integral_constant<int, 2>{});
+            step(std::integral_constant<int, 3>{});
+        }
+        if (n < S) { step(std::integral_constant<int, 0>{}); n++; }
+        if (n < S) { step(std::integral_constant<int, 1>{}); n++; }
+        if (n < S) step(std::integral_constant<int, 2>{});
+        return;
+    }
+    // ---- helpers: job i of a group is step g + NGRP i
+    const int hw = wave - 4 * DH / 64, g = hw / UW, u0 = (hw % UW) * 64, unit = u0 + (lane < UL ? lane : 0);
+    const bool there = lane < UL;
+    const unsigned row_bytes = (unsigned)(step_h * 4), state_bytes = (unsigned)(step_s * 4);   // (from row to row of a state, from state to state)
+    const unsigned lane_off = 4u * (unsigned)(hd * DH + unit);
+    float* const myring = &lds.ring[hw][0][0];
+    const unsigned ring_base = __builtin_amdgcn_readfirstlane(mlstm::lds_offset_of(myring));
+    // Rows 0..6 are those of state t, 7..9 rows 4..6 of the state before it; offsets count from that one.  A lane's piece of load l (WIDE: 16 bytes,
+    // RPL rows a load) and whether it is of state t.
+    constexpr int JOB = (BWD_SAVED + 1) * UL, PIECES = WIDE ? NLOAD : 1, LAST_LANES = (BWD_SAVED - (NLOAD - 1) * RPL) * UL / 4;
+    unsigned off[PIECES];
+    bool of_t[PIECES];
+    if constexpr (WIDE) {
+#pragma unroll
+        for (int l = 0; l < PIECES; l++) {
+            int v = l * RPL + lane / (UL / 4);
+            v = v < BWD_SAVED ? v : BWD_SAVED - 1;
+            of_t[l] = v < 7;
+            off[l] = (unsigned)(v < 7 ? v : v - 3) * row_bytes + (v < 7 ? state_bytes : 0u) + 4u * (unsigned)(hd * DH + u0 + 4 * (lane % (UL / 4)));
+        }
+    }
+    int tf = S - 1 - g;                                                       // the row that is requested next
+    const float* sf = saved + ((size_t)b * S + tf - 1) * step_s;              // the state before it (not read where tf < 1)
+    const float* df = dh + ((size_t)b * S + tf) * step_h;
+    const float* const s_first = saved + (size_t)b * S * step_s;
+    const float* const d_first = dh + (size_t)b * S * step_h;
+    unsigned at = ring_base;
+    auto fetch = [&]() __attribute__((always_inline)) {   // (steps past the last one: row 0; there is no state before that: its own)
+        const bool inside = tf >= 1;
+        const float* const base = inside ? sf : s_first;
+        if constexpr (WIDE) {
+#pragma unroll
+            for (int l = 0; l < PIECES; l++) {
+                const unsigned o = inside || !of_t[l] ? off[l] : off[l] - state_bytes;
+                if (l < PIECES - 1 || lane < LAST_LANES)
+                    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(o), "s"(base), "s"(at + 1024 * l) : "memory", "m0");
+            }
+        } else if (there) {
+#pragma unroll
+            for (int v = 0; v < BWD_SAVED; v++)
+                ring_load(base, lane_off + (unsigned)(v < 7 ? v : v - 3) * row_bytes + (v < 7 && inside ? state_bytes : 0u), at + 4 * UL * v);
+        }
+        if (there) ring_load(tf >= 0 ? df : d_first, lane_off, at + 4 * UL * BWD_SAVED);
+        tf -= NGRP;
+        sf -= NGRP * step_s;
+        df -= NGRP * step_h;
+        at = at == ring_base + (RING - 1) * JOB * 4 ? ring_base : at + JOB * 4;
+    };
+    float in[BWD_SAVED], dht = 0.f;
+    auto take = [&](int i) __attribute__((always_inline)) {
+        const float* const from = myring + (i & (RING - 1)) * JOB + (there ? lane : 0);
+#pragma unroll
+        for (int v = 0; v < BWD_SAVED; v++) in[v] = from[v * UL];
+        dht = from[BWD_SAVED * UL];
+        if (g + NGRP * i >= S - 1) { in[7] = 0.f; in[8] = 0.f; in[9] = -INFINITY; }
+    };
+    float A = 0.f, B = 0.f, O = 0.f, fp = 0.f, P0 = 0.f, Q0 = 0.f, P1 = 0.f, Q1 = 0.f, P2 = 0.f;
+    auto factors = [&]() __attribute__((always_inline)) {
+        const float it = in[0], logf = in[1], z = in[2], o = in[3], ct = in[4], nt = in[5], mt = in[6];
         const float ip = fast_exp(it - mt);
-        float fp = fast_exp(logf + sp[2] - mt);
+        fp = fast_exp(logf + in[9] - mt);
         const float inv_n = fast_rcp(nt), psi = ct * inv_n;
-        float A = o * inv_n, B = -A * psi, O = psi * o * (1.0f - o);
+        A = o * inv_n; B = -A * psi; O = psi * o * (1.0f - o);
         // d i~ = (dc z + dn) i',  d f~ = (dc c_{t-1} + dn n_{t-1}) f' (sigmoid gate: sigmoid(-f~) = 1 - exp(log f)),  d z~ = dc i' (1 - z^2)
         const float fs = FS ? fp * (1.0f - fast_exp(logf)) : fp;
-        float P = pick(is0, is1, true, z * ip, sp[0] * fs, ip * (1.0f - z * z), 0.f);
-        float Q = pick(is0, is1, true, ip, sp[1] * fs, 0.f, 0.f), dht_own = dht;
-        // (here, not among the multiply-adds below)
-        mlstm::pin(A); mlstm::pin(B); mlstm::pin(O); mlstm::pin(P); mlstm::pin(Q); mlstm::pin(fp); mlstm::pin(dht_own);
-        ring_wait(wait_n);
-        take(u + 1);
-        __builtin_amdgcn_sched_barrier(0);
-        float a[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int e = 0; e < PE; e++)
-#pragma unroll
-            for (int x = 0; x < 4; x++) a[x] += rc[e][x] * dl[e >> 2][e & 3];
-        // (row_ror: lane i takes from lane i - 4s of its row, whose s-th unit is this quad's own)
-        const float dhrec = quad_sum((a[0] + quad_perm<0x124>(a[1])) + (quad_perm<0x128>(a[2]) + quad_perm<0x12C>(a[3])));
-        const float d_h = dht_own + dhrec;
-        const float dc = d_h * A + dc_next, dn = d_h * B + dn_next;
-        const float lin = dc * P + dn * Q;
-        mine = q == 3 ? d_h * O : lin;
-        delta[(u & 1) ^ 1][mine_at] = mine;
-        dc_next = dc * fp;
-        dn_next = dn * fp;
-        mlstm::pin(sp);   // (its unused fourth value must not lend its register to the sums while the read is under way)
-        __syncthreads();
+        P0 = z * ip; Q0 = ip;
+        P1 = in[7] * fs; Q1 = in[8] * fs;
+        P2 = ip * (1.0f - z * z);
     };
-    // Step n (of S, counted down in time) takes rows n + 1 and n + 2 for its successor.  Row m >= PF was loaded in step
-    // m - PF + 1, as the last of its operations: behind row n + 2 lie the OPS operations of each of PF - 3 steps (the wait
-    // allows one step's fewer).  The rows before come from the prologue, with the later slots' loads and the operations of
-    // steps 1 .. n (one step's fewer again) behind them.  All of them are the quad's own wave's loads.
+    auto put = [&](int i) __attribute__((always_inline)) {
+        if (there) {
+            const int slot = (g + NGRP * i) & (SLOTS - 1);
+            *reinterpret_cast<f32x4*>(shared_of[slot][unit]) = f32x4{A, B, fp, dht};
+            *reinterpret_cast<f32x4*>(own_of[slot][unit][0]) = f32x4{P0, Q0, P1, Q1};
+            *reinterpret_cast<f32x4*>(own_of[slot][unit][2]) = f32x4{P2, 0.f, O, 0.f};
+        }
+    };
+    const int grad_at = (4 * unit / PE) * PS + 4 * unit % PE;
+    unsigned gate_off[4];
 #pragma unroll
-    for (int u = 0; u < PF; u++)
-        if (S - 1 - u >= 0)
-            step(u, S - 1 - u, u < PF - 2 ? 2 * (PF - 3 - u) + (u > 0 ? OPS * (u - 1) : 0) : OPS * (PF - 4), u == 0);
-    for (int t0 = S - 1 - PF; t0 >= 0; t0 -= PF) {
+    for (int x = 0; x < 4; x++) gate_off[x] = lane_off + (unsigned)x * row_bytes;
+    auto store = [&](int n) __attribute__((always_inline)) {   // the gradients of step n
+        const f32x4 v = *reinterpret_cast<const f32x4*>(delta[(n & 1) ^ 1] + grad_at);
+        char* const row = reinterpret_cast<char*>(dwx + ((size_t)b * S + (S - 1 - n)) * step_wx);
+        if (there) {
 #pragma unroll
-        for (int u = 0; u < PF; u++)
-            if (t0 - u >= 0) step(u, t0 - u, OPS * (PF - 4), false);
+            for (int x = 0; x < 4; x++) *reinterpret_cast<float*>(row + gate_off[x]) = v[x];
+        }
+    };
+#pragma unroll 1
+    for (int i = 0; i < RING; i++) fetch();
+    ring_wait(0);
+    take(0);
+    factors();
+    put(0);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (slot 0 has been read)
+    if (g == 0) fetch();
+    __syncthreads();
+    // Interval n lies between barriers n and n + 1, beside step n.  A group's turn for job i (of step g + NGRP i) begins NGRP intervals ahead: the values
+    // out of the ring; the factors; these to LDS, one interval at least before they are read; then the loads of the job RING on, into the same
+    // place, and the store of step n - 1.  A job's loads are waited for with those of one job less than are younger still under way (stores
+    // only make the wait longer).
+    int n = 0;
+    for (; n < g && n < S; n++) {   // (the end of the turn whose job 0 is done)
+        if (n == g - 1) {
+            fetch();
+            if (n > 0) store(n - 1);
+        }
+        __syncthreads();
     }
-    dwrow[at_gate] = mine;
+    for (int job = 1; n < S; job++) {
+        ring_wait((RING - 2) * (NLOAD + 1));
+        take(job);
+        if constexpr (NGRP == 2) { factors(); put(job); }
+        __syncthreads();
+        if (++n == S) break;
+        if constexpr (NGRP == 4) {
+            factors();
+            __syncthreads();
+            if (++n == S) break;
+            put(job);
+            __syncthreads();
+            if (++n == S) break;
+        }
+        fetch();
+        store(n - 1);
+        __syncthreads();
+        n++;
+    }
+    if ((S - g) % NGRP == NGRP - 1 || (S < g && S == g - 1)) store(S - 1);
 }
 
 constexpr int dr_parts(int DH) { return DH <= 64 ? 4 : 1; }   // partial sums per slice (slstm_dr_kernel's PARTS)
@@ -517,16 +640,22 @@ int forward_t(const float* wx, const float* r, const float* b, float* h, float* 
     return forward_launch<DH, false, false>(wx, r, b, h, saved, B, NH, S, st);
 }
 
+template <int DH, bool FS, bool WIDE>
+int backward_launch_w(const float* dh, const float* r, const float* saved, float* dwx, int B, int NH, int S, hipStream_t st) {
+    if (int rc = mlstm::no_scratch_once<slstm_backward_kernel<DH, FS, WIDE>>()) return rc;
+    hipLaunchKernelGGL((slstm_backward_kernel<DH, FS, WIDE>), dim3(B * NH), dim3(BwdCfg<DH>::THREADS), 0, st, dh, r, saved, dwx, NH, S);
+    return (int)hipGetLastError();
+}
+template <int DH, bool FS>
+int backward_launch(const float* dh, const float* r, const float* saved, float* dwx, int B, int NH, int S, hipStream_t st) {
+    return reinterpret_cast<size_t>(saved) & 15 ? backward_launch_w<DH, FS, false>(dh, r, saved, dwx, B, NH, S, st)
+                                                : backward_launch_w<DH, FS, true>(dh, r, saved, dwx, B, NH, S, st);
+}
+
 template <int DH>
 int backward_t(const float* dh, const float* h, const float* r, const float* saved, float* dwx, float* dr, float* db, int B, int NH, int S,
                int fs, char* ws, hipStream_t st) {
-    if (fs) {
-        if (int rc = mlstm::no_scratch_once<slstm_backward_kernel<DH, true>>()) return rc;
-        hipLaunchKernelGGL((slstm_backward_kernel<DH, true>), dim3(B * NH), dim3(4 * DH), 0, st, dh, r, saved, dwx, NH, S);
-    } else {
-        if (int rc = mlstm::no_scratch_once<slstm_backward_kernel<DH, false>>()) return rc;
-        hipLaunchKernelGGL((slstm_backward_kernel<DH, false>), dim3(B * NH), dim3(4 * DH), 0, st, dh, r, saved, dwx, NH, S);
-    }
+    if (int rc = fs ? backward_launch<DH, true>(dh, r, saved, dwx, B, NH, S, st) : backward_launch<DH, false>(dh, r, saved, dwx, B, NH, S, st)) return rc;
     const int ns = slices_for(B, NH, S);
     const size_t nr = (size_t)NH * 4 * DH * DH, nb = (size_t)NH * 4 * DH;
     float* part_r = reinterpret_cast<float*>(ws);
