@@ -178,3 +178,20 @@ def test_backward_at_every_turn_of_the_helpers(S, DH):
             return torch.empty(x.numel() + skip, dtype=x.dtype, device="cuda")[skip:].view(x.shape).copy_(x)
         for g, w in zip(slstm_backward_hip(away(dh), h, r.cuda(), away(saved), forget_sigmoid=True), got):
             assert torch.equal(g, w)
+
+
+@pytest.mark.parametrize("DH", [32, 64, 128])
+@pytest.mark.parametrize("S", [1, 2, 3, 7, 8, 9, 10, 11, 17, 26])
+def test_forward_at_every_turn_of_the_helpers(S, DH):
+    # Waves beside the walk bring its inputs and write out what it keeps, a step and two behind it: sequences that end around the turns of the
+    # ring.  Inputs off a 16-byte boundary go a float a lane: the same values, so the same bits.
+    from slstm import slstm_forward_hip
+    wx, r, b, _ = SO.make_inputs(3, 2, S, DH, seed=90 + S, f_mean=0.5)
+    h, saved = slstm_forward_hip(*gpu(wx, r, b), forget_sigmoid=True)
+    assert_close(h, SO.slstm_forward(wx, r, b, True), torch.float32, "h")
+    flat = torch.empty(wx.numel() + 3, device="cuda")
+    for off in (1, 3):
+        other = flat[off:off + wx.numel()].view(wx.shape).copy_(wx)
+        h2, saved2 = slstm_forward_hip(other, r.cuda(), b.cuda(), forget_sigmoid=True)
+        h3, _ = slstm_forward_hip(other, r.cuda(), b.cuda(), forget_sigmoid=True, save=False)
+        assert torch.equal(h2, h) and torch.equal(saved2, saved) and torch.equal(h3, h)

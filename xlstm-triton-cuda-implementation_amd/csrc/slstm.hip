@@ -9,7 +9,7 @@
 // workgroup per (batch, head) walks the sequence with the head's four recurrent matrices in registers.
 //   slstm_forward_kernel   eight lanes per two units, each with an eighth of the units' rows of all four R_g: partial
 //                          pre-activations from h_{t-1} (LDS), one gate's sum per lane; every lane then updates the cell of its
-//                          unit.  Gate values and (c, n, m) are kept for the backward.
+//                          unit.  Gate values and (c, n, m) are kept for the backward.  Helper waves bring the inputs and write the outputs.
 //   slstm_backward_kernel  back through time: rows of 16 lanes form R^T delta_{t+1} for their four units (a sixteenth of the
 //                          gradient vector per lane, summed over the row), which is what step t+1 sent back to h_t; the
 //                          lanes of a unit's quad turn (dh_t + that, dc, dn) into one pre-activation gradient each (= dWx_t).
@@ -34,13 +34,12 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ float fast_exp(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896340736f); }
 __device__ __forceinline__ float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 
-// Inputs of a step come from memory PF steps ahead of it, as direct-to-LDS loads into a ring (a trip to memory is several
-// steps long, and a step must not wait for one).  The loads are issued and waited for by hand: every wave issues the same
-// number of memory operations per step, in the same order (OPS: its stores, then its ring loads, none under a branch), so
+// Inputs of a step come from memory several steps ahead, as direct-to-LDS loads into a ring (a trip to memory is several
+// steps long, and a step must not wait for one).  The loads are issued and waited for by hand, by helper waves that issue the same
+// number of memory operations in every interval between two barriers, in the same order, so that
 // "the loads of step t have landed" is a counted wait -- memory operations of a wave complete in the order issued.  The
-// kernels' own code has only stores besides, for which the compiler places no waits.  (Left to the compiler, ordinary
-// loads into a ring of registers ended in a wait for everything at every step.)  A lane only ever reads ring values that
-// its own wave loaded, so the wait needs no barrier behind it.
+// helpers' own code has only stores besides, for which the compiler places no waits.  (Left to the compiler, ordinary
+// loads into a ring of registers ended in a wait for everything at every step.)
 constexpr int PF = 8;
 // (a row's address is uniform, the lane's place in it an offset in bytes)
 __device__ __forceinline__ void ring_load(const float* row, unsigned lane_off, unsigned lds_off) {
@@ -101,125 +100,216 @@ __device__ __forceinline__ float pick(bool is0, bool is1, bool is2, float a, flo
 // one logarithm serve the three kinds side by side), the quad exchanges the four results, and every lane updates the cell, all
 // four alike (c, n, m are kept four times, the same bits).  A step has no hand-over between waves but h itself: one LDS write,
 // one barrier (h in two buffers, taken in turns).
-// What bounds it is the serial chain of a step, 340 ns or some 800 cycles (DH = 64): the trip of h through LDS and the barrier about
-// 300, 64 multiply-adds at 4 cycles on the one wave of a SIMD, the gates 160.  Eighths and not quarters because the LDS reads of
-// h (32 DH floats a step) were the longest part of that trip; whatever a step does not hand on -- its stores, the ring's refill,
-// its own input -- is done in the NEXT step, while that waits for h from LDS.  Row broadcasts in the place of wide LDS reads were
+// What bounds it is the serial chain of a step, 300 ns or some 720 cycles (DH = 64): the trip of h through LDS and the barrier about
+// 250, 64 multiply-adds at 4 cycles on the one wave of a SIMD, the gates 200.  Eighths and not quarters because the LDS reads of
+// h (32 DH floats a step) were the longest part of that trip.  Row broadcasts in the place of wide LDS reads were
 // slower (DH = 128: 831 to 889 us): a broadcast, alone or as an operand of the multiply-add, costs as much as one.
-// Forward, B16 NH4, before (quarters, all four gates in every lane, stores ahead of the barrier) -> now: DH = 64, S = 2048 716 ->
-// 700 us; DH = 128, S = 1024 627 -> 559; DH = 32, S = 1024 285 -> 281.
-template <int DH, bool SAVE, bool FS>
-__global__ __launch_bounds__(4 * DH) void slstm_forward_kernel(const float* __restrict__ wx, const float* __restrict__ r,
-                                                               const float* __restrict__ bias, float* __restrict__ h,
-                                                               float* __restrict__ saved, int NH, int S) {
+// Global memory belongs to helper waves: they bring the steps' inputs into a ring, PF steps ahead, and write out what a step keeps, which the
+// walk leaves in LDS in the NEXT step, while that waits for h.  With its own stores and ring loads in that place a step issued 28 instructions
+// there, more than the wait hides.
+// Forward, B16 NH4, us, quarters / eighths / helpers: DH = 64, S = 2048 716 / 690 / 613; DH = 128, S = 1024 627 / 559 / 553 (545 without the saved state); DH = 32,
+// S = 1024 285 / 281 / 246.
+template <int DH>
+struct FwdCfg {
+    static constexpr int UW = DH > 64 ? DH / 64 : 1;   // helper waves: a 16-byte piece of a step's input per lane
+    static constexpr int THREADS = 4 * DH + 64 * UW;
+};
+// WIDE: wx, h and saved are on 16-byte boundaries (their rows then are, too)
+template <int DH, bool SAVE, bool FS, bool WIDE>
+__global__ __launch_bounds__(FwdCfg<DH>::THREADS) void slstm_forward_kernel(const float* __restrict__ wx, const float* __restrict__ r,
+                                                                            const float* __restrict__ bias, float* __restrict__ h,
+                                                                            float* __restrict__ saved, int NH, int S) {
+    using Cfg = FwdCfg<DH>;
     constexpr int KP = DH / 8, KS = KP < 16 ? KP : KP + 4;   // a part of h, and its place in LDS (eight parts, no bank twice)
+    constexpr int SR = DH + 16;                              // a row of `stage` (the four rows that a wave writes: no bank twice)
     __shared__ __attribute__((aligned(16))) float hs[2][8 * KS];
-    __shared__ __attribute__((aligned(16))) float ring[PF][4 * DH];   // wx of the next PF steps: [slot][unit * 4 + gate]
-    const int tid = threadIdx.x, j = tid >> 2, q = tid & 3, wave = tid >> 6;
-    const bool is0 = q == 0, is1 = q == 1, is2 = q == 2;
+    __shared__ __attribute__((aligned(16))) float ring[PF][4 * DH];             // wx of the next PF steps: [slot][unit / 4][gate][unit % 4]
+    __shared__ __attribute__((aligned(16))) float stage[SAVE ? 2 : 1][SAVE ? 8 * SR : 4];   // [step mod 2][i~, log f, z, o, c, n, m, unused][unit]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int b = blockIdx.x / NH, hd = blockIdx.x % NH;
-    const int p = tid & 7;
-    float ro[4][KP], rx[4][KP];   // part p of the rows of the own unit, [s: gate q ^ s], and of the octet's other one, [s: gate q ^ 3 ^ s]
-#pragma unroll
-    for (int s = 0; s < 4; s++) {
-        const float* own = r + (((size_t)hd * 4 + (q ^ s)) * DH + j) * DH + p * KP;
-        const float* oth = r + (((size_t)hd * 4 + (q ^ 3 ^ s)) * DH + (j ^ 1)) * DH + p * KP;
-#pragma unroll
-        for (int k = 0; k < KP; k += 4) {
-            const f32x4 v = *reinterpret_cast<const f32x4*>(own + k), w = *reinterpret_cast<const f32x4*>(oth + k);
-#pragma unroll
-            for (int e = 0; e < 4; e++) { ro[s][k + e] = v[e]; rx[s][k + e] = w[e]; }
-        }
-    }
-    const float bq = bias[((size_t)hd * 4 + q) * DH + j];
     const size_t step_wx = (size_t)4 * NH * DH, step_h = (size_t)NH * DH, step_s = (size_t)7 * NH * DH;
-    // rows that walk with the steps (uniform), and the lane's place in them
-    const unsigned at_gate = (unsigned)((q * NH + hd) * DH + j);
-    const float* wnext = wx + (size_t)b * S * step_wx;   // the row the ring takes next
-    float* srow = SAVE ? saved + (size_t)b * S * step_s : nullptr;
-    // value 4 + q of the saved state; for q = 3, h itself
-    float* out2 = q == 3 ? h + (size_t)b * S * step_h + (size_t)hd * DH + j
-                         : (SAVE ? saved + (size_t)b * S * step_s + ((size_t)(4 + q) * NH + hd) * DH + j : nullptr);
-    const size_t step2 = q == 3 ? step_h : step_s;
-    // the gate's nonlinearity: e = exp2(coef |x|) (sigmoid: of x itself)
-    const float coef = is2 ? -2.0f * 1.44269504088896340736f : -1.44269504088896340736f;
-    const unsigned sign_off = q == 3 ? 0xffffffffu : 0x7fffffffu;
-    for (int e = tid; e < 8 * KS; e += 4 * DH) hs[0][e] = 0.f;
-    const int h_at = j / KP * KS + j % KP;
-    // (the stabiliser starts at -inf rather than the paper's 0: with c_0 = n_0 = 0 it only sets the scale of the first
-    // step, and this way the first input gate is exp(0) whatever the first forget gate says)
-    float c = 0.f, n = 0.f, m = -INFINITY, hnew = 0.f, val = 0.f;
-    // Memory operations per wave and step, the same in every wave: two stores (without the saved state one: every wave has
-    // lanes with q = 3), then the ring load.
-    constexpr int OPS = SAVE ? 3 : 2;
-    const unsigned ring_base = __builtin_amdgcn_readfirstlane(mlstm::lds_offset_of(&ring[0][0]) + wave * 256);
+    for (int e = tid; e < 8 * KS; e += Cfg::THREADS) hs[0][e] = 0.f;
+    // Interval t lies between barriers t and t + 1; the walk's step t is in it.  Step t takes h_{t-1} from hs[t & 1] and leaves h_t in the other; it
+    // writes what step t - 1 keeps to stage[(t - 1) & 1] and reads its successor's input from the ring.
+    if (wave < 4 * DH / 64) {
+        const int j = tid >> 2, q = tid & 3, p = tid & 7;
+        const bool is0 = q == 0, is1 = q == 1, is2 = q == 2;
+        float ro[4][KP], rx[4][KP];   // part p of the rows of the own unit, [s: gate q ^ s], and of the octet's other one, [s: gate q ^ 3 ^ s]
 #pragma unroll
-    for (int u = 0; u < PF; u++) {   // (past the end of the sequence the last row is loaded again)
-        ring_load(wnext, 4 * at_gate, ring_base + u * (4 * DH * 4));
-        if (u + 1 < S) wnext += step_wx;
-    }
-    auto store = [&]() __attribute__((always_inline)) {   // what a step keeps, from the registers it left it in
-        if (SAVE) { *reinterpret_cast<float*>(reinterpret_cast<char*>(srow) + 4 * at_gate) = val; srow += step_s; }
-        if (SAVE || q == 3) { *out2 = pick(is0, is1, is2, c, n, m, hnew); out2 += step2; }
-    };
-    __syncthreads();
-    // One step, u = t mod PF.  wait_n: how many of the wave's memory operations may still be under way when the step's input
-    // is taken from the ring.
-    auto step = [&](int u, int t, int wait_n, bool first) __attribute__((always_inline)) {
-        const float* hcur = hs[u & 1] + p * KS;   // (PF is even: the buffers alternate across rounds too)
-        f32x4 hv[KP / 4];
+        for (int s = 0; s < 4; s++) {
+            const float* own = r + (((size_t)hd * 4 + (q ^ s)) * DH + j) * DH + p * KP;
+            const float* oth = r + (((size_t)hd * 4 + (q ^ 3 ^ s)) * DH + (j ^ 1)) * DH + p * KP;
 #pragma unroll
-        for (int k = 0; k < KP / 4; k++) hv[k] = *reinterpret_cast<const f32x4*>(hcur + 4 * k);
-        __builtin_amdgcn_sched_barrier(0);
-        if (!first) {   // the step before: its results go out, and its ring slot takes the row PF steps on
-            store();
-            ring_load(wnext, 4 * at_gate, ring_base + ((u + PF - 1) % PF) * (4 * DH * 4));
-            if (t + PF < S) wnext += step_wx;
+            for (int k = 0; k < KP; k += 4) {
+                const f32x4 v = *reinterpret_cast<const f32x4*>(own + k), w = *reinterpret_cast<const f32x4*>(oth + k);
+#pragma unroll
+                for (int e = 0; e < 4; e++) { ro[s][k + e] = v[e]; rx[s][k + e] = w[e]; }
+            }
         }
-        ring_wait(wait_n);
-        const float wv = ring[u][tid];   // (its own wave's load)
-        __builtin_amdgcn_sched_barrier(0);
-        float a[4] = {0.f, 0.f, 0.f, 0.f}, x4[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int k = 0; k < KP / 4; k++)
-#pragma unroll
-            for (int e = 0; e < 4; e++)
-#pragma unroll
-                for (int s = 0; s < 4; s++) {
-                    a[s] += ro[s][4 * k + e] * hv[k][e];
-                    x4[s] += rx[s][4 * k + e] * hv[k][e];
-                }
-        // own unit: what the octet's mirror lane (7 - p, of gate q ^ 3) has of it, then gate q from lanes q, q ^ 1, q ^ 2, q ^ 3
-#pragma unroll
-        for (int s = 0; s < 4; s++) a[s] += quad_perm<0x141>(x4[s]);   // row_half_mirror
-        const float x = ((a[0] + quad_perm<0xB1>(a[1])) + (quad_perm<0x4E>(a[2]) + quad_perm<0x1B>(a[3]))) + (wv + bq);
-        const float e = __builtin_amdgcn_exp2f(coef * __builtin_bit_cast(float, __builtin_bit_cast(unsigned, x) & sign_off));
-        const float d = 1.0f + e, rd = fast_rcp(d);
-        const float th = __builtin_copysignf((1.0f - e) * rd, x);                                             // tanh
-        const float ls = FS ? fminf(x, 0.0f) - __builtin_amdgcn_logf(d) * 0.69314718055994530942f : x;        // log sigmoid
-        val = pick(is0, is1, is2, x, ls, th, rd);   // i~, log f, z, o
-        const float it = quad_perm<0x00>(val), logf = quad_perm<0x55>(val), z = quad_perm<0xAA>(val), o = quad_perm<0xFF>(val);
-        const float fm = logf + m, mn = fmaxf(fm, it);
-        const float ip = fast_exp(it - mn), fp = fast_exp(fm - mn);
-        n = fp * n + ip;
-        c = fp * c + ip * z;
-        m = mn;
-        hnew = o * c * fast_rcp(n);
-        hs[(u & 1) ^ 1][h_at] = hnew;   // (the quad's four lanes write the same bits)
+        const float bq = bias[((size_t)hd * 4 + q) * DH + j];
+        // the gate's nonlinearity: e = exp2(coef |x|) (sigmoid: of x itself)
+        const float coef = is2 ? -2.0f * 1.44269504088896340736f : -1.44269504088896340736f;
+        const unsigned sign_off = q == 3 ? 0xffffffffu : 0x7fffffffu;
+        const int h_at = j / KP * KS + j % KP, in_at = (j >> 2) * 16 + q * 4 + (j & 3), keep_at = q * SR + j;
+        // (the stabiliser starts at -inf rather than the paper's 0: with c_0 = n_0 = 0 it only sets the scale of the first
+        // step, and this way the first input gate is exp(0) whatever the first forget gate says)
+        float c = 0.f, n = 0.f, m = -INFINITY, val = 0.f;
+        auto keep = [&](int slot) __attribute__((always_inline)) {   // what a step keeps, from the registers it left it in
+            if constexpr (SAVE) {
+                stage[slot][keep_at] = val;
+                stage[slot][keep_at + 4 * SR] = pick(is0, is1, true, c, n, m, m);
+            }
+        };
         __syncthreads();
-    };
-    // The ring load of row t >= PF was issued in step t - PF + 1, as the last of its operations: when step t asks for it, the
-    // OPS operations of each of the PF - 1 steps since are younger (the wait allows one step's fewer).  The rows before come
-    // from the prologue, with the later slots' loads behind them and the operations of steps 1 .. t (one step's fewer again).
+        float wv = ring[0][in_at];
+        auto step = [&](int u) __attribute__((always_inline)) {   // u = t mod PF
+            const float* hcur = hs[u & 1] + p * KS;   // (PF is even: the buffers alternate across rounds too)
+            constexpr int AHEAD = KP / 4 < 4 ? KP / 4 : 2;   // (reads under way: DH = 128 has registers for no more)
+            f32x4 hv[KP / 4];
 #pragma unroll
-    for (int u = 0; u < PF; u++)
-        if (u < S) step(u, u, PF - 1 - u + (u > 0 ? OPS * (u - 1) : 0), u == 0);
-    for (int t0 = PF; t0 < S; t0 += PF) {
+            for (int k = 0; k < AHEAD; k++) hv[k] = *reinterpret_cast<const f32x4*>(hcur + 4 * k);
+            __builtin_amdgcn_sched_barrier(0);
+            keep((u & 1) ^ 1);   // (at t = 0 nothing that is read)
+            const float in = wv + bq;
+            wv = ring[(u + 1) % PF][in_at];
+            __builtin_amdgcn_sched_barrier(0);
+            float a[4] = {0.f, 0.f, 0.f, 0.f}, x4[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int u = 0; u < PF; u++)
-            if (t0 + u < S) step(u, t0 + u, OPS * (PF - 2), false);
+            for (int k = 0; k < KP / 4; k++) {
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+#pragma unroll
+                    for (int s = 0; s < 4; s++) {
+                        a[s] += ro[s][4 * k + e] * hv[k][e];
+                        x4[s] += rx[s][4 * k + e] * hv[k][e];
+                    }
+                if (k + AHEAD < KP / 4) {   // (the sums so far are formed before the next read is issued)
+                    asm volatile("" : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(x4[0]), "+v"(x4[1]), "+v"(x4[2]), "+v"(x4[3]));
+                    __builtin_amdgcn_sched_barrier(0);
+                    hv[k + AHEAD] = *reinterpret_cast<const f32x4*>(hcur + 4 * (k + AHEAD));
+                }
+            }
+            // own unit: what the octet's mirror lane (7 - p, of gate q ^ 3) has of it, then gate q from lanes q, q ^ 1, q ^ 2, q ^ 3
+#pragma unroll
+            for (int s = 0; s < 4; s++) a[s] += quad_perm<0x141>(x4[s]);   // row_half_mirror
+            const float x = ((a[0] + quad_perm<0xB1>(a[1])) + (quad_perm<0x4E>(a[2]) + quad_perm<0x1B>(a[3]))) + in;
+            const float e = __builtin_amdgcn_exp2f(coef * __builtin_bit_cast(float, __builtin_bit_cast(unsigned, x) & sign_off));
+            const float d = 1.0f + e, rd = fast_rcp(d);
+            const float th = __builtin_copysignf((1.0f - e) * rd, x);                                             // tanh
+            const float ls = FS ? fminf(x, 0.0f) - __builtin_amdgcn_logf(d) * 0.69314718055994530942f : x;        // log sigmoid
+            val = pick(is0, is1, is2, x, ls, th, rd);   // i~, log f, z, o
+            const float it = quad_perm<0x00>(val), logf = quad_perm<0x55>(val), z = quad_perm<0xAA>(val), o = quad_perm<0xFF>(val);
+            const float fm = logf + m, mn = fmaxf(fm, it);
+            const float ip = fast_exp(it - mn), fp = fast_exp(fm - mn);
+            n = fp * n + ip;
+            c = fp * c + ip * z;
+            m = mn;
+            hs[(u & 1) ^ 1][h_at] = o * c * fast_rcp(n);   // (the quad's four lanes write the same bits)
+            __syncthreads();
+        };
+        int t = 0;
+        for (; t + PF <= S; t += PF) {
+#pragma unroll
+            for (int u = 0; u < PF; u++) step(u);
+        }
+#pragma unroll
+        for (int u = 0; u < PF - 1; u++)
+            if (t + u < S) step(u);
+        keep((S - 1) & 1);
+        __syncthreads();
+        return;
     }
-    store();
+    // ---- helpers.  In interval t they request input row t + PF, write out h_{t-1} and what step t - 2 keeps, and wait for row t + 2.
+    const int hl = tid - 4 * DH, hwave = wave - 4 * DH / 64;
+    // Input: piece hl of a row's 4 DH floats is gate hl % 4 of units 4 (hl / 4) ..; without 16-byte boundaries a load brings a float of 64 places.
+    constexpr int LOADS = WIDE ? 1 : (4 * DH / Cfg::UW) / 64;
+    unsigned in_off[LOADS];
+#pragma unroll
+    for (int i = 0; i < LOADS; i++) {
+        const int piece = WIDE ? hl : 64 * hwave + (64 * i + lane) / 4, e = WIDE ? 0 : lane & 3;
+        in_off[i] = 4u * (unsigned)(((piece & 3) * NH + hd) * DH + 4 * (piece >> 2) + e);
+    }
+    const float* wnext = wx + (size_t)b * S * step_wx;   // the row that is requested next (past the end of the sequence the last one again)
+    const unsigned ring_base = __builtin_amdgcn_readfirstlane(mlstm::lds_offset_of(&ring[0][0]) + hwave * 1024);
+    int row = 0;
+    auto request = [&](int slot) __attribute__((always_inline)) {
+        const unsigned at = ring_base + slot * (4 * DH * 4);
+        if constexpr (WIDE) {
+            if (hl < DH)
+                asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(in_off[0]), "s"(wnext), "s"(at) : "memory", "m0");
+        } else {
+#pragma unroll
+            for (int i = 0; i < LOADS; i++) ring_load(wnext, in_off[i], at + 256 * i);
+        }
+        if (++row < S) wnext += step_wx;
+    };
+    // Output: 16-byte pieces of the seven rows of the saved state, then of h
+    constexpr int PIECES = SAVE ? 2 * DH / (64 * Cfg::UW) : 1, PR = DH / 4;
+    const float *from[PIECES], *next[PIECES];   // (of this interval's buffer and of the other)
+    char* to[PIECES];
+    size_t stride[PIECES];
+    bool is_h[PIECES];
+#pragma unroll
+    for (int i = 0; i < PIECES; i++) {
+        const int piece = hl + 64 * Cfg::UW * i, v = SAVE ? piece / PR : 7, u4 = 4 * (piece % PR);
+        is_h[i] = v == 7;
+        if (SAVE && v < 7) {
+            from[i] = &stage[0][v * SR + u4];
+            next[i] = &stage[SAVE ? 1 : 0][v * SR + u4];
+            to[i] = reinterpret_cast<char*>(saved + (size_t)b * S * step_s + ((size_t)v * NH + hd) * DH + u4);
+            stride[i] = step_s * 4;
+        } else {
+            from[i] = &hs[0][u4 / KP * KS + u4 % KP];
+            next[i] = &hs[1][u4 / KP * KS + u4 % KP];
+            to[i] = reinterpret_cast<char*>(h + (size_t)b * S * step_h + (size_t)hd * DH + u4);
+            stride[i] = step_h * 4;
+        }
+    }
+    auto put_out = [&](bool with_state, bool with_h) __attribute__((always_inline)) {   // (once per interval)
+#pragma unroll
+        for (int i = 0; i < PIECES; i++) {
+            if ((is_h[i] ? with_h : with_state) && (SAVE || hl < PR)) {
+                const f32x4 v = *reinterpret_cast<const f32x4*>(from[i]);
+                if constexpr (WIDE) *reinterpret_cast<f32x4*>(to[i]) = v;
+                else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) reinterpret_cast<float*>(to[i])[e] = v[e];
+                }
+                to[i] += stride[i];
+            }
+            const float* const now = from[i];
+            from[i] = next[i];
+            next[i] = now;
+        }
+    };
+#pragma unroll 1
+    for (int u = 0; u < PF; u++) request(u);
+    ring_wait(0);
+    __syncthreads();
+    // Rows PF on: row t + 2 was requested in interval t + 2 - PF, and the PF - 2 intervals since have a request each and, from interval 2 on, the stores
+    // (without the saved state those of h, of the first helper wave alone): one interval fewer is waited for.
+    constexpr int STORES = (WIDE ? 1 : 4) * PIECES, OPS = LOADS + STORES;
+    auto wait = [&]() __attribute__((always_inline)) {
+        if (SAVE || hwave == 0) mlstm::dma_wait_but<((PF - 3) * OPS < 63 ? (PF - 3) * OPS : 63)>();
+        else mlstm::dma_wait_but<((PF - 3) * LOADS < 63 ? (PF - 3) * LOADS : 63)>();
+    };
+    int t = 0;
+    for (; t < 2 && t < S; t++) {
+        request(t);
+        put_out(false, t > 0);
+        wait();
+        __syncthreads();
+    }
+    for (int slot = t; t < S; t++) {
+        put_out(true, true);
+        request(slot);
+        slot = (slot + 1) % PF;
+        wait();
+        __syncthreads();
+    }
+    put_out(S > 1, true);
+    __syncthreads();
+    put_out(true, false);
 }
 
 // Back through time with the same quads, but what step t + 1 sends back to h_t -- R^T delta_{t+1}, a vector of 4 DH gradients
@@ -627,9 +717,14 @@ int slices_for(int B, int NH, int S) {
 // (the step kernels count their waits for the input ring by hand: see no_scratch_once)
 template <int DH, bool SAVE, bool FS>
 int forward_launch(const float* wx, const float* r, const float* b, float* h, float* saved, int B, int NH, int S, hipStream_t st) {
-    if (int rc = mlstm::no_scratch_once<slstm_forward_kernel<DH, SAVE, FS>>()) return rc;
-    hipLaunchKernelGGL((slstm_forward_kernel<DH, SAVE, FS>), dim3(B * NH), dim3(4 * DH), 0, st, wx, r, b, h, saved, NH, S);
-    return (int)hipGetLastError();
+    auto launch = [&](auto wide) {
+        constexpr auto kernel = slstm_forward_kernel<DH, SAVE, FS, decltype(wide)::value>;
+        if (int rc = mlstm::no_scratch_once<kernel>()) return rc;
+        hipLaunchKernelGGL(kernel, dim3(B * NH), dim3(FwdCfg<DH>::THREADS), 0, st, wx, r, b, h, saved, NH, S);
+        return (int)hipGetLastError();
+    };
+    const size_t at = reinterpret_cast<size_t>(wx) | reinterpret_cast<size_t>(h) | reinterpret_cast<size_t>(saved);
+    return at & 15 ? launch(std::false_type{}) : launch(std::true_type{});
 }
 
 template <int DH>
