@@ -37,18 +37,36 @@ __device__ __forceinline__ f32x16 mma_f32(float a, float b, f32x16 c) { return _
 // fetches its quarter of the head dimension in blocks of FBW columns with whole 128-byte lines per row (four blocks in
 // flight), passes them through a piece of LDS of its own (rows padded by four floats: conflict-free both ways) and reads
 // the operands from there.
+// Shared partial numerators start from zero: two key ranges add to each element, and 0 + a + b is the same number in either
+// order, so results do not depend on which comes first.  Workgroups behind those of the chunks write the zeros (SCAN_ZERO_WG floats each),
+// beside their loads and not in a pass of its own.  Whole call, us, a pass of its own / beside: forward 4 heads x 2048 x 1024 318 / 312, 16 x 1024 x 512
+// 180 / 175, 4 x 64 x 1024 34.0 / 32.5; forward + backward 2 x 2048 x 1024 908 / 888, 40 x 2048 x 256 1989 / 1976.
+constexpr int SCAN_ZERO_WG = 16384;
+__device__ __forceinline__ void scan_zeros(float* h, float* hpart, size_t n, size_t total, int wg) {
+#pragma unroll 4
+    for (int i = 0; i < SCAN_ZERO_WG / 1024; i++) {
+        const size_t e = (size_t)wg * SCAN_ZERO_WG + 1024 * i + 4 * threadIdx.x;
+        if (e < total) *reinterpret_cast<f32x4*>(e < n ? h + e : hpart + (e - n)) = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+}
 template <int D>
-__global__ __launch_bounds__(256) void scan_intra_kernel(ScanArgs a) {
+__global__ __launch_bounds__(256) void scan_intra_kernel(ScanArgs a, int parts) {
     constexpr int DW = D / 4, FBW = DW < 32 ? DW : 32, NB = DW / FBW;   // columns per wave, per block; blocks
     constexpr int LPR = FBW / 4, RPI = 64 / LPR, NLD = LPR;             // lanes per row, rows per load instruction, loads per block
     constexpr int LST = FBW + 4, PD = NB < 4 ? NB : 4;                  // LDS row stride (floats); blocks in flight
     __shared__ __align__(16) float stage[4][64 * LST];                  // per wave: 32 rows of q, then 32 rows of k
     static_assert(64 * LST >= 16 * 64, "the partial sums reuse a wave's stage");
     auto red_at = [&](int w, int r, int l) -> float& { return stage[w][r * 64 + l]; };
+    const int wgs = a.BH * a.NC * 4;
+    if ((int)blockIdx.x >= wgs) {
+        const size_t n = (size_t)a.BH * a.S * D;
+        scan_zeros(a.h, a.hpart, n, n * parts, blockIdx.x - wgs);
+        return;
+    }
     // Consecutive workgroups go to the eight XCDs in turn; the four roles of a chunk read the same rows of q and k, so
     // they take workgroups of one XCD (eight apart), which share an L2.
     int role, cidx;
-    if ((gridDim.x & 31) == 0) {
+    if ((wgs & 31) == 0) {
         const int xcd = blockIdx.x & 7, r = blockIdx.x >> 3;
         role = r & 3; cidx = (r >> 2) * 8 + xcd;
     } else {
@@ -588,13 +606,6 @@ __global__ __launch_bounds__(SCAN_NW * 64) void scan_state_kernel(ScanArgs a) {
     }
 }
 
-// Shared partial numerators start from zero.  Two key ranges add to each element, and 0 + a + b is the same number in either
-// order, so results do not depend on which comes first.
-__global__ __launch_bounds__(256) void scan_zero_kernel(float* h, float* hpart, size_t n4, int parts) {
-    for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < n4 * parts; e += (size_t)gridDim.x * 256)
-        *reinterpret_cast<f32x4*>((e < n4 ? h : hpart) + 4 * (e < n4 ? e : e - n4)) = f32x4{0.f, 0.f, 0.f, 0.f};
-}
-
 // States at the segment ends from the segments' own sums, in place: x_s = exp(A_{e(s-1)} - A_{e(s)}) x_{s-1} + x_s with
 // e(s) the last position of segment s.  One thread per state element; elems = floats per segment, wg_elems = floats per
 // workgroup of the state kernel (whose index modulo BH is the head).
@@ -795,15 +806,12 @@ static ScanTile scan_tile(int BH, int D) {
 template <int D>
 static int launch_scan_d(const ScanArgs& a, int parts, hipStream_t st, void (*mark)(int, hipStream_t, bool)) {
     mark(MLSTM_K_SCAN_CARRY, st, true);
-    hipLaunchKernelGGL(scan_intra_kernel<D>, dim3(a.BH * a.NC * 4), dim3(256), 0, st, a);
+    const size_t zeros = a.shared ? (size_t)a.BH * a.S * D * parts : 0;
+    hipLaunchKernelGGL(scan_intra_kernel<D>, dim3(a.BH * a.NC * 4 + (unsigned)((zeros + SCAN_ZERO_WG - 1) / SCAN_ZERO_WG)), dim3(256), 0, st, a, parts);
     if (a.finish_mode != 2 || a.ep.vec) hipLaunchKernelGGL(scan_ncarry_kernel, dim3((D + 255) / 256, a.BH), dim3(256), 0, st, a);
     mark(MLSTM_K_SCAN_CARRY, st, false);
     mark(MLSTM_K_SCAN_STATE, st, true);
     const ScanTile tile = scan_tile(a.BH, D);
-    if (a.shared) {
-        const size_t n4 = (size_t)a.BH * a.S * D / 4, want = (n4 * parts + 255) / 256;
-        hipLaunchKernelGGL(scan_zero_kernel, dim3((unsigned)(want < 8192 ? want : 8192)), dim3(256), 0, st, a.h, a.hpart, n4, parts);
-    }
     if (tile.nkb == 2) launch_state_r<D, 2, 2>(a, st);
     else if (tile.vb == 2) launch_state_r<D, 2, 1>(a, st);
     else launch_state_r<D, 1, 1>(a, st);
@@ -822,8 +830,8 @@ void launch_scan_ncarry(const ScanArgs& a, hipStream_t st) {
 
 // Key ranges per value tile.  A walk with 64 value columns per workgroup has twice the key ranges that one with 32 would have; pairs
 // of them share a partial numerator, so that the workspace does not grow with them (in tensors beside the output: D = 1024 from 4
-// heads on one instead of three, D = 512 from 16 heads on none instead of one).  It costs a pass that writes zeros and adds in place of
-// stores, in us apart / shared: forward 4 heads x 2048 x 1024 306 / 311, 2 x 2048 x 1024 210 / 224, 16 x 1024 x 512 172 / 178,
+// heads on one instead of three, D = 512 from 16 heads on none instead of one).  It costs zeros and adds in place of stores, in us apart / shared
+// with the zeros in a pass of their own (now 1 to 3 % less, see scan_zeros): forward 4 heads x 2048 x 1024 306 / 311, 2 x 2048 x 1024 210 / 224, 16 x 1024 x 512 172 / 178,
 // 8 x 1024 x 512 118 / 129, 40 x 2048 x 256 456 / 474; forward + backward 2 x 2048 x 1024 868 / 905, 8 x 1024 x 512 482 / 521,
 // 40 x 2048 x 256 1902 / 2001.
 bool scan_can_share(int BH, int D) { return scan_tile(BH, D).vb == 2 && scan_key_splits(BH, D) >= 2; }
