@@ -195,3 +195,20 @@ def test_forward_at_every_turn_of_the_helpers(S, DH):
         h2, saved2 = slstm_forward_hip(other, r.cuda(), b.cuda(), forget_sigmoid=True)
         h3, _ = slstm_forward_hip(other, r.cuda(), b.cuda(), forget_sigmoid=True, save=False)
         assert torch.equal(h2, h) and torch.equal(saved2, saved) and torch.equal(h3, h)
+
+
+@pytest.mark.parametrize("DH", [32, 64, 128])
+@pytest.mark.parametrize("B,NH,S", [(40, 2, 15), (21, 1, 16), (18, 3, 17), (5, 4, 333), (2, 1, 1000)])
+def test_recurrent_gradients_over_slices(B, NH, S, DH):
+    # dR and db from dWx and h, sixteen pairs of (sequence, step) at a time: rounds inside a sequence, across the start of one, at the end of a
+    # slice, sequences shorter than a round.  Products of three bf16 terms keep 24 bits, sums are fp32 over at most B S terms in chains of 1/8 of a slice.
+    from slstm import slstm_backward_hip, slstm_forward_hip
+    wx, r, b, dh = SO.make_inputs(B, NH, S, DH, seed=B + DH, f_mean=1.0)
+    h, saved = slstm_forward_hip(*gpu(wx, r, b), forget_sigmoid=True)
+    dwx, dr, db = slstm_backward_hip(dh.cuda(), h, r.cuda(), saved, forget_sigmoid=True)
+    d, prev = dwx.double().cpu(), torch.nn.functional.pad(h.double().cpu(), (0, 0, 0, 0, 1, 0))[:, :-1]
+    d2, p2 = d.permute(3, 2, 4, 0, 1).reshape(NH, 4, DH, B * S), prev.permute(2, 3, 0, 1).reshape(NH, 1, DH, B * S)
+    size = d2.abs() @ p2.abs().transpose(-1, -2).contiguous()
+    bound = 2.0 ** -24 * (B * S) ** 0.5 * 4
+    assert bool(((dr.double().cpu() - d2 @ p2.transpose(-1, -2).contiguous()).abs() <= bound * size + 1e-30).all())
+    assert bool(((db.double().cpu() - d2.sum(-1)).abs() <= bound * d2.abs().sum(-1) + 1e-30).all())

@@ -561,17 +561,19 @@ __global__ __launch_bounds__(BwdCfg<DH>::THREADS) void slstm_backward_kernel(con
     if ((S - g) % NGRP == NGRP - 1 || (S < g && S == g - 1)) store(S - 1);
 }
 
-constexpr int dr_parts(int DH) { return DH <= 64 ? 4 : 1; }   // partial sums per slice (slstm_dr_kernel's PARTS)
+constexpr int dr_parts(int DH) { return DH <= 64 ? 4 : 1; }   // waves that share a slice's pairs (slstm_dr_kernel's PARTS)
+constexpr int dr_lds(int DH) { return DH <= 64 ? 4 * (DH * DH + DH) * (int)sizeof(float) : 0; }
 // dR[h][g][j][k] and db[h][g][j] over one slice of the (b, t) pairs, on the matrix units: per head and gate this is the
 // product of dWx[g] ([pairs] x DH, taken transposed) with h_{t-1} ([pairs] x DH), the pairs being the inner dimension.
 // Every fp32 operand is three bf16 terms (mlstm::Tr<float>: 24 significant bits); a lane holds row or column l % 32 at eight
 // successive pairs, 8 (l / 32) + e of a round's sixteen, so both
 // come straight from global memory, one dword per lane, rows of 128 bytes; nothing passes through LDS.  One workgroup per
 // (head, gate, slice), four waves: up to DH = 64 every wave forms the whole DH x DH block over a quarter of the slice's
-// pairs (chunks of 16, taken in turns) and leaves it as a partial sum of its own; at DH = 128 every wave forms one 64 x 64
+// pairs (chunks of 16, taken in turns), and the four add up in LDS, a quarter of the block each; at DH = 128 every wave forms one 64 x 64
 // quadrant over all the pairs.
-// B16 NH4 S2048 DH64: 70 us on v_mfma_f32_32x32x2_f32, bound by its 512 cycles per 32 x 32 x 16 block; 53 now (192, and the splits),
-// 134 MB of dWx and four readings of h (by gate, 34 MB each out of the caches).
+// B16 NH4 S2048 DH64: 70 us on v_mfma_f32_32x32x2_f32, bound by its 512 cycles per 32 x 32 x 16 block; 57 on three bf16 terms (192, and the splits),
+// with 33 MB of partial sums, one per wave, and a place in the sequence looked up and tested for every load; 46 now that only rounds that meet the start of a
+// sequence or the end of the slice do that, and the others load from uniform rows: 134 MB of dWx and four readings of h (by gate, 34 MB each out of the caches).
 template <int DH>
 __global__ __launch_bounds__(256, 2) void slstm_dr_kernel(const float* __restrict__ dwx, const float* __restrict__ h, float* __restrict__ part_r,
                                                        float* __restrict__ part_b, int B, int NH, int S, int nslice) {
@@ -582,15 +584,16 @@ __global__ __launch_bounds__(256, 2) void slstm_dr_kernel(const float* __restric
     constexpr int U = 8, CH = 2 * U;        // pairs per lane and round, pairs per round
     typedef mlstm::Tr<float> X;
     const int hg = blockIdx.x, hd = hg / 4, g = hg % 4, slice = blockIdx.y;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l32 = lane & 31, hh = lane >> 5;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l32 = lane & 31, hh = lane >> 5;
     const int part = PARTS > 1 ? wave : 0, quad = PARTS > 1 ? 0 : wave;
     const int j0 = (quad >> 1) * 64, k0 = (quad & 1) * 64;   // the block's corner
     const long long total = (long long)B * S, per = (total + nslice - 1) / nslice;
     const long long lo = slice * per, hi = lo + per < total ? lo + per : total;
     const size_t step_wx = (size_t)4 * NH * DH, step_h = (size_t)NH * DH;
-    // (a lane's place inside a pair of rows, as one 32-bit offset: the rows' own addresses are the same for the whole wave)
-    const unsigned la = (unsigned)(U * hh * step_wx + ((size_t)g * NH + hd) * DH + j0 + l32);
-    const unsigned lb = (unsigned)(U * hh * step_h + (size_t)hd * DH + k0 + l32);
+    // (a lane's place inside a pair of rows, as one 32-bit offset in bytes: the rows' own addresses are the same for the whole wave)
+    const unsigned la = 4u * (unsigned)(U * hh * step_wx + ((size_t)g * NH + hd) * DH + j0 + l32);
+    const unsigned lb = 4u * (unsigned)(U * hh * step_h + (size_t)hd * DH + k0 + l32);
+    auto at = [](const float* row, unsigned off) __attribute__((always_inline)) { return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(row) + off); };
     f32x16 acc[T][T];
     float bsum[T];
 #pragma unroll
@@ -602,25 +605,35 @@ __global__ __launch_bounds__(256, 2) void slstm_dr_kernel(const float* __restric
             for (int e = 0; e < 16; e++) acc[x][y][e] = 0.f;
     }
     X::frag a[2][T], bv[2][T];
-    // the operands of the round that starts at pair p0 (this lane's first pair: p0 + 8 hh, t0 steps into its sequence)
+    // the operands of the round that starts at pair p0, t0 steps into its sequence (this lane's first pair: 8 hh on)
     auto load = [&](int set, long long p0, int t0) __attribute__((always_inline)) {
+        const float* const ra = dwx + p0 * (long long)step_wx;
+        const float* const rb = h + (p0 - 1) * (long long)step_h;
+        if (p0 + CH <= hi && t0 > 0 && t0 + CH <= S) {
+#pragma unroll
+            for (int e = 0; e < U; e++)
+#pragma unroll
+                for (int x = 0; x < T; x++) {
+                    a[set][x][e] = at(ra + e * step_wx + 32 * x, la);
+                    bv[set][x][e] = at(rb + e * step_h + 32 * x, lb);
+                }
+            return;
+        }
 #pragma unroll
         for (int e = 0; e < U; e++) {
             const long long pp = p0 + U * hh + e;
-            int t = t0 + e;
+            int t = t0 + U * hh + e;
             if (t >= S) t %= S;
             const bool in = pp < hi, prev = in && t != 0;   // (h_{-1} = 0: the first step of a sequence adds nothing to dR)
-            const float* ra = dwx + (p0 + e) * (long long)step_wx;
-            const float* rb = h + (p0 + e - 1) * (long long)step_h;
 #pragma unroll
             for (int x = 0; x < T; x++) {
-                a[set][x][e] = in ? ra[la + 32 * x] : 0.f;
-                bv[set][x][e] = prev ? rb[lb + 32 * x] : 0.f;
+                a[set][x][e] = in ? at(ra + e * step_wx + 32 * x, la) : 0.f;
+                bv[set][x][e] = prev ? at(rb + e * step_h + 32 * x, lb) : 0.f;
             }
         }
     };
     long long p0 = lo + (long long)part * CH;
-    int t0 = (int)((p0 + U * hh) % S);
+    int t0 = (int)(p0 % S);
     if (p0 < hi) load(0, p0, t0);
     // one round on operand set `set` (a constant at each call); the next round's operands are under way while it multiplies
     auto round = [&](int set) __attribute__((always_inline)) {
@@ -652,49 +665,87 @@ __global__ __launch_bounds__(256, 2) void slstm_dr_kernel(const float* __restric
 #pragma unroll
     for (int x = 0; x < T; x++) bsum[x] += __shfl_xor(bsum[x], 32);
     // accumulator register e of a lane: column l % 32, row 8 (e / 4) + 4 (l / 32) + e % 4 of its tile
-    // (every wave's partial sum is a slice of its own for the kernel that adds the slices)
-    const size_t sl = (size_t)slice * PARTS + part;
-    float* out = part_r + ((sl * NH * 4 + hg) * DH) * DH;
-    float seen = 0.f;
-#pragma unroll
-    for (int x = 0; x < T; x++)
-#pragma unroll
-        for (int y = 0; y < T; y++)
-#pragma unroll
-            for (int e = 0; e < 16; e++) seen = mlstm::not_finite(seen, acc[x][y][e]);
-    if (__any(seen != 0.f)) {   // a block that is not finite, in fp32 multiply-adds straight from memory (see not_finite in mlstm_device.h)
+    float* const out = part_r + (((size_t)slice * NH * 4 + hg) * DH) * DH;
+    float* const out_b = part_b + ((size_t)slice * NH * 4 + hg) * DH;
+    // an element that is not finite, in fp32 multiply-adds straight from memory (see not_finite in mlstm_device.h)
+    auto exact = [&](int j, int k) {
+        float sum = 0.f;
 #pragma unroll 1
-        for (int n = lane; n < W * W; n += 64) {
-            const int j = j0 + n / W, k = k0 + n % W;
-            float sum = 0.f;
-#pragma unroll 1
-            for (long long c0 = lo + (long long)part * CH; c0 < hi; c0 += (long long)PARTS * CH)
-#pragma unroll 1
-                for (long long pp = c0; pp < c0 + CH && pp < hi; pp++)
-                    if (pp % S != 0) sum += dwx[pp * step_wx + ((size_t)g * NH + hd) * DH + j] * h[(pp - 1) * step_h + (size_t)hd * DH + k];
-            out[(size_t)j * DH + k] = sum;
+        for (long long pp = lo; pp < hi; pp++)
+            if (pp % S != 0) sum += dwx[pp * step_wx + ((size_t)g * NH + hd) * DH + j] * h[(pp - 1) * step_h + (size_t)hd * DH + k];
+        return sum;
+    };
+    if constexpr (PARTS > 1) {
+        constexpr int Q = T * T * 4, QW = Q / PARTS;   // groups of four registers, of those a wave's to add up
+        extern __shared__ __attribute__((aligned(16))) f32x4 sums[];   // [wave][group][lane], then [wave][row]: sums of dWx
+        float* const sums_b = reinterpret_cast<float*>(sums + PARTS * Q * 64);
+#pragma unroll
+        for (int q = 0; q < Q; q++) {
+            const f32x16& v = acc[q / 4 / T][q / 4 % T];
+            const int e = 4 * (q % 4);
+            sums[(wave * Q + q) * 64 + lane] = f32x4{v[e], v[e + 1], v[e + 2], v[e + 3]};
         }
+        if (hh == 0) {
+#pragma unroll
+            for (int x = 0; x < T; x++) sums_b[wave * DH + 32 * x + l32] = bsum[x];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int n = 0; n < QW; n++) {
+            const int q = wave * QW + n, j = 32 * (q / 4 / T) + 8 * (q % 4) + 4 * hh, k = 32 * (q / 4 % T) + l32;
+            const f32x4* const from = sums + q * 64 + lane;
+            f32x4 v = (from[0] + from[Q * 64]) + (from[2 * Q * 64] + from[3 * Q * 64]);
+            float seen = 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; e++) seen = mlstm::not_finite(seen, v[e]);
+            if (__any(seen != 0.f)) {
+#pragma unroll 1
+                for (int e = 0; e < 4; e++) out[(size_t)(j + e) * DH + k] = exact(j + e, k);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; e++) out[(size_t)(j + e) * DH + k] = v[e];
+            }
+        }
+        if ((int)threadIdx.x < DH)
+            out_b[threadIdx.x] = (sums_b[threadIdx.x] + sums_b[DH + threadIdx.x]) + (sums_b[2 * DH + threadIdx.x] + sums_b[3 * DH + threadIdx.x]);
     } else {
+        float seen = 0.f;
 #pragma unroll
         for (int x = 0; x < T; x++)
 #pragma unroll
             for (int y = 0; y < T; y++)
 #pragma unroll
-                for (int e = 0; e < 16; e++)
-                    out[(size_t)(j0 + 32 * x + 8 * (e / 4) + 4 * hh + e % 4) * DH + k0 + 32 * y + l32] = acc[x][y][e];
-    }
-    if (k0 == 0 && hh == 0) {
+                for (int e = 0; e < 16; e++) seen = mlstm::not_finite(seen, acc[x][y][e]);
+        if (__any(seen != 0.f)) {
+#pragma unroll 1
+            for (int n = lane; n < W * W; n += 64) out[(size_t)(j0 + n / W) * DH + k0 + n % W] = exact(j0 + n / W, k0 + n % W);
+        } else {
 #pragma unroll
-        for (int x = 0; x < T; x++) part_b[(sl * NH * 4 + hg) * DH + j0 + 32 * x + l32] = bsum[x];
+            for (int x = 0; x < T; x++)
+#pragma unroll
+                for (int y = 0; y < T; y++)
+#pragma unroll
+                    for (int e = 0; e < 16; e++)
+                        out[(size_t)(j0 + 32 * x + 8 * (e / 4) + 4 * hh + e % 4) * DH + k0 + 32 * y + l32] = acc[x][y][e];
+        }
+        if (k0 == 0 && hh == 0) {
+#pragma unroll
+            for (int x = 0; x < T; x++) out_b[j0 + 32 * x + l32] = bsum[x];
+        }
     }
 }
 
 // out[e] = sum over the partial sums, in a fixed order: 64 elements per workgroup, four threads per element with every
-// fourth partial sum each, their four sums added in order.
-__global__ __launch_bounds__(256) void slstm_reduce_kernel(const float* __restrict__ part, float* __restrict__ out, size_t n, int nslice) {
+// fourth partial sum each, their four sums added in order.  The workgroups behind those of dR add up db (a launch of its own: 7 us).
+struct Reduce { const float* part; float* out; size_t n; };
+__global__ __launch_bounds__(256) void slstm_reduce_kernel(Reduce r, Reduce b, int nslice) {
     __shared__ float red[4][64];
     const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
-    const size_t e = (size_t)blockIdx.x * 64 + x;
+    const size_t wgs = (r.n + 63) / 64;
+    const bool first = blockIdx.x < wgs;
+    const float* const part = first ? r.part : b.part;
+    float* const out = first ? r.out : b.out;
+    const size_t n = first ? r.n : b.n, e = (size_t)(first ? blockIdx.x : blockIdx.x - wgs) * 64 + x;
     float s0 = 0.f, s1 = 0.f;
     if (e < n) {
         int i = y;
@@ -754,11 +805,11 @@ int backward_t(const float* dh, const float* h, const float* r, const float* sav
     const int ns = slices_for(B, NH, S);
     const size_t nr = (size_t)NH * 4 * DH * DH, nb = (size_t)NH * 4 * DH;
     float* part_r = reinterpret_cast<float*>(ws);
-    const int np = ns * dr_parts(DH);   // partial sums to add
-    float* part_b = part_r + (size_t)np * nr;
-    hipLaunchKernelGGL(slstm_dr_kernel<DH>, dim3(NH * 4, ns), dim3(256), 0, st, dwx, h, part_r, part_b, B, NH, S, ns);
-    hipLaunchKernelGGL(slstm_reduce_kernel, dim3((unsigned)((nr + 63) / 64)), dim3(256), 0, st, part_r, dr, nr, np);
-    hipLaunchKernelGGL(slstm_reduce_kernel, dim3((unsigned)((nb + 63) / 64)), dim3(256), 0, st, part_b, db, nb, np);
+    float* part_b = part_r + (size_t)ns * nr;
+    if constexpr (dr_lds(DH) > 0)
+        if (hipError_t e = mlstm::lds_limit_once<slstm_dr_kernel<DH>>(dr_lds(DH)); e != hipSuccess) return (int)e;
+    hipLaunchKernelGGL(slstm_dr_kernel<DH>, dim3(NH * 4, ns), dim3(256), dr_lds(DH), st, dwx, h, part_r, part_b, B, NH, S, ns);
+    hipLaunchKernelGGL(slstm_reduce_kernel, dim3((unsigned)((nr + 63) / 64 + (nb + 63) / 64)), dim3(256), 0, st, Reduce{part_r, dr, nr}, Reduce{part_b, db, nb}, ns);
     return (int)hipGetLastError();
 }
 
@@ -775,7 +826,7 @@ size_t slstm_saved_bytes(int B, int NH, int S, int DH) {
 
 size_t slstm_workspace_bytes(int B, int NH, int S, int DH) {
     if (B <= 0 || NH <= 0 || S <= 0 || !slstm::good_dh(DH)) return 0;
-    return (size_t)slstm::slices_for(B, NH, S) * slstm::dr_parts(DH) * NH * 4 * ((size_t)DH * DH + DH) * sizeof(float);
+    return (size_t)slstm::slices_for(B, NH, S) * NH * 4 * ((size_t)DH * DH + DH) * sizeof(float);
 }
 
 int slstm_forward_ex(const float* wx, const float* r, const float* b, float* h, float* saved, int B, int NH, int S, int DH,
