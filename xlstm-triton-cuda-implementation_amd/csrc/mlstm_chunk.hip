@@ -16,6 +16,7 @@
 //   chunk_carry_kernel  C~_c = gamma_c C~_{c-1} + dC_c over the chunks of a head (gamma_c = exp(A_{e_{c-1}} - A_{e_c})),
 //                       element-wise, written in the element type; n~_c likewise, in place, fp32.
 //   chunk_sum_small_kernel, chunk_carry_small_kernel  the same two steps for fp32 and for 16-bit types at D = 64 (fp32 MFMA).
+//   chunk_sum_terms_kernel  the chunk sums of bf16 at D = 64, outside split mode, with the weighted values as three bf16 terms.
 // State rows are stored in the order in which the row kernel's second product contracts them (see PERM16 below).
 #include "mlstm_device.h"
 #include "mlstm_kernels.h"
@@ -560,6 +561,157 @@ __global__ __launch_bounds__(256) void chunk_sum_narrow_kernel(ChunkArgs a) {
             for (int g = 0; g < NPG; g++) sum += red[g * W + tid];
             a.Nst[((size_t)bh * a.NCS + cc) * D + kcol + tid] = sum;
         }
+    }
+#endif
+}
+
+// The chunk sums of bf16 at D = 64: chunk_sum_small_kernel forms them in fp32 products; here each weighted value, w_j v_j in fp32, is three bf16 terms (24
+// bits, as in Tr<float>) and a key is one, so that three bf16 products do at 96 cycles per 32 x 32 x 16 block what the fp32 ones do at 512.  One
+// workgroup per (head, chunk) forms the whole 64 x 64 block, a 32 x 32 one per wave: all of a chunk of 256 positions is requested at once in whole lines, 16 bytes
+// a lane (that kernel: two bytes, and every row twice), and passes through LDS in parts of 64 (of 128, two workgroups per CU and not three: 38.6 us for 35.6).
+// A block that is not finite is formed again in fp32 multiply-adds (see not_finite).  Split mode and fp16, whose keys would be two terms and
+// whose sums are relied upon bit by bit, stay on fp32 products.
+// us, fp32 products / here, forward and reverse sums together: 64 heads x 8192 160 / 75 (K and V take 26 each way at the rate of a copy), 8 x 4096 18.2 / 17.5, 1 x 1100
+// 17.0 / 16.0; training step of 64 x 8192 642 / 565.  Errors against 64 bits (h and all gradients, 1100 and 1500 positions) 0.998 to
+// 1.001 of those before.
+struct ChunkTermsCfg {
+    static constexpr int L = 256, W = 64, PART = 64;
+    static constexpr size_t TILE_BYTES = (size_t)PART * W * 2, LDS_BYTES = 4 * TILE_BYTES + 2 * L * sizeof(float);
+};
+__global__ __launch_bounds__(256) void chunk_sum_terms_kernel(ChunkArgs a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    typedef __bf16 T;
+    using R = Tr<T>;
+    using Cfg = ChunkTermsCfg;
+    using Z = Swz<T, Cfg::W>;
+    typedef typename R::frag frag;
+    typedef typename R::vec4 V4;
+    struct Pair { V4 lo, hi; };
+    constexpr int L = Cfg::L, W = Cfg::W, PART = Cfg::PART, KW = R::KW, D = 64, NP = PART * Z::CPR / 256, ROWS = 256 / Z::CPR;   // pieces per thread and part, rows of 256 threads
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    char* const kt = smem;
+    auto vt = [&](int term) { return smem + (1 + term) * Cfg::TILE_BYTES; };
+    float* const sw = reinterpret_cast<float*>(smem + 4 * Cfg::TILE_BYTES);
+    float* const sw2 = sw + L;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5, c32 = lane & 31;
+    const int cc = blockIdx.x % a.NCS, bh = blockIdx.x / a.NCS, S = a.S;
+    const size_t poff = (size_t)bh * a.NG * GRAN, goff = (size_t)bh * a.NG;
+    const int p0 = (a.reverse ? cc + 1 : cc) * L, pe = a.reverse ? p0 - 1 : p0 + L - 1;   // (see chunk_sum_kernel)
+    const size_t rsK = (size_t)a.lk.ss, rsV = (size_t)a.lv.ss;
+    const T* const Kh = reinterpret_cast<const T*>(a.K) + a.lk.head(bh) + (size_t)p0 * rsK;
+    const T* const Vh = reinterpret_cast<const T*>(a.V) + a.lv.head(bh) + (size_t)p0 * rsV;
+
+    // what the weight of position tid needs, then all of the chunk
+    const int pos = p0 + tid < S ? p0 + tid : S - 1;
+    const float bend = a.beta2[poff + pe];
+    const double Gend = a.G2[goff + pe / GRAN], xg = a.G2[goff + pos / GRAN];
+    const float x0 = a.reverse ? a.beta2[poff + pos] : a.alpha2[poff + pos];
+    const float x1 = a.reverse ? a.inv_n[poff + pos] : 0.f, x2 = a.reverse ? a.db[poff + pos] : 0.f;
+    const int vrow = tid / Z::CPR, vch = tid % Z::CPR;   // a thread's 16-byte pieces: row vrow + ROWS i, piece vch
+    const bool whole = p0 + L <= S;
+    u32x4 kset[L / PART][NP], vset[L / PART][NP];
+#pragma unroll
+    for (int p = 0; p < L / PART; p++)
+#pragma unroll
+        for (int i = 0; i < NP; i++) {
+            const int r = PART * p + vrow + ROWS * i, rr = whole || p0 + r < S ? r : S - 1 - p0;   // (rows past the end, with weights of 0, become its last)
+            kset[p][i] = *reinterpret_cast<const u32x4*>(Kh + (size_t)rr * rsK + Z::EPC * vch);
+            vset[p][i] = *reinterpret_cast<const u32x4*>(Vh + (size_t)rr * rsV + Z::EPC * vch);
+        }
+    {
+        const float log2scale = -0.5f * __log2f((float)D);
+        float w = 0.f, w2 = 0.f;
+        if (p0 + tid < S) {
+            if (a.reverse) {
+                const float rho = fast_exp2(bend - x0 + (float)(xg - Gend) + log2scale);
+                w = rho * x1;
+                w2 = rho * x2;
+            } else {
+                w = w2 = fast_exp2(x0 - bend + (float)(Gend - xg) + log2scale);
+            }
+        }
+        sw[tid] = w;
+        sw2[tid] = w2;
+    }
+    // per-lane offsets of the transposing reads (see frag_transposed): rows 16 apart meet the same swizzle
+    const int kb = wave & 1, vb = wave >> 1;
+    const int j16 = lane & 15, sub = (lane >> 4) & 1, trow = 4 * h + (j16 >> 2), tcol = 16 * sub + 4 * (j16 & 3);
+    const int ko0 = Z::off(trow, 32 * kb + tcol), ko1 = Z::off(trow + 8, 32 * kb + tcol);
+    const int vo0 = Z::off(trow, 32 * vb + tcol), vo1 = Z::off(trow + 8, 32 * vb + tcol);
+    auto read = [&](const char* tile, int o0, int o1) __attribute__((always_inline)) {
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_PTR(s16x4))(tile + o0));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_PTR(s16x4))(tile + o1));
+        return __builtin_bit_cast(frag, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    };
+    f32x16 acc, small;   // (the products of the smaller terms apart: the large ones' sum then has one rounding per 16 positions)
+#pragma unroll
+    for (int x = 0; x < 16; x++) acc[x] = small[x] = 0.f;
+    float n0 = 0.f, n1 = 0.f;   // the vector state of keys 2 k2, 2 k2 + 1 over every eighth position
+    const int k2 = tid & 31, pg = tid >> 5;
+#pragma unroll
+    for (int p = 0; p < L / PART; p++) {
+        __syncthreads();   // the weights are there; the part before has been read
+#pragma unroll
+        for (int i = 0; i < NP; i++) {
+            const int row = vrow + ROWS * i, to = Z::off(row, Z::EPC * vch);
+            *reinterpret_cast<u32x4*>(kt + to) = kset[p][i];
+            const float w = sw[PART * p + row];
+            float x[8];
+            unpack8<T>(vset[p][i], x);
+            f32x4 lo4{x[0] * w, x[1] * w, x[2] * w, x[3] * w}, hi4{x[4] * w, x[5] * w, x[6] * w, x[7] * w};
+#pragma unroll
+            for (int term = 0; term < 3; term++) {
+                const Pair t{R::cvt4(lo4), R::cvt4(hi4)};
+                *reinterpret_cast<Pair*>(vt(term) + to) = t;
+                lo4 -= __builtin_convertvector(t.lo, f32x4);
+                hi4 -= __builtin_convertvector(t.hi, f32x4);
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int n = 0; n < PART / KW; n++) {
+            const int at = KW * n * Z::ROW_BYTES;
+            const frag af = read(kt + at, ko0, ko1);
+            R::mma(small, af, read(vt(2) + at, vo0, vo1));
+            R::mma(small, af, read(vt(1) + at, vo0, vo1));
+            R::mma(acc, af, read(vt(0) + at, vo0, vo1));
+        }
+#pragma unroll 8
+        for (int r = pg; r < PART; r += 8) {
+            typedef T T2 __attribute__((ext_vector_type(2)));
+            const T2 kv = *reinterpret_cast<const T2*>(kt + Z::off(r, 2 * k2));
+            const float w2 = sw2[PART * p + r];
+            n0 = fmaf((float)kv[0], w2, n0);
+            n1 = fmaf((float)kv[1], w2, n1);
+        }
+    }
+    acc += small;
+    float seen = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; r++) seen = not_finite(seen, acc[r]);
+    float* const out = a.dC + ((size_t)bh * a.NCS + cc) * D * D + (size_t)(32 * kb) * D + 32 * vb + c32;
+    if (__any(seen != 0.f)) {
+#pragma unroll 1
+        for (int r = 0; r < 16; r++) {
+            const int k = 8 * (r >> 2) + 4 * h + (r & 3);
+            float sum = 0.f;
+#pragma unroll 1
+            for (int j = 0; j < L && p0 + j < S; j++) sum = fmaf((float)Kh[(size_t)j * rsK + 32 * kb + k], (float)Vh[(size_t)j * rsV + 32 * vb + c32] * sw[j], sum);
+            out[(size_t)k * D] = sum;
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < 16; r++) out[(size_t)(8 * (r >> 2) + 4 * h + (r & 3)) * D] = acc[r];
+    }
+    __syncthreads();
+    float* const red = reinterpret_cast<float*>(smem);   // [eighth][key]
+    *reinterpret_cast<float2*>(red + pg * W + 2 * k2) = make_float2(n0, n1);
+    __syncthreads();
+    if (tid < W) {
+        float sum = 0.f;
+#pragma unroll
+        for (int g = 0; g < 8; g++) sum += red[g * W + tid];
+        a.Nst[((size_t)bh * a.NCS + cc) * D + tid] = sum;
     }
 #endif
 }
@@ -1452,6 +1604,14 @@ static int launch_chunk_small(const ChunkArgs& a, hipStream_t st) {
     if (!a.precise && (a.Cst_lo || a.CstT_lo)) return MLSTM_EINVAL;
     if (a.dot_part && !(a.CstT && a.dot_with)) return MLSTM_EINVAL;
     if (a.NCS > 1024) return MLSTM_ESHAPE;
+    if constexpr (std::is_same<T, __bf16>::value) {   // (other chunk lengths, which only mlstm_set_chunk_length asks for, go to the kernel below)
+        using C = ChunkTermsCfg;
+        if (a.L == C::L && !a.precise) {
+            if (hipError_t e = lds_limit_once<chunk_sum_terms_kernel>((int)C::LDS_BYTES); e != hipSuccess) return (int)e;
+            hipLaunchKernelGGL(chunk_sum_terms_kernel, dim3(a.BH * a.NCS), dim3(256), C::LDS_BYTES, st, a);
+            return launch_chunk_carry_small<T, D>(a, st);
+        }
+    }
     hipLaunchKernelGGL((chunk_sum_small_kernel<T, D>), dim3(a.BH * a.NCS * (D / 32)), dim3(256), 0, st, a);
     return launch_chunk_carry_small<T, D>(a, st);
 }
