@@ -375,11 +375,11 @@ def run_slstm(ffi, steps, warmup, shape=(16, 4, 2048, 64)):
         # the quantity the kernels are built around: wall time per step of the recurrence (B * NH walks side by side)
         "ns_per_recurrence_step": {"forward": f_ms * 1e6 / S, "backward": b_ms * 1e6 / S},
         # Latency model of the sequential walk: one wave per SIMD issues an instruction about every four cycles whatever it is,
-        # the compiled step loops have 143 (forward) / 170 (backward) instructions, the clock under load is about 2.1 GHz:
+        # the compiled step loops of the walking waves have 120 (forward) / 102 (backward) instructions, the clock under load is about 2.1 GHz:
         # the floor is instructions x 4 cycles per step; `frac` = that floor over the measured time per step.
         "roofline": {"bound": "latency", "kernel": "slstm_forward_kernel + slstm_backward_kernel (one step of the recurrence)",
-                     "achieved": (f_ms + b_ms) * 1e6 / S, "peak": (143 + 170) * 4 / 2.1, "unit": "ns/step",
-                     "frac": ((143 + 170) * 4 / 2.1) / ((f_ms + b_ms) * 1e6 / S) if f_ms + b_ms > 0 else None, "traffic": None},
+                     "achieved": (f_ms + b_ms) * 1e6 / S, "peak": (120 + 102) * 4 / 2.1, "unit": "ns/step",
+                     "frac": ((120 + 102) * 4 / 2.1) / ((f_ms + b_ms) * 1e6 / S) if f_ms + b_ms > 0 else None, "traffic": None},
         "hbm_gbs": bytes_compulsory / (ms_step * 1e-3) / 1e9, "hbm_frac": bytes_compulsory / (ms_step * 1e-3) / 8e12,
     }
 
