@@ -212,3 +212,21 @@ def test_recurrent_gradients_over_slices(B, NH, S, DH):
     bound = 2.0 ** -24 * (B * S) ** 0.5 * 4
     assert bool(((dr.double().cpu() - d2 @ p2.transpose(-1, -2).contiguous()).abs() <= bound * size + 1e-30).all())
     assert bool(((db.double().cpu() - d2.sum(-1)).abs() <= bound * d2.abs().sum(-1) + 1e-30).all())
+
+
+@pytest.mark.parametrize("DH", [32, 64, 128])
+def test_forward_of_a_full_grid_off_a_16_byte_boundary(DH):
+    # Thousands of steps in every workgroup, inputs that no cache holds: a step that took its input from the ring before it was there would take that of
+    # eight steps before.
+    from slstm import slstm_forward_hip
+    B, NH, S = 16, 4, 2048
+    g = torch.Generator(device="cuda").manual_seed(DH)
+    wx = torch.randn(B, S, 4, NH, DH, device="cuda", generator=g)
+    r, b = torch.randn(NH, 4, DH, DH, device="cuda", generator=g) / DH ** 0.5, torch.randn(NH, 4, DH, device="cuda", generator=g)
+    h, saved = slstm_forward_hip(wx, r, b, forget_sigmoid=True)
+    assert bool(torch.isfinite(h).all())
+    for off in (1, 2, 3):
+        other = torch.empty(wx.numel() + off, device="cuda")[off:].view(wx.shape).copy_(wx)
+        h2, saved2 = slstm_forward_hip(other, r, b, forget_sigmoid=True)
+        h3, _ = slstm_forward_hip(other, r, b, forget_sigmoid=True, save=False)
+        assert torch.equal(h2, h) and torch.equal(saved2, saved) and torch.equal(h3, h)

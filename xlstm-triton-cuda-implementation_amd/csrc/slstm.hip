@@ -35,11 +35,11 @@ __device__ __forceinline__ float fast_exp(float x) { return __builtin_amdgcn_exp
 __device__ __forceinline__ float fast_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 
 // Inputs of a step come from memory several steps ahead, as direct-to-LDS loads into a ring (a trip to memory is several
-// steps long, and a step must not wait for one).  The loads are issued and waited for by hand, by helper waves that issue the same
+// steps long, and a step must not wait for one).  The loads are issued and waited for by hand, by helper waves that issue at least a known
 // number of memory operations in every interval between two barriers, in the same order, so that
-// "the loads of step t have landed" is a counted wait -- memory operations of a wave complete in the order issued.  The
-// helpers' own code has only stores besides, for which the compiler places no waits.  (Left to the compiler, ordinary
-// loads into a ring of registers ended in a wait for everything at every step.)
+// "the loads of step t have landed" is a counted wait -- memory operations of a wave complete in the order issued, and a count that is
+// too low only waits for more.  The helpers' own code has only stores besides, for which the compiler places no waits.  (Left to the
+// compiler, ordinary loads into a ring of registers ended in a wait for everything at every step.)
 constexpr int PF = 8;
 // (a row's address is uniform, the lane's place in it an offset in bytes)
 __device__ __forceinline__ void ring_load(const float* row, unsigned lane_off, unsigned lds_off) {
@@ -287,11 +287,14 @@ __global__ __launch_bounds__(FwdCfg<DH>::THREADS) void slstm_forward_kernel(cons
     ring_wait(0);
     __syncthreads();
     // Rows PF on: row t + 2 was requested in interval t + 2 - PF, and the PF - 2 intervals since have a request each and, from interval 2 on, the stores
-    // (without the saved state those of h, of the first helper wave alone): one interval fewer is waited for.
-    constexpr int STORES = (WIDE ? 1 : 4) * PIECES, OPS = LOADS + STORES;
+    // (without the saved state those of h, of the first helper wave alone): one interval fewer is waited for.  What may stay under way counts only
+    // operations that are certain to be issued: the loads are asm, one each, but a piece that is stored float by float need not be four stores (the
+    // compiler makes one of 16 bytes of it, which may lie on any boundary of four).  Counted as four the wait never came to bear.
+    constexpr int OPS = LOADS + PIECES;
+    static_assert((PF - 3) * OPS < 64, "a count that the wait can hold");
     auto wait = [&]() __attribute__((always_inline)) {
-        if (SAVE || hwave == 0) mlstm::dma_wait_but<((PF - 3) * OPS < 63 ? (PF - 3) * OPS : 63)>();
-        else mlstm::dma_wait_but<((PF - 3) * LOADS < 63 ? (PF - 3) * LOADS : 63)>();
+        if (SAVE || hwave == 0) mlstm::dma_wait_but<(PF - 3) * OPS>();
+        else mlstm::dma_wait_but<(PF - 3) * LOADS>();
     };
     int t = 0;
     for (; t < 2 && t < S; t++) {
