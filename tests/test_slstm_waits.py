@@ -56,3 +56,38 @@ def test_the_wait_for_an_input_row_covers_it(kernels, DH, save, sigmoid, wide):
         assert waits and len(waits) <= len(issued), waits
         assert all(wait <= ahead * most for wait, most in zip(waits, issued)), (loads, stores, waits)
     assert steady
+
+
+@pytest.mark.parametrize("DH", [32, 64, 128])
+@pytest.mark.parametrize("save,sigmoid,wide", [(s, f, w) for s in (0, 1) for f in (0, 1) for w in (0, 1)])
+def test_the_first_input_is_read_before_its_place_is_refilled(kernels, DH, save, sigmoid, wide):
+    # The rows of the first round are there at a barrier.  The walk reads the first one behind it, the helpers request the row that takes its place: with
+    # a barrier more between the two.
+    lines = kernels[DH, save, sigmoid, wide]
+    at = lambda start, *ops: next(n for n in range(start, len(lines)) if lines[n].startswith(ops))  # noqa: E731
+    label = {line.split(":")[0]: n for n, line in enumerate(lines) if line.startswith(".LBB")}
+
+    def passed(start, op):
+        """for every line with `op` that a way from `start` comes to first: the lines of a shortest way there"""
+        ways, seen, ends = [(start,)], {start}, []
+        for way in ways:
+            line = lines[way[-1]]
+            if line.startswith(op) and len(way) > 1:
+                ends.append([lines[n] for n in way])
+                continue
+            jump = re.match(r"s_(c?)branch\w* (\.LBB\w+)", line)
+            following = ([label[jump.group(2)]] if jump else []) + ([] if line == "s_endpgm" or jump and not jump.group(1) else [way[-1] + 1])
+            for n in following:
+                if n not in seen and n < len(lines):
+                    seen.add(n)
+                    ways.append(way + (n,))
+        return ends
+    there = at(at(0, "global_load_lds"), "s_waitcnt vmcnt(0)")
+    ways = passed(there, "global_load_lds")
+    assert ways and all(sum(x.startswith("s_barrier") for x in way) >= 2 for way in ways)
+    first = at(at(0, "global_load_dwordx4"), "s_barrier")   # (the walk begins with its part of R)
+    ways = passed(first, "s_barrier")
+    assert ways
+    for way in ways:
+        read = next(n for n, x in enumerate(way) if x.startswith("ds_read_b32"))
+        assert any("lgkmcnt(0)" in x for x in way[read:])

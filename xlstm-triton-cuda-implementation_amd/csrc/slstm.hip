@@ -129,8 +129,9 @@ __global__ __launch_bounds__(FwdCfg<DH>::THREADS) void slstm_forward_kernel(cons
     const int b = blockIdx.x / NH, hd = blockIdx.x % NH;
     const size_t step_wx = (size_t)4 * NH * DH, step_h = (size_t)NH * DH, step_s = (size_t)7 * NH * DH;
     for (int e = tid; e < 8 * KS; e += Cfg::THREADS) hs[0][e] = 0.f;
-    // Interval t lies between barriers t and t + 1; the walk's step t is in it.  Step t takes h_{t-1} from hs[t & 1] and leaves h_t in the other; it
-    // writes what step t - 1 keeps to stage[(t - 1) & 1] and reads its successor's input from the ring.
+    // Interval t lies between barriers t + 1 and t + 2 (the walk reads the first input between barriers 0 and 1); the walk's step t is in it.  Step t
+    // takes h_{t-1} from hs[t & 1] and leaves h_t in the other; it writes what step t - 1 keeps to stage[(t - 1) & 1] and reads its successor's input
+    // from the ring.
     if (wave < 4 * DH / 64) {
         const int j = tid >> 2, q = tid & 3, p = tid & 7;
         const bool is0 = q == 0, is1 = q == 1, is2 = q == 2;
@@ -162,6 +163,7 @@ __global__ __launch_bounds__(FwdCfg<DH>::THREADS) void slstm_forward_kernel(cons
         };
         __syncthreads();
         float wv = ring[0][in_at];
+        __syncthreads();   // (its place may be refilled; every later one is read an interval ahead of that)
         auto step = [&](int u) __attribute__((always_inline)) {   // u = t mod PF
             const float* hcur = hs[u & 1] + p * KS;   // (PF is even: the buffers alternate across rounds too)
             constexpr int AHEAD = KP / 4 < 4 ? KP / 4 : 2;   // (reads under way: DH = 128 has registers for no more)
@@ -286,6 +288,7 @@ __global__ __launch_bounds__(FwdCfg<DH>::THREADS) void slstm_forward_kernel(cons
     for (int u = 0; u < PF; u++) request(u);
     ring_wait(0);
     __syncthreads();
+    __syncthreads();   // the walk has read row 0
     // Rows PF on: row t + 2 was requested in interval t + 2 - PF, and the PF - 2 intervals since have a request each and, from interval 2 on, the stores
     // (without the saved state those of h, of the first helper wave alone): one interval fewer is waited for.  What may stay under way counts only
     // operations that are certain to be issued: the loads are asm, one each, but a piece that is stored float by float need not be four stores (the
