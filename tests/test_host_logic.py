@@ -82,6 +82,15 @@ def test_tile_copy_index_arithmetic_stays_inside_the_tiles():
     assert out.returncode == 0 and "tile_bounds: ok" in out.stdout, out.stdout + out.stderr
 
 
+def test_gates_formed_in_a_row_kernel_go_to_that_kernel_alone():
+    """tests/harness/row_dispatch (the library's own choice of a row kernel, compiled for the host): once the pre-pass is left to roww_kernel no
+    other kernel is launched in its place."""
+    here = os.path.join(os.path.dirname(os.path.abspath(__file__)), "harness")
+    subprocess.check_call(["make", "-C", here, "row_dispatch"])
+    out = subprocess.run([os.path.join(here, "row_dispatch")], capture_output=True, text=True)
+    assert out.returncode == 0 and "row_dispatch: ok" in out.stdout, out.stdout + out.stderr
+
+
 def test_operators_do_without_the_native_host_path(monkeypatch):
     """The extension belongs to one torch release; missing, or another release's, it is left out with a warning and the calls go
     through ctypes (every function says that it serves nothing)."""

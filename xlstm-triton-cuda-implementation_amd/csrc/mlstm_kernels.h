@@ -136,7 +136,7 @@ int launch_row_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t 
 int launch_rowf_kernel(int mode, int D, const RowArgs& a, hipStream_t st);
 // eight waves (producer / consumer pairs per SIMD); 16-bit types and D in {128, 256} only
 int launch_row8_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t st);
-// the same bits on 64 rows per workgroup, for launches that leave the chip part empty; 16-bit types and D in {128, 256} only
+// the same bits on 64 or 32 rows per workgroup, for launches that leave the chip part empty; 16-bit types and D in {128, 256} only
 int launch_roww_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t st);
 // split mode on 64 rows per workgroup, the bits of the four-wave kernel, for the same launches; not with an output gate
 int launch_rowx_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t st);
@@ -160,6 +160,8 @@ inline bool roww_serves(int dtype, int D, const RowArgs& a) {
 }
 // (the four-wave kernel serves every other case: fp32, D = 64, split mode -- in chunks too --, large launches at D = 128 and the test switch)
 inline int launch_row_best(int mode, int dtype, int D, const RowArgs& a, hipStream_t st) {
+    // (what a kernel that forms the gates is to read is not there for any other, also where a switch was turned since that was decided)
+    if (a.gate_F) return launch_roww_kernel(mode, dtype, D, a, st);
     if (dtype != MLSTM_F32 && (D == 128 || D == 256) && !g_force_generic) {
         int rc = MLSTM_ESHAPE;
         if (roww_serves(dtype, D, a)) rc = launch_roww_kernel(mode, dtype, D, a, st);
