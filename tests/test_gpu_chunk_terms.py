@@ -46,3 +46,22 @@ def test_values_that_are_not_finite():
     # (its block of the state is formed again in another order: one rounding to bf16 of the state apart, 2^-8 of what the sum is made of)
     a, b = h[0, 1][:, others].float(), clean[0, 1][:, others].float()
     assert bool(torch.isfinite(a).all()) and float((a - b).norm() / b.norm()) <= 2.0 ** -8
+
+
+@pytest.mark.parametrize("S", [1025, 1056, 1279])
+def test_an_infinite_last_query_of_a_partial_chunk(S):
+    # Column 5 of the last query is infinite, and all that meets it on the way to dK of earlier chunks is positive (values, dh and, by an h that
+    # opposes dh, the row's share of the normaliser): dK is infinite there and not NaN, which a row past the end with a weight of zero would make it.
+    q, k, v, f, i, dh = [t.cuda() for t in O.make_inputs(1, 2, S, 64, torch.bfloat16, seed=S, f_mean=6.0)]
+    v = v.abs() + 0.5
+    dh[:, :, -1] = dh[:, :, -1].abs() + 0.5
+    h, m, b, saved = mm.mlstm_forward_save_hip(q, k, v, f, i)
+    b[:, :, -1] = b[:, :, -1].abs() + 10   # (above the normaliser's floor)
+    h[:, :, -1] = -dh[:, :, -1]
+    clean = mm.mlstm_backward_saved_hip(dh, q, k, v, f, i, h, m, b, saved)[1]
+    assert bool(torch.isfinite(clean).all())
+    q[:, :, -1, 5] = float("inf")
+    dk = mm.mlstm_backward_saved_hip(dh, q, k, v, f, i, h, m, b, saved)[1]
+    assert bool(torch.isposinf(dk[:, :, :1024, 5]).all())
+    others = [c for c in range(64) if c != 5]
+    assert bool(torch.isfinite(dk[:, :, :1024][..., others]).all())

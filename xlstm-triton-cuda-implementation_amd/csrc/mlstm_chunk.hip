@@ -614,7 +614,7 @@ __global__ __launch_bounds__(256) void chunk_sum_terms_kernel(ChunkArgs a) {
     for (int p = 0; p < L / PART; p++)
 #pragma unroll
         for (int i = 0; i < NP; i++) {
-            const int r = PART * p + vrow + ROWS * i, rr = whole || p0 + r < S ? r : S - 1 - p0;   // (rows past the end, with weights of 0, become its last)
+            const int r = PART * p + vrow + ROWS * i, rr = whole || p0 + r < S ? r : S - 1 - p0;   // (past the end: the last row, whose place takes zeros below)
             kset[p][i] = *reinterpret_cast<const u32x4*>(Kh + (size_t)rr * rsK + Z::EPC * vch);
             vset[p][i] = *reinterpret_cast<const u32x4*>(Vh + (size_t)rr * rsV + Z::EPC * vch);
         }
@@ -654,10 +654,12 @@ __global__ __launch_bounds__(256) void chunk_sum_terms_kernel(ChunkArgs a) {
 #pragma unroll
         for (int i = 0; i < NP; i++) {
             const int row = vrow + ROWS * i, to = Z::off(row, Z::EPC * vch);
-            *reinterpret_cast<u32x4*>(kt + to) = kset[p][i];
+            u32x4 k8 = kset[p][i], v8 = vset[p][i];
+            if (!whole && p0 + PART * p + row >= S) k8 = v8 = u32x4{0, 0, 0, 0};   // (a weight of 0 would not do: the last row may be infinite)
+            *reinterpret_cast<u32x4*>(kt + to) = k8;
             const float w = sw[PART * p + row];
             float x[8];
-            unpack8<T>(vset[p][i], x);
+            unpack8<T>(v8, x);
             f32x4 lo4{x[0] * w, x[1] * w, x[2] * w, x[3] * w}, hi4{x[4] * w, x[5] * w, x[6] * w, x[7] * w};
 #pragma unroll
             for (int term = 0; term < 3; term++) {
