@@ -385,6 +385,10 @@ __device__ __forceinline__ void dma16(const void* g, unsigned lds_off) {
 __device__ __forceinline__ void dma4(const void* g, unsigned lds_off) {
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off" ::"v"(g), "s"(lds_off) : "memory", "m0");
 }
+// two bytes per lane, each lane's as a dword with zeros above them
+__device__ __forceinline__ void dma2(const void* g, unsigned lds_off) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_ushort %0, off" ::"v"(g), "s"(lds_off) : "memory", "m0");
+}
 __device__ __forceinline__ void dma_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 // everything but the N newest of the wave's memory operations (others than the counted loads among them, a spill's, only make it wait longer)
 template <int N> __device__ __forceinline__ void dma_wait_but() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }

@@ -111,23 +111,28 @@ __global__ __launch_bounds__(256 * RB) void roww_kernel(RowArgs a) {
         if (2 * r + 1 < nJ) copy_tile(y2_at(r, 1), Y2, 2 * r + 1);
     };
     // The gates of the head's granules up to the rows' own, granule wave + NW k in turn k, are requested first: copies into LDS (the places of
-    // their key weights), so that a counted wait can leave the tiles behind them under way while the gates are formed.  16-bit values come as the
-    // dword that holds them.  Two launches / one, forward, us: 1 x 64 x 128 7.9 / 6.3, 1 x 320 10.5 / 9.6, 1 x 640 12.9 / 12.9 (a granule is 250
+    // their key weights), so that a counted wait can leave the tiles behind them under way while the gates are formed.  (16-bit values one
+    // by one: the dword that holds one reaches beyond the tensor at either of its ends.)  Two launches / one, forward, us: 1 x 64 x 128 7.9 / 6.3, 1 x 320 10.5 / 9.6, 1 x 640 12.9 / 12.9 (a granule is 250
     // instructions, 100 of them its logarithms, and a workgroup forms all of its head's: 2 us of a CU for ten), 8 x 1000 19.5 / 18.1, 15 x 1001
     // 22.7 / 19.2, 16 x 256 10.7 / 9.0; D = 256, 1 x 640 15.6 / 15.0, 8 x 1000 24.5 / 22.8, 24 x 1000 31.5 / 29.3, 100 x 128 12.3 / 9.5.
     constexpr int NW = NT / 64, TURNS = FUSED ? RW_MOST_KEYS / GRAN / NW : 1;
     if constexpr (FUSED) {
-        const size_t off = a.lg.head(bh), ss = (size_t)a.lg.ss, el = a.gate_dtype == MLSTM_F32 ? 4 : 2;
+        const size_t off = a.lg.head(bh), ss = (size_t)a.lg.ss;
+        auto request = [&](auto gate, auto&& copy) __attribute__((always_inline)) {
+            typedef decltype(gate) G;
 #pragma unroll
-        for (int k = 0; k < TURNS; k++) {
-            const int g = tid / 64 + NW * k;
-            if (g < nJ) {
-                const int t = g * GRAN + lane;
-                const size_t at = (off + (size_t)(t < S ? t : S - 1) * ss) * el;
-                dma4((const void*)(((size_t)a.gate_F + at) & ~(size_t)3), __builtin_amdgcn_readfirstlane(lds_offset_of(sek + GRAN * g)));
-                dma4((const void*)(((size_t)a.gate_I + at) & ~(size_t)3), __builtin_amdgcn_readfirstlane(lds_offset_of(sal + GRAN * g)));
+            for (int k = 0; k < TURNS; k++) {
+                const int g = tid / 64 + NW * k;
+                if (g < nJ) {
+                    const int t = g * GRAN + lane;
+                    const size_t at = off + (size_t)(t < S ? t : S - 1) * ss;
+                    copy(reinterpret_cast<const G*>(a.gate_F) + at, __builtin_amdgcn_readfirstlane(lds_offset_of(sek + GRAN * g)));
+                    copy(reinterpret_cast<const G*>(a.gate_I) + at, __builtin_amdgcn_readfirstlane(lds_offset_of(sal + GRAN * g)));
+                }
             }
-        }
+        };
+        if (a.gate_dtype == MLSTM_F32) request(0.f, dma4);
+        else request((unsigned short)0, dma2);
     }
     // (plain loads first: what they bring is used behind the copies' issue)
     const double g_rows = FUSED ? 0.0 : a.G2[goff + gt], g_mine = FUSED ? 0.0 : a.G2[goff + (tid < nJ ? tid : 0)], g_end = chunk > 0 ? a.G2[goff - 1] : 0.0;
@@ -190,22 +195,16 @@ __global__ __launch_bounds__(256 * RB) void roww_kernel(RowArgs a) {
             constexpr int N = decltype(n_tag)::value;
             float lf[N], ig[N], cs[N], al[N];
             GateLocal vs[N];
-            const size_t off = a.lg.head(bh), ss = (size_t)a.lg.ss;
 #pragma unroll
             for (int k = 0; k < N; k++) {
                 const int t = (wave + NW * k) * GRAN + lane, tr = (wave + NW * k < nJ ? t : lane);   // (a turn too many: some place that is there)
                 unsigned x = __builtin_bit_cast(unsigned, sek[tr]), y = __builtin_bit_cast(unsigned, sal[tr]);
-                if (a.gate_dtype != MLSTM_F32) {
-                    const size_t e = off + (size_t)(t < S ? t : S - 1) * ss;
-                    x >>= (((size_t)a.gate_F >> 1) + e) & 1 ? 16 : 0;
-                    y >>= (((size_t)a.gate_I >> 1) + e) & 1 ? 16 : 0;
-                    if (a.gate_dtype == MLSTM_F16) {
-                        x = __builtin_bit_cast(unsigned, (float)__builtin_bit_cast(_Float16, (unsigned short)x));
-                        y = __builtin_bit_cast(unsigned, (float)__builtin_bit_cast(_Float16, (unsigned short)y));
-                    } else {
-                        x <<= 16;
-                        y <<= 16;
-                    }
+                if (a.gate_dtype == MLSTM_F16) {
+                    x = __builtin_bit_cast(unsigned, (float)__builtin_bit_cast(_Float16, (unsigned short)x));
+                    y = __builtin_bit_cast(unsigned, (float)__builtin_bit_cast(_Float16, (unsigned short)y));
+                } else if (a.gate_dtype == MLSTM_BF16) {
+                    x <<= 16;
+                    y <<= 16;
                 }
                 const GateIn in{__builtin_bit_cast(float, x), 0.f, __builtin_bit_cast(float, y)};
                 lf[k] = forget_log(in, t, a.gate_form);
