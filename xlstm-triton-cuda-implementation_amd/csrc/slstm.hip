@@ -45,36 +45,6 @@ constexpr int PF = 8;
 __device__ __forceinline__ void ring_load(const float* row, unsigned lane_off, unsigned lds_off) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dword %0, %1" ::"v"(lane_off), "s"(row), "s"(lds_off) : "memory", "m0");
 }
-// (n is a constant once the step loops are unrolled; anything out of range waits for everything)
-__device__ __forceinline__ void ring_wait(int n) {
-    switch (n) {
-        case 1: asm volatile("s_waitcnt vmcnt(1)" ::: "memory"); break;
-        case 2: asm volatile("s_waitcnt vmcnt(2)" ::: "memory"); break;
-        case 3: asm volatile("s_waitcnt vmcnt(3)" ::: "memory"); break;
-        case 4: asm volatile("s_waitcnt vmcnt(4)" ::: "memory"); break;
-        case 5: asm volatile("s_waitcnt vmcnt(5)" ::: "memory"); break;
-        case 6: asm volatile("s_waitcnt vmcnt(6)" ::: "memory"); break;
-        case 7: asm volatile("s_waitcnt vmcnt(7)" ::: "memory"); break;
-        case 8: asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); break;
-        case 9: asm volatile("s_waitcnt vmcnt(9)" ::: "memory"); break;
-        case 10: asm volatile("s_waitcnt vmcnt(10)" ::: "memory"); break;
-        case 11: asm volatile("s_waitcnt vmcnt(11)" ::: "memory"); break;
-        case 12: asm volatile("s_waitcnt vmcnt(12)" ::: "memory"); break;
-        case 13: asm volatile("s_waitcnt vmcnt(13)" ::: "memory"); break;
-        case 14: asm volatile("s_waitcnt vmcnt(14)" ::: "memory"); break;
-        case 15: asm volatile("s_waitcnt vmcnt(15)" ::: "memory"); break;
-        case 16: asm volatile("s_waitcnt vmcnt(16)" ::: "memory"); break;
-        case 17: asm volatile("s_waitcnt vmcnt(17)" ::: "memory"); break;
-        case 18: asm volatile("s_waitcnt vmcnt(18)" ::: "memory"); break;
-        case 19: asm volatile("s_waitcnt vmcnt(19)" ::: "memory"); break;
-        case 20: asm volatile("s_waitcnt vmcnt(20)" ::: "memory"); break;
-        case 21: asm volatile("s_waitcnt vmcnt(21)" ::: "memory"); break;
-        case 22: asm volatile("s_waitcnt vmcnt(22)" ::: "memory"); break;
-        case 23: asm volatile("s_waitcnt vmcnt(23)" ::: "memory"); break;
-        case 24: asm volatile("s_waitcnt vmcnt(24)" ::: "memory"); break;
-        default: asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); break;
-    }
-}
 
 // Sum over the four lanes of a quad (lanes 4a .. 4a+3), the same bits in all four: two exchanges inside the quad.
 template <int CTRL>
@@ -286,7 +256,7 @@ __global__ __launch_bounds__(FwdCfg<DH>::THREADS) void slstm_forward_kernel(cons
     };
 #pragma unroll 1
     for (int u = 0; u < PF; u++) request(u);
-    ring_wait(0);
+    mlstm::dma_wait();
     __syncthreads();
     __syncthreads();   // the walk has read row 0
     // Rows PF on: row t + 2 was requested in interval t + 2 - PF, and the PF - 2 intervals since have a request each and, from interval 2 on, the stores
@@ -358,6 +328,7 @@ __global__ __launch_bounds__(BwdCfg<DH>::THREADS) void slstm_backward_kernel(con
     constexpr int PS = PE + 4;       // ... and four floats, so that the 16 parts of a row's read start in different banks
     constexpr int UW = Cfg::UW, NGRP = Cfg::NGRP, RING = Cfg::RING, SLOTS = Cfg::SLOTS, UL = DH < 64 ? DH : 64;   // UL: units per helper wave
     constexpr int RPL = WIDE ? 256 / UL : 1, NLOAD = (BWD_SAVED + RPL - 1) / RPL;   // rows per load, loads per job
+    static_assert((RING - 2) * (NLOAD + 1) < 64, "a count that the wait can hold");
     struct Lds {   // (what the steps read comes first: within an offset of the instructions)
         float delta[2][16 * PS];             // [buffer][part][unit * 4 + gate within the part]
         float shared_of[SLOTS][DH][4];       // A, B, f', dh of a unit
@@ -526,7 +497,7 @@ __global__ __launch_bounds__(BwdCfg<DH>::THREADS) void slstm_backward_kernel(con
     };
 #pragma unroll 1
     for (int i = 0; i < RING; i++) fetch();
-    ring_wait(0);
+    mlstm::dma_wait();
     take(0);
     factors();
     put(0);
@@ -546,7 +517,7 @@ __global__ __launch_bounds__(BwdCfg<DH>::THREADS) void slstm_backward_kernel(con
         __syncthreads();
     }
     for (int job = 1; n < S; job++) {
-        ring_wait((RING - 2) * (NLOAD + 1));
+        mlstm::dma_wait_but<(RING - 2) * (NLOAD + 1)>();
         take(job);
         if constexpr (NGRP == 2) { factors(); put(job); }
         __syncthreads();
