@@ -230,3 +230,29 @@ def test_forward_of_a_full_grid_off_a_16_byte_boundary(DH):
         h2, saved2 = slstm_forward_hip(other, r, b, forget_sigmoid=True)
         h3, _ = slstm_forward_hip(other, r, b, forget_sigmoid=True, save=False)
         assert torch.equal(h2, h) and torch.equal(saved2, saved) and torch.equal(h3, h)
+
+
+def test_a_batch_of_more_threads_than_a_launch_holds():
+    # 22.5 million sequences of one step: beyond 2^32 threads of either step kernel, whose batches then take several launches
+    from slstm import slstm_backward_hip, slstm_forward_hip
+    B, DH = 22_500_000, 32
+    if torch.cuda.mem_get_info()[0] < 60e9:
+        pytest.skip("needs 60 GB of GPU memory")
+    g = torch.Generator(device="cuda").manual_seed(1)
+    wx = torch.empty(B, 1, 4, 1, DH, device="cuda").normal_(generator=g)
+    r, b = torch.randn(1, 4, DH, DH, device="cuda", generator=g) / DH ** 0.5, torch.randn(1, 4, DH, device="cuda", generator=g)
+    dh = torch.empty(B, 1, 1, DH, device="cuda").normal_(generator=g)
+    h, saved = slstm_forward_hip(wx, r, b, forget_sigmoid=True)
+    dwx, dr, db = slstm_backward_hip(dh, h, r, saved, forget_sigmoid=True)
+    del saved
+    some = torch.tensor([0, 1, *[n * 2 ** 32 // threads + k for n, threads in ((1, 192), (1, 384), (2, 384)) for k in (-2, -1, 0, 1)], B - 1], device="cuda")
+    h1, saved1 = slstm_forward_hip(wx[some], r, b, forget_sigmoid=True)
+    assert torch.equal(h[some], h1) and bool(torch.isfinite(h1).all())
+    assert torch.equal(dwx[some], slstm_backward_hip(dh[some], h1, r, saved1, forget_sigmoid=True)[0])
+    assert not bool(dr.any())   # (h before the first step is zero)
+    want = torch.stack([dwx[:, 0, x, 0].double().sum(0) for x in range(4)])
+    # (fp32 sums over 128 slices of 176 thousand terms each, in chains of an eighth of a slice)
+    size = torch.stack([dwx[:, 0, x, 0].abs().double().sum(0) for x in range(4)])
+    assert bool(((db[0].double() - want).abs() <= 2.0 ** -24 * 22000 ** 0.5 * 4 * size).all())
+    del wx, dh, h, dwx
+    torch.cuda.empty_cache()

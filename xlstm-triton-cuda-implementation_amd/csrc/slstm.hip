@@ -742,14 +742,26 @@ int slices_for(int B, int NH, int S) {
     return (int)(n < 1 ? 1 : n);
 }
 
+// A launch holds fewer than 2^32 threads: a batch of more sequences in several, launch(first sequence, how many).
+template <typename F>
+int over_batch(int B, int NH, int threads, F&& launch) {
+    const long long fit = (long long)(0xffffffffu / (unsigned)threads) / NH, most = fit > 1 ? fit : 1;
+    for (long long b0 = 0; b0 < B; b0 += most)
+        if (int rc = launch(b0, (int)(B - b0 < most ? B - b0 : most))) return rc;
+    return 0;
+}
+
 // (the step kernels count their waits for the input ring by hand: see no_scratch_once)
 template <int DH, bool SAVE, bool FS>
 int forward_launch(const float* wx, const float* r, const float* b, float* h, float* saved, int B, int NH, int S, hipStream_t st) {
     auto launch = [&](auto wide) {
         constexpr auto kernel = slstm_forward_kernel<DH, SAVE, FS, decltype(wide)::value>;
         if (int rc = mlstm::no_scratch_once<kernel>()) return rc;
-        hipLaunchKernelGGL(kernel, dim3(B * NH), dim3(FwdCfg<DH>::THREADS), 0, st, wx, r, b, h, saved, NH, S);
-        return (int)hipGetLastError();
+        return over_batch(B, NH, FwdCfg<DH>::THREADS, [&](long long b0, int n) {
+            const size_t at = (size_t)b0 * S * NH * DH;
+            hipLaunchKernelGGL(kernel, dim3(n * NH), dim3(FwdCfg<DH>::THREADS), 0, st, wx + 4 * at, r, b, h + at, SAVE ? saved + 7 * at : nullptr, NH, S);
+            return (int)hipGetLastError();
+        });
     };
     const size_t at = reinterpret_cast<size_t>(wx) | reinterpret_cast<size_t>(h) | reinterpret_cast<size_t>(saved);
     return at & 15 ? launch(std::false_type{}) : launch(std::true_type{});
@@ -766,8 +778,11 @@ int forward_t(const float* wx, const float* r, const float* b, float* h, float* 
 template <int DH, bool FS, bool WIDE>
 int backward_launch_w(const float* dh, const float* r, const float* saved, float* dwx, int B, int NH, int S, hipStream_t st) {
     if (int rc = mlstm::no_scratch_once<slstm_backward_kernel<DH, FS, WIDE>>()) return rc;
-    hipLaunchKernelGGL((slstm_backward_kernel<DH, FS, WIDE>), dim3(B * NH), dim3(BwdCfg<DH>::THREADS), 0, st, dh, r, saved, dwx, NH, S);
-    return (int)hipGetLastError();
+    return over_batch(B, NH, BwdCfg<DH>::THREADS, [&](long long b0, int n) {
+        const size_t at = (size_t)b0 * S * NH * DH;
+        hipLaunchKernelGGL((slstm_backward_kernel<DH, FS, WIDE>), dim3(n * NH), dim3(BwdCfg<DH>::THREADS), 0, st, dh + at, r, saved + 7 * at, dwx + 4 * at, NH, S);
+        return (int)hipGetLastError();
+    });
 }
 template <int DH, bool FS>
 int backward_launch(const float* dh, const float* r, const float* saved, float* dwx, int B, int NH, int S, hipStream_t st) {
