@@ -256,3 +256,25 @@ def test_a_batch_of_more_threads_than_a_launch_holds():
     assert bool(((db[0].double() - want).abs() <= 2.0 ** -24 * 22000 ** 0.5 * 4 * size).all())
     del wx, dh, h, dwx
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("NH", [260_000, 300_000])
+def test_recurrent_gradients_of_more_heads_than_a_launch_holds(NH):
+    # a workgroup per 64 elements: dR and db of 260 000 heads of 32 units are 2^32 threads together, of 300 000 dR is by itself
+    from slstm import slstm_backward_hip, slstm_forward_hip
+    S, DH = 2, 32
+    if torch.cuda.mem_get_info()[0] < 20e9:
+        pytest.skip("needs 20 GB of GPU memory")
+    g = torch.Generator(device="cuda").manual_seed(2)
+    wx, dh = torch.randn(1, S, 4, NH, DH, device="cuda", generator=g), torch.randn(1, S, NH, DH, device="cuda", generator=g)
+    r, b = torch.randn(NH, 4, DH, DH, device="cuda", generator=g).mul_(DH ** -0.5), torch.randn(NH, 4, DH, device="cuda", generator=g)
+    h, saved = slstm_forward_hip(wx, r, b, forget_sigmoid=True)
+    dwx, dr, db = slstm_backward_hip(dh, h, r, saved, forget_sigmoid=True)
+    for lo in (0, NH // 2, NH - 3):   # (a few heads by themselves: the same bits)
+        few = slice(lo, lo + 3)
+        h1, saved1 = slstm_forward_hip(wx[:, :, :, few].contiguous(), r[few].contiguous(), b[few].contiguous(), forget_sigmoid=True)
+        got = slstm_backward_hip(dh[:, :, few].contiguous(), h1, r[few].contiguous(), saved1, forget_sigmoid=True)
+        for x, y in zip(got, (dwx[:, :, :, few], dr[few], db[few])):
+            assert torch.equal(x, y)
+    del wx, dh, r, dwx, dr, saved
+    torch.cuda.empty_cache()

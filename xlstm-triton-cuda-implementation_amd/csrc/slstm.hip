@@ -712,26 +712,30 @@ __global__ __launch_bounds__(256, 2) void slstm_dr_kernel(const float* __restric
     }
 }
 
-// out[e] = sum over the partial sums, in a fixed order: 64 elements per workgroup, four threads per element with every
-// fourth partial sum each, their four sums added in order.  The workgroups behind those of dR add up db (a launch of its own: 7 us).
+// out[e] = sum over the partial sums, in a fixed order: 64 elements per workgroup and turn, four threads per element with every
+// fourth partial sum each, their four sums added in order.  Behind the elements of dR come those of db (a launch of its own: 7 us).  (More than one
+// turn only where a workgroup per 64 elements would be more threads than a launch holds.)
 struct Reduce { const float* part; float* out; size_t n; };
 __global__ __launch_bounds__(256) void slstm_reduce_kernel(Reduce r, Reduce b, int nslice) {
     __shared__ float red[4][64];
     const int x = threadIdx.x & 63, y = threadIdx.x >> 6;
-    const size_t wgs = (r.n + 63) / 64;
-    const bool first = blockIdx.x < wgs;
-    const float* const part = first ? r.part : b.part;
-    float* const out = first ? r.out : b.out;
-    const size_t n = first ? r.n : b.n, e = (size_t)(first ? blockIdx.x : blockIdx.x - wgs) * 64 + x;
-    float s0 = 0.f, s1 = 0.f;
-    if (e < n) {
-        int i = y;
-        for (; i + 4 < nslice; i += 8) { s0 += part[(size_t)i * n + e]; s1 += part[(size_t)(i + 4) * n + e]; }
-        if (i < nslice) s0 += part[(size_t)i * n + e];
+    const size_t wgs = (r.n + 63) / 64, all = wgs + (b.n + 63) / 64;
+    for (size_t wg = blockIdx.x; wg < all; wg += gridDim.x) {
+        const bool first = wg < wgs;
+        const float* const part = first ? r.part : b.part;
+        float* const out = first ? r.out : b.out;
+        const size_t n = first ? r.n : b.n, e = (first ? wg : wg - wgs) * 64 + x;
+        float s0 = 0.f, s1 = 0.f;
+        if (e < n) {
+            int i = y;
+            for (; i + 4 < nslice; i += 8) { s0 += part[(size_t)i * n + e]; s1 += part[(size_t)(i + 4) * n + e]; }
+            if (i < nslice) s0 += part[(size_t)i * n + e];
+        }
+        red[y][x] = s0 + s1;
+        __syncthreads();
+        if (y == 0 && e < n) out[e] = (red[0][x] + red[1][x]) + (red[2][x] + red[3][x]);
+        __syncthreads();
     }
-    red[y][x] = s0 + s1;
-    __syncthreads();
-    if (y == 0 && e < n) out[e] = (red[0][x] + red[1][x]) + (red[2][x] + red[3][x]);
 }
 
 int slices_for(int B, int NH, int S) {
@@ -801,7 +805,8 @@ int backward_t(const float* dh, const float* h, const float* r, const float* sav
     if constexpr (dr_lds(DH) > 0)
         if (hipError_t e = mlstm::lds_limit_once<slstm_dr_kernel<DH>>(dr_lds(DH)); e != hipSuccess) return (int)e;
     hipLaunchKernelGGL(slstm_dr_kernel<DH>, dim3(NH * 4, ns), dim3(256), dr_lds(DH), st, dwx, h, part_r, part_b, B, NH, S, ns);
-    hipLaunchKernelGGL(slstm_reduce_kernel, dim3((unsigned)((nr + 63) / 64 + (nb + 63) / 64)), dim3(256), 0, st, Reduce{part_r, dr, nr}, Reduce{part_b, db, nb}, ns);
+    const size_t wgs = (nr + 63) / 64 + (nb + 63) / 64, most = 1 << 23;
+    hipLaunchKernelGGL(slstm_reduce_kernel, dim3((unsigned)(wgs < most ? wgs : most)), dim3(256), 0, st, Reduce{part_r, dr, nr}, Reduce{part_b, db, nb}, ns);
     return (int)hipGetLastError();
 }
 
