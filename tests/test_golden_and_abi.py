@@ -39,6 +39,15 @@ def test_oracle_reproduces_scan_golden():
     assert torch.allclose(h.float(), g["h"], rtol=1e-5, atol=1e-6)
 
 
+def test_slstm_backward_refuses_more_units_than_its_offsets_hold():
+    L = submodule("_ffi").lib()
+    null, one = ctypes.c_void_p(0), ctypes.c_void_p(16)   # never dereferenced
+    most = (2 ** 32 - 1) // 144   # nine rows of dWx, four gates of fp32 each, in 32 bits
+    for DH in (32, 64, 128):
+        for NH, rc in ((most // DH, -3), (most // DH + 1, -2)):   # (no workspace; no such shape)
+            assert L.slstm_backward_ex(*([one] * 7), 1, NH, 1, DH, 0, null, 0, null) == rc, (DH, NH)
+
+
 def test_library_exports_every_declared_symbol():
     ffi = submodule("_ffi")
     header = open(os.path.join(ROOT, "include", "mlstm_hip.h")).read()

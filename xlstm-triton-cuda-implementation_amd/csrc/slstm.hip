@@ -843,6 +843,8 @@ int slstm_backward_ex(const float* dh, const float* h, const float* r, const flo
                       int NH, int S, int DH, int forget_sigmoid, void* workspace, size_t workspace_bytes, void* stream) {
     if (!dh || !h || !r || !saved || !dwx || !dr || !db || B <= 0 || NH <= 0 || S <= 0) return MLSTM_EINVAL;
     if (!slstm::good_dh(DH)) return MLSTM_ESHAPE;
+    // (the kernels' offsets inside nine rows of dWx are 32 bits)
+    if ((size_t)NH * DH > 0xffffffffu / (9 * 4 * sizeof(float))) return MLSTM_ESHAPE;
     if (!workspace || workspace_bytes < slstm_workspace_bytes(B, NH, S, DH)) return MLSTM_EWORKSPACE;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     const int fs = forget_sigmoid ? 1 : 0;
