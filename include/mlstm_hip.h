@@ -275,7 +275,7 @@ int mlstm_scan_backward_saved_ex(const void* dh_gated, const void* q, const void
  * slstm_forward_ex writes what the backward needs into `saved` (slstm_saved_bytes; may be NULL for inference; opaque:
  * written and read by the same build of the library).  All tensors dense.
  * slstm_backward_ex needs a workspace of slstm_workspace_bytes.  One workgroup per (batch, head) walks the sequence:
- * the cell is sequential in t by construction.
+ * the cell is sequential in t by construction.  It takes up to 29.8 million units (NH * DH; beyond that MLSTM_ESHAPE).
  */
 size_t slstm_saved_bytes(int B, int NH, int S, int DH);
 size_t slstm_workspace_bytes(int B, int NH, int S, int DH);
@@ -295,7 +295,8 @@ size_t mlstm_workspace_bytes(int op, int B, int NH, int S, int D, int dtype);
  * mlstm_timing_read waits for the recorded launches of one kernel, returns their summed duration and count, and
  * forgets them.  Off by default; enabling it is process-wide.
  */
-#define MLSTM_K_GATES 0     /* gate pre-pass */
+#define MLSTM_K_GATES 0     /* gate pre-pass (none in forwards of 16-bit sequences that are not cut at D = 128 and 256 on few workgroups:
+                             * the tile kernel forms the gates there, and its time holds both) */
 #define MLSTM_K_ROW_FWD 1   /* forward tile kernel (H, b) */
 #define MLSTM_K_COL 3       /* backward tile kernel (dK, dV, dI, row partials) */
 #define MLSTM_K_ROW_DQ 4    /* backward tile kernel (dQ) */

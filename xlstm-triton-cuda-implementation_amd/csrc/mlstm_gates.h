@@ -35,8 +35,8 @@ __device__ __forceinline__ double wave_scan_inclusive_d(double v, int lane) {
     return Op::f(c, v);
 }
 
-// fp64 prefix over up to 64 granules, one per lane: exclusive sum G of the totals behind `run`, and the running maximum R of (P - G) over
-// EARLIER granules, `rmax` those before the 64.  The totals of 64 logarithms are floats: their sums are exact in fp64, in any order, unless they
+// fp64 prefix over up to 64 granules, one per lane: inclusive sum of their totals, exclusive sum G behind `run`, and the running maximum of (P - G) up to and
+// with a granule (before_lane: over the EARLIER ones).  The totals of 64 logarithms are floats: their sums are exact in fp64, in any order, unless they
 // lie 2^18 apart.  (By log-step lane shuffles, an LDS round trip each, the two scans took 0.9 us; these take 0.2.)
 __device__ __forceinline__ void granule_scan(double tot, double p, double run, int lane, double& incl, double& excl, double& mx) {
     incl = wave_scan_inclusive_d<AddD>(tot, lane);

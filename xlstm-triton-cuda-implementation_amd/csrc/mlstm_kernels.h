@@ -165,13 +165,14 @@ inline int launch_row_best(int mode, int dtype, int D, const RowArgs& a, hipStre
     if (dtype != MLSTM_F32 && (D == 128 || D == 256) && !g_force_generic) {
         int rc = MLSTM_ESHAPE;
         if (roww_serves(dtype, D, a)) rc = launch_roww_kernel(mode, dtype, D, a, st);
-        // Split mode: row_kernel / rowx_kernel, forward and dQ pass, us --
-        // D = 128   64: 21.3, 23.2 / 13.5, 15.7   256: 23.4, 24.9 / 16.1, 18.4   384: 23.9, 26.5 / 22.6, 27.0   512: 24.8, 27.6 / 26.2, 29.8
-        // D = 256   64: 39.3, 43.8 / 22.6, 26.9   256: 41.8, 47.3 / 26.0, 30.2   384: 42.9, 47.6 / 36.9, 42.4   512: 44.1, 49.0 / 40.8, 46.8
+        // Split mode: row_kernel / rowx_kernel, forward and dQ pass, us (heads x positions: 2, 8 and 16 x 2048, 12 and 16 x 1500) --
+        // D = 128   64: 19.0, 21.8 / 14.4, 16.4   256: 21.4, 23.2 / 16.3, 18.6   288: 21.0, 23.5 / 16.7, 20.6   384: 21.5, 24.1 / 22.0, 25.2   512: 22.6, 26.0 / 25.8, 29.3
+        // D = 256   64: 34.6, 39.2 / 23.1, 27.0   256: 38.0, 42.3 / 25.6, 30.4   288: 37.3, 41.4 / 25.8, 32.1   384: 37.9, 41.8 / 33.4, 39.2   512: 40.1, 44.7 / 40.1, 46.3
+        //           (8 heads, whose tiles share an XCD's cache one by one: 376, 8 x 3000, 38.2, 42.0 / 36.8, 44.2   512, 8 x 4096, 40.1, 44.7 / 46.7, 54.2)
         if ((long long)a.BH * a.NG <= (D == 128 ? 256 : 512) && a.precise) rc = launch_rowx_kernel(mode, dtype, D, a, st);
         // D = 128 beyond 512 of them, row_kernel, whose workgroups share a CU in pairs: row8_kernel / row_kernel, forward and dQ pass, us --
-        //   512: 18.2, 21.1 / 19.0, 22.6   768: 26.9, 30.8 / 23.6, 27.6   1024: 31.6, 36.4 / 25.4, 30.8   2048: 49.7, 59.3 / 41.0, 48.9
-        //   8192: 224, 259 / 180, 224      16384: 416, 482 / 330, 412     not in chunks, 1024: 40.7, 43.0 / 29.4, 33.1
+        //   512: 17.8, 20.5 / 17.2, 20.8   768: 27.2, 31.1 / 20.9, 25.4   1024: 30.0, 34.4 / 23.2, 28.4   2048: 49.1, 56.8 / 36.7, 45.0
+        //   8192: 212, 245 / 141, 182      16384: 415, 489 / 275, 368     not in chunks, 1024: 35.2, 38.7 / 26.7, 29.8
         // (and as long as the granules a row may meet leave the LDS for two: uncut sequences of up to 118784 positions)
         const bool pairs = D == 128 && (long long)a.BH * a.NG > 512 && a.spin_limit == DEFAULT_SPIN_LIMIT && (a.chunk_len > 0 || a.NG <= 1856);
         if (rc == MLSTM_ESHAPE && !a.precise && !pairs) rc = launch_row8_kernel(mode, dtype, D, a, st);

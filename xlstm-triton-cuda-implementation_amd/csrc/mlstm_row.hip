@@ -24,18 +24,19 @@
 //            q_i . dQ_i of dD over the keys before the chunk.
 // In split mode the state comes as two terms, hi + lo (one tile each per stage), and takes two MFMAs per fragment.
 //
-// 16-bit tensors at D = 128: two workgroups per CU (256 registers per lane, 66 KB of LDS), so that one of them multiplies while the other waits
-// for its first tiles or writes out.  64 heads x 16384 x 128, forward and dQ pass: 330 and 412 us, one eight-wave workgroup per CU
-// (mlstm_row8.hip) 416 and 482; with what a workgroup does once in whole lines and one trip to memory 283 and 378.  (The figures below are from before that.)
-// Split mode at D = 128: two as well (244 to 256 registers, before 271 to 280 and hence one), forward and dQ pass, us before / after, by workgroups:
-// 384: 34.8, 34.9 / 35.2, 35.7   512: 44.8, 48.6 / 36.5, 38.5   2048: 156, 176 / 125, 136.  At D = 64 its forward missed two by two
-// registers: 432: 21.4 / 16.0   512: 31.8 / 25.2   1416: 54.0 / 38.6   4096: 160 / 116; its dQ pass on registers of one kind 137 / 127.
-// D = 64, dQ pass: three (168 registers) instead of two, us before / after: 18 heads x 1000 21.2 / 17.9, 64 x 1000 25.4 / 21.6,
-// 59 x 3008 40.0 / 34.0, 64 x 8192 117 / 101.  The forward pass takes three in chunks (432 workgroups: 13.7 / 11.6, 4096: 81 / 69, on fewer
-// than one per CU the same) and stays at two where the sequence is not cut, where three lose (18 x 1000: 17.9 / 19.6, 64 x 1000:
-// 20.4 / 22.4); in split mode they lose too (18 x 1000: 21.4 / 23.5).
-// fp32 at D = 64: two (256 registers, before 319 and hence one).  A training step, us before / after: 16 heads x 1000 98.7 / 95.7,
-// 64 x 300 104 / 103, 16 x 4096 240 / 224, 48 x 4096 618 / 555.  At D = 128 the 131 KB of LDS leave room for one.
+// Workgroups per CU, by the registers that a lane may have (heads x positions, us per launch).
+// 16-bit tensors at D = 128: two (256 registers, 66 KB of LDS), so that one of them multiplies while the other waits for its first tiles or writes out.
+// Forward, one / two: 16 x 4096 31.5 / 23.9, 64 x 4096 102 / 70.9, 64 x 16384 406 / 270; the dQ pass keeps to 256 by itself: 29.0, 94.2 and 365.  One eight-wave
+// workgroup per CU (mlstm_row8.hip) takes 415 and 489 at 64 x 16384.
+// Split mode at D = 128: two; forward and dQ pass, one / two: 12 x 4096 38.4, 43.3 / 30.5, 35.1   16 x 4096 44.0, 49.5 / 34.4, 38.9
+// 64 x 4096 146, 173 / 112, 135.
+// Split mode at D = 64: two; forward, one / two / three: 18 x 1000 22.0 / 20.2 / 25.3   18 x 3008 21.1 / 16.1 / 16.7   59 x 3008 51.5 / 35.6 / 36.3   64 x 8192
+// 143 / 89.0 / 84.9; dQ pass 24.5 / 20.8 / 21.5   18.6 / 18.5 / 18.7   41.2 / 40.4 / 38.6   123 / 120 / 118.
+// D = 64: three in the dQ pass (168 registers) and in the forward in chunks, which gain where there are workgroups for them: dQ pass, two / three: 18 x 1000
+// 17.1 / 17.2   64 x 1000 20.6 / 21.4   18 x 3008 15.1 / 14.6   59 x 3008 33.3 / 31.7   64 x 8192 93.1 / 86.2; forward in chunks 18 x 3008 11.4 / 12.1
+// 59 x 3008 26.1 / 26.4   64 x 8192 67.9 / 61.8.  The forward of a sequence that is not cut stays at two: 18 x 1000 16.9 / 20.2, 64 x 1000 20.0 / 22.5.
+// fp32 at D = 64: two; forward and dQ pass, one / two: 16 x 1000 15.5, 17.0 / 15.3, 16.3   64 x 300 23.5, 24.1 / 23.6, 23.6   16 x 4096 32.7, 37.2 / 26.2, 29.5
+// 48 x 4096 91.8, 107 / 64.1, 73.7.  At D = 128 the 131 KB of LDS leave room for one.
 #include <mutex>
 #include <type_traits>
 #include "mlstm_device.h"
@@ -899,7 +900,7 @@ static int launch_row_d(int D, const RowArgs& a, hipStream_t st) {
 
 int launch_row_kernel(int mode, int dtype, int D, const RowArgs& a, hipStream_t st) {
     // fp32 up to one (D = 64) or two (D = 128) workgroups of 32 rows per CU: row_kernel / rowf_kernel, forward, us, in chunks of 128 --
-    //   D = 64    256: 15.7 / 10.3   384: 16.0 / 17.4     D = 128   256: 27.8 / 13.7   512: 28.9 / 25.4   640 (uncut): 36.7 / 36.6   1024: 32.5 / 45.1
+    //   D = 64    256: 14.0 / 10.8   384: 14.3 / 17.4     D = 128   256: 27.6 / 16.9   512: 28.8 / 28.8   640 (uncut): 38.6 / 38.0   1024: 33.1 / 49.5
     if (dtype == MLSTM_F32 && D <= 128 && !g_force_generic && 2ll * a.BH * a.NG <= (D == 64 ? 256 : 512)) return launch_rowf_kernel(mode, D, a, st);
     if (mode == MODE_FWD) {
         switch (dtype) {

@@ -112,9 +112,9 @@ __global__ __launch_bounds__(256 * RB) void roww_kernel(RowArgs a) {
     };
     // The gates of the head's granules up to the rows' own, granule wave + NW k in turn k, are requested first: copies into LDS (the places of
     // their key weights), so that a counted wait can leave the tiles behind them under way while the gates are formed.  (16-bit values one
-    // by one: the dword that holds one reaches beyond the tensor at either of its ends.)  Two launches / one, forward, us: 1 x 64 x 128 7.9 / 6.3, 1 x 320 10.5 / 9.6, 1 x 640 12.9 / 12.9 (a granule is 250
-    // instructions, 100 of them its logarithms, and a workgroup forms all of its head's: 2 us of a CU for ten), 8 x 1000 19.5 / 18.1, 15 x 1001
-    // 22.7 / 19.2, 16 x 256 10.7 / 9.0; D = 256, 1 x 640 15.6 / 15.0, 8 x 1000 24.5 / 22.8, 24 x 1000 31.5 / 29.3, 100 x 128 12.3 / 9.5.
+    // by one: the dword that holds one reaches beyond the tensor at either of its ends.)  Two launches / one, forward, us: 1 x 64 x 128 7.9 / 6.3, 1 x 320 10.9 / 9.7, 1 x 640 13.4 / 13.1 (a granule is 250
+    // instructions, 100 of them its logarithms, and a workgroup forms all of its head's: 2 us of a CU for ten), 8 x 1000 17.7 / 17.6, 15 x 1001
+    // 22.0 / 19.0, 16 x 256 9.9 / 8.3; D = 256, 1 x 640 15.8 / 15.7, 8 x 1000 22.7 / 22.1, 24 x 1000 29.0 / 26.7, 100 x 128 11.6 / 9.2.
     constexpr int NW = NT / 64, TURNS = FUSED ? RW_MOST_KEYS / GRAN / NW : 1;
     if constexpr (FUSED) {
         const size_t off = a.lg.head(bh), ss = (size_t)a.lg.ss;

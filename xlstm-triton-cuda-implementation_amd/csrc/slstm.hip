@@ -78,7 +78,8 @@ __device__ __forceinline__ float pick(bool is0, bool is1, bool is2, float a, flo
 // walk leaves in LDS in the NEXT step, while that waits for h.  With its own stores and ring loads in that place a step issued 28 instructions
 // there, more than the wait hides.
 // Forward, B16 NH4, us, quarters / eighths / helpers: DH = 64, S = 2048 716 / 690 / 613; DH = 128, S = 1024 627 / 559 / 553 (545 without the saved state); DH = 32,
-// S = 1024 285 / 281 / 246.
+// S = 1024 285 / 281 / 246.  DH = 32, eighths / helpers, by workgroups: 256, S = 300 85 / 75; 512, S = 200 70.2 / 71.5 (two on a CU, the helpers of either on a
+// SIMD with a walk of the other); 1024 110 / 84.
 template <int DH>
 struct FwdCfg {
     static constexpr int UW = DH > 64 ? DH / 64 : 1;   // helper waves: a 16-byte piece of a step's input per lane
