@@ -1173,73 +1173,63 @@ __global__ __launch_bounds__(256, 4) void chunk_carry_t_kernel(ChunkArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// The same states in ONE pass: a workgroup owns a 64 x D/2 block of a head's state (64 keys x D/2 values) and walks the
-// head's chunks in their order (forward: first to last; reverse: last to first), the running state in its accumulators:
-// at a chunk's end the block is written in the element type (either layout, the accumulator's own rounding being the
-// only one), decays by gamma, and takes the next chunk's products.  No fp32 chunk sums travel through memory (4 + 4
-// bytes per state element in the two-kernel form above), no second launch.  (D/64) * 2 workgroups per head: for
-// launches with enough heads to fill the chip (launch_chunk_states decides); not in split mode.
+// The same states in ONE pass, bit for bit those of the two kernels above: a workgroup owns 64 keys x VW values of a head's
+// state and walks the head's chunks in their order (forward: first to last; reverse: last to first).  Two sets of
+// accumulators: the chunk's own sum, and the running state that takes it at the chunk's end (state = gamma * state + sum) and is
+// written in the element type.  No fp32 chunk sums travel through memory (4 + 4 bytes per state element in the two-kernel form), no
+// second launch.  WPH workgroups per head; not in split mode; chunk_seq_serves decides.
 //
-// Eight waves.  Waves 4..7 bring the tiles (64 positions: K's 64 columns, V's D/2 columns, and the positions' gate
-// rows) by direct global->LDS copies, PF tiles ahead, into NS = PF + 1 stages; one tile ahead of the product they
-// leave the positions' weights in LDS and add up the vector state from K.  Waves 0..3 multiply straight out of the
-// stages -- the weights go onto the K^T fragments in registers, eight products per fragment (a weighted copy of a
-// tile in LDS costs every wave a chain of LDS round trips per tile, and those chains, not the copies or the MFMAs, set
-// the pace: measured) -- write the states and own every global store.  One barrier per tile.  The copies are counted
-// by hand: a feeder wave issues exactly NI direct loads per tile and no other vector memory operation after the
-// prologue, and waits with vmcnt((PF - 2) * NI) -- everything but the newest PF - 2 tiles -- before the barrier that
-// hands a tile on; the launch is refused if the compiled kernel uses scratch memory.
+// Eight waves, two on every SIMD.  Waves 0..3 multiply straight out of the stages: the positions' weights go onto the V fragments in
+// registers (rounded to the element type as chunk_sum_kernel rounds its weighted V rows); a wave owns 32 values, so that at
+// D = 256 a weighted fragment serves two products.  Operands are requested two contraction steps ahead and weighed one step ahead,
+// across the tiles.  They write the states and own every global store.  Waves 4 and 5 copy: the tiles (64 positions: K's 64
+// columns, V's VW columns) and the positions' gate rows by direct global->LDS loads, the tiles PF ahead into NS = PF + 1 stages, the gate
+// rows one further ahead; and form the positions' weights, two tiles ahead.  Waves 6 and 7 add up the vector state from K.  (All
+// four copying and adding up in turn: a wave sits 600 cycles per tile in the issue of its copies, and what it does behind them came on top,
+// 1900 cycles per tile where the products need 1100.)  One barrier per tile; behind it tiles t and t + 1 and the weights
+// of both are there.  The copies are counted by hand: a copying wave issues exactly NI direct loads per tile and no other vector
+// memory operation, and waits with vmcnt((PF - 2) * NI) -- everything but the newest PF - 2 tiles -- before the barrier
+// that hands a tile on; the launch is refused if the compiled kernel uses scratch memory.
 template <typename T, int D>
 struct SeqCfg {
     static constexpr int KR = 64, VW = D / 2;
-    static constexpr int VP = GRAN * VW * (int)sizeof(T) / 16 / 256;   // direct loads of V per feeder wave and tile
-    static constexpr int NI = 2 + VP + 1;                              // direct loads per feeder wave and tile: K, V, one gate row
+    static constexpr int NKB = VW / 64;                                // key blocks of a multiplying wave
+    static constexpr int KP = GRAN * KR * (int)sizeof(T) / 16 / 128, VP = GRAN * VW * (int)sizeof(T) / 16 / 128;   // direct loads per copying wave and tile: K, V
+    static constexpr int NI = KP + VP + 2;                             // ... and two gate rows
     static constexpr int MAX_STEPS = 256;                              // chunk states per head
+    static constexpr int NPG = 2048 / D;                               // groups of rows of the vector sum (as in chunk_sum_kernel)
     static constexpr size_t K_BYTES = (size_t)GRAN * KR * sizeof(T), V_BYTES = (size_t)GRAN * VW * sizeof(T), AUX_BYTES = 4 * GRAN * sizeof(float);
     static constexpr size_t STAGE_BYTES = K_BYTES + V_BYTES + AUX_BYTES;
+    static constexpr size_t SW_BYTES = 4 * 2 * GRAN * sizeof(float);   // [tile modulo 4][matrix, vector][position]
+    static constexpr size_t RED_BYTES = 2 * NPG * 32 * sizeof(float);  // [parity of the step][group][key]
     static constexpr size_t TABLE_BYTES = MAX_STEPS * (sizeof(double) + 2 * sizeof(float));
-    static constexpr size_t RED_BYTES = 32 * KR * sizeof(float) + 64;
-    static constexpr size_t SW_BYTES = 8 * GRAN * sizeof(float);
+    static constexpr size_t FIXED_BYTES = SW_BYTES + RED_BYTES + TABLE_BYTES;
     // tiles requested ahead: as many stages as LDS holds
-    static constexpr int NS = (int)((160 * 1024 - TABLE_BYTES - RED_BYTES - SW_BYTES) / STAGE_BYTES) < 8
-                                  ? (int)((160 * 1024 - TABLE_BYTES - RED_BYTES - SW_BYTES) / STAGE_BYTES) : 8;
-    static constexpr int PF = NS - 1;
-    static_assert(PF >= 3 && (PF - 1) * NI < 64, "the counted wait must fit vmcnt's six bits");
-    static constexpr size_t LDS_BYTES = NS * STAGE_BYTES + SW_BYTES + TABLE_BYTES + RED_BYTES;
-    static constexpr int WPH = (D / KR) * 2;                           // workgroups per head
+    static constexpr int FIT = (int)((160 * 1024 - FIXED_BYTES) / STAGE_BYTES), NS = FIT < 8 ? FIT : 8, PF = NS - 1;
+    static_assert(PF >= 3 && (PF - 2) * NI < 64, "the counted wait must fit vmcnt's six bits");
+    static constexpr size_t LDS_BYTES = NS * STAGE_BYTES + FIXED_BYTES;
+    static constexpr int WPH = (D / KR) * (D / VW);                    // workgroups per head
 };
 
-// cycle stamps of the one-pass kernel's two kinds of waves (a measurement build only: -DMLSTM_SEQ_PROF; the sums go to
-// the unused chunk-sum scratch, 16 floats per workgroup)
-#if defined(MLSTM_SEQ_PROF)
-#define SQ_DECL float prof_[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}; long long last_ = (long long)__builtin_amdgcn_s_memtime()
-#define SQ_STAMP(k) do { const long long now_ = (long long)__builtin_amdgcn_s_memtime(); prof_[k] += (float)(now_ - last_); last_ = now_; } while (0)
-#define SQ_DUMP(kind) do { if ((threadIdx.x & 255) == 0) for (int z_ = 0; z_ < 8; z_++) a.dC[(size_t)blockIdx.x * 16 + 8 * (kind) + z_] = prof_[z_]; } while (0)
-#else
-#define SQ_DECL do {} while (0)
-#define SQ_STAMP(k) do {} while (0)
-#define SQ_DUMP(kind) do {} while (0)
-#endif
-
-template <typename T, int D, bool DOT>
+// KM, VM: key-major and value-major states are written (ChunkArgs::Cst, CstT); DOT: the contraction with another set on the way
+template <typename T, int D, bool KM, bool VM, bool DOT>
 __global__ __launch_bounds__(512) void chunk_seq_kernel(ChunkArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using R = Tr<T>;
     using Cfg = SeqCfg<T, D>;
     typedef typename R::frag frag;
+    typedef typename R::vec4 V4;
     static_assert(R::HALF && (D == 128 || D == 256), "16-bit types, D = 128 or 256");
-    constexpr int VW = Cfg::VW, NB = VW / 64, KW = R::KW, NS = Cfg::NS, PF = Cfg::PF, NI = Cfg::NI, VP = Cfg::VP;
+    constexpr int VW = Cfg::VW, NKB = Cfg::NKB, KW = R::KW, NS = Cfg::NS, PF = Cfg::PF, NI = Cfg::NI, NPG = Cfg::NPG;
+    constexpr int SB = (int)Cfg::STAGE_BYTES, KB = (int)Cfg::K_BYTES, AUX = (int)(Cfg::K_BYTES + Cfg::V_BYTES);
     using ZK = Swz<T, 64>;
+    using ZV = Swz<T, VW>;
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    float* const sw = reinterpret_cast<float*>(smem + NS * Cfg::STAGE_BYTES);   // [4][2][64]: the weights of two tiles, a copy per multiplying wave
-    double* const tGend = reinterpret_cast<double*>(sw + 8 * GRAN);
+    float* const sw = reinterpret_cast<float*>(smem + NS * SB);     // [4][2][64]
+    float* const red = sw + 4 * 2 * GRAN;                           // [2][NPG][32]
+    double* const tGend = reinterpret_cast<double*>(red + 2 * NPG * 32);
     float* const tbend = reinterpret_cast<float*>(tGend + Cfg::MAX_STEPS);
     float* const tgam = tbend + Cfg::MAX_STEPS;
-    float* const red = tgam + Cfg::MAX_STEPS;     // [32][64]: the feeders' partial vector sums of a chunk
-    float* const dotred = red + 32 * 64;          // [4]
-    auto stage_k = [&](int st) { return reinterpret_cast<T*>(smem + st * Cfg::STAGE_BYTES); };
-    auto stage_v = [&](int st) { return reinterpret_cast<T*>(smem + st * Cfg::STAGE_BYTES + Cfg::K_BYTES); };
-    auto stage_aux = [&](int st) { return reinterpret_cast<float*>(smem + st * Cfg::STAGE_BYTES + Cfg::K_BYTES + Cfg::V_BYTES); };
 
     const bool feeder = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 8) != 0;
     const int tid = threadIdx.x & 255, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5, c32 = lane & 31;
@@ -1255,278 +1245,370 @@ __global__ __launch_bounds__(512) void chunk_seq_kernel(ChunkArgs a) {
     // the first, the sequence's last chunk, may be short
     const int NT0 = rev ? (S - NCS * L + GRAN - 1) / GRAN : NT;
     const int NTOT = NT0 + (NCS - 1) * NT;
+    auto state_of = [&](int s) { return rev ? NCS - 1 - s : s; };
     auto step_base = [&](int s) { return rev ? (NCS - s) * L : s * L; };
-    auto step_tiles = [&](int s) { return s == 0 ? NT0 : NT; };
-    struct Cur {   // a tile of the walk
-        int s, tt;
-    };
-    auto advance = [&](Cur& c) { if (++c.tt == step_tiles(c.s)) { c.tt = 0; c.s++; } };
-
-    // per-step tables, by everybody: reference exponent of the step's weights and the decay between steps
+    // per step: the reference exponent of its weights and the decay into it
     for (int s = threadIdx.x; s < NCS; s += 512) {
-        const int c = rev ? NCS - 1 - s : s;
-        const int pe = (c + 1) * L - 1;   // forward: the chunk's last position; reverse: the last position before the chunk
+        const int c = state_of(s), pe = (c + 1) * L - 1;   // forward: the chunk's last position; reverse: the last position before the chunk
         tbend[s] = a.beta2[poff + pe];
         tGend[s] = a.G2[goff + pe / GRAN];
         tgam[s] = s > 0 ? carry_gamma(a, poff, goff, rev ? c + 1 : c) : 0.f;
     }
-    const float log2scale = -0.5f * __log2f((float)D);
-    const size_t rsK = (size_t)a.lk.ss, rsV = (size_t)a.lv.ss;
-    const T* Kh = reinterpret_cast<const T*>(a.K) + a.lk.head(bh) + 64 * kq;
-    const T* Vh = reinterpret_cast<const T*>(a.V) + a.lv.head(bh) + VW * vh;
-    dma_wait();        // (the last plain loads of the feeder waves: from here on their vmcnt counts direct loads only)
-    __syncthreads();
 
-    if (feeder) {
-        TileDma<T, 64, GRAN, 256> kdma;
-        TileDma<T, VW, GRAN, 256> vdma;
+    // Places in the walk, each advanced tile by tile: the step, how many of its tiles are left (this one included), the stage (bytes), and what
+    // its user needs of the position.  Between steps only the reverse walk jumps, from the end of a chunk to the start of the one before.
+    const int jump0 = -(NT0 * GRAN + L), jump = -(NT * GRAN + L);   // (the first step may be a short one)
+    struct Place { int s, left, st; };
+    const Place start{0, NT0, 0};
+    auto next = [&](Place& c, auto&& jumped) __attribute__((always_inline)) {
+        c.st = c.st == (NS - 1) * SB ? 0 : c.st + SB;
+        if (__builtin_expect(--c.left == 0, 0)) {
+            if (rev) jumped(c.s == 0 ? jump0 : jump);
+            c.s++;
+            c.left = NT;
+        }
+    };
+    if (feeder && wave < 2) {   // ---- copies
+        const size_t rsK = (size_t)a.lk.ss, rsV = (size_t)a.lv.ss;
+        const T* Kh = reinterpret_cast<const T*>(a.K) + a.lk.head(bh) + 64 * kq;
+        const T* Vh = reinterpret_cast<const T*>(a.V) + a.lv.head(bh) + VW * vh;
+        TileDma<T, 64, GRAN, 128> kdma;
+        TileDma<T, VW, GRAN, 128> vdma;
         kdma.init(tid);
         vdma.init(tid);
         const auto krows = kdma.rows(tid, (unsigned)(rsK * sizeof(T)));
         const auto vrows = vdma.rows(tid, (unsigned)(rsV * sizeof(T)));
-        static_assert(TileDma<T, 64, GRAN, 256>::PER_WAVE == 2 && TileDma<T, VW, GRAN, 256>::PER_WAVE == VP, "direct loads per tile");
-        // gate rows of a tile: wave 0 alpha (forward) or beta (reverse), waves 1 and 2 the dQ pass's 1/n and db (reverse; the
-        // forward repeats alpha), wave 3 the granule's G (two dwords; the other lanes read them again)
-        const float* auxsrc;
-        if (wave == 3) auxsrc = reinterpret_cast<const float*>(a.G2 + goff) + (lane & 1);
-        else if (!rev || wave == 0) auxsrc = (rev ? a.beta2 : a.alpha2) + poff + lane;
-        else auxsrc = (wave == 1 ? a.inv_n : a.db) + poff + lane;
-        const int auxstep = wave == 3 ? 2 : GRAN;   // floats per tile
-        auto issue = [&](const Cur& c, int st) __attribute__((always_inline)) {
-            const int pos0 = step_base(c.s) + GRAN * c.tt;
-            if (pos0 + GRAN <= S) {
-                kdma.issue(stage_k(st), Kh + (size_t)pos0 * rsK, krows);
-                vdma.issue(stage_v(st), Vh + (size_t)pos0 * rsV, vrows);
+        static_assert(TileDma<T, 64, GRAN, 128>::PER_WAVE == Cfg::KP && TileDma<T, VW, GRAN, 128>::PER_WAVE == Cfg::VP, "direct loads per tile");
+        // gate rows of a tile: 0 alpha (forward) or beta (reverse), 1 and 2 the dQ pass's 1/n and db (reverse; the forward repeats
+        // alpha), 3 the granule's G (two dwords; the other lanes read them again).  Wave 0 brings rows 0 and 1, wave 1 rows 2 and 3.
+        const float* const row0 = (rev ? a.beta2 : a.alpha2) + poff + lane;
+        const float* ap0 = wave == 0 ? row0 : (rev ? a.db + poff + lane : row0);
+        const float* ap1 = wave == 0 ? (rev ? a.inv_n + poff + lane : row0) : reinterpret_cast<const float*>(a.G2 + goff) + (lane & 1);
+        const int ap1step = wave == 0 ? GRAN : 2;   // floats per tile
+        dma_wait();   // (from here on this wave's vmcnt counts direct loads only)
+
+        Place pi = start, pa = start, pw = start;   // the next tile to request, the next gate rows, the next tile to form weights for
+        int pos_i = step_base(0), pos_w = pos_i;
+        const T* kp = Kh + (size_t)pos_i * rsK;
+        const T* vp = Vh + (size_t)pos_i * rsV;
+        ap0 += pos_i;
+        ap1 += pos_i / GRAN * ap1step;
+        const size_t kstep = GRAN * rsK, vstep = GRAN * rsV;
+        auto next_i = [&]() __attribute__((always_inline)) {
+            pos_i += GRAN; kp += kstep; vp += vstep;
+            next(pi, [&](int d) { pos_i += d; kp += (long long)d * (long long)rsK; vp += (long long)d * (long long)rsV; });
+        };
+        auto next_a = [&]() __attribute__((always_inline)) {
+            ap0 += GRAN; ap1 += ap1step;
+            next(pa, [&](int d) { ap0 += d; ap1 += d / GRAN * ap1step; });
+        };
+        auto issue_aux = [&]() __attribute__((always_inline)) {
+            const unsigned to = __builtin_amdgcn_readfirstlane(lds_offset_of(smem + pa.st + AUX)) + wave * 512;
+            dma4(ap0, to);
+            dma4(ap1, to + 256);
+        };
+        auto issue = [&]() __attribute__((always_inline)) {
+            T* const ks = reinterpret_cast<T*>(smem + pi.st);
+            T* const vs = reinterpret_cast<T*>(smem + pi.st + KB);
+            if (__builtin_expect(pos_i + GRAN <= S, 1)) {
+                kdma.issue(ks, kp, krows);
+                vdma.issue(vs, vp, vrows);
             } else {   // the sequence's last tile: rows past the end are clamped (their weights are 0)
-                tile_dma<T, 64, GRAN, 256>(stage_k(st), Kh, pos0, S, tid, rsK);
-                tile_dma<T, VW, GRAN, 256>(stage_v(st), Vh, pos0, S, tid, rsV);
-            }
-            dma4(auxsrc + (size_t)(pos0 / GRAN) * auxstep, __builtin_amdgcn_readfirstlane(lds_offset_of(stage_aux(st))) + wave * 256);
-        };
-        // Tile c (landed in stage st, published by a barrier): the vector sum from K, two 16-byte pieces per thread (rows
-        // tid / 8 and tid / 8 + 32), in the workgroups that own it
-        f32x8 nacc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        const int prow = tid / ZK::CPR, pch = tid % ZK::CPR;
-        auto prepare = [&](const Cur& c, int st) __attribute__((always_inline)) {
-            if (vh != 0) return;
-            const float* ax = stage_aux(st);
-            const int pos0 = step_base(c.s) + GRAN * c.tt;
-            const float bend = tbend[c.s];
-            const float dG = (float)(rev ? *reinterpret_cast<const double*>(ax + 3 * GRAN) - tGend[c.s]
-                                         : tGend[c.s] - *reinterpret_cast<const double*>(ax + 3 * GRAN));
-            u32x4 raw[2];
-            if (vh == 0) {
-#pragma unroll
-                for (int it = 0; it < 2; it++) raw[it] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(stage_k(st)) + ZK::off(prow + 32 * it, 8 * pch));
-            }
-#pragma unroll
-            for (int it = 0; it < 2; it++) {
-                const int row = prow + 32 * it;
-                const float e = rev ? bend - ax[row] : ax[row] - bend;
-                float rho = fast_exp2(e + dG + log2scale);
-                if (pos0 + row >= S) rho = 0.f;
-                const float w2 = rev ? rho * ax[2 * GRAN + row] : rho;
-                {
-                    float x[8];
-                    unpack8<T>(raw[it], x);
-#pragma unroll
-                    for (int e8 = 0; e8 < 8; e8++) nacc[e8] += x[e8] * w2;
-                }
-            }
-            if (vh == 0 && c.tt == step_tiles(c.s) - 1) {   // the step's last tile: the partial sums go to the multiplying waves
-                *reinterpret_cast<f32x8*>(red + prow * 64 + 8 * pch) = nacc;
-#pragma unroll
-                for (int e8 = 0; e8 < 8; e8++) nacc[e8] = 0.f;
+                tile_dma_rolled<T, 64, GRAN, 128>(ks, Kh, pos_i, S, tid, rsK);
+                tile_dma_rolled<T, VW, GRAN, 128>(vs, Vh, pos_i, S, tid, rsV);
             }
         };
-        Cur ci{0, 0}, ct{0, 0};   // the next tile to request, the next one to prepare
-#pragma unroll
-        for (int p = 0; p < PF; p++)
-            if (p < NTOT) { issue(ci, p % NS); advance(ci); }
-        if (NTOT >= PF) dma_wait_but<(PF - 1) * NI>(); else dma_wait();
-        __syncthreads();   // tile 0 has landed
-        prepare(ct, 0);
-        advance(ct);
-        if (NTOT >= PF) dma_wait_but<(PF - 2) * NI>(); else dma_wait();
-        __syncthreads();   // tile 1 has landed
-        SQ_DECL;
-        for (int t = 0; t < NTOT; t++) {
-            if (t + PF < NTOT) { issue(ci, (t + PF) % NS); advance(ci); }
-            SQ_STAMP(0);
-            if (t + 1 < NTOT) { prepare(ct, (t + 1) % NS); advance(ct); }
-            SQ_STAMP(1);
-            if (t + PF < NTOT) dma_wait_but<(PF - 2) * NI>(); else dma_wait();
-            SQ_STAMP(2);
-            __syncthreads();
-            SQ_STAMP(3);
+        // the positions' weights of tile n (see chunk_sum_kernel), by the two waves in turns
+        const float log2scale = -0.5f * __log2f((float)D);
+        struct Gate { float x0, x1, x2, bend; double xg, Gend; } g{};
+        auto gate_rows = [&]() __attribute__((always_inline)) {
+            const float* const ax = reinterpret_cast<const float*>(smem + pw.st + AUX);
+            g = Gate{ax[lane], ax[GRAN + lane], ax[2 * GRAN + lane], tbend[pw.s], *reinterpret_cast<const double*>(ax + 3 * GRAN), tGend[pw.s]};
+        };
+        auto weigh = [&](int n) __attribute__((always_inline)) {
+            float wm, w2;
+            if (rev) {
+                const float rho = fast_exp2(g.bend - g.x0 + (float)(g.xg - g.Gend) + log2scale);
+                wm = rho * g.x1;
+                w2 = rho * g.x2;
+            } else {
+                wm = w2 = fast_exp2(g.x0 - g.bend + (float)(g.Gend - g.xg) + log2scale);
+            }
+            if (pos_w + lane >= S) wm = w2 = 0.f;
+            float* const o = sw + (n & 3) * 2 * GRAN + lane;
+            o[0] = wm;
+            o[GRAN] = w2;
+        };
+        auto next_w = [&]() __attribute__((always_inline)) {
+            pos_w += GRAN;
+            next(pw, [&](int d) { pos_w += d; });
+        };
+        issue_aux();
+        next_a();
+        int t = 0;
+        for (; t < PF && t < NTOT; t++) {   // (behind the last tile its own gate rows again: the count stays the same)
+            issue();
+            next_i();
+            issue_aux();
+            if (t + 2 < NTOT) next_a();
         }
-        SQ_DUMP(0);
+        __syncthreads();   // the tables are there
+        if (NTOT >= PF) dma_wait_but<(PF - 2) * NI>(); else dma_wait();
+        __syncthreads();   // tiles 0 and 1 have landed, and the gate rows up to tile 2
+        if (wave == 0) { gate_rows(); weigh(0); }
+        next_w();
+        if (NTOT > 1) {
+            if (wave == 1) { gate_rows(); weigh(1); }
+            next_w();
+        }
+        __syncthreads();   // their weights are there
+        for (t = 0; t < NTOT; t++) {
+            const bool more = t + PF < NTOT, ahead = t + 2 < NTOT, mine = wave == (t & 1);
+            if (ahead && mine) gate_rows();
+            __builtin_amdgcn_sched_barrier(0);
+            if (more) {   // (into the stage of tile t - 1)
+                issue();
+                next_i();
+                issue_aux();
+                if (t + PF + 2 < NTOT) next_a();
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (ahead) {
+                if (mine) weigh(t + 2);
+                next_w();
+            }
+            if (more) dma_wait_but<(PF - 2) * NI>(); else dma_wait();
+            __syncthreads();   // tile t + 2 has landed
+        }
+    } else if (feeder) {   // ---- the vector state
+        const int ft = tid - 128;
+        Place pv = start;   // the tile to add up
+        // The vector sum of the workgroup's half of its 64 keys, in the order of chunk_sum_kernel: NPG partial sums per key, each over
+        // every NPG-th row.  A lane takes KPL keys of one group of rows.
+        constexpr int KPL = NPG / 4, RPT = GRAN / NPG;   // keys per lane, rows per lane and tile
+        typedef T KVec __attribute__((ext_vector_type(KPL)));
+        const int kl = KPL * (ft % (32 / KPL)), pg = ft / (32 / KPL);
+        float nacc[KPL];
+#pragma unroll
+        for (int e = 0; e < KPL; e++) nacc[e] = 0.f;
+        __syncthreads();   // the tables are there
+        __syncthreads();   // tiles 0 and 1 have landed, and the gate rows up to tile 2
+        __syncthreads();   // their weights are there
+        KVec x[RPT], xn[RPT];
+        float wr[RPT], wn[RPT];
+        auto request = [&](int st, int t) __attribute__((always_inline)) {   // (stage in bytes)
+#pragma unroll
+            for (int it = 0; it < RPT; it++) {
+                xn[it] = *reinterpret_cast<const KVec*>(smem + st + ZK::off(pg + NPG * it, 32 * vh + kl));
+                wn[it] = sw[(t & 3) * 2 * GRAN + GRAN + pg + NPG * it];
+            }
+        };
+        request(0, 0);
+        for (int t = 0; t < NTOT; t++) {
+#pragma unroll
+            for (int it = 0; it < RPT; it++) { x[it] = xn[it]; wr[it] = wn[it]; }
+            request(pv.st == (NS - 1) * SB ? 0 : pv.st + SB, t + 1);   // (behind the sequence's last tile what lies there, unused)
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int it = 0; it < RPT; it++)
+#pragma unroll
+                for (int e = 0; e < KPL; e++) nacc[e] = fmaf((float)x[it][e], wr[it], nacc[e]);
+            if (__builtin_expect(pv.left == 1, 0)) {   // the step's last tile: the partial sums go to a multiplying wave
+                float* const r = red + ((pv.s & 1) * NPG + pg) * 32 + kl;
+#pragma unroll
+                for (int e = 0; e < KPL; e++) { r[e] = nacc[e]; nacc[e] = 0.f; }
+            }
+            next(pv, [](int) {});
+            __syncthreads();
+        }
     } else {
-        const int wk = wave & 1, wv = wave >> 1;
-        f32x16 acc[NB];
+        const int wv = NKB == 2 ? wave : wave >> 1, wk = NKB == 2 ? 0 : wave & 1;   // the wave's 32 values; its (first) 32 keys
+        f32x16 acc[NKB], run[NKB];
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++)
+        for (int kb = 0; kb < NKB; kb++)
 #pragma unroll
-            for (int x = 0; x < 16; x++) acc[nb][x] = 0.f;
-        float nrun = 0.f;
-        Cur cm{0, 0};
-        __syncthreads();
-        __syncthreads();
-        int pending_dot = -1;   // state whose contraction's parts lie in dotred
-        // per-lane byte offsets of the transposing reads (see swz_frag_transposed), contraction step s4 = 0: K block wk and
-        // V blocks NB wv + nb; a step further lies 16 tile rows on (the swizzle key has a period of 16 rows)
+            for (int x = 0; x < 16; x++) { acc[kb][x] = 0.f; run[kb][x] = 0.f; }
+        // per-lane byte offsets of the transposing reads (see swz_frag_transposed), contraction step 0; a step further lies 16 tile rows
+        // on (the swizzle key has a period of 16 rows)
         const int tj = lane & 15, tsub = (lane >> 4) & 1;
-        int koff[2], voff[NB][2];
+        int koff[NKB][2], voff[2];
 #pragma unroll
         for (int hi = 0; hi < 2; hi++) {
-            koff[hi] = ZK::off(4 * h + (tj >> 2) + 8 * hi, 32 * wk + 16 * tsub + 4 * (tj & 3));
 #pragma unroll
-            for (int nb = 0; nb < NB; nb++) voff[nb][hi] = Swz<T, VW>::off(4 * h + (tj >> 2) + 8 * hi, 32 * (NB * wv + nb) + 16 * tsub + 4 * (tj & 3));
+            for (int kb = 0; kb < NKB; kb++) koff[kb][hi] = ZK::off(4 * h + (tj >> 2) + 8 * hi, 32 * (wk + kb) + 16 * tsub + 4 * (tj & 3));
+            voff[hi] = ZV::off(4 * h + (tj >> 2) + 8 * hi, 32 * wv + 16 * tsub + 4 * (tj & 3));
         }
-        auto read_tr = [&](const T* tile, const int (&off)[2], int row_bytes, int s4) __attribute__((always_inline)) {
-            const char* base = reinterpret_cast<const char*>(tile) + KW * s4 * row_bytes;
+        auto read_tr = [&](const char* base, const int (&off)[2]) __attribute__((always_inline)) {
             s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_PTR(s16x4))(base + off[0]));
             s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_PTR(s16x4))(base + off[1]));
             return __builtin_bit_cast(frag, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
         };
-        float* const wt = sw + wave * 2 * GRAN;   // this wave's copies of two tiles' weights
-        // the weight of position `lane` of tile c (in stage st) into the wave's copy wb: written and read in program order
-        auto weigh = [&](const Cur& c, int st, int wb) __attribute__((always_inline)) {
-            const float* ax = stage_aux(st);
-            const int pos0 = step_base(c.s) + GRAN * c.tt;
-            const float dG = (float)(rev ? *reinterpret_cast<const double*>(ax + 3 * GRAN) - tGend[c.s]
-                                         : tGend[c.s] - *reinterpret_cast<const double*>(ax + 3 * GRAN));
-            const float e = rev ? tbend[c.s] - ax[lane] : ax[lane] - tbend[c.s];
-            float rho = fast_exp2(e + dG + log2scale);
-            if (pos0 + lane >= S) rho = 0.f;
-            wt[wb * GRAN + lane] = rev ? rho * ax[GRAN + lane] : rho;
-        };
         constexpr int NSTEP = GRAN / KW;
-        frag af[2], bf[2][NB];
-        f32x4 w0[2], w1[2];
-        // fragment s4 of K^T holds, for the lane's key, positions 16 s4 + 4 h + (0..3) and 16 s4 + 8 + 4 h + (0..3)
-        auto rd = [&](int tile, int s4) __attribute__((always_inline)) {
-            const T* kt = stage_k(tile % NS);
-            const T* vt = stage_v(tile % NS);
-            const float* wv4 = wt + (tile & 1) * GRAN + KW * s4;
-            af[s4 & 1] = read_tr(kt, koff, ZK::ROW_BYTES, s4);
-            w0[s4 & 1] = *reinterpret_cast<const f32x4*>(wv4 + 4 * h);
-            w1[s4 & 1] = *reinterpret_cast<const f32x4*>(wv4 + 8 + 4 * h);
-#pragma unroll
-            for (int nb = 0; nb < NB; nb++) bf[s4 & 1][nb] = read_tr(vt, voff[nb], Swz<T, VW>::ROW_BYTES, s4);
+        static_assert(NSTEP == 4, "two registers of weights");
+        frag kf[NSTEP][NKB], vf[NSTEP], vw;
+        // The weights of a tile in two registers: a V fragment holds, for the lane's value, positions 16 s4 + 4 h + (0..3) and
+        // 16 s4 + 8 + 4 h + (0..3) as elements 0..7, and element e of step s4 finds its weight in lane 8 (s4 & 1) + e of its row of 16
+        // lanes, register s4 / 2 (one DPP operand; as two 16-byte reads per step the weights were a third of all LDS traffic).
+        const int wl = lane & 15, wpos = 16 * (wl >> 3) + 4 * h + (wl & 3) + 8 * ((wl >> 2) & 1);
+        float wr[2], wnext[2];
+        auto request_weights = [&](int t) __attribute__((always_inline)) {
+            const float* const wp = sw + (t & 3) * 2 * GRAN + wpos;
+            wnext[0] = wp[0];
+            wnext[1] = wp[32];
         };
-        // The reads of a tile's first step, and its weights, are requested during the tile before it (both tiles are
-        // published by then): a tile's product is a chain of LDS round trips, and with one barrier per tile nothing else
-        // would cover them.
-        Cur cn{0, 0};   // the tile whose weights are formed next
-        weigh(cn, 0, 0);
-        advance(cn);
-        rd(0, 0);
-        SQ_DECL;
-        for (int t = 0; t < NTOT; t++) {
-            if (t + 1 < NTOT) { weigh(cn, (t + 1) % NS, (t + 1) & 1); advance(cn); }
-            if (DOT && pending_dot >= 0 && tid == 0) {
-                a.dot_part[((size_t)bh * NCS + pending_dot) * Cfg::WPH + w] = (dotred[0] + dotred[1]) + (dotred[2] + dotred[3]);
+        auto request = [&](int st, int s4) __attribute__((always_inline)) {   // the operands of contraction step s4 of the tile in stage st
+            const char* const ks = smem + st * SB;
+            vf[s4] = read_tr(ks + KB + KW * s4 * ZV::ROW_BYTES, voff);
+#pragma unroll
+            for (int kb = 0; kb < NKB; kb++) kf[s4][kb] = read_tr(ks + KW * s4 * ZK::ROW_BYTES, koff[kb]);
+        };
+        auto weighed = [&](auto s4_tag, const float (&wt)[2]) __attribute__((always_inline)) {
+            constexpr int s4 = decltype(s4_tag)::value, l0 = 8 * (s4 & 1);
+            float x[8];
+            unpack8<T>(__builtin_bit_cast(u32x4, vf[s4]), x);
+            const float wv4 = wt[s4 >> 1];
+            auto weight = [&](auto e) __attribute__((always_inline)) {   // row_newbcast
+                return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, wv4), 0x150 + l0 + decltype(e)::value, 0xf, 0xf, true));
+            };
+            static_for<8>([&](auto e) __attribute__((always_inline)) { x[decltype(e)::value] *= weight(e); });
+            struct Pair { V4 lo, hi; } p;
+            p.lo = R::cvt4(f32x4{x[0], x[1], x[2], x[3]});
+            p.hi = R::cvt4(f32x4{x[4], x[5], x[6], x[7]});
+            return __builtin_bit_cast(frag, p);
+        };
+        const int vg = VW * vh + 32 * wv + c32;        // the lane's value
+        const int krow0 = 64 * kq + 32 * wk + 8 * h;   // state row of its first key: that of key 32 kb + 8 g4 + 4 h lies 32 kb + 16 (g4 / 2) + 4 (g4 % 2) on
+        const size_t hbase = (size_t)bh * NCS * D * D, toff = hbase + (size_t)state_row(vg) * D + 64 * kq + 32 * wk + 4 * h;
+        const unsigned odd = lane & 1, sel = odd ? 0x03020706u : 0x05040100u;
+        T* const dst_t = reinterpret_cast<T*>(a.CstT) + toff;
+        T* const dst_k = reinterpret_cast<T*>(a.Cst) + hbase + (size_t)(krow0 + odd) * D + (vg & ~1);
+        const T* const other = reinterpret_cast<const T*>(a.dot_with) + toff;
+        V4 y[DOT ? NKB : 1][4];
+        float nrun = 0.f;
+        auto carry_vector = [&](int s) __attribute__((always_inline)) {   // by one wave, behind the barrier that follows the step's last tile
+            float sum = 0.f;
+#pragma unroll
+            for (int g = 0; g < NPG; g++) sum += red[((s & 1) * NPG + g) * 32 + c32];
+            nrun = nrun * tgam[s] + sum;
+            if (h == 0) a.Nst[((size_t)bh * NCS + state_of(s)) * D + 64 * kq + 32 * vh + c32] = nrun;
+        };
+        __syncthreads();
+        __syncthreads();
+        __syncthreads();   // tiles 0 and 1 have landed and their weights are there
+        request(0, 0);
+        request(0, 1);
+        request_weights(0);
+        wr[0] = wnext[0]; wr[1] = wnext[1];
+        vw = weighed(std::integral_constant<int, 0>{}, wr);
+        int st = 0, t = 0;
+        for (int s = 0; s < NCS; s++) {
+            const int nt = s == 0 ? NT0 : NT;
+            const size_t so = (size_t)state_of(s) * D * D;
+            if (s > 0 && wave == 3) carry_vector(s - 1);
+            if constexpr (DOT) {   // (used at the end of the step)
+#pragma unroll
+                for (int kb = 0; kb < NKB; kb++)
+#pragma unroll
+                    for (int g4 = 0; g4 < 4; g4++) y[kb][g4] = *reinterpret_cast<const V4*>(other + so + 32 * kb + 8 * g4);
             }
-            pending_dot = -1;
+            for (int tt = 0; tt < nt; tt++) {
+                const int stn = st + 1 == NS ? 0 : st + 1;
+                static_for<NSTEP>([&](auto tag) __attribute__((always_inline)) {
+                    constexpr int s4 = decltype(tag)::value;
+                    // (behind the sequence's last tile what lies in the next stage, unused)
+                    if constexpr (s4 + 2 < NSTEP) {
+                        request(st, s4 + 2);
+                    } else {
+                        if constexpr (s4 + 2 == NSTEP) request_weights(t + 1);
+                        request(stn, s4 + 2 - NSTEP);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int s4 = 0; s4 < NSTEP; s4++) {
-                if (s4 + 1 < NSTEP) rd(t, s4 + 1);
-                else if (t + 1 < NTOT) rd(t + 1, 0);
-                float x[8];
-                unpack8<T>(__builtin_bit_cast(u32x4, af[s4 & 1]), x);
-                const f32x4 lo = f32x4{x[0], x[1], x[2], x[3]} * w0[s4 & 1], hi = f32x4{x[4], x[5], x[6], x[7]} * w1[s4 & 1];
-                typedef typename R::vec4 V4;
-                struct Pair { V4 lo, hi; } wa{R::cvt4(lo), R::cvt4(hi)};
-                const frag aw = __builtin_bit_cast(frag, wa);
+                    for (int kb = 0; kb < NKB; kb++) R::mma(acc[kb], kf[s4][kb], vw);
+                    if constexpr (s4 + 1 < NSTEP) vw = weighed(std::integral_constant<int, s4 + 1>{}, wr);
+                    else vw = weighed(std::integral_constant<int, 0>{}, wnext);
+                    __builtin_amdgcn_sched_barrier(0);
+                });
+                wr[0] = wnext[0]; wr[1] = wnext[1];
+                if (tt == nt - 1) {   // the step's state leaves
+                    const float gam = tgam[s];
 #pragma unroll
-                for (int nb = 0; nb < NB; nb++) R::mma(acc[nb], aw, bf[s4 & 1][nb]);
-            }
-            SQ_STAMP(0);
-            if (cm.tt == step_tiles(cm.s) - 1) {   // the step's last tile: state c leaves, the running state decays
-                const int c = rev ? NCS - 1 - cm.s : cm.s;
-                const size_t sbase = ((size_t)bh * NCS + c) * D * D;
-                float dot = 0.f;
+                    for (int kb = 0; kb < NKB; kb++) {
+                        run[kb] = run[kb] * gam + acc[kb];
 #pragma unroll
-                for (int nb = 0; nb < NB; nb++) {
-                    const int vg = VW * vh + 32 * (NB * wv + nb) + c32;
-                    const size_t vrow_off = sbase + (size_t)state_row(vg) * D;
-#pragma unroll
-                    for (int g4 = 0; g4 < 4; g4++) {
-                        const int kg = 64 * kq + 32 * wk + 8 * g4 + 4 * h;
-                        const typename R::vec4 hi = R::cvt4(f32x4{acc[nb][4 * g4], acc[nb][4 * g4 + 1], acc[nb][4 * g4 + 2], acc[nb][4 * g4 + 3]});
-                        if (a.CstT) *reinterpret_cast<typename R::vec4*>(reinterpret_cast<T*>(a.CstT) + vrow_off + kg) = hi;
-                        if (a.Cst) {
-#pragma unroll
-                            for (int e = 0; e < 4; e++) reinterpret_cast<T*>(a.Cst)[sbase + (size_t)state_row(kg + e) * D + vg] = hi[e];
+                        for (int x = 0; x < 16; x++) {
+                            asm volatile("" : "+v"(run[kb][x]));   // (see chunk_carry_t_kernel: the fp32 value is fixed before any conversion)
+                            acc[kb][x] = 0.f;
                         }
-                        if constexpr (DOT) {
-                            const f32x4 o = __builtin_convertvector(*reinterpret_cast<const typename R::vec4*>(reinterpret_cast<const T*>(a.dot_with) + vrow_off + kg), f32x4);
-                            const f32x4 x = __builtin_convertvector(hi, f32x4);
-                            dot += (x[0] * o[0] + x[1] * o[1]) + (x[2] * o[2] + x[3] * o[3]);
+                        float part[4];
+#pragma unroll
+                        for (int g4 = 0; g4 < 4; g4++) {
+                            const V4 hi = R::cvt4(f32x4{run[kb][4 * g4], run[kb][4 * g4 + 1], run[kb][4 * g4 + 2], run[kb][4 * g4 + 3]});
+                            if constexpr (VM) *reinterpret_cast<V4*>(dst_t + so + 32 * kb + 8 * g4) = hi;
+                            if constexpr (KM) {   // two keys x two values per dword: a lane of even value stores the first key of a pair, its neighbour the second
+                                struct U2 { unsigned k01, k23; };
+                                const U2 own = __builtin_bit_cast(U2, hi);
+                                T* const dk = dst_k + so + (size_t)(32 * kb + 16 * (g4 >> 1) + 4 * (g4 & 1)) * D;
+                                const unsigned n01 = __builtin_amdgcn_mov_dpp((int)own.k01, 0xb1, 0xf, 0xf, false), n23 = __builtin_amdgcn_mov_dpp((int)own.k23, 0xb1, 0xf, 0xf, false);
+                                *reinterpret_cast<unsigned*>(dk) = __builtin_amdgcn_perm(n01, own.k01, sel);
+                                *reinterpret_cast<unsigned*>(dk + 2 * D) = __builtin_amdgcn_perm(n23, own.k23, sel);
+                            }
+                            if constexpr (DOT) part[g4] = sum_halves(dot_group(__builtin_convertvector(hi, f32x4), __builtin_convertvector(y[kb][g4], f32x4)));
+                        }
+                        if constexpr (DOT) {   // (the tree of dot_group's comment: groups of four keys, then the 32 values)
+                            float dot = (part[0] + part[1]) + (part[2] + part[3]);
+                            dot += dpp_f<0xb1>(0.f, dot);    // quad_perm 1 0 3 2
+                            dot += dpp_f<0x4e>(0.f, dot);    // quad_perm 2 3 0 1
+                            dot += dpp_f<0x141>(0.f, dot);   // row_half_mirror
+                            dot += dpp_f<0x140>(0.f, dot);   // row_mirror
+                            dot += __shfl_xor(dot, 16);
+                            if (lane == 0) a.dot_part[((size_t)bh * NCS + state_of(s)) * (D / 32) * (D / 32) + (2 * kq + wk + kb) * (D / 32) + (VW / 32) * vh + wv] = dot;
                         }
                     }
                 }
-                if constexpr (DOT) {
-                    dot = wave_scan_inclusive<OpAdd>(dot);
-                    if (lane == 63) dotred[wave] = dot;
-                    pending_dot = c;
-                }
-                if (vh == 0 && wave == 0) {   // the vector state: the feeders' partial sums of this step, carried like the matrix
-                    float sum = 0.f;
-#pragma unroll 8
-                    for (int g = 0; g < 32; g++) sum += red[g * 64 + lane];
-                    nrun = nrun * tgam[cm.s] + sum;
-                    a.Nst[((size_t)bh * NCS + c) * D + 64 * kq + lane] = nrun;
-                }
-                if (cm.s + 1 < NCS) {
-                    const float gam = tgam[cm.s + 1];
-#pragma unroll
-                    for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-                        for (int x = 0; x < 16; x++) acc[nb][x] *= gam;
-                }
+                st = stn;
+                t++;
+                __syncthreads();
             }
-            advance(cm);
-            SQ_STAMP(1);
-            __syncthreads();
-            SQ_STAMP(3);
         }
-        SQ_DUMP(1);
-        if (DOT && pending_dot >= 0 && tid == 0)
-            a.dot_part[((size_t)bh * NCS + pending_dot) * Cfg::WPH + w] = (dotred[0] + dotred[1]) + (dotred[2] + dotred[3]);
+        if (wave == 3) carry_vector(NCS - 1);
     }
 #endif
 }
 
-// Whether the one-pass kernel serves a launch: on request only (set_state_kernel(2)), a table's worth of states, no split
-// mode.  Measured at B4 H8 S4096 D256 and B2 H32 S16384 D128 (256 workgroups each) it takes the same 68 / 234 us per
-// direction as the two kernels above (69 / 231 us): it moves half the bytes, but with one workgroup per CU and one
-// barrier per tile each of its waves spends 1500 to 2000 cycles per tile on some 150 instructions (cycle stamps: direct
-// loads 700, vector sum 600, products 1500, state write-out 400 per tile on average), so the launch stays with the two
-// kernels until that per-tile cost is halved (two workgroups per CU, or two tiles per barrier).
-int g_state_kernel = 0;   // 0 and 1 = chunk sums + carry, 2 = one pass where it can serve
+// Whether the one-pass kernel serves a launch: no split mode, a table's worth of states, and where nothing asks for one form or the other by how
+// full its workgroups leave the chip (one per CU, each as long as its walk).  Rounds of workgroups three quarters full at the least: whatever the number of states.  One round
+// that is emptier: up to as many states as it has thirty-twos of workgroups.  us, the two kernels / one pass, forward, forward that keeps states, backward, whole
+// passes (bf16; heads x states):
+//   D = 256   4 x 3: 31.5, 32.0, 68.8 / 37.3, 39.8, 74.7   8 x 2: 33.2, 33.5, 70.7 / 31.8, 34.0, 68.2   8 x 3: 37.6, 38.3, 76.8 / 38.0, 40.9, 77.5
+//             12 x 3: 50.7, 51.8, 105 / 46.8, 49.5, 100   16 x 7: 83.4, 85.1, 191.4 / 89.1, 94.6, 190.8   20 x 3: 64.3, 66.7, 145.5 / 57.8, 61.1, 138.3
+//             24 x 7: 119, 127, 297 / 106, 111, 279   32 x 2: 54.0, 55.0, 118 / 43.1, 45.1, 105   32 x 7: 152, 156, 369 / 130, 138, 346
+//             36 x 3: 86.0, 87.8, 215 / 96.6, 102, 225   40 x 3: 86.9, 88.9, 244.5 / 89.9, 94.4, 245.3   48 x 7: 226, 239, 541 / 209, 228, 532   64 x 3: 144, 147, 341 / 122, 130, 327
+//   D = 128   16 x 2: 29.6, 30.0, 53.5 / 28.7, 29.7, 51.1   16 x 3: 32.6, 33.1, 65.6 / 34.4, 35.6, 67.0   24 x 3: 39.1, 39.8, 91.1 / 38.3, 39.4, 88.7   32 x 7: 62.7, 64.2, 157 / 71.8, 74.1, 160
+//             48 x 3: 51.4, 51.7, 122 / 48.6, 49.7, 117   48 x 15: 172, 178, 448 / 169, 179, 446   64 x 2: 42.0, 43.9, 99.9 / 37.0, 38.2, 91.0   64 x 31: 465, 489, 1165 / 434, 454, 1138
+//             72 x 7: 126, 131, 336 / 140, 145, 343   96 x 7: 169, 176, 442 / 171, 178, 436   128 x 7: 223, 238, 581 / 211, 221, 567
+int g_state_kernel = 0;   // 0 = the rule, 1 = chunk sums + carry, 2 = one pass where it can serve
 template <typename T, int D>
 static bool chunk_seq_serves(const ChunkArgs& a) {
     using Cfg = SeqCfg<T, D>;
-    if (a.precise || a.NCS > Cfg::MAX_STEPS || (a.Cst && a.dot_part)) return false;
-    return g_state_kernel == 2;
+    if (a.precise || a.NCS > Cfg::MAX_STEPS || (a.Cst && a.dot_part) || g_state_kernel == 1) return false;
+    constexpr long long CUS = 256;
+    const long long wgs = (long long)a.BH * Cfg::WPH, rounds = (wgs + CUS - 1) / CUS;
+    return g_state_kernel == 2 || 4 * wgs >= 3 * CUS * rounds || (rounds == 1 && 32ll * a.NCS <= wgs);
+}
+template <typename T, int D, bool KM, bool VM, bool DOT>
+static int launch_chunk_seq_t(const ChunkArgs& a, hipStream_t st) {
+    using Cfg = SeqCfg<T, D>;
+    if (int rc = no_scratch_once<chunk_seq_kernel<T, D, KM, VM, DOT>>()) return rc;
+    if (hipError_t e = lds_limit_once<chunk_seq_kernel<T, D, KM, VM, DOT>>(160 * 1024); e != hipSuccess) return (int)e;
+    hipLaunchKernelGGL((chunk_seq_kernel<T, D, KM, VM, DOT>), dim3(a.BH * Cfg::WPH), dim3(512), Cfg::LDS_BYTES, st, a);
+    return (int)hipGetLastError();
 }
 template <typename T, int D>
 static int launch_chunk_seq(const ChunkArgs& a, hipStream_t st) {
-    using Cfg = SeqCfg<T, D>;
-    const dim3 grid(a.BH * Cfg::WPH);
-    if (a.dot_part) {
-        if (!a.dot_with || a.dot_with_lo) return MLSTM_EINVAL;
-        if (int rc = no_scratch_once<chunk_seq_kernel<T, D, true>>()) return rc;
-        if (hipError_t e = lds_limit_once<chunk_seq_kernel<T, D, true>>(160 * 1024); e != hipSuccess) return (int)e;
-        hipLaunchKernelGGL((chunk_seq_kernel<T, D, true>), grid, dim3(512), Cfg::LDS_BYTES, st, a);
-    } else {
-        if (int rc = no_scratch_once<chunk_seq_kernel<T, D, false>>()) return rc;
-        if (hipError_t e = lds_limit_once<chunk_seq_kernel<T, D, false>>(160 * 1024); e != hipSuccess) return (int)e;
-        hipLaunchKernelGGL((chunk_seq_kernel<T, D, false>), grid, dim3(512), Cfg::LDS_BYTES, st, a);
-    }
-    return (int)hipGetLastError();
+    if (a.dot_part) return a.CstT && a.dot_with && !a.dot_with_lo ? launch_chunk_seq_t<T, D, false, true, true>(a, st) : MLSTM_EINVAL;
+    if (a.Cst && a.CstT) return launch_chunk_seq_t<T, D, true, true, false>(a, st);
+    return a.Cst ? launch_chunk_seq_t<T, D, true, false, false>(a, st) : launch_chunk_seq_t<T, D, false, true, false>(a, st);
 }
 
 template <typename T, int D, bool STRICT>
@@ -1683,13 +1765,7 @@ int launch_chunk_states(int dtype, int D, const ChunkArgs& a, hipStream_t st) {
 }
 
 int chunk_states_dot_parts(int dtype, int D, const ChunkArgs& a) {
-    if (dtype == MLSTM_F32 || D == 64) return (D / 32) * (D / 32);
-    bool seq = false;
-    if (dtype == MLSTM_BF16 && D == 128) seq = chunk_seq_serves<__bf16, 128>(a);
-    if (dtype == MLSTM_BF16 && D == 256) seq = chunk_seq_serves<__bf16, 256>(a);
-    if (dtype == MLSTM_F16 && D == 128) seq = chunk_seq_serves<_Float16, 128>(a);
-    if (dtype == MLSTM_F16 && D == 256) seq = chunk_seq_serves<_Float16, 256>(a);
-    return seq ? (D / 64) * 2 : (D / 32) * (D / 32);
+    return (D / 32) * (D / 32);
 }
 
 int set_state_kernel(int variant) {
