@@ -344,7 +344,7 @@ int mlstm_set_column_kernel(int variant);
  * Measurement and test aid: which kernels form the chunk states of the 16-bit types at D = 128 and 256.
  * 0 = the library's choice by the size of the launch, 1 = chunk sums and carry (two kernels, any size, split mode),
  * 2 = the one-pass kernel ((D / 64) * 2 workgroups per head walk the chunks in order, no fp32 sums through memory)
- * wherever it can serve (not in split mode, at most 256 states per head).  Both give the same bits.
+ * wherever it can serve (split mode at D = 256 only, at most 256 states per head).  Both give the same bits.
  * Process-wide; returns 0, or MLSTM_EINVAL.  No counterpart in the reference.
  */
 int mlstm_set_state_kernel(int variant);

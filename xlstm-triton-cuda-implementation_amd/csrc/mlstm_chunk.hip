@@ -1177,7 +1177,7 @@ __global__ __launch_bounds__(256, 4) void chunk_carry_t_kernel(ChunkArgs a) {
 // state and walks the head's chunks in their order (forward: first to last; reverse: last to first).  Two sets of
 // accumulators: the chunk's own sum, and the running state that takes it at the chunk's end (state = gamma * state + sum) and is
 // written in the element type.  No fp32 chunk sums travel through memory (4 + 4 bytes per state element in the two-kernel form), no
-// second launch.  WPH workgroups per head; not in split mode; chunk_seq_serves decides.
+// second launch.  WPH workgroups per head; chunk_seq_serves decides.
 //
 // Eight waves, two on every SIMD.  Waves 0..3 multiply straight out of the stages: the positions' weights go onto the V fragments in
 // registers (rounded to the element type as chunk_sum_kernel rounds its weighted V rows); a wave owns 32 values, so that at
@@ -1211,8 +1211,9 @@ struct SeqCfg {
     static constexpr int WPH = (D / KR) * (D / VW);                    // workgroups per head
 };
 
-// KM, VM: key-major and value-major states are written (ChunkArgs::Cst, CstT); DOT: the contraction with another set on the way
-template <typename T, int D, bool KM, bool VM, bool DOT>
+// KM, VM: key-major and value-major states are written (ChunkArgs::Cst, CstT); DOT: the contraction with another set on the way; STRICT: split
+// mode (ChunkArgs::precise): the weighted values and the states as two terms
+template <typename T, int D, bool KM, bool VM, bool DOT, bool STRICT>
 __global__ __launch_bounds__(512) void chunk_seq_kernel(ChunkArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using R = Tr<T>;
@@ -1445,7 +1446,9 @@ __global__ __launch_bounds__(512) void chunk_seq_kernel(ChunkArgs a) {
         };
         constexpr int NSTEP = GRAN / KW;
         static_assert(NSTEP == 4, "two registers of weights");
-        frag kf[NSTEP][NKB], vf[NSTEP], vw;
+        struct Weighed { frag hi, lo; };   // (lo: split mode)
+        frag kf[NSTEP][NKB], vf[NSTEP];
+        Weighed vw;
         // The weights of a tile in two registers: a V fragment holds, for the lane's value, positions 16 s4 + 4 h + (0..3) and
         // 16 s4 + 8 + 4 h + (0..3) as elements 0..7, and element e of step s4 finds its weight in lane 8 (s4 & 1) + e of its row of 16
         // lanes, register s4 / 2 (one DPP operand; as two 16-byte reads per step the weights were a third of all LDS traffic).
@@ -1471,10 +1474,18 @@ __global__ __launch_bounds__(512) void chunk_seq_kernel(ChunkArgs a) {
                 return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, wv4), 0x150 + l0 + decltype(e)::value, 0xf, 0xf, true));
             };
             static_for<8>([&](auto e) __attribute__((always_inline)) { x[decltype(e)::value] *= weight(e); });
-            struct Pair { V4 lo, hi; } p;
-            p.lo = R::cvt4(f32x4{x[0], x[1], x[2], x[3]});
-            p.hi = R::cvt4(f32x4{x[4], x[5], x[6], x[7]});
-            return __builtin_bit_cast(frag, p);
+            struct Pair { V4 lo, hi; } p, rest;
+            Weighed out{};
+            if constexpr (STRICT) {
+                R::cvt4_split(f32x4{x[0], x[1], x[2], x[3]}, p.lo, rest.lo);
+                R::cvt4_split(f32x4{x[4], x[5], x[6], x[7]}, p.hi, rest.hi);
+                out.lo = __builtin_bit_cast(frag, rest);
+            } else {
+                p.lo = R::cvt4(f32x4{x[0], x[1], x[2], x[3]});
+                p.hi = R::cvt4(f32x4{x[4], x[5], x[6], x[7]});
+            }
+            out.hi = __builtin_bit_cast(frag, p);
+            return out;
         };
         const int vg = VW * vh + 32 * wv + c32;        // the lane's value
         const int krow0 = 64 * kq + 32 * wk + 8 * h;   // state row of its first key: that of key 32 kb + 8 g4 + 4 h lies 32 kb + 16 (g4 / 2) + 4 (g4 % 2) on
@@ -1482,8 +1493,12 @@ __global__ __launch_bounds__(512) void chunk_seq_kernel(ChunkArgs a) {
         const unsigned odd = lane & 1, sel = odd ? 0x03020706u : 0x05040100u;
         T* const dst_t = reinterpret_cast<T*>(a.CstT) + toff;
         T* const dst_k = reinterpret_cast<T*>(a.Cst) + hbase + (size_t)(krow0 + odd) * D + (vg & ~1);
+        // (low-order terms: as far behind the others as the arrays are apart)
+        const ptrdiff_t t_lo = STRICT && VM ? reinterpret_cast<T*>(a.CstT_lo) - reinterpret_cast<T*>(a.CstT) : 0;
+        const ptrdiff_t k_lo = STRICT && KM ? reinterpret_cast<T*>(a.Cst_lo) - reinterpret_cast<T*>(a.Cst) : 0;
+        const ptrdiff_t o_lo = STRICT && DOT ? reinterpret_cast<const T*>(a.dot_with_lo) - reinterpret_cast<const T*>(a.dot_with) : 0;
         const T* const other = reinterpret_cast<const T*>(a.dot_with) + toff;
-        V4 y[DOT ? NKB : 1][4];
+        V4 y[DOT ? NKB : 1][4], yl[DOT && STRICT ? NKB : 1][4];
         float nrun = 0.f;
         auto carry_vector = [&](int s) __attribute__((always_inline)) {   // by one wave, behind the barrier that follows the step's last tile
             float sum = 0.f;
@@ -1509,7 +1524,10 @@ __global__ __launch_bounds__(512) void chunk_seq_kernel(ChunkArgs a) {
 #pragma unroll
                 for (int kb = 0; kb < NKB; kb++)
 #pragma unroll
-                    for (int g4 = 0; g4 < 4; g4++) y[kb][g4] = *reinterpret_cast<const V4*>(other + so + 32 * kb + 8 * g4);
+                    for (int g4 = 0; g4 < 4; g4++) {
+                        y[kb][g4] = *reinterpret_cast<const V4*>(other + so + 32 * kb + 8 * g4);
+                        if constexpr (STRICT) yl[kb][g4] = *reinterpret_cast<const V4*>(other + o_lo + so + 32 * kb + 8 * g4);
+                    }
             }
             for (int tt = 0; tt < nt; tt++) {
                 const int stn = st + 1 == NS ? 0 : st + 1;
@@ -1524,7 +1542,11 @@ __global__ __launch_bounds__(512) void chunk_seq_kernel(ChunkArgs a) {
                     }
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int kb = 0; kb < NKB; kb++) R::mma(acc[kb], kf[s4][kb], vw);
+                    for (int kb = 0; kb < NKB; kb++) R::mma(acc[kb], kf[s4][kb], vw.hi);
+                    if constexpr (STRICT) {
+#pragma unroll
+                        for (int kb = 0; kb < NKB; kb++) R::mma(acc[kb], kf[s4][kb], vw.lo);
+                    }
                     if constexpr (s4 + 1 < NSTEP) vw = weighed(std::integral_constant<int, s4 + 1>{}, wr);
                     else vw = weighed(std::integral_constant<int, 0>{}, wnext);
                     __builtin_amdgcn_sched_barrier(0);
@@ -1543,17 +1565,30 @@ __global__ __launch_bounds__(512) void chunk_seq_kernel(ChunkArgs a) {
                         float part[4];
 #pragma unroll
                         for (int g4 = 0; g4 < 4; g4++) {
-                            const V4 hi = R::cvt4(f32x4{run[kb][4 * g4], run[kb][4 * g4 + 1], run[kb][4 * g4 + 2], run[kb][4 * g4 + 3]});
-                            if constexpr (VM) *reinterpret_cast<V4*>(dst_t + so + 32 * kb + 8 * g4) = hi;
-                            if constexpr (KM) {   // two keys x two values per dword: a lane of even value stores the first key of a pair, its neighbour the second
-                                struct U2 { unsigned k01, k23; };
-                                const U2 own = __builtin_bit_cast(U2, hi);
-                                T* const dk = dst_k + so + (size_t)(32 * kb + 16 * (g4 >> 1) + 4 * (g4 & 1)) * D;
-                                const unsigned n01 = __builtin_amdgcn_mov_dpp((int)own.k01, 0xb1, 0xf, 0xf, false), n23 = __builtin_amdgcn_mov_dpp((int)own.k23, 0xb1, 0xf, 0xf, false);
-                                *reinterpret_cast<unsigned*>(dk) = __builtin_amdgcn_perm(n01, own.k01, sel);
-                                *reinterpret_cast<unsigned*>(dk + 2 * D) = __builtin_amdgcn_perm(n23, own.k23, sel);
+                            const f32x4 four = f32x4{run[kb][4 * g4], run[kb][4 * g4 + 1], run[kb][4 * g4 + 2], run[kb][4 * g4 + 3]};
+                            V4 hi, lo{};
+                            if constexpr (STRICT) R::cvt4_split(four, hi, lo); else hi = R::cvt4(four);
+                            if constexpr (VM) {
+                                *reinterpret_cast<V4*>(dst_t + so + 32 * kb + 8 * g4) = hi;
+                                if constexpr (STRICT) *reinterpret_cast<V4*>(dst_t + t_lo + so + 32 * kb + 8 * g4) = lo;
                             }
-                            if constexpr (DOT) part[g4] = sum_halves(dot_group(__builtin_convertvector(hi, f32x4), __builtin_convertvector(y[kb][g4], f32x4)));
+                            if constexpr (KM) {   // two keys x two values per dword: a lane of even value stores the first key of a pair, its neighbour the second
+                                T* const dk = dst_k + so + (size_t)(32 * kb + 16 * (g4 >> 1) + 4 * (g4 & 1)) * D;
+                                auto store_pairs = [&](T* to, const V4& x) __attribute__((always_inline)) {
+                                    struct U2 { unsigned k01, k23; };
+                                    const U2 own = __builtin_bit_cast(U2, x);
+                                    const unsigned n01 = __builtin_amdgcn_mov_dpp((int)own.k01, 0xb1, 0xf, 0xf, false), n23 = __builtin_amdgcn_mov_dpp((int)own.k23, 0xb1, 0xf, 0xf, false);
+                                    *reinterpret_cast<unsigned*>(to) = __builtin_amdgcn_perm(n01, own.k01, sel);
+                                    *reinterpret_cast<unsigned*>(to + 2 * D) = __builtin_amdgcn_perm(n23, own.k23, sel);
+                                };
+                                store_pairs(dk, hi);
+                                if constexpr (STRICT) store_pairs(dk + k_lo, lo);
+                            }
+                            if constexpr (DOT) {   // (the states as they are written: in split mode the sums of their terms)
+                                f32x4 xs = __builtin_convertvector(hi, f32x4), ys = __builtin_convertvector(y[kb][g4], f32x4);
+                                if constexpr (STRICT) { xs += __builtin_convertvector(lo, f32x4); ys += __builtin_convertvector(yl[kb][g4], f32x4); }
+                                part[g4] = sum_halves(dot_group(xs, ys));
+                            }
                         }
                         if constexpr (DOT) {   // (the tree of dot_group's comment: groups of four keys, then the 32 values)
                             float dot = (part[0] + part[1]) + (part[2] + part[3]);
@@ -1576,7 +1611,7 @@ __global__ __launch_bounds__(512) void chunk_seq_kernel(ChunkArgs a) {
 #endif
 }
 
-// Whether the one-pass kernel serves a launch: no split mode, a table's worth of states, and where nothing asks for one form or the other by how
+// Whether the one-pass kernel serves a launch: a table's worth of states, split mode at D = 256 only, and where nothing asks for one form or the other by how
 // full its workgroups leave the chip (one per CU, each as long as its walk).  Rounds of workgroups three quarters full at the least: whatever the number of states.  One round
 // that is emptier: up to as many states as it has thirty-twos of workgroups.  us, the two kernels / one pass, forward, forward that keeps states, backward, whole
 // passes (bf16; heads x states):
@@ -1587,28 +1622,34 @@ __global__ __launch_bounds__(512) void chunk_seq_kernel(ChunkArgs a) {
 //   D = 128   16 x 2: 29.6, 30.0, 53.5 / 28.7, 29.7, 51.1   16 x 3: 32.6, 33.1, 65.6 / 34.4, 35.6, 67.0   24 x 3: 39.1, 39.8, 91.1 / 38.3, 39.4, 88.7   32 x 7: 62.7, 64.2, 157 / 71.8, 74.1, 160
 //             48 x 3: 51.4, 51.7, 122 / 48.6, 49.7, 117   48 x 15: 172, 178, 448 / 169, 179, 446   64 x 2: 42.0, 43.9, 99.9 / 37.0, 38.2, 91.0   64 x 31: 465, 489, 1165 / 434, 454, 1138
 //             72 x 7: 126, 131, 336 / 140, 145, 343   96 x 7: 169, 176, 442 / 171, 178, 436   128 x 7: 223, 238, 581 / 211, 221, 567
+//   Split mode, D = 256 (two products per fragment, twice the states to write; one round from three eighths full on)   8 x 2: 42.0, 43.4, 89.9 / 42.8, 48.2, 92.6
+//             12 x 3: 70.4, 72.5, 148 / 63.6, 70.6, 142   16 x 7: 116, 124, 266 / 127, 143, 280   24 x 7: 172, 194, 406 / 151, 179, 394   32 x 2: 73.1, 78.5, 158 / 59.8, 68.1, 145
+//             32 x 7: 207, 231, 491 / 182, 215, 480   64 x 3: 193, 216, 463 / 175, 203, 453    (D = 128 64 x 3: 76.1, 84.2, 212 / 75.6, 82.9, 213   96 x 7: 224, 254, 646 / 237, 267, 664)
 int g_state_kernel = 0;   // 0 = the rule, 1 = chunk sums + carry, 2 = one pass where it can serve
 template <typename T, int D>
 static bool chunk_seq_serves(const ChunkArgs& a) {
     using Cfg = SeqCfg<T, D>;
-    if (a.precise || a.NCS > Cfg::MAX_STEPS || (a.Cst && a.dot_part) || g_state_kernel == 1) return false;
+    if ((a.precise && D == 128) || a.NCS > Cfg::MAX_STEPS || (a.Cst && a.dot_part) || g_state_kernel == 1) return false;
     constexpr long long CUS = 256;
     const long long wgs = (long long)a.BH * Cfg::WPH, rounds = (wgs + CUS - 1) / CUS;
-    return g_state_kernel == 2 || 4 * wgs >= 3 * CUS * rounds || (rounds == 1 && 32ll * a.NCS <= wgs);
+    return g_state_kernel == 2 || 4 * wgs >= 3 * CUS * rounds || (rounds == 1 && 32ll * a.NCS <= wgs && (!a.precise || 8 * wgs >= 3 * CUS));
 }
-template <typename T, int D, bool KM, bool VM, bool DOT>
+template <typename T, int D, bool STRICT, bool KM, bool VM, bool DOT>
 static int launch_chunk_seq_t(const ChunkArgs& a, hipStream_t st) {
     using Cfg = SeqCfg<T, D>;
-    if (int rc = no_scratch_once<chunk_seq_kernel<T, D, KM, VM, DOT>>()) return rc;
-    if (hipError_t e = lds_limit_once<chunk_seq_kernel<T, D, KM, VM, DOT>>(160 * 1024); e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL((chunk_seq_kernel<T, D, KM, VM, DOT>), dim3(a.BH * Cfg::WPH), dim3(512), Cfg::LDS_BYTES, st, a);
+    if (int rc = no_scratch_once<chunk_seq_kernel<T, D, KM, VM, DOT, STRICT>>()) return rc;
+    if (hipError_t e = lds_limit_once<chunk_seq_kernel<T, D, KM, VM, DOT, STRICT>>(160 * 1024); e != hipSuccess) return (int)e;
+    hipLaunchKernelGGL((chunk_seq_kernel<T, D, KM, VM, DOT, STRICT>), dim3(a.BH * Cfg::WPH), dim3(512), Cfg::LDS_BYTES, st, a);
     return (int)hipGetLastError();
 }
-template <typename T, int D>
+template <typename T, int D, bool STRICT>
 static int launch_chunk_seq(const ChunkArgs& a, hipStream_t st) {
-    if (a.dot_part) return a.CstT && a.dot_with && !a.dot_with_lo ? launch_chunk_seq_t<T, D, false, true, true>(a, st) : MLSTM_EINVAL;
-    if (a.Cst && a.CstT) return launch_chunk_seq_t<T, D, true, true, false>(a, st);
-    return a.Cst ? launch_chunk_seq_t<T, D, true, false, false>(a, st) : launch_chunk_seq_t<T, D, false, true, false>(a, st);
+    if (a.dot_part) {
+        if (!a.CstT || !a.dot_with || STRICT != (a.dot_with_lo != nullptr)) return MLSTM_EINVAL;
+        return launch_chunk_seq_t<T, D, STRICT, false, true, true>(a, st);
+    }
+    if (a.Cst && a.CstT) return launch_chunk_seq_t<T, D, STRICT, true, true, false>(a, st);
+    return a.Cst ? launch_chunk_seq_t<T, D, STRICT, true, false, false>(a, st) : launch_chunk_seq_t<T, D, STRICT, false, true, false>(a, st);
 }
 
 template <typename T, int D, bool STRICT>
@@ -1665,7 +1706,12 @@ static int launch_chunk_carry_small(const ChunkArgs& a, hipStream_t st) {
 template <typename T, int D>
 static int launch_chunk_t(const ChunkArgs& a, hipStream_t st) {
     if (a.precise && ((a.Cst && !a.Cst_lo) || (a.CstT && !a.CstT_lo))) return MLSTM_EINVAL;
-    if (chunk_seq_serves<T, D>(a)) return launch_chunk_seq<T, D>(a, st);
+    if (chunk_seq_serves<T, D>(a)) {
+        if constexpr (D == 256) {
+            if (a.precise) return launch_chunk_seq<T, D, true>(a, st);
+        }
+        return launch_chunk_seq<T, D, false>(a, st);
+    }
     if (int rc = a.precise ? launch_chunk_sum<T, D, true>(a, st) : launch_chunk_sum<T, D, false>(a, st)) return rc;
     // one carry kernel: the value-major one writes both layouts and the vector states
     if (a.dot_part && !(a.CstT && a.dot_with)) return MLSTM_EINVAL;
