@@ -42,13 +42,19 @@ struct ColCfg {
     // no longer fits two query stages and runs single-staged.
     static constexpr int PLANES = !Tr<T>::HALF ? 3 : (STRICT ? 2 : 1);
     static constexpr size_t GW_BYTES = 2 * PLANES * G_BYTES;
-    static constexpr size_t FIXED_BYTES = GW_BYTES + 6 * GRAN * sizeof(float);   // + row sums [2][64], far column sums [4][64]
+    // 16-bit D = 64: in chunks a workgroup has two or three query tiles, and what surrounds them is most of its time.  The keys'
+    // fragments come from the tiles of the state phase instead of memory, their weights are formed when they are first used, and
+    // the copies are not spread over the few products: 210 registers instead of 252, bf16, 64 heads x 8192: 217 -> 203 us, 16 x 4000:
+    // 28.4 -> 25.5 us; split mode, 64 x 4096: 114 -> 107 us.  (Three workgroups per CU, 168 registers: 69 of them spilled, 313 us.)
+    static constexpr bool LEAN = Tr<T>::HALF && D == 64;
+    static constexpr size_t FIXED_BYTES = GW_BYTES + (LEAN ? 7 : 6) * GRAN * sizeof(float);   // + row sums [2][64], far column sums [4][64]
     static constexpr int STAGES = (2 * STAGE_BYTES + FIXED_BYTES + 2048 * sizeof(float) <= 160 * 1024) ? 2 : 1;
     static constexpr size_t LDS_BYTES = STAGES * STAGE_BYTES + FIXED_BYTES;  // plus one float per key tile, appended at launch
     // In chunks the keys' own K and V tiles lie in LDS during the state phase: in the second stage where there is one;
     // otherwise K in the (not yet used) G / W area and V in an extra tile between the fixed part and the granule bases
     static constexpr size_t TILE_BYTES = TILE_ELEMS * sizeof(T);
     static constexpr size_t EXTRA_CHUNK_BYTES = STAGES == 2 ? 0 : TILE_BYTES;
+    static_assert(!LEAN || STAGES == 2, "the keys' tiles outlive the state phase");
     static_assert(STAGES == 2 || GW_BYTES >= TILE_BYTES, "the keys' K tile fits the G / W area");
 };
 
@@ -59,7 +65,7 @@ __device__ __forceinline__ int gkey(int q) { return (((q >> 1) & 1) << 2) | ((q 
 
 // STRICT (16-bit types): split mode, see ColArgs::precise.
 template <typename T, int D, bool STRICT>
-__global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
+__global__ __launch_bounds__(256, (ColCfg<T, D, STRICT>::LEAN ? 2 : 1)) void col_kernel(ColArgs a) {
 #if defined(__HIP_DEVICE_COMPILE__)  // the body uses device-only builtins; the host pass only needs the stub
     using R = Tr<T>;
     using Cfg = ColCfg<T, D, STRICT>;
@@ -168,33 +174,52 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
 
     const int kstartA = GRAN * jt + 32 * kbA;
     const int keyA = kstartA + c32, keyAc = keyA < S ? keyA : S - 1;
+    constexpr bool LEAN = Cfg::LEAN;
+    float* const sAl = cpart + 4 * GRAN;   // LEAN: the tile's alphas
     frag kf[NS], vf[NS];
-#pragma unroll
-    for (int s = 0; s < NS; s++) {
-        kf[s] = frag_rowmajor<T>(K + (size_t)keyAc * rsA, s, h);
-        vf[s] = frag_rowmajor<T>(V + (size_t)keyAc * rsA, s, h);
-    }
-    float al[16];
-#pragma unroll
-    for (int r = 0; r < 16; r++) al[r] = a.alpha2[poff + kstartA + 8 * (r >> 2) + 4 * h + (r & 3)];
-#pragma unroll
-    for (int s = 0; s < NS; s++) { pin(kf[s]); pin(vf[s]); }
     typename R::terms kt[NS], vt[NS];
+    auto keys_global = [&]() {
 #pragma unroll
-    for (int s = 0; s < NS; s++) { kt[s] = R::split(kf[s]); vt[s] = R::split(vf[s]); }
+        for (int s = 0; s < NS; s++) {
+            kf[s] = frag_rowmajor<T>(K + (size_t)keyAc * rsA, s, h);
+            vf[s] = frag_rowmajor<T>(V + (size_t)keyAc * rsA, s, h);
+        }
+    };
+    auto keys_done = [&]() {
+#pragma unroll
+        for (int s = 0; s < NS; s++) { pin(kf[s]); pin(vf[s]); }
+#pragma unroll
+        for (int s = 0; s < NS; s++) { kt[s] = R::split(kf[s]); vt[s] = R::split(vf[s]); }
+    };
+    float al[16], ekr[16], amaxA;
+    auto al_load = [&]() {
+#pragma unroll
+        for (int r = 0; r < 16; r++) al[r] = LEAN ? sAl[32 * kbA + 8 * (r >> 2) + 4 * h + (r & 3)] : a.alpha2[poff + kstartA + 8 * (r >> 2) + 4 * h + (r & 3)];
+    };
     // factorised weights for the steps below the diagonal: ekr[r] = exp2(alpha_key(r) - c0), c0 the block maximum
-    float ekr[16], amaxA;
-    {
+    auto ekr_make = [&]() {
         float mx = al[0];
 #pragma unroll
         for (int r = 1; r < 16; r++) mx = fmaxf(mx, al[r]);
         amaxA = fmaxf(mx, __shfl_xor(mx, 32));
 #pragma unroll
         for (int r = 0; r < 16; r++) ekr[r] = amaxA > -INFINITY ? fast_exp2(al[r] - amaxA) : 0.f;
-    }
+    };
+    if constexpr (LEAN) {
+        if (tid < GRAN) sAl[tid] = a.alpha2[poff + GRAN * jt + tid];
+        if (!has_state) keys_global();
+        amaxA = 0.f;
 #pragma unroll
-    for (int r = 0; r < 16; r++) { pin(al[r]); pin(ekr[r]); }
-    pin(amaxA);
+        for (int r = 0; r < 16; r++) ekr[r] = 0.f;
+    } else {
+        keys_global();
+        al_load();
+        keys_done();
+        ekr_make();
+#pragma unroll
+        for (int r = 0; r < 16; r++) { pin(al[r]); pin(ekr[r]); }
+        pin(amaxA);
+    }
     // (sG becomes visible, and the first tile is waited for, at the barrier that opens the first step; every plain
     // global load above has been waited for by pin)
     const float log2scale = -0.5f * __log2f((float)D);
@@ -212,7 +237,7 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
 
     constexpr bool FAST_TR = R::HALF && Swz<T, D>::CPR >= 16;
     SwzRowReader<T, D> qrd;
-    qrd.init(lane);
+    if constexpr (!LEAN) qrd.init(lane);
     constexpr bool F32 = !R::HALF;
     typename std::conditional<F32, SwzTransReaderF32<D>, SwzTransReader<typename std::conditional<FAST_TR, T, __bf16>::type, FAST_TR ? D : 256>>::type trd;
     if constexpr (FAST_TR || F32) trd.init(lane, BOTH_KB ? wave * NXW : 0);
@@ -341,6 +366,14 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
         return __builtin_bit_cast(gfrag, both);
     };
 
+    if constexpr (LEAN) {
+        qrd.init(lane);
+        if (has_state) {
+#pragma unroll
+            for (int s = 0; s < NS; s++) { kf[s] = qrd.read(Kt, kbA, s); vf[s] = qrd.read(Vt, kbA, s); }
+        }
+        keys_done();
+    }
     // One step = one 64-query tile.  FIRST (the diagonal tile, it == jt) carries the causal masks and the skipped
     // block; every later tile takes the mask-free path.  Two instantiations instead of a run-time branch keep each
     // loop body a single code path.
@@ -353,6 +386,7 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
         // tile `it` has landed and every wave is past phase B of the previous step
         dma_wait();
         __syncthreads();
+        if constexpr (LEAN && FIRST) al_load();
         const int stn = stage ^ 1;
         if constexpr (STAGES == 2) {
             if constexpr (SPREAD) {
@@ -417,14 +451,16 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
             const float er = !qvalid ? 0.f : (F32 ? fast_exp2((float)((Base)(amaxA + nbeta) + crow)) : fast_exp2((float)crow + amaxA));
             // below the diagonal E = ekr[key] * er[query]: the query factor goes into the per-lane scalars, which leaves
             // seven operations per element (G = dC~ E, W = C~ / n, dD = C~ dC~ with C~ = S E, dC~ = dC / n + db)
+            // (the diagonal tile) keys above this one, counted from 4 h, are masked: all of a query past the end, those behind the query
+            const int lastkey = !qvalid ? -1 : diag ? c32 - 4 * h : GRAN;
             const float inv_er = inv * er, dbv_er = dbv * er;
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 // dD: the column sums add it up as it is rounded (mlstm_colf.hip hands it from wave to wave), the row sums before it is
                 float dd;
                 if constexpr (FIRST) {
-                    float e = fast_exp2(F32 ? (al[r] + nbeta) + (float)crow : al[r] + (float)crow);
-                    if (!qvalid || (diag && (8 * (r >> 2) + 4 * h + (r & 3) > c32))) e = 0.f;
+                    const bool masked = 8 * (r >> 2) + (r & 3) > lastkey;
+                    const float e = fast_exp2(masked ? -INFINITY : F32 ? (al[r] + nbeta) + (float)crow : al[r] + (float)crow);
                     const float ct = sacc[r] * e;
                     const float dct = fmaf(dacc[r], inv, dbv);
                     dd = product_apart(ct, dct);
@@ -565,7 +601,10 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
     const int lim = (NGe < full_tiles ? NGe : full_tiles) - 1;   // last step index that may spread is lim - 1
     step(std::true_type{}, std::false_type{}, jt);  // the diagonal step skips a block in some waves: it copies in one go
     int it = jt + 1;
-    for (; it < lim; it++) step(std::false_type{}, std::true_type{}, it);
+    if constexpr (LEAN) {
+        if (it < NGe) { al_load(); ekr_make(); }
+    }
+    if constexpr (!LEAN) for (; it < lim; it++) step(std::false_type{}, std::true_type{}, it);
     for (; it < NGe; it++) step(std::false_type{}, std::false_type{}, it);
 #undef COL_DMA
 #undef ST_Q
@@ -597,13 +636,14 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
 
     // ---- epilogue: dK, dV.  A lane holds 4 consecutive columns of its key's row: stored directly that would be 8-byte
     // pieces scattered over 32 rows per instruction.  Each tensor goes through an LDS tile (rows padded by 16 bytes)
-    // and leaves in 16-byte pieces, a row at a time.
+    // of its own and leaves in 16-byte pieces, a row at a time.
     {
         constexpr int RB = D * (int)sizeof(T) + 16, CPR = D * (int)sizeof(T) / 16;
-        char* const stage = smem;  // the Q / dH stages are free once every wave is past its last phase B
+        static_assert((size_t)2 * GRAN * RB <= STAGES * Cfg::STAGE_BYTES + Cfg::GW_BYTES, "both staged outputs fit");
+        __syncthreads();   // the Q / dH stages (and the G / W tiles behind them) are free once every wave is past its last phase B
 #pragma unroll
         for (int which = 0; which < 2; which++) {
-            __syncthreads();
+            char* const stage = smem + which * GRAN * RB;
 #pragma unroll
             for (int kb = 0; kb < NKB; kb++)
 #pragma unroll
@@ -616,27 +656,30 @@ __global__ __launch_bounds__(256, 1) void col_kernel(ColArgs a) {
                         const int d = 32 * (BOTH_KB ? wave * NXW + x : dsel + 2 * x) + 8 * a4 + 4 * h;
                         *reinterpret_cast<typename R::vec4*>(stage + (32 * (BOTH_KB ? kb : kbB) + c32) * RB + d * (int)sizeof(T)) = R::cvt4(v);
                     }
-            __syncthreads();
-            char* const gout = reinterpret_cast<char*>(which ? a.dV : a.dK) + (offA + (size_t)GRAN * jt * rsA) * sizeof(T);
+        }
+        __syncthreads();
 #pragma unroll
-            for (int i = 0; i < GRAN * CPR / 256; i++) {
-                const int c = tid + 256 * i, row = c / CPR, cc = c % CPR;
-                if (GRAN * jt + row < S)
-                    *reinterpret_cast<uint4*>(gout + (size_t)row * rsA * sizeof(T) + 16 * cc) = *reinterpret_cast<const uint4*>(stage + row * RB + 16 * cc);
-            }
+        for (int which = 0; which < 2; which++) {
+            const char* const stage = smem + which * GRAN * RB;
+            char* const gout = reinterpret_cast<char*>(which ? a.dV : a.dK) + (offA + (size_t)GRAN * jt * rsA) * sizeof(T);
+            pieces_out<GRAN * CPR / 256>(
+                [&](int i) { const int c = tid + 256 * i; return *reinterpret_cast<const uint4*>(stage + (c / CPR) * RB + 16 * (c % CPR)); },
+                [&](int i, uint4 v) {
+                    const int c = tid + 256 * i, row = c / CPR;
+                    if (GRAN * jt + row < S) *reinterpret_cast<uint4*>(gout + (size_t)row * rsA * sizeof(T) + 16 * (c % CPR)) = v;
+                });
         }
     }
-    // ---- column sums: reduce over the 32 query lanes, then over the two query blocks through LDS
+    // ---- column sums: reduce over the 32 query lanes, then over the two query blocks through LDS.  (Five shuffles a register, one
+    // behind the other and a branch between registers, were some 80 LDS round trips: with them, the masks of the diagonal step as
+    // branches and a barrier pair per output, bf16 D = 64, 64 heads x 8192 took 264 us, now 217; fp32, 64 x 4096: 380 -> 338.)
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-        float v = colacc[r];
-        v += __shfl_xor(v, 1);
-        v += __shfl_xor(v, 2);
-        v += __shfl_xor(v, 4);
-        v += __shfl_xor(v, 8);
-        v += __shfl_xor(v, 16);
-        if (c32 == 0) rowtmp[qbA * GRAN + 32 * kbA + 8 * (r >> 2) + 4 * h + (r & 3)] = v;
+    for (int a4 = 0; a4 < 4; a4++) {
+        f32x4 v;
+#pragma unroll
+        for (int c = 0; c < 4; c++) v[c] = sum_half_wave(colacc[4 * a4 + c]);
+        if (c32 == 0) *reinterpret_cast<f32x4*>(rowtmp + qbA * GRAN + 32 * kbA + 8 * a4 + 4 * h) = v;
     }
     __syncthreads();
     if (tid < GRAN && GRAN * jt + tid < S) a.colsum[hoff + GRAN * jt + tid] = rowtmp[tid] + rowtmp[GRAN + tid] + (has_state ? cpart[tid] : 0.f);

@@ -811,6 +811,25 @@ __device__ __forceinline__ float sum_half_wave(float v) {
     return __builtin_bit_cast(float, (int)r[0]) + __builtin_bit_cast(float, (int)r[1]);
 }
 
+// The last copies of a workgroup, from LDS to memory: N 16-byte pieces a lane, read(i) eight at a time ahead of write(i, piece).  With
+// "read, then store if the row is there" a branch lies between any two pieces and each waits for its own read: N LDS round trips
+// at the end of a workgroup, when nothing else may be on its CU.
+template <int N, typename Read, typename Write>
+__device__ __forceinline__ void pieces_out(Read read, Write write) {
+    constexpr int B = N < 8 ? N : 8;
+    static_assert(N % B == 0, "whole sets");
+#pragma unroll
+    for (int i0 = 0; i0 < N; i0 += B) {
+        uint4 v[B];
+#pragma unroll
+        for (int i = 0; i < B; i++) v[i] = read(i0 + i);
+#pragma unroll
+        for (int i = 0; i < B; i++) asm volatile("" : "+v"(v[i].x), "+v"(v[i].y), "+v"(v[i].z), "+v"(v[i].w));   // (the reads stay here)
+#pragma unroll
+        for (int i = 0; i < B; i++) write(i0 + i, v[i]);
+    }
+}
+
 template <typename T> __device__ __forceinline__ float to_f32(T x) { return (float)x; }
 
 // Per-row scalars of the backward, computed by the lanes that already hold the row's dh fragments (xf):
