@@ -199,7 +199,12 @@ __global__ __launch_bounds__(256, D == 128 && !STRICT ? 2 : 1) void cold_kernel(
     } while (0)
 
     // ---- prologue: the V tile (stays), the first state tiles or the first query tile, the wave's K rows into registers
-    tile_dma<T, D, CD_KEYS, 256>(Vt, V, CD_KEYS * jt, S, tid, rsA);   // (rows past the end are clamped)
+    if (CD_KEYS * (jt + 1) <= S) {   // (in query tiles' pieces, whose lane offsets are there anyway: clamped rows are some two hundred instructions)
+#pragma unroll
+        for (int i = 0; i < CD_KEYS / CD_QT; i++) qdma.issue(Vt + (size_t)i * CD_QT * D, V + (size_t)(CD_KEYS * jt + CD_QT * i) * rsA, ra);
+    } else {
+        tile_dma_rolled<T, D, CD_KEYS, 256>(Vt, V, CD_KEYS * jt, S, tid, rsA);   // (rows past the end are clamped)
+    }
     const size_t sbase = has_state ? ((size_t)bh * a.n_states + chunk) * D * D : 0;
     const T* const Evc = reinterpret_cast<const T*>(a.Ev) + sbase;
     const T* const Evl = STRICT ? reinterpret_cast<const T*>(a.Ev_lo) + sbase : nullptr;
@@ -554,6 +559,9 @@ __global__ __launch_bounds__(256, D == 128 && !STRICT ? 2 : 1) void cold_kernel(
     }
 #undef COLD_DMA
 
+    // (Each piece of the epilogue used to wait for its own LDS read, 64 of them one behind the other; with the vector state a block
+    // ahead and the copies read eight at a time, and the V tile's copy above without clamps, bf16: D = 128, 64 heads x 16384: 601 -> 586 us;
+    // D = 256, 32 x 4096: 192.3 -> 190.8.)
     // ---- epilogue: column sums, the last step's row sums, then dK and dV through LDS (the V tile and the stages are free
     // once every wave is past its last phase B): rows of D elements, 16-byte chunk c of row r at chunk c ^ (r & 31), so that
     // the lanes' 8-byte pieces of 32 different rows spread over the banks; the rows leave 16 bytes at a time.
@@ -572,42 +580,54 @@ __global__ __launch_bounds__(256, D == 128 && !STRICT ? 2 : 1) void cold_kernel(
     {
         constexpr int ROWB = D * (int)sizeof(T), CPR = ROWB / 16, NPC = CD_KEYS * CPR / 256;
         static_assert(2 * (size_t)CD_KEYS * ROWB <= Cfg::V_BYTES + Cfg::STAGES_BYTES, "both staged outputs fit the V tile and the stages");
-#pragma unroll
-        for (int which = 0; which < 2; which++) {
+        const float s_end = !END_SCALE ? 1.f : LEAN ? keyvals[2 * CD_KEYS + 32 * kb + c32] : scale_s;   // the keys' weights: see the state phase
+        auto stage_out = [&](auto which_tag, auto state_tag) __attribute__((always_inline)) {
+            constexpr bool which = decltype(which_tag)::value, STATE = decltype(state_tag)::value;
             char* const out = smem + (size_t)which * CD_KEYS * ROWB;
             const int row = 32 * kb + c32;
+            // (the vector state a block ahead: read where it is added, each piece would wait for its own)
+            f32x4 gq[2][4];
+            auto read_g = [&](int x) __attribute__((always_inline)) {
 #pragma unroll
-            for (int x = 0; x < NXD; x++)
+                for (int a4 = 0; a4 < 4; a4++) gq[x & 1][a4] = *reinterpret_cast<const f32x4*>(gvl + 32 * x + 8 * a4 + 4 * h);
+            };
+            if constexpr (STATE) read_g(0);
+#pragma unroll
+            for (int x = 0; x < NXD; x++) {
+                if constexpr (STATE) { if (x + 1 < NXD) read_g(x + 1); }
 #pragma unroll
                 for (int a4 = 0; a4 < 4; a4++) {
                     const int d = 32 * x + 8 * a4 + 4 * h;               // first of the four columns
                     f32x4 v;
 #pragma unroll
                     for (int c = 0; c < 4; c++) v[c] = which ? dvacc[x][4 * a4 + c] : dkacc[x][4 * a4 + c];
-                    if constexpr (END_SCALE) {   // the keys' weights: see the state phase
-                        v *= LEAN ? keyvals[2 * CD_KEYS + 32 * kb + c32] : scale_s;
-                        if (!which && has_state) {
-                            const f32x4 g4 = *reinterpret_cast<const f32x4*>(gvl + d);
+                    if constexpr (END_SCALE) v *= s_end;
+                    if constexpr (STATE) {
 #pragma unroll
-                            for (int c = 0; c < 4; c++) v[c] = fmaf(g4[c], wkg, v[c]);
-                        }
+                        for (int c = 0; c < 4; c++) v[c] = fmaf(gq[x & 1][a4][c], wkg, v[c]);
                     }
                     const int chunk16 = (d * (int)sizeof(T)) >> 4, within = (d * (int)sizeof(T)) & 15;
                     *reinterpret_cast<typename R::vec4*>(out + row * ROWB + (((chunk16 ^ (row & 31)) & (CPR - 1)) << 4) + within) = R::cvt4(v);
                 }
-        }
+            }
+        };
+        if (END_SCALE && has_state) stage_out(std::false_type{}, std::integral_constant<bool, END_SCALE>{});
+        else stage_out(std::false_type{}, std::false_type{});
+        stage_out(std::true_type{}, std::false_type{});
         __syncthreads();
 #pragma unroll
         for (int which = 0; which < 2; which++) {
             const char* const out = smem + (size_t)which * CD_KEYS * ROWB;
             char* const gout = reinterpret_cast<char*>(which ? a.dV : a.dK) + (offA + (size_t)CD_KEYS * jt * rsA) * sizeof(T);
-#pragma unroll
-            for (int i = 0; i < NPC; i++) {
-                const int c = tid + 256 * i, row = c / CPR, cc = c % CPR;
-                if (CD_KEYS * jt + row < S)
-                    *reinterpret_cast<uint4*>(gout + (size_t)row * rsA * sizeof(T) + 16 * cc) =
-                        *reinterpret_cast<const uint4*>(out + row * ROWB + (((cc ^ (row & 31)) & (CPR - 1)) << 4));
-            }
+            pieces_out<NPC>(
+                [&](int i) {
+                    const int c = tid + 256 * i, row = c / CPR, cc = c % CPR;
+                    return *reinterpret_cast<const uint4*>(out + row * ROWB + (((cc ^ (row & 31)) & (CPR - 1)) << 4));
+                },
+                [&](int i, uint4 v) {
+                    const int c = tid + 256 * i, row = c / CPR;
+                    if (CD_KEYS * jt + row < S) *reinterpret_cast<uint4*>(gout + (size_t)row * rsA * sizeof(T) + 16 * (c % CPR)) = v;
+                });
         }
     }
 #ifdef MLSTM_COLD_PROF
