@@ -76,7 +76,7 @@ __global__ __launch_bounds__(512) void colw_kernel(ColArgs a) {
     const T* dH = reinterpret_cast<const T*>(a.dH) + offB;
     const T* K = reinterpret_cast<const T*>(a.K) + offA;
     const T* V = reinterpret_cast<const T*>(a.V) + offA;
-    const int key = GRAN * jt + 32 * kb + c32, keyc = key < S ? key : S - 1;
+    const int key = GRAN * jt + 32 * kb + c32;
     const int chunk = a.chunk_len > 0 ? jt / (a.chunk_len / GRAN) : 0;
     const int jq_end = a.chunk_len > 0 && (chunk + 1) * (a.chunk_len / GRAN) < NG ? (chunk + 1) * (a.chunk_len / GRAN) : NG;
     const int nG = jq_end - jt;                                               // granules of queries, the keys' own first
@@ -368,14 +368,18 @@ __global__ __launch_bounds__(512) void colw_kernel(ColArgs a) {
                 piece(n + 2);
             }
             // k . (E v + g) w, the column sums of dD over the queries behind the chunk (and, for fp16, the scaling itself)
+            // (K out of its slot: tile AHEAD + 1, the first one there, is copied in the second step.  From memory, the
+            // rows came behind the copies under way: with them and an epilogue that waited for each of its LDS reads, bf16, chunks of 512: D = 128,
+            // 16 x 2048 32.1 us, now 30.2; split mode, D = 256, 8 x 1500: 42.9 -> 41.8)
+            static_assert((AHEAD + 1 + 2) % NSLOT == 0, "K outlives the first step");
             if (role == 0) {
-                const T* krow = K + (size_t)keyc * rsA + 4 * h;
+                const char* const kt = reinterpret_cast<const char*>(slot_at(0));
                 float cp = 0.f;
 #pragma unroll
                 for (int x = 0; x < NXD; x++) {
 #pragma unroll
                     for (int a4 = 0; a4 < 4; a4++) {
-                        const f32x4 kv = __builtin_convertvector(*reinterpret_cast<const typename R::vec4*>(krow + 32 * x + 8 * a4), f32x4);
+                        const f32x4 kv = __builtin_convertvector(*reinterpret_cast<const typename R::vec4*>(kt + Z::off(32 * kb + c32, 32 * x + 8 * a4) + 4 * h * (int)sizeof(T)), f32x4);
                         const f32x4 g4 = *reinterpret_cast<const f32x4*>(gvl + 32 * x + 8 * a4 + 4 * h);
 #pragma unroll
                         for (int c = 0; c < 4; c++) {
@@ -459,35 +463,48 @@ __global__ __launch_bounds__(512) void colw_kernel(ColArgs a) {
         constexpr int ROWB = D * (int)sizeof(T), CPR = ROWB / 16;
         char* const out = smem + (size_t)role * GRAN * ROWB;
         const int row = 32 * kb + c32;
+        auto stage_out = [&](auto state_tag) __attribute__((always_inline)) {
+            constexpr bool STATE = decltype(state_tag)::value;
+            f32x4 gq[2][4];   // (a block ahead, see mlstm_cold.hip)
+            auto read_g = [&](int x) __attribute__((always_inline)) {
 #pragma unroll
-        for (int x = 0; x < NXD; x++)
+                for (int a4 = 0; a4 < 4; a4++) gq[x & 1][a4] = *reinterpret_cast<const f32x4*>(gvl + 32 * x + 8 * a4 + 4 * h);
+            };
+            if constexpr (STATE) read_g(0);
 #pragma unroll
-            for (int a4 = 0; a4 < 4; a4++) {
-                const int d = 32 * x + 8 * a4 + 4 * h;
-                f32x4 w;
+            for (int x = 0; x < NXD; x++) {
+                if constexpr (STATE) { if (x + 1 < NXD) read_g(x + 1); }
 #pragma unroll
-                for (int c = 0; c < 4; c++) w[c] = acc[x][4 * a4 + c];
-                if constexpr (END_SCALE) {
-                    w *= scale_s;
-                    if (!role && has_state) {
-                        const f32x4 g4 = *reinterpret_cast<const f32x4*>(gvl + d);
+                for (int a4 = 0; a4 < 4; a4++) {
+                    const int d = 32 * x + 8 * a4 + 4 * h;
+                    f32x4 w;
 #pragma unroll
-                        for (int c = 0; c < 4; c++) w[c] = fmaf(g4[c], wkg, w[c]);
+                    for (int c = 0; c < 4; c++) w[c] = acc[x][4 * a4 + c];
+                    if constexpr (END_SCALE) w *= scale_s;
+                    if constexpr (STATE) {
+#pragma unroll
+                        for (int c = 0; c < 4; c++) w[c] = fmaf(gq[x & 1][a4][c], wkg, w[c]);
                     }
+                    const int chunk16 = (d * (int)sizeof(T)) >> 4, within = (d * (int)sizeof(T)) & 15;
+                    *reinterpret_cast<typename R::vec4*>(out + row * ROWB + (((chunk16 ^ (row & 31)) & (CPR - 1)) << 4) + within) = R::cvt4(w);
                 }
-                const int chunk16 = (d * (int)sizeof(T)) >> 4, within = (d * (int)sizeof(T)) & 15;
-                *reinterpret_cast<typename R::vec4*>(out + row * ROWB + (((chunk16 ^ (row & 31)) & (CPR - 1)) << 4) + within) = R::cvt4(w);
             }
+        };
+        if (END_SCALE && !role && has_state) stage_out(std::integral_constant<bool, END_SCALE>{});
+        else stage_out(std::false_type{});
     }
     __syncthreads();
     constexpr int ROWB = D * (int)sizeof(T), CPR = ROWB / 16, NPC = 2 * GRAN * CPR / 512;
-#pragma unroll
-    for (int i = 0; i < NPC; i++) {
-        const int c = tid + 512 * i, row2 = c / CPR, cc = c % CPR, row = row2 % GRAN, which = row2 / GRAN;
-        if (GRAN * jt + row < S)
-            *reinterpret_cast<uint4*>(reinterpret_cast<char*>(which ? a.dV : a.dK) + (offA + (size_t)(GRAN * jt + row) * rsA) * sizeof(T) + 16 * cc) =
-                *reinterpret_cast<const uint4*>(smem + row2 * ROWB + (((cc ^ (row & 31)) & (CPR - 1)) << 4));
-    }
+    pieces_out<NPC>(
+        [&](int i) {
+            const int c = tid + 512 * i, row2 = c / CPR, cc = c % CPR;
+            return *reinterpret_cast<const uint4*>(smem + row2 * ROWB + (((cc ^ (row2 & 31)) & (CPR - 1)) << 4));
+        },
+        [&](int i, uint4 v) {
+            const int c = tid + 512 * i, row2 = c / CPR, row = row2 % GRAN, which = row2 / GRAN;
+            if (GRAN * jt + row < S)
+                *reinterpret_cast<uint4*>(reinterpret_cast<char*>(which ? a.dV : a.dK) + (offA + (size_t)(GRAN * jt + row) * rsA) * sizeof(T) + 16 * (c % CPR)) = v;
+        });
 #endif
 }
 
