@@ -239,10 +239,13 @@ __global__ __launch_bounds__(256, 1) void colf_kernel(ColArgs a) {
             const bool qvalid = qrow < S, diag = key0 == qstart;
             const float er = !qvalid ? 0.f : fast_exp2((float)((double)(amaxA + nbeta) + crow));
             const float inv_er = inv * er, dbv_er = dbv * er;
+            // keys above this one, counted from 4 h, are masked.  (As a condition on the weight, each element of the diagonal granule was a branch
+            // of its own: 17.4 us, now 16.6, at D = 64, 4 x 2048; D = 128, 32 x 4096: 337 -> 328.)
+            const int lastkey = !qvalid ? -1 : diag ? c32 - 4 * h : 32;
             auto element = [&](auto first_tag, int x) __attribute__((always_inline)) {
                 if constexpr (decltype(first_tag)::value) {
-                    float e = fast_exp2((al[x] + nbeta) + (float)crow);
-                    if (!qvalid || (diag && (8 * (x >> 2) + 4 * h + (x & 3) > c32))) e = 0.f;
+                    const bool masked = 8 * (x >> 2) + (x & 3) > lastkey;
+                    const float e = fast_exp2(masked ? -INFINITY : (al[x] + nbeta) + (float)crow);
                     const float ct = s[x] * e;
                     const float dct = fmaf(d[x], inv, dbv);
                     dd[x] = product_apart(ct, dct);   // (as in col_kernel)
