@@ -15,6 +15,7 @@
 //   chunk_sum_narrow_kernel  the same sums, bit for bit, on 64 x 64 blocks, for few heads.
 //   chunk_carry_kernel  C~_c = gamma_c C~_{c-1} + dC_c over the chunks of a head (gamma_c = exp(A_{e_{c-1}} - A_{e_c})),
 //                       element-wise, written in the element type; n~_c likewise, in place, fp32.
+//   chunk_seq_kernel    both in one pass, bit for bit, for launches that fill the chip.
 //   chunk_sum_small_kernel, chunk_carry_small_kernel  the same two steps for fp32 and for 16-bit types at D = 64 (fp32 MFMA).
 //   chunk_sum_terms_kernel  the chunk sums of bf16 at D = 64, outside split mode, with the weighted values as three bf16 terms.
 // State rows are stored in the order in which the row kernel's second product contracts them (see PERM16 below).
