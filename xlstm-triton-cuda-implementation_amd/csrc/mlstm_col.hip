@@ -727,9 +727,9 @@ static int launch_col_d(int D, const ColArgs& a, hipStream_t st) {
     return MLSTM_ESHAPE;
 }
 
-// col_kernel / colf_kernel, fp32, workgroups of 32 keys, us: D = 64, chunks of 128   128: 23.9 / 16.7   256: 25.6 / 18.1   320: 26.1 / 30.0
-//   uncut (300 positions)   240: 34.5 / 26.7   480: 36.8 / 38.1     D = 128, chunks of 128   256: 46.5 / 25.7   512: 50.0 / 45.3
-//   2048: 198 / 170   8192: 748 / 655   uncut   480: 60 / 50   1000: 101 / 105
+// col_kernel / colf_kernel, fp32, workgroups of 32 keys, us: D = 64, chunks of 128   128: 21.5 / 14.8   256: 22.9 / 16.0   320: 23.4 / 27.8
+//   uncut (300 positions)   240: 32.1 / 26.4   480: 34.1 / 37.0     D = 128, chunks of 128   256: 45.6 / 25.0   512: 49 / 45
+//   1024: 94.5 / 81   2048: 169 / 160   8192: 617 / 647   uncut   480: 60 / 48   1000: 100 / 103
 bool colf_serves(int dtype, int D, const ColArgs& a) {
     if (dtype != MLSTM_F32 || D > 128 || g_force_generic || a.RS > D || (a.chunk_len > 0 ? a.chunk_len > 1024 : a.S > 2048)) return false;
     const long long wgs = 2ll * a.BH * a.NG;

@@ -221,14 +221,15 @@ inline bool colw_serves(int dtype, int D, const ColArgs& a) {
     if (dtype == MLSTM_F32 || (D != 128 && D != 256) || g_force_generic || g_col_variant != 0) return false;
     if ((a.chunk_len > 0 && a.chunk_len < a.NG * GATE_GRANULE ? a.chunk_len : a.NG * GATE_GRANULE) > CW_MOST_QUERIES) return false;
     // Workgroups of 64 keys up to which colw_kernel is the faster one; cold_kernel / colw_kernel, us (bf16, workgroups of 64 keys):
-    //   D = 128, S = 1000 (not in chunks)  256: 57 / 30   512: 61 / 39   768: 80 / 60
-    //   D = 128 in chunks of 512           256: 37 / 22   512: 39 / 32   768: 44 / 48    in split mode   128: 38 / 26   256: 40 / 28   512: 43 / 41   768: 61 / 60
-    //   D = 256, S = 1000                   64: 69 / 40   256: 72 / 45   512: 76 / 57
-    //   D = 256 in chunks                  128: 51 / 33   256: 53 / 36   512: 56 / 54   768: 82 / 82
-    //   D = 256 in split mode              128: 65 / 42   256: 67 / 47   512: 72 / 70   768: 108 / 103
-    //   fp16 (at D = 256 with 50 registers spilled where bf16 has 8, one or two reloads per tile of a weighing wave): D = 128, S = 1000  768: 74 / 54   in chunks 512: 37 / 30   768: 49 / 49
-    //     in split mode 768: 57 / 53      D = 256, S = 1000  768: 131 / 89   in chunks 512: 68 / 58   768: 107 / 86   in split mode 768: 128 / 104
-    return (long long)a.BH * a.NG <= (D == 128 && a.chunk_len > 0 && !a.precise ? 512 : 768);
+    //   D = 128, S = 1000 (not in chunks)  256: 56 / 29   512: 59 / 38   768: 65 / 57   1024: 66 / 68    (S = 300, 640: 24.6 / 26.4)
+    //   D = 128 in chunks of 512           256: 35 / 21   512: 37 / 30   544: 41 / 37.5   640: 45 / 38.5   768: 47 / 42   1024: 49 / 53
+    //     in split mode                    128: 38 / 26   256: 39 / 27   512: 42 / 40   768: 58 / 57   1024: 60 / 73
+    //   D = 256, S = 1000                   64: 69 / 40   256: 71 / 44   512: 74 / 58   768: 79 / 89 (fp16 88 / 87)   1024: 97 / 118
+    //   D = 256 in chunks                  128: 51 / 32   256: 51 / 34   512: 56 / 53   768: 81 / 80   1024: 86 / 103
+    //   D = 256 in split mode              128: 64 / 41   256: 65 / 44   512: 70 / 66   768: 105 / 99   1024: 110 / 130
+    //   fp16 (at D = 256 with 50 registers spilled where bf16 has 10, one or two reloads per tile of a weighing wave): D = 128, S = 1000  768: 58 / 51
+    //     in chunks 512: 35 / 27   640: 43 / 36   768: 46 / 40   832: 41.5 / 46   in split mode 768: 55 / 51      D = 256 in chunks 512: 66 / 53   768: 103 / 79   in split mode 768: 123 / 99
+    return (long long)a.BH * a.NG <= 768;
 }
 inline int launch_col_best(int dtype, int D, const ColArgs& a, hipStream_t st) {
     const bool half_big = dtype != MLSTM_F32 && (D == 128 || D == 256);
