@@ -74,10 +74,12 @@ __global__ __launch_bounds__(512) void row8_kernel(RowArgs a) {
             // Workgroups go round-robin to the 8 XCDs: XCD x gets the heads x, x + 8, ... and works on them two at a
             // time, heaviest row tiles first (K and V of two heads are 8 MB at S = 4096, D = 256 against 4 MB of L2 per
             // XCD; all heads of an XCD at once measured 1 % slower, one head at a time 7 % slower: its last, light tiles
-            // leave CUs idle at every change of head).
+            // leave CUs idle at every change of head).  Up to two rounds of workgroups, short uncut sequences, the changes of pair cost more: all
+            // together, D = 256, forward / dQ, us: 40 x 1000 40.7, 48.0 -> 31.6, 38.0   64 x 1000 50.6, 57.6 -> 44.3, 53.3   64 x 600 28.3, 36.5 -> 25.4, 32.4;
+            // beyond, 128 x 600 45.3, 58.0 -> 52.8, 64.8   256 x 300 40.2, 52.6 -> 48.5, 61.9   128 x 1000 103, 119 -> 101, 118.
             const int rest = bid >> 3, ngrp = a.BH >> 3;
             const int paired = (ngrp >> 1) * 2 * nQT;   // workgroups of this XCD that belong to complete pairs of heads
-            if (a.chunk_len > 0) {
+            if (a.chunk_len > 0 || a.BH * nQT <= 512) {
                 // In chunks a row tile reads the keys of its own chunk and one state, so the L2 holds what many heads
                 // need at once, and what counts is the balance: all heads of the XCD together (4.5 % faster than in
                 // pairs at D = 256, 4 % at D = 128; one head at a time 5 % slower than in pairs).
