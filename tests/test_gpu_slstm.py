@@ -118,6 +118,29 @@ def test_gates_far_from_zero_stay_finite():
     assert_close(h, SO.slstm_forward(wx, r, b), torch.float32, "h")
 
 
+@pytest.mark.parametrize("forget_sigmoid", [False, True])
+@pytest.mark.parametrize("DH", [32, 64, 128])
+def test_a_pre_activation_takes_its_input_last(DH, forget_sigmoid):
+    # From the kernel's own h_{t-1}, so that only one step's roundings are left.  A rounding at the size of x has the variance ulp(x)^2 / 12.  There is one of
+    # wx + b and one of the whole sum; the recurrent sum, eight chains of DH / 8 multiply-adds and three levels of adds, has at most DH / 8 + 3 on the way of each of
+    # its terms, at the size of what it adds up alone.  With the input ahead of the recurrent sum, those are at the size of the whole: 1.8 (DH = 32) to 2.6 (128)
+    # times the root mean square that this predicts, where the input last is at 0.9 (both orders on the CPU).
+    from slstm import slstm_forward_hip
+    B, NH, S = 4, 2, 200
+    wx, r, b, _ = (x.double() for x in SO.make_inputs(B, NH, S, DH, seed=DH))
+    h, saved = slstm_forward_hip(*gpu(wx.float(), r.float(), b.float()), forget_sigmoid=forget_sigmoid)
+    before = torch.cat([torch.zeros(B, 1, NH, DH).double(), h[:, :-1].double().cpu()], 1)
+    recurrent = lambda m, v: torch.matmul(m, v.unsqueeze(3).unsqueeze(-1)).squeeze(-1).transpose(2, 3)  # noqa: E731  [B,S,4,NH,DH]
+    given = wx + b.transpose(0, 1)
+    want = given + recurrent(r, before)
+    ulp = lambda x: 2.0 ** (x.abs().clamp_min(1e-30).log2().floor() - 23)  # noqa: E731
+    variance = (ulp(given) ** 2 + ulp(want) ** 2 + (DH / 8 + 3) * 2.0 ** -46 * recurrent(r ** 2, before ** 2)) / 12
+    kept = saved.view(torch.float32).view(B, S, 7, NH, DH)
+    for gate in (0,) if forget_sigmoid else (0, 1):   # what is kept of the other gates has been through their nonlinearity
+        error = kept[:, :, gate].double().cpu() - want[:, :, gate]
+        assert error.square().mean() <= 1.25 ** 2 * variance[:, :, gate].mean(), (gate, error.square().mean().sqrt(), variance[:, :, gate].mean().sqrt())
+
+
 def test_autograd_function_and_repeatability():
     from slstm import slstm
     wx, r, b, dh = SO.make_inputs(2, 2, 64, 64, seed=7)

@@ -66,7 +66,7 @@ __device__ __forceinline__ float pick(bool is0, bool is1, bool is2, float a, flo
 // A quad of lanes owns a unit j, an octet two of them: lane p of the octet keeps, for all four gates of both units, part p (an
 // eighth) of their rows of R_g and forms its part of the eight pre-activations from its part of h_{t-1}.  Lane q of a quad holds
 // gate q ^ s of its own unit, and q ^ 3 ^ s of the other, as its s-th, so that seven exchanges with an add each (the octet's mirror
-// image, then the quad) leave the whole sum of gate q in lane q, which began its sum with the input; it applies that gate's nonlinearity
+// image, then the quad) leave the whole sum of gate q in lane q, which adds the input last; it applies that gate's nonlinearity
 // (one exp2, one reciprocal, one logarithm serve the three kinds side by side), the quad exchanges the four results -- i~ before there is an
 // exponential, each from where it is formed, so that the selects that make one value per lane of them are needed for the saved state alone --
 // and every lane updates the cell, all four alike (c, n, m are kept four times, the same bits).  A step has no hand-over between waves but h itself: one LDS write,
@@ -81,8 +81,10 @@ __device__ __forceinline__ float pick(bool is0, bool is1, bool is2, float a, flo
 // Forward, B16 NH4, us, quarters / eighths / helpers: DH = 64, S = 2048 716 / 690 / 613; DH = 128, S = 1024 627 / 559 / 553 (545 without the saved state); DH = 32,
 // S = 1024 285 / 281 / 246.  DH = 32, eighths / helpers, by workgroups: 256, S = 300 85 / 75; 512, S = 200 70.2 / 71.5 (two on a CU, the helpers of either on a
 // SIMD with a walk of the other); 1024 110 / 84.
-// With selects before the exchange / the exchange straight from the gates, without the saved state: DH = 64 613 / 597, DH = 128 533 / 517, DH = 32 241 / 235 and by
-// workgroups (256, 512, 1024) 74.1 / 72.5, 70.8 / 63.0, 72.0 / 67.9; with it 614 / 605, 552 / 544, 244 / 240 and (256, 512) 75.4 / 74.2, 72.2 / 65.4.
+// With selects before the exchange / the exchange straight from the gates, without the saved state: DH = 64 614 / 602, DH = 128 537 / 530, DH = 32 245 / 240 and by
+// workgroups (256, S = 300; 512, 200; 1024, 100) 74.5 / 72.8, 71.1 / 67.4, 38.6 / 36.6; with it 617 / 610, 558 / 549, 246 / 242 and 75.6 / 74.6, 71.9 / 70.6, 39.8 / 39.4.
+// (The input as the first term of its lane's sum would save the add at the end, 4, 11 and 2 us of these, and round every multiply-add behind it at the
+// size of the whole pre-activation: its error by root mean square 1.9, 2.3 and 2.9 times as large at DH = 32, 64 and 128.)
 template <int DH>
 struct FwdCfg {
     static constexpr int UW = DH > 64 ? DH / 64 : 1;   // helper waves: a 16-byte piece of a step's input per lane
@@ -146,9 +148,10 @@ __global__ __launch_bounds__(FwdCfg<DH>::THREADS) void slstm_forward_kernel(cons
             for (int k = 0; k < AHEAD; k++) hv[k] = *reinterpret_cast<const f32x4*>(hcur + 4 * k);
             __builtin_amdgcn_sched_barrier(0);
             keep((u & 1) ^ 1);   // (at t = 0 nothing that is read)
-            float a[4] = {wv + bq, 0.f, 0.f, 0.f}, x4[4] = {0.f, 0.f, 0.f, 0.f};
+            const float in = wv + bq;
             wv = ring[(u + 1) % PF][in_at];
             __builtin_amdgcn_sched_barrier(0);
+            float a[4] = {0.f, 0.f, 0.f, 0.f}, x4[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int k = 0; k < KP / 4; k++) {
 #pragma unroll
@@ -168,7 +171,7 @@ __global__ __launch_bounds__(FwdCfg<DH>::THREADS) void slstm_forward_kernel(cons
 #pragma unroll
             for (int s = 0; s < 4; s++) a[s] += quad_perm<0x141>(x4[s]);   // row_half_mirror
             // (what the other lanes need goes to them as each lane has it, whether it is that lane's gate or not; the selects are off the chain)
-            const float x = (a[0] + quad_perm<0xB1>(a[1])) + (quad_perm<0x4E>(a[2]) + quad_perm<0x1B>(a[3]));
+            const float x = ((a[0] + quad_perm<0xB1>(a[1])) + (quad_perm<0x4E>(a[2]) + quad_perm<0x1B>(a[3]))) + in;
             const float it = quad_perm<0x00>(x);
             const float e = __builtin_amdgcn_exp2f(coef * __builtin_bit_cast(float, __builtin_bit_cast(unsigned, x) & sign_off));
             const float d = 1.0f + e, rd = fast_rcp(d);
