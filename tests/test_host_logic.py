@@ -91,6 +91,16 @@ def test_gates_formed_in_a_row_kernel_go_to_that_kernel_alone():
     assert out.returncode == 0 and "row_dispatch: ok" in out.stdout, out.stdout + out.stderr
 
 
+@pytest.mark.parametrize("scratch", [[], ["scratch"]])
+def test_chunk_states_of_a_kernel_with_scratch_memory_go_to_the_two_others(scratch):
+    """tests/harness/chunk_dispatch (the library's own choice of the kernels of the chunk states, compiled for the host): a one-pass kernel that a compiler
+    gave scratch memory is replaced where the library chose it and refused where the caller named it."""
+    here = os.path.join(os.path.dirname(os.path.abspath(__file__)), "harness")
+    subprocess.check_call(["make", "-C", here, "chunk_dispatch"])
+    out = subprocess.run([os.path.join(here, "chunk_dispatch"), *scratch], capture_output=True, text=True)
+    assert out.returncode == 0 and "cases ok" in out.stdout, out.stdout + out.stderr
+
+
 def test_operators_do_without_the_native_host_path(monkeypatch):
     """The extension belongs to one torch release; missing, or another release's, it is left out with a warning and the calls go
     through ctypes (every function says that it serves nothing)."""

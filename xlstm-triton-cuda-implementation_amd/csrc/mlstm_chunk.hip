@@ -1190,7 +1190,7 @@ __global__ __launch_bounds__(256, 4) void chunk_carry_t_kernel(ChunkArgs a) {
 // 1900 cycles per tile where the products need 1100.)  One barrier per tile; behind it tiles t and t + 1 and the weights
 // of both are there.  The copies are counted by hand: a copying wave issues exactly NI direct loads per tile and no other vector
 // memory operation, and waits with vmcnt((PF - 2) * NI) -- everything but the newest PF - 2 tiles -- before the barrier
-// that hands a tile on; the launch is refused if the compiled kernel uses scratch memory.
+// that hands a tile on; a compiled kernel that uses scratch memory is not launched (launch_chunk_t then takes the two kernels).
 template <typename T, int D>
 struct SeqCfg {
     static constexpr int KR = 64, VW = D / 2;
@@ -1628,12 +1628,12 @@ __global__ __launch_bounds__(512) void chunk_seq_kernel(ChunkArgs a) {
 //             32 x 7: 207, 231, 491 / 182, 215, 480   64 x 3: 193, 216, 463 / 175, 203, 453    (D = 128 64 x 3: 76.1, 84.2, 212 / 75.6, 82.9, 213   96 x 7: 224, 254, 646 / 237, 267, 664)
 int g_state_kernel = 0;   // 0 = the rule, 1 = chunk sums + carry, 2 = one pass where it can serve
 template <typename T, int D>
-static bool chunk_seq_serves(const ChunkArgs& a) {
+static bool chunk_seq_serves(const ChunkArgs& a, int form) {   // form: see g_state_kernel
     using Cfg = SeqCfg<T, D>;
-    if ((a.precise && D == 128) || a.NCS > Cfg::MAX_STEPS || (a.Cst && a.dot_part) || g_state_kernel == 1) return false;
+    if ((a.precise && D == 128) || a.NCS > Cfg::MAX_STEPS || (a.Cst && a.dot_part) || form == 1) return false;
     constexpr long long CUS = 256;
     const long long wgs = (long long)a.BH * Cfg::WPH, rounds = (wgs + CUS - 1) / CUS;
-    return g_state_kernel == 2 || 4 * wgs >= 3 * CUS * rounds || (rounds == 1 && 32ll * a.NCS <= wgs && (!a.precise || 8 * wgs >= 3 * CUS));
+    return form == 2 || 4 * wgs >= 3 * CUS * rounds || (rounds == 1 && 32ll * a.NCS <= wgs && (!a.precise || 8 * wgs >= 3 * CUS));
 }
 template <typename T, int D, bool STRICT, bool KM, bool VM, bool DOT>
 static int launch_chunk_seq_t(const ChunkArgs& a, hipStream_t st) {
@@ -1707,11 +1707,13 @@ static int launch_chunk_carry_small(const ChunkArgs& a, hipStream_t st) {
 template <typename T, int D>
 static int launch_chunk_t(const ChunkArgs& a, hipStream_t st) {
     if (a.precise && ((a.Cst && !a.Cst_lo) || (a.CstT && !a.CstT_lo))) return MLSTM_EINVAL;
-    if (chunk_seq_serves<T, D>(a)) {
-        if constexpr (D == 256) {
-            if (a.precise) return launch_chunk_seq<T, D, true>(a, st);
-        }
-        return launch_chunk_seq<T, D, false>(a, st);
+    const int form = g_state_kernel;
+    if (chunk_seq_serves<T, D>(a, form)) {
+        int rc;
+        if constexpr (D == 256) rc = a.precise ? launch_chunk_seq<T, D, true>(a, st) : launch_chunk_seq<T, D, false>(a, st);
+        else rc = launch_chunk_seq<T, D, false>(a, st);
+        // (not launched because the compiler gave the kernel scratch memory: the two kernels give the same bits; refused only where the form is named)
+        if (rc != MLSTM_EBUILD || form == 2) return rc;
     }
     if (int rc = a.precise ? launch_chunk_sum<T, D, true>(a, st) : launch_chunk_sum<T, D, false>(a, st)) return rc;
     // one carry kernel: the value-major one writes both layouts and the vector states

@@ -18,8 +18,8 @@ inline hipError_t lds_limit_once(int bytes) {
 // For kernels that wait in every step for memory that is counted by hand (s_waitcnt vmcnt(n) with n the operations the SOURCE issues behind the
 // ones it waits for).  Operations that the count does not know, the compiler's own for a spilled register among them, never let a load pass
 // as landed that has not: they only push counted ones out of the newest n, and the wait takes in copies that were meant to stay under
-// way.  In a step that is all latency that is its whole point gone, so the launch is refused (MLSTM_EBUILD) if the compiled kernel uses any
-// scratch memory at all.  Asked once per process and kernel.
+// way.  In a step that is all latency that is its whole point gone, so the kernel is not launched (MLSTM_EBUILD) if it was compiled to use any
+// scratch memory at all; where others give the same results (launch_chunk_t), they take its place.  Asked once per process and kernel.
 template <auto KERN>
 inline int no_scratch_once() {
     static const int rc = [] {
