@@ -562,8 +562,8 @@ __global__ __launch_bounds__(256, D == 128 && !STRICT ? 2 : 1) void cold_kernel(
     }
 #undef COLD_DMA
 
-    // (Each piece of the epilogue used to wait for its own LDS read, 64 of them one behind the other; with the vector state a block
-    // ahead and the copies read eight at a time, and the V tile's copy above without clamps, bf16: D = 128, 64 heads x 16384: 601 -> 586 us;
+    // (Each piece of the epilogue used to wait for its own LDS read, 64 of them one behind the other; with the vector state a block at a
+    // time and the copies read eight at a time, and the V tile's copy above without clamps, bf16: D = 128, 64 heads x 16384: 601 -> 586 us;
     // D = 256, 32 x 4096: 192.3 -> 190.8.)
     // ---- epilogue: column sums, the last step's row sums, then dK and dV through LDS (the V tile and the stages are free
     // once every wave is past its last phase B): rows of D elements, 16-byte chunk c of row r at chunk c ^ (r & 31), so that
@@ -585,36 +585,38 @@ __global__ __launch_bounds__(256, D == 128 && !STRICT ? 2 : 1) void cold_kernel(
         static_assert(2 * (size_t)CD_KEYS * ROWB <= Cfg::V_BYTES + Cfg::STAGES_BYTES, "both staged outputs fit the V tile and the stages");
         const float s_end = !END_SCALE ? 1.f : LEAN ? keyvals[2 * CD_KEYS + 32 * kb + c32] : scale_s;   // the keys' weights: see the state phase
         auto stage_out = [&](auto which_tag, auto state_tag) __attribute__((always_inline)) {
-            constexpr bool which = decltype(which_tag)::value, STATE = decltype(state_tag)::value;
+            constexpr bool which = decltype(which_tag)::value, STATE = decltype(state_tag)::value, AHEAD = STATE && D == 128;
             char* const out = smem + (size_t)which * CD_KEYS * ROWB;
             const int row = 32 * kb + c32;
-            // (the vector state a block ahead: read where it is added, each piece would wait for its own)
-            f32x4 gq[2][4];
+            // (the vector state: read piece by piece where it is added, each piece would wait for its own.  D = 128: a block ahead.  D = 256, where the accumulators
+            // leave no registers for that -- 6 were spilled, in split mode 7, and 20 MB more moved at 32 heads x 4096 -- a block's four at once, under a branch that
+            // keeps them there: 181.1 -> 180.0 us, split mode 236.0 -> 234.0, 64 x 1000 uncut 103.4 -> 102.2; piece by piece 1 % slower than either)
+            f32x4 gq[AHEAD ? 2 : 1][4];
             auto read_g = [&](int x) __attribute__((always_inline)) {
 #pragma unroll
-                for (int a4 = 0; a4 < 4; a4++) gq[x & 1][a4] = *reinterpret_cast<const f32x4*>(gvl + 32 * x + 8 * a4 + 4 * h);
+                for (int a4 = 0; a4 < 4; a4++) gq[x % (AHEAD ? 2 : 1)][a4] = *reinterpret_cast<const f32x4*>(gvl + 32 * x + 8 * a4 + 4 * h);
             };
-            if constexpr (STATE) read_g(0);
+            if constexpr (AHEAD) read_g(0);
 #pragma unroll
             for (int x = 0; x < NXD; x++) {
-                if constexpr (STATE) { if (x + 1 < NXD) read_g(x + 1); }
+                if constexpr (AHEAD) { if (x + 1 < NXD) read_g(x + 1); }
+                f32x16& acc = which ? dvacc[x] : dkacc[x];
+                if constexpr (END_SCALE) acc *= s_end;
+                if (AHEAD || (STATE && has_state)) {
+                    if constexpr (!AHEAD) read_g(x);
+#pragma unroll
+                    for (int r = 0; r < 16; r++) acc[r] = fmaf(gq[x % (AHEAD ? 2 : 1)][r >> 2][r & 3], wkg, acc[r]);
+                }
 #pragma unroll
                 for (int a4 = 0; a4 < 4; a4++) {
                     const int d = 32 * x + 8 * a4 + 4 * h;               // first of the four columns
-                    f32x4 v;
-#pragma unroll
-                    for (int c = 0; c < 4; c++) v[c] = which ? dvacc[x][4 * a4 + c] : dkacc[x][4 * a4 + c];
-                    if constexpr (END_SCALE) v *= s_end;
-                    if constexpr (STATE) {
-#pragma unroll
-                        for (int c = 0; c < 4; c++) v[c] = fmaf(gq[x & 1][a4][c], wkg, v[c]);
-                    }
+                    const f32x4 v = {acc[4 * a4], acc[4 * a4 + 1], acc[4 * a4 + 2], acc[4 * a4 + 3]};
                     const int chunk16 = (d * (int)sizeof(T)) >> 4, within = (d * (int)sizeof(T)) & 15;
                     *reinterpret_cast<typename R::vec4*>(out + row * ROWB + (((chunk16 ^ (row & 31)) & (CPR - 1)) << 4) + within) = R::cvt4(v);
                 }
             }
         };
-        if (END_SCALE && has_state) stage_out(std::false_type{}, std::integral_constant<bool, END_SCALE>{});
+        if (END_SCALE && (D == 256 || has_state)) stage_out(std::false_type{}, std::integral_constant<bool, END_SCALE>{});
         else stage_out(std::false_type{}, std::false_type{});
         stage_out(std::true_type{}, std::false_type{});
         __syncthreads();
