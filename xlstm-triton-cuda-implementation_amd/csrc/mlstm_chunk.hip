@@ -33,6 +33,17 @@ namespace mlstm {
 __device__ __forceinline__ int perm16(int u) { return (u & ~12) | ((u & 4) << 1) | ((u & 8) >> 1); }
 __device__ __forceinline__ int state_row(int u) { return (u & ~15) | perm16(u & 15); }
 
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+
+// What the chunk sums read for a position past the sequence's end: a piece of zeros.  (The sequence's last row in its place, with a weight of 0, would make
+// every sum that an infinity or NaN of that row enters NaN; and how many such rows a kernel reads depends on its tiles.)
+__device__ const u32x4 zero_piece = {0, 0, 0, 0};
+// A piece of a row, if the row is there.  (Both addresses as global ones: constants have an address space of their own, and a choice between the two is a flat
+// load, whose waits cost the sums 3 to 7 %; a variable that is no constant has its address fetched from memory.)
+typedef const __attribute__((address_space(1))) u32x4* GlobalPiece;
+__device__ __forceinline__ u32x4 piece_or_zeros(bool there, const void* piece) { return *(there ? (GlobalPiece)(size_t)piece : (GlobalPiece)(size_t)&zero_piece); }
+
+
 // STRICT: split mode, the weighted V rows go to LDS as two tiles, hi and lo (ChunkArgs::precise)
 template <typename T, int D, bool STRICT = false>
 struct ChunkCfg {
@@ -44,8 +55,6 @@ struct ChunkCfg {
     static constexpr size_t TILE_BYTES = STAGES * (K_BYTES + V_BYTES);   // plus one float per position of the chunk
     static constexpr int MAX_L = (int)((160 * 1024 - TILE_BYTES) / (2 * sizeof(float))) / 128 * 128;
 };
-
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 
 // Eight 16-bit elements (four dwords) as floats.  bf16 by hand: one shift or mask per element (the generic vector
 // conversion costs several instructions per element, in a kernel that is bound by instruction issue).
@@ -114,17 +123,17 @@ __global__ __launch_bounds__(512) void chunk_sum_kernel(ChunkArgs a) {
     f32x8 nacc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     // Tiles travel memory -> registers -> LDS.  A thread's pieces of a tile: KP 16-byte pieces of K (piece tid + 256 it of
     // the tile's rows of CPR pieces) and four of V (rows tid/16 + 16 it, piece tid%16); tile j uses register set j % 3 and
-    // LDS stage j % 2.  Rows past the end of the sequence are clamped (their weights are 0).
+    // LDS stage j % 2.  Rows past the end of the sequence are zeros.
     constexpr int KP = GRAN * ZK::CPR / 256, LPT = KP + 4;   // loads per thread and tile
     const int vrow = tid >> 4, vch = tid & 15;
     u32x4 kset[Cfg::RSETS][KP], vset[Cfg::RSETS][4];
     // A thread's pieces lie a fixed number of rows apart (K: 256 / CPR, V: 16): one per-lane element offset each, everything
-    // else of an address is the same for all lanes.  Only the last tile of a short last chunk needs its rows clamped.
+    // else of an address is the same for all lanes.  Only the tiles of a short last chunk need a look at each row.
     constexpr int KROWS = 256 / ZK::CPR;
     const unsigned koff = (unsigned)((tid / ZK::CPR) * rsK + 8 * (tid % ZK::CPR)), voff = (unsigned)(vrow * rsV + 8 * vch);
     auto issue = [&](auto set_tag, int j) __attribute__((always_inline)) {
         constexpr int P = decltype(set_tag)::value;
-        if (p0 + GRAN * (j + 1) <= S) {
+        if (__builtin_expect(p0 + GRAN * (j + 1) <= S, 1)) {
             const T* kt = Kh + (size_t)GRAN * j * rsK;
             const T* vt = Vh + (size_t)GRAN * j * rsV;
 #pragma unroll
@@ -134,16 +143,13 @@ __global__ __launch_bounds__(512) void chunk_sum_kernel(ChunkArgs a) {
         } else {
 #pragma unroll
             for (int it = 0; it < KP; it++) {
-                const int pc = tid + 256 * it;
-                int pos = GRAN * j + pc / ZK::CPR;
-                pos = p0 + pos < S ? pos : S - 1 - p0;
-                kset[P][it] = *reinterpret_cast<const u32x4*>(Kh + (size_t)pos * rsK + 8 * (pc % ZK::CPR));
+                const int pc = tid + 256 * it, pos = GRAN * j + pc / ZK::CPR;
+                kset[P][it] = piece_or_zeros(p0 + pos < S, Kh + (size_t)pos * rsK + 8 * (pc % ZK::CPR));
             }
 #pragma unroll
             for (int it = 0; it < 4; it++) {
-                int pos = GRAN * j + vrow + 16 * it;
-                pos = p0 + pos < S ? pos : S - 1 - p0;
-                vset[P][it] = *reinterpret_cast<const u32x4*>(Vh + (size_t)pos * rsV + 8 * vch);
+                const int pos = GRAN * j + vrow + 16 * it;
+                vset[P][it] = piece_or_zeros(p0 + pos < S, Vh + (size_t)pos * rsV + 8 * vch);
             }
         }
         __builtin_amdgcn_sched_barrier(0);   // the loads go out here, not where the scheduler would like them
@@ -427,18 +433,30 @@ __global__ __launch_bounds__(256) void chunk_sum_narrow_kernel(ChunkArgs a) {
     const int vrow = tid / Z::CPR, vch = tid % Z::CPR;
     u32x4 vset[NP];
     const bool whole = p0 + L <= S;
-    auto row_of = [&](int r) { return whole || p0 + r < S ? r : S - 1 - p0; };   // (rows past the end, with weights of 0, become its last)
+    auto request_v = [&](auto whole_tag) __attribute__((always_inline)) {   // (rows past the end are zeros)
 #pragma unroll
-    for (int i = 0; i < NP; i++) vset[i] = *reinterpret_cast<const u32x4*>(Vh + (size_t)row_of(vrow + 32 * i) * rsV + Z::EPC * vch);
+        for (int i = 0; i < NP; i++) {
+            const int r = vrow + 32 * i;
+            vset[i] = piece_or_zeros(decltype(whole_tag)::value || p0 + r < S, Vh + (size_t)r * rsV + Z::EPC * vch);
+        }
+    };
+    if (whole) request_v(std::true_type{});
+    else request_v(std::false_type{});
     // K: 1 KB (eight rows) per load of a wave; piece c of row r at piece c ^ key(r) of the row
     auto copy_k = [&](int p) __attribute__((always_inline)) {
         const unsigned kbase = lds_offset_of(kpart(p));
         const int kr = lane / Z::CPR, kc = lane % Z::CPR;
+        auto rows = [&](auto whole_tag) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < PART / 32; i++) {
-            const int r = 32 * i + 8 * wave;
-            dma16(Kh + (size_t)row_of(PART * p + r + kr) * rsK + Z::EPC * (kc ^ Z::key(r + kr)), __builtin_amdgcn_readfirstlane(kbase + r * Z::ROW_BYTES));
-        }
+            for (int i = 0; i < PART / 32; i++) {
+                const int r = 32 * i + 8 * wave;
+                const T* piece = Kh + (size_t)(PART * p + r + kr) * rsK + Z::EPC * (kc ^ Z::key(r + kr));
+                if (!decltype(whole_tag)::value && p0 + PART * p + r + kr >= S) piece = reinterpret_cast<const T*>(&zero_piece);
+                dma16(piece, __builtin_amdgcn_readfirstlane(kbase + r * Z::ROW_BYTES));
+            }
+        };
+        if (whole) rows(std::true_type{});
+        else rows(std::false_type{});
     };
     copy_k(0);
     if constexpr (STRICT) copy_k(1);
@@ -1272,6 +1290,7 @@ __global__ __launch_bounds__(512) void chunk_seq_kernel(ChunkArgs a) {
     };
     if (feeder && wave < 2) {   // ---- copies
         const size_t rsK = (size_t)a.lk.ss, rsV = (size_t)a.lv.ss;
+        const T* const zeros = reinterpret_cast<const T*>(&zero_piece);
         const T* Kh = reinterpret_cast<const T*>(a.K) + a.lk.head(bh) + 64 * kq;
         const T* Vh = reinterpret_cast<const T*>(a.V) + a.lv.head(bh) + VW * vh;
         TileDma<T, 64, GRAN, 128> kdma;
@@ -1315,9 +1334,9 @@ __global__ __launch_bounds__(512) void chunk_seq_kernel(ChunkArgs a) {
             if (__builtin_expect(pos_i + GRAN <= S, 1)) {
                 kdma.issue(ks, kp, krows);
                 vdma.issue(vs, vp, vrows);
-            } else {   // the sequence's last tile: rows past the end are clamped (their weights are 0)
-                tile_dma_rolled<T, 64, GRAN, 128>(ks, Kh, pos_i, S, tid, rsK);
-                tile_dma_rolled<T, VW, GRAN, 128>(vs, Vh, pos_i, S, tid, rsV);
+            } else {   // the sequence's last tile: rows past the end are zeros
+                tile_dma_rolled<T, 64, GRAN, 128>(ks, Kh, pos_i, S, tid, rsK, zeros);
+                tile_dma_rolled<T, VW, GRAN, 128>(vs, Vh, pos_i, S, tid, rsV, zeros);
             }
         };
         // the positions' weights of tile n (see chunk_sum_kernel), by the two waves in turns

@@ -424,9 +424,10 @@ __device__ __forceinline__ void tile_dma(T* tile, const T* g, int row0, int S, i
 }
 
 // The same copy as a loop that stays a loop, for the places where it rarely runs (a sequence's last, partial tile) but would
-// otherwise keep one 64-bit address per block alive across code that needs every register.
+// otherwise keep one 64-bit address per block alive across code that needs every register.  past: 16 bytes of memory that take
+// the place of every piece of the rows past S-1.
 template <typename T, int D, int ROWS, int NT>
-__device__ __forceinline__ void tile_dma_rolled(T* tile, const T* g, int row0, int S, int tid, size_t row_stride = D) {
+__device__ __forceinline__ void tile_dma_rolled(T* tile, const T* g, int row0, int S, int tid, size_t row_stride = D, const T* past = nullptr) {
     using Z = Swz<T, D>;
     constexpr int NW = NT / 64, BLOCKS = ROWS * Z::CPR / 64;
     static_assert(BLOCKS % NW == 0, "tile must divide evenly over the waves");
@@ -438,9 +439,10 @@ __device__ __forceinline__ void tile_dma_rolled(T* tile, const T* g, int row0, i
         const int p = blk * 64 + lane;
         const int r = p / Z::CPR, pc = p % Z::CPR;
         const int c = pc ^ Z::key(r);
-        int gr = row0 + r;
-        gr = gr < S ? gr : S - 1;
-        dma16(g + (size_t)gr * row_stride + c * Z::EPC, __builtin_amdgcn_readfirstlane(base + blk * 1024));
+        const int gr = row0 + r;
+        const T* src = g + (size_t)(gr < S ? gr : S - 1) * row_stride + c * Z::EPC;
+        if (past) src = gr < S ? src : past;
+        dma16(src, __builtin_amdgcn_readfirstlane(base + blk * 1024));
     }
 }
 
