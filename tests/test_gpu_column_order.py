@@ -20,6 +20,9 @@ def _grads(x, dh, precise):
     ("bf16", 64, False, 16, 1700), ("f16", 64, False, 40, 300), ("bf16", 64, True, 16, 1700), ("f32", 64, False, 16, 1700), ("f32", 64, False, 64, 300),
     ("bf16", 128, False, 32, 1700), ("bf16", 128, False, 64, 1000), ("bf16", 128, False, 17, 2048), ("f16", 128, False, 24, 2048), ("bf16", 128, False, 25, 2048),
     ("bf16", 256, False, 32, 1700), ("bf16", 256, False, 40, 1000), ("f16", 256, False, 40, 1000), ("bf16", 256, True, 32, 1700), ("f32", 128, False, 48, 300),
+    ("bf16", 256, False, 36, 1000), ("bf16", 256, False, 37, 1000), ("bf16", 256, True, 37, 1000), ("bf16", 256, False, 30, 1100), ("bf16", 256, True, 24, 2048),
+    ("bf16", 256, False, 320, 128), ("bf16", 256, False, 321, 128), ("bf16", 256, True, 600, 64), ("f16", 256, False, 40, 1100),
+    ("bf16", 128, False, 101, 384), ("f16", 128, False, 102, 384), ("bf16", 128, False, 35, 1100), ("f16", 128, False, 36, 1100), ("f16", 128, True, 30, 1100), ("bf16", 128, True, 24, 2048),
 ])
 def test_a_head_among_many(dt, D, precise, NH, S):
     g = torch.Generator(device="cuda").manual_seed(S + D + NH)

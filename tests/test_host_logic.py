@@ -91,6 +91,14 @@ def test_gates_formed_in_a_row_kernel_go_to_that_kernel_alone():
     assert out.returncode == 0 and "row_dispatch: ok" in out.stdout, out.stdout + out.stderr
 
 
+def test_the_column_kernel_taken_is_the_one_measured_to_be_faster():
+    """tests/harness/col_dispatch (the library's own choice of a column kernel, compiled for the host)"""
+    here = os.path.join(os.path.dirname(os.path.abspath(__file__)), "harness")
+    subprocess.check_call(["make", "-C", here, "col_dispatch"])
+    out = subprocess.run([os.path.join(here, "col_dispatch")], capture_output=True, text=True)
+    assert out.returncode == 0 and "col_dispatch: ok" in out.stdout, out.stdout + out.stderr
+
+
 @pytest.mark.parametrize("scratch", [[], ["scratch"]])
 def test_chunk_states_of_a_kernel_with_scratch_memory_go_to_the_two_others(scratch):
     """tests/harness/chunk_dispatch (the library's own choice of the kernels of the chunk states, compiled for the host): a one-pass kernel that a compiler

@@ -728,8 +728,10 @@ static int launch_col_d(int D, const ColArgs& a, hipStream_t st) {
 }
 
 // col_kernel / colf_kernel, fp32, workgroups of 32 keys, us: D = 64, chunks of 128   128: 21.5 / 14.8   256: 22.9 / 16.0   320: 23.4 / 27.8
-//   uncut (300 positions)   240: 32.1 / 26.4   480: 34.1 / 37.0     D = 128, chunks of 128   256: 45.6 / 25.0   512: 49 / 45
-//   1024: 94.5 / 81   2048: 169 / 160   8192: 617 / 647   uncut   480: 60 / 48   1000: 100 / 103
+//   uncut (300 positions)   240: 32.1 / 26.4   480: 34.1 / 37.0     D = 128, uncut   300: 64 / 41   500: 66 / 58   1000: 100 / 103
+//   D = 128, chunks of 128 (heads)   256 (8): 46 / 27   512 (8): 51 / 47   1024 (32): 91 / 80   2048 (16): 182 / 159, (64): 160 / 157, (128): 152 / 160
+//     4096 (8): 364 / 348, (32): 325 / 323, (64): 315 / 324, (128): 313 / 331   8192 (16): 710 / 634, (32): 631 / 627, (64): 621 / 643   10240 (40): 804 / 774
+//   (col_kernel is up to 5 % faster where many heads make whole rounds of its one workgroup per CU, colf_kernel up to 11 % everywhere else: no line by size)
 bool colf_serves(int dtype, int D, const ColArgs& a) {
     if (dtype != MLSTM_F32 || D > 128 || g_force_generic || a.RS > D || (a.chunk_len > 0 ? a.chunk_len > 1024 : a.S > 2048)) return false;
     const long long wgs = 2ll * a.BH * a.NG;

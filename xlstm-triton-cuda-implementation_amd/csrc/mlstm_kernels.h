@@ -217,19 +217,29 @@ int launch_cold_kernel(int dtype, int D, const ColArgs& a, hipStream_t st);
 int launch_colw_kernel(int dtype, int D, const ColArgs& a, hipStream_t st);
 extern int g_col_variant;   // see mlstm_set_column_kernel: 0 = the library's choice, 1 = col16_kernel, 2 = cold_kernel, 3 = col_kernel
 constexpr int CW_MOST_QUERIES = 1024;    // queries a key of colw_kernel may meet: their scalars stay in LDS for the whole kernel
+// Workgroups of 64 keys up to which colw_kernel is the faster one.  It runs them in rounds of 256, one per CU; cold_kernel has one per 128 keys, one per CU too,
+// but two at D = 128 outside split mode.  Up to 512 colw_kernel's two rounds are shorter than cold_kernel's one or two.  Of 513 to 768 it needs a third: a short one
+// if the last tiles of a long head are in it (tiles go heaviest first), a whole one if heads are short or a sequence has a few chunks only, while cold_kernel is still in its
+// second, which a short last chunk leaves nearly empty.  cold_kernel / colw_kernel, us, workgroups of 64 keys (heads):
+//   D = 256, bf16, uncut   S = 64   579: 46 / 39   768: 50 / 44        S = 128   516: 42 / 40   580: 43 / 41   642: 43 / 44        S = 320   515: 41 / 45   768: 52 / 62
+//     S = 512   512: 48 / 43   576: 50 / 52   768: 59 / 67     S = 640   580: 59 / 65   640: 60 / 63     S = 768   576: 66 / 64   648: 71 / 79     S = 1000   512: 76 / 62   576: 84 / 78   640: 81 / 80   768: 83 / 94
+//     in chunks of 512   S = 1100   522: 59 / 61   594: 60 / 74   756: 75 / 85     S = 1536   600: 65 / 69   768: 76 / 76     S = 2048   512: 56 / 54   672: 76 / 75   768: 82 / 83     S = 4096   576: 76 / 70   768: 93 / 86
+//     in split mode   S = 1000   576: 97 / 88   768: 98 / 107     S = 1100   594: 76 / 92     S = 2048   768: 107 / 104     S = 4096   768: 119 / 107
+//   D = 256, fp16 (cold_kernel with some 95 registers spilled)   S = 320   515: 55 / 47   768: 68 / 64     S = 1100   594: 81 / 79   738: 98 / 91     S = 4096   768: 113 / 87     split mode   S = 1000   768: 102 / 102
+//   D = 128, bf16 (fp16 alike), uncut   S = 200   512: 21.5 / 19.9   580: 24 / 26   768: 24 / 28     S = 320   515: 28 / 29   768: 30 / 39     S = 384   576: 30 / 29   642: 32 / 35     S = 448   644: 35 / 34   770: 37 / 42
+//     S = 512   768: 40 / 38     S = 1000   512: 59 / 38   768: 63 / 56     in chunks   S = 1100   594: 42 / 42   756: 43 / 45     S = 1400   682: 43 / 42   770: 43 / 45     S = 1536   768: 46 / 42     S = 2048   768: 48 / 44
+//     in split mode   S = 64   768: 32 / 29     S = 320   515: 29 / 34     S = 1000   512: 63 / 51   640: 64 / 68   768: 66 / 76     S = 1100   595: 45 / 52     S = 1800   667: 51 / 55     S = 2048   768: 59 / 58     S = 4096   768: 67 / 58
+inline int colw_most_workgroups(int dtype, int D, const ColArgs& a) {
+    const bool paired = D == 128 && !a.precise;   // (cold_kernel's, on a CU)
+    if (dtype == MLSTM_F16 && D == 256) return 768;
+    if (a.chunk_len > 0 && a.chunk_len < a.NG * GATE_GRANULE) return a.S >= (paired ? 3ll : 4ll) * a.chunk_len ? 768 : paired ? 640 : 512;
+    if (paired) return a.NG <= 5 ? 512 : a.NG >= 8 ? 768 : 512 + 96 * (a.NG - 5);
+    return a.NG == 1 ? 768 : a.NG == 2 ? 640 : a.NG < 12 ? 512 : 576;
+}
 inline bool colw_serves(int dtype, int D, const ColArgs& a) {
     if (dtype == MLSTM_F32 || (D != 128 && D != 256) || g_force_generic || g_col_variant != 0) return false;
     if ((a.chunk_len > 0 && a.chunk_len < a.NG * GATE_GRANULE ? a.chunk_len : a.NG * GATE_GRANULE) > CW_MOST_QUERIES) return false;
-    // Workgroups of 64 keys up to which colw_kernel is the faster one; cold_kernel / colw_kernel, us (bf16, workgroups of 64 keys):
-    //   D = 128, S = 1000 (not in chunks)  256: 56 / 29   512: 59 / 38   768: 65 / 57   1024: 66 / 68    (S = 300, 640: 24.6 / 26.4)
-    //   D = 128 in chunks of 512           256: 35 / 21   512: 37 / 30   544: 41 / 37.5   640: 45 / 38.5   768: 47 / 42   1024: 49 / 53
-    //     in split mode                    128: 38 / 26   256: 39 / 27   512: 42 / 40   768: 58 / 57   1024: 60 / 73
-    //   D = 256, S = 1000                   64: 69 / 40   256: 71 / 44   512: 74 / 58   768: 79 / 89 (fp16 88 / 87)   1024: 97 / 118
-    //   D = 256 in chunks                  128: 51 / 32   256: 51 / 34   512: 56 / 53   768: 81 / 80   1024: 86 / 103
-    //   D = 256 in split mode              128: 64 / 41   256: 65 / 44   512: 70 / 66   768: 105 / 99   1024: 110 / 130
-    //   fp16 (at D = 256 with 50 registers spilled where bf16 has 10, one or two reloads per tile of a weighing wave): D = 128, S = 1000  768: 58 / 51
-    //     in chunks 512: 35 / 27   640: 43 / 36   768: 46 / 40   832: 41.5 / 46   in split mode 768: 55 / 51      D = 256 in chunks 512: 66 / 53   768: 103 / 79   in split mode 768: 123 / 99
-    return (long long)a.BH * a.NG <= 768;
+    return (long long)a.BH * a.NG <= colw_most_workgroups(dtype, D, a);
 }
 inline int launch_col_best(int dtype, int D, const ColArgs& a, hipStream_t st) {
     const bool half_big = dtype != MLSTM_F32 && (D == 128 || D == 256);
