@@ -61,11 +61,8 @@ SIZES = [
 ]
 
 
-@pytest.mark.parametrize("dt,precise", TYPES)
-@pytest.mark.parametrize("B,NH,S,D,L,strided", SIZES)
-def test_same_bits_as_two_kernels(dt, precise, B, NH, S, D, L, strided):
-    if precise and D == 128:
-        pytest.skip("one form only")
+@pytest.mark.parametrize("B,NH,S,D,L,strided,dt,precise", [(*size, *t) for size in SIZES for t in TYPES if not (t[1] and size[3] == 128)])
+def test_same_bits_as_two_kernels(B, NH, S, D, L, strided, dt, precise):
     x, dh = _inputs(dt, B, NH, S, D, strided, S + D + L)
     for t in _same(x, dh, precise, L):
         assert torch.isfinite(t).all()
@@ -73,13 +70,11 @@ def test_same_bits_as_two_kernels(dt, precise, B, NH, S, D, L, strided):
 
 # A decay between chunks of 0 (in every chunk; behind a position in the middle), input gates that nothing else comes near, values that are not finite in a whole
 # chunk and at the sequence's last position, whose tile may be short or the only one of a short chunk.
-@pytest.mark.parametrize("dt,precise", TYPES)
-@pytest.mark.parametrize("B,NH,S,D,L", [(1, 3, 1088, 256, 0), (1, 2, 1100, 256, 0), (1, 3, 1600, 128, 0), (1, 2, 1777, 128, 0), (1, 26, 1088, 256, 0), (1, 40, 1600, 128, 0),
-                                        (1, 2, 1088, 128, 256), (1, 3, 700, 256, 384)])
+@pytest.mark.parametrize("B,NH,S,D,L,dt,precise", [(*size, *t) for size in [
+    (1, 3, 1088, 256, 0), (1, 2, 1100, 256, 0), (1, 3, 1600, 128, 0), (1, 2, 1777, 128, 0), (1, 26, 1088, 256, 0), (1, 40, 1600, 128, 0), (1, 2, 1088, 128, 256), (1, 3, 700, 256, 384),
+] for t in TYPES if not (t[1] and size[3] == 128)])
 @pytest.mark.parametrize("what", ["forgets", "forgets once", "large input gates", "infinite", "infinite last", "nan last"])
-def test_same_bits_at_the_ends_of_the_ranges(what, dt, precise, B, NH, S, D, L):
-    if precise and D == 128:
-        pytest.skip("one form only")
+def test_same_bits_at_the_ends_of_the_ranges(what, B, NH, S, D, L, dt, precise):
     (q, k, v, f, i), dh = _inputs(dt, B, NH, S, D, False, S + D)
     if what == "forgets":
         f -= 60

@@ -736,7 +736,6 @@ int backward_impl(const void* dh, const void* q, const void* k, const void* v, c
     float* gvec = c.take<float>(z.BH * w.ncs * z.D);
     float* rowinter = c.take<float>(z.BH * z.S);
     float* anchor = c.take<float>(z.BH * w.ncs * z.anchor_parts());
-    int anchor_parts = 0;
     // (the one-kernel dF pass adds the parts up; see DfArgs)
     const bool fused_anchor = w.L <= 1024;
     char* hlo_buf = c.take<char>(z.precise ? z.BH * z.S * z.D * z.el : 0);
@@ -796,15 +795,13 @@ int backward_impl(const void* dh, const void* q, const void* k, const void* v, c
         ra2.lk = z.la; ra2.lv = z.lb;
         ra2.precise = z.precise ? 1 : 0;
         ra2.CstT_lo = z.precise ? Ev + lo_off : nullptr;
-        if (fused_anchor) {
-            ra2.dot_with = CstT; ra2.dot_with_lo = z.precise ? CstT + lo_off : nullptr; ra2.dot_part = anchor;
-            anchor_parts = mlstm::chunk_states_dot_parts(dtype, D, ra2);
-        }
+        if (fused_anchor) { ra2.dot_with = CstT; ra2.dot_with_lo = z.precise ? CstT + lo_off : nullptr; ra2.dot_part = anchor; }
         if (int e = launch_chunk_states(dtype, D, ra2, st)) return e;
-        if (fused_anchor) {
-        } else if (int e = launch_anchor(dtype, D, CstT, Ev, z.precise ? CstT + lo_off : nullptr, z.precise ? Ev + lo_off : nullptr, Nst, gvec, anchor,
-                                  (int)z.BH, (int)w.ncs, st))
-            return e;   // (both value-major)
+        if (!fused_anchor) {   // (both value-major)
+            if (int e = launch_anchor(dtype, D, CstT, Ev, z.precise ? CstT + lo_off : nullptr, z.precise ? Ev + lo_off : nullptr, Nst, gvec, anchor,
+                                      (int)z.BH, (int)w.ncs, st))
+                return e;
+        }
     }
     ColArgs ca{};
     ca.la = z.la; ca.lb = z.lb;
@@ -823,7 +820,7 @@ int backward_impl(const void* dh, const void* q, const void* k, const void* v, c
     DfArgs da{f, colsum, rowpart, df, di, (int)z.BH, (int)z.S, (int)z.NG, (int)z.row_slices(), ca.rowpart2, colw_serves(dtype, D, ca), col_chunks ? w.L : 0, rowinter, anchor, (int)w.ncs};
     da.lg = z.lg; da.gate_form = z.gate_form; da.stamp = stamp;
     if (col_chunks && fused_anchor) {
-        da.anchor = nullptr; da.anchor_part = anchor; da.anchor_parts = anchor_parts; da.anchor_va = Nst; da.anchor_vb = gvec; da.D = D;
+        da.anchor = nullptr; da.anchor_part = anchor; da.anchor_parts = (int)z.anchor_parts(); da.anchor_va = Nst; da.anchor_vb = gvec; da.D = D;
     }
     Timed t(MLSTM_K_DF, st);
     return launch_df(gate_dtype, da, st);

@@ -1832,10 +1832,6 @@ int launch_chunk_states(int dtype, int D, const ChunkArgs& a, hipStream_t st) {
     return MLSTM_ESHAPE;
 }
 
-int chunk_states_dot_parts(int dtype, int D, const ChunkArgs& a) {
-    return (D / 32) * (D / 32);
-}
-
 int set_state_kernel(int variant) {
     if (variant < 0 || variant > 2) return MLSTM_EINVAL;
     g_state_kernel = variant;

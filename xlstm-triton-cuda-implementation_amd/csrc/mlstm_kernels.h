@@ -307,16 +307,14 @@ struct ChunkArgs {
     int precise;
     void* Cst_lo;
     void* CstT_lo;
-    // The value-major carry can contract the states it forms (before rounding) with another set in the same layout
-    // (dot_with, dot_with_lo: its low-order terms or null): dot_part[bh][c][workgroup of the head] receives the partial
-    // sums of <state_c, dot_with_c>, chunk_states_dot_parts() per state.
+    // What writes the value-major states can contract them, as it writes them, with another set in the same layout (dot_with,
+    // dot_with_lo: its low-order terms or null): dot_part[bh][c][block] receives the partial sums of <state_c, dot_with_c>, one
+    // per block of 32 keys x 32 values (block = key block * D / 32 + value block).
     const void* dot_with = nullptr;
     const void* dot_with_lo = nullptr;
     float* dot_part = nullptr;
 };
 int launch_chunk_states(int dtype, int D, const ChunkArgs& a, hipStream_t st);
-// partial sums per state that the launch with these arguments leaves in ChunkArgs::dot_part
-int chunk_states_dot_parts(int dtype, int D, const ChunkArgs& a);
 // test and measurement aid: 0 = the library's choice by the size of the launch, 1 = chunk sums and carry (two kernels),
 // 2 = the one-pass kernel wherever it can serve
 int set_state_kernel(int variant);
