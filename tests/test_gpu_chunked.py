@@ -291,3 +291,26 @@ def test_one_pass_state_kernel(dt, B, NH, S, D, L):
     assert_matches_oracle(dtype, *(sl(x) for x in (q, k, v, f, i, dh)), h=sl(h), m=sl(m), b=sl(b), grads=[sl(g) for g in got], chunk_len=Lc)
     for name, x, y in zip(["h", "m", "b", "dq", "dk", "dv", "df", "di"], outs[0], outs[1]):
         assert torch.equal(x, y), name
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.float32, 64), (torch.float32, 128), (torch.float16, 64)])
+@pytest.mark.parametrize("S", [1025, 1055, 1057, 1150])
+def test_an_infinite_last_query_behind_a_tile_that_is_not_whole(dtype, D, S):
+    # The kernel for these shapes takes 32 positions at a time.  Column 5 of the last query is infinite, and all that meets it on the way to dK of earlier
+    # chunks is positive (values, dh and, by an h that opposes dh, the row's share of the normaliser): dK is infinite there and not NaN, which a row
+    # past the end with a weight of zero would make it.
+    q, k, v, f, i, dh = dev(*O.make_inputs(1, 2, S, D, dtype, seed=S, f_mean=6.0))
+    v = v.abs() + 0.5
+    dh[:, :, -1] = dh[:, :, -1].abs() + 0.5
+    L = length_in_use(0, S, D, dtype)
+    full = (S - 1) // L * L
+    assert 0 < full < S
+    h, m, b, saved = mm.mlstm_forward_save_hip(q, k, v, f, i)
+    b[:, :, -1] = b[:, :, -1].abs() + 10   # (above the normaliser's floor)
+    h[:, :, -1] = -dh[:, :, -1]
+    clean = mm.mlstm_backward_saved_hip(dh, q, k, v, f, i, h, m, b, saved)[1]
+    assert bool(torch.isfinite(clean).all())
+    q[:, :, -1, 5] = float("inf")
+    dk = mm.mlstm_backward_saved_hip(dh, q, k, v, f, i, h, m, b, saved)[1][:, :, :full]
+    assert bool(torch.isposinf(dk[..., 5]).all()), (int(dk[..., 5].isnan().sum()), int(torch.isfinite(dk[..., 5]).sum()))
+    assert bool(torch.isfinite(dk[..., [c for c in range(D) if c != 5]]).all())

@@ -42,7 +42,11 @@ __device__ const u32x4 zero_piece = {0, 0, 0, 0};
 // load, whose waits cost the sums 3 to 7 %; a variable that is no constant has its address fetched from memory.)
 typedef const __attribute__((address_space(1))) u32x4* GlobalPiece;
 __device__ __forceinline__ u32x4 piece_or_zeros(bool there, const void* piece) { return *(there ? (GlobalPiece)(size_t)piece : (GlobalPiece)(size_t)&zero_piece); }
-
+template <typename T>
+__device__ __forceinline__ T element_or_zero(bool there, const T* element) {
+    typedef const __attribute__((address_space(1))) T* Global;
+    return *(there ? (Global)(size_t)element : (Global)(size_t)&zero_piece);
+}
 
 // STRICT: split mode, the weighted V rows go to LDS as two tiles, hi and lo (ChunkArgs::precise)
 template <typename T, int D, bool STRICT = false>
@@ -779,18 +783,17 @@ __global__ __launch_bounds__(256, 2) void chunk_sum_small_kernel(ChunkArgs a) {
             t.x1 = a.reverse ? a.inv_n[poff + pos] : 0.f;
             t.x2 = a.reverse ? a.db[poff + pos] : 0.f;
         }
-        if (t0 + TP <= S) {
-            const T* kt = Kh + (size_t)t0 * rsK;   // (the same for all lanes)
-            const T* vt = Vh + (size_t)t0 * rsV;
-            const unsigned ko = (unsigned)(h * rsK) + c32, vo = (unsigned)(h * rsV) + c32;
+        const T* kt = Kh + (size_t)t0 * rsK;   // (the same for all lanes)
+        const T* vt = Vh + (size_t)t0 * rsV;
+        const unsigned ko = (unsigned)(h * rsK) + c32, vo = (unsigned)(h * rsV) + c32;
+        if (__builtin_expect(t0 + TP <= S, 1)) {
 #pragma unroll
             for (int s = 0; s < NS; s++) { t.k[s] = (kt + (size_t)(2 * s) * rsK)[ko]; t.v[s] = (vt + (size_t)(2 * s) * rsV)[vo]; }
-        } else {
+        } else {   // (rows past the end are zeros)
 #pragma unroll
             for (int s = 0; s < NS; s++) {
-                const int pos = t0 + 2 * s + h < S ? t0 + 2 * s + h : S - 1;
-                t.k[s] = Kh[(size_t)pos * rsK + c32];
-                t.v[s] = Vh[(size_t)pos * rsV + c32];
+                t.k[s] = element_or_zero(t0 + 2 * s + h < S, kt + (size_t)(2 * s) * rsK + ko);
+                t.v[s] = element_or_zero(t0 + 2 * s + h < S, vt + (size_t)(2 * s) * rsV + vo);
             }
         }
     };
